@@ -441,6 +441,36 @@ size_t sswin_tall_linear_weight_grad_workspace_bytes(int64_t N, int P, int K);
 int sswin_tall_linear_weight_grad(const float* dy, const float* x, int64_t N, int P, int K, float* dw,
                                   float* db, void* ws, size_t ws_bytes, void* stream);
 
+/* Dense layers of fp32, fp16 or bf16 tokens with what follows the product folded in (nn.Linear at swin3d_base.py:606-610 and
+ * :722-735; sswin_dense_supported: K and P multiples of 16).
+ * y [N, P] = last step of x [N, K] Wop + bias: transposed == 0: Wop = W^T of w [P, K] (the layer); 1: Wop = w [K, P] as stored
+ * (the input gradient of a layer with K outputs and P inputs; no bias).  x: dtype; w and bias: w_dtype (dtype, or fp32 under
+ * mixed precision); y: out_dtype (dtype, or fp32 with SSWIN_DENSE_RESIDUAL under mixed precision).
+ * epilogue SSWIN_DENSE_GELU: y = gelu(.), slope [N, P] = its derivative (or null); SSWIN_DENSE_RESIDUAL: y = . + extra [N, P]
+ * of out_dtype; SSWIN_DENSE_SCALE (transposed only): y = . * extra [N, P] of dtype.  Accumulation in fp32. */
+enum { SSWIN_DENSE_PLAIN = 0, SSWIN_DENSE_GELU = 1, SSWIN_DENSE_RESIDUAL = 2, SSWIN_DENSE_SCALE = 3 };
+int sswin_dense_supported(int dtype, int P, int K);
+int sswin_dense_forward(int dtype, int w_dtype, int out_dtype, int transposed, int epilogue, const void* x, int64_t N, int K,
+                        const void* w, const void* bias, int P, const void* extra, void* y, void* slope, void* stream);
+/* dw [P, K] = dy^T x and db [P] = column sums of dy (or null) for dy [N, P], x [N, K] of dtype; dw, db of out_dtype (dtype or
+ * fp32).  Partial sums over row chunks are added in a fixed order: the same bits on every run. */
+size_t sswin_dense_weight_grad_workspace_bytes(int dtype, int64_t N, int P, int K);
+int sswin_dense_weight_grad(int dtype, int out_dtype, const void* dy, const void* x, int64_t N, int P, int K, void* dw, void* db,
+                            void* ws, size_t ws_bytes, void* stream);
+
+/* nn.LayerNorm over rows of D values (swin3d_base.py:706, 722).  x of x_dtype; y of y_dtype (x_dtype, or a 16-bit type for
+ * fp32 x); gamma, beta fp32 for fp32 x, else of x_dtype.  stats: fp32 [2][N] mean and reciprocal deviation for the backward, or
+ * null.  sswin_layer_norm_supported: rows of whole 16-byte pieces, at most 8 x 64 of them.
+ * backward: dx = gradient of x through the norm + dres (the gradient arriving over a residual path, of x_dtype, or null);
+ * dgamma, dbeta summed in a fixed order. */
+int sswin_layer_norm_supported(int x_dtype, int D);
+int sswin_layer_norm_forward(int x_dtype, int y_dtype, const void* x, int64_t N, int D, const void* gamma, const void* beta,
+                             float eps, void* y, float* stats, void* stream);
+size_t sswin_layer_norm_backward_workspace_bytes(int x_dtype, int64_t N, int D);
+int sswin_layer_norm_backward(int x_dtype, int dy_dtype, const void* dy, const void* x, const float* stats, int64_t N, int D,
+                              const void* gamma, const void* dres, void* dx, void* dgamma, void* dbeta, void* ws, size_t ws_bytes,
+                              void* stream);
+
 /* ---- window-resident attention (whole forward / backward of the attention core) ---------- */
 
 /* Forward of sparse_swin/swin3d_base.py:660-672 for every (window, head) group in one pass:

@@ -82,6 +82,14 @@ SIGNATURES = {
     "sswin_tall_linear_input_grad": (_i32, [_vp, _i64, _i32, _vp, _i32, _vp, _vp]),
     "sswin_tall_linear_weight_grad_workspace_bytes": (_sz, [_i64, _i32, _i32]),
     "sswin_tall_linear_weight_grad": (_i32, [_vp, _vp, _i64, _i32, _i32, _vp, _vp, _vp, _sz, _vp]),
+    "sswin_dense_supported": (_i32, [_i32, _i32, _i32]),
+    "sswin_dense_forward": (_i32, [_i32, _i32, _i32, _i32, _i32, _vp, _i64, _i32, _vp, _vp, _i32, _vp, _vp, _vp, _vp]),
+    "sswin_dense_weight_grad_workspace_bytes": (_sz, [_i32, _i64, _i32, _i32]),
+    "sswin_dense_weight_grad": (_i32, [_i32, _i32, _vp, _vp, _i64, _i32, _i32, _vp, _vp, _vp, _sz, _vp]),
+    "sswin_layer_norm_supported": (_i32, [_i32, _i32]),
+    "sswin_layer_norm_forward": (_i32, [_i32, _i32, _vp, _i64, _i32, _vp, _vp, C.c_float, _vp, _vp, _vp]),
+    "sswin_layer_norm_backward_workspace_bytes": (_sz, [_i32, _i64, _i32]),
+    "sswin_layer_norm_backward": (_i32, [_i32, _i32, _vp, _vp, _vp, _i64, _i32, _vp, _vp, _vp, _vp, _vp, _vp, _sz, _vp]),
     "sswin_window_indices": (_i32, [_vp, _i64, _i32, _vp, _vp, _vp, _vp, _vp]),
     "sswin_shift_mask": (_i32, [_vp, _vp, _vp, _vp, _vp]),
     "sswin_window_coords": (_i32, [_vp, _i64, _i64, _vp, _vp, _vp, _vp]),
@@ -95,7 +103,7 @@ SIGNATURES = {
                                                _vp, _i64, _i32, _vp, _i64, _i32, _vp, _i64, _i32, _vp, _i32, _vp]),
 }
 
-ABI_VERSION = 29
+ABI_VERSION = 30
 _lib = None
 
 # A list turns on timing of the library's launches: every call that takes a stream is bracketed by events on that
@@ -161,6 +169,49 @@ def load():
         raise RuntimeError(f"libsswin3d ABI {lib.sswin_abi_version()} != binding ABI {ABI_VERSION}; rebuild")
     _lib = lib
     return lib
+
+
+_native = None
+
+
+def native():
+    """The compiled host path of the modules (``csrc/native.cpp``).  Raises :class:`LibraryMissing` if it has not been
+    built.  While ``launch_timer`` is a list its launches are recorded there too."""
+    global _native
+    if _native is None:
+        load()                           # the library first, behind PyTorch's HIP runtime
+        try:
+            from . import _native as mod
+        except ImportError as e:
+            raise LibraryMissing(f"sparseswin3d_amd/_native: {e}; build it with `python -m sparseswin3d_amd.build`") from e
+        _native = mod
+    if launch_timer is not _native_timed[0]:
+        _native_timed[0] = launch_timer
+        _native.set_recorder(None if launch_timer is None else _NativeRecorder(launch_timer))
+    return _native
+
+
+_native_timed = [None]
+
+
+class _NativeRecorder:
+    """Brackets the launches of the compiled host path by events, as :class:`_TimedLibrary` does for ctypes calls."""
+
+    def __init__(self, timer):
+        self.timer, self.open = timer, None
+
+    def __call__(self, call, before):
+        import torch
+        name = call.split("(", 1)[0].strip()
+        if launch_timer is not self.timer or (launch_timer_only is not None and name not in launch_timer_only):
+            return
+        event = torch.cuda.Event(enable_timing=True)
+        event.record()
+        if before:
+            self.open = event
+        elif self.open is not None:
+            self.timer.append((name, (), self.open, event))
+            self.open = None
 
 
 class _NoSwitch:
