@@ -272,7 +272,7 @@ KERNEL_SYMBOLS = {
 
 # operator-path table row -> (library entry point, leading integer arguments or None for any) of the launch it times
 OPERATOR_LAUNCHES = {
-    "token plan, one of a stage's two (operand map + group table)": ("sswin_token_plan", None),
+    "token plan, one of a stage's two (operand map + group table)": ("sswin_token_plan_batch", None),
     "sorted_coo_indices [4,E], Q/V": ("sswin_sorted_coo_indices", None),
     "operand_copy_qkv, voxel rows -> Q*scale, K^T, V": ("sswin_operand_copy_qkv", (0, 1)),
     "operand_copy_qkv, gradients -> voxel rows": ("sswin_operand_copy_qkv", (0, 0)),

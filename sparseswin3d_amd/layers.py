@@ -20,7 +20,7 @@ from torch.autograd import Function
 from torch.autograd.function import once_differentiable
 
 from . import _lib
-from .window_attention import WindowAttentionSparse, prefetch_plans, replace_feature, tall_linear
+from .window_attention import WindowAttentionSparse, _token_plan, prefetch_plans, replace_feature, tall_linear
 
 _DTYPE_CODE = {torch.float32: 0, torch.float16: 1, torch.bfloat16: 2}
 
@@ -165,13 +165,8 @@ def sparse_window_indices(indices: torch.Tensor, batch_size: int, dims: Sequence
         raise RuntimeError("sparse_window_indices runs on the GPU only; there is no CPU fallback")
     if indices.dtype != torch.int32 or indices.dim() != 2 or indices.shape[1] != 4:
         raise RuntimeError("sparse_window_indices: indices must be int32 [N, 4]")
-    indices = indices.contiguous()
-    out = torch.empty((indices.shape[0], 2), dtype=torch.int32, device=indices.device)
-    with _lib.on_device(indices.device):
-        _lib.check(_lib.load().sswin_window_indices(_ptr(indices), indices.shape[0], int(batch_size), _i32x3(dims),
-                                                    _i32x3(window_size), _i32x3(shift_size), _ptr(out),
-                                                    _stream(indices.device)))
-    return out
+    return _lib.native().window_indices(indices, int(batch_size), [int(e) for e in dims], [int(e) for e in window_size],
+                                        [int(e) for e in shift_size])
 
 
 class _PoolWindows(Function):
@@ -226,12 +221,36 @@ def downsample_plan(x, factor: int = 2, plan=None):
     if plan is None:
         req = downsample_plan_request(x, f)
         plan = TokenPlan(*req[:4], tasks=req[4], order_only=req[5])
-    plan.finish()
-    coords = torch.empty((plan.windows, 4), dtype=torch.int32, device=x.indices.device)
-    with _lib.on_device(coords.device):
-        _lib.check(_lib.load().sswin_window_coords(_ptr(plan.plan), plan.g_cap, plan.windows, _i32x3(dims), _i32x3(win),
-                                                   _ptr(coords), _stream(coords.device)))
+    coords = _lib.native().window_coords(plan.native, dims, win)
     return plan, coords, [e // f for e in dims]
+
+
+def _unhooked(*modules) -> bool:
+    return not any(m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks for m in modules)
+
+
+def _plain(*modules) -> bool:
+    """Modules of exactly these types without hooks: calling them is applying their parameters."""
+    return all(type(m) in (nn.LayerNorm, nn.Linear, nn.GELU) for m in modules) and _unhooked(*modules)
+
+
+def _norm_fits(norm, features) -> bool:
+    """``norm`` is a LayerNorm over the rows of ``features`` with gain and offset in the types the kernels take."""
+    return type(norm) is nn.LayerNorm and norm.weight is not None and norm.bias is not None and len(norm.normalized_shape) == 1 \
+        and norm.normalized_shape[0] == features.shape[1] and norm.weight.dtype == features.dtype \
+        and _lib.native().norm_supported(features)
+
+
+def _fused_dtype(features, weight):
+    """The type dense layers compute in for these features (autocast's inside an autocast region), or None where the
+    fused kernels do not take them."""
+    if not (features.is_cuda and features.dim() == 2 and features.dtype in _DTYPE_CODE):
+        return None
+    if torch.is_autocast_enabled("cuda"):
+        # a 16-bit residual stream under autocast mixes types in ways the kernels are not built for
+        dtype = torch.get_autocast_dtype("cuda")
+        return dtype if features.dtype == torch.float32 and weight.dtype == torch.float32 and dtype in _DTYPE_CODE else None
+    return features.dtype if weight.dtype == features.dtype else None
 
 
 class PoolDownsample(nn.Module):
@@ -256,10 +275,16 @@ class PoolDownsample(nn.Module):
 
     def forward(self, x, plan=None):
         plan, coords, shape = downsample_plan(x, 2, plan)
-        pooled = _PoolWindows.apply(x.features, plan, True)
+        dtype = _fused_dtype(x.features, self.reduction.weight) if _plain(self.norm, self.reduction) else None
+        if dtype is not None and _norm_fits(self.norm, x.features) and self.reduction.bias is None:
+            # pooling, norm and the dense layer in one autograd node
+            features = _lib.native().merge(x.features, self.norm.weight, self.norm.bias, self.reduction.weight, plan.native, self.norm.eps,
+                                           dtype)
+        else:
+            pooled = _PoolWindows.apply(x.features, plan, True)
+            features = tall_linear(self.norm(pooled), self.reduction)
         out = copy.copy(x)
-        out.indices, out.spatial_shape = coords, shape
-        out.features = tall_linear(self.norm(pooled), self.reduction)
+        out.indices, out.spatial_shape, out.features = coords, shape, features
         return out
 
 
@@ -336,6 +361,10 @@ class SwinTransformerBlock(nn.Module):
 
     def window_view(self, x):
         """``x`` seen as (window, position) tokens for this block's shift, and whether the block is shifted."""
+        view, shifted = self._view_of(x)
+        return replace_feature(view, x.features), shifted
+
+    def _view_of(self, x):
         d, h, w = x.spatial_shape
         window_size, shift_size = get_window_size((d, h, w), self.window_size, self.shift_size)
         shifted = any(s > 0 for s in shift_size)
@@ -356,7 +385,7 @@ class SwinTransformerBlock(nn.Module):
             view.plan_cache = {}
             if cache is not None:
                 cache[key] = view
-        return replace_feature(view, x.features), shifted
+        return view, shifted
 
     def prefetch(self, x):
         """Enqueue this block's window indices and token plan (see ``WindowAttentionSparse.prefetch_plan``);
@@ -382,7 +411,39 @@ class SwinTransformerBlock(nn.Module):
         x = replace_feature(x, self.norm2(x.features))
         return replace_feature(x, self.drop_path(self.mlp(x.features)))
 
+    def _fused_arguments(self, x):
+        """The compute dtype where the whole block runs as one autograd node, else None: LayerNorm, the fused attention path, GELU, and no dropout that is switched on."""
+        attn, mlp, f = self.attn, self.mlp, x.features
+        if self.training and (mlp.drop1.p > 0 or mlp.drop2.p > 0 or attn.proj_drop.p > 0 or
+                              (type(self.drop_path) is not nn.Identity and self.drop_path.drop_prob > 0)):
+            return None
+        if type(mlp) is not MLP or type(mlp.fn) is not nn.GELU or mlp.fn.approximate != "none" or \
+                type(attn) is not WindowAttentionSparse or not _unhooked(attn, mlp) or not _plain(self.norm1, self.norm2, attn.qkv, attn.proj, mlp.linear1, mlp.linear2, mlp.fn):
+            return None
+        if not (x.indices.is_cuda and x.indices.dtype == torch.int32 and x.indices.shape[0] > 0 and attn.num_heads < 256):
+            return None
+        weight = attn.qkv.weight
+        dtype = _fused_dtype(f, weight)
+        if dtype is None or not (_norm_fits(self.norm1, f) and _norm_fits(self.norm2, f)) or \
+                any(m.weight.dtype != weight.dtype for m in (attn.proj, mlp.linear1, mlp.linear2)):
+            return None
+        return dtype
+
     def forward(self, x, mask_matrix):
+        dtype = self._fused_arguments(x)
+        if dtype is not None:
+            view, shifted = self._view_of(x)
+            attn, mlp, n = self.attn, self.mlp, view.spatial_shape[0]
+            how = attn._fused_arguments(x.features, n)
+            if how is not None and how[0] is not None:
+                ti, resident, _ = how
+                plan = _token_plan(attn, view)
+                y = _lib.native().block(
+                    [x.features, self.norm1.weight, self.norm1.bias, attn.qkv.weight, attn.qkv.bias, attn.relative_position_bias_table,
+                     attn.proj.weight, attn.proj.bias, self.norm2.weight, self.norm2.bias, mlp.linear1.weight, mlp.linear1.bias,
+                     mlp.linear2.weight, mlp.linear2.bias], plan.native, mask_matrix if shifted else None, ti.code, ti.offset0, n,
+                    attn.num_heads, attn.scale, resident, self.norm1.eps, self.norm2.eps, dtype)
+                return replace_feature(x, y)
         shortcut = x
         x = self.forward_part1(x, mask_matrix)
         x = replace_feature(x, shortcut.features + self.drop_path(x.features))

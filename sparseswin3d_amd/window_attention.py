@@ -747,33 +747,41 @@ class WindowAttentionSparse(nn.Module):
         several blocks with shared launches."""
         return prefetch_plans([(self, x)])[0]
 
+    def _fused_arguments(self, features, n):
+        """(BiasTableIndex or None, window-resident kernels?, compute dtype) where the fused path takes this call, else
+        None.  Under autocast the projections and the attention run in its type, as ``nn.Linear`` would."""
+        from . import fused
+        if not self.fused:
+            return None
+        dtype = torch.get_autocast_dtype("cuda") if torch.is_autocast_enabled("cuda") else features.dtype
+        weight = self.qkv.weight.dtype
+        if dtype not in fused._DTYPE_CODE or weight not in (dtype, torch.float32) or self.proj.weight.dtype != weight:
+            return None
+        if features.dtype != dtype and not torch.is_autocast_enabled("cuda"):
+            return None
+        ti = self._table_index(n)
+        if n > 384 if ti is not None else n * n * 4 > 64 * 1024:
+            return None
+        can = self.dim == 32 * self.num_heads and n <= 128
+        return ti, can if self.resident is None else bool(self.resident), dtype
+
     def forward(self, x, mask):
         n = x.spatial_shape[0]
         b = x.batch_size
         c = x.features.shape[-1]
         plan = None
-        from . import fused
         if _takes_token_plan(self, x):
             # the token plan is enqueued first; the projection below runs while its totals travel.
-            # A stage hands the same window indices to several blocks: they share one plan.
-            cache = getattr(x, "plan_cache", None)
-            plan = cache.get(self.num_heads) if cache is not None else None
-            if plan is None:
-                plan = fused.TokenPlan(x.indices, b, n, self.num_heads, defer=True)
-                if cache is not None:
-                    cache[self.num_heads] = plan
+            plan = _token_plan(self, x)
+            native = self._fused_arguments(x.features, n)
+            if native is not None:
+                from . import fused
+                ti, resident, dtype = native
+                bias = self.relative_position_bias_table if ti is not None else self.relative_position_bias(n, torch.float32)
+                out = fused.fused_window_attention(None, bias, x.indices, mask, b, n, self.scale, resident, plan, ti,
+                                                   (x.features, self.qkv, self.proj, self.num_heads, dtype))
+                return replace_feature(x, self.proj_drop(out))
         qkv = tall_linear(x.features, self.qkv).reshape(-1, 3, self.num_heads, c // self.num_heads)
-        table_index = self._table_index(n) if plan is not None and self.fused else None
-        if plan is not None and self.fused and fused.supports(x.features, n, table_index is not None):
-            resident = fused.supports_resident(qkv, n) if self.resident is None else self.resident
-            if table_index is not None:
-                out = fused.fused_window_attention(qkv, self.relative_position_bias_table, x.indices, mask, b, n,
-                                                   self.scale, resident, plan, table_index)
-            else:
-                out = fused.fused_window_attention(qkv, self.relative_position_bias(n, torch.float32), x.indices,
-                                                   mask, b, n, self.scale, resident, plan)
-            x = replace_feature(x, out)
-            return replace_feature(x, self.proj_drop(tall_linear(x.features, self.proj)))
         q, k_t, v = qkv_sparse_cuda(qkv, x.indices, b, n, plan, q_scale=self.scale)         # q = q * self.scale
         attn = spspmm_block_naive(q, k_t, "q_k")
         biased = sp_add_table_bias_and_mask(attn, self.relative_position_bias_table, self._table_index(n), mask, plan)
@@ -803,6 +811,19 @@ def _takes_token_plan(attn, x) -> bool:
     GPU."""
     return x.features.is_cuda and x.indices.is_cuda and x.indices.dtype == torch.int32 and x.indices.shape[0] > 0 \
         and attn.num_heads < 256
+
+
+def _token_plan(attn, x):
+    """The token plan of ``x``'s window indices for ``attn``'s heads, possibly still in flight.  A stage hands the same
+    window indices to several blocks: they share one plan through ``x.plan_cache``."""
+    from . import fused
+    cache = getattr(x, "plan_cache", None)
+    plan = cache.get(attn.num_heads) if cache is not None else None
+    if plan is None:
+        plan = fused.TokenPlan(x.indices, x.batch_size, x.spatial_shape[0], attn.num_heads, defer=True)
+        if cache is not None:
+            cache[attn.num_heads] = plan
+    return plan
 
 
 def prefetch_plans(pairs, extra=()):

@@ -1,0 +1,214 @@
+"""GPU parity of the dense layers with a folded last step (``sswin_dense_*``), of the row norm (``sswin_layer_norm_*``) and
+of the modules' compiled host path against float64 arithmetic on the same inputs.
+
+Bounds: fp32 products are held to 1e-6 of the sum of the absolute products (what an fp32 GEMM reaches); 16-bit results to
+one rounding of the result (2^-8 bf16, 2^-11 fp16) plus the same 1e-6; a last step adds its own value to the scale."""
+import ctypes as C
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+CODE = {torch.float32: 0, torch.float16: 1, torch.bfloat16: 2}
+ROUND = {torch.float32: 0.0, torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8}
+PLAIN, GELU, RESIDUAL, SCALE = range(4)
+
+
+def _ptr(t):
+    return C.c_void_p(t.data_ptr() if t is not None else None)
+
+
+def _stream():
+    return C.c_void_p(torch.cuda.current_stream().cuda_stream)
+
+
+def _rand(gen, *shape, dtype=torch.float32, spread=3):
+    # values over several binades, so that every piece of a split carries bits
+    return (torch.randn(*shape, generator=gen) * torch.exp2(torch.randint(-spread, spread + 1, shape, generator=gen).float())).to(dtype).cuda()
+
+
+def _check(got, ref, scale, dtype, what):
+    assert not torch.isnan(got).any(), what
+    err = (got.double() - ref).abs()
+    bound = 1e-6 * scale + ROUND[dtype] * ref.abs() + (2.0 ** -24 if dtype == torch.float16 else 1e-30)
+    assert (err <= bound).all(), f"{what}: {(err / bound).max().item():.2f} of the bound"
+
+
+def _forward(lib, _lib, x, w, b, transposed, epi, extra, out):
+    N, K = x.shape
+    P = w.shape[1] if transposed else w.shape[0]
+    y = torch.full((N, P), float("nan"), dtype=out, device="cuda")
+    slope = torch.full((N, P), float("nan"), dtype=out, device="cuda") if epi == GELU else None
+    _lib.check(lib.sswin_dense_forward(CODE[x.dtype], CODE[w.dtype], CODE[out], transposed, epi, _ptr(x), N, K, _ptr(w), _ptr(b), P,
+                                       _ptr(extra), _ptr(y), _ptr(slope), _stream()))
+    return y, slope
+
+
+# one row, part of a tile, tile edges, many tiles; reductions of one step, of odd counts of steps, of whole blocks; columns of
+# part of a column block and of several; the few-rows kernel and the tiled ones; 96 channels: the kernel with W in LDS
+SHAPES = [(1, 16, 16), (31, 48, 144), (33, 96, 96), (300, 384, 1152), (129, 1536, 48), (9000, 48, 192), (9001, 112, 208),
+          (30000, 96, 288), (20001, 144, 48), (20000, 288, 96)]
+
+
+@pytest.mark.parametrize("N,K,P", SHAPES)
+@pytest.mark.parametrize("dtype,wdtype,out", [(torch.float32, torch.float32, torch.float32), (torch.bfloat16, torch.bfloat16, torch.bfloat16),
+                                              (torch.float16, torch.float32, torch.float16), (torch.float16, torch.float32, torch.float32)],
+                         ids=["fp32", "bf16", "fp16-w32", "fp16-w32-out32"])
+def test_dense_forward_and_input_gradient(N, K, P, dtype, wdtype, out):
+    from sparseswin3d_amd import _lib
+    lib = _lib.load()
+    gen = torch.Generator().manual_seed(N + 3 * K + 7 * P)
+    x, w, b = _rand(gen, N, K, dtype=dtype), _rand(gen, P, K, dtype=wdtype, spread=1) / K ** 0.5, _rand(gen, P, dtype=wdtype)
+    extra = _rand(gen, N, P, dtype=out)
+    w = w.to(wdtype)
+    wd = w.to(dtype).double()                                    # fp32 weights are rounded to the tokens' type
+    pre = x.double() @ wd.T + b.double()
+    mag = x.double().abs() @ wd.abs().T + b.double().abs()
+    if out == dtype:
+        y, _ = _forward(lib, _lib, x, w, b, 0, PLAIN, None, out)
+        _check(y, pre, mag, out, "plain")
+        y, slope = _forward(lib, _lib, x, w, b, 0, GELU, None, out)
+        cdf = 0.5 * (1 + torch.erf(pre / 2 ** 0.5))
+        # |gelu'| < 1.13 and |gelu''| < 0.8: an error of the product passes into both results at most at that size
+        _check(y, pre * cdf, 1.13 * mag + pre.abs(), out, "gelu")
+        _check(slope, cdf + pre * torch.exp(-0.5 * pre ** 2) / (2 * torch.pi) ** 0.5, 0.8 * mag + 1.2, out, "gelu'")
+        dy, f = _rand(gen, N, P, dtype=dtype), _rand(gen, N, K, dtype=dtype)
+        dx, _ = _forward(lib, _lib, dy, w, None, 1, PLAIN, None, out)
+        ref, dmag = dy.double() @ wd, dy.double().abs() @ wd.abs()
+        _check(dx, ref, dmag, out, "input gradient")
+        dx, _ = _forward(lib, _lib, dy, w, None, 1, SCALE, f, out)
+        _check(dx, ref * f.double(), dmag * f.double().abs(), out, "input gradient times a factor")
+    y, _ = _forward(lib, _lib, x, w, b, 0, RESIDUAL, extra, out)
+    _check(y, pre + extra.double(), mag + extra.double().abs(), out, "residual")
+
+
+@pytest.mark.parametrize("N,P,K", [(1, 16, 16), (17, 144, 48), (1024, 96, 96), (1025, 48, 208), (1100, 288, 96), (9001, 208, 192), (70001, 48, 144)])
+@pytest.mark.parametrize("dtype,out", [(torch.float32, torch.float32), (torch.bfloat16, torch.bfloat16), (torch.float16, torch.float32)],
+                         ids=["fp32", "bf16", "fp16-out32"])
+def test_dense_weight_gradient(N, P, K, dtype, out):
+    from sparseswin3d_amd import _lib
+    lib = _lib.load()
+    gen = torch.Generator().manual_seed(N + P + K)
+    dy, x = _rand(gen, N, P, dtype=dtype), _rand(gen, N, K, dtype=dtype)
+    results = []
+    for _ in range(2):
+        dw, db = (torch.full(s, float("nan"), dtype=out, device="cuda") for s in ((P, K), (P,)))
+        nb = lib.sswin_dense_weight_grad_workspace_bytes(CODE[dtype], N, P, K)
+        ws = torch.empty(max(nb, 1), dtype=torch.uint8, device="cuda")
+        _lib.check(lib.sswin_dense_weight_grad(CODE[dtype], CODE[out], _ptr(dy), _ptr(x), N, P, K, _ptr(dw), _ptr(db), _ptr(ws), nb, _stream()))
+        results.append((dw, db))
+    _check(results[0][0], dy.double().T @ x.double(), dy.double().abs().T @ x.double().abs(), out, "dW")
+    _check(results[0][1], dy.double().sum(0), dy.double().abs().sum(0), out, "db")
+    assert torch.equal(results[0][0], results[1][0]) and torch.equal(results[0][1], results[1][1])       # fixed order of the sums
+
+
+def test_dense_refuses_what_it_does_not_take():
+    from sparseswin3d_amd import _lib
+    lib = _lib.load()
+    x = torch.zeros(4, 24, device="cuda")
+    assert not lib.sswin_dense_supported(0, 16, 24) and lib.sswin_dense_supported(2, 16, 32) and not lib.sswin_dense_supported(3, 16, 16)
+    assert lib.sswin_dense_forward(0, 0, 0, 0, PLAIN, _ptr(x), 4, 24, _ptr(x), None, 16, None, _ptr(x), None, _stream()) != 0
+    assert b"multiples of 16" in lib.sswin_last_error()
+    assert lib.sswin_dense_forward(0, 0, 0, 0, SCALE, _ptr(x), 4, 16, _ptr(x), None, 16, _ptr(x), _ptr(x), None, _stream()) != 0
+    assert lib.sswin_dense_forward(0, 0, 0, 0, RESIDUAL, _ptr(x), 4, 16, _ptr(x), None, 16, None, _ptr(x), None, _stream()) != 0
+    assert lib.sswin_dense_forward(0, 0, 0, 0, PLAIN, None, 0, 16, None, None, 16, None, None, None, _stream()) == 0
+
+
+@pytest.mark.parametrize("N,D", [(1, 16), (7, 48), (1000, 96), (33, 192), (257, 768), (5, 80), (63, 1536), (4, 2048), (50000, 96)])
+@pytest.mark.parametrize("dtype,out", [(torch.float32, torch.float32), (torch.float32, torch.float16), (torch.bfloat16, torch.bfloat16)],
+                         ids=["fp32", "fp32-fp16", "bf16"])
+def test_layer_norm(N, D, dtype, out):
+    from sparseswin3d_amd import _lib
+    lib = _lib.load()
+    assert lib.sswin_layer_norm_supported(CODE[dtype], D)
+    gen = torch.Generator().manual_seed(N + D)
+    x, dy, dres = _rand(gen, N, D, dtype=dtype), _rand(gen, N, D, dtype=out), _rand(gen, N, D, dtype=dtype)
+    g, b = _rand(gen, D, dtype=dtype, spread=1), _rand(gen, D, dtype=dtype, spread=1)
+    y, stats = torch.full((N, D), float("nan"), dtype=out, device="cuda"), torch.empty(2, N, device="cuda")
+    _lib.check(lib.sswin_layer_norm_forward(CODE[dtype], CODE[out], _ptr(x), N, D, _ptr(g), _ptr(b), 1e-5, _ptr(y), _ptr(stats), _stream()))
+    xd, gd, dyd = x.double(), g.double(), dy.double()
+    mean, var = xd.mean(1, keepdim=True), xd.var(1, unbiased=False, keepdim=True)
+    rstd = (var + 1e-5).rsqrt()
+    xh = (xd - mean) * rstd
+    # the mean of a row carries an error of its magnitude times the sum's rounding, which the norm scales by 1 / deviation
+    slack = 1 + xd.abs().amax(1, keepdim=True) * rstd
+    _check(y, xh * gd + b.double(), gd.abs() * slack + b.double().abs(), out, "norm")
+    nb = lib.sswin_layer_norm_backward_workspace_bytes(CODE[dtype], N, D)
+    ws = torch.empty(nb, dtype=torch.uint8, device="cuda")
+    dx, dg, db = (torch.full(s, float("nan"), dtype=dtype, device="cuda") for s in ((N, D), (D,), (D,)))
+    _lib.check(lib.sswin_layer_norm_backward(CODE[dtype], CODE[out], _ptr(dy), _ptr(x), _ptr(stats), N, D, _ptr(g), _ptr(dres), _ptr(dx), _ptr(dg),
+                                             _ptr(db), _ptr(ws), nb, _stream()))
+    gy = dyd * gd
+    ref = rstd * (gy - gy.mean(1, keepdim=True) - xh * (gy * xh).mean(1, keepdim=True)) + dres.double()
+    _check(dx, ref, rstd * (gy.abs() + gy.abs().mean(1, keepdim=True) * (1 + xh.abs() * xh.abs().amax(1, keepdim=True))) * slack + dres.double().abs(), dtype,
+           "dx")
+    _check(dg, (dyd * xh).sum(0), (dyd.abs() * (xh.abs() + slack)).sum(0), dtype, "d gain")
+    _check(db, dyd.sum(0), dyd.abs().sum(0), dtype, "d offset")
+
+
+def _stage_pieces(dim, heads, window, dtype, merge, seed, grid=(21, 18, 11), n=3000, qkv_bias=True):
+    import numpy as np
+    from sparseswin3d_amd.layers import BasicLayer, PoolDownsample
+    from sparseswin3d_amd.window_attention import SparseVoxelTensor
+    rng = np.random.default_rng(seed)
+    cells = rng.choice(int(np.prod(grid)), size=n, replace=False)
+    c4 = np.stack([np.zeros_like(cells), *np.unravel_index(cells, grid)], 1).astype(np.int32)
+    torch.manual_seed(seed)
+    layer = BasicLayer(dim, 2, heads, (window,) * 3, 0.0, qkv_bias=qkv_bias, downsample=PoolDownsample if merge else None)
+    with torch.no_grad():
+        for p in layer.parameters():
+            p.add_(0.05 * torch.randn_like(p))
+    layer = layer.cuda().to(dtype)
+    feats = torch.randn(n, dim).cuda().to(dtype)
+    return layer, lambda x: layer(SparseVoxelTensor(x, torch.from_numpy(c4).cuda(), grid, 1)).features, feats
+
+
+@pytest.mark.parametrize("dim,heads,window,merge,qkv_bias", [(96, 3, 5, True, True), (48, 3, 7, False, True), (192, 6, 5, True, False), (80, 5, 5, False, True)])
+@pytest.mark.parametrize("mode", ["fp32", "bf16", "amp"])
+def test_stage_as_single_nodes_equals_its_composition(dim, heads, window, merge, qkv_bias, mode, monkeypatch):
+    """BasicLayer with each block (and the merge) as one autograd node against the same layer composed of its modules, all
+    gradients included.  fp32: both chains carry fp32 rounding only (2e-5 of the norm of a result); 16-bit: the composition
+    rounds every intermediate to 16 bits, one node fewer of them, so the two differ by roundings of the type."""
+    from sparseswin3d_amd import layers
+    dtype = torch.bfloat16 if mode == "bf16" else torch.float32
+    layer, run, feats = _stage_pieces(dim, heads, window, dtype, merge, dim + window, qkv_bias=qkv_bias)
+    results = []
+    for single in (True, False):
+        if not single:
+            monkeypatch.setattr(layers, "_fused_dtype", lambda *a: None)
+        layer.zero_grad(set_to_none=True)
+        x = feats.clone().requires_grad_(True)
+        with torch.autocast("cuda", dtype=torch.float16, enabled=mode == "amp"):
+            y = run(x)
+        gen = torch.Generator(device="cuda").manual_seed(1)
+        up = torch.randn(y.shape, generator=gen, device="cuda").to(y.dtype)
+        assert (("MergeNode" if merge else "BlockNode") in y.grad_fn.name()) == single, y.grad_fn.name()
+        y.backward(up)
+        results.append([("out", y.detach()), ("dx", x.grad)] + [(k, p.grad) for k, p in layer.named_parameters()])
+        with torch.no_grad(), torch.autocast("cuda", dtype=torch.float16, enabled=mode == "amp"):
+            # inference differs from the training forward in what it keeps, and where nothing rounds in between not in its result
+            assert torch.equal(run(feats), y.detach()), "inference"
+    tol = {"fp32": 2e-5, "bf16": 4e-2, "amp": 8e-3}[mode]
+    for (k, a), (_, b) in zip(*results):
+        assert a.dtype == b.dtype and a.shape == b.shape, k
+        rel = ((a.double() - b.double()).norm() / b.double().norm()).item()
+        assert rel < tol, (k, rel)
+
+
+def test_blocks_with_dropout_or_hooks_run_their_modules():
+    layer, run, feats = _stage_pieces(96, 3, 5, torch.float32, False, 5)
+    calls = []
+    handle = layer.blocks[0].norm2.register_forward_hook(lambda *a: calls.append(1))
+    a = run(feats)
+    assert calls == [1]
+    handle.remove()
+    b = run(feats)
+    assert calls == [1] and torch.allclose(a, b, rtol=1e-4, atol=1e-5)
+    layer.blocks[1].mlp.drop1.p = 0.5
+    layer.train()
+    torch.manual_seed(0)
+    c = run(feats)
+    assert not torch.allclose(b, c, rtol=1e-3, atol=1e-3)
+    layer.eval()
+    assert torch.allclose(run(feats), b, rtol=1e-4, atol=1e-5)
