@@ -458,6 +458,25 @@ size_t sswin_dense_weight_grad_workspace_bytes(int dtype, int64_t N, int P, int 
 int sswin_dense_weight_grad(int dtype, int out_dtype, const void* dy, const void* x, int64_t N, int P, int K, void* dw, void* db,
                             void* ws, size_t ws_bytes, void* stream);
 
+/* Window attention for heads of 16 or 32 channels and windows of any size, the attention matrix kept in registers
+ * (swin3d_base.py:654-675 from the projected qkv [N, 3 H hd] to the output [N, H hd] in voxel order, and its backward).  The bias
+ * comes from the relative position table [rows, H] (fp32): bias of positions p, q = table[code[p] - code[q] + offset0], codes
+ * not negative, at most 4096 rows.  sswin_flash_supported tells whether a shape is taken.
+ * sswin_flash_tokens: word [N] (what a token contributes to table index, mask and window comparisons) and tok_sq [N] (sum of
+ *   c * c over the windows before the token's own; or null) from a token plan's group table and tokens; mask [nmw, n] int8 region
+ *   ids or null.
+ * forward: lse fp32 [H, N] for the backward.
+ * backward: dqkv; ds (or null) = gradient of the scores in the groups' [c x c] blocks, for sswin_bias_table_grad; delta fp32 [H, N]
+ *   scratch. */
+int sswin_flash_supported(int dtype, int64_t N, int H, int hd, int rows);
+int sswin_flash_tokens(const int32_t* plan, int64_t g_cap, int64_t groups, const int32_t* tokens, int64_t N, int H, int n,
+                       const int32_t* code, const int8_t* mask, int nmw, int32_t* word, int32_t* tok_sq, void* stream);
+int sswin_flash_forward(int dtype, const int32_t* tokens, const int32_t* word, int64_t N, int H, int hd, int n, const void* qkv,
+                        float scale, const float* table, int rows, int offset0, void* out, float* lse, void* stream);
+int sswin_flash_backward(int dtype, const int32_t* tokens, const int32_t* word, const int32_t* tok_sq, int64_t N, int H, int hd, int n,
+                         const void* qkv, float scale, const float* table, int rows, int offset0, const void* out, const float* lse,
+                         const void* dout, void* dqkv, float* delta, float* ds, void* stream);
+
 /* nn.LayerNorm over rows of D values (swin3d_base.py:706, 722).  x of x_dtype; y of y_dtype (x_dtype, or a 16-bit type for
  * fp32 x); gamma, beta fp32 for fp32 x, else of x_dtype.  stats: fp32 [2][N] mean and reciprocal deviation for the backward, or
  * null.  sswin_layer_norm_supported: rows of whole 16-byte pieces, at most 8 x 64 of them.

@@ -86,6 +86,11 @@ SIGNATURES = {
     "sswin_dense_forward": (_i32, [_i32, _i32, _i32, _i32, _i32, _vp, _i64, _i32, _vp, _vp, _i32, _vp, _vp, _vp, _vp]),
     "sswin_dense_weight_grad_workspace_bytes": (_sz, [_i32, _i64, _i32, _i32]),
     "sswin_dense_weight_grad": (_i32, [_i32, _i32, _vp, _vp, _i64, _i32, _i32, _vp, _vp, _vp, _sz, _vp]),
+    "sswin_flash_supported": (_i32, [_i32, _i64, _i32, _i32, _i32]),
+    "sswin_flash_tokens": (_i32, [_vp, _i64, _i64, _vp, _i64, _i32, _i32, _vp, _vp, _i32, _vp, _vp, _vp]),
+    "sswin_flash_forward": (_i32, [_i32, _vp, _vp, _i64, _i32, _i32, _i32, _vp, C.c_float, _vp, _i32, _i32, _vp, _vp, _vp]),
+    "sswin_flash_backward": (_i32, [_i32, _vp, _vp, _vp, _i64, _i32, _i32, _i32, _vp, C.c_float, _vp, _i32, _i32, _vp, _vp, _vp, _vp, _vp,
+                                    _vp, _vp]),
     "sswin_layer_norm_supported": (_i32, [_i32, _i32]),
     "sswin_layer_norm_forward": (_i32, [_i32, _i32, _vp, _i64, _i32, _vp, _vp, C.c_float, _vp, _vp, _vp]),
     "sswin_layer_norm_backward_workspace_bytes": (_sz, [_i32, _i64, _i32]),
@@ -103,7 +108,7 @@ SIGNATURES = {
                                                _vp, _i64, _i32, _vp, _i64, _i32, _vp, _i64, _i32, _vp, _i32, _vp]),
 }
 
-ABI_VERSION = 30
+ABI_VERSION = 31
 _lib = None
 
 # A list turns on timing of the library's launches: every call that takes a stream is bracketed by events on that

@@ -1,0 +1,708 @@
+// Window attention for windows of any size with heads of 16 or 32 channels, the attention matrix kept in registers
+// (WindowAttention.forward, sparse_swin/swin3d_base.py:654-675, from the projected qkv to the attention output, and its
+// backward).  It serves what the kernels of window_attention.hip do not take: heads of 16 channels, windows of more than 128
+// positions (the reference's own setting: 7^3 windows, heads of 16).
+//
+// Work: the token ranks (sorted by window) are cut into chunks of 32 and a wavefront owns the blocks that start in its chunk:
+// 32 tokens of a large window, or several small windows together up to 32 tokens, so that sparse scenes do not pay a tile
+// per window.  A block walks over the tokens of its window(s) 16 at a time; all products are 16 x 16 tiles, so that padding
+// stops at 16 rows.  No task list, no barrier in the loop; the next 16 rows are covered by the other wavefronts of the SIMD.
+//
+// Layouts: v_mfma_f32_16x16x*: operand lane l = (row l % 16, reduction slots 4 (l / 16) + j), accumulator lane l = (column
+// l % 16, rows 4 (l / 16) + r).  An accumulator packed in place is therefore the operand of the next product over its rows:
+// S^T = K Q^T gives P^T as the operand of O^T = V^T P^T, and the row of a query (its maximum, sum and rescaling) lies in the
+// four lanes l % 16.  fp32 tokens take four 16x16x4 fp32 products per 16 slots, 16-bit tokens one 16x16x16.
+//
+// Softmax as the operators define it: exp(s - m) / (sum exp(s - m) + 1e-8), m = max(0, row maximum).  The running offset is the
+// maximum over the first 16 tokens (so that 16-bit P keeps its precision where all scores are far below 0) and moves only when
+// a score exceeds it by 10 in units of log 2: a row usually needs one exchange between its lanes at the start and one at the
+// end, where the 1e-8 is scaled to the offset that was used.
+//
+// The relative position bias is read from the table of the head in LDS: index of (p, q) = code[p] - code[q] + offset.  A token
+// carries {4 code, mask region, window} in one word, so one subtraction gives the table address and whether mask or window
+// differ.
+//
+// 112 700 voxels, windows of 7^3, 3 heads of 16 (27 million scores): fp32 forward 63 us, backward 212 us (the store of dS 36 of
+// them); fp16 39 and 118.  The block products with the attention matrix in memory take 195 and 258 us (fp32).  The vector ALU is
+// busy for half of a launch, the fp32 matrix instructions (which occupy it) for another quarter; leaving out the bias reads, the
+// exponentials or the row loads one by one changes the forward by less than 3 %, the rows of the backward by 15 %.
+#include <math.h>
+
+#include <algorithm>
+#include <type_traits>
+
+#include "sswin_common.hpp"
+
+namespace sswin {
+namespace flash {
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+
+constexpr float LOG2E = 1.4426950408889634f;
+constexpr float MASKED = -100.f * LOG2E;       // what sp_add_mask adds, in units of log 2
+constexpr int WAVES = 4;
+constexpr int MAX_ROWS = 4096;
+constexpr int64_t MAX_TOKENS = 1 << 24;    // row numbers are multiplied in 24 bits
+
+// four reduction slots of one operand row
+template <typename T> struct Frag;
+template <> struct Frag<float> {
+    f32x4 v;
+    __device__ __forceinline__ void load(const float* p) { v = *reinterpret_cast<const f32x4*>(p); }
+};
+template <> struct Frag<__half> {
+    f16x4 v;
+    __device__ __forceinline__ void load(const __half* p) { v = *reinterpret_cast<const f16x4*>(p); }
+};
+template <> struct Frag<__hip_bfloat16> {
+    s16x4 v;
+    __device__ __forceinline__ void load(const __hip_bfloat16* p) { v = *reinterpret_cast<const s16x4*>(p); }
+};
+
+__device__ __forceinline__ f32x4 mma(const Frag<float>& a, const Frag<float>& b, f32x4 c) {
+#pragma unroll
+    for (int s = 0; s < 4; ++s) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a.v[s], b.v[s], c, 0, 0, 0);
+    return c;
+}
+__device__ __forceinline__ f32x4 mma(const Frag<__half>& a, const Frag<__half>& b, const f32x4& c) {
+    return __builtin_amdgcn_mfma_f32_16x16x16f16(a.v, b.v, c, 0, 0, 0);
+}
+__device__ __forceinline__ f32x4 mma(const Frag<__hip_bfloat16>& a, const Frag<__hip_bfloat16>& b, const f32x4& c) {
+    return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a.v, b.v, c, 0, 0, 0);
+}
+
+template <typename T> __device__ __forceinline__ Frag<T> packed(const f32x4& c);
+template <> __device__ __forceinline__ Frag<float> packed<float>(const f32x4& c) { return Frag<float>{c}; }
+template <> __device__ __forceinline__ Frag<__half> packed<__half>(const f32x4& c) {
+    return Frag<__half>{f16x4{(_Float16)c[0], (_Float16)c[1], (_Float16)c[2], (_Float16)c[3]}};
+}
+template <> __device__ __forceinline__ Frag<__hip_bfloat16> packed<__hip_bfloat16>(const f32x4& c) {
+    s16x4 o;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[e] = __builtin_bit_cast(short, __float2bfloat16(c[e]));
+    return Frag<__hip_bfloat16>{o};
+}
+
+struct Args {
+    const int32_t* order;      // voxel of token rank r
+    const int32_t* tok_T;      // rank of the first token of r's window
+    const int32_t* tok_c;      // tokens of r's window
+    const uint32_t* word;      // 4 code | region << 15 | first rank << 23 | several regions << 31 of token r (flash_tokens_kernel)
+    int64_t N;
+    int H, rows, offset4;
+    float scale;               // of the scores
+    const float* table;        // [rows, H]
+    const void* qkv;           // [N, 3 H hd] voxel rows
+    void* out;                 // [N, H hd]
+    float* lse;                // [H, N] by rank: offset + log2 of the row sum
+    // backward
+    const void* dout;          // [N, H hd]
+    float* delta;              // [H, N] by rank: dO . O
+    void* dqkv;                // [N, 3 H hd]
+    float* ds;                 // [c x c] blocks of the groups, or null
+    const int32_t* tok_sq;     // sum of c * c over the windows before r's
+};
+
+// What a token contributes to the table index, mask and window comparisons, one word per rank, and the sum of c * c over
+// the windows before its own; a wavefront per window
+__global__ __launch_bounds__(256) void flash_tokens_kernel(const int32_t* __restrict__ plan, int64_t g_cap, int64_t windows, int H,
+                                                           const int32_t* __restrict__ tok_pos, const int32_t* __restrict__ code,
+                                                           const int8_t* __restrict__ mask, int nmw, int n, uint32_t* __restrict__ word,
+                                                           int32_t* __restrict__ tok_sq) {
+    const int64_t k = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (k >= windows) return;
+    const int64_t g = k * H;                                             // the window's first group (head 0)
+    const int c = plan[g], T = plan[g_cap + g], sq = plan[2 * g_cap + g] / H, w = plan[3 * g_cap + g];
+    const int8_t* region = mask ? mask + (int64_t)(w % nmw) * n : nullptr;
+    uint32_t several = 0;                                                // several regions in this window
+    if (region) {
+        const int8_t r0 = region[tok_pos[T]];
+        bool differ = false;
+        for (int i = threadIdx.x & 63; i < c; i += 64) differ = differ || region[tok_pos[T + i]] != r0;
+        several = __any(differ) ? 0x80000000u : 0u;
+    }
+    for (int i = threadIdx.x & 63; i < c; i += 64) {
+        const int p = tok_pos[T + i];
+        word[T + i] = (uint32_t)code[p] * 4u | (region ? ((uint32_t)(uint8_t)region[p]) << 15 : 0u) | ((uint32_t)T & 0xffu) << 23 | several;
+        if (tok_sq) tok_sq[T + i] = sq;
+    }
+}
+
+// Block of work: own ranks [a, a + len), the ranks [from, to) of the windows they belong to
+struct Block {
+    int a, len, from, to;
+    bool merged;               // several windows
+};
+
+// The blocks that start in the 32 ranks of a chunk, one after the other.  Lane l holds what is known of rank r0 + l (a block
+// may reach 31 ranks past its chunk); all of it is requested together, before the bias table is waited for.
+struct Blocks {
+    int r0, T, c, voxel;
+    uint32_t word, starts;
+    __device__ __forceinline__ Blocks(const Args& g, int64_t chunk) {
+        r0 = (int)(chunk * 32);
+        const int r = r0 + (int)(threadIdx.x & 63), at = (int)(r < g.N ? r : g.N - 1);
+        T = g.tok_T[at];
+        c = g.tok_c[at];
+        voxel = g.order[at];
+        word = g.word[at];
+    }
+    __device__ __forceinline__ void begin(const Args& g) {
+        const int lane = threadIdx.x & 63, r = r0 + lane;
+        starts = (uint32_t)__ballot(lane < 32 && r < g.N && ((r - T) & 31) == 0);
+    }
+    // of the block's own token s * 16 + l % 16 (the last one again behind it)
+    __device__ __forceinline__ int slot(const Block& b, int s) const { return b.a - r0 + min(s * 16 + (int)(threadIdx.x & 15), b.len - 1); }
+    __device__ __forceinline__ bool next(Block& b) {
+        if (!starts) return false;
+        int j = __builtin_ctz(starts);
+        starts &= starts - 1;
+        const int T0 = __builtin_amdgcn_readlane(T, j), c0 = __builtin_amdgcn_readlane(c, j);
+        b.a = r0 + j;
+        b.from = T0;
+        b.to = T0 + c0;
+        b.merged = false;
+        if (c0 >= 32) {
+            b.len = min(32, b.to - b.a);
+            return true;
+        }
+        // small windows that follow each other share a block as long as they fit
+        while (starts) {
+            j = __builtin_ctz(starts);
+            const int cn = __builtin_amdgcn_readlane(c, j);
+            if (cn >= 32 || b.to - b.a + cn > 32) break;
+            starts &= starts - 1;
+            b.to += cn;
+            b.merged = true;
+        }
+        b.len = b.to - b.a;
+        return true;
+    }
+};
+
+__device__ __forceinline__ float across(float v, bool maximum) {         // over the four lanes that hold a column
+    float o = __shfl_xor(v, 16, 64);
+    v = maximum ? fmaxf(v, o) : v + o;
+    o = __shfl_xor(v, 32, 64);
+    return maximum ? fmaxf(v, o) : v + o;
+}
+
+// Workgroup -> head and first chunk: the heads of the same tokens follow each other on one XCD, whose L2 holds their rows
+__device__ __forceinline__ void place(int H, int64_t groups, int& h, int64_t& first) {
+    const int64_t b = blockIdx.x, full = groups / 8 * 8 * H;
+    if (b < full) {
+        const int64_t i = b / 8;
+        h = (int)(i % H);
+        first = (i / H * 8 + b % 8) * WAVES;
+    } else {
+        const int64_t i = b - full, rest = groups % 8;
+        h = (int)(i / rest);
+        first = (groups / 8 * 8 + i % rest) * WAVES;
+    }
+}
+
+template <typename T, int HD> struct Rows {
+    static constexpr int NB = HD / 16;
+    const T* base;
+    uint32_t pitch, col;       // values; col: of this lane's first value in a row operand
+    __device__ __forceinline__ Rows(const void* p, int64_t pitch_, int64_t col0) : base(static_cast<const T*>(p) + col0), pitch((uint32_t)pitch_) {
+        col = ((threadIdx.x & 63) >> 4) * 4;
+    }
+    // row operand of token voxel v: lane (row, slots 4 (l / 16) + j)
+    __device__ __forceinline__ void row(uint32_t v, Frag<T> (&f)[NB]) const {
+#pragma unroll
+        for (int b = 0; b < NB; ++b) f[b].load(base + (__umul24(v, pitch) + col + b * 16));
+    }
+    // column operand: lane (channel 16 b + l % 16, slots = the tokens 4 (l / 16) + j with voxels v[j])
+    __device__ __forceinline__ void column(const int (&v)[4], const Frag<T> (&rows)[NB], Frag<T> (&f)[NB]) const {
+        if constexpr (sizeof(T) == 4) {
+#pragma unroll
+            for (int b = 0; b < NB; ++b)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) f[b].v[j] = base[__umul24((uint32_t)v[j], pitch) + b * 16 + (threadIdx.x & 15)];
+        } else {
+            // the row operand turned on the matrix core: a product with the identity, exact for 16-bit values
+            f32x4 one;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) one[j] = (int)(((threadIdx.x & 63) >> 4) * 4 + j) == (int)(threadIdx.x & 15) ? 1.f : 0.f;
+            const Frag<T> id = packed<T>(one);
+#pragma unroll
+            for (int b = 0; b < NB; ++b) f[b] = packed<T>(mma(rows[b], id, f32x4{0.f, 0.f, 0.f, 0.f}));
+        }
+    }
+};
+
+template <typename T> __device__ __forceinline__ void store4(T* p, const f32x4& v);
+template <> __device__ __forceinline__ void store4<float>(float* p, const f32x4& v) { *reinterpret_cast<f32x4*>(p) = v; }
+template <> __device__ __forceinline__ void store4<__half>(__half* p, const f32x4& v) { *reinterpret_cast<f16x4*>(p) = packed<__half>(v).v; }
+template <> __device__ __forceinline__ void store4<__hip_bfloat16>(__hip_bfloat16* p, const f32x4& v) {
+    *reinterpret_cast<s16x4*>(p) = packed<__hip_bfloat16>(v).v;
+}
+
+typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint32_t u32x4_any __attribute__((ext_vector_type(4), aligned(4)));
+
+// What a step of 16 tokens needs before their rows can be read: the voxel of this lane's row, and the voxels and words of the
+// four tokens in this lane's reduction slots.  Requested a step ahead.  Full steps (all but a window's last) read 16 bytes.
+template <typename T> struct Step {
+    int row;
+    int v[4];
+    uint32_t w[4];
+    __device__ __forceinline__ void load(const Args& g, int r0, int to) {
+        const int l16 = threadIdx.x & 15, quad = (threadIdx.x & 63) >> 4, last = to - 1 - r0;
+        row = g.order[r0 + min(l16, last)];
+        if (last >= 15) {
+            const u32x4_any x = *reinterpret_cast<const u32x4_any*>(g.word + r0 + quad * 4);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) w[j] = x[j];
+            if (sizeof(T) == 4) {
+                const u32x4_any y = *reinterpret_cast<const u32x4_any*>(g.order + r0 + quad * 4);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) v[j] = (int)y[j];
+            }
+        } else {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int r = r0 + min(quad * 4 + j, last);
+                w[j] = g.word[r];
+                if (sizeof(T) == 4) v[j] = g.order[r];
+            }
+        }
+    }
+};
+
+// the head's bias table, in units of log 2
+__device__ __forceinline__ void stage_table(const Args& g, int h, float* table) {
+    for (int i = threadIdx.x; i < g.rows; i += WAVES * 64) table[i] = g.table[(int64_t)i * g.H + h] * LOG2E;
+    __syncthreads();
+}
+
+// A score in units of log 2, less what the accumulator started from: product + bias, and where a window has several mask
+// regions the mask; other windows of a merged block do not take part.
+template <bool FAST>
+__device__ __forceinline__ float score(float acc, float scale2, uint32_t pq, uint32_t pk, const float* table) {
+    const uint32_t d = pq - pk;
+    float x = fmaf(acc, scale2, *reinterpret_cast<const float*>(reinterpret_cast<const char*>(table) + (d & 0x7ffcu)));
+    if (!FAST && d >> 15) x = (pq ^ pk) >> 23 ? -INFINITY : x + MASKED;
+    return x;
+}
+
+// ------------------------------------------------------------------------------------------
+// forward: own = queries
+// ------------------------------------------------------------------------------------------
+template <typename T, int HD>
+__global__ __launch_bounds__(WAVES * 64) void flash_forward_kernel(Args g, int64_t groups) {
+    constexpr int NB = HD / 16;
+    extern __shared__ float table[];
+    int h;
+    int64_t first;
+    place(g.H, groups, h, first);
+    const int lane = threadIdx.x & 63, l16 = lane & 15, quad = lane >> 4;
+    const int64_t chunk = first + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    Blocks blocks(g, chunk * 32 < g.N ? chunk : 0);
+    stage_table(g, h, table);
+    if (chunk * 32 >= g.N) return;
+    blocks.begin(g);
+    const int64_t D = (int64_t)g.H * HD;
+    const Rows<T, HD> q_rows(g.qkv, 3 * D, h * HD), k_rows(g.qkv, 3 * D, D + h * HD), v_rows(g.qkv, 3 * D, 2 * D + h * HD);
+    const float scale2 = g.scale * LOG2E, unscale = 1.f / scale2;
+    Block b;
+    while (blocks.next(b)) {
+        const int subs = (b.len + 15) >> 4;
+        Frag<T> q[2][NB];
+        uint32_t pq[2];
+        int vq[2];
+        float offset[2] = {0.f, 0.f}, sum[2] = {0.f, 0.f}, top[2] = {-INFINITY, -INFINITY};
+        f32x4 o[2][NB];
+        Step<T> ahead;
+        ahead.load(g, b.from, b.to);
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            vq[s] = __shfl(blocks.voxel, blocks.slot(b, s), 64);
+            pq[s] = __shfl(blocks.word, blocks.slot(b, s), 64) + (uint32_t)g.offset4;
+#pragma unroll
+            for (int c = 0; c < NB; ++c) o[s][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+        const bool general = b.merged || __builtin_amdgcn_readfirstlane(pq[0]) >> 31;   // not one window of one mask region
+#pragma unroll
+        for (int s = 0; s < 2; ++s) q_rows.row((uint32_t)vq[s], q[s]);
+        Frag<T> k_next[NB], v_next[NB];                                  // rows a step ahead, voxels and words two
+        uint32_t w_next[4];
+        auto request = [&]() {
+            k_rows.row((uint32_t)ahead.row, k_next);
+            if (sizeof(T) == 4) v_rows.column(ahead.v, v_next, v_next);
+            else v_rows.row((uint32_t)ahead.row, v_next);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) w_next[j] = ahead.w[j];
+        };
+        request();
+        if (b.to - b.from > 16) ahead.load(g, b.from + 16, b.to);
+        for (int k0 = b.from; k0 < b.to; k0 += 16) {
+            const int last = b.to - 1 - k0;
+            Frag<T> k[NB], v[NB], vt[NB];
+            uint32_t pk[4];
+#pragma unroll
+            for (int c = 0; c < NB; ++c) k[c] = k_next[c], v[c] = v_next[c];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) pk[j] = w_next[j];
+            if (last >= 16) request();
+            if (last >= 32) ahead.load(g, k0 + 32, b.to);
+            if (sizeof(T) == 4) {
+#pragma unroll
+                for (int c = 0; c < NB; ++c) vt[c] = v[c];
+            } else {
+                const int none[4] = {0, 0, 0, 0};
+                v_rows.column(none, v, vt);
+            }
+            auto tile = [&](auto fast_tag) {
+                constexpr bool FAST = decltype(fast_tag)::value;
+#pragma unroll
+                for (int s = 0; s < 2; ++s) {
+                    if (s >= subs) break;
+                    const float from = -offset[s] * unscale;             // the accumulator starts at minus the offset
+                    f32x4 acc = {from, from, from, from};
+#pragma unroll
+                    for (int c = 0; c < NB; ++c) acc = mma(k[c], q[s][c], acc);
+                    float x[4];
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        x[j] = score<FAST>(acc[j], scale2, pq[s], pk[j], table);
+                        if (!FAST && quad * 4 + j > last) x[j] = -INFINITY;
+                    }
+                    const float xm = fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3])), before = top[s];
+                    top[s] = fmaxf(before, xm);
+                    if (!FAST || k0 == b.from || __any(xm > 10.f)) {     // the first tokens; later only by chance
+                        const float m = across(xm, true);
+                        const bool fresh = across(before, true) == -INFINITY;
+                        const float by = m == -INFINITY ? 0.f : fresh ? m : fmaxf(0.f, m), f = fresh ? 0.f : __builtin_amdgcn_exp2f(-by);
+                        offset[s] += by;
+                        top[s] -= by;
+                        sum[s] *= f;
+#pragma unroll
+                        for (int c = 0; c < NB; ++c) o[s][c] *= f;
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) x[j] -= by;
+                    }
+                    f32x4 p;
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) p[j] = __builtin_amdgcn_exp2f(x[j]);
+                    sum[s] += (p[0] + p[1]) + (p[2] + p[3]);
+                    const Frag<T> pt = packed<T>(p);
+#pragma unroll
+                    for (int c = 0; c < NB; ++c) o[s][c] = mma(vt[c], pt, o[s][c]);
+                }
+            };
+            if (last >= 15 && !general) tile(std::true_type{});
+            else tile(std::false_type{});
+        }
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            if (s >= subs) break;
+            // top: the row's maximum less the offset
+            const float z = across(sum[s], false) + 1e-8f * __builtin_amdgcn_exp2f(fmaxf(across(top[s], true), -offset[s]));
+            const float inv = 1.f / z;
+            if (s * 16 + l16 < b.len) {
+                T* row = static_cast<T*>(g.out) + (int64_t)vq[s] * D + h * HD + quad * 4;
+#pragma unroll
+                for (int c = 0; c < NB; ++c) store4<T>(row + c * 16, o[s][c] * inv);
+                if (quad == 0) g.lse[h * g.N + b.a + s * 16 + l16] = offset[s] + __builtin_amdgcn_logf(z);
+            }
+        }
+    }
+}
+
+// ------------------------------------------------------------------------------------------
+// backward, own = queries: D = dO . O, dQ = scale dS K, dS stored for the bias gradient
+// ------------------------------------------------------------------------------------------
+template <typename T, int HD>
+__global__ __launch_bounds__(WAVES * 64) void flash_backward_q_kernel(Args g, int64_t groups) {
+    constexpr int NB = HD / 16;
+    extern __shared__ float table[];
+    int h;
+    int64_t first;
+    place(g.H, groups, h, first);
+    const int lane = threadIdx.x & 63, l16 = lane & 15, quad = lane >> 4;
+    const int64_t chunk = first + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    Blocks blocks(g, chunk * 32 < g.N ? chunk : 0);
+    stage_table(g, h, table);
+    if (chunk * 32 >= g.N) return;
+    blocks.begin(g);
+    const int64_t D = (int64_t)g.H * HD;
+    const Rows<T, HD> q_rows(g.qkv, 3 * D, h * HD), k_rows(g.qkv, 3 * D, D + h * HD), v_rows(g.qkv, 3 * D, 2 * D + h * HD);
+    const Rows<T, HD> do_rows(g.dout, D, h * HD), o_rows(g.out, D, h * HD);
+    const float scale2 = g.scale * LOG2E, unscale = 1.f / scale2;
+    Block b;
+    while (blocks.next(b)) {
+        const int subs = (b.len + 15) >> 4;
+        Frag<T> q[2][NB], d_o[2][NB];
+        uint32_t pq[2];
+        int vq[2];
+        int64_t at[2];         // first value of the query's row of dS, less its window's first rank
+        float lse[2], delta[2];
+        f32x4 dq[2][NB];
+        Step<T> ahead;
+        ahead.load(g, b.from, b.to);
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            const int r = b.a + min(s * 16 + l16, b.len - 1);
+            vq[s] = __shfl(blocks.voxel, blocks.slot(b, s), 64);
+            pq[s] = __shfl(blocks.word, blocks.slot(b, s), 64) + (uint32_t)g.offset4;
+            lse[s] = g.lse[h * g.N + r];
+            if (g.ds) {
+                const int c = __shfl(blocks.c, blocks.slot(b, s), 64), T0 = __shfl(blocks.T, blocks.slot(b, s), 64);
+                at[s] = (int64_t)g.tok_sq[r] * g.H + (int64_t)h * c * c + (int64_t)(r - T0) * c - T0;
+            }
+        }
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            Frag<T> o[NB];
+            q_rows.row((uint32_t)vq[s], q[s]);
+            do_rows.row((uint32_t)vq[s], d_o[s]);
+            o_rows.row((uint32_t)vq[s], o);
+            float dot = 0.f;
+#pragma unroll
+            for (int c = 0; c < NB; ++c) {
+                dq[s][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+                const T* x = reinterpret_cast<const T*>(&d_o[s][c].v);
+                const T* y = reinterpret_cast<const T*>(&o[c].v);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) dot = fmaf(to_acc(x[j]), to_acc(y[j]), dot);
+            }
+            delta[s] = across(dot, false);
+            if (quad == 0 && s * 16 + l16 < b.len) g.delta[h * g.N + b.a + s * 16 + l16] = delta[s];
+        }
+        const bool general = b.merged || __builtin_amdgcn_readfirstlane(pq[0]) >> 31;   // not one window of one mask region
+        for (int k0 = b.from; k0 < b.to; k0 += 16) {
+            const int last = b.to - 1 - k0;
+            const Step<T> step = ahead;
+            Frag<T> k[NB], v[NB], kt[NB];
+            k_rows.row((uint32_t)step.row, k);
+            v_rows.row((uint32_t)step.row, v);
+            k_rows.column(step.v, k, kt);
+            if (last >= 16) ahead.load(g, k0 + 16, b.to);
+            auto tile = [&](auto fast_tag) {
+                constexpr bool FAST = decltype(fast_tag)::value;
+#pragma unroll
+                for (int s = 0; s < 2; ++s) {
+                    if (s >= subs) break;
+                    // the accumulators start at minus the row's log-sum-exp and minus its dO . O
+                    const float a0 = -lse[s] * unscale, d0 = -delta[s];
+                    f32x4 acc = {a0, a0, a0, a0}, dp = {d0, d0, d0, d0}, ds;
+#pragma unroll
+                    for (int c = 0; c < NB; ++c) acc = mma(k[c], q[s][c], acc), dp = mma(v[c], d_o[s][c], dp);
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        float x = score<FAST>(acc[j], scale2, pq[s], step.w[j], table);
+                        if (!FAST && quad * 4 + j > last) x = -INFINITY;
+                        ds[j] = __builtin_amdgcn_exp2f(x) * dp[j];
+                    }
+                    if (g.ds && s * 16 + l16 < b.len) {                  // four neighbours of a row of dS per lane
+                        float* row = g.ds + at[s] + k0 + quad * 4;
+                        if (FAST || (last >= 15 && !b.merged)) {
+                            *reinterpret_cast<f32x4_any*>(row) = ds;
+                        } else {
+#pragma unroll
+                            for (int j = 0; j < 4; ++j)
+                                if (quad * 4 + j <= last && !((pq[s] ^ step.w[j]) >> 23)) row[j] = ds[j];
+                        }
+                    }
+                    const Frag<T> dst = packed<T>(ds);
+#pragma unroll
+                    for (int c = 0; c < NB; ++c) dq[s][c] = mma(kt[c], dst, dq[s][c]);
+                }
+            };
+            if (last >= 15 && !general) tile(std::true_type{});
+            else tile(std::false_type{});
+        }
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            if (s * 16 + l16 < b.len) {
+                T* row = static_cast<T*>(g.dqkv) + (int64_t)vq[s] * 3 * D + h * HD + quad * 4;
+#pragma unroll
+                for (int c = 0; c < NB; ++c) store4<T>(row + c * 16, dq[s][c] * g.scale);
+            }
+        }
+    }
+}
+
+// ------------------------------------------------------------------------------------------
+// backward, own = keys: dV = P^T dO, dK = scale dS^T Q
+// ------------------------------------------------------------------------------------------
+template <typename T, int HD>
+__global__ __launch_bounds__(WAVES * 64) void flash_backward_kv_kernel(Args g, int64_t groups) {
+    constexpr int NB = HD / 16;
+    extern __shared__ float table[];
+    int h;
+    int64_t first;
+    place(g.H, groups, h, first);
+    const int lane = threadIdx.x & 63, l16 = lane & 15, quad = lane >> 4;
+    const int64_t chunk = first + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    Blocks blocks(g, chunk * 32 < g.N ? chunk : 0);
+    stage_table(g, h, table);
+    if (chunk * 32 >= g.N) return;
+    blocks.begin(g);
+    const int64_t D = (int64_t)g.H * HD;
+    const Rows<T, HD> q_rows(g.qkv, 3 * D, h * HD), k_rows(g.qkv, 3 * D, D + h * HD), v_rows(g.qkv, 3 * D, 2 * D + h * HD);
+    const Rows<T, HD> do_rows(g.dout, D, h * HD);
+    const float scale2 = g.scale * LOG2E, unscale = 1.f / scale2;
+    Block b;
+    while (blocks.next(b)) {
+        const int subs = (b.len + 15) >> 4;
+        Frag<T> k[2][NB], v[2][NB];
+        uint32_t pk[2];
+        int vk[2];
+        f32x4 dk[2][NB], dv[2][NB];
+        Step<T> ahead;
+        ahead.load(g, b.from, b.to);
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            vk[s] = __shfl(blocks.voxel, blocks.slot(b, s), 64);
+            pk[s] = __shfl(blocks.word, blocks.slot(b, s), 64);
+        }
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            k_rows.row((uint32_t)vk[s], k[s]);
+            v_rows.row((uint32_t)vk[s], v[s]);
+#pragma unroll
+            for (int c = 0; c < NB; ++c) dk[s][c] = dv[s][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+        const bool general = b.merged || __builtin_amdgcn_readfirstlane(pk[0]) >> 31;
+        for (int q0 = b.from; q0 < b.to; q0 += 16) {
+            const int last = b.to - 1 - q0;
+            const Step<T> step = ahead;
+            f32x4 lse, delta;
+            if (last >= 15) {
+                lse = *reinterpret_cast<const f32x4_any*>(g.lse + h * g.N + q0 + quad * 4);
+                delta = *reinterpret_cast<const f32x4_any*>(g.delta + h * g.N + q0 + quad * 4);
+            } else {
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const int64_t r = h * g.N + q0 + min(quad * 4 + j, last);
+                    lse[j] = quad * 4 + j <= last ? g.lse[r] : INFINITY;   // rows past the end: P = 0
+                    delta[j] = g.delta[r];
+                }
+            }
+            Frag<T> q[NB], d_o[NB], qt[NB], dot[NB];
+            q_rows.row((uint32_t)step.row, q);
+            do_rows.row((uint32_t)step.row, d_o);
+            q_rows.column(step.v, q, qt);
+            do_rows.column(step.v, d_o, dot);
+            if (last >= 16) ahead.load(g, q0 + 16, b.to);
+            const f32x4 a0 = lse * -unscale, d0 = -delta;               // what the accumulators start from
+            auto tile = [&](auto fast_tag) {
+                constexpr bool FAST = decltype(fast_tag)::value;
+#pragma unroll
+                for (int s = 0; s < 2; ++s) {
+                    if (s >= subs) break;
+                    f32x4 acc = a0, dp = d0, p, ds;
+#pragma unroll
+                    for (int c = 0; c < NB; ++c) acc = mma(q[c], k[s][c], acc), dp = mma(d_o[c], v[s][c], dp);
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        p[j] = __builtin_amdgcn_exp2f(score<FAST>(acc[j], scale2, step.w[j] + (uint32_t)g.offset4, pk[s], table));
+                        ds[j] = p[j] * dp[j];
+                    }
+                    const Frag<T> pf = packed<T>(p), df = packed<T>(ds);
+#pragma unroll
+                    for (int c = 0; c < NB; ++c) dv[s][c] = mma(dot[c], pf, dv[s][c]), dk[s][c] = mma(qt[c], df, dk[s][c]);
+                }
+            };
+            if (last >= 15 && !general) tile(std::true_type{});
+            else tile(std::false_type{});
+        }
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            if (s * 16 + l16 < b.len) {
+                T* row = static_cast<T*>(g.dqkv) + (int64_t)vk[s] * 3 * D + h * HD + quad * 4;
+#pragma unroll
+                for (int c = 0; c < NB; ++c) {
+                    store4<T>(row + D + c * 16, dk[s][c] * g.scale);
+                    store4<T>(row + 2 * D + c * 16, dv[s][c]);
+                }
+            }
+        }
+    }
+}
+
+template <typename K> static int launch(K kernel, const Args& g, hipStream_t s, const char* what) {
+    const int64_t groups = (g.N + 32 * WAVES - 1) / (32 * WAVES);
+    SSWIN_CHECK(groups * g.H < (1ll << 31), "%s: too many tokens", what);
+    hipLaunchKernelGGL(kernel, dim3((unsigned)(groups * g.H)), dim3(WAVES * 64), (size_t)g.rows * sizeof(float), s, g, groups);
+    return launch_ok(what);
+}
+
+}  // namespace flash
+}  // namespace sswin
+
+using namespace sswin;
+using namespace sswin::flash;
+
+static int flash_check(const char* what, int dtype, int64_t N, int H, int hd, int n, int rows, int offset0) {
+    SSWIN_CHECK(dtype >= SSWIN_F32 && dtype <= SSWIN_BF16, "%s: value type %d", what, dtype);
+    SSWIN_CHECK(N >= 0 && N < MAX_TOKENS && H > 0 && H < 256, "%s: bad sizes", what);
+    SSWIN_CHECK(hd == 16 || hd == 32, "%s: heads of %d channels (16 or 32 are supported)", what, hd);
+    SSWIN_CHECK(n > 0 && rows > 0 && rows <= MAX_ROWS && offset0 >= 0, "%s: a bias table of at most %d rows", what, MAX_ROWS);
+    SSWIN_CHECK(N * 3 * H * hd < (1ll << 32), "%s: token rows need 32-bit offsets", what);
+    return 0;
+}
+
+extern "C" {
+
+int sswin_flash_supported(int dtype, int64_t N, int H, int hd, int rows) {
+    return dtype >= SSWIN_F32 && dtype <= SSWIN_BF16 && N > 0 && N < MAX_TOKENS && (hd == 16 || hd == 32) && rows > 0 && rows <= MAX_ROWS && H > 0 && H < 256 &&
+           N * 3 * H * hd < (1ll << 32);
+}
+
+int sswin_flash_tokens(const int32_t* plan, int64_t g_cap, int64_t groups, const int32_t* tokens, int64_t N, int H, int n, const int32_t* code,
+                       const int8_t* mask, int nmw, int32_t* word, int32_t* tok_sq, void* stream) {
+    SSWIN_CHECK(N >= 0 && n > 0 && H > 0 && groups >= 0 && groups <= g_cap && groups % H == 0, "flash_tokens: bad sizes");
+    if (N == 0 || groups == 0) return 0;
+    SSWIN_CHECK(plan && tokens && code && word && (!mask || nmw > 0), "flash_tokens: null pointer");
+    const int64_t windows = groups / H;
+    hipLaunchKernelGGL(flash_tokens_kernel, dim3((unsigned)((windows + 3) / 4)), dim3(256), 0, static_cast<hipStream_t>(stream), plan, g_cap, windows, H,
+                       tokens + 3 * N, code, mask, nmw, n, reinterpret_cast<uint32_t*>(word), tok_sq);
+    return launch_ok("flash_tokens");
+}
+
+int sswin_flash_forward(int dtype, const int32_t* tokens, const int32_t* word, int64_t N, int H, int hd, int n, const void* qkv, float scale, const float* table,
+                        int rows, int offset0, void* out, float* lse, void* stream) {
+    if (int rc = flash_check("flash_forward", dtype, N, H, hd, n, rows, offset0)) return rc;
+    if (N == 0) return 0;
+    SSWIN_CHECK(tokens && word && qkv && table && out && lse, "flash_forward: null pointer");
+    SSWIN_CHECK(((uintptr_t)qkv | (uintptr_t)out) % 16 == 0, "flash_forward: pointers must be 16-byte aligned");
+    Args g = {};
+    g.order = tokens, g.tok_T = tokens + N, g.tok_c = tokens + 2 * N, g.word = reinterpret_cast<const uint32_t*>(word);
+    g.N = N, g.H = H, g.rows = rows, g.offset4 = offset0 * 4, g.scale = scale, g.table = table, g.qkv = qkv, g.out = out, g.lse = lse;
+    hipStream_t s = static_cast<hipStream_t>(stream);
+#define FLASH(K, T) (hd == 16 ? launch(K<T, 16>, g, s, #K) : launch(K<T, 32>, g, s, #K))
+    if (dtype == SSWIN_F32) return FLASH(flash_forward_kernel, float);
+    if (dtype == SSWIN_F16) return FLASH(flash_forward_kernel, __half);
+    return FLASH(flash_forward_kernel, __hip_bfloat16);
+}
+
+int sswin_flash_backward(int dtype, const int32_t* tokens, const int32_t* word, const int32_t* tok_sq, int64_t N, int H, int hd, int n, const void* qkv, float scale,
+                         const float* table, int rows, int offset0, const void* out, const float* lse, const void* dout, void* dqkv, float* delta, float* ds,
+                         void* stream) {
+    if (int rc = flash_check("flash_backward", dtype, N, H, hd, n, rows, offset0)) return rc;
+    if (N == 0) return 0;
+    SSWIN_CHECK(tokens && word && qkv && table && out && lse && dout && dqkv && delta && (!ds || tok_sq), "flash_backward: null pointer");
+    SSWIN_CHECK(((uintptr_t)qkv | (uintptr_t)out | (uintptr_t)dout | (uintptr_t)dqkv) % 16 == 0, "flash_backward: pointers must be 16-byte aligned");
+    Args g = {};
+    g.order = tokens, g.tok_T = tokens + N, g.tok_c = tokens + 2 * N, g.word = reinterpret_cast<const uint32_t*>(word);
+    g.N = N, g.H = H, g.rows = rows, g.offset4 = offset0 * 4, g.scale = scale, g.table = table, g.qkv = qkv, g.out = const_cast<void*>(out);
+    g.lse = const_cast<float*>(lse), g.dout = dout, g.delta = delta, g.dqkv = dqkv, g.ds = ds, g.tok_sq = tok_sq;
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    int rc;
+    if (dtype == SSWIN_F32) rc = FLASH(flash_backward_q_kernel, float);
+    else if (dtype == SSWIN_F16) rc = FLASH(flash_backward_q_kernel, __half);
+    else rc = FLASH(flash_backward_q_kernel, __hip_bfloat16);
+    if (rc) return rc;
+    if (dtype == SSWIN_F32) return FLASH(flash_backward_kv_kernel, float);
+    if (dtype == SSWIN_F16) return FLASH(flash_backward_kv_kernel, __half);
+    return FLASH(flash_backward_kv_kernel, __hip_bfloat16);
+#undef FLASH
+}
+
+}  // extern "C"

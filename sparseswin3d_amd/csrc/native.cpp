@@ -310,24 +310,39 @@ struct Attention : torch::CustomClassHolder {
     Tensor code;            // int32 position codes of the bias table, or undefined: the bias is [H, n, n]
     int offset0 = 0, n = 0, H = 0;
     double scale = 1.0;
-    bool resident = false;
+    bool resident = false;  // the window-resident kernels (heads of 32, windows of at most 128 positions)
+    bool flash = false;     // the kernels for heads of 16 or 32 and windows of any size
 
     int regions() const { return mask.defined() ? (int)mask.size(0) : 0; }
 };
 using AttentionPtr = c10::intrusive_ptr<Attention>;
 
 struct AttentionSaved {
-    Tensor bias32, aux;     // aux: log-sum-exp of every attention row (resident), or P
+    Tensor bias32, aux;     // bias or table; log-sum-exp of every attention row, or P
+    Tensor words;           // flash: int32 [2, N] token words and window offsets
 };
 
-Tensor attention_forward(const Attention& a, const Tensor& qkv, const Tensor& bias, AttentionSaved& saved) {
+Tensor attention_forward(Attention& a, const Tensor& qkv, const Tensor& bias, AttentionSaved& saved) {
     Plan& tp = *a.plan;
     tp.finish();
+    if (a.flash && !(a.scale > 0 && sswin_flash_supported(code_of(qkv.scalar_type()), qkv.size(0), a.H, (int)(qkv.size(1) / 3 / a.H), (int)bias.size(0))))
+        a.flash = false;                                                 // more tokens than the kernels address: the products
     TORCH_CHECK(!a.resident || tp.oversize == 0, "window-resident attention: ", tp.oversize, " groups hold more than 128 tokens");
     const int64_t N = qkv.size(0), D = qkv.size(1) / 3;
     const int hd = (int)(D / a.H), dt = code_of(qkv.scalar_type());
     void* s = current_stream(qkv);
     const Tensor table32 = bias.to(at::kFloat).contiguous();
+    if (a.flash) {
+        saved.bias32 = table32;
+        saved.words = at::empty({2, N}, tp.tokens.options());
+        saved.aux = at::empty({a.H, N}, table32.options());
+        Tensor o = at::empty({N, D}, qkv.options());
+        RUN(sswin_flash_tokens(i32(tp.plan), tp.g_cap, tp.G, i32(tp.tokens), N, a.H, a.n, i32(a.code), a.mask.defined() ? a.mask.data_ptr<int8_t>() : nullptr,
+                               a.regions(), i32(saved.words), i32(saved.words) + N, s));
+        RUN(sswin_flash_forward(dt, i32(tp.tokens), i32(saved.words), N, a.H, hd, a.n, ptr(qkv), (float)a.scale, f32(table32), (int)table32.size(0), a.offset0,
+                                ptr(o), f32(saved.aux), s));
+        return o;
+    }
     if (a.code.defined()) {
         saved.bias32 = at::empty({a.H, a.n, a.n}, table32.options());
         RUN(sswin_bias_from_table(f32(table32), (int)table32.size(0), a.H, i32(a.code), a.offset0, a.n, f32(saved.bias32), s));
@@ -386,6 +401,13 @@ Tensor attention_backward(const Attention& a, const Tensor& qkv, const Tensor& b
     void* s = current_stream(qkv);
     Tensor d_qkv = at::empty_like(qkv);
     const auto fopt = qkv.options().dtype(at::kFloat);
+    if (a.flash) {
+        Tensor d_s = want_bias ? at::empty({std::max<int64_t>(tp.A, 1)}, fopt) : Tensor(), delta = at::empty({a.H, N}, fopt);
+        RUN(sswin_flash_backward(dt, i32(tp.tokens), i32(saved.words), i32(saved.words) + N, N, a.H, hd, a.n, ptr(qkv), (float)a.scale, f32(saved.bias32),
+                                 (int)saved.bias32.size(0), a.offset0, ptr(out), f32(saved.aux), ptr(d_out), ptr(d_qkv), f32(delta), f32(d_s), s));
+        if (want_bias) d_bias = bias_gradient(a, d_s, bias);
+        return d_qkv;
+    }
     if (a.resident) {
         const int8_t* mask = a.mask.defined() ? a.mask.data_ptr<int8_t>() : nullptr;
         Tensor d_s = want_bias ? at::empty({std::max<int64_t>(tp.A, 1)}, fopt) : Tensor();
@@ -447,12 +469,12 @@ bool wants_grad(std::initializer_list<const Tensor*> ts) {
 struct AttentionNode : torch::autograd::Function<AttentionNode> {
     static Tensor forward(AutogradContext* ctx, const Tensor& qkv, const Tensor& bias, AttentionPtr a) {
         NoAutocast off;
-        const Tensor x = qkv.contiguous();
+        const Tensor x = ready(qkv);
         const Tensor flat = x.view({x.size(0), -1});
         AttentionSaved saved;
         Tensor out = attention_forward(*a, flat, bias, saved);
         if (ctx) {
-            ctx->save_for_backward({flat, bias, saved.bias32, saved.aux, out});
+            ctx->save_for_backward({flat, bias, saved.bias32, saved.aux, out, saved.words});
             ctx->saved_data["a"] = capsule(a);
             ctx->saved_data["shape"] = qkv.sizes();
             ctx->saved_data["bias"] = bias.requires_grad();
@@ -466,7 +488,7 @@ struct AttentionNode : torch::autograd::Function<AttentionNode> {
         c10::hip::HIPGuardMasqueradingAsCUDA guard(v[0].device());
         Tensor d_bias;
         const Tensor d_out = ready(grads[0].to(v[0].scalar_type()));
-        Tensor d = attention_backward(*a, v[0], v[1], AttentionSaved{v[2], v[3]}, v[4], d_out, ctx->saved_data["bias"].toBool(), d_bias);
+        Tensor d = attention_backward(*a, v[0], v[1], AttentionSaved{v[2], v[3], v[5]}, v[4], d_out, ctx->saved_data["bias"].toBool(), d_bias);
         return once({d.view(ctx->saved_data["shape"].toIntVector()), d_bias, Tensor()});
     }
 };
@@ -483,7 +505,7 @@ struct ModuleNode : torch::autograd::Function<ModuleNode> {
         Tensor o = attention_forward(*a, qkv, bias, saved);
         Tensor y = dense(o, proj_w, proj_b);
         if (ctx) {
-            ctx->save_for_backward({x, qkv_w, bias, proj_w, qkv, saved.bias32, saved.aux, o});
+            ctx->save_for_backward({x, qkv_w, bias, proj_w, qkv, saved.bias32, saved.aux, o, saved.words});
             ctx->saved_data["a"] = capsule(a);
             ctx->saved_data["how"] = std::vector<int64_t>{(int64_t)x_in.scalar_type(), x_in.requires_grad(), qkv_w.requires_grad(), asks(qkv_b),
                                                           bias.requires_grad(), proj_w.requires_grad(), asks(proj_b)};
@@ -502,7 +524,7 @@ struct ModuleNode : torch::autograd::Function<ModuleNode> {
         if (how[5] || how[6]) d_proj = dense_dw(dy, o, how[6], proj_w.scalar_type());
         Tensor d_bias, dx;
         const Tensor d_o = dense_dx(dy, proj_w);
-        const Tensor d_qkv = attention_backward(*a, qkv, bias, AttentionSaved{v[5], v[6]}, o, d_o, how[4], d_bias);
+        const Tensor d_qkv = attention_backward(*a, qkv, bias, AttentionSaved{v[5], v[6], v[8]}, o, d_o, how[4], d_bias);
         if (how[2] || how[3]) d_qkvw = dense_dw(d_qkv, x, how[3], qkv_w.scalar_type());
         if (how[1]) dx = dense_dx(d_qkv, qkv_w).to((ScalarType)how[0]);
         return once({dx, d_qkvw.first, d_qkvw.second, d_bias, d_proj.first, d_proj.second, Tensor(), Tensor()});
@@ -531,7 +553,7 @@ struct BlockNode : torch::autograd::Function<BlockNode> {
         Tensor y = dense(g, p[W2], p[C2], SSWIN_DENSE_RESIDUAL, h, nullptr, stream_type);
         if (ctx) {
             ctx->save_for_backward({x, p[G1], p[QKVW], p[TABLE], p[PROJW], p[G2], p[W1], p[W2], stats1, x1, qkv, saved.bias32, saved.aux, o, h, stats2, x2, g,
-                                    slope});
+                                    slope, saved.words});
             ctx->saved_data["a"] = capsule(a);
             ctx->saved_data["which"] = which;
             std::vector<int64_t> asked;
@@ -563,7 +585,7 @@ struct BlockNode : torch::autograd::Function<BlockNode> {
         const Tensor dht = dh.to(type);
         keep(PROJW, dht, o);
         const Tensor d_o = dense_dx(dht, projw);
-        const Tensor d_qkv = attention_backward(*a, qkv, table, AttentionSaved{v[11], v[12]}, o, d_o, ask[TABLE], out[TABLE]);
+        const Tensor d_qkv = attention_backward(*a, qkv, table, AttentionSaved{v[11], v[12], v[19]}, o, d_o, ask[TABLE], out[TABLE]);
         keep(QKVW, d_qkv, x1);
         out[X] = norm_backward(dense_dx(d_qkv, qkvw), x, stats1, g1, dh, out[G1], out[B1]);
         variable_list result;
@@ -612,36 +634,40 @@ struct MergeNode : torch::autograd::Function<MergeNode> {
 // ------------------------------------------------------------------------------------------
 // Python entry points
 // ------------------------------------------------------------------------------------------
+// path: "resident", "flash" or "products" (the attention matrix in memory)
 AttentionPtr make_attention(const PlanPtr& plan, const OptTensor& mask, const OptTensor& code, int64_t offset0, int64_t n, int64_t heads, double scale,
-                            bool resident) {
+                            const std::string& path) {
     auto a = c10::make_intrusive<Attention>();
     a->plan = plan;
     if (mask) a->mask = mask->to(at::kChar).contiguous();
     if (code) a->code = *code;
-    a->offset0 = (int)offset0, a->n = (int)n, a->H = (int)heads, a->scale = scale, a->resident = resident;
+    a->offset0 = (int)offset0, a->n = (int)n, a->H = (int)heads, a->scale = scale;
+    a->resident = path == "resident", a->flash = path == "flash";
+    TORCH_CHECK(a->resident || a->flash || path == "products", "attention path ", path);
+    TORCH_CHECK(!a->flash || code, "the flash path takes its bias from a relative position table");
     return a;
 }
 
 Tensor attention(const Tensor& qkv, const Tensor& bias, const PlanPtr& plan, const OptTensor& mask, const OptTensor& code, int64_t offset0, int64_t n,
-                 double scale, bool resident) {
+                 double scale, const std::string& path) {
     c10::hip::HIPGuardMasqueradingAsCUDA guard(qkv.device());
-    auto a = make_attention(plan, mask, code, offset0, n, qkv.size(2), scale, resident);
+    auto a = make_attention(plan, mask, code, offset0, n, qkv.size(2), scale, path);
     if (!wants_grad({&qkv, &bias})) return AttentionNode::forward(nullptr, qkv, bias, a);
     return AttentionNode::apply(qkv, bias, a);
 }
 
 Tensor attention_module(const Tensor& x, const Tensor& qkv_w, const OptTensor& qkv_b, const Tensor& bias, const Tensor& proj_w, const OptTensor& proj_b,
                         const PlanPtr& plan, const OptTensor& mask, const OptTensor& code, int64_t offset0, int64_t n, int64_t heads, double scale,
-                        bool resident, ScalarType type) {
+                        const std::string& path, ScalarType type) {
     c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
-    auto a = make_attention(plan, mask, code, offset0, n, heads, scale, resident);
+    auto a = make_attention(plan, mask, code, offset0, n, heads, scale, path);
     const Tensor qb = or_undefined(qkv_b), pb = or_undefined(proj_b);
     if (!wants_grad({&x, &qkv_w, &qb, &bias, &proj_w, &pb})) return ModuleNode::forward(nullptr, x, qkv_w, qkv_b, bias, proj_w, proj_b, a, type);
     return ModuleNode::apply(x, qkv_w, qkv_b, bias, proj_w, proj_b, a, type);
 }
 
 Tensor block(std::vector<OptTensor> params, const PlanPtr& plan, const OptTensor& mask, const Tensor& code, int64_t offset0, int64_t n, int64_t heads,
-             double scale, bool resident, double eps1, double eps2, ScalarType type) {
+             double scale, const std::string& path, double eps1, double eps2, ScalarType type) {
     TORCH_CHECK(params.size() == BlockNode::PARAMS, "block: ", (int)BlockNode::PARAMS, " tensors expected");
     variable_list given;
     std::vector<int64_t> which;
@@ -653,7 +679,7 @@ Tensor block(std::vector<OptTensor> params, const PlanPtr& plan, const OptTensor
             which.push_back((int64_t)i);
         }
     c10::hip::HIPGuardMasqueradingAsCUDA guard(given.at(0).device());
-    auto a = make_attention(plan, mask, code, offset0, n, heads, scale, resident);
+    auto a = make_attention(plan, mask, code, offset0, n, heads, scale, path);
     if (!grad || !at::GradMode::is_enabled()) return BlockNode::forward(nullptr, given, which, a, eps1, eps2, type);
     return BlockNode::apply(at::TensorList(given), which, a, eps1, eps2, type);
 }

@@ -147,8 +147,9 @@ class BiasTableIndex:
     sparse_swin/swin3d_base.py:630-647).  :meth:`build` returns None if an index is not of
     that form or the table is too large for the table-gradient kernel."""
 
-    def __init__(self, flat, code, offset0):
+    def __init__(self, flat, code, offset0, ascending=False):
         self.flat, self.code, self.offset0 = flat, code, offset0
+        self.ascending = ascending          # no negative code: what the kernels that read the table itself take
 
     @staticmethod
     def build(index: torch.Tensor, table_rows: int):
@@ -156,15 +157,13 @@ class BiasTableIndex:
         if index.dim() != 2 or index.shape[1] != n or n > 384 or table_rows > 4096 or n == 0:
             return None
         idx = index.to(torch.int64)
-        code = idx[:, 0]
-        offset0 = int(idx[0, 0]) - 0
-        # index[p, q] = code[p] - code[q] + offset0 with code[0] carrying offset0 out again
-        code = code - int(code[0])
-        if not torch.equal(idx, code[:, None] - code[None, :] + offset0):
+        # index[p, q] = code[p] - code[q] + offset0 with code[0] = 0; every check in one read from the device
+        code = idx[:, 0] - idx[0, 0]
+        linear, low, high, offset0, first = torch.stack([
+            (idx == code[:, None] - code[None, :] + idx[0, 0]).all().to(torch.int64), idx.min(), idx.max(), idx[0, 0], code.min()]).tolist()
+        if not linear or low < 0 or high >= table_rows:
             return None
-        if int(idx.min()) < 0 or int(idx.max()) >= table_rows:
-            return None
-        return BiasTableIndex(idx.reshape(-1).contiguous(), code.to(torch.int32).contiguous(), offset0)
+        return BiasTableIndex(idx.reshape(-1).contiguous(), code.to(torch.int32).contiguous(), offset0, first >= 0)
 
 
 def fused_window_attention(qkv, bias, indices, mask, batch_size, n, scale, resident=None, plan=None,
@@ -172,8 +171,8 @@ def fused_window_attention(qkv, bias, indices, mask, batch_size, n, scale, resid
     """``qkv`` [N,3,H,hd], ``bias`` [H,n,n], ``indices`` int32 [N,2] (window,pos), ``mask`` int8
     [nW,n] or None -> attention output [N, H*hd] in the caller's voxel order.
 
-    ``resident`` selects the window-resident kernels (default: whenever they apply, i.e. heads
-    of 32 channels); otherwise the block products with the attention matrix in HBM are used.
+    ``resident``: None = the kernels that keep the attention matrix in registers wherever they apply (:func:`attention_path`),
+    True = the window-resident ones (heads of 32 channels), False = block products with the attention matrix in HBM.
     ``plan``: a :class:`TokenPlan` of ``indices`` made earlier (possibly still in flight).
     ``table_index``: a :class:`BiasTableIndex`; ``bias`` is then the [rows, H] bias table and its
     gradient is computed without the [H, n, n] detour.
@@ -184,11 +183,22 @@ def fused_window_attention(qkv, bias, indices, mask, batch_size, n, scale, resid
         features, to_qkv, proj, heads, dtype = projections
         tp = plan if plan is not None else TokenPlan(indices, batch_size, n, heads, defer=True)
         return _lib.native().attention_module(features, to_qkv.weight, to_qkv.bias, bias, proj.weight, proj.bias, tp.native, mask, code,
-                                              offset0, n, heads, scale, resident, dtype)
-    if resident is None:
-        resident = supports_resident(qkv, n)
+                                              offset0, n, heads, scale,
+                                              attention_path(features.shape[1] // heads, n, table_index, resident), dtype)
     tp = plan if plan is not None else TokenPlan(indices, batch_size, n, qkv.shape[2], defer=True)
-    return _lib.native().attention(qkv, bias, tp.native, mask, code, offset0, int(n), float(scale), bool(resident))
+    return _lib.native().attention(qkv, bias, tp.native, mask, code, offset0, int(n), float(scale),
+                                   attention_path(qkv.shape[3], n, table_index, resident))
+
+
+def attention_path(head_dim: int, n: int, table_index, resident=None) -> str:
+    """Which kernels run an attention the fused path takes.  "resident": heads of 32 channels, windows of at most 128 positions;
+    "flash": heads of 16 or 32 channels and any window, the bias read from the relative position table; "products": block
+    products with the attention matrix in memory (any head size)."""
+    if resident or (resident is None and head_dim == 32 and n <= 128):
+        return "resident"
+    if resident is None and head_dim in (16, 32) and table_index is not None and table_index.ascending:
+        return "flash"
+    return "products"
 
 
 def supports_resident(qkv: torch.Tensor, n: int) -> bool:

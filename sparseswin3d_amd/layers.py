@@ -20,6 +20,7 @@ from torch.autograd import Function
 from torch.autograd.function import once_differentiable
 
 from . import _lib
+from .fused import attention_path
 from .window_attention import WindowAttentionSparse, _token_plan, prefetch_plans, replace_feature, tall_linear
 
 _DTYPE_CODE = {torch.float32: 0, torch.float16: 1, torch.bfloat16: 2}
@@ -436,13 +437,13 @@ class SwinTransformerBlock(nn.Module):
             attn, mlp, n = self.attn, self.mlp, view.spatial_shape[0]
             how = attn._fused_arguments(x.features, n)
             if how is not None and how[0] is not None:
-                ti, resident, _ = how
+                ti = how[0]
                 plan = _token_plan(attn, view)
                 y = _lib.native().block(
                     [x.features, self.norm1.weight, self.norm1.bias, attn.qkv.weight, attn.qkv.bias, attn.relative_position_bias_table,
                      attn.proj.weight, attn.proj.bias, self.norm2.weight, self.norm2.bias, mlp.linear1.weight, mlp.linear1.bias,
                      mlp.linear2.weight, mlp.linear2.bias], plan.native, mask_matrix if shifted else None, ti.code, ti.offset0, n,
-                    attn.num_heads, attn.scale, resident, self.norm1.eps, self.norm2.eps, dtype)
+                    attn.num_heads, attn.scale, attention_path(attn.dim // attn.num_heads, n, ti, attn.resident), self.norm1.eps, self.norm2.eps, dtype)
                 return replace_feature(x, y)
         shortcut = x
         x = self.forward_part1(x, mask_matrix)

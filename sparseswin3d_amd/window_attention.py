@@ -692,12 +692,11 @@ class WindowAttentionSparse(nn.Module):
 
     ``fused`` (class or instance attribute, default True) selects the fused HIP path of
     :mod:`sparseswin3d_amd.fused` wherever it is supported (windows up to 384 positions with a relative
-    position table, 7^3 included; measured faster than the operator path there too: 1.05 against 1.19 ms per
-    module call on a room of 112 000 voxels, 3 heads of 16 channels); with ``fused = False`` the forward pass is
-    the operator-by-operator composition of the reference.  ``resident`` picks between the two
-    fused variants: True = window-resident kernels (attention matrix kept in registers, heads
-    of 32 channels only), False = block products with the attention matrix in HBM, None =
-    resident whenever it applies.  All paths give the same result.
+    position table, 7^3 included); with ``fused = False`` the forward pass is the operator-by-operator composition
+    of the reference.  ``resident`` picks among the fused kernels: None = the attention matrix kept in registers
+    wherever that applies (heads of 32 channels: the window-resident kernels; heads of 16, or windows of more than
+    128 positions: the flash kernels), True = window-resident kernels, False = block products with the attention
+    matrix in HBM.  All paths give the same result.
     """
 
     fused = True
@@ -748,7 +747,7 @@ class WindowAttentionSparse(nn.Module):
         return prefetch_plans([(self, x)])[0]
 
     def _fused_arguments(self, features, n):
-        """(BiasTableIndex or None, window-resident kernels?, compute dtype) where the fused path takes this call, else
+        """(BiasTableIndex or None, compute dtype) where the fused path takes this call, else
         None.  Under autocast the projections and the attention run in its type, as ``nn.Linear`` would."""
         from . import fused
         if not self.fused:
@@ -762,8 +761,7 @@ class WindowAttentionSparse(nn.Module):
         ti = self._table_index(n)
         if n > 384 if ti is not None else n * n * 4 > 64 * 1024:
             return None
-        can = self.dim == 32 * self.num_heads and n <= 128
-        return ti, can if self.resident is None else bool(self.resident), dtype
+        return ti, dtype
 
     def forward(self, x, mask):
         n = x.spatial_shape[0]
@@ -776,9 +774,9 @@ class WindowAttentionSparse(nn.Module):
             native = self._fused_arguments(x.features, n)
             if native is not None:
                 from . import fused
-                ti, resident, dtype = native
+                ti, dtype = native
                 bias = self.relative_position_bias_table if ti is not None else self.relative_position_bias(n, torch.float32)
-                out = fused.fused_window_attention(None, bias, x.indices, mask, b, n, self.scale, resident, plan, ti,
+                out = fused.fused_window_attention(None, bias, x.indices, mask, b, n, self.scale, self.resident, plan, ti,
                                                    (x.features, self.qkv, self.proj, self.num_heads, dtype))
                 return replace_feature(x, self.proj_drop(out))
         qkv = tall_linear(x.features, self.qkv).reshape(-1, 3, self.num_heads, c // self.num_heads)

@@ -1,0 +1,72 @@
+"""The attention kernels for heads of 16 / 32 channels and windows of any size (``sswin_flash_*``) against the block products
+with the attention matrix in memory (the other implementation of the same softmax), all gradients included.
+
+fp32: both carry fp32 rounding of sums of at most 384 terms (2e-5 of a result's norm, bias gradient included); 16-bit: P and dS are
+rounded to the tokens' type before the second products here (as the other 16-bit kernels do), a relative 2^-8 / 2^-11 of each term."""
+import numpy as np
+import pytest
+import torch
+
+from helpers import random_window_indices, ragged_window_indices
+
+pytestmark = pytest.mark.gpu
+
+MIXES = {
+    "tiny": ([1, 2, 3, 1, 0, 5, 31, 1, 1, 7, 9, 15, 16, 17, 2, 1], 125),          # many windows in one block
+    "edges": ([32, 33, 31, 63, 64, 65, 16, 48, 1, 125, 0, 96, 97], 125),
+    "large": ([343, 129, 1, 200, 31, 256, 257, 5, 5, 5, 30, 343, 128], 343),
+    "one": ([1], 27),
+}
+
+
+@pytest.mark.parametrize("mix", list(MIXES))
+@pytest.mark.parametrize("hd,dtype", [(16, torch.float32), (32, torch.float32), (16, torch.float16), (16, torch.bfloat16), (32, torch.bfloat16)],
+                         ids=["16-fp32", "32-fp32", "16-fp16", "16-bf16", "32-bf16"])
+@pytest.mark.parametrize("use_mask", [False, True], ids=["plain", "mask"])
+def test_flash_against_block_products(mix, hd, dtype, use_mask):
+    from sparseswin3d_amd.fused import BiasTableIndex, TokenPlan, attention_path, fused_window_attention
+    from sparseswin3d_amd.window_attention import relative_position_index_3d
+    counts, n = MIXES[mix]
+    w = round(n ** (1 / 3))
+    H = 3
+    rng = np.random.default_rng(len(counts) + hd)
+    ind = torch.from_numpy(ragged_window_indices(rng, counts, n)).cuda()
+    ti = BiasTableIndex.build(relative_position_index_3d((w, w, w)).cuda(), (2 * w - 1) ** 3)
+    assert attention_path(hd, n, ti, None) == ("flash" if hd == 16 or n > 128 else "resident")
+    torch.manual_seed(hd)
+    qkv = (torch.randn(len(ind), 3, H, hd) * 1.5).to(dtype).cuda()
+    qkv[::7] *= 6                                                  # some rows with large scores: the running offset moves
+    table = torch.randn((2 * w - 1) ** 3, H).cuda()
+    mask = torch.from_numpy(rng.integers(0, 27, (len(counts), n)).astype(np.int8)).cuda() if use_mask else None
+    up = torch.randn(len(ind), H * hd).to(dtype).cuda()
+    got = []
+    from sparseswin3d_amd import _lib
+    for path in ("flash", "products"):
+        x, t = qkv.clone().requires_grad_(True), table.clone().requires_grad_(True)
+        plan = TokenPlan(ind, len(counts), n, H)
+        out = _lib.native().attention(x, t, plan.native, mask, ti.code, ti.offset0, n, hd ** -0.5, path)
+        out.backward(up)
+        got.append((out.detach(), x.grad, t.grad))
+        with torch.no_grad():
+            assert torch.equal(_lib.native().attention(qkv, table, plan.native, mask, ti.code, ti.offset0, n, hd ** -0.5, path), out)
+    tol = {torch.float32: 2e-5, torch.float16: 4e-3, torch.bfloat16: 3e-2}[dtype]
+    for a, b, what in zip(*got, ("out", "d qkv", "d table")):
+        assert not torch.isnan(a).any(), what
+        # a lone token's dS is zero up to the rounding of dP - D, two numbers of order ten: held to the bound of a result of norm 1
+        rel = ((a.double() - b.double()).norm() / b.double().norm().clamp_min(1.0)).item()
+        assert rel < tol, (what, rel)
+
+
+def test_flash_many_windows_and_heads():
+    """Workgroups in whole rounds over the XCDs and in the remainder; head and chunk numbers of every workgroup."""
+    from sparseswin3d_amd.fused import BiasTableIndex, TokenPlan
+    from sparseswin3d_amd.window_attention import relative_position_index_3d
+    from sparseswin3d_amd import _lib
+    rng = np.random.default_rng(0)
+    ti = BiasTableIndex.build(relative_position_index_3d((5, 5, 5)).cuda(), 729)
+    for N, H in ((2600, 5), (257, 2), (20000, 1)):
+        ind = torch.from_numpy(random_window_indices(rng, 700, 125, N)).cuda()
+        qkv, table = torch.randn(N, 3, H, 16).cuda(), torch.randn(729, H).cuda()
+        plan = TokenPlan(ind, 700, 125, H)
+        a, b = (_lib.native().attention(qkv, table, plan.native, None, ti.code, ti.offset0, 125, 0.25, p) for p in ("flash", "products"))
+        assert ((a - b).norm() / b.norm()).item() < 1e-5, (N, H)
