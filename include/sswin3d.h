@@ -444,14 +444,20 @@ int sswin_tall_linear_weight_grad(const float* dy, const float* x, int64_t N, in
 /* Dense layers of fp32, fp16 or bf16 tokens with what follows the product folded in (nn.Linear at swin3d_base.py:606-610 and
  * :722-735; sswin_dense_supported: K and P multiples of 16).
  * y [N, P] = last step of x [N, K] Wop + bias: transposed == 0: Wop = W^T of w [P, K] (the layer); 1: Wop = w [K, P] as stored
- * (the input gradient of a layer with K outputs and P inputs; no bias).  x: dtype; w and bias: w_dtype (dtype, or fp32 under
- * mixed precision); y: out_dtype (dtype, or fp32 with SSWIN_DENSE_RESIDUAL under mixed precision).
+ * (the input gradient of a layer with K outputs and P inputs; no bias).  x, w and bias: dtype; y: out_dtype (dtype, or fp32
+ * with SSWIN_DENSE_RESIDUAL under mixed precision, where the residual stream is fp32).
  * epilogue SSWIN_DENSE_GELU: y = gelu(.), slope [N, P] = its derivative (or null); SSWIN_DENSE_RESIDUAL: y = . + extra [N, P]
  * of out_dtype; SSWIN_DENSE_SCALE (transposed only): y = . * extra [N, P] of dtype.  Accumulation in fp32. */
 enum { SSWIN_DENSE_PLAIN = 0, SSWIN_DENSE_GELU = 1, SSWIN_DENSE_RESIDUAL = 2, SSWIN_DENSE_SCALE = 3 };
 int sswin_dense_supported(int dtype, int P, int K);
-int sswin_dense_forward(int dtype, int w_dtype, int out_dtype, int transposed, int epilogue, const void* x, int64_t N, int K,
-                        const void* w, const void* bias, int P, const void* extra, void* y, void* slope, void* stream);
+int sswin_dense_forward(int dtype, int out_dtype, int transposed, int epilogue, const void* x, int64_t N, int K, const void* w,
+                        const void* bias, int P, const void* extra, void* y, void* slope, void* ws, size_t ws_bytes, void* stream);
+/* up to SSWIN_CAST_PARTS fp32 arrays (16-byte aligned, sizes[i] values, multiples of 8) behind each other in dst as fp16 or bf16,
+ * rounded to nearest: the parameters of a block under mixed precision. */
+enum { SSWIN_CAST_PARTS = 8 };
+int sswin_cast_parts(int dtype, const void* const* src, const int64_t* sizes, int count, void* dst, void* stream);
+/* scratch for long reductions over few rows (shares of the reduction added in a fixed order); with less the call runs without */
+size_t sswin_dense_forward_workspace_bytes(int dtype, int64_t N, int K, int P);
 /* dw [P, K] = dy^T x and db [P] = column sums of dy (or null) for dy [N, P], x [N, K] of dtype; dw, db of out_dtype (dtype or
  * fp32).  Partial sums over row chunks are added in a fixed order: the same bits on every run. */
 size_t sswin_dense_weight_grad_workspace_bytes(int dtype, int64_t N, int P, int K);

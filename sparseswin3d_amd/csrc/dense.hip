@@ -6,16 +6,17 @@
 // pieces (x = h + m + l by truncation and exact subtraction) and a product is the sum of the six piece products that
 // weigh at least 2^-16 of the leading one; what is dropped is below 2^-23 of the product.
 //
-// dense_rows_kernel: a workgroup of WM wavefronts owns BM = 32 MT WM rows and 96 columns.  Both operands pass through
-// registers (conversion, splitting) into LDS in matrix operand order, [k step][row tile][plane][lane] pieces of 16
-// bytes, so that every operand read is one conflict-free 16-byte read per lane; two buffers, one barrier per BK columns
-// of the reduction, the next BK in flight meanwhile.  96 columns because every layer of a stage has a multiple of 48.
-// The tile of the result goes back through LDS, so that bias, residual and result are touched in 16-byte pieces of whole
-// row segments.
+// dense_rows_kernel (fp32): a workgroup of WM wavefronts owns BM = 32 MT WM rows and 96 columns.  Both operands pass through
+// registers, where they are split, into LDS in matrix operand order, [row tile][plane][lane] pieces of 16 bytes, so that every
+// operand read is one conflict-free 16-byte read per lane; two buffers, one barrier per 16 columns of the reduction, the next
+// 16 in flight meanwhile.  96 columns because every layer of a stage has a multiple of 48.  The tile of the result goes back
+// through LDS, so that bias, residual and result are touched in 16-byte pieces of whole row segments.
+// dense16_rows_kernel (16 bit): tiles straight from memory to LDS.
 // dense_small_kernel: few rows and many channels (the deep stages): 32 x 32 tiles, the wavefronts of a workgroup share
 // the reduction instead of the rows, so that a few hundred rows still put a wavefront on every SIMD.
-// dense_wgrad_kernel: dW = dY^T X, db = column sums of dY: the reduction runs over the rows, both operands are read as
-// 8 rows x 2 columns per lane and turned in registers.  Row chunks are added by a second kernel in a fixed order.
+// dense_wgrad_kernel, dense16_wgrad_kernel: dW = dY^T X, db = column sums of dY: the reduction runs over the rows; fp32 operands
+// are read as 8 rows x 2 columns per lane and turned in registers, 16-bit ones by the transposing LDS load.  Row chunks are
+// added by a second kernel in a fixed order.
 #include <math.h>
 
 #include <algorithm>
@@ -59,15 +60,6 @@ template <> struct Op<__hip_bfloat16> {
     }
 };
 
-template <typename T> __device__ __forceinline__ uint32_t pack2(float a, float b);
-template <> __device__ __forceinline__ uint32_t pack2<__half>(float a, float b) {
-    return (uint32_t)__half_as_ushort(__float2half(a)) | ((uint32_t)__half_as_ushort(__float2half(b)) << 16);
-}
-template <> __device__ __forceinline__ uint32_t pack2<__hip_bfloat16>(float a, float b) {
-    const __hip_bfloat16 x = __float2bfloat16(a), y = __float2bfloat16(b);
-    return (uint32_t)__builtin_bit_cast(uint16_t, x) | ((uint32_t)__builtin_bit_cast(uint16_t, y) << 16);
-}
-
 __device__ __forceinline__ void split2(float x0, float x1, uint32_t& h, uint32_t& m, uint32_t& l) {
     const uint32_t u0 = __builtin_bit_cast(uint32_t, x0), u1 = __builtin_bit_cast(uint32_t, x1);
     const float r0 = x0 - __builtin_bit_cast(float, u0 & 0xffff0000u), r1 = x1 - __builtin_bit_cast(float, u1 & 0xffff0000u);
@@ -98,10 +90,10 @@ __device__ __forceinline__ void planes_of(const float (&v)[8], u32x4 (&out)[Op<T
 // Raw values of a unit on their way from memory to LDS.
 // Along: 8 consecutive values of one row (reduction along the row).  Down: 8 rows x 2 columns (reduction down the rows).
 // ------------------------------------------------------------------------------------------
-template <typename T, typename TS> struct Along {
-    static constexpr bool WIDE = sizeof(TS) == 4;
+template <typename T> struct Along {
+    static constexpr bool WIDE = sizeof(T) == 4;
     u32x4 r[WIDE ? 2 : 1];
-    __device__ __forceinline__ void load(const TS* p) {
+    __device__ __forceinline__ void load(const T* p) {
         r[0] = *reinterpret_cast<const u32x4*>(p);
         if constexpr (WIDE) r[1] = *reinterpret_cast<const u32x4*>(p + 4);
     }
@@ -121,30 +113,26 @@ template <typename T, typename TS> struct Along {
     }
 };
 
-template <typename T, typename TS> struct Down {
-    static constexpr bool WIDE = sizeof(TS) == 4;
-    uint32_t r[8][WIDE ? 2 : 1];
-    __device__ __forceinline__ void load(int e, const TS* p) {
+struct Down {
+    uint32_t r[8][2];
+    __device__ __forceinline__ void load(int e, const float* p) {
         r[e][0] = reinterpret_cast<const uint32_t*>(p)[0];
-        if constexpr (WIDE) r[e][1] = reinterpret_cast<const uint32_t*>(p)[1];
+        r[e][1] = reinterpret_cast<const uint32_t*>(p)[1];
     }
-    __device__ __forceinline__ void zero(int e) {
-        r[e][0] = 0;
-        if constexpr (WIDE) r[e][1] = 0;
-    }
+    __device__ __forceinline__ void zero(int e) { r[e][0] = r[e][1] = 0; }
     // column c (0 or 1) of the pair
-    __device__ __forceinline__ void planes(int c, u32x4 (&out)[Op<T>::PL]) const {
-        if constexpr (WIDE) {
-            float v[8];
+    __device__ __forceinline__ void planes(int c, u32x4 (&out)[3]) const {
+        float v[8];
 #pragma unroll
-            for (int e = 0; e < 8; ++e) v[e] = __builtin_bit_cast(float, r[e][c]);
-            planes_of<T>(v, out);
-        } else {
-#pragma unroll
-            for (int q = 0; q < 4; ++q) out[0][q] = __builtin_amdgcn_perm(r[2 * q + 1][0], r[2 * q][0], c ? 0x07060302u : 0x05040100u);
-        }
+        for (int e = 0; e < 8; ++e) v[e] = __builtin_bit_cast(float, r[e][c]);
+        planes_of<float>(v, out);
     }
-    __device__ __forceinline__ float sum(int c) const;
+    __device__ __forceinline__ float sum(int c) const {
+        float s = 0.f;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) s += __builtin_bit_cast(float, r[e][c]);
+        return s;
+    }
 };
 template <typename T> __device__ __forceinline__ float half_of(uint32_t w, int c);
 template <> __device__ __forceinline__ float half_of<__half>(uint32_t w, int c) {
@@ -153,19 +141,10 @@ template <> __device__ __forceinline__ float half_of<__half>(uint32_t w, int c) 
 template <> __device__ __forceinline__ float half_of<__hip_bfloat16>(uint32_t w, int c) {
     return __builtin_bit_cast(float, c ? w & 0xffff0000u : w << 16);
 }
-template <typename T, typename TS> __device__ __forceinline__ float Down<T, TS>::sum(int c) const {
-    float s = 0.f;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-        if constexpr (WIDE) s += __builtin_bit_cast(float, r[e][c]);
-        else s += half_of<T>(r[e][0], c);
-    }
-    return s;
-}
 
 // position of (row, 8-value chunk) inside its 32-row operand block: the rows of a chunk are rotated by the chunk, so
 // that lanes which hold the chunks of one row write to different banks
-template <int BK> __device__ __forceinline__ int swz(int chunk) { return BK == 16 ? (chunk & 1) * 4 : chunk & 7; }
+__device__ __forceinline__ int swz(int chunk) { return (chunk & 1) * 4; }
 
 // workgroups b, b + 8, b + 16 ... share an XCD and its L2: the column blocks of one row block are dealt to such workgroups
 __device__ __forceinline__ void block_of(int groups, int& cg, int64_t& rb) {
@@ -182,14 +161,14 @@ __device__ __forceinline__ void block_of(int groups, int& cg, int64_t& rb) {
 // ------------------------------------------------------------------------------------------
 // y [N, P] = last step of x [N, K] Wop, Wop [K, P] = W^T of W [P, K] (DOWN = false) or W [K, P] itself (DOWN = true)
 // ------------------------------------------------------------------------------------------
-template <typename T, typename TB, typename TO, int EPI, bool DOWN, int WM, int MT, int OCC>
-__global__ __launch_bounds__(WM * 64) __attribute__((amdgpu_waves_per_eu(OCC, OCC))) void dense_rows_kernel(const T* __restrict__ x, int64_t N, int K, const TB* __restrict__ w, int P,
-                                                             int groups, Epilogue ep) {
-    constexpr int PL = Op<T>::PL, BK = PL == 3 ? 16 : 48, KS = BK / 16, KC = BK / 8;
+template <int EPI, bool DOWN, int WM, int MT, int OCC>
+__global__ __launch_bounds__(WM * 64) __attribute__((amdgpu_waves_per_eu(OCC, OCC))) void dense_rows_kernel(
+    const float* __restrict__ x, int64_t N, int K, const float* __restrict__ w, int P, int groups, Epilogue ep) {
+    constexpr int PL = 3, BK = 16, KC = BK / 8;
     constexpr int NT = 3, BN = 96, BM = WM * MT * 32, THREADS = WM * 64;
     constexpr int A_UNITS = BM * KC, UA = (A_UNITS + THREADS - 1) / THREADS;
     constexpr int B_UNITS = (DOWN ? BN / 2 : BN) * KC, UB = (B_UNITS + THREADS - 1) / THREADS;
-    constexpr int A_LDS = KS * (BM / 32) * PL * 64, B_LDS = KS * NT * PL * 64, BUF = A_LDS + B_LDS;      // 16-byte pieces
+    constexpr int A_LDS = BM / 32 * PL * 64, B_LDS = NT * PL * 64, BUF = A_LDS + B_LDS;      // 16-byte pieces
     extern __shared__ __attribute__((aligned(16))) u32x4 lds[];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, half = lane >> 5, l32 = lane & 31;
     int cg;
@@ -199,8 +178,8 @@ __global__ __launch_bounds__(WM * 64) __attribute__((amdgpu_waves_per_eu(OCC, OC
     const int col0 = cg * BN;
 
     // addresses: a uniform base that moves along the reduction plus 32-bit lane offsets formed once
-    Along<T, T> ra[UA];
-    typename std::conditional<DOWN, Down<T, TB>, Along<T, TB>>::type rw[UB];
+    Along<float> ra[UA];
+    typename std::conditional<DOWN, Down, Along<float>>::type rw[UB];
     uint32_t oa[UA], ow[UB];
     const int last = (int)(N - 1 - row0 < BM - 1 ? N - 1 - row0 : BM - 1);   // rows past the end repeat the last one
 #pragma unroll
@@ -214,36 +193,28 @@ __global__ __launch_bounds__(WM * 64) __attribute__((amdgpu_waves_per_eu(OCC, OC
         if (DOWN) ow[i] = (uint32_t)((u / (BN / 2)) * 8 * P + min(col0 + (u % (BN / 2)) * 2, P - 2));
         else ow[i] = (uint32_t)(min(col0 + u / KC, P - 1) * K + (u % KC) * 8);
     }
-    const T* xb = x + row0 * K;
+    const float* xb = x + row0 * K;
     auto request = [&](int k0) {
 #pragma unroll
         for (int i = 0; i < UA; ++i) {
             const int u = threadIdx.x + i * THREADS;
-            if (A_UNITS % THREADS == 0 || u < A_UNITS) {
-                if (BK == 16 || k0 + (u % KC) * 8 < K) ra[i].load(xb + k0 + oa[i]);
-                else ra[i].zero();
-            }
+            if (A_UNITS % THREADS == 0 || u < A_UNITS) ra[i].load(xb + k0 + oa[i]);
         }
 #pragma unroll
         for (int i = 0; i < UB; ++i) {
             const int u = threadIdx.x + i * THREADS;
             if (B_UNITS % THREADS == 0 || u < B_UNITS) {
                 if constexpr (DOWN) {
-                    const bool in = BK == 16 || k0 + (u / (BN / 2)) * 8 < K;
 #pragma unroll
-                    for (int e = 0; e < 8; ++e) {
-                        if (in) rw[i].load(e, w + (int64_t)(k0 + e) * P + ow[i]);
-                        else rw[i].zero(e);
-                    }
+                    for (int e = 0; e < 8; ++e) rw[i].load(e, w + (int64_t)(k0 + e) * P + ow[i]);
                 } else {
-                    if (BK == 16 || k0 + (u % KC) * 8 < K) rw[i].load(w + k0 + ow[i]);
-                    else rw[i].zero();
+                    rw[i].load(w + k0 + ow[i]);
                 }
             }
         }
     };
     auto put = [&](u32x4* base, int tiles, int row, int c, const u32x4 (&p)[PL]) {
-        u32x4* dst = base + (((c >> 1) * tiles + (row >> 5)) * PL) * 64 + (c & 1) * 32 + ((row & 31) ^ swz<BK>(c));
+        u32x4* dst = base + (((c >> 1) * tiles + (row >> 5)) * PL) * 64 + (c & 1) * 32 + ((row & 31) ^ swz(c));
 #pragma unroll
         for (int q = 0; q < PL; ++q) dst[q * 64] = p[q];
     };
@@ -280,33 +251,30 @@ __global__ __launch_bounds__(WM * 64) __attribute__((amdgpu_waves_per_eu(OCC, OC
     for (int i = 0; i < MT; ++i)
 #pragma unroll
         for (int j = 0; j < NT; ++j) acc[i][j] = f32x16{0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-    const int nk = (K + BK - 1) / BK;
+    const int nk = K / BK;
     request(0);
     store(lds);
     for (int kb = 0; kb < nk; ++kb) {
         __syncthreads();
         if (kb + 1 < nk) request((kb + 1) * BK);
         const u32x4* buf = lds + (kb & 1) * BUF;
+        const int at = half * 32 + (l32 ^ swz(half));
+        u32x4 a[MT][PL], b[NT][PL];
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-            const int at = half * 32 + (l32 ^ swz<BK>(ks * 2 + half));
-            u32x4 a[MT][PL], b[NT][PL];
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+            for (int q = 0; q < PL; ++q) a[i][q] = buf[((wave * MT + i) * PL + q) * 64 + at];
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+#pragma unroll
+            for (int q = 0; q < PL; ++q) b[j][q] = buf[A_LDS + (j * PL + q) * 64 + at];
+#pragma unroll
+        for (int p = 0; p < Op<float>::NP; ++p)
 #pragma unroll
             for (int i = 0; i < MT; ++i)
 #pragma unroll
-                for (int q = 0; q < PL; ++q) a[i][q] = buf[((ks * (BM / 32) + wave * MT + i) * PL + q) * 64 + at];
-#pragma unroll
-            for (int j = 0; j < NT; ++j)
-#pragma unroll
-                for (int q = 0; q < PL; ++q) b[j][q] = buf[A_LDS + ((ks * NT + j) * PL + q) * 64 + at];
-#pragma unroll
-            for (int p = 0; p < Op<T>::NP; ++p)
-#pragma unroll
-                for (int i = 0; i < MT; ++i)
-#pragma unroll
-                    for (int j = 0; j < NT; ++j) acc[i][j] = Op<T>::mfma(a[i][Op<T>::PA[p]], b[j][Op<T>::PB[p]], acc[i][j]);
-            __builtin_amdgcn_sched_barrier(0);                           // operands of later steps stay out of registers
-        }
+                for (int j = 0; j < NT; ++j) acc[i][j] = Op<float>::mfma(a[i][Op<float>::PA[p]], b[j][Op<float>::PB[p]], acc[i][j]);
+        __builtin_amdgcn_sched_barrier(0);                               // the next operands' splitting stays behind the products
         if (kb + 1 < nk) store(lds + ((kb + 1) & 1) * BUF);
     }
     // the tile of the wavefront, 32 rows at a time, through its own part of LDS (pitch 100: rows start 4 banks apart)
@@ -321,13 +289,357 @@ __global__ __launch_bounds__(WM * 64) __attribute__((amdgpu_waves_per_eu(OCC, OC
 #pragma unroll
             for (int r = 0; r < 16; ++r) mine[acc_row(r, half) * PITCH + j * 32 + l32] = acc[i][j][r];
         __builtin_amdgcn_wave_barrier();
+        constexpr int PIECES = 32 * (BN / 4) / 64;
+        Second4<float, float, EPI> second[PIECES];
 #pragma unroll
-        for (int q = 0; q < 32 * (BN / 4) / 64; ++q) {
+        for (int q = 0; q < PIECES; ++q) {
+            const int e = q * 64 + lane, rr = e / (BN / 4), cc = (e % (BN / 4)) * 4;
+            if (r0 + rr < N && col0 + cc < P) second[q].load(ep, r0 + rr, col0 + cc, P);
+        }
+#pragma unroll
+        for (int q = 0; q < PIECES; ++q) {
             const int e = q * 64 + lane, rr = e / (BN / 4), cc = (e % (BN / 4)) * 4;
             const f32x4 v = *reinterpret_cast<const f32x4*>(mine + rr * PITCH + cc);
-            if (r0 + rr < N && col0 + cc < P) finish4<T, TB, TO, EPI>(ep, r0 + rr, col0 + cc, P, v);
+            if (r0 + rr < N && col0 + cc < P) finish4<float, float, EPI>(ep, r0 + rr, col0 + cc, P, v, second[q]);
         }
         __builtin_amdgcn_wave_barrier();
+    }
+}
+
+// ------------------------------------------------------------------------------------------
+// 16-bit operands: the same products with tiles that go from memory to LDS directly (no registers in between), the next
+// block of the reduction in flight, and operands that lie across the reduction read through the transposing LDS load
+// (ds_read_b64_tr_b16: a group of 16 lanes reads 4 rows x 16 columns and lane i receives column i).
+//
+// Tile layouts are the memory's own: [row][BK] for operands along the reduction, the pieces of a row exchanged;
+// [row of the reduction][96] for operands down the reduction (192-byte rows: the four rows of a transposing read lie in
+// different banks).  A wavefront waits for its own loads of the oldest block (vmcnt), one barrier makes the block
+// complete, the next loads go into the buffer that was read one block ago.
+//
+// WM x WN wavefronts share the tile (32 MT rows x 96 columns each), KG = 2 groups of them the steps of a block.  What
+// bounds it: at 96 channels the traffic of the result (219 000 rows 96 -> 288, 168 MB: 44 us, with operands through registers
+// 57; its input gradient 33 and 43), at long reductions what passes from L2 into LDS, 14 TB/s over the chip (8119 rows
+// 768 -> 3072: 57 us, through registers 73).
+// ------------------------------------------------------------------------------------------
+typedef short s16x4_t __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) s16x4_t lds_s16x4;
+
+// 64 lanes x 16 bytes: lane l's piece lands at lds + 16 l
+__device__ __forceinline__ void copy_to_lds(const void* src, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(src) : "memory", "m0");
+}
+__device__ __forceinline__ uint32_t lds_address(const void* p) {
+    return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)p;
+}
+template <int N> __device__ __forceinline__ void wait_copies() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
+__device__ __forceinline__ void block_barrier() {
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
+// place of a 16-byte piece in its row of BK values: pieces are exchanged by the row's number, so that the lanes of a read
+// (consecutive rows, the same piece) lie in different banks
+template <int BK> __device__ __forceinline__ int swapped(int row, int piece) {
+    static_assert(BK == 32 || BK == 64, "four or eight pieces a row");
+    return BK == 32 ? piece ^ (((row >> 1) ^ (row >> 3)) & 3) : piece ^ (row & 7);
+}
+// operand of 32 rows x 16 reduction slots from a tile whose rows run along the reduction
+template <typename T, int BK>
+__device__ __forceinline__ u32x4 along_operand(const T* tile, int row0, int ks) {
+    const int row = row0 + (threadIdx.x & 31);
+    return *reinterpret_cast<const u32x4*>(tile + row * BK + swapped<BK>(row, ks * 2 + ((threadIdx.x & 63) >> 5)) * 8);
+}
+// the same from a tile whose rows run across it ([reduction][96])
+template <typename T>
+__device__ __forceinline__ u32x4 down_operand(const T* tile, int col, int ks) {
+    const int lane = threadIdx.x & 63, g = lane >> 4, i = lane & 15;
+    const T* p = tile + (ks * 16 + (g >> 1) * 8 + (i >> 2)) * 96 + col + (g & 1) * 16 + (i & 3) * 4;
+    union {
+        s16x4_t h[2];
+        u32x4 v;
+    } o;
+    o.h[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)p);
+    o.h[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(p + 4 * 96));
+    return o.v;
+}
+
+template <typename T, typename TO, int EPI, bool DOWN, int BK, int WM, int WN, int KG, int MT, int STAGES, int OCC>
+__global__ __launch_bounds__(WM * WN * KG * 64) __attribute__((amdgpu_waves_per_eu(OCC, OCC))) void dense16_rows_kernel(
+    const T* __restrict__ x, int64_t N, int K, const T* __restrict__ w, int P, int groups, int ksplit, float* __restrict__ part, Epilogue ep) {
+    constexpr int PR = BK / 8, NT = 3, BN = 96 * WN, BM = WM * MT * 32, THREADS = WM * WN * KG * 64;
+    constexpr int A_PIECES = BM * PR, B_PIECES = BN * PR, UA = (A_PIECES + THREADS - 1) / THREADS, UB = (B_PIECES + THREADS - 1) / THREADS;
+    static_assert(A_PIECES % 64 == 0 && B_PIECES % 64 == 0 && BK % (16 * KG) == 0, "whole wavefronts of pieces");
+    constexpr int BUF = (A_PIECES + B_PIECES) * 8;                       // values
+    extern __shared__ __attribute__((aligned(16))) u32x4 lds[];
+    T* const tiles = reinterpret_cast<T*>(lds);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, half = lane >> 5, l32 = lane & 31;
+    const int wk = wave / (WM * WN), wm = wave % (WM * WN) / WN, wn = wave % WN;
+    int cg;
+    int64_t rb;
+    block_of(groups * ksplit, cg, rb);
+    const int part_no = cg / groups;                                     // share of the reduction
+    cg %= groups;
+    const int64_t row0 = rb * BM;
+    const int col0 = cg * BN;
+    const int all = (K + BK - 1) / BK, k_first = all * part_no / ksplit, nk = all * (part_no + 1) / ksplit - k_first;
+    const int last = (int)(N - 1 - row0 < BM - 1 ? N - 1 - row0 : BM - 1);   // rows past the end repeat the last one
+    // this lane's pieces: row and first value of a piece of X; row (of the output, or of the reduction) and first value of Wop
+    const T* pa[UA];
+    const T* pb[UB];
+    auto a_k = [](int u) { return swapped<BK>(u / PR, u % PR) * 8; };
+    auto b_k = [](int u) { return DOWN ? u % (BK * 12) / 12 : swapped<BK>(u / PR, u % PR) * 8; };
+#pragma unroll
+    for (int i = 0; i < UA; ++i) {
+        const int u = i * THREADS + threadIdx.x;
+        pa[i] = x + (row0 + min(u / PR, last)) * K + k_first * BK + a_k(u);
+    }
+#pragma unroll
+    for (int i = 0; i < UB; ++i) {
+        const int u = i * THREADS + threadIdx.x;
+        if (DOWN) pb[i] = w + (int64_t)(k_first * BK + b_k(u)) * P + min(col0 + u / (BK * 12) * 96 + (u % 12) * 8, P - 8);
+        else pb[i] = w + (int64_t)min(col0 + u / PR, P - 1) * K + k_first * BK + b_k(u);
+    }
+    const int64_t step_b = DOWN ? (int64_t)BK * P : BK;
+    const uint32_t base = lds_address(tiles);
+    auto request = [&](int kb) {
+        const uint32_t buf = base + (uint32_t)(kb % STAGES) * BUF * 2;
+        const int k0 = (k_first + kb) * BK;
+        const bool ragged = k0 + BK > K;                                 // then the last piece or row inside; cleared below
+#pragma unroll
+        for (int i = 0; i < UA; ++i)
+            if (i * THREADS + wave * 64 < A_PIECES) {                    // uniform in the wavefront
+                const int over = ragged ? max(k0 + a_k(i * THREADS + threadIdx.x) - (K - 8), 0) : 0;
+                copy_to_lds(pa[i] - over, buf + (uint32_t)(i * THREADS + wave * 64) * 16);
+                pa[i] += BK;
+            }
+#pragma unroll
+        for (int i = 0; i < UB; ++i)
+            if (i * THREADS + wave * 64 < B_PIECES) {
+                const int over = ragged ? max(k0 + b_k(i * THREADS + threadIdx.x) - (K - (DOWN ? 1 : 8)), 0) : 0;
+                copy_to_lds(pb[i] - (DOWN ? (int64_t)over * P : over), buf + (uint32_t)(A_PIECES + i * THREADS + wave * 64) * 16);
+                pb[i] += step_b;
+            }
+    };
+    // a wavefront's loads per block, for the counter of outstanding loads: all wavefronts wait for the smallest number that is safe
+    constexpr int FEWEST = A_PIECES / THREADS + B_PIECES / THREADS;
+
+    f32x16 acc[MT][NT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) acc[i][j] = f32x16{0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+    for (int p = 0; p < STAGES - 1; ++p)
+        if (p < nk) request(p);
+    for (int kb = 0; kb < nk; ++kb) {
+        if (kb + STAGES - 1 <= nk) wait_copies<FEWEST * (STAGES - 2)>();
+        else wait_copies<0>();
+        block_barrier();
+        if (kb + STAGES - 1 < nk) request(kb + STAGES - 1);
+        T* ta = tiles + (kb % STAGES) * BUF;
+        T* tb = ta + A_PIECES * 8;
+        const int left = K - (k_first + kb) * BK;
+        if (left < BK) {
+            for (int u = threadIdx.x; u < A_PIECES; u += THREADS)
+                if (a_k(u) >= left) reinterpret_cast<u32x4*>(ta)[u] = u32x4{0, 0, 0, 0};
+            for (int u = threadIdx.x; u < B_PIECES; u += THREADS)
+                if (b_k(u) >= left) reinterpret_cast<u32x4*>(tb)[u] = u32x4{0, 0, 0, 0};
+            block_barrier();
+        }
+#pragma unroll
+        for (int q = 0; q < BK / 16 / KG; ++q) {
+            const int ks = wk * (BK / 16 / KG) + q;
+            u32x4 a[MT], b[NT];
+#pragma unroll
+            for (int i = 0; i < MT; ++i) a[i] = along_operand<T, BK>(ta, (wm * MT + i) * 32, ks);
+#pragma unroll
+            for (int j = 0; j < NT; ++j) b[j] = DOWN ? down_operand(tb + wn * BK * 96, j * 32, ks) : along_operand<T, BK>(tb, wn * 96 + j * 32, ks);
+#pragma unroll
+            for (int i = 0; i < MT; ++i)
+#pragma unroll
+                for (int j = 0; j < NT; ++j) acc[i][j] = Op<T>::mfma(a[i], b[j], acc[i][j]);
+        }
+    }
+    block_barrier();
+    if constexpr (KG == 2) {                                             // the two halves of each block's steps
+        float* other = reinterpret_cast<float*>(lds) + (wave % (WM * WN)) * MT * NT * 16 * 64;
+        if (wk == 1) {
+#pragma unroll
+            for (int i = 0; i < MT; ++i)
+#pragma unroll
+                for (int j = 0; j < NT; ++j)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) other[((i * NT + j) * 16 + r) * 64 + lane] = acc[i][j][r];
+        }
+        block_barrier();
+        if (wk == 0) {
+#pragma unroll
+            for (int i = 0; i < MT; ++i)
+#pragma unroll
+                for (int j = 0; j < NT; ++j)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) acc[i][j][r] += other[((i * NT + j) * 16 + r) * 64 + lane];
+        }
+        block_barrier();
+        if (wk == 1) return;
+    }
+    // through LDS, 32 columns at a time, so that every lane holds four neighbouring columns
+    constexpr int PITCH = 36;
+    float* mine = reinterpret_cast<float*>(lds) + wave * 32 * PITCH;
+    const int rr = lane >> 3, cc = (lane & 7) * 4;
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+        const int64_t r0 = row0 + (wm * MT + i) * 32 + rr;
+        const int c0 = col0 + wn * 96 + cc;
+#pragma unroll
+        for (int j = 0; j < NT; ++j) {
+            Second4<T, TO, EPI> second[4];
+            if (!part)
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    if (r0 + q * 8 < N && c0 + j * 32 < P) second[q].load(ep, r0 + q * 8, c0 + j * 32, P);
+#pragma unroll
+            for (int r = 0; r < 16; ++r) mine[acc_row(r, half) * PITCH + l32] = acc[i][j][r];
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const f32x4 v = *reinterpret_cast<const f32x4*>(mine + (q * 8 + rr) * PITCH + cc);
+                const int64_t row = r0 + q * 8;
+                const int col = c0 + j * 32;
+                if (row < N && col < P) {
+                    if (part) *reinterpret_cast<f32x4*>(part + ((int64_t)part_no * N + row) * P + col) = v;
+                    else finish4<T, TO, EPI>(ep, row, col, P, v, second[q]);
+                }
+            }
+            __builtin_amdgcn_wave_barrier();
+        }
+    }
+}
+
+// the shares of the reduction added in order, then the last step
+template <typename T, typename TO, int EPI>
+__global__ __launch_bounds__(256) void dense_parts_kernel(const float* __restrict__ part, int64_t N, int P, int parts, Epilogue ep) {
+    const int64_t quads = N * (P / 4), i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= quads) return;
+    const int64_t row = i / (P / 4);
+    const int col = (int)(i % (P / 4)) * 4;
+    Second4<T, TO, EPI> second;
+    second.load(ep, row, col, P);
+    f32x4 v = *reinterpret_cast<const f32x4*>(part + i * 4);
+    for (int p = 1; p < parts; ++p) v += *reinterpret_cast<const f32x4*>(part + (int64_t)p * N * P + i * 4);
+    finish4<T, TO, EPI>(ep, row, col, P, v, second);
+}
+
+// dW [P, K] = dY^T X for one chunk of rows; WM x WN wavefronts of (32 MT) x 96 each, BM = 32 MT WM columns of dY (a multiple of
+// 96), BN = 96 WN columns of X
+// (219 000 rows 96 -> 288, 168 MB: 39 us; 384 -> 96 45; the traffic's own time at copy rate is 33 and 41)
+template <typename T, int WM, int WN, int MT, int STAGES, int OCC>
+__global__ __launch_bounds__(WM * WN * 64) __attribute__((amdgpu_waves_per_eu(OCC, OCC))) void dense16_wgrad_kernel(
+    const T* __restrict__ dy, const T* __restrict__ x, int64_t N, int P, int K, int tiles_p, int tiles_k, int64_t rows_per_chunk, float* __restrict__ part_w,
+    float* __restrict__ part_b) {
+    constexpr int BK = 32, NT = 3, BM = WM * MT * 32, BN = WN * 96, THREADS = WM * WN * 64;
+    static_assert(BM % 96 == 0, "sub-tiles of 96 columns");
+    constexpr int SUB = BK * 12;                                         // pieces of a sub-tile of 96 columns
+    constexpr int PIECES = (BM / 96 + WN) * SUB, U = PIECES / THREADS, BUF = PIECES * 8;
+    static_assert(PIECES % THREADS == 0, "whole rounds of pieces");
+    extern __shared__ __attribute__((aligned(16))) u32x4 lds[];
+    T* const tiles = reinterpret_cast<T*>(lds);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, half = lane >> 5, l32 = lane & 31;
+    const int wm = wave / WN, wn = wave % WN;
+    int tile;
+    int64_t chunk;
+    block_of(tiles_p * tiles_k, tile, chunk);
+    const int p0 = (tile / tiles_k) * BM, k0 = (tile % tiles_k) * BN;
+    const int64_t begin = chunk * rows_per_chunk, end = begin + rows_per_chunk < N ? begin + rows_per_chunk : N;
+    const int nk = (int)((end - begin + BK - 1) / BK);
+    const bool sums_here = part_b && k0 == 0 && wn == 0;
+    // piece u: sub-tile u / SUB (those of dY first), row (u % SUB) / 12, 8 columns u % 12
+    auto source = [&](int u, int64_t n0) -> const T* {
+        const int sub = u / SUB, r = u % SUB / 12, c = u % 12 * 8;
+        const int64_t n = n0 + r < end ? n0 + r : end - 1;               // rows past the end are cleared below
+        if (sub < BM / 96) return dy + n * P + min(p0 + sub * 96 + c, P - 8);
+        return x + n * K + min(k0 + (sub - BM / 96) * 96 + c, K - 8);
+    };
+    const T* p[U];
+    int64_t step[U];
+#pragma unroll
+    for (int i = 0; i < U; ++i) {
+        const int u = i * THREADS + threadIdx.x;
+        p[i] = source(u, begin);
+        step[i] = (int64_t)BK * (u / SUB < BM / 96 ? P : K);
+    }
+    const uint32_t base = lds_address(tiles);
+    auto request = [&](int kb) {
+        const uint32_t buf = base + (uint32_t)(kb % STAGES) * BUF * 2;
+        const bool ragged = begin + (int64_t)(kb + 1) * BK > end;
+#pragma unroll
+        for (int i = 0; i < U; ++i) {
+            copy_to_lds(ragged ? source(i * THREADS + threadIdx.x, begin + (int64_t)kb * BK) : p[i], buf + (uint32_t)(i * THREADS + wave * 64) * 16);
+            p[i] += step[i];
+        }
+    };
+    f32x16 acc[MT][NT];
+    float bs[MT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+        bs[i] = 0.f;
+#pragma unroll
+        for (int j = 0; j < NT; ++j) acc[i][j] = f32x16{0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+    }
+#pragma unroll
+    for (int q = 0; q < STAGES - 1; ++q)
+        if (q < nk) request(q);
+    for (int kb = 0; kb < nk; ++kb) {
+        if (kb + STAGES - 1 <= nk) wait_copies<U * (STAGES - 2)>();
+        else wait_copies<0>();
+        block_barrier();
+        if (kb + STAGES - 1 < nk) request(kb + STAGES - 1);
+        T* t = tiles + (kb % STAGES) * BUF;
+        const int left = (int)(end - begin - (int64_t)kb * BK);
+        if (left < BK) {                                                 // the last block of the rows: zero past the end
+            for (int q = threadIdx.x; q < PIECES; q += THREADS)
+                if (q % SUB / 12 >= left) reinterpret_cast<u32x4*>(t)[q] = u32x4{0, 0, 0, 0};
+            block_barrier();
+        }
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) {
+            u32x4 a[MT], b[NT];
+#pragma unroll
+            for (int i = 0; i < MT; ++i) {
+                const int col = (wm * MT + i) * 32;
+                a[i] = down_operand(t + col / 96 * SUB * 8, col % 96, ks);
+            }
+#pragma unroll
+            for (int j = 0; j < NT; ++j) b[j] = down_operand(t + (BM / 96 + wn) * SUB * 8, j * 32, ks);
+            if (sums_here) {
+#pragma unroll
+                for (int i = 0; i < MT; ++i) {
+                    float s = 0.f;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) s += half_of<T>(a[i][e], 0) + half_of<T>(a[i][e], 1);
+                    bs[i] += s;
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < MT; ++i)
+#pragma unroll
+                for (int j = 0; j < NT; ++j) acc[i][j] = Op<T>::mfma(a[i], b[j], acc[i][j]);
+        }
+    }
+    float* pw = part_w + chunk * (int64_t)P * K;
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int pp = p0 + (wm * MT + i) * 32 + acc_row(r, half), kk = k0 + wn * 96 + j * 32 + l32;
+                if (pp < P && kk < K) pw[(int64_t)pp * K + kk] = acc[i][j][r];
+            }
+        if (sums_here) {
+            const float s = bs[i] + __shfl_xor(bs[i], 32, 64);           // the two halves of the reduction slots
+            const int pp = p0 + (wm * MT + i) * 32 + l32;
+            if (half == 0 && pp < P) part_b[chunk * P + pp] = s;
+        }
     }
 }
 
@@ -336,8 +648,8 @@ __global__ __launch_bounds__(WM * 64) __attribute__((amdgpu_waves_per_eu(OCC, OC
 // and add their tiles through LDS in a fixed order.
 // ------------------------------------------------------------------------------------------
 constexpr int SMALL_WAVES = 8;
-template <typename T, typename TB, typename TO, int EPI, bool DOWN>
-__global__ __launch_bounds__(SMALL_WAVES * 64) void dense_small_kernel(const T* __restrict__ x, int64_t N, int K, const TB* __restrict__ w, int P,
+template <typename T, typename TO, int EPI, bool DOWN>
+__global__ __launch_bounds__(SMALL_WAVES * 64) void dense_small_kernel(const T* __restrict__ x, int64_t N, int K, const T* __restrict__ w, int P,
                                                                     int groups, Epilogue ep) {
     constexpr int PL = Op<T>::PL;
     __shared__ __attribute__((aligned(16))) float sums[SMALL_WAVES][32 * 36];
@@ -350,8 +662,8 @@ __global__ __launch_bounds__(SMALL_WAVES * 64) void dense_small_kernel(const T* 
     const T* xp = x + row * K + half * 8;
     f32x16 acc = f32x16{0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
     constexpr int AHEAD = 3;                                             // steps of a wavefront in flight
-    Along<T, T> ra[AHEAD];
-    Along<T, TB> rb[DOWN ? 1 : AHEAD];
+    Along<T> ra[AHEAD];
+    Along<T> rb[DOWN ? 1 : AHEAD];
     float vb[DOWN ? AHEAD : 1][8];
     auto request = [&](int slot, int s) {
         ra[slot].load(xp + s * 16);
@@ -385,25 +697,28 @@ __global__ __launch_bounds__(SMALL_WAVES * 64) void dense_small_kernel(const T* 
     __syncthreads();
     if (threadIdx.x < 256) {
         const int rr = threadIdx.x >> 3, cc = (threadIdx.x & 7) * 4;
+        const bool in = row0 + rr < N && col0 + cc < P;
+        Second4<T, TO, EPI> second;
+        if (in) second.load(ep, row0 + rr, col0 + cc, P);
         f32x4 v = *reinterpret_cast<const f32x4*>(&sums[0][rr * 36 + cc]);
 #pragma unroll
         for (int q = 1; q < SMALL_WAVES; ++q) v += *reinterpret_cast<const f32x4*>(&sums[q][rr * 36 + cc]);
-        if (row0 + rr < N && col0 + cc < P) finish4<T, TB, TO, EPI>(ep, row0 + rr, col0 + cc, P, v);
+        if (in) finish4<T, TO, EPI>(ep, row0 + rr, col0 + cc, P, v, second);
     }
 }
 
 // ------------------------------------------------------------------------------------------
 // dW [P, K] = dY^T X, db [P] = column sums of dY.  A workgroup owns BM x BN of dW for one chunk of rows.
 // ------------------------------------------------------------------------------------------
-template <typename T, int WM, int WN, int MT, int NT, int OCC>
-__global__ __launch_bounds__(WM * WN * 64) __attribute__((amdgpu_waves_per_eu(OCC, OCC))) void dense_wgrad_kernel(const T* __restrict__ dy, const T* __restrict__ x, int64_t N, int P, int K,
-                                                                   int tiles_p, int tiles_k, int64_t rows_per_chunk, float* __restrict__ part_w,
-                                                                   float* __restrict__ part_b) {
-    constexpr int PL = Op<T>::PL, BK = PL == 3 ? 16 : 32, KS = BK / 16, KC = BK / 8;
+template <int WM, int WN, int MT, int NT, int OCC>
+__global__ __launch_bounds__(WM * WN * 64) __attribute__((amdgpu_waves_per_eu(OCC, OCC))) void dense_wgrad_kernel(
+    const float* __restrict__ dy, const float* __restrict__ x, int64_t N, int P, int K, int tiles_p, int tiles_k, int64_t rows_per_chunk,
+    float* __restrict__ part_w, float* __restrict__ part_b) {
+    constexpr int PL = 3, BK = 16, KC = BK / 8;
     constexpr int BM = WM * MT * 32, BN = WN * NT * 32, THREADS = WM * WN * 64;
     constexpr int A_UNITS = BM / 2 * KC, UA = (A_UNITS + THREADS - 1) / THREADS;
     constexpr int B_UNITS = BN / 2 * KC, UB = (B_UNITS + THREADS - 1) / THREADS;
-    constexpr int A_LDS = KS * (BM / 32) * PL * 64, B_LDS = KS * (BN / 32) * PL * 64, BUF = A_LDS + B_LDS;
+    constexpr int A_LDS = BM / 32 * PL * 64, B_LDS = BN / 32 * PL * 64, BUF = A_LDS + B_LDS;
     extern __shared__ __attribute__((aligned(16))) u32x4 lds[];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, half = lane >> 5, l32 = lane & 31;
     const int wm = wave / WN, wn = wave % WN;
@@ -414,7 +729,7 @@ __global__ __launch_bounds__(WM * WN * 64) __attribute__((amdgpu_waves_per_eu(OC
     const int64_t begin = chunk * rows_per_chunk, end = begin + rows_per_chunk < N ? begin + rows_per_chunk : N;
     const bool sums_here = part_b && k0 == 0;
 
-    Down<T, T> ra[UA], rx[UB];
+    Down ra[UA], rx[UB];
     float bs[UA][2];
 #pragma unroll
     for (int i = 0; i < UA; ++i) bs[i][0] = bs[i][1] = 0.f;
@@ -430,8 +745,8 @@ __global__ __launch_bounds__(WM * WN * 64) __attribute__((amdgpu_waves_per_eu(OC
         ox[i] = (uint32_t)((u / (BN / 2)) * 8 * K + min(k0 + (u % (BN / 2)) * 2, K - 2));
     }
     auto request = [&](int64_t n0) {
-        const T* yb = dy + n0 * P;
-        const T* xb = x + n0 * K;
+        const float* yb = dy + n0 * P;
+        const float* xb = x + n0 * K;
         if (n0 + BK <= end) {
 #pragma unroll
             for (int i = 0; i < UA; ++i)
@@ -511,25 +826,22 @@ __global__ __launch_bounds__(WM * WN * 64) __attribute__((amdgpu_waves_per_eu(OC
         __syncthreads();
         if (kb + 1 < nk) request(begin + (int64_t)(kb + 1) * BK);
         const u32x4* buf = lds + (kb & 1) * BUF;
+        u32x4 a[MT][PL], b[NT][PL];
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-            u32x4 a[MT][PL], b[NT][PL];
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+            for (int q = 0; q < PL; ++q) a[i][q] = buf[((wm * MT + i) * PL + q) * 64 + lane];
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+#pragma unroll
+            for (int q = 0; q < PL; ++q) b[j][q] = buf[A_LDS + ((wn * NT + j) * PL + q) * 64 + lane];
+#pragma unroll
+        for (int p = 0; p < Op<float>::NP; ++p)
 #pragma unroll
             for (int i = 0; i < MT; ++i)
 #pragma unroll
-                for (int q = 0; q < PL; ++q) a[i][q] = buf[((ks * (BM / 32) + wm * MT + i) * PL + q) * 64 + lane];
-#pragma unroll
-            for (int j = 0; j < NT; ++j)
-#pragma unroll
-                for (int q = 0; q < PL; ++q) b[j][q] = buf[A_LDS + ((ks * (BN / 32) + wn * NT + j) * PL + q) * 64 + lane];
-#pragma unroll
-            for (int p = 0; p < Op<T>::NP; ++p)
-#pragma unroll
-                for (int i = 0; i < MT; ++i)
-#pragma unroll
-                    for (int j = 0; j < NT; ++j) acc[i][j] = Op<T>::mfma(a[i][Op<T>::PA[p]], b[j][Op<T>::PB[p]], acc[i][j]);
-            __builtin_amdgcn_sched_barrier(0);                           // operands of later steps stay out of registers
-        }
+                for (int j = 0; j < NT; ++j) acc[i][j] = Op<float>::mfma(a[i][Op<float>::PA[p]], b[j][Op<float>::PB[p]], acc[i][j]);
+        __builtin_amdgcn_sched_barrier(0);                               // the next operands' splitting stays behind the products
         if (kb + 1 < nk) store(lds + ((kb + 1) & 1) * BUF);
     }
     float* pw = part_w + chunk * (int64_t)P * K;
@@ -675,12 +987,20 @@ template <typename F> static int allow_lds(F* kernel, size_t bytes) {
     return 0;
 }
 
-template <typename T, typename TB, typename TO, int EPI, bool DOWN, int WM, int MT, int OCC>
-static int launch_rows(const T* x, int64_t N, int K, const TB* w, int P, const Epilogue& ep, hipStream_t s) {
-    constexpr int PL = Op<T>::PL, BK = PL == 3 ? 16 : 48, BM = WM * MT * 32;
-    constexpr size_t tiles = 2 * (size_t)(BK / 16) * (BM / 32 + 3) * PL * 64 * 16, out = (size_t)WM * 32 * 100 * 4;
+template <typename T, typename TO, int EPI>
+static int launch_parts(const float* part, int64_t N, int P, int parts, const Epilogue& ep, hipStream_t s) {
+    const int64_t blocks = (N * (P / 4) + 255) / 256;
+    SSWIN_CHECK(blocks < (1ll << 31), "dense: too many rows");
+    hipLaunchKernelGGL((dense_parts_kernel<T, TO, EPI>), dim3((unsigned)blocks), dim3(256), 0, s, part, N, P, parts, ep);
+    return launch_ok("dense, parts");
+}
+
+template <int EPI, bool DOWN, int WM, int MT, int OCC>
+static int launch_rows(const float* x, int64_t N, int K, const float* w, int P, const Epilogue& ep, hipStream_t s) {
+    constexpr int BM = WM * MT * 32;
+    constexpr size_t tiles = 2 * (size_t)(BM / 32 + 3) * 3 * 64 * 16, out = (size_t)WM * 32 * 100 * 4;
     constexpr size_t bytes = tiles > out ? tiles : out;
-    auto* k = dense_rows_kernel<T, TB, TO, EPI, DOWN, WM, MT, OCC>;
+    auto* k = dense_rows_kernel<EPI, DOWN, WM, MT, OCC>;
     static const int configured = allow_lds(k, bytes);
     if (configured) return configured;
     const int groups = (P + 95) / 96;
@@ -690,35 +1010,94 @@ static int launch_rows(const T* x, int64_t N, int K, const TB* w, int P, const E
     return launch_ok("dense");
 }
 
-template <typename T, typename TB, typename TO, int EPI, bool DOWN>
-static int launch_forward(const void* x, int64_t N, int K, const void* w, int P, const Epilogue& ep, hipStream_t s) {
+template <typename T, typename TO, int EPI, bool DOWN, int BK, int WM, int WN, int KG, int MT, int STAGES, int OCC>
+static int launch_rows16(const T* x, int64_t N, int K, const T* w, int P, int ksplit, float* ws, const Epilogue& ep, hipStream_t s) {
+    constexpr int BM = WM * MT * 32, BN = WN * 96;
+    constexpr size_t tiles = STAGES * (size_t)(BM + BN) * BK * 2, out = (size_t)WM * WN * (KG == 2 ? MT * 96 : 36) * 32 * 4;
+    constexpr size_t bytes = tiles > out ? tiles : out;
+    auto* k = dense16_rows_kernel<T, TO, EPI, DOWN, BK, WM, WN, KG, MT, STAGES, OCC>;
+    static const int configured = allow_lds(k, bytes);
+    if (configured) return configured;
+    const int groups = (P + BN - 1) / BN;
+    const int64_t blocks = (N + BM - 1) / BM * groups * ksplit;
+    SSWIN_CHECK(blocks < (1ll << 31), "dense: too many rows");
+    hipLaunchKernelGGL(k, dim3((unsigned)blocks), dim3(WM * WN * KG * 64), bytes, s, x, N, K, w, P, groups, ksplit, ksplit > 1 ? ws : nullptr, ep);
+    if (int rc = launch_ok("dense, 16 bit")) return rc;
+    return ksplit > 1 ? launch_parts<T, TO, EPI>(ws, N, P, ksplit, ep, s) : 0;
+}
+
+// How a product is cut.
+//   few rows: 32 x 32 tiles while the workgroups of the larger tiles would leave most of the chip idle.  fp32: below 150 tiles of
+//     128 x 96.  16 bit: the tiles' own time grows with the reduction, so the line is tiles x K: 500 rows 768 -> 768 (24 576)
+//     7.8 us against 12.2, 1364 rows 768 -> 768 (67 584) 15.5 against 12.6, 2000 rows 1152 -> 384 (73 728) 15.5 against 13.8.
+//   ksplit (16 bit): shares of the reduction, each at least 576 long, while the tiles alone do not fill the chip: 1364 rows
+//     3072 -> 768 (88 tiles) 36 us with one share, 24 with two, 23 with four; 2729 rows (176 tiles) 37, 33 and 36.
+struct Cut {
+    bool few;
+    int ksplit;
+};
+static Cut cut_of(int dtype, int64_t N, int K, int P) {
+    const int64_t tiles = (N + 127) / 128 * ((P + 95) / 96);
+    if (dtype == SSWIN_F32) return {tiles < 150, 1};
+    if (tiles * K <= 50000) return {true, 1};
+    const int64_t shares = std::min<int64_t>({4, 400 / tiles, K / 576});
+    return {false, (int)std::max<int64_t>(shares, 1)};
+}
+
+template <typename T, typename TO, int EPI, bool DOWN>
+static int launch_forward(const void* x, int64_t N, int K, const void* w, int P, const Epilogue& ep, float* ws, size_t ws_bytes, hipStream_t s) {
     const T* xp = static_cast<const T*>(x);
-    const TB* wp = static_cast<const TB*>(w);
-    const int64_t small_blocks = (N + 31) / 32 * ((P + 31) / 32);
-    // 128-row workgroups hide the latency of a step only from about 150 of them on: bf16 384 -> 1152 at 300 rows 5.3 us in 32 x 32
-    // tiles and 10.7 here, at 2000 rows (192 workgroups) 15.9 and 11.6; fp32 96 -> 96 at 8000 rows (63) 5.7 and 9.5, at 16000 equal
-    if ((N + 127) / 128 * ((P + 95) / 96) < 150 && small_blocks < (1ll << 31)) {
-        hipLaunchKernelGGL((dense_small_kernel<T, TB, TO, EPI, DOWN>), dim3((unsigned)small_blocks), dim3(SMALL_WAVES * 64), 0, s, xp, N, K, wp, P,
+    const T* wp = static_cast<const T*>(w);
+    const int64_t few_blocks = (N + 31) / 32 * ((P + 31) / 32);
+    Cut cut = cut_of(Op<T>::PL == 3 ? SSWIN_F32 : SSWIN_F16, N, K, P);
+    if (cut.few && few_blocks < (1ll << 31)) {
+        hipLaunchKernelGGL((dense_small_kernel<T, TO, EPI, DOWN>), dim3((unsigned)few_blocks), dim3(SMALL_WAVES * 64), 0, s, xp, N, K, wp, P,
                            (P + 31) / 32, ep);
         return launch_ok("dense, few rows");
     }
-    // fp32 and 96 channels: the kernel that keeps Wop in LDS (219 000 rows, 96 -> 288: 89 us against 120 here, with a residual 133
-    // and 202)
-    if constexpr (Op<T>::PL == 3)
+    if constexpr (Op<T>::PL == 3) {
+        // 96 channels: the kernel that keeps Wop in LDS (219 000 rows, 96 -> 288: 89 us against 120 here, with a residual 133 and 202)
         if (K == 96 && P % 96 == 0) return staged_layer_96(xp, N, wp, P, DOWN, EPI, ep, s);
-    // wavefronts per SIMD: what the registers allow without spilling (four: forward equal, input gradient 89 us against 40)
-    return launch_rows<T, TB, TO, EPI, DOWN, 4, 1, 3>(xp, N, K, wp, P, ep, s);
+        // wavefronts per SIMD: what the registers allow without spilling (four: forward equal, input gradient 89 us against 40)
+        return launch_rows<EPI, DOWN, 4, 1, 3>(xp, N, K, wp, P, ep, s);
+    } else {
+        if (ws_bytes < (size_t)cut.ksplit * N * P * sizeof(float)) cut.ksplit = 1;
+        const int64_t rows = (N + 127) / 128, tiles = rows * ((P + 95) / 96) * cut.ksplit;
+        // long reductions into many columns: fewest bytes through LDS (8119 rows, 768 -> 3072: 57 us against 70 with the next two)
+        if (K >= 384 && P % 192 == 0 && rows * (P / 192) >= 512) return launch_rows16<T, TO, EPI, DOWN, 64, 2, 2, 1, 2, 2, 2>(xp, N, K, wp, P, 1, ws, ep, s);
+        // up to two workgroups a compute unit: eight wavefronts each (8119 rows, 1536 -> 384: 22 us against 30), above that five
+        // workgroups of four, whose loads and stores overlap (219 000 rows, 96 -> 288: 44 us against 80)
+        if (tiles <= 512) return launch_rows16<T, TO, EPI, DOWN, 64, 4, 1, 2, 1, 2, 4>(xp, N, K, wp, P, cut.ksplit, ws, ep, s);
+        return launch_rows16<T, TO, EPI, DOWN, 32, 4, 1, 1, 1, 2, 5>(xp, N, K, wp, P, 1, ws, ep, s);
+    }
 }
 
-template <typename T, typename TB, typename TO>
-static int pick_forward(int epi, bool down, const void* x, int64_t N, int K, const void* w, int P, const Epilogue& ep, hipStream_t s) {
+template <typename T, typename TO>
+static int pick_forward(int epi, bool down, const void* x, int64_t N, int K, const void* w, int P, const Epilogue& ep, float* ws, size_t ws_bytes, hipStream_t s) {
     if (down) {
-        if (epi == EPI_NONE) return launch_forward<T, TB, TO, EPI_NONE, true>(x, N, K, w, P, ep, s);
-        return launch_forward<T, TB, TO, EPI_SCALE, true>(x, N, K, w, P, ep, s);
+        if (epi == EPI_NONE) return launch_forward<T, TO, EPI_NONE, true>(x, N, K, w, P, ep, ws, ws_bytes, s);
+        return launch_forward<T, TO, EPI_SCALE, true>(x, N, K, w, P, ep, ws, ws_bytes, s);
     }
-    if (epi == EPI_NONE) return launch_forward<T, TB, TO, EPI_NONE, false>(x, N, K, w, P, ep, s);
-    if (epi == EPI_GELU) return launch_forward<T, TB, TO, EPI_GELU, false>(x, N, K, w, P, ep, s);
-    return launch_forward<T, TB, TO, EPI_RESIDUAL, false>(x, N, K, w, P, ep, s);
+    if (epi == EPI_NONE) return launch_forward<T, TO, EPI_NONE, false>(x, N, K, w, P, ep, ws, ws_bytes, s);
+    if (epi == EPI_GELU) return launch_forward<T, TO, EPI_GELU, false>(x, N, K, w, P, ep, ws, ws_bytes, s);
+    return launch_forward<T, TO, EPI_RESIDUAL, false>(x, N, K, w, P, ep, ws, ws_bytes, s);
+}
+
+// fp32 parameters of a block in the tokens' type, one launch for all of them (a launch each: about 4 us x 8)
+struct CastParts {
+    const float* src[SSWIN_CAST_PARTS];
+    int64_t first[SSWIN_CAST_PARTS + 1];                                 // of each in the destination, in pieces of 8 values
+};
+template <typename T> __global__ __launch_bounds__(256) void cast_parts_kernel(CastParts p, int count, T* __restrict__ dst) {
+    const int64_t piece = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (piece >= p.first[count]) return;
+    int which = 0;
+    while (piece >= p.first[which + 1]) ++which;
+    const f32x4* src = reinterpret_cast<const f32x4*>(p.src[which] + (piece - p.first[which]) * 8);
+    const f32x4 a = src[0], b = src[1];
+    u32x4 out;
+    out[0] = pack2<T>(a[0], a[1]), out[1] = pack2<T>(a[2], a[3]), out[2] = pack2<T>(b[0], b[1]), out[3] = pack2<T>(b[2], b[3]);
+    reinterpret_cast<u32x4*>(dst)[piece] = out;
 }
 
 // tiles of dW and row chunks: about `per_cu` workgroups per compute unit
@@ -740,24 +1119,20 @@ static WgradPlan wgrad_plan(int64_t N, int P, int K, int bk, int bm, int bn, int
 
 // rows up to which one launch of 32 x 32 tiles beats row chunks and their sums (284 rows 384 -> 1152: 19 us in chunks)
 constexpr int64_t WGRAD_SMALL_ROWS = 1024;
-// 128 x 192 tiles where dW has that many columns, otherwise 96 x 96 with more workgroups per compute unit: bf16, 219 000 rows
-// 96 -> 288: 48 us in 96 x 96, 73 in 128 x 192; 8 119 rows 768 -> 2304: 107 and 77; fp32 35 569 rows 192 -> 576: 91 and 78
+// fp32: 128 x 192 tiles where dW has that many columns, otherwise 96 x 96 with more workgroups per compute unit (35 569 rows
+// 192 -> 576: 91 and 78 us).  16 bit: 96 x 96 (219 000 rows 96 -> 288: 39 us; 192 x 192 tiles 58, 192 x 96 44).
 static bool wgrad_large(int K) { return K >= 192; }
 static WgradPlan wgrad_plan(int dtype, int64_t N, int P, int K) {
-    const int bk = dtype == SSWIN_F32 ? 16 : 32;
-    return wgrad_large(K) ? wgrad_plan(N, P, K, bk, 128, 192, 2) : wgrad_plan(N, P, K, bk, 96, 96, 4);
+    if (dtype == SSWIN_F32) return wgrad_large(K) ? wgrad_plan(N, P, K, 16, 128, 192, 2) : wgrad_plan(N, P, K, 16, 96, 96, 4);
+    return wgrad_plan(N, P, K, 32, 96, 96, 3);
 }
 
-template <typename T, typename TO, int WM, int WN, int MT, int NT, int OCC>
-static int launch_wgrad_as(const WgradPlan& pl, const void* dy, const void* x, int64_t N, int P, int K, void* dw, void* db, float* ws, hipStream_t s) {
-    constexpr int PL = Op<T>::PL, BK = PL == 3 ? 16 : 32;
-    constexpr size_t bytes = 2 * (size_t)(BK / 16) * (WM * MT + WN * NT) * PL * 64 * 16;
-    auto* k = dense_wgrad_kernel<T, WM, WN, MT, NT, OCC>;
-    static const int configured = allow_lds(k, bytes);
-    if (configured) return configured;
+template <typename T, typename TO, typename F>
+static int launch_wgrad_as(F* k, int threads, size_t lds, const WgradPlan& pl, const void* dy, const void* x, int64_t N, int P, int K, void* dw, void* db,
+                           float* ws, hipStream_t s) {
     float* part_b = ws + (size_t)pl.chunks * P * K;
-    hipLaunchKernelGGL(k, dim3((unsigned)(pl.tiles_p * pl.tiles_k * pl.chunks)), dim3(WM * WN * 64), bytes, s, static_cast<const T*>(dy),
-                       static_cast<const T*>(x), N, P, K, pl.tiles_p, pl.tiles_k, pl.rows, ws, db ? part_b : nullptr);
+    hipLaunchKernelGGL(k, dim3((unsigned)(pl.tiles_p * pl.tiles_k * pl.chunks)), dim3(threads), lds, s, static_cast<const T*>(dy), static_cast<const T*>(x), N,
+                       P, K, pl.tiles_p, pl.tiles_k, pl.rows, ws, db ? part_b : nullptr);
     if (int rc = launch_ok("dense weight gradient")) return rc;
     const int64_t PK = (int64_t)P * K;
     hipLaunchKernelGGL((dense_wgrad_sum_kernel<TO>), dim3((unsigned)((PK + P + 63) / 64)), dim3(256), 0, s, ws, part_b, pl.chunks, PK, P,
@@ -773,9 +1148,15 @@ static int launch_wgrad(const void* dy, const void* x, int64_t N, int P, int K, 
                            static_cast<const T*>(x), N, P, K, tk, static_cast<TO*>(dw), static_cast<TO*>(db));
         return launch_ok("dense weight gradient, few rows");
     }
-    const WgradPlan pl = wgrad_plan(Op<T>::PL == 3 ? SSWIN_F32 : SSWIN_F16, N, P, K);
-    if (wgrad_large(K)) return launch_wgrad_as<T, TO, 2, 2, 2, 3, 2>(pl, dy, x, N, P, K, dw, db, ws, s);
-    return launch_wgrad_as<T, TO, 3, 1, 1, 3, 3>(pl, dy, x, N, P, K, dw, db, ws, s);
+    if constexpr (Op<T>::PL == 3) {
+        const WgradPlan pl = wgrad_plan(SSWIN_F32, N, P, K);
+        constexpr size_t large = 2 * (2 * 2 + 2 * 3) * 3 * 1024, plain = 2 * (3 + 3) * 3 * 1024;         // two buffers of (row tiles) x 3 planes
+        if (wgrad_large(K)) return launch_wgrad_as<T, TO>(dense_wgrad_kernel<2, 2, 2, 3, 2>, 256, large, pl, dy, x, N, P, K, dw, db, ws, s);
+        return launch_wgrad_as<T, TO>(dense_wgrad_kernel<3, 1, 1, 3, 3>, 192, plain, pl, dy, x, N, P, K, dw, db, ws, s);
+    } else {
+        constexpr size_t lds = 3 * 2 * 32 * 192;                         // three stages of two tiles of 32 x 96
+        return launch_wgrad_as<T, TO>(dense16_wgrad_kernel<T, 3, 1, 1, 3, 3>, 192, lds, wgrad_plan(SSWIN_F16, N, P, K), dy, x, N, P, K, dw, db, ws, s);
+    }
 }
 
 }  // namespace dense
@@ -790,8 +1171,14 @@ int sswin_dense_supported(int dtype, int P, int K) {
     return (dtype == SSWIN_F32 || dtype == SSWIN_F16 || dtype == SSWIN_BF16) && P > 0 && K > 0 && P % 16 == 0 && K % 16 == 0;
 }
 
-int sswin_dense_forward(int dtype, int w_dtype, int out_dtype, int transposed, int epilogue, const void* x, int64_t N, int K, const void* w, const void* bias,
-                        int P, const void* extra, void* y, void* slope, void* stream) {
+size_t sswin_dense_forward_workspace_bytes(int dtype, int64_t N, int K, int P) {
+    if (N <= 0 || !sswin_dense_supported(dtype, P, K)) return 0;
+    const Cut c = cut_of(dtype, N, K, P);
+    return c.ksplit > 1 ? (size_t)c.ksplit * N * P * sizeof(float) : 0;
+}
+
+int sswin_dense_forward(int dtype, int out_dtype, int transposed, int epilogue, const void* x, int64_t N, int K, const void* w, const void* bias,
+                        int P, const void* extra, void* y, void* slope, void* ws, size_t ws_bytes, void* stream) {
     SSWIN_CHECK(N >= 0, "dense_forward: bad sizes");
     SSWIN_CHECK(sswin_dense_supported(dtype, P, K), "dense_forward: %d -> %d channels of type %d are not supported (multiples of 16)", K, P, dtype);
     SSWIN_CHECK(epilogue >= 0 && epilogue <= 3, "dense_forward: epilogue %d", epilogue);
@@ -803,22 +1190,41 @@ int sswin_dense_forward(int dtype, int w_dtype, int out_dtype, int transposed, i
     SSWIN_CHECK(((uintptr_t)x | (uintptr_t)w | (uintptr_t)bias | (uintptr_t)extra | (uintptr_t)y | (uintptr_t)slope) % 16 == 0,
                 "dense_forward: pointers must be 16-byte aligned");
     const Epilogue ep = {bias, extra, y, slope};
+    SSWIN_CHECK(((uintptr_t)ws) % 16 == 0, "dense_forward: the workspace must be 16-byte aligned");
+    float* f = static_cast<float*>(ws);
     hipStream_t s = static_cast<hipStream_t>(stream);
     const bool down = transposed != 0;
-#define DENSE_RUN(T, TB, TO) return pick_forward<T, TB, TO>(epilogue, down, x, N, K, w, P, ep, s)
-    if (dtype == SSWIN_F32 && w_dtype == SSWIN_F32 && out_dtype == SSWIN_F32) DENSE_RUN(float, float, float);
-    if (dtype == SSWIN_F16 && w_dtype == SSWIN_F16 && out_dtype == SSWIN_F16) DENSE_RUN(__half, __half, __half);
-    if (dtype == SSWIN_BF16 && w_dtype == SSWIN_BF16 && out_dtype == SSWIN_BF16) DENSE_RUN(__hip_bfloat16, __hip_bfloat16, __hip_bfloat16);
-    if (dtype == SSWIN_F16 && w_dtype == SSWIN_F32 && out_dtype == SSWIN_F16) DENSE_RUN(__half, float, __half);
-    if (dtype == SSWIN_BF16 && w_dtype == SSWIN_F32 && out_dtype == SSWIN_BF16) DENSE_RUN(__hip_bfloat16, float, __hip_bfloat16);
+#define DENSE_RUN(T, TO) return pick_forward<T, TO>(epilogue, down, x, N, K, w, P, ep, f, ws_bytes, s)
+    if (dtype == SSWIN_F32 && out_dtype == SSWIN_F32) DENSE_RUN(float, float);
+    if (dtype == SSWIN_F16 && out_dtype == SSWIN_F16) DENSE_RUN(__half, __half);
+    if (dtype == SSWIN_BF16 && out_dtype == SSWIN_BF16) DENSE_RUN(__hip_bfloat16, __hip_bfloat16);
     if (epilogue == EPI_RESIDUAL) {                                      // mixed precision: the residual stream stays fp32
-        if (dtype == SSWIN_F16 && w_dtype == SSWIN_F32 && out_dtype == SSWIN_F32)
-            return launch_forward<__half, float, float, EPI_RESIDUAL, false>(x, N, K, w, P, ep, s);
-        if (dtype == SSWIN_BF16 && w_dtype == SSWIN_F32 && out_dtype == SSWIN_F32)
-            return launch_forward<__hip_bfloat16, float, float, EPI_RESIDUAL, false>(x, N, K, w, P, ep, s);
+        if (dtype == SSWIN_F16 && out_dtype == SSWIN_F32) return launch_forward<__half, float, EPI_RESIDUAL, false>(x, N, K, w, P, ep, f, ws_bytes, s);
+        if (dtype == SSWIN_BF16 && out_dtype == SSWIN_F32)
+            return launch_forward<__hip_bfloat16, float, EPI_RESIDUAL, false>(x, N, K, w, P, ep, f, ws_bytes, s);
     }
 #undef DENSE_RUN
-    return fail("dense_forward: tokens of type %d with weights of type %d and a result of type %d are not supported", dtype, w_dtype, out_dtype);
+    return fail("dense_forward: operands of type %d with a result of type %d are not supported", dtype, out_dtype);
+}
+
+int sswin_cast_parts(int dtype, const void* const* src, const int64_t* sizes, int count, void* dst, void* stream) {
+    SSWIN_CHECK(count >= 1 && count <= SSWIN_CAST_PARTS && src && sizes && dst, "cast_parts: 1 to %d parts", SSWIN_CAST_PARTS);
+    SSWIN_CHECK(dtype == SSWIN_F16 || dtype == SSWIN_BF16, "cast_parts: type %d", dtype);
+    CastParts p;
+    p.first[0] = 0;
+    for (int i = 0; i < count; ++i) {
+        SSWIN_CHECK(src[i] && sizes[i] >= 0 && sizes[i] % 8 == 0 && (uintptr_t)src[i] % 16 == 0, "cast_parts: parts are multiples of 8 values, 16-byte aligned");
+        p.src[i] = static_cast<const float*>(src[i]);
+        p.first[i + 1] = p.first[i] + sizes[i] / 8;
+    }
+    SSWIN_CHECK((uintptr_t)dst % 16 == 0, "cast_parts: pointers must be 16-byte aligned");
+    const int64_t blocks = (p.first[count] + 255) / 256;
+    SSWIN_CHECK(blocks < (1ll << 31), "cast_parts: too many values");
+    if (blocks == 0) return 0;
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    if (dtype == SSWIN_F16) hipLaunchKernelGGL((cast_parts_kernel<__half>), dim3((unsigned)blocks), dim3(256), 0, s, p, count, static_cast<__half*>(dst));
+    else hipLaunchKernelGGL((cast_parts_kernel<__hip_bfloat16>), dim3((unsigned)blocks), dim3(256), 0, s, p, count, static_cast<__hip_bfloat16*>(dst));
+    return launch_ok("cast_parts");
 }
 
 size_t sswin_dense_weight_grad_workspace_bytes(int dtype, int64_t N, int P, int K) {

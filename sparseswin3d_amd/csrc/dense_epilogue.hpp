@@ -18,20 +18,34 @@ enum { EPI_NONE = SSWIN_DENSE_PLAIN, EPI_GELU = SSWIN_DENSE_GELU, EPI_RESIDUAL =
 // ------------------------------------------------------------------------------------------
 // the last step on four consecutive columns of a row
 // ------------------------------------------------------------------------------------------
+// u Phi(u) and its derivative.  1 - Phi(|u|) = exp(-u^2/2) Q(t), t = 1/(1 + c|u|) (Hastings' form); for fp32 results and
+// |u| < 1 Phi = 1/2 + u R(u^2).  Q and R are least squares fits made for this file (to 1.4e-8 and 3e-10).  fp32: Phi to 9e-8,
+// u Phi to 4e-7 up to |u| = 12, as the form with erff; 16 bit (Q alone): 2.3e-7 and 4e-7, a thousandth of their rounding.
+// No branch, and the exponential serves both results: with erff the vector units bound the feed-forward layers (219 000 rows
+// 96 -> 384 bf16 with the derivative: 171 us, without the step 53).
+template <bool WIDE>
 __device__ __forceinline__ void gelu_and_slope(float u, float& g, float& d) {
-    const float cdf = 0.5f * (1.f + erff(u * 0.70710678118654752f));
+    const float a = fabsf(u), s = u * u, e = __builtin_amdgcn_exp2f(s * -0.72134752044f), t = __builtin_amdgcn_rcpf(fmaf(a, 0.282842726f, 1.f));
+    float q = fmaf(-0.100168057f, t, 0.354737073f);
+    q = fmaf(fmaf(fmaf(fmaf(q, t, -0.185730487f), t, 0.234369889f), t, 0.080814302f), t, 0.115977287f) * t * e;
+    float cdf = u < 0.f ? q : 1.f - q;
+    if constexpr (WIDE) {
+        float r = fmaf(-7.66468293e-06f, s, 0.000113512666f);
+        r = fmaf(fmaf(fmaf(fmaf(r, s, -0.00118635304f), s, 0.00997333135f), s, -0.0664903596f), s, 0.398942292f);
+        cdf = a < 1.f ? fmaf(u, r, 0.5f) : cdf;
+    }
     g = u * cdf;
-    d = cdf + u * 0.3989422804014327f * __expf(-0.5f * u * u);
+    d = fmaf(u * 0.3989422804014327f, e, cdf);
 }
 
 // one value: what follows the product, with its column's bias already added
-template <int EPI>
+template <int EPI, bool WIDE = true>
 __device__ __forceinline__ float finish1(float v, float extra, float& slope) {
     if constexpr (EPI == EPI_RESIDUAL) return v + extra;
     if constexpr (EPI == EPI_SCALE) return v * extra;
     if constexpr (EPI == EPI_GELU) {
         float g;
-        gelu_and_slope(v, g, slope);
+        gelu_and_slope<WIDE>(v, g, slope);
         return g;
     }
     return v;
@@ -39,44 +53,60 @@ __device__ __forceinline__ float finish1(float v, float extra, float& slope) {
 
 template <typename T> struct alignas(sizeof(T) * 4) Vec4 { T v[4]; };
 
+template <typename T> __device__ __forceinline__ uint32_t pack2(float a, float b);
+template <> __device__ __forceinline__ uint32_t pack2<__half>(float a, float b) {
+    return (uint32_t)__half_as_ushort(__float2half(a)) | ((uint32_t)__half_as_ushort(__float2half(b)) << 16);
+}
+template <> __device__ __forceinline__ uint32_t pack2<__hip_bfloat16>(float a, float b) {
+    return pack_bf16(a, b);
+}
+template <typename T> __device__ __forceinline__ Vec4<T> pack4(const float (&v)[4]) {
+    if constexpr (sizeof(T) == 4) {
+        return Vec4<T>{v[0], v[1], v[2], v[3]};
+    } else {
+        struct { uint32_t a, b; } w = {pack2<T>(v[0], v[1]), pack2<T>(v[2], v[3])};
+        return __builtin_bit_cast(Vec4<T>, w);
+    }
+}
+
 struct Epilogue {
-    const void* bias;       // [P] of the weights' type, or null
+    const void* bias;       // [P] of the operands' type, or null
     const void* extra;      // residual [N, P] (type of y) or factor [N, P] (type of the tokens)
     void* y;                // [N, P]
     void* slope;            // GELU: its derivative [N, P] (type of y), or null
 };
 
-template <typename T, typename TB, typename TO, int EPI>
-__device__ __forceinline__ void finish4(const Epilogue& ep, int64_t row, int col, int P, const f32x4& acc) {
+// residual or factor of four consecutive columns (loaded ahead of the last step, which would wait for it)
+template <typename T, typename TO, int EPI> struct Second4 {
+    static constexpr bool USED = EPI == EPI_RESIDUAL || EPI == EPI_SCALE;
+    using TE = typename std::conditional<EPI == EPI_SCALE, T, TO>::type;
+    Vec4<TE> r;
+    __device__ __forceinline__ void load(const Epilogue& ep, int64_t row, int col, int P) {
+        if constexpr (USED) r = *reinterpret_cast<const Vec4<TE>*>(static_cast<const TE*>(ep.extra) + row * P + col);
+    }
+};
+
+template <typename T, typename TO, int EPI>
+__device__ __forceinline__ void finish4(const Epilogue& ep, int64_t row, int col, int P, const f32x4& acc, const Second4<T, TO, EPI>& second) {
     float v[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) v[e] = acc[e];
     if (ep.bias) {
-        const Vec4<TB> b = *reinterpret_cast<const Vec4<TB>*>(static_cast<const TB*>(ep.bias) + col);
+        const Vec4<T> b = *reinterpret_cast<const Vec4<T>*>(static_cast<const T*>(ep.bias) + col);
 #pragma unroll
         for (int e = 0; e < 4; ++e) v[e] += to_acc(b.v[e]);
     }
     const int64_t at = row * P + col;
-    Vec4<TO> s;
-    float extra[4] = {0.f, 0.f, 0.f, 0.f};
-    if constexpr (EPI == EPI_RESIDUAL || EPI == EPI_SCALE) {
-        using TE = typename std::conditional<EPI == EPI_SCALE, T, TO>::type;
-        const Vec4<TE> r = *reinterpret_cast<const Vec4<TE>*>(static_cast<const TE*>(ep.extra) + at);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) extra[e] = to_acc(r.v[e]);
-    }
+    float d[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-        float d = 0.f;
-        v[e] = finish1<EPI>(v[e], extra[e], d);
-        s.v[e] = from_acc<TO>(d);
+        float extra = 0.f;
+        if constexpr (Second4<T, TO, EPI>::USED) extra = to_acc(second.r.v[e]);
+        v[e] = finish1<EPI, sizeof(TO) == 4>(v[e], extra, d[e]);
     }
     if constexpr (EPI == EPI_GELU)
-        if (ep.slope) *reinterpret_cast<Vec4<TO>*>(static_cast<TO*>(ep.slope) + at) = s;
-    Vec4<TO> o;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) o.v[e] = from_acc<TO>(v[e]);
-    *reinterpret_cast<Vec4<TO>*>(static_cast<TO*>(ep.y) + at) = o;
+        if (ep.slope) *reinterpret_cast<Vec4<TO>*>(static_cast<TO*>(ep.slope) + at) = pack4<TO>(d);
+    *reinterpret_cast<Vec4<TO>*>(static_cast<TO*>(ep.y) + at) = pack4<TO>(v);
 }
 
 // fp32 layers of 96 reduction channels and a multiple of 96 outputs (tall_linear.hip): x [N >= 32, 96], all of Wop in LDS

@@ -79,10 +79,8 @@ template <> __device__ __forceinline__ Frag<__half> packed<__half>(const f32x4& 
     return Frag<__half>{f16x4{(_Float16)c[0], (_Float16)c[1], (_Float16)c[2], (_Float16)c[3]}};
 }
 template <> __device__ __forceinline__ Frag<__hip_bfloat16> packed<__hip_bfloat16>(const f32x4& c) {
-    s16x4 o;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) o[e] = __builtin_bit_cast(short, __float2bfloat16(c[e]));
-    return Frag<__hip_bfloat16>{o};
+    struct { uint32_t a, b; } w = {pack_bf16(c[0], c[1]), pack_bf16(c[2], c[3])};
+    return Frag<__hip_bfloat16>{__builtin_bit_cast(s16x4, w)};
 }
 
 struct Args {

@@ -14,6 +14,7 @@
 #include <torch/csrc/autograd/functions/basic_ops.h>
 #include <hip/hip_runtime.h>
 
+#include <array>
 #include <mutex>
 #include <optional>
 #include <string>
@@ -206,11 +207,45 @@ Tensor ready(const Tensor& t) {
 }
 
 bool dense_takes(const Tensor& x, const Tensor& w, int64_t P, int64_t K) {
-    return sswin_dense_supported(code_of(x.scalar_type()), (int)P, (int)K) && (w.scalar_type() == x.scalar_type() || w.scalar_type() == at::kFloat);
+    return sswin_dense_supported(code_of(x.scalar_type()), (int)P, (int)K) && w.scalar_type() == x.scalar_type();
 }
-// 16-bit layers with long reductions over many rows: the library's tiles are ahead
+// 16-bit layers with long reductions over many rows: the library's tiles are ahead (1364 rows 768 -> 2304: 11 us against 18,
+// 8119 rows 768 -> 3072: 47 and 57; 8119 rows 384 -> 1152: 23 and 19)
 bool library_ahead(const Tensor& x, int64_t P, int64_t K) {
-    return x.scalar_type() != at::kFloat && K >= 384 && P >= 192 && x.size(0) >= 1024;
+    return x.scalar_type() != at::kFloat && K >= 768 && P >= 192 && x.size(0) >= 1024;
+}
+
+// parameters in the type of the products; fp32 ones under mixed precision are converted together by one launch
+template <size_t COUNT> std::array<Tensor, COUNT> in_type(const std::array<Tensor, COUNT>& params, ScalarType type) {
+    static_assert(COUNT <= SSWIN_CAST_PARTS, "parts of one launch");
+    std::array<Tensor, COUNT> out;
+    const void* src[COUNT];
+    int64_t sizes[COUNT], total = 0;
+    int which[COUNT], n = 0;
+    for (size_t i = 0; i < COUNT; ++i) {
+        const Tensor& p = params[i];
+        if (!p.defined()) continue;
+        if (p.scalar_type() == type || p.scalar_type() != at::kFloat || p.numel() % 8 != 0 || p.numel() == 0) {
+            out[i] = ready(p.to(type));
+            continue;
+        }
+        out[i] = ready(p);
+        src[n] = out[i].data_ptr();
+        sizes[n] = p.numel();
+        total += sizes[n];
+        which[n++] = (int)i;
+    }
+    if (n == 0) return out;
+    const Tensor& first = out[which[0]];
+    const Tensor all = at::empty({total}, first.options().dtype(type));
+    RUN(sswin_cast_parts(code_of(type), src, sizes, n, ptr(all), current_stream(first)));
+    int64_t at = 0;
+    for (int i = 0; i < n; ++i) {
+        Tensor& t = out[which[i]];
+        t = all.narrow(0, at, sizes[i]).view(t.sizes());
+        at += sizes[i];
+    }
+    return out;
 }
 
 // x [N, K], w [P, K] -> last step of x w^T + b
@@ -219,11 +254,13 @@ Tensor dense(const Tensor& x, const Tensor& w_in, const Tensor& b_in, int epilog
     const int64_t N = x.size(0), K = x.size(1), P = w_in.size(0);
     const ScalarType out = out_type.value_or(x.scalar_type());
     const Tensor w = ready(w_in), b = ready(b_in);
-    if (dense_takes(x, w, P, K) && !(epilogue == SSWIN_DENSE_PLAIN && library_ahead(x, P, K))) {
+    if (dense_takes(x, w, P, K) && (!b.defined() || b.scalar_type() == x.scalar_type()) && !(epilogue == SSWIN_DENSE_PLAIN && library_ahead(x, P, K))) {
         Tensor y = at::empty({N, P}, x.options().dtype(out));
         if (slope) *slope = at::empty({N, P}, x.options().dtype(out));
-        RUN(sswin_dense_forward(code_of(x.scalar_type()), code_of(w.scalar_type()), code_of(out), 0, epilogue, ptr(x), N, (int)K, ptr(w), ptr(b), (int)P,
-                                ptr(extra), ptr(y), slope ? ptr(*slope) : nullptr, current_stream(x)));
+        const size_t nb = sswin_dense_forward_workspace_bytes(code_of(x.scalar_type()), N, (int)K, (int)P);
+        const Tensor ws = nb ? bytes(nb, x) : Tensor();
+        RUN(sswin_dense_forward(code_of(x.scalar_type()), code_of(out), 0, epilogue, ptr(x), N, (int)K, ptr(w), ptr(b), (int)P,
+                                ptr(extra), ptr(y), slope ? ptr(*slope) : nullptr, ptr(ws), nb, current_stream(x)));
         return y;
     }
     RocBlas backend;
@@ -244,8 +281,10 @@ Tensor dense_dx(const Tensor& dy, const Tensor& w_in, int epilogue = SSWIN_DENSE
     const int64_t N = dy.size(0), P = dy.size(1), K = w.size(1);
     if (dense_takes(dy, w, K, P) && !(epilogue == SSWIN_DENSE_PLAIN && library_ahead(dy, K, P))) {
         Tensor dx = at::empty({N, K}, dy.options());
-        RUN(sswin_dense_forward(code_of(dy.scalar_type()), code_of(w.scalar_type()), code_of(dy.scalar_type()), 1, epilogue, ptr(dy), N, (int)P, ptr(w), nullptr,
-                                (int)K, ptr(extra), ptr(dx), nullptr, current_stream(dy)));
+        const size_t nb = sswin_dense_forward_workspace_bytes(code_of(dy.scalar_type()), N, (int)P, (int)K);
+        const Tensor ws = nb ? bytes(nb, dy) : Tensor();
+        RUN(sswin_dense_forward(code_of(dy.scalar_type()), code_of(dy.scalar_type()), 1, epilogue, ptr(dy), N, (int)P, ptr(w), nullptr,
+                                (int)K, ptr(extra), ptr(dx), nullptr, ptr(ws), nb, current_stream(dy)));
         return dx;
     }
     RocBlas backend;
@@ -500,15 +539,17 @@ struct ModuleNode : torch::autograd::Function<ModuleNode> {
         NoAutocast off;
         const Tensor qkv_b = or_undefined(qkv_bias), proj_b = or_undefined(proj_bias);
         const Tensor x = ready(x_in.to(type));
-        const Tensor qkv = dense(x, qkv_w, qkv_b);
+        const auto w = in_type<4>({qkv_w, qkv_b, proj_w, proj_b}, type);
+        const Tensor qkv = dense(x, w[0], w[1]);
         AttentionSaved saved;
         Tensor o = attention_forward(*a, qkv, bias, saved);
-        Tensor y = dense(o, proj_w, proj_b);
+        Tensor y = dense(o, w[2], w[3]);
         if (ctx) {
-            ctx->save_for_backward({x, qkv_w, bias, proj_w, qkv, saved.bias32, saved.aux, o, saved.words});
+            ctx->save_for_backward({x, w[0], bias, w[2], qkv, saved.bias32, saved.aux, o, saved.words});
             ctx->saved_data["a"] = capsule(a);
             ctx->saved_data["how"] = std::vector<int64_t>{(int64_t)x_in.scalar_type(), x_in.requires_grad(), qkv_w.requires_grad(), asks(qkv_b),
-                                                          bias.requires_grad(), proj_w.requires_grad(), asks(proj_b)};
+                                                          bias.requires_grad(), proj_w.requires_grad(), asks(proj_b), (int64_t)qkv_w.scalar_type(),
+                                                          (int64_t)proj_w.scalar_type()};
         }
         return y;
     }
@@ -521,11 +562,11 @@ struct ModuleNode : torch::autograd::Function<ModuleNode> {
         c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
         const Tensor dy = ready(grads[0].to(x.scalar_type()));
         std::pair<Tensor, Tensor> d_proj, d_qkvw;
-        if (how[5] || how[6]) d_proj = dense_dw(dy, o, how[6], proj_w.scalar_type());
+        if (how[5] || how[6]) d_proj = dense_dw(dy, o, how[6], (ScalarType)how[8]);
         Tensor d_bias, dx;
         const Tensor d_o = dense_dx(dy, proj_w);
         const Tensor d_qkv = attention_backward(*a, qkv, bias, AttentionSaved{v[5], v[6], v[8]}, o, d_o, how[4], d_bias);
-        if (how[2] || how[3]) d_qkvw = dense_dw(d_qkv, x, how[3], qkv_w.scalar_type());
+        if (how[2] || how[3]) d_qkvw = dense_dw(d_qkv, x, how[3], (ScalarType)how[7]);
         if (how[1]) dx = dense_dx(d_qkv, qkv_w).to((ScalarType)how[0]);
         return once({dx, d_qkvw.first, d_qkvw.second, d_bias, d_proj.first, d_proj.second, Tensor(), Tensor()});
     }
@@ -542,23 +583,26 @@ struct BlockNode : torch::autograd::Function<BlockNode> {
         for (size_t i = 0; i < which.size(); ++i) p[which[i]] = given[i];
         const Tensor x = ready(p[X]);
         const ScalarType stream_type = x.scalar_type();                  // of the residual stream
+        const ScalarType params_type = p[QKVW].scalar_type();
         Tensor stats1, stats2, slope;
+        const auto w = in_type<8>({p[QKVW], p[QKVB], p[PROJW], p[PROJB], p[W1], p[C1], p[W2], p[C2]}, type);
         const Tensor x1 = norm_forward(x, p[G1], p[B1], eps1, type, ctx ? &stats1 : nullptr);
-        const Tensor qkv = dense(x1, p[QKVW], p[QKVB]);
+        const Tensor qkv = dense(x1, w[0], w[1]);
         AttentionSaved saved;
         const Tensor o = attention_forward(*a, qkv, p[TABLE], saved);
-        const Tensor h = dense(o, p[PROJW], p[PROJB], SSWIN_DENSE_RESIDUAL, x, nullptr, stream_type);
+        const Tensor h = dense(o, w[2], w[3], SSWIN_DENSE_RESIDUAL, x, nullptr, stream_type);
         const Tensor x2 = norm_forward(h, p[G2], p[B2], eps2, type, ctx ? &stats2 : nullptr);
-        const Tensor g = dense(x2, p[W1], p[C1], SSWIN_DENSE_GELU, Tensor(), ctx ? &slope : nullptr);
-        Tensor y = dense(g, p[W2], p[C2], SSWIN_DENSE_RESIDUAL, h, nullptr, stream_type);
+        const Tensor g = dense(x2, w[4], w[5], SSWIN_DENSE_GELU, Tensor(), ctx ? &slope : nullptr);
+        Tensor y = dense(g, w[6], w[7], SSWIN_DENSE_RESIDUAL, h, nullptr, stream_type);
         if (ctx) {
-            ctx->save_for_backward({x, p[G1], p[QKVW], p[TABLE], p[PROJW], p[G2], p[W1], p[W2], stats1, x1, qkv, saved.bias32, saved.aux, o, h, stats2, x2, g,
+            ctx->save_for_backward({x, p[G1], w[0], p[TABLE], w[2], p[G2], w[4], w[6], stats1, x1, qkv, saved.bias32, saved.aux, o, h, stats2, x2, g,
                                     slope, saved.words});
             ctx->saved_data["a"] = capsule(a);
             ctx->saved_data["which"] = which;
             std::vector<int64_t> asked;
             for (const Tensor& t : p) asked.push_back(asks(t));
             ctx->saved_data["asked"] = asked;
+            ctx->saved_data["params"] = (int64_t)params_type;
         }
         return y;
     }
@@ -570,7 +614,7 @@ struct BlockNode : torch::autograd::Function<BlockNode> {
         const Tensor &x = v[0], &g1 = v[1], &qkvw = v[2], &table = v[3], &projw = v[4], &g2 = v[5], &w1 = v[6], &w2 = v[7], &stats1 = v[8], &x1 = v[9],
                      &qkv = v[10], &o = v[13], &h = v[14], &stats2 = v[15], &x2 = v[16], &g = v[17], &slope = v[18];
         c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
-        const ScalarType type = x1.scalar_type(), wt = qkvw.scalar_type();
+        const ScalarType type = x1.scalar_type(), wt = (ScalarType)ctx->saved_data["params"].toInt();
         const Tensor dy = ready(grads[0]);
         const Tensor dyt = dy.to(type);
         Tensor out[PARAMS];
@@ -607,9 +651,11 @@ struct MergeNode : torch::autograd::Function<MergeNode> {
         RUN(sswin_pool_windows(code_of(x.scalar_type()), 0, 1, i32(plan->plan), plan->g_cap, M, i32(plan->tokens), plan->N, ptr(x), D, (int)D, ptr(pooled), D,
                                current_stream(x)));
         const Tensor x1 = norm_forward(pooled, gamma, beta, eps, type, ctx ? &stats : nullptr);
-        Tensor y = dense(x1, w, Tensor());
+        const auto wt = in_type<1>({w}, type);
+        Tensor y = dense(x1, wt[0], Tensor());
         if (ctx) {
-            ctx->save_for_backward({gamma, w, pooled, stats, x1});
+            ctx->save_for_backward({gamma, wt[0], pooled, stats, x1});
+            ctx->saved_data["params"] = (int64_t)w.scalar_type();
             ctx->saved_data["p"] = capsule(plan);
         }
         return y;
@@ -621,7 +667,7 @@ struct MergeNode : torch::autograd::Function<MergeNode> {
         const Tensor &gamma = v[0], &w = v[1], &pooled = v[2], &stats = v[3], &x1 = v[4];
         c10::hip::HIPGuardMasqueradingAsCUDA guard(pooled.device());
         const Tensor dy = ready(grads[0].to(x1.scalar_type()));
-        Tensor dg, db, dw = dense_dw(dy, x1, false, w.scalar_type()).first;
+        Tensor dg, db, dw = dense_dw(dy, x1, false, (ScalarType)ctx->saved_data["params"].toInt()).first;
         const Tensor d_pool = norm_backward(dense_dx(dy, w), pooled, stats, gamma, Tensor(), dg, db);
         const int64_t D = pooled.size(1);
         Tensor dx = at::empty({plan->N, D}, pooled.options());

@@ -138,6 +138,11 @@ template <> __device__ __forceinline__ __half from_acc<__half>(float v) { return
 template <> __device__ __forceinline__ __hip_bfloat16 from_acc<__hip_bfloat16>(float v) {
     return __float2bfloat16(v);
 }
+// two values with one conversion (__float2bfloat16 twice is two, a shift and an or)
+__device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) {
+    typedef __bf16 pair __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t, pair{(__bf16)lo, (__bf16)hi});
+}
 
 // Zeros by a kernel instead of hipMemsetAsync: callers may capture these entry points into a HIP graph, and memset
 // nodes have given wrong results on replays of a captured graph.

@@ -98,9 +98,7 @@ __device__ __forceinline__ uint32_t pack2(float lo, float hi, __half) {
     return __builtin_bit_cast(uint32_t, __floats2half2_rn(lo, hi));
 }
 __device__ __forceinline__ uint32_t pack2(float lo, float hi, __hip_bfloat16) {
-    const uint32_t a = __builtin_bit_cast(uint16_t, __float2bfloat16(lo));
-    const uint32_t b = __builtin_bit_cast(uint16_t, __float2bfloat16(hi));
-    return a | (b << 16);
+    return pack_bf16(lo, hi);
 }
 
 // ------------------------------------------------------------------------------------------

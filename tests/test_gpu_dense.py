@@ -40,29 +40,30 @@ def _forward(lib, _lib, x, w, b, transposed, epi, extra, out):
     P = w.shape[1] if transposed else w.shape[0]
     y = torch.full((N, P), float("nan"), dtype=out, device="cuda")
     slope = torch.full((N, P), float("nan"), dtype=out, device="cuda") if epi == GELU else None
-    _lib.check(lib.sswin_dense_forward(CODE[x.dtype], CODE[w.dtype], CODE[out], transposed, epi, _ptr(x), N, K, _ptr(w), _ptr(b), P,
-                                       _ptr(extra), _ptr(y), _ptr(slope), _stream()))
+    nb = lib.sswin_dense_forward_workspace_bytes(CODE[x.dtype], N, K, P)
+    ws = torch.empty(max(nb, 1), dtype=torch.uint8, device="cuda")
+    _lib.check(lib.sswin_dense_forward(CODE[x.dtype], CODE[out], transposed, epi, _ptr(x), N, K, _ptr(w), _ptr(b), P,
+                                       _ptr(extra), _ptr(y), _ptr(slope), _ptr(ws), nb, _stream()))
     return y, slope
 
 
 # one row, part of a tile, tile edges, many tiles; reductions of one step, of odd counts of steps, of whole blocks; columns of
-# part of a column block and of several; the few-rows kernel and the tiled ones; 96 channels: the kernel with W in LDS
+# part of a column block and of several; the few-rows kernel and the tiled ones; 96 channels: the kernel with W in LDS; 16 bit:
+# shares of the reduction (ragged ones too), eight wavefronts a tile, tiles of 192 columns
 SHAPES = [(1, 16, 16), (31, 48, 144), (33, 96, 96), (300, 384, 1152), (129, 1536, 48), (9000, 48, 192), (9001, 112, 208),
-          (30000, 96, 288), (20001, 144, 48), (20000, 288, 96)]
+          (30000, 96, 288), (20001, 144, 48), (20000, 288, 96), (500, 1552, 384), (1300, 784, 368), (1364, 3072, 96), (8100, 400, 1536)]
 
 
 @pytest.mark.parametrize("N,K,P", SHAPES)
-@pytest.mark.parametrize("dtype,wdtype,out", [(torch.float32, torch.float32, torch.float32), (torch.bfloat16, torch.bfloat16, torch.bfloat16),
-                                              (torch.float16, torch.float32, torch.float16), (torch.float16, torch.float32, torch.float32)],
-                         ids=["fp32", "bf16", "fp16-w32", "fp16-w32-out32"])
-def test_dense_forward_and_input_gradient(N, K, P, dtype, wdtype, out):
+@pytest.mark.parametrize("dtype,out", [(torch.float32, torch.float32), (torch.bfloat16, torch.bfloat16), (torch.float16, torch.float16),
+                                       (torch.float16, torch.float32)], ids=["fp32", "bf16", "fp16", "fp16-out32"])
+def test_dense_forward_and_input_gradient(N, K, P, dtype, out):
     from sparseswin3d_amd import _lib
     lib = _lib.load()
     gen = torch.Generator().manual_seed(N + 3 * K + 7 * P)
-    x, w, b = _rand(gen, N, K, dtype=dtype), _rand(gen, P, K, dtype=wdtype, spread=1) / K ** 0.5, _rand(gen, P, dtype=wdtype)
+    x, w, b = _rand(gen, N, K, dtype=dtype), (_rand(gen, P, K, spread=1) / K ** 0.5).to(dtype), _rand(gen, P, dtype=dtype)
     extra = _rand(gen, N, P, dtype=out)
-    w = w.to(wdtype)
-    wd = w.to(dtype).double()                                    # fp32 weights are rounded to the tokens' type
+    wd = w.double()
     pre = x.double() @ wd.T + b.double()
     mag = x.double().abs() @ wd.abs().T + b.double().abs()
     if out == dtype:
@@ -103,16 +104,30 @@ def test_dense_weight_gradient(N, P, K, dtype, out):
     assert torch.equal(results[0][0], results[1][0]) and torch.equal(results[0][1], results[1][1])       # fixed order of the sums
 
 
+@pytest.mark.parametrize("sizes", [(8,), (96 * 288, 288, 96 * 96, 96, 8, 16, 2056, 24)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_cast_parts(sizes, dtype):
+    from sparseswin3d_amd import _lib
+    lib = _lib.load()
+    gen = torch.Generator().manual_seed(len(sizes))
+    src = [_rand(gen, n) for n in sizes]
+    dst = torch.full((sum(sizes),), float("nan"), dtype=dtype, device="cuda")
+    _lib.check(lib.sswin_cast_parts(CODE[dtype], (C.c_void_p * len(src))(*[t.data_ptr() for t in src]), (C.c_int64 * len(src))(*sizes), len(src), _ptr(dst),
+                                    _stream()))
+    assert torch.equal(dst, torch.cat(src).to(dtype))
+    assert lib.sswin_cast_parts(CODE[dtype], (C.c_void_p * 1)(src[0].data_ptr()), (C.c_int64 * 1)(4), 1, _ptr(dst), _stream()) != 0
+
+
 def test_dense_refuses_what_it_does_not_take():
     from sparseswin3d_amd import _lib
     lib = _lib.load()
     x = torch.zeros(4, 24, device="cuda")
     assert not lib.sswin_dense_supported(0, 16, 24) and lib.sswin_dense_supported(2, 16, 32) and not lib.sswin_dense_supported(3, 16, 16)
-    assert lib.sswin_dense_forward(0, 0, 0, 0, PLAIN, _ptr(x), 4, 24, _ptr(x), None, 16, None, _ptr(x), None, _stream()) != 0
+    assert lib.sswin_dense_forward(0, 0, 0, PLAIN, _ptr(x), 4, 24, _ptr(x), None, 16, None, _ptr(x), None, None, 0, _stream()) != 0
     assert b"multiples of 16" in lib.sswin_last_error()
-    assert lib.sswin_dense_forward(0, 0, 0, 0, SCALE, _ptr(x), 4, 16, _ptr(x), None, 16, _ptr(x), _ptr(x), None, _stream()) != 0
-    assert lib.sswin_dense_forward(0, 0, 0, 0, RESIDUAL, _ptr(x), 4, 16, _ptr(x), None, 16, None, _ptr(x), None, _stream()) != 0
-    assert lib.sswin_dense_forward(0, 0, 0, 0, PLAIN, None, 0, 16, None, None, 16, None, None, None, _stream()) == 0
+    assert lib.sswin_dense_forward(0, 0, 0, SCALE, _ptr(x), 4, 16, _ptr(x), None, 16, _ptr(x), _ptr(x), None, None, 0, _stream()) != 0
+    assert lib.sswin_dense_forward(0, 0, 0, RESIDUAL, _ptr(x), 4, 16, _ptr(x), None, 16, None, _ptr(x), None, None, 0, _stream()) != 0
+    assert lib.sswin_dense_forward(0, 0, 0, PLAIN, None, 0, 16, None, None, 16, None, None, None, None, 0, _stream()) == 0
 
 
 @pytest.mark.parametrize("N,D", [(1, 16), (7, 48), (1000, 96), (33, 192), (257, 768), (5, 80), (63, 1536), (4, 2048), (50000, 96)])
