@@ -11,10 +11,12 @@
 // Layouts: v_mfma_f32_16x16x*: operand lane l = (row l % 16, reduction slots 4 (l / 16) + j), accumulator lane l = (column
 // l % 16, rows 4 (l / 16) + r).  An accumulator packed in place is therefore the operand of the next product over its rows:
 // S^T = K Q^T gives P^T as the operand of O^T = V^T P^T, and the row of a query (its maximum, sum and rescaling) lies in the
-// four lanes l % 16.  fp32 tokens take four 16x16x4 fp32 products per 16 slots, 16-bit tokens one 16x16x16.
+// four lanes l % 16.  fp32 tokens take four 16x16x4 fp32 products per 16 slots, products of two 16-bit tokens one 16x16x16.  P
+// and dS stay fp32 for 16-bit tokens as well (as in the operators; dS of fp16 tokens would leave fp16's range): their products
+// are the fp32 ones, with the tokens widened.
 //
 // Softmax as the operators define it: exp(s - m) / (sum exp(s - m) + 1e-8), m = max(0, row maximum).  The running offset is the
-// maximum over the first 16 tokens (so that 16-bit P keeps its precision where all scores are far below 0) and moves only when
+// maximum over the first 16 tokens (exponentials of its rows are of order one, however far below 0 the scores lie) and moves only when
 // a score exceeds it by 10 in units of log 2: a row usually needs one exchange between its lanes at the start and one at the
 // end, where the 1e-8 is scaled to the offset that was used.
 //
@@ -23,7 +25,8 @@
 // differ.
 //
 // 112 700 voxels, windows of 7^3, 3 heads of 16 (27 million scores): fp32 forward 63 us, backward 212 us (the store of dS 36 of
-// them); fp16 39 and 118.  The block products with the attention matrix in memory take 195 and 258 us (fp32).  The vector ALU is
+// them).  219 000 voxels, fp16: forward 84 us, backward 292 (72 and 273 with P and dS rounded to fp16, which loses the operators'
+// precision).  The block products with the attention matrix in memory take 195 and 258 us (112 700 voxels, fp32).  The vector ALU is
 // busy for half of a launch, the fp32 matrix instructions (which occupy it) for another quarter; leaving out the bias reads, the
 // exponentials or the row loads one by one changes the forward by less than 3 %, the rows of the backward by 15 %.
 #include <math.h>
@@ -213,21 +216,21 @@ template <typename T, int HD> struct Rows {
 #pragma unroll
         for (int b = 0; b < NB; ++b) f[b].load(base + (__umul24(v, pitch) + col + b * 16));
     }
-    // column operand: lane (channel 16 b + l % 16, slots = the tokens 4 (l / 16) + j with voxels v[j])
-    __device__ __forceinline__ void column(const int (&v)[4], const Frag<T> (&rows)[NB], Frag<T> (&f)[NB]) const {
+    // fp32 column operand: lane (channel 16 b + l % 16, slots = the tokens 4 (l / 16) + j with voxels v[j])
+    __device__ __forceinline__ void column(const int (&v)[4], const Frag<T> (&rows)[NB], Frag<float> (&f)[NB]) const {
         if constexpr (sizeof(T) == 4) {
 #pragma unroll
             for (int b = 0; b < NB; ++b)
 #pragma unroll
                 for (int j = 0; j < 4; ++j) f[b].v[j] = base[__umul24((uint32_t)v[j], pitch) + b * 16 + (threadIdx.x & 15)];
         } else {
-            // the row operand turned on the matrix core: a product with the identity, exact for 16-bit values
+            // the row operand turned and widened on the matrix core: a product with the identity, exact for 16-bit values
             f32x4 one;
 #pragma unroll
             for (int j = 0; j < 4; ++j) one[j] = (int)(((threadIdx.x & 63) >> 4) * 4 + j) == (int)(threadIdx.x & 15) ? 1.f : 0.f;
             const Frag<T> id = packed<T>(one);
 #pragma unroll
-            for (int b = 0; b < NB; ++b) f[b] = packed<T>(mma(rows[b], id, f32x4{0.f, 0.f, 0.f, 0.f}));
+            for (int b = 0; b < NB; ++b) f[b].v = mma(rows[b], id, f32x4{0.f, 0.f, 0.f, 0.f});
         }
     }
 };
@@ -330,7 +333,7 @@ __global__ __launch_bounds__(WAVES * 64) void flash_forward_kernel(Args g, int64
         uint32_t w_next[4];
         auto request = [&]() {
             k_rows.row((uint32_t)ahead.row, k_next);
-            if (sizeof(T) == 4) v_rows.column(ahead.v, v_next, v_next);
+            if constexpr (sizeof(T) == 4) v_rows.column(ahead.v, v_next, v_next);
             else v_rows.row((uint32_t)ahead.row, v_next);
 #pragma unroll
             for (int j = 0; j < 4; ++j) w_next[j] = ahead.w[j];
@@ -339,7 +342,8 @@ __global__ __launch_bounds__(WAVES * 64) void flash_forward_kernel(Args g, int64
         if (b.to - b.from > 16) ahead.load(g, b.from + 16, b.to);
         for (int k0 = b.from; k0 < b.to; k0 += 16) {
             const int last = b.to - 1 - k0;
-            Frag<T> k[NB], v[NB], vt[NB];
+            Frag<T> k[NB], v[NB];
+            Frag<float> vt[NB];
             uint32_t pk[4];
 #pragma unroll
             for (int c = 0; c < NB; ++c) k[c] = k_next[c], v[c] = v_next[c];
@@ -347,7 +351,7 @@ __global__ __launch_bounds__(WAVES * 64) void flash_forward_kernel(Args g, int64
             for (int j = 0; j < 4; ++j) pk[j] = w_next[j];
             if (last >= 16) request();
             if (last >= 32) ahead.load(g, k0 + 32, b.to);
-            if (sizeof(T) == 4) {
+            if constexpr (sizeof(T) == 4) {
 #pragma unroll
                 for (int c = 0; c < NB; ++c) vt[c] = v[c];
             } else {
@@ -387,7 +391,7 @@ __global__ __launch_bounds__(WAVES * 64) void flash_forward_kernel(Args g, int64
 #pragma unroll
                     for (int j = 0; j < 4; ++j) p[j] = __builtin_amdgcn_exp2f(x[j]);
                     sum[s] += (p[0] + p[1]) + (p[2] + p[3]);
-                    const Frag<T> pt = packed<T>(p);
+                    const Frag<float> pt = {p};
 #pragma unroll
                     for (int c = 0; c < NB; ++c) o[s][c] = mma(vt[c], pt, o[s][c]);
                 }
@@ -475,7 +479,8 @@ __global__ __launch_bounds__(WAVES * 64) void flash_backward_q_kernel(Args g, in
         for (int k0 = b.from; k0 < b.to; k0 += 16) {
             const int last = b.to - 1 - k0;
             const Step<T> step = ahead;
-            Frag<T> k[NB], v[NB], kt[NB];
+            Frag<T> k[NB], v[NB];
+            Frag<float> kt[NB];
             k_rows.row((uint32_t)step.row, k);
             v_rows.row((uint32_t)step.row, v);
             k_rows.column(step.v, k, kt);
@@ -506,7 +511,7 @@ __global__ __launch_bounds__(WAVES * 64) void flash_backward_q_kernel(Args g, in
                                 if (quad * 4 + j <= last && !((pq[s] ^ step.w[j]) >> 23)) row[j] = ds[j];
                         }
                     }
-                    const Frag<T> dst = packed<T>(ds);
+                    const Frag<float> dst = {ds};
 #pragma unroll
                     for (int c = 0; c < NB; ++c) dq[s][c] = mma(kt[c], dst, dq[s][c]);
                 }
@@ -582,7 +587,8 @@ __global__ __launch_bounds__(WAVES * 64) void flash_backward_kv_kernel(Args g, i
                     delta[j] = g.delta[r];
                 }
             }
-            Frag<T> q[NB], d_o[NB], qt[NB], dot[NB];
+            Frag<T> q[NB], d_o[NB];
+            Frag<float> qt[NB], dot[NB];
             q_rows.row((uint32_t)step.row, q);
             do_rows.row((uint32_t)step.row, d_o);
             q_rows.column(step.v, q, qt);
@@ -602,7 +608,7 @@ __global__ __launch_bounds__(WAVES * 64) void flash_backward_kv_kernel(Args g, i
                         p[j] = __builtin_amdgcn_exp2f(score<FAST>(acc[j], scale2, step.w[j] + (uint32_t)g.offset4, pk[s], table));
                         ds[j] = p[j] * dp[j];
                     }
-                    const Frag<T> pf = packed<T>(p), df = packed<T>(ds);
+                    const Frag<float> pf = {p}, df = {ds};
 #pragma unroll
                     for (int c = 0; c < NB; ++c) dv[s][c] = mma(dot[c], pf, dv[s][c]), dk[s][c] = mma(qt[c], df, dk[s][c]);
                 }
