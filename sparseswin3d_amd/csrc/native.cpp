@@ -251,7 +251,11 @@ template <size_t COUNT> std::array<Tensor, COUNT> in_type(const std::array<Tenso
 // x [N, K], w [P, K] -> last step of x w^T + b
 Tensor dense(const Tensor& x, const Tensor& w_in, const Tensor& b_in, int epilogue = SSWIN_DENSE_PLAIN, const Tensor& extra = Tensor(),
              Tensor* slope = nullptr, std::optional<ScalarType> out_type = std::nullopt) {
+    TORCH_CHECK(w_in.dim() == 2 && w_in.size(1) == x.size(1) && (!b_in.defined() || (b_in.dim() == 1 && b_in.size(0) == w_in.size(0))),
+                "a dense layer of weight ", w_in.sizes(), " on rows of ", x.size(1), " values");
     const int64_t N = x.size(0), K = x.size(1), P = w_in.size(0);
+    TORCH_CHECK(epilogue != SSWIN_DENSE_RESIDUAL || (extra.dim() == 2 && extra.size(0) == N && extra.size(1) == P), "a dense layer of ", P,
+                " columns added to rows of ", extra.sizes());
     const ScalarType out = out_type.value_or(x.scalar_type());
     const Tensor w = ready(w_in), b = ready(b_in);
     if (dense_takes(x, w, P, K) && (!b.defined() || b.scalar_type() == x.scalar_type()) && !(epilogue == SSWIN_DENSE_PLAIN && library_ahead(x, P, K))) {
@@ -364,6 +368,11 @@ struct AttentionSaved {
 Tensor attention_forward(Attention& a, const Tensor& qkv, const Tensor& bias, AttentionSaved& saved) {
     Plan& tp = *a.plan;
     tp.finish();
+    TORCH_CHECK(qkv.dim() == 2 && qkv.size(0) == tp.N && qkv.size(1) % (3 * a.H) == 0 && tp.H == a.H && tp.n == a.n, "attention: qkv of ", qkv.sizes(),
+                " for a plan of ", tp.N, " tokens in windows of ", tp.n, " and ", tp.H, " heads");
+    TORCH_CHECK(a.code.defined() ? bias.dim() == 2 && bias.size(1) == a.H : bias.dim() == 3 && bias.size(0) == a.H && bias.size(1) == a.n && bias.size(2) == a.n,
+                "attention: bias of ", bias.sizes());
+    TORCH_CHECK(!a.mask.defined() || (a.mask.dim() == 2 && a.mask.size(0) > 0 && a.mask.size(1) == a.n), "attention: mask of ", a.mask.sizes());
     if (a.flash && !(a.scale > 0 && sswin_flash_supported(code_of(qkv.scalar_type()), qkv.size(0), a.H, (int)(qkv.size(1) / 3 / a.H), (int)bias.size(0))))
         a.flash = false;                                                 // more tokens than the kernels address: the products
     TORCH_CHECK(!a.resident || tp.oversize == 0, "window-resident attention: ", tp.oversize, " groups hold more than 128 tokens");
@@ -497,10 +506,12 @@ template <typename T> c10::intrusive_ptr<T> opened(const c10::IValue& v) { retur
 Tensor or_undefined(const OptTensor& t) { return t ? *t : Tensor(); }
 bool asks(const Tensor& t) { return t.defined() && t.requires_grad(); }
 
-bool wants_grad(std::initializer_list<const Tensor*> ts) {
-    if (!at::GradMode::is_enabled()) return false;
+// Whether a call has to be an autograd node.  A forward-mode tangent counts with gradients switched off as well: the node
+// refuses it, the bare computation would drop it.
+bool wants_node(const Tensor& t) { return t.defined() && ((at::GradMode::is_enabled() && t.requires_grad()) || t._fw_grad(0).defined()); }
+bool wants_node(std::initializer_list<const Tensor*> ts) {
     for (const Tensor* t : ts)
-        if (t->defined() && t->requires_grad()) return true;
+        if (wants_node(*t)) return true;
     return false;
 }
 
@@ -698,7 +709,7 @@ Tensor attention(const Tensor& qkv, const Tensor& bias, const PlanPtr& plan, con
                  double scale, const std::string& path) {
     c10::hip::HIPGuardMasqueradingAsCUDA guard(qkv.device());
     auto a = make_attention(plan, mask, code, offset0, n, qkv.size(2), scale, path);
-    if (!wants_grad({&qkv, &bias})) return AttentionNode::forward(nullptr, qkv, bias, a);
+    if (!wants_node({&qkv, &bias})) return AttentionNode::forward(nullptr, qkv, bias, a);
     return AttentionNode::apply(qkv, bias, a);
 }
 
@@ -708,7 +719,7 @@ Tensor attention_module(const Tensor& x, const Tensor& qkv_w, const OptTensor& q
     c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
     auto a = make_attention(plan, mask, code, offset0, n, heads, scale, path);
     const Tensor qb = or_undefined(qkv_b), pb = or_undefined(proj_b);
-    if (!wants_grad({&x, &qkv_w, &qb, &bias, &proj_w, &pb})) return ModuleNode::forward(nullptr, x, qkv_w, qkv_b, bias, proj_w, proj_b, a, type);
+    if (!wants_node({&x, &qkv_w, &qb, &bias, &proj_w, &pb})) return ModuleNode::forward(nullptr, x, qkv_w, qkv_b, bias, proj_w, proj_b, a, type);
     return ModuleNode::apply(x, qkv_w, qkv_b, bias, proj_w, proj_b, a, type);
 }
 
@@ -717,22 +728,22 @@ Tensor block(std::vector<OptTensor> params, const PlanPtr& plan, const OptTensor
     TORCH_CHECK(params.size() == BlockNode::PARAMS, "block: ", (int)BlockNode::PARAMS, " tensors expected");
     variable_list given;
     std::vector<int64_t> which;
-    bool grad = false;
+    bool node = false;
     for (size_t i = 0; i < params.size(); ++i)
         if (params[i] && params[i]->defined()) {
-            grad = grad || params[i]->requires_grad();
+            node = node || wants_node(*params[i]);
             given.push_back(*params[i]);
             which.push_back((int64_t)i);
         }
     c10::hip::HIPGuardMasqueradingAsCUDA guard(given.at(0).device());
     auto a = make_attention(plan, mask, code, offset0, n, heads, scale, path);
-    if (!grad || !at::GradMode::is_enabled()) return BlockNode::forward(nullptr, given, which, a, eps1, eps2, type);
+    if (!node) return BlockNode::forward(nullptr, given, which, a, eps1, eps2, type);
     return BlockNode::apply(at::TensorList(given), which, a, eps1, eps2, type);
 }
 
 Tensor merge(const Tensor& x, const Tensor& gamma, const Tensor& beta, const Tensor& w, const PlanPtr& plan, double eps, ScalarType type) {
     c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
-    if (!wants_grad({&x, &gamma, &beta, &w})) return MergeNode::forward(nullptr, x, gamma, beta, w, plan, eps, type);
+    if (!wants_node({&x, &gamma, &beta, &w})) return MergeNode::forward(nullptr, x, gamma, beta, w, plan, eps, type);
     return MergeNode::apply(x, gamma, beta, w, plan, eps, type);
 }
 

@@ -750,13 +750,18 @@ class WindowAttentionSparse(nn.Module):
         """(BiasTableIndex or None, compute dtype) where the fused path takes this call, else
         None.  Under autocast the projections and the attention run in its type, as ``nn.Linear`` would."""
         from . import fused
-        if not self.fused:
+        if not self.fused or features.dim() != 2:
             return None
-        dtype = torch.get_autocast_dtype("cuda") if torch.is_autocast_enabled("cuda") else features.dtype
+        autocast = torch.is_autocast_enabled("cuda")
+        # under autocast the projections are called as modules (tall_linear), which may be anything
+        if autocast and any(type(m) is not nn.Linear or m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks
+                            for m in (self.qkv, self.proj)):
+            return None
+        dtype = torch.get_autocast_dtype("cuda") if autocast else features.dtype
         weight = self.qkv.weight.dtype
         if dtype not in fused._DTYPE_CODE or weight not in (dtype, torch.float32) or self.proj.weight.dtype != weight:
             return None
-        if features.dtype != dtype and not torch.is_autocast_enabled("cuda"):
+        if features.dtype != dtype and not autocast:
             return None
         ti = self._table_index(n)
         if n > 384 if ti is not None else n * n * 4 > 64 * 1024:
@@ -768,18 +773,23 @@ class WindowAttentionSparse(nn.Module):
         b = x.batch_size
         c = x.features.shape[-1]
         plan = None
+        from . import fused
         if _takes_token_plan(self, x):
             # the token plan is enqueued first; the projection below runs while its totals travel.
             plan = _token_plan(self, x)
             native = self._fused_arguments(x.features, n)
             if native is not None:
-                from . import fused
                 ti, dtype = native
                 bias = self.relative_position_bias_table if ti is not None else self.relative_position_bias(n, torch.float32)
                 out = fused.fused_window_attention(None, bias, x.indices, mask, b, n, self.scale, self.resident, plan, ti,
                                                    (x.features, self.qkv, self.proj, self.num_heads, dtype))
                 return replace_feature(x, self.proj_drop(out))
         qkv = tall_linear(x.features, self.qkv).reshape(-1, 3, self.num_heads, c // self.num_heads)
+        table_index = self._table_index(n) if plan is not None and self.fused else None
+        if plan is not None and self.fused and fused.supports(qkv, n, table_index is not None):
+            bias = self.relative_position_bias_table if table_index is not None else self.relative_position_bias(n, torch.float32)
+            out = fused.fused_window_attention(qkv, bias, x.indices, mask, b, n, self.scale, self.resident, plan, table_index)
+            return replace_feature(x, self.proj_drop(tall_linear(out, self.proj)))
         q, k_t, v = qkv_sparse_cuda(qkv, x.indices, b, n, plan, q_scale=self.scale)         # q = q * self.scale
         attn = spspmm_block_naive(q, k_t, "q_k")
         biased = sp_add_table_bias_and_mask(attn, self.relative_position_bias_table, self._table_index(n), mask, plan)

@@ -227,3 +227,54 @@ def test_blocks_with_dropout_or_hooks_run_their_modules():
     assert not torch.allclose(b, c, rtol=1e-3, atol=1e-3)
     layer.eval()
     assert torch.allclose(run(feats), b, rtol=1e-4, atol=1e-5)
+
+
+def test_modules_refuse_what_their_layers_do_not_fit():
+    """Host checks of the compiled path: rows of another width, a plan of other voxels, forward-mode tangents."""
+    import numpy as np
+    from helpers import random_window_indices
+    from sparseswin3d_amd.window_attention import SparseVoxelTensor, WindowAttentionSparse
+    torch.manual_seed(0)
+    attn = WindowAttentionSparse(96, 3, (5, 5, 5), qkv_bias=True).cuda()
+    ind = torch.from_numpy(random_window_indices(np.random.default_rng(0), 40, 125, 700)).cuda()
+    run = lambda f, i=ind: attn(SparseVoxelTensor(f, i, (125,), 40), None).features
+    x = torch.randn(700, 96, device="cuda")
+    for grad in (True, False):
+        with torch.set_grad_enabled(grad):
+            with pytest.raises(RuntimeError):
+                run(torch.randn(700, 48, device="cuda"))
+            with pytest.raises(RuntimeError):
+                run(x[:600].contiguous())
+            with torch.autograd.forward_ad.dual_level():
+                with pytest.raises(RuntimeError, match="jvp"):
+                    run(torch.autograd.forward_ad.make_dual(x, torch.ones_like(x)))
+    layer, stage, feats = _stage_pieces(96, 3, 5, torch.float32, True, 7)
+    with torch.no_grad(), torch.autograd.forward_ad.dual_level(), pytest.raises(RuntimeError, match="jvp"):
+        stage(torch.autograd.forward_ad.make_dual(feats, torch.ones_like(feats)))
+    with pytest.raises(RuntimeError):
+        stage(feats[:, :48].contiguous())
+
+
+def test_projections_that_are_no_plain_linears_run_under_autocast():
+    """Under autocast the projections are called as modules: a wrapper or a hook takes part."""
+    import numpy as np
+    from helpers import random_window_indices
+    from sparseswin3d_amd.window_attention import SparseVoxelTensor, WindowAttentionSparse
+
+    class Scaled(torch.nn.Linear):
+        def forward(self, x):
+            return 0 * super().forward(x)
+
+    torch.manual_seed(0)
+    attn = WindowAttentionSparse(96, 3, (5, 5, 5), qkv_bias=True).cuda()
+    ind = torch.from_numpy(random_window_indices(np.random.default_rng(0), 40, 125, 700)).cuda()
+    x = torch.randn(700, 96, device="cuda")
+    with torch.autocast("cuda", dtype=torch.float16):
+        plain = attn(SparseVoxelTensor(x, ind, (125,), 40), None).features
+        calls = []
+        handle = attn.qkv.register_forward_hook(lambda *a: calls.append(1))
+        hooked = attn(SparseVoxelTensor(x, ind, (125,), 40), None).features
+        handle.remove()
+        assert calls == [1] and torch.allclose(plain, hooked, rtol=2e-2, atol=2e-2)
+        attn.proj = Scaled(96, 96).cuda()
+        assert not attn(SparseVoxelTensor(x, ind, (125,), 40), None).features.any()
