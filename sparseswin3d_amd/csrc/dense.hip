@@ -178,7 +178,7 @@ __global__ __launch_bounds__(WM * 64) __attribute__((amdgpu_waves_per_eu(OCC, OC
     const int col0 = cg * BN;
 
     // addresses: a uniform base that moves along the reduction plus 32-bit lane offsets formed once
-    Along<float> ra[UA];
+    Along<float> ra[2][UA];                                              // of the next two steps
     typename std::conditional<DOWN, Down, Along<float>>::type rw[UB];
     uint32_t oa[UA], ow[UB];
     const int last = (int)(N - 1 - row0 < BM - 1 ? N - 1 - row0 : BM - 1);   // rows past the end repeat the last one
@@ -194,12 +194,12 @@ __global__ __launch_bounds__(WM * 64) __attribute__((amdgpu_waves_per_eu(OCC, OC
         else ow[i] = (uint32_t)(min(col0 + u / KC, P - 1) * K + (u % KC) * 8);
     }
     const float* xb = x + row0 * K;
-    auto request = [&](int k0) {
+    static_assert(A_UNITS % THREADS == 0, "every lane reads the same number of pieces of x");
+    auto request_x = [&](int slot, int k0) {
 #pragma unroll
-        for (int i = 0; i < UA; ++i) {
-            const int u = threadIdx.x + i * THREADS;
-            if (A_UNITS % THREADS == 0 || u < A_UNITS) ra[i].load(xb + k0 + oa[i]);
-        }
+        for (int i = 0; i < UA; ++i) ra[slot][i].load(xb + k0 + oa[i]);
+    };
+    auto request_w = [&](int k0) {
 #pragma unroll
         for (int i = 0; i < UB; ++i) {
             const int u = threadIdx.x + i * THREADS;
@@ -218,15 +218,13 @@ __global__ __launch_bounds__(WM * 64) __attribute__((amdgpu_waves_per_eu(OCC, OC
 #pragma unroll
         for (int q = 0; q < PL; ++q) dst[q * 64] = p[q];
     };
-    auto store = [&](u32x4* buf) {
+    auto store = [&](int slot, u32x4* buf) {
 #pragma unroll
         for (int i = 0; i < UA; ++i) {
             const int u = threadIdx.x + i * THREADS;
-            if (A_UNITS % THREADS == 0 || u < A_UNITS) {
-                u32x4 p[PL];
-                ra[i].planes(p);
-                put(buf, BM / 32, u / KC, u % KC, p);
-            }
+            u32x4 p[PL];
+            ra[slot][i].planes(p);
+            put(buf, BM / 32, u / KC, u % KC, p);
         }
 #pragma unroll
         for (int i = 0; i < UB; ++i) {
@@ -252,12 +250,17 @@ __global__ __launch_bounds__(WM * 64) __attribute__((amdgpu_waves_per_eu(OCC, OC
 #pragma unroll
         for (int j = 0; j < NT; ++j) acc[i][j] = f32x16{0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
     const int nk = K / BK;
-    request(0);
-    store(lds);
-    for (int kb = 0; kb < nk; ++kb) {
+    // x comes from memory: two steps ahead (219 000 rows 288 -> 96: 106 us with one, 96 with two).  w lies in L2: one step
+    // ahead, and requested before x, so that waiting for it leaves the x behind it in flight.
+    request_w(0);
+    request_x(0, 0);
+    if (nk > 1) request_x(1, BK);
+    store(0, lds);
+    auto step = [&](int kb, int slot, bool next, bool after) {           // next, after: whether there is a step kb + 1, kb + 2
         __syncthreads();
-        if (kb + 1 < nk) request((kb + 1) * BK);
-        const u32x4* buf = lds + (kb & 1) * BUF;
+        if (next) request_w((kb + 1) * BK);
+        if (after) request_x(slot, (kb + 2) * BK);
+        const u32x4* buf = lds + slot * BUF;
         const int at = half * 32 + (l32 ^ swz(half));
         u32x4 a[MT][PL], b[NT][PL];
 #pragma unroll
@@ -275,10 +278,18 @@ __global__ __launch_bounds__(WM * 64) __attribute__((amdgpu_waves_per_eu(OCC, OC
 #pragma unroll
                 for (int j = 0; j < NT; ++j) acc[i][j] = Op<float>::mfma(a[i][Op<float>::PA[p]], b[j][Op<float>::PB[p]], acc[i][j]);
         __builtin_amdgcn_sched_barrier(0);                               // the next operands' splitting stays behind the products
-        if (kb + 1 < nk) store(lds + ((kb + 1) & 1) * BUF);
+        if (next) store(slot ^ 1, lds + (slot ^ 1) * BUF);
+    };
+    int kb = 0;
+    for (; kb + 3 < nk; kb += 2) {                                       // no branch around a request here: the waits count them
+        step(kb, 0, true, true);
+        step(kb + 1, 1, true, true);
     }
-    // the tile of the wavefront, 32 rows at a time, through its own part of LDS (pitch 100: rows start 4 banks apart)
+    step(kb, 0, kb + 1 < nk, kb + 2 < nk);
+    if (kb + 1 < nk) step(kb + 1, 1, kb + 2 < nk, false);
+    if (kb + 2 < nk) step(kb + 2, 0, false, false);
     __syncthreads();
+    // the tile of the wavefront, 32 rows at a time, through its own part of LDS (pitch 100: rows start 4 banks apart)
     constexpr int PITCH = BN + 4;
     float* mine = reinterpret_cast<float*>(lds) + wave * 32 * PITCH;
 #pragma unroll
@@ -708,7 +719,9 @@ __global__ __launch_bounds__(SMALL_WAVES * 64) void dense_small_kernel(const T* 
 }
 
 // ------------------------------------------------------------------------------------------
-// dW [P, K] = dY^T X, db [P] = column sums of dY.  A workgroup owns BM x BN of dW for one chunk of rows.
+// dW [P, K] = dY^T X, db [P] = column sums of dY.  A workgroup owns BM x BN of dW for one chunk of rows.  Operands are requested
+// two steps of 16 rows ahead: with one, a step waited for memory (8500 cycles of which 1150 are products; 219 000 rows 384 -> 96:
+// 190 us, with two 146; 35 569 rows 192 -> 576 and 192 -> 192 60 and 48).
 // ------------------------------------------------------------------------------------------
 template <int WM, int WN, int MT, int NT, int OCC>
 __global__ __launch_bounds__(WM * WN * 64) __attribute__((amdgpu_waves_per_eu(OCC, OCC))) void dense_wgrad_kernel(
@@ -729,56 +742,54 @@ __global__ __launch_bounds__(WM * WN * 64) __attribute__((amdgpu_waves_per_eu(OC
     const int64_t begin = chunk * rows_per_chunk, end = begin + rows_per_chunk < N ? begin + rows_per_chunk : N;
     const bool sums_here = part_b && k0 == 0;
 
-    Down ra[UA], rx[UB];
+    Down ra[2][UA], rx[2][UB];                                           // of the next two steps
     float bs[UA][2];
 #pragma unroll
     for (int i = 0; i < UA; ++i) bs[i][0] = bs[i][1] = 0.f;
     uint32_t oa[UA], ox[UB];
 #pragma unroll
     for (int i = 0; i < UA; ++i) {
-        const int u = threadIdx.x + i * THREADS;
+        const int u = min((int)threadIdx.x + i * THREADS, A_UNITS - 1);
         oa[i] = (uint32_t)((u / (BM / 2)) * 8 * P + min(p0 + (u % (BM / 2)) * 2, P - 2));
     }
 #pragma unroll
     for (int i = 0; i < UB; ++i) {
-        const int u = threadIdx.x + i * THREADS;
+        const int u = min((int)threadIdx.x + i * THREADS, B_UNITS - 1);
         ox[i] = (uint32_t)((u / (BN / 2)) * 8 * K + min(k0 + (u % (BN / 2)) * 2, K - 2));
     }
-    auto request = [&](int64_t n0) {
+    // 16 whole rows.  Lanes without a unit read the last one again: no branch around the loads, so that the waits can count them
+    auto request = [&](int slot, int64_t n0) {
         const float* yb = dy + n0 * P;
         const float* xb = x + n0 * K;
-        if (n0 + BK <= end) {
 #pragma unroll
-            for (int i = 0; i < UA; ++i)
-                if (A_UNITS % THREADS == 0 || (int)threadIdx.x + i * THREADS < A_UNITS)
+        for (int i = 0; i < UA; ++i)
 #pragma unroll
-                    for (int e = 0; e < 8; ++e) ra[i].load(e, yb + e * P + oa[i]);
+            for (int e = 0; e < 8; ++e) ra[slot][i].load(e, yb + e * P + oa[i]);
 #pragma unroll
-            for (int i = 0; i < UB; ++i)
-                if (B_UNITS % THREADS == 0 || (int)threadIdx.x + i * THREADS < B_UNITS)
+        for (int i = 0; i < UB; ++i)
 #pragma unroll
-                    for (int e = 0; e < 8; ++e) rx[i].load(e, xb + e * K + ox[i]);
-        } else {                                                         // the ragged end of the rows: zeros past it
-            const int left = (int)(end - n0);
+            for (int e = 0; e < 8; ++e) rx[slot][i].load(e, xb + e * K + ox[i]);
+    };
+    auto request_end = [&](int slot, int64_t n0) {                       // zeros past the last row
+        const float* yb = dy + n0 * P;
+        const float* xb = x + n0 * K;
+        const int left = (int)(end - n0);
 #pragma unroll
-            for (int i = 0; i < UA; ++i) {
-                const int u = threadIdx.x + i * THREADS, n = (u / (BM / 2)) * 8;
-                if (A_UNITS % THREADS == 0 || u < A_UNITS)
+        for (int i = 0; i < UA; ++i) {
+            const int n = min((int)threadIdx.x + i * THREADS, A_UNITS - 1) / (BM / 2) * 8;
 #pragma unroll
-                    for (int e = 0; e < 8; ++e) {
-                        if (n + e < left) ra[i].load(e, yb + e * P + oa[i]);
-                        else ra[i].zero(e);
-                    }
+            for (int e = 0; e < 8; ++e) {
+                if (n + e < left) ra[slot][i].load(e, yb + e * P + oa[i]);
+                else ra[slot][i].zero(e);
             }
+        }
 #pragma unroll
-            for (int i = 0; i < UB; ++i) {
-                const int u = threadIdx.x + i * THREADS, n = (u / (BN / 2)) * 8;
-                if (B_UNITS % THREADS == 0 || u < B_UNITS)
+        for (int i = 0; i < UB; ++i) {
+            const int n = min((int)threadIdx.x + i * THREADS, B_UNITS - 1) / (BN / 2) * 8;
 #pragma unroll
-                    for (int e = 0; e < 8; ++e) {
-                        if (n + e < left) rx[i].load(e, xb + e * K + ox[i]);
-                        else rx[i].zero(e);
-                    }
+            for (int e = 0; e < 8; ++e) {
+                if (n + e < left) rx[slot][i].load(e, xb + e * K + ox[i]);
+                else rx[slot][i].zero(e);
             }
         }
     };
@@ -787,7 +798,7 @@ __global__ __launch_bounds__(WM * WN * 64) __attribute__((amdgpu_waves_per_eu(OC
 #pragma unroll
         for (int q = 0; q < PL; ++q) dst[q * 64] = p[q];
     };
-    auto store = [&](u32x4* buf) {
+    auto store = [&](int slot, u32x4* buf) {
 #pragma unroll
         for (int i = 0; i < UA; ++i) {
             const int u = threadIdx.x + i * THREADS, pair = u % (BM / 2), c = u / (BM / 2);
@@ -795,9 +806,9 @@ __global__ __launch_bounds__(WM * WN * 64) __attribute__((amdgpu_waves_per_eu(OC
 #pragma unroll
                 for (int h = 0; h < 2; ++h) {
                     u32x4 p[PL];
-                    ra[i].planes(h, p);
+                    ra[slot][i].planes(h, p);
                     put(buf, BM / 32, pair * 2 + h, c, p);
-                    if (sums_here) bs[i][h] += ra[i].sum(h);
+                    if (sums_here) bs[i][h] += ra[slot][i].sum(h);
                 }
             }
         }
@@ -808,7 +819,7 @@ __global__ __launch_bounds__(WM * WN * 64) __attribute__((amdgpu_waves_per_eu(OC
 #pragma unroll
                 for (int h = 0; h < 2; ++h) {
                     u32x4 p[PL];
-                    rx[i].planes(h, p);
+                    rx[slot][i].planes(h, p);
                     put(buf + A_LDS, BN / 32, pair * 2 + h, c, p);
                 }
             }
@@ -819,13 +830,12 @@ __global__ __launch_bounds__(WM * WN * 64) __attribute__((amdgpu_waves_per_eu(OC
     for (int i = 0; i < MT; ++i)
 #pragma unroll
         for (int j = 0; j < NT; ++j) acc[i][j] = f32x16{0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-    const int nk = (int)((end - begin + BK - 1) / BK);
-    request(begin);
-    store(lds);
-    for (int kb = 0; kb < nk; ++kb) {
-        __syncthreads();
-        if (kb + 1 < nk) request(begin + (int64_t)(kb + 1) * BK);
-        const u32x4* buf = lds + (kb & 1) * BUF;
+    const int nk = (int)((end - begin + BK - 1) / BK), whole = (int)((end - begin) / BK);
+    request_end(0, begin);
+    if (nk > 1) request_end(1, begin + BK);
+    store(0, lds);
+    auto products = [&](int slot) {
+        const u32x4* buf = lds + slot * BUF;
         u32x4 a[MT][PL], b[NT][PL];
 #pragma unroll
         for (int i = 0; i < MT; ++i)
@@ -842,7 +852,26 @@ __global__ __launch_bounds__(WM * WN * 64) __attribute__((amdgpu_waves_per_eu(OC
 #pragma unroll
                 for (int j = 0; j < NT; ++j) acc[i][j] = Op<float>::mfma(a[i][Op<float>::PA[p]], b[j][Op<float>::PB[p]], acc[i][j]);
         __builtin_amdgcn_sched_barrier(0);                               // the next operands' splitting stays behind the products
-        if (kb + 1 < nk) store(lds + ((kb + 1) & 1) * BUF);
+    };
+    int kb = 0;
+    for (; kb + 3 < whole; kb += 2) {
+#pragma unroll
+        for (int slot = 0; slot < 2; ++slot) {
+            __syncthreads();
+            request(slot, begin + (int64_t)(kb + slot + 2) * BK);
+            products(slot);
+            store(slot ^ 1, lds + (slot ^ 1) * BUF);
+        }
+    }
+    for (; kb < nk; kb += 2) {
+#pragma unroll
+        for (int slot = 0; slot < 2; ++slot) {
+            if (kb + slot >= nk) break;
+            __syncthreads();
+            if (kb + slot + 2 < nk) request_end(slot, begin + (int64_t)(kb + slot + 2) * BK);
+            products(slot);
+            if (kb + slot + 1 < nk) store(slot ^ 1, lds + (slot ^ 1) * BUF);
+        }
     }
     float* pw = part_w + chunk * (int64_t)P * K;
 #pragma unroll
@@ -938,25 +967,28 @@ __global__ __launch_bounds__(SMALL_WAVES * 64) void dense_wgrad_small_kernel(con
     }
 }
 
-// out[e] = sum over chunks of part[chunk][e] for the weights and the bias behind each other; a block takes 16 x 4
-// outputs, 16 threads share an output, each adds every 16th chunk in order, the 16 sums in a fixed tree
-template <typename TO>
+// out[e] = sum over chunks of part[chunk][e] for the weights and the bias behind each other; a block takes 4 EL outputs,
+// CL = 256 / EL threads share four of them, each adds every CL-th chunk in order, the CL sums in a fixed tree.
+// EL = 16; 4 from 256 chunks on, where small layers leave the chip idle and the sums one after the other take the time
+// (1024 chunks of 144 x 48 and 48 x 48: 16.8 us on average, with 4 6.8)
+template <typename TO, int EL>
 __global__ __launch_bounds__(256) void dense_wgrad_sum_kernel(const float* __restrict__ part_w, const float* __restrict__ part_b, int chunks,
                                                               int64_t PK, int P, TO* __restrict__ dw, TO* __restrict__ db) {
-    __shared__ f32x4 sums[16][17];
-    const int el = threadIdx.x & 15, cl = threadIdx.x >> 4;
-    const int64_t e = ((int64_t)blockIdx.x * 16 + el) * 4;
+    constexpr int CL = 256 / EL;
+    __shared__ f32x4 sums[CL][EL + 1];
+    const int el = threadIdx.x % EL, cl = threadIdx.x / EL;
+    const int64_t e = ((int64_t)blockIdx.x * EL + el) * 4;
     const bool weight = e < PK, valid = weight || (db && e - PK < P);
     f32x4 sum = {0.f, 0.f, 0.f, 0.f};
     if (valid) {
         const float* src = weight ? part_w + e : part_b + (e - PK);
         const int64_t pitch = weight ? PK : P;
-        for (int c = cl; c < chunks; c += 16) sum += *reinterpret_cast<const f32x4*>(src + c * pitch);
+        for (int c = cl; c < chunks; c += CL) sum += *reinterpret_cast<const f32x4*>(src + c * pitch);
     }
     sums[cl][el] = sum;
     __syncthreads();
 #pragma unroll
-    for (int w = 8; w >= 1; w >>= 1) {
+    for (int w = CL / 2; w >= 1; w >>= 1) {
         if (cl < w) sums[cl][el] += sums[cl + w][el];
         __syncthreads();
     }
@@ -1135,8 +1167,12 @@ static int launch_wgrad_as(F* k, int threads, size_t lds, const WgradPlan& pl, c
                        P, K, pl.tiles_p, pl.tiles_k, pl.rows, ws, db ? part_b : nullptr);
     if (int rc = launch_ok("dense weight gradient")) return rc;
     const int64_t PK = (int64_t)P * K;
-    hipLaunchKernelGGL((dense_wgrad_sum_kernel<TO>), dim3((unsigned)((PK + P + 63) / 64)), dim3(256), 0, s, ws, part_b, pl.chunks, PK, P,
-                       static_cast<TO*>(dw), static_cast<TO*>(db));
+    if (pl.chunks >= 256)
+        hipLaunchKernelGGL((dense_wgrad_sum_kernel<TO, 4>), dim3((unsigned)((PK + P + 15) / 16)), dim3(256), 0, s, ws, part_b, pl.chunks, PK, P,
+                           static_cast<TO*>(dw), static_cast<TO*>(db));
+    else
+        hipLaunchKernelGGL((dense_wgrad_sum_kernel<TO, 16>), dim3((unsigned)((PK + P + 63) / 64)), dim3(256), 0, s, ws, part_b, pl.chunks, PK, P,
+                           static_cast<TO*>(dw), static_cast<TO*>(db));
     return launch_ok("dense weight gradient, sums");
 }
 
