@@ -1151,12 +1151,23 @@ static WgradPlan wgrad_plan(int64_t N, int P, int K, int bk, int bm, int bn, int
 
 // rows up to which one launch of 32 x 32 tiles beats row chunks and their sums (284 rows 384 -> 1152: 19 us in chunks)
 constexpr int64_t WGRAD_SMALL_ROWS = 1024;
-// fp32: 128 x 192 tiles where dW has that many columns, otherwise 96 x 96 with more workgroups per compute unit (35 569 rows
-// 192 -> 576: 91 and 78 us).  16 bit: 96 x 96 (219 000 rows 96 -> 288: 39 us; 192 x 192 tiles 58, 192 x 96 44).
-static bool wgrad_large(int K) { return K >= 192; }
+// Tiles of dW.  fp32: by the columns it has, since a tile wider than dW works on copies of its last columns.
+//   128 x 192 from 192 columns of X on (35 569 rows 192 -> 576: 91 and 78 us with 96 x 96), 64 x 192 where dY has at most 64;
+//   192 x 64 and 64 x 64 up to 64 columns of X (112 700 rows 48 -> 144 and 48 -> 48: 32 and 20 us, 39 on average with 96 x 96);
+//   96 x 96 between, with more workgroups per compute unit.
+// 16 bit: 96 x 96 (219 000 rows 96 -> 288: 39 us; 192 x 192 tiles 58, 192 x 96 44).
+struct WgradTile {
+    int bm, bn, per_cu;
+};
+static WgradTile wgrad_tile(int P, int K) {
+    if (K >= 192) return P <= 64 ? WgradTile{64, 192, 2} : WgradTile{128, 192, 2};
+    if (K <= 64) return P <= 64 ? WgradTile{64, 64, 4} : WgradTile{192, 64, 2};
+    return {96, 96, 4};
+}
 static WgradPlan wgrad_plan(int dtype, int64_t N, int P, int K) {
-    if (dtype == SSWIN_F32) return wgrad_large(K) ? wgrad_plan(N, P, K, 16, 128, 192, 2) : wgrad_plan(N, P, K, 16, 96, 96, 4);
-    return wgrad_plan(N, P, K, 32, 96, 96, 3);
+    if (dtype != SSWIN_F32) return wgrad_plan(N, P, K, 32, 96, 96, 3);
+    const WgradTile t = wgrad_tile(P, K);
+    return wgrad_plan(N, P, K, 16, t.bm, t.bn, t.per_cu);
 }
 
 template <typename T, typename TO, typename F>
@@ -1186,9 +1197,13 @@ static int launch_wgrad(const void* dy, const void* x, int64_t N, int P, int K, 
     }
     if constexpr (Op<T>::PL == 3) {
         const WgradPlan pl = wgrad_plan(SSWIN_F32, N, P, K);
-        constexpr size_t large = 2 * (2 * 2 + 2 * 3) * 3 * 1024, plain = 2 * (3 + 3) * 3 * 1024;         // two buffers of (row tiles) x 3 planes
-        if (wgrad_large(K)) return launch_wgrad_as<T, TO>(dense_wgrad_kernel<2, 2, 2, 3, 2>, 256, large, pl, dy, x, N, P, K, dw, db, ws, s);
-        return launch_wgrad_as<T, TO>(dense_wgrad_kernel<3, 1, 1, 3, 3>, 192, plain, pl, dy, x, N, P, K, dw, db, ws, s);
+        const WgradTile t = wgrad_tile(P, K);
+        const size_t lds = 2 * (size_t)((t.bm + t.bn) / 32) * 3 * 1024;                                  // two buffers of (row tiles) x 3 planes
+        if (t.bm == 128) return launch_wgrad_as<T, TO>(dense_wgrad_kernel<2, 2, 2, 3, 2>, 256, lds, pl, dy, x, N, P, K, dw, db, ws, s);
+        if (t.bn == 192) return launch_wgrad_as<T, TO>(dense_wgrad_kernel<2, 2, 1, 3, 2>, 256, lds, pl, dy, x, N, P, K, dw, db, ws, s);
+        if (t.bm == 192) return launch_wgrad_as<T, TO>(dense_wgrad_kernel<3, 1, 2, 2, 2>, 192, lds, pl, dy, x, N, P, K, dw, db, ws, s);
+        if (t.bm == 64) return launch_wgrad_as<T, TO>(dense_wgrad_kernel<2, 1, 1, 2, 3>, 128, lds, pl, dy, x, N, P, K, dw, db, ws, s);
+        return launch_wgrad_as<T, TO>(dense_wgrad_kernel<3, 1, 1, 3, 3>, 192, lds, pl, dy, x, N, P, K, dw, db, ws, s);
     } else {
         constexpr size_t lds = 3 * 2 * 32 * 192;                         // three stages of two tiles of 32 x 96
         return launch_wgrad_as<T, TO>(dense16_wgrad_kernel<T, 3, 1, 1, 3, 3>, 192, lds, wgrad_plan(SSWIN_F16, N, P, K), dy, x, N, P, K, dw, db, ws, s);
