@@ -8,8 +8,8 @@
 //
 // dense_rows_kernel (fp32): a workgroup of WM wavefronts owns BM = 32 MT WM rows and 96 columns.  Both operands pass through
 // registers, where they are split, into LDS in matrix operand order, [row tile][plane][lane] pieces of 16 bytes, so that every
-// operand read is one conflict-free 16-byte read per lane; two buffers, one barrier per 16 columns of the reduction, the next
-// 16 in flight meanwhile.  96 columns because every layer of a stage has a multiple of 48.  The tile of the result goes back
+// operand read is one conflict-free 16-byte read per lane; 32 columns of the reduction at a time, the next 32 in flight
+// meanwhile.  96 columns because every layer of a stage has a multiple of 48.  The tile of the result goes back
 // through LDS, so that bias, residual and result are touched in 16-byte pieces of whole row segments.
 // dense16_rows_kernel (16 bit): tiles straight from memory to LDS.
 // dense_small_kernel: few rows and many channels (the deep stages): 32 x 32 tiles, the wavefronts of a workgroup share
@@ -144,7 +144,7 @@ template <> __device__ __forceinline__ float half_of<__hip_bfloat16>(uint32_t w,
 
 // position of (row, 8-value chunk) inside its 32-row operand block: the rows of a chunk are rotated by the chunk, so
 // that lanes which hold the chunks of one row write to different banks
-__device__ __forceinline__ int swz(int chunk) { return (chunk & 1) * 4; }
+__device__ __forceinline__ int swz(int chunk) { return (chunk & 1) * 4 | (chunk & 2); }
 
 // workgroups b, b + 8, b + 16 ... share an XCD and its L2: the column blocks of one row block are dealt to such workgroups
 __device__ __forceinline__ void block_of(int groups, int& cg, int64_t& rb) {
@@ -164,11 +164,11 @@ __device__ __forceinline__ void block_of(int groups, int& cg, int64_t& rb) {
 template <int EPI, bool DOWN, int WM, int MT, int OCC>
 __global__ __launch_bounds__(WM * 64) __attribute__((amdgpu_waves_per_eu(OCC, OCC))) void dense_rows_kernel(
     const float* __restrict__ x, int64_t N, int K, const float* __restrict__ w, int P, int groups, Epilogue ep) {
-    constexpr int PL = 3, BK = 16, KC = BK / 8;
+    constexpr int PL = 3, BK = 32, KC = BK / 8;
     constexpr int NT = 3, BN = 96, BM = WM * MT * 32, THREADS = WM * 64;
     constexpr int A_UNITS = BM * KC, UA = (A_UNITS + THREADS - 1) / THREADS;
     constexpr int B_UNITS = (DOWN ? BN / 2 : BN) * KC, UB = (B_UNITS + THREADS - 1) / THREADS;
-    constexpr int A_LDS = BM / 32 * PL * 64, B_LDS = NT * PL * 64, BUF = A_LDS + B_LDS;      // 16-byte pieces
+    constexpr int A_LDS = BM / 32 * PL * 64, B_LDS = NT * PL * 64;       // 16-byte pieces of 16 columns
     extern __shared__ __attribute__((aligned(16))) u32x4 lds[];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, half = lane >> 5, l32 = lane & 31;
     int cg;
@@ -178,7 +178,7 @@ __global__ __launch_bounds__(WM * 64) __attribute__((amdgpu_waves_per_eu(OCC, OC
     const int col0 = cg * BN;
 
     // addresses: a uniform base that moves along the reduction plus 32-bit lane offsets formed once
-    Along<float> ra[2][UA];                                              // of the next two steps
+    Along<float> ra[UA];
     typename std::conditional<DOWN, Down, Along<float>>::type rw[UB];
     uint32_t oa[UA], ow[UB];
     const int last = (int)(N - 1 - row0 < BM - 1 ? N - 1 - row0 : BM - 1);   // rows past the end repeat the last one
@@ -194,21 +194,24 @@ __global__ __launch_bounds__(WM * 64) __attribute__((amdgpu_waves_per_eu(OCC, OC
         else ow[i] = (uint32_t)(min(col0 + u / KC, P - 1) * K + (u % KC) * 8);
     }
     const float* xb = x + row0 * K;
-    static_assert(A_UNITS % THREADS == 0, "every lane reads the same number of pieces of x");
-    auto request_x = [&](int slot, int k0) {
+    // 32 columns from k0 on; where only 16 are left, the upper half repeats them
+    auto request = [&](int k0) {
+        const bool half_step = k0 + 16 == K;
 #pragma unroll
-        for (int i = 0; i < UA; ++i) ra[slot][i].load(xb + k0 + oa[i]);
-    };
-    auto request_w = [&](int k0) {
+        for (int i = 0; i < UA; ++i) {
+            const int u = threadIdx.x + i * THREADS;
+            if (A_UNITS % THREADS == 0 || u < A_UNITS) ra[i].load(xb + k0 + (oa[i] - (half_step ? (u % KC / 2) * 16 : 0)));
+        }
 #pragma unroll
         for (int i = 0; i < UB; ++i) {
             const int u = threadIdx.x + i * THREADS;
             if (B_UNITS % THREADS == 0 || u < B_UNITS) {
                 if constexpr (DOWN) {
+                    const uint32_t at = ow[i] - (half_step ? u / (BN / 2) / 2 * 16 * P : 0);
 #pragma unroll
-                    for (int e = 0; e < 8; ++e) rw[i].load(e, w + (int64_t)(k0 + e) * P + ow[i]);
+                    for (int e = 0; e < 8; ++e) rw[i].load(e, w + (int64_t)(k0 + e) * P + at);
                 } else {
-                    rw[i].load(w + k0 + ow[i]);
+                    rw[i].load(w + k0 + (ow[i] - (half_step ? (u % KC / 2) * 16 : 0)));
                 }
             }
         }
@@ -218,13 +221,15 @@ __global__ __launch_bounds__(WM * 64) __attribute__((amdgpu_waves_per_eu(OCC, OC
 #pragma unroll
         for (int q = 0; q < PL; ++q) dst[q * 64] = p[q];
     };
-    auto store = [&](int slot, u32x4* buf) {
+    auto store = [&](u32x4* buf) {
 #pragma unroll
         for (int i = 0; i < UA; ++i) {
             const int u = threadIdx.x + i * THREADS;
-            u32x4 p[PL];
-            ra[slot][i].planes(p);
-            put(buf, BM / 32, u / KC, u % KC, p);
+            if (A_UNITS % THREADS == 0 || u < A_UNITS) {
+                u32x4 p[PL];
+                ra[i].planes(p);
+                put(buf, BM / 32, u / KC, u % KC, p);
+            }
         }
 #pragma unroll
         for (int i = 0; i < UB; ++i) {
@@ -233,12 +238,12 @@ __global__ __launch_bounds__(WM * 64) __attribute__((amdgpu_waves_per_eu(OCC, OC
                 u32x4 p[PL];
                 if constexpr (DOWN) {
                     rw[i].planes(0, p);
-                    put(buf + A_LDS, NT, (u % (BN / 2)) * 2, u / (BN / 2), p);
+                    put(buf + 2 * A_LDS, NT, (u % (BN / 2)) * 2, u / (BN / 2), p);
                     rw[i].planes(1, p);
-                    put(buf + A_LDS, NT, (u % (BN / 2)) * 2 + 1, u / (BN / 2), p);
+                    put(buf + 2 * A_LDS, NT, (u % (BN / 2)) * 2 + 1, u / (BN / 2), p);
                 } else {
                     rw[i].planes(p);
-                    put(buf + A_LDS, NT, u / KC, u % KC, p);
+                    put(buf + 2 * A_LDS, NT, u / KC, u % KC, p);
                 }
             }
         }
@@ -249,45 +254,36 @@ __global__ __launch_bounds__(WM * 64) __attribute__((amdgpu_waves_per_eu(OCC, OC
     for (int i = 0; i < MT; ++i)
 #pragma unroll
         for (int j = 0; j < NT; ++j) acc[i][j] = f32x16{0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-    const int nk = K / BK;
-    // x comes from memory: two steps ahead (219 000 rows 288 -> 96: 106 us with one, 96 with two).  w lies in L2: one step
-    // ahead, and requested before x, so that waiting for it leaves the x behind it in flight.
-    request_w(0);
-    request_x(0, 0);
-    if (nk > 1) request_x(1, BK);
-    store(0, lds);
-    auto step = [&](int kb, int slot, bool next, bool after) {           // next, after: whether there is a step kb + 1, kb + 2
+    // One buffer of 32 columns, whole 128-byte lines of x and w: in steps of 16 columns a line was fetched from L2 twice, once
+    // per half, since the rows of three workgroups overflow L1 in between (219 000 rows 288 -> 96 and 384 -> 96, input gradients: 96 us
+    // on average, with whole lines 87; 384 -> 96 with a residual 171 and 166; the traffic's own time is 72 and 95).
+    request(0);
+    for (int k0 = 0; k0 < K; k0 += BK) {
+        if (k0) __syncthreads();                                         // the last step's operands have been read
+        store(lds);
+        if (k0 + BK < K) request(k0 + BK);
         __syncthreads();
-        if (next) request_w((kb + 1) * BK);
-        if (after) request_x(slot, (kb + 2) * BK);
-        const u32x4* buf = lds + slot * BUF;
-        const int at = half * 32 + (l32 ^ swz(half));
-        u32x4 a[MT][PL], b[NT][PL];
 #pragma unroll
-        for (int i = 0; i < MT; ++i)
-#pragma unroll
-            for (int q = 0; q < PL; ++q) a[i][q] = buf[((wave * MT + i) * PL + q) * 64 + at];
-#pragma unroll
-        for (int j = 0; j < NT; ++j)
-#pragma unroll
-            for (int q = 0; q < PL; ++q) b[j][q] = buf[A_LDS + (j * PL + q) * 64 + at];
-#pragma unroll
-        for (int p = 0; p < Op<float>::NP; ++p)
+        for (int h = 0; h < 2; ++h) {
+            if (h && k0 + 16 == K) break;
+            const int at = half * 32 + (l32 ^ swz(2 * h + half));
+            u32x4 a[MT][PL], b[NT][PL];
 #pragma unroll
             for (int i = 0; i < MT; ++i)
 #pragma unroll
-                for (int j = 0; j < NT; ++j) acc[i][j] = Op<float>::mfma(a[i][Op<float>::PA[p]], b[j][Op<float>::PB[p]], acc[i][j]);
-        __builtin_amdgcn_sched_barrier(0);                               // the next operands' splitting stays behind the products
-        if (next) store(slot ^ 1, lds + (slot ^ 1) * BUF);
-    };
-    int kb = 0;
-    for (; kb + 3 < nk; kb += 2) {                                       // no branch around a request here: the waits count them
-        step(kb, 0, true, true);
-        step(kb + 1, 1, true, true);
+                for (int q = 0; q < PL; ++q) a[i][q] = lds[h * A_LDS + ((wave * MT + i) * PL + q) * 64 + at];
+#pragma unroll
+            for (int j = 0; j < NT; ++j)
+#pragma unroll
+                for (int q = 0; q < PL; ++q) b[j][q] = lds[2 * A_LDS + h * B_LDS + (j * PL + q) * 64 + at];
+#pragma unroll
+            for (int p = 0; p < Op<float>::NP; ++p)
+#pragma unroll
+                for (int i = 0; i < MT; ++i)
+#pragma unroll
+                    for (int j = 0; j < NT; ++j) acc[i][j] = Op<float>::mfma(a[i][Op<float>::PA[p]], b[j][Op<float>::PB[p]], acc[i][j]);
+        }
     }
-    step(kb, 0, kb + 1 < nk, kb + 2 < nk);
-    if (kb + 1 < nk) step(kb + 1, 1, kb + 2 < nk, false);
-    if (kb + 2 < nk) step(kb + 2, 0, false, false);
     __syncthreads();
     // the tile of the wavefront, 32 rows at a time, through its own part of LDS (pitch 100: rows start 4 banks apart)
     constexpr int PITCH = BN + 4;
