@@ -311,8 +311,11 @@ int sswin_token_plan_totals(int64_t* totals, int H, int64_t g_cap);
  * skipped (totals all zero).  After waiting for `stream`, decode each totals_out with
  * sswin_token_plan_totals.  Rejects count > 4.
  * flags: SSWIN_PLAN_ORDER_ONLY writes only the first row of `tokens` (voxel of rank r; `tokens` may then hold N
- * entries): what the stride-2 merge reads (sswin_pool_windows), four scattered stores per voxel fewer. */
+ * entries): what the stride-2 merge reads (sswin_pool_windows).
+ * SSWIN_PLAN_TOTALS_DIRECT: totals_out is pinned host memory the device can write (hipHostMalloc): the raw totals are stored by
+ * the last kernel instead of a copy behind it. */
 #define SSWIN_PLAN_ORDER_ONLY 1
+#define SSWIN_PLAN_TOTALS_DIRECT 2
 typedef struct sswin_token_plan_desc {
     const int32_t* indices;
     int64_t N;

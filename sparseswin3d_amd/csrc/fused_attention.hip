@@ -77,6 +77,7 @@ struct TokenPlanArgs {
     int32_t* tokens;         // [5 * N]
     int blocks;              // ceil(B / window slots per block) of the launch the plan goes into
     int order_only;          // tokens holds its first row only (voxel of rank r)
+    int64_t* host_totals;    // host memory the totals go to directly, or null
 };
 
 __device__ __forceinline__ int32_t* tp_counters(const TokenPlanArgs& a) { return reinterpret_cast<int32_t*>(a.totals + 2); }
@@ -279,15 +280,43 @@ __device__ __forceinline__ void tp_phase_windows(const TokenPlanArgs& a, int blk
     }
 }
 
-// per voxel -> entries by token rank: source voxel, first rank and size of its window, pos, window
-__device__ __forceinline__ void tp_phase_rank(const TokenPlanArgs& a, int64_t gtid, int64_t gthreads) {
-    const int W = a.W;
-    const int64_t N = a.N;
-    int32_t* order = a.tokens;
+// per word of the bitmap -> what follows from it by token rank: first rank and size of the window, pos, window.  The tokens
+// of a word are neighbours, so these four rows are written in runs; from the voxels, which come in any order, each was a
+// scattered store (219 000 voxels in windows of 7^3, three plans: 57 us against 42)
+__device__ __forceinline__ void tp_phase_tokens(const TokenPlanArgs& a, int64_t gtid, int64_t gthreads) {
+    if (a.order_only) return;
+    const int64_t N = a.N, words = (int64_t)a.B * a.W;
     int32_t* tok_T = a.tokens + N;
     int32_t* tok_c = a.tokens + 2 * N;
     int32_t* tok_pos = a.tokens + 3 * N;
     int32_t* tok_win = a.tokens + 4 * N;
+    for (int64_t i = gtid; i < words; i += gthreads) {
+        uint32_t x = a.bits[i];
+        if (!x) continue;
+        const int w = (int)(a.W == 4 ? i >> 2 : i / a.W), word = (int)(i - (int64_t)w * a.W);
+        int below = 0, c = 0;
+        for (int k = 0; k < a.W; ++k) {
+            const int pc = __popc(a.bits[(int64_t)w * a.W + k]);
+            c += pc;
+            below += k < word ? pc : 0;
+        }
+        const int T = a.win_T[w];
+        for (int64_t r = (int64_t)T + below; x && r < N; ++r, x &= x - 1) {
+            tok_T[r] = T;
+            tok_c[r] = c;
+            tok_pos[r] = word * 32 + __ffs((int)x) - 1;
+            tok_win[r] = w;
+        }
+    }
+}
+
+// per voxel -> source voxel by token rank, and the token records
+__device__ __forceinline__ void tp_phase_rank(const TokenPlanArgs& a, int64_t gtid, int64_t gthreads) {
+    const int W = a.W;
+    const int64_t N = a.N;
+    int32_t* order = a.tokens;
+    // the totals are complete since the windows phase
+    if (gtid < 8 && a.host_totals) __hip_atomic_store(a.host_totals + gtid, a.totals[gtid], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     for (int64_t v = gtid; v < N; v += gthreads) {
         const int2 wp = *reinterpret_cast<const int2*>(a.ind + 2 * v);
         if ((unsigned)wp.x >= (unsigned)a.B || (unsigned)wp.y >= (unsigned)a.n) continue;   // counted in phase 2
@@ -315,11 +344,6 @@ __device__ __forceinline__ void tp_phase_rank(const TokenPlanArgs& a, int64_t gt
         const int r = T + below;
         if (r < N) {                                            // duplicates cannot push a rank past the end, but stay inside anyway
             order[r] = (int32_t)v;
-            if (a.order_only) continue;
-            tok_T[r] = T;
-            tok_c[r] = c;
-            tok_pos[r] = wp.y;
-            tok_win[r] = wp.x;
         }
         if (a.recs != nullptr) {
             // Token records of the window-resident kernels: one record of 32 {voxel, pos} entries per (window, tile
@@ -372,8 +396,12 @@ __global__ __launch_bounds__(TP_BLOCK) void tp_windows_kernel(TokenPlanBatch b) 
     const TokenPlanArgs& a = b.p[blockIdx.y];
     if ((int)blockIdx.x < a.blocks) tp_phase_windows<ITEMS>(a, blockIdx.x, sh);
 }
-__global__ __launch_bounds__(256) void tp_rank_kernel(TokenPlanBatch b) {
-    tp_phase_rank(b.p[blockIdx.y], (int64_t)blockIdx.x * 256 + threadIdx.x, (int64_t)gridDim.x * 256);
+// the first voxel_blocks blocks: voxels, the others: words
+__global__ __launch_bounds__(256) void tp_rank_kernel(TokenPlanBatch b, int voxel_blocks) {
+    if ((int)blockIdx.x < voxel_blocks)
+        tp_phase_rank(b.p[blockIdx.y], (int64_t)blockIdx.x * 256 + threadIdx.x, (int64_t)voxel_blocks * 256);
+    else
+        tp_phase_tokens(b.p[blockIdx.y], (int64_t)(blockIdx.x - voxel_blocks) * 256 + threadIdx.x, (int64_t)(gridDim.x - voxel_blocks) * 256);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -1501,7 +1529,8 @@ size_t sswin_token_plan_task_ints(int64_t N, int64_t g_cap, int H) {
 static int token_plan_args(const int32_t* indices, int64_t N, int B, int n, int H, int32_t* tokens, int32_t* plan,
                            int64_t g_cap, int32_t* tasks, int64_t* totals_out, void* ws, size_t ws_bytes, int flags,
                            TokenPlanArgs& a) {
-    SSWIN_CHECK((flags & ~SSWIN_PLAN_ORDER_ONLY) == 0, "token_plan: unknown flags %d", flags);
+    SSWIN_CHECK((flags & ~(SSWIN_PLAN_ORDER_ONLY | SSWIN_PLAN_TOTALS_DIRECT)) == 0, "token_plan: unknown flags %d", flags);
+    a.host_totals = (flags & SSWIN_PLAN_TOTALS_DIRECT) ? totals_out : nullptr;
     a.order_only = (flags & SSWIN_PLAN_ORDER_ONLY) ? 1 : 0;
     SSWIN_CHECK(N > 0 && B > 0 && n > 0 && H > 0 && H < 256, "token_plan: bad sizes");
     SSWIN_CHECK(indices && tokens && plan && ws && totals_out, "token_plan: null pointer");
@@ -1537,13 +1566,14 @@ static int token_plan_args(const int32_t* indices, int64_t N, int B, int n, int 
 // The five launches for `count` plans (1..TP_MAX_BATCH) and the copies of their raw totals to the host.
 static int token_plan_launch(const TokenPlanArgs* args, int64_t* const* totals_out, int count, hipStream_t s) {
     TokenPlanBatch b;
-    size_t words = 0;
+    size_t words = 0, token_words = 0;
     int64_t voxels = 0;
     int blocks = 0;
     for (int k = 0; k < TP_MAX_BATCH; ++k) {
         b.p[k] = args[k < count ? k : 0];  // unused slots repeat the first plan; no block ever reads them
         if (k >= count) continue;
         words = std::max(words, (size_t)args[k].B * args[k].W);
+        if (!args[k].order_only) token_words = std::max(token_words, (size_t)args[k].B * args[k].W);
         voxels = std::max(voxels, args[k].N);
         blocks = std::max(blocks, args[k].blocks);
     }
@@ -1568,11 +1598,12 @@ static int token_plan_launch(const TokenPlanArgs* args, int64_t* const* totals_o
         hipLaunchKernelGGL(tp_block_sums_kernel<1>, dim3((unsigned)blocks, y), dim3(TP_BLOCK), 0, s, b);
         hipLaunchKernelGGL(tp_windows_kernel<1>, dim3((unsigned)blocks, y), dim3(TP_BLOCK), 0, s, b);
     }
-    hipLaunchKernelGGL(tp_rank_kernel, dim3(nb, y), dim3(256), 0, s, b);
+    const unsigned word_blocks = (unsigned)std::max<size_t>(1, std::min<size_t>((token_words + 255) / 256, 4096));
+    hipLaunchKernelGGL(tp_rank_kernel, dim3(nb + word_blocks, y), dim3(256), 0, s, b, (int)nb);
     if (launch_ok("token plan")) return 1;
     // raw totals: the caller decodes them with sswin_token_plan_totals once the copies have landed
     for (int k = 0; k < count; ++k)
-        SSWIN_HIP(hipMemcpyAsync(totals_out[k], args[k].totals, 8 * sizeof(int64_t), hipMemcpyDeviceToHost, s));
+        if (!args[k].host_totals) SSWIN_HIP(hipMemcpyAsync(totals_out[k], args[k].totals, 8 * sizeof(int64_t), hipMemcpyDeviceToHost, s));
     return 0;
 }
 

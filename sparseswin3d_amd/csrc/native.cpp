@@ -166,7 +166,7 @@ void enqueue_plans(const std::vector<PlanPtr>& plans) {
             TORCH_CHECK(p.indices.device() == like.device(), "TokenPlan.batch: all index sets must live on one device");
             d[i] = sswin_token_plan_desc{};
             d[i].indices = i32(p.indices), d[i].N = p.N, d[i].B = (int32_t)p.B, d[i].n = (int32_t)p.n, d[i].H = p.H;
-            d[i].flags = p.order_only ? 1 : 0;
+            d[i].flags = (p.order_only ? SSWIN_PLAN_ORDER_ONLY : 0) | SSWIN_PLAN_TOTALS_DIRECT;
             d[i].tokens = i32(p.tokens), d[i].plan = i32(p.plan), d[i].g_cap = p.g_cap, d[i].tasks = i32(p.tasks);
             d[i].totals_out = p.totals.data_ptr<int64_t>(), d[i].ws = p.ws.data_ptr(), d[i].ws_bytes = (size_t)p.ws.numel();
         }
