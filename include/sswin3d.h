@@ -389,6 +389,9 @@ int sswin_fused_bias_grad(const int32_t* plan, int64_t g_cap, int64_t G, const i
  * swin3d_base.py:644-647 in one launch (code as for sswin_bias_table_grad).  Asynchronous. */
 int sswin_bias_from_table(const float* table, int table_rows, int H, const int32_t* code, int offset0,
                           int n, float* bias, void* stream);
+/* The same from a table of fp32, fp16 or bf16 values. */
+int sswin_bias_from_typed_table(int dtype, const void* table, int table_rows, int H, const int32_t* code, int offset0, int n,
+                                float* bias, void* stream);
 
 /* Gradient of the relative position bias table itself (swin3d_base.py:624-652 gathers the
  * [H,n,n] bias from a [(2w-1)^3, H] table by relative_position_index; autograd scatters back with

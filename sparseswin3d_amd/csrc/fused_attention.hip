@@ -1142,14 +1142,15 @@ __global__ __launch_bounds__(256) void rpb_grad_reduce_kernel(const float* __res
 // ------------------------------------------------------------------------------------------
 // bias[h][p][q] = table[code[p] - code[q] + offset0][h]: the gather of swin3d_base.py:644-647 and its
 // permute(2, 0, 1) in one pass (entries whose table row is out of range read as zero).
-__global__ __launch_bounds__(256) void rpb_gather_kernel(const float* __restrict__ table, int rows, int H,
+template <typename T>
+__global__ __launch_bounds__(256) void rpb_gather_kernel(const T* __restrict__ table, int rows, int H,
                                                          const int32_t* __restrict__ code, int offset0, int n,
                                                          float* __restrict__ bias) {
     const int e = blockIdx.x * 256 + threadIdx.x;
     if (e >= n * n) return;
     const int p = e / n, q = e - p * n;
     const unsigned r = (unsigned)(code[p] - code[q] + offset0);
-    for (int h = 0; h < H; ++h) bias[(int64_t)h * n * n + e] = r < (unsigned)rows ? table[(int64_t)r * H + h] : 0.f;
+    for (int h = 0; h < H; ++h) bias[(int64_t)h * n * n + e] = r < (unsigned)rows ? to_acc(table[(int64_t)r * H + h]) : 0.f;
 }
 
 constexpr int RPBT_MAX_ROWS = 4096;
@@ -1916,10 +1917,24 @@ int sswin_bias_table_grad_tasks(const int32_t* tasks, int64_t g_cap, const int64
 
 int sswin_bias_from_table(const float* table, int table_rows, int H, const int32_t* code, int offset0, int n, float* bias,
                           void* stream) {
+    return sswin_bias_from_typed_table(SSWIN_F32, table, table_rows, H, code, offset0, n, bias, stream);
+}
+
+int sswin_bias_from_typed_table(int dtype, const void* table, int table_rows, int H, const int32_t* code, int offset0, int n, float* bias,
+                                void* stream) {
     SSWIN_CHECK(table_rows > 0 && H > 0 && n > 0 && n <= 4096, "bias_from_table: bad sizes");
     SSWIN_CHECK(table && code && bias, "bias_from_table: null pointer");
-    hipLaunchKernelGGL(rpb_gather_kernel, dim3((unsigned)((n * n + 255) / 256)), dim3(256), 0, static_cast<hipStream_t>(stream),
-                       table, table_rows, H, code, offset0, n, bias);
+    const dim3 grid((unsigned)((n * n + 255) / 256)), block(256);
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    if (dtype == SSWIN_F32)
+        hipLaunchKernelGGL(rpb_gather_kernel<float>, grid, block, 0, s, static_cast<const float*>(table), table_rows, H, code, offset0, n, bias);
+    else if (dtype == SSWIN_F16)
+        hipLaunchKernelGGL(rpb_gather_kernel<__half>, grid, block, 0, s, static_cast<const __half*>(table), table_rows, H, code, offset0, n, bias);
+    else if (dtype == SSWIN_BF16)
+        hipLaunchKernelGGL(rpb_gather_kernel<__hip_bfloat16>, grid, block, 0, s, static_cast<const __hip_bfloat16*>(table), table_rows, H, code, offset0, n,
+                           bias);
+    else
+        return fail("bias_from_table: a table of type %d", dtype);
     return launch_ok("bias_from_table");
 }
 

@@ -379,11 +379,11 @@ Tensor attention_forward(Attention& a, const Tensor& qkv, const Tensor& bias, At
     const int64_t N = qkv.size(0), D = qkv.size(1) / 3;
     const int hd = (int)(D / a.H), dt = code_of(qkv.scalar_type());
     void* s = current_stream(qkv);
-    const Tensor table32 = bias.to(at::kFloat).contiguous();
+    const auto fopt = qkv.options().dtype(at::kFloat);
     if (a.flash) {
-        saved.bias32 = table32;
+        const Tensor table32 = saved.bias32 = bias.to(at::kFloat).contiguous();
         saved.words = at::empty({2, N}, tp.tokens.options());
-        saved.aux = at::empty({a.H, N}, table32.options());
+        saved.aux = at::empty({a.H, N}, fopt);
         Tensor o = at::empty({N, D}, qkv.options());
         RUN(sswin_flash_tokens(i32(tp.plan), tp.g_cap, tp.G, i32(tp.tokens), N, a.H, a.n, i32(a.code), a.mask.defined() ? a.mask.data_ptr<int8_t>() : nullptr,
                                a.regions(), i32(saved.words), i32(saved.words) + N, s));
@@ -392,21 +392,23 @@ Tensor attention_forward(Attention& a, const Tensor& qkv, const Tensor& bias, At
         return o;
     }
     if (a.code.defined()) {
-        saved.bias32 = at::empty({a.H, a.n, a.n}, table32.options());
-        RUN(sswin_bias_from_table(f32(table32), (int)table32.size(0), a.H, i32(a.code), a.offset0, a.n, f32(saved.bias32), s));
+        const ScalarType kind = bias.scalar_type();
+        const Tensor table = (kind == at::kHalf || kind == at::kBFloat16 ? bias : bias.to(at::kFloat)).contiguous();
+        saved.bias32 = at::empty({a.H, a.n, a.n}, fopt);
+        RUN(sswin_bias_from_typed_table(code_of(table.scalar_type()), ptr(table), (int)table.size(0), a.H, i32(a.code), a.offset0, a.n, f32(saved.bias32), s));
     } else {
-        saved.bias32 = table32;
+        saved.bias32 = bias.to(at::kFloat).contiguous();
     }
     Tensor out = at::empty({N, D}, qkv.options());
     const int8_t* mask = a.mask.defined() ? a.mask.data_ptr<int8_t>() : nullptr;
     if (a.resident) {
-        saved.aux = at::empty({std::max<int64_t>(a.H * N, 1)}, table32.options());
+        saved.aux = at::empty({std::max<int64_t>(a.H * N, 1)}, fopt);
         RUN(sswin_window_attention_forward(dt, i32(tp.tasks), tp.g_cap, tp.buckets, i32(tp.tokens), N, a.H, hd, ptr(qkv), 3 * D, 0, ptr(qkv), 3 * D, (int)D,
                                            ptr(qkv), 3 * D, (int)(2 * D), (float)a.scale, f32(saved.bias32), a.n, mask, a.regions(), ptr(out), D, 0,
                                            f32(saved.aux), s));
         return out;
     }
-    Tensor p = saved.aux = at::empty({tp.A}, table32.options());
+    Tensor p = saved.aux = at::empty({tp.A}, fopt);
     RUN(sswin_fused_tokens_to_sq(dt, 1, i32(tp.plan), tp.g_cap, tp.G, i32(tp.tokens), tp.N, tp.H, hd, ptr(qkv), 3 * D, 0, ptr(qkv), 3 * D, (int)D,
                                  (float)a.scale, f32(saved.bias32), a.n, mask, a.regions(), f32(p), nullptr, s));
     RUN(sswin_group_softmax(0, i32(tp.plan), tp.g_cap, tp.G, tp.N, tp.H, (int)tp.c_max, f32(p), nullptr, f32(p), s));

@@ -457,6 +457,13 @@ def test_bias_from_table_matches_the_gather():
                                              C.c_void_p(torch.cuda.current_stream().cuda_stream)))
         ref = table[index.reshape(-1)].reshape(n, n, H).permute(2, 0, 1)
         assert torch.equal(out, ref)
+        for dtype, code in ((torch.float16, 1), (torch.bfloat16, 2)):
+            out.fill_(float("nan"))
+            typed = table.to(dtype)
+            _lib.check(lib.sswin_bias_from_typed_table(code, C.c_void_p(typed.data_ptr()), rows, H, C.c_void_p(ti.code.data_ptr()),
+                                                       ti.offset0, n, C.c_void_p(out.data_ptr()),
+                                                       C.c_void_p(torch.cuda.current_stream().cuda_stream)))
+            assert torch.equal(out, typed.float()[index.reshape(-1)].reshape(n, n, H).permute(2, 0, 1))
 
 
 def test_sums_over_nothing_are_zero():
