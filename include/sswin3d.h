@@ -469,6 +469,11 @@ size_t sswin_dense_forward_workspace_bytes(int dtype, int64_t N, int K, int P);
 size_t sswin_dense_weight_grad_workspace_bytes(int dtype, int64_t N, int P, int K);
 int sswin_dense_weight_grad(int dtype, int out_dtype, const void* dy, const void* x, int64_t N, int P, int K, void* dw, void* db,
                             void* ws, size_t ws_bytes, void* stream);
+/* Input gradient (epilogue: plain, or the factor `extra`) and weight gradient of a layer on few rows in one launch;
+ * sswin_dense_backward_small_supported: the shapes it takes.  db may be null. */
+int sswin_dense_backward_small_supported(int dtype, int64_t N, int P, int K);
+int sswin_dense_backward_small(int dtype, int out_dtype, int epilogue, const void* dy, const void* x, const void* w, int64_t N, int P, int K,
+                               const void* extra, void* dx, void* dw, void* db, void* stream);
 
 /* Window attention for heads of 16 or 32 channels and windows of any size, the attention matrix kept in registers
  * (swin3d_base.py:654-675 from the projected qkv [N, 3 H hd] to the output [N, H hd] in voxel order, and its backward).  The bias

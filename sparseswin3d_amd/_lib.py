@@ -87,6 +87,8 @@ SIGNATURES = {
     "sswin_cast_parts": (_i32, [_i32, _vp, _vp, _i32, _vp, _vp]),
     "sswin_dense_forward": (_i32, [_i32, _i32, _i32, _i32, _vp, _i64, _i32, _vp, _vp, _i32, _vp, _vp, _vp, _vp, _sz, _vp]),
     "sswin_dense_forward_workspace_bytes": (_sz, [_i32, _i64, _i32, _i32]),
+    "sswin_dense_backward_small_supported": (_i32, [_i32, _i64, _i32, _i32]),
+    "sswin_dense_backward_small": (_i32, [_i32, _i32, _i32, _vp, _vp, _vp, _i64, _i32, _i32, _vp, _vp, _vp, _vp, _vp]),
     "sswin_dense_weight_grad_workspace_bytes": (_sz, [_i32, _i64, _i32, _i32]),
     "sswin_dense_weight_grad": (_i32, [_i32, _i32, _vp, _vp, _i64, _i32, _i32, _vp, _vp, _vp, _sz, _vp]),
     "sswin_flash_supported": (_i32, [_i32, _i64, _i32, _i32, _i32]),

@@ -655,15 +655,17 @@ __global__ __launch_bounds__(WM * WN * 64) __attribute__((amdgpu_waves_per_eu(OC
 // and add their tiles through LDS in a fixed order.
 // ------------------------------------------------------------------------------------------
 constexpr int SMALL_WAVES = 8;
+struct SmallLds {
+    __attribute__((aligned(16))) float sums[SMALL_WAVES][32 * 36];
+    float colsum[SMALL_WAVES][64];
+};
 template <typename T, typename TO, int EPI, bool DOWN>
-__global__ __launch_bounds__(SMALL_WAVES * 64) void dense_small_kernel(const T* __restrict__ x, int64_t N, int K, const T* __restrict__ w, int P,
-                                                                    int groups, Epilogue ep) {
+__device__ __forceinline__ void small_tile(int block, const T* __restrict__ x, int64_t N, int K, const T* __restrict__ w, int P, int groups,
+                                           const Epilogue& ep, float (&sums)[SMALL_WAVES][32 * 36]) {
     constexpr int PL = Op<T>::PL;
-    __shared__ __attribute__((aligned(16))) float sums[SMALL_WAVES][32 * 36];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, half = lane >> 5, l32 = lane & 31;
-    const int cg = blockIdx.x % groups;
-    const int64_t row0 = (int64_t)(blockIdx.x / groups) * 32;
-    const int col0 = cg * 32, steps = K / 16;
+    const int64_t row0 = (int64_t)(block / groups) * 32;
+    const int col0 = block % groups * 32, steps = K / 16;
     const int64_t row = row0 + l32 < N ? row0 + l32 : N - 1;
     const int col = min(col0 + l32, P - 1);
     const T* xp = x + row * K + half * 8;
@@ -712,6 +714,12 @@ __global__ __launch_bounds__(SMALL_WAVES * 64) void dense_small_kernel(const T* 
         for (int q = 1; q < SMALL_WAVES; ++q) v += *reinterpret_cast<const f32x4*>(&sums[q][rr * 36 + cc]);
         if (in) finish4<T, TO, EPI>(ep, row0 + rr, col0 + cc, P, v, second);
     }
+}
+template <typename T, typename TO, int EPI, bool DOWN>
+__global__ __launch_bounds__(SMALL_WAVES * 64) void dense_small_kernel(const T* __restrict__ x, int64_t N, int K, const T* __restrict__ w, int P,
+                                                                    int groups, Epilogue ep) {
+    __shared__ SmallLds lds;
+    small_tile<T, TO, EPI, DOWN>((int)blockIdx.x, x, N, K, w, P, groups, ep, lds.sums);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -901,13 +909,13 @@ __global__ __launch_bounds__(WM * WN * 64) __attribute__((amdgpu_waves_per_eu(OC
 // The same for few rows: a workgroup owns a 32 x 32 tile of dW, its 8 wavefronts take every 8th step of 16 rows and add
 // their tiles through LDS in a fixed order, so that the result leaves in one launch.
 template <typename T, typename TO>
-__global__ __launch_bounds__(SMALL_WAVES * 64) void dense_wgrad_small_kernel(const T* __restrict__ dy, const T* __restrict__ x, int64_t N, int P, int K,
-                                                                             int tiles_k, TO* __restrict__ dw, TO* __restrict__ db) {
+__device__ __forceinline__ void wgrad_small_tile(int block, const T* __restrict__ dy, const T* __restrict__ x, int64_t N, int P, int K, int tiles_k,
+                                                 TO* __restrict__ dw, TO* __restrict__ db, SmallLds& lds) {
     constexpr int PL = Op<T>::PL, AHEAD = 2;
-    __shared__ __attribute__((aligned(16))) float sums[SMALL_WAVES][32 * 36];
-    __shared__ float colsum[SMALL_WAVES][64];
+    auto& sums = lds.sums;
+    auto& colsum = lds.colsum;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, half = lane >> 5, l32 = lane & 31;
-    const int p0 = (int)(blockIdx.x / tiles_k) * 32, k0 = (int)(blockIdx.x % tiles_k) * 32;
+    const int p0 = block / tiles_k * 32, k0 = block % tiles_k * 32;
     const int pc = min(p0 + l32, P - 1), kc = min(k0 + l32, K - 1), steps = (int)((N + 15) / 16);
     float va[AHEAD][8], vb[AHEAD][8], bsum = 0.f;
     auto request = [&](int slot, int s) {
@@ -961,6 +969,24 @@ __global__ __launch_bounds__(SMALL_WAVES * 64) void dense_wgrad_small_kernel(con
         for (int q = 0; q < SMALL_WAVES; ++q) v += colsum[q][c] + colsum[q][c + 32];
         db[p0 + c] = from_acc<TO>(v);
     }
+}
+template <typename T, typename TO>
+__global__ __launch_bounds__(SMALL_WAVES * 64) void dense_wgrad_small_kernel(const T* __restrict__ dy, const T* __restrict__ x, int64_t N, int P, int K,
+                                                                             int tiles_k, TO* __restrict__ dw, TO* __restrict__ db) {
+    __shared__ SmallLds lds;
+    wgrad_small_tile<T, TO>((int)blockIdx.x, dy, x, N, P, K, tiles_k, dw, db, lds);
+}
+
+// The whole backward of a layer on few rows: the input gradient's tiles, then the weight gradient's, which read the same dY and
+// do not depend on them.  Latency bounds both; as two launches they run one after the other (500 rows fp32, 384 -> 1152 and
+// 384 -> 384 on average: 18 us in two launches, 13 in one; 1536 -> 384 19 to 21 either way, bound by what passes from L2).
+template <typename T, typename TO, int EPI>
+__global__ __launch_bounds__(SMALL_WAVES * 64) void dense_backward_small_kernel(const T* __restrict__ dy, const T* __restrict__ x, const T* __restrict__ w,
+                                                                                int64_t N, int P, int K, int dx_tiles, int tiles_k, Epilogue ep,
+                                                                                TO* __restrict__ dw, TO* __restrict__ db) {
+    __shared__ SmallLds lds;
+    if ((int)blockIdx.x < dx_tiles) small_tile<T, T, EPI, true>((int)blockIdx.x, dy, N, P, w, K, tiles_k, ep, lds.sums);
+    else wgrad_small_tile<T, TO>((int)blockIdx.x - dx_tiles, dy, x, N, P, K, tiles_k, dw, db, lds);
 }
 
 // out[e] = sum over chunks of part[chunk][e] for the weights and the bias behind each other; a block takes 4 EL outputs,
@@ -1206,6 +1232,20 @@ static int launch_wgrad(const void* dy, const void* x, int64_t N, int P, int K, 
     }
 }
 
+template <typename T, typename TO>
+static int launch_backward_small(int epi, const void* dy, const void* x, const void* w, int64_t N, int P, int K, const Epilogue& ep, void* dw, void* db,
+                                 hipStream_t s) {
+    const int tiles_k = (K + 31) / 32, dx_tiles = (int)((N + 31) / 32) * tiles_k, dw_tiles = (P + 31) / 32 * tiles_k;
+    const dim3 grid((unsigned)(dx_tiles + dw_tiles)), block(SMALL_WAVES * 64);
+    if (epi == EPI_SCALE)
+        hipLaunchKernelGGL((dense_backward_small_kernel<T, TO, EPI_SCALE>), grid, block, 0, s, static_cast<const T*>(dy), static_cast<const T*>(x),
+                           static_cast<const T*>(w), N, P, K, dx_tiles, tiles_k, ep, static_cast<TO*>(dw), static_cast<TO*>(db));
+    else
+        hipLaunchKernelGGL((dense_backward_small_kernel<T, TO, EPI_NONE>), grid, block, 0, s, static_cast<const T*>(dy), static_cast<const T*>(x),
+                           static_cast<const T*>(w), N, P, K, dx_tiles, tiles_k, ep, static_cast<TO*>(dw), static_cast<TO*>(db));
+    return launch_ok("dense backward, few rows");
+}
+
 }  // namespace dense
 }  // namespace sswin
 
@@ -1272,6 +1312,30 @@ int sswin_cast_parts(int dtype, const void* const* src, const int64_t* sizes, in
     if (dtype == SSWIN_F16) hipLaunchKernelGGL((cast_parts_kernel<__half>), dim3((unsigned)blocks), dim3(256), 0, s, p, count, static_cast<__half*>(dst));
     else hipLaunchKernelGGL((cast_parts_kernel<__hip_bfloat16>), dim3((unsigned)blocks), dim3(256), 0, s, p, count, static_cast<__hip_bfloat16*>(dst));
     return launch_ok("cast_parts");
+}
+
+int sswin_dense_backward_small_supported(int dtype, int64_t N, int P, int K) {
+    // where both gradients would take their few-rows kernels
+    return N > 0 && N <= WGRAD_SMALL_ROWS && sswin_dense_supported(dtype, P, K) && cut_of(dtype, N, P, K).few;
+}
+
+int sswin_dense_backward_small(int dtype, int out_dtype, int epilogue, const void* dy, const void* x, const void* w, int64_t N, int P, int K,
+                               const void* extra, void* dx, void* dw, void* db, void* stream) {
+    SSWIN_CHECK(sswin_dense_backward_small_supported(dtype, N, P, K), "dense_backward_small: %lld rows, %d -> %d channels of type %d are not supported",
+                (long long)N, K, P, dtype);
+    SSWIN_CHECK(epilogue == EPI_NONE || (epilogue == EPI_SCALE && extra), "dense_backward_small: epilogue %d", epilogue);
+    SSWIN_CHECK(dy && x && w && dx && dw, "dense_backward_small: null pointer");
+    SSWIN_CHECK(((uintptr_t)dy | (uintptr_t)x | (uintptr_t)w | (uintptr_t)extra | (uintptr_t)dx | (uintptr_t)dw | (uintptr_t)db) % 16 == 0,
+                "dense_backward_small: pointers must be 16-byte aligned");
+    const Epilogue ep = {nullptr, extra, dx, nullptr};
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    if (dtype == SSWIN_F32 && out_dtype == SSWIN_F32) return launch_backward_small<float, float>(epilogue, dy, x, w, N, P, K, ep, dw, db, s);
+    if (dtype == SSWIN_F16 && out_dtype == SSWIN_F16) return launch_backward_small<__half, __half>(epilogue, dy, x, w, N, P, K, ep, dw, db, s);
+    if (dtype == SSWIN_F16 && out_dtype == SSWIN_F32) return launch_backward_small<__half, float>(epilogue, dy, x, w, N, P, K, ep, dw, db, s);
+    if (dtype == SSWIN_BF16 && out_dtype == SSWIN_BF16)
+        return launch_backward_small<__hip_bfloat16, __hip_bfloat16>(epilogue, dy, x, w, N, P, K, ep, dw, db, s);
+    if (dtype == SSWIN_BF16 && out_dtype == SSWIN_F32) return launch_backward_small<__hip_bfloat16, float>(epilogue, dy, x, w, N, P, K, ep, dw, db, s);
+    return fail("dense_backward_small: operands of type %d with gradients of type %d are not supported", dtype, out_dtype);
 }
 
 size_t sswin_dense_weight_grad_workspace_bytes(int dtype, int64_t N, int P, int K) {

@@ -320,6 +320,31 @@ std::pair<Tensor, Tensor> dense_dw(const Tensor& dy, const Tensor& x, bool want_
     return {at::mm(dy.t(), x).to(out), want_bias ? dy.sum(0).to(out) : Tensor()};
 }
 
+struct DenseGrads {
+    Tensor dx, dw, db;
+};
+// all gradients of a layer: dy [N, P], x [N, K], w [P, K]; which of them are asked for
+DenseGrads dense_backward(const Tensor& dy, const Tensor& x, const Tensor& w_in, bool want_dx, bool want_weight, bool want_bias, ScalarType out,
+                          int epilogue = SSWIN_DENSE_PLAIN, const Tensor& extra = Tensor()) {
+    DenseGrads g;
+    const int64_t N = x.size(0), P = dy.size(1), K = x.size(1);
+    const int dt = code_of(x.scalar_type());
+    if (want_dx && (want_weight || want_bias) && dy.scalar_type() == x.scalar_type() && w_in.scalar_type() == x.scalar_type() &&
+        sswin_dense_backward_small_supported(dt, N, (int)P, (int)K) && !(epilogue == SSWIN_DENSE_PLAIN && library_ahead(dy, K, P))) {
+        const Tensor w = ready(w_in);
+        const auto opt = x.options().dtype(out);
+        g.dx = at::empty({N, K}, dy.options());
+        g.dw = at::empty({P, K}, opt);
+        if (want_bias) g.db = at::empty({P}, opt);
+        RUN(sswin_dense_backward_small(dt, code_of(out), epilogue, ptr(dy), ptr(x), ptr(w), N, (int)P, (int)K, ptr(extra), ptr(g.dx), ptr(g.dw), ptr(g.db),
+                                       current_stream(x)));
+        return g;
+    }
+    if (want_weight || want_bias) std::tie(g.dw, g.db) = dense_dw(dy, x, want_bias, out);
+    if (want_dx) g.dx = dense_dx(dy, w_in, epilogue, extra);
+    return g;
+}
+
 // ------------------------------------------------------------------------------------------
 // row normalisation
 // ------------------------------------------------------------------------------------------
@@ -574,14 +599,12 @@ struct ModuleNode : torch::autograd::Function<ModuleNode> {
         const Tensor &x = v[0], &qkv_w = v[1], &bias = v[2], &proj_w = v[3], &qkv = v[4], &o = v[7];
         c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
         const Tensor dy = ready(grads[0].to(x.scalar_type()));
-        std::pair<Tensor, Tensor> d_proj, d_qkvw;
-        if (how[5] || how[6]) d_proj = dense_dw(dy, o, how[6], (ScalarType)how[8]);
-        Tensor d_bias, dx;
-        const Tensor d_o = dense_dx(dy, proj_w);
-        const Tensor d_qkv = attention_backward(*a, qkv, bias, AttentionSaved{v[5], v[6], v[8]}, o, d_o, how[4], d_bias);
-        if (how[2] || how[3]) d_qkvw = dense_dw(d_qkv, x, how[3], (ScalarType)how[7]);
-        if (how[1]) dx = dense_dx(d_qkv, qkv_w).to((ScalarType)how[0]);
-        return once({dx, d_qkvw.first, d_qkvw.second, d_bias, d_proj.first, d_proj.second, Tensor(), Tensor()});
+        Tensor d_bias;
+        const DenseGrads d_proj = dense_backward(dy, o, proj_w, true, how[5], how[6], (ScalarType)how[8]);
+        const Tensor d_qkv = attention_backward(*a, qkv, bias, AttentionSaved{v[5], v[6], v[8]}, o, d_proj.dx, how[4], d_bias);
+        const DenseGrads d_in = dense_backward(d_qkv, x, qkv_w, how[1], how[2], how[3], (ScalarType)how[7]);
+        const Tensor dx = how[1] ? d_in.dx.to((ScalarType)how[0]) : Tensor();
+        return once({dx, d_in.dw, d_in.db, d_bias, d_proj.dw, d_proj.db, Tensor(), Tensor()});
     }
 };
 
@@ -631,20 +654,17 @@ struct BlockNode : torch::autograd::Function<BlockNode> {
         const Tensor dy = ready(grads[0]);
         const Tensor dyt = dy.to(type);
         Tensor out[PARAMS];
-        auto keep = [&](int w, const Tensor& d, const Tensor& in) {
-            if (!ask[w] && !ask[w + 1]) return;
-            std::tie(out[w], out[w + 1]) = dense_dw(d, in, ask[w + 1], wt);
+        auto through = [&](int w, const Tensor& d, const Tensor& in, const Tensor& weight, int epilogue = SSWIN_DENSE_PLAIN, const Tensor& extra = Tensor()) {
+            DenseGrads r = dense_backward(d, in, weight, true, ask[w], ask[w + 1], wt, epilogue, extra);
+            out[w] = r.dw, out[w + 1] = r.db;
+            return r.dx;
         };
-        keep(W2, dyt, g);
-        const Tensor du = dense_dx(dyt, w2, SSWIN_DENSE_SCALE, slope);
-        keep(W1, du, x2);
-        const Tensor dh = norm_backward(dense_dx(du, w1), h, stats2, g2, dy, out[G2], out[B2]);
+        const Tensor du = through(W2, dyt, g, w2, SSWIN_DENSE_SCALE, slope);
+        const Tensor dh = norm_backward(through(W1, du, x2, w1), h, stats2, g2, dy, out[G2], out[B2]);
         const Tensor dht = dh.to(type);
-        keep(PROJW, dht, o);
-        const Tensor d_o = dense_dx(dht, projw);
+        const Tensor d_o = through(PROJW, dht, o, projw);
         const Tensor d_qkv = attention_backward(*a, qkv, table, AttentionSaved{v[11], v[12], v[19]}, o, d_o, ask[TABLE], out[TABLE]);
-        keep(QKVW, d_qkv, x1);
-        out[X] = norm_backward(dense_dx(d_qkv, qkvw), x, stats1, g1, dh, out[G1], out[B1]);
+        out[X] = norm_backward(through(QKVW, d_qkv, x1, qkvw), x, stats1, g1, dh, out[G1], out[B1]);
         variable_list result;
         for (int64_t w : which) result.push_back(ask[w] ? out[w] : Tensor());
         result.resize(which.size() + 5);                                 // the arguments that are no tensors
@@ -680,13 +700,14 @@ struct MergeNode : torch::autograd::Function<MergeNode> {
         const Tensor &gamma = v[0], &w = v[1], &pooled = v[2], &stats = v[3], &x1 = v[4];
         c10::hip::HIPGuardMasqueradingAsCUDA guard(pooled.device());
         const Tensor dy = ready(grads[0].to(x1.scalar_type()));
-        Tensor dg, db, dw = dense_dw(dy, x1, false, (ScalarType)ctx->saved_data["params"].toInt()).first;
-        const Tensor d_pool = norm_backward(dense_dx(dy, w), pooled, stats, gamma, Tensor(), dg, db);
+        Tensor dg, db;
+        const DenseGrads d = dense_backward(dy, x1, w, true, true, false, (ScalarType)ctx->saved_data["params"].toInt());
+        const Tensor d_pool = norm_backward(d.dx, pooled, stats, gamma, Tensor(), dg, db);
         const int64_t D = pooled.size(1);
         Tensor dx = at::empty({plan->N, D}, pooled.options());
         RUN(sswin_pool_windows(code_of(dx.scalar_type()), 1, 1, i32(plan->plan), plan->g_cap, plan->windows, i32(plan->tokens), plan->N, ptr(d_pool), D, (int)D,
                                ptr(dx), D, current_stream(dx)));
-        return once({dx, dg, db, dw, Tensor(), Tensor(), Tensor()});
+        return once({dx, dg, db, d.dw, Tensor(), Tensor(), Tensor()});
     }
 };
 

@@ -279,3 +279,30 @@ def test_projections_that_are_no_plain_linears_run_under_autocast():
         assert calls == [1] and torch.allclose(plain, hooked, rtol=2e-2, atol=2e-2)
         attn.proj = Scaled(96, 96).cuda()
         assert not attn(SparseVoxelTensor(x, ind, (125,), 40), None).features.any()
+
+
+@pytest.mark.parametrize("N,P,K", [(1, 16, 16), (33, 96, 384), (284, 208, 80), (500, 1536, 384), (1024, 48, 144)])
+@pytest.mark.parametrize("dtype,out", [(torch.float32, torch.float32), (torch.bfloat16, torch.bfloat16), (torch.float16, torch.float32)],
+                         ids=["fp32", "bf16", "fp16-out32"])
+@pytest.mark.parametrize("factor", [False, True], ids=["plain", "factor"])
+def test_dense_backward_of_few_rows_in_one_launch(N, P, K, dtype, out, factor):
+    """Both gradients from one launch against the two launches: the same tiles, so the same bits."""
+    from sparseswin3d_amd import _lib
+    lib = _lib.load()
+    assert lib.sswin_dense_backward_small_supported(CODE[dtype], N, P, K) and not lib.sswin_dense_backward_small_supported(CODE[dtype], 1025, P, K)
+    gen = torch.Generator().manual_seed(N + P + K)
+    dy, x, w = _rand(gen, N, P, dtype=dtype), _rand(gen, N, K, dtype=dtype), _rand(gen, P, K, dtype=dtype)
+    f = _rand(gen, N, K, dtype=dtype) if factor else None
+    epi = SCALE if factor else PLAIN
+    dx, dw, db = (torch.full(s, float("nan"), dtype=t, device="cuda") for s, t in (((N, K), dtype), ((P, K), out), ((P,), out)))
+    _lib.check(lib.sswin_dense_backward_small(CODE[dtype], CODE[out], epi, _ptr(dy), _ptr(x), _ptr(w), N, P, K, _ptr(f), _ptr(dx), _ptr(dw), _ptr(db),
+                                              _stream()))
+    assert torch.equal(dx, _forward(lib, _lib, dy, w, None, 1, epi, f, dtype)[0])
+    dw2, db2 = torch.empty_like(dw), torch.empty_like(db)
+    nb = lib.sswin_dense_weight_grad_workspace_bytes(CODE[dtype], N, P, K)
+    ws = torch.empty(max(nb, 1), dtype=torch.uint8, device="cuda")
+    _lib.check(lib.sswin_dense_weight_grad(CODE[dtype], CODE[out], _ptr(dy), _ptr(x), N, P, K, _ptr(dw2), _ptr(db2), _ptr(ws), nb, _stream()))
+    assert torch.equal(dw, dw2) and torch.equal(db, db2)
+    dw.fill_(float("nan"))
+    _lib.check(lib.sswin_dense_backward_small(CODE[dtype], CODE[out], epi, _ptr(dy), _ptr(x), _ptr(w), N, P, K, _ptr(f), _ptr(dx), _ptr(dw), None, _stream()))
+    assert torch.equal(dw, dw2)
