@@ -992,7 +992,8 @@ __global__ __launch_bounds__(SMALL_WAVES * 64) void dense_backward_small_kernel(
 // out[e] = sum over chunks of part[chunk][e] for the weights and the bias behind each other; a block takes 4 EL outputs,
 // CL = 256 / EL threads share four of them, each adds every CL-th chunk in order, the CL sums in a fixed tree.
 // EL = 16; 4 from 256 chunks on, where small layers leave the chip idle and the sums one after the other take the time
-// (1024 chunks of 144 x 48 and 48 x 48: 16.8 us on average, with 4 6.8)
+// (1024 chunks of 144 x 48 and 48 x 48: 16.8 us on average, with 4 6.8); 64 up to 16 chunks, where most of 16 threads have none
+// (weight gradients of 2000 and 8119 rows 768 -> 2304: 35.5 -> 24.7 us and 73.0 -> 68.6)
 template <typename TO, int EL>
 __global__ __launch_bounds__(256) void dense_wgrad_sum_kernel(const float* __restrict__ part_w, const float* __restrict__ part_b, int chunks,
                                                               int64_t PK, int P, TO* __restrict__ dw, TO* __restrict__ db) {
@@ -1177,19 +1178,24 @@ constexpr int64_t WGRAD_SMALL_ROWS = 1024;
 //   128 x 192 from 192 columns of X on (35 569 rows 192 -> 576: 91 and 78 us with 96 x 96), 64 x 192 where dY has at most 64;
 //   192 x 64 and 64 x 64 up to 64 columns of X (112 700 rows 48 -> 144 and 48 -> 48: 32 and 20 us, 39 on average with 96 x 96);
 //   96 x 96 between, with more workgroups per compute unit.
-// 16 bit: 96 x 96 (219 000 rows 96 -> 288: 39 us; 192 x 192 tiles 58, 192 x 96 44).
+// 16 bit: 96 x 96 (219 000 rows 96 -> 288: 39 us; 192 x 192 tiles 58, 192 x 96 44); 192 x 192 where dW has at least 48 such tiles
+//   and the rows are many, so that half the bytes pass from L2 (8119 rows 768 -> 2304: 69 us and 57, 768 -> 3072 80 and 61;
+//   2000 rows 768 -> 2304 25 and 26; 9000 rows 384 -> 1536 30 either way).
 struct WgradTile {
     int bm, bn, per_cu;
 };
-static WgradTile wgrad_tile(int P, int K) {
+static WgradTile wgrad_tile(int dtype, int64_t N, int P, int K) {
+    if (dtype != SSWIN_F32) {
+        if (N >= 4096 && P % 192 == 0 && K % 192 == 0 && (int64_t)P * K >= 48 * 192 * 192) return {192, 192, 1};
+        return {96, 96, 3};
+    }
     if (K >= 192) return P <= 64 ? WgradTile{64, 192, 2} : WgradTile{128, 192, 2};
     if (K <= 64) return P <= 64 ? WgradTile{64, 64, 4} : WgradTile{192, 64, 2};
     return {96, 96, 4};
 }
 static WgradPlan wgrad_plan(int dtype, int64_t N, int P, int K) {
-    if (dtype != SSWIN_F32) return wgrad_plan(N, P, K, 32, 96, 96, 3);
-    const WgradTile t = wgrad_tile(P, K);
-    return wgrad_plan(N, P, K, 16, t.bm, t.bn, t.per_cu);
+    const WgradTile t = wgrad_tile(dtype, N, P, K);
+    return wgrad_plan(N, P, K, dtype == SSWIN_F32 ? 16 : 32, t.bm, t.bn, t.per_cu);
 }
 
 template <typename T, typename TO, typename F>
@@ -1200,7 +1206,10 @@ static int launch_wgrad_as(F* k, int threads, size_t lds, const WgradPlan& pl, c
                        P, K, pl.tiles_p, pl.tiles_k, pl.rows, ws, db ? part_b : nullptr);
     if (int rc = launch_ok("dense weight gradient")) return rc;
     const int64_t PK = (int64_t)P * K;
-    if (pl.chunks >= 256)
+    if (pl.chunks <= 16)
+        hipLaunchKernelGGL((dense_wgrad_sum_kernel<TO, 64>), dim3((unsigned)((PK + P + 255) / 256)), dim3(256), 0, s, ws, part_b, pl.chunks, PK, P,
+                           static_cast<TO*>(dw), static_cast<TO*>(db));
+    else if (pl.chunks >= 256)
         hipLaunchKernelGGL((dense_wgrad_sum_kernel<TO, 4>), dim3((unsigned)((PK + P + 15) / 16)), dim3(256), 0, s, ws, part_b, pl.chunks, PK, P,
                            static_cast<TO*>(dw), static_cast<TO*>(db));
     else
@@ -1219,7 +1228,7 @@ static int launch_wgrad(const void* dy, const void* x, int64_t N, int P, int K, 
     }
     if constexpr (Op<T>::PL == 3) {
         const WgradPlan pl = wgrad_plan(SSWIN_F32, N, P, K);
-        const WgradTile t = wgrad_tile(P, K);
+        const WgradTile t = wgrad_tile(SSWIN_F32, N, P, K);
         const size_t lds = 2 * (size_t)((t.bm + t.bn) / 32) * 3 * 1024;                                  // two buffers of (row tiles) x 3 planes
         if (t.bm == 128) return launch_wgrad_as<T, TO>(dense_wgrad_kernel<2, 2, 2, 3, 2>, 256, lds, pl, dy, x, N, P, K, dw, db, ws, s);
         if (t.bn == 192) return launch_wgrad_as<T, TO>(dense_wgrad_kernel<2, 2, 1, 3, 2>, 256, lds, pl, dy, x, N, P, K, dw, db, ws, s);
@@ -1228,7 +1237,14 @@ static int launch_wgrad(const void* dy, const void* x, int64_t N, int P, int K, 
         return launch_wgrad_as<T, TO>(dense_wgrad_kernel<3, 1, 1, 3, 3>, 192, lds, pl, dy, x, N, P, K, dw, db, ws, s);
     } else {
         constexpr size_t lds = 3 * 2 * 32 * 192;                         // three stages of two tiles of 32 x 96
-        return launch_wgrad_as<T, TO>(dense16_wgrad_kernel<T, 3, 1, 1, 3, 3>, 192, lds, wgrad_plan(SSWIN_F16, N, P, K), dy, x, N, P, K, dw, db, ws, s);
+        const WgradPlan pl = wgrad_plan(SSWIN_F16, N, P, K);
+        if (wgrad_tile(SSWIN_F16, N, P, K).bm == 192) {
+            auto* k = dense16_wgrad_kernel<T, 3, 2, 2, 3, 2>;
+            static const int configured = allow_lds(k, 2 * lds);
+            if (configured) return configured;
+            return launch_wgrad_as<T, TO>(k, 384, 2 * lds, pl, dy, x, N, P, K, dw, db, ws, s);
+        }
+        return launch_wgrad_as<T, TO>(dense16_wgrad_kernel<T, 3, 1, 1, 3, 3>, 192, lds, pl, dy, x, N, P, K, dw, db, ws, s);
     }
 }
 

@@ -85,7 +85,7 @@ def test_dense_forward_and_input_gradient(N, K, P, dtype, out):
 
 
 @pytest.mark.parametrize("N,P,K", [(1, 16, 16), (17, 144, 48), (1024, 96, 96), (1025, 48, 208), (1100, 288, 96), (9001, 208, 192), (70001, 48, 144),
-                                   (2000, 16, 16), (30001, 64, 48), (40001, 144, 48), (1100, 400, 64), (3003, 64, 400)])
+                                   (2000, 16, 16), (30001, 64, 48), (40001, 144, 48), (1100, 400, 64), (3003, 64, 400), (4501, 2304, 768)])
 @pytest.mark.parametrize("dtype,out", [(torch.float32, torch.float32), (torch.bfloat16, torch.bfloat16), (torch.float16, torch.float32)],
                          ids=["fp32", "bf16", "fp16-out32"])
 def test_dense_weight_gradient(N, P, K, dtype, out):
