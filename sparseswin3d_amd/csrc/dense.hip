@@ -489,37 +489,47 @@ __global__ __launch_bounds__(WM * WN * KG * 64) __attribute__((amdgpu_waves_per_
         block_barrier();
         if (wk == 1) return;
     }
-    // through LDS, 32 columns at a time, so that every lane holds four neighbouring columns
-    constexpr int PITCH = 36;
-    float* mine = reinterpret_cast<float*>(lds) + wave * 32 * PITCH;
-    const int rr = lane >> 3, cc = (lane & 7) * 4;
+    // Through LDS, 16 rows x 96 columns of a wavefront at a time, so that every lane holds eight neighbouring columns and a row
+    // leaves in one run of 192 bytes (32 columns at a time, runs of 64 bytes: 450 000 rows 96 -> 288 bf16 138 us, now 115;
+    // 219 000 rows 96 -> 96 with a residual 31 and 25; 192 -> 48 times a factor, fp16, 59 and 41)
+    constexpr int PITCH = 100, PIECES = 16 * 12 / 64;
+    float* mine = reinterpret_cast<float*>(lds) + wave * 16 * PITCH;
 #pragma unroll
-    for (int i = 0; i < MT; ++i) {
-        const int64_t r0 = row0 + (wm * MT + i) * 32 + rr;
-        const int c0 = col0 + wn * 96 + cc;
+    for (int i = 0; i < MT; ++i)
 #pragma unroll
-        for (int j = 0; j < NT; ++j) {
-            Second4<T, TO, EPI> second[4];
+        for (int h = 0; h < 2; ++h) {
+            const int64_t r0 = row0 + (wm * MT + i) * 32 + h * 16;
+            const int c0 = col0 + wn * 96;
+            Second8<T, TO, EPI> second[PIECES];
             if (!part)
 #pragma unroll
-                for (int q = 0; q < 4; ++q)
-                    if (r0 + q * 8 < N && c0 + j * 32 < P) second[q].load(ep, r0 + q * 8, c0 + j * 32, P);
+                for (int q = 0; q < PIECES; ++q) {
+                    const int e = q * 64 + lane, rr = e / 12, cc = e % 12 * 8;
+                    if (r0 + rr < N && c0 + cc < P) second[q].load(ep, r0 + rr, c0 + cc, P);
+                }
 #pragma unroll
-            for (int r = 0; r < 16; ++r) mine[acc_row(r, half) * PITCH + l32] = acc[i][j][r];
+            for (int j = 0; j < NT; ++j)
+#pragma unroll
+                for (int r = 0; r < 8; ++r) mine[acc_row(r, half) * PITCH + j * 32 + l32] = acc[i][j][h * 8 + r];
             __builtin_amdgcn_wave_barrier();
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const f32x4 v = *reinterpret_cast<const f32x4*>(mine + (q * 8 + rr) * PITCH + cc);
-                const int64_t row = r0 + q * 8;
-                const int col = c0 + j * 32;
+            for (int q = 0; q < PIECES; ++q) {
+                const int e = q * 64 + lane, rr = e / 12, cc = e % 12 * 8;
+                const f32x4 v[2] = {*reinterpret_cast<const f32x4*>(mine + rr * PITCH + cc), *reinterpret_cast<const f32x4*>(mine + rr * PITCH + cc + 4)};
+                const int64_t row = r0 + rr;
+                const int col = c0 + cc;
                 if (row < N && col < P) {
-                    if (part) *reinterpret_cast<f32x4*>(part + ((int64_t)part_no * N + row) * P + col) = v;
-                    else finish4<T, TO, EPI>(ep, row, col, P, v, second[q]);
+                    if (part) {
+                        f32x4* at = reinterpret_cast<f32x4*>(part + ((int64_t)part_no * N + row) * P + col);
+                        at[0] = v[0];
+                        at[1] = v[1];
+                    } else {
+                        finish8<T, TO, EPI>(ep, row, col, P, v, second[q]);
+                    }
                 }
             }
             __builtin_amdgcn_wave_barrier();
         }
-    }
 }
 
 // the shares of the reduction added in order, then the last step
@@ -1068,7 +1078,7 @@ static int launch_rows(const float* x, int64_t N, int K, const float* w, int P, 
 template <typename T, typename TO, int EPI, bool DOWN, int BK, int WM, int WN, int KG, int MT, int STAGES, int OCC>
 static int launch_rows16(const T* x, int64_t N, int K, const T* w, int P, int ksplit, float* ws, const Epilogue& ep, hipStream_t s) {
     constexpr int BM = WM * MT * 32, BN = WN * 96;
-    constexpr size_t tiles = STAGES * (size_t)(BM + BN) * BK * 2, out = (size_t)WM * WN * (KG == 2 ? MT * 96 : 36) * 32 * 4;
+    constexpr size_t tiles = STAGES * (size_t)(BM + BN) * BK * 2, out = (size_t)WM * WN * (KG == 2 ? MT * 96 : 50) * 32 * 4;
     constexpr size_t bytes = tiles > out ? tiles : out;
     auto* k = dense16_rows_kernel<T, TO, EPI, DOWN, BK, WM, WN, KG, MT, STAGES, OCC>;
     static const int configured = allow_lds(k, bytes);

@@ -109,6 +109,38 @@ __device__ __forceinline__ void finish4(const Epilogue& ep, int64_t row, int col
     *reinterpret_cast<Vec4<TO>*>(static_cast<TO*>(ep.y) + at) = pack4<TO>(v);
 }
 
+// the same for eight consecutive columns: 16-bit rows are touched in 16-byte pieces
+template <typename T> struct alignas(16) Vec8 { Vec4<T> q[2]; };
+template <typename T, typename TO, int EPI> struct Second8 {
+    using TE = typename Second4<T, TO, EPI>::TE;
+    Vec8<TE> r;
+    __device__ __forceinline__ void load(const Epilogue& ep, int64_t row, int col, int P) {
+        if constexpr (Second4<T, TO, EPI>::USED) r = *reinterpret_cast<const Vec8<TE>*>(static_cast<const TE*>(ep.extra) + row * P + col);
+    }
+};
+template <typename T, typename TO, int EPI>
+__device__ __forceinline__ void finish8(const Epilogue& ep, int64_t row, int col, int P, const f32x4 (&acc)[2], const Second8<T, TO, EPI>& second) {
+    Vec8<T> b;
+    if (ep.bias) b = *reinterpret_cast<const Vec8<T>*>(static_cast<const T*>(ep.bias) + col);
+    const int64_t at = row * P + col;
+    Vec8<TO> y, slope;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        float v[4], d[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            float extra = 0.f;
+            if constexpr (Second4<T, TO, EPI>::USED) extra = to_acc(second.r.q[h].v[e]);
+            v[e] = finish1<EPI, sizeof(TO) == 4>(ep.bias ? acc[h][e] + to_acc(b.q[h].v[e]) : acc[h][e], extra, d[e]);
+        }
+        y.q[h] = pack4<TO>(v);
+        if constexpr (EPI == EPI_GELU) slope.q[h] = pack4<TO>(d);
+    }
+    if constexpr (EPI == EPI_GELU)
+        if (ep.slope) *reinterpret_cast<Vec8<TO>*>(static_cast<TO*>(ep.slope) + at) = slope;
+    *reinterpret_cast<Vec8<TO>*>(static_cast<TO*>(ep.y) + at) = y;
+}
+
 // fp32 layers of 96 reduction channels and a multiple of 96 outputs (tall_linear.hip): x [N >= 32, 96], all of Wop in LDS
 int staged_layer_96(const float* x, int64_t N, const float* w, int P, bool transposed, int epilogue, const Epilogue& ep, hipStream_t s);
 
