@@ -506,6 +506,10 @@ size_t sswin_layer_norm_backward_workspace_bytes(int x_dtype, int64_t N, int D);
 int sswin_layer_norm_backward(int x_dtype, int dy_dtype, const void* dy, const void* x, const float* stats, int64_t N, int D,
                               const void* gamma, const void* dres, void* dx, void* dgamma, void* dbeta, void* ws, size_t ws_bytes,
                               void* stream);
+/* The same with dx also in dy's type (dx_copy, or null): what a 16-bit layer in front of the norm takes. */
+int sswin_layer_norm_backward_copy(int x_dtype, int dy_dtype, const void* dy, const void* x, const float* stats, int64_t N, int D,
+                                   const void* gamma, const void* dres, void* dx, void* dx_copy, void* dgamma, void* dbeta, void* ws,
+                                   size_t ws_bytes, void* stream);
 
 /* ---- window-resident attention (whole forward / backward of the attention core) ---------- */
 

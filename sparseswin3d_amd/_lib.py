@@ -100,6 +100,7 @@ SIGNATURES = {
     "sswin_layer_norm_forward": (_i32, [_i32, _i32, _vp, _i64, _i32, _vp, _vp, C.c_float, _vp, _vp, _vp]),
     "sswin_layer_norm_backward_workspace_bytes": (_sz, [_i32, _i64, _i32]),
     "sswin_layer_norm_backward": (_i32, [_i32, _i32, _vp, _vp, _vp, _i64, _i32, _vp, _vp, _vp, _vp, _vp, _vp, _sz, _vp]),
+    "sswin_layer_norm_backward_copy": (_i32, [_i32, _i32, _vp, _vp, _vp, _i64, _i32, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _sz, _vp]),
     "sswin_window_indices": (_i32, [_vp, _i64, _i32, _vp, _vp, _vp, _vp, _vp]),
     "sswin_shift_mask": (_i32, [_vp, _vp, _vp, _vp, _vp]),
     "sswin_window_coords": (_i32, [_vp, _i64, _i64, _vp, _vp, _vp, _vp]),
@@ -113,7 +114,7 @@ SIGNATURES = {
                                                _vp, _i64, _i32, _vp, _i64, _i32, _vp, _i64, _i32, _vp, _i32, _vp]),
 }
 
-ABI_VERSION = 32
+ABI_VERSION = 33
 _lib = None
 
 # A list turns on timing of the library's launches: every call that takes a stream is bracketed by events on that

@@ -357,15 +357,19 @@ Tensor norm_forward(const Tensor& x, const Tensor& gamma_in, const Tensor& beta_
     return y;
 }
 
-Tensor norm_backward(const Tensor& dy, const Tensor& x, const Tensor& stats, const Tensor& gamma_in, const Tensor& dres, Tensor& dgamma, Tensor& dbeta) {
+// copy: dx in dy's type as well
+Tensor norm_backward(const Tensor& dy, const Tensor& x, const Tensor& stats, const Tensor& gamma_in, const Tensor& dres, Tensor& dgamma, Tensor& dbeta,
+                     Tensor* copy = nullptr) {
     const Tensor gamma = ready(gamma_in);
     Tensor dx = at::empty_like(x);
     dgamma = at::empty_like(gamma);
     dbeta = at::empty_like(gamma);
     const size_t nb = sswin_layer_norm_backward_workspace_bytes(code_of(x.scalar_type()), x.size(0), (int)x.size(1));
     Tensor ws = bytes(nb, x);
-    RUN(sswin_layer_norm_backward(code_of(x.scalar_type()), code_of(dy.scalar_type()), ptr(dy), ptr(x), f32(stats), x.size(0), (int)x.size(1), ptr(gamma),
-                                  ptr(dres), ptr(dx), ptr(dgamma), ptr(dbeta), ptr(ws), nb, current_stream(x)));
+    if (copy) *copy = dy.scalar_type() == x.scalar_type() ? dx : at::empty(x.sizes(), dy.options());
+    RUN(sswin_layer_norm_backward_copy(code_of(x.scalar_type()), code_of(dy.scalar_type()), ptr(dy), ptr(x), f32(stats), x.size(0), (int)x.size(1),
+                                       ptr(gamma), ptr(dres), ptr(dx), copy && !copy->is_same(dx) ? ptr(*copy) : nullptr, ptr(dgamma), ptr(dbeta), ptr(ws),
+                                       nb, current_stream(x)));
     return dx;
 }
 
@@ -660,8 +664,8 @@ struct BlockNode : torch::autograd::Function<BlockNode> {
             return r.dx;
         };
         const Tensor du = through(W2, dyt, g, w2, SSWIN_DENSE_SCALE, slope);
-        const Tensor dh = norm_backward(through(W1, du, x2, w1), h, stats2, g2, dy, out[G2], out[B2]);
-        const Tensor dht = dh.to(type);
+        Tensor dht;                                                      // dh in the layers' type
+        const Tensor dh = norm_backward(through(W1, du, x2, w1), h, stats2, g2, dy, out[G2], out[B2], &dht);
         const Tensor d_o = through(PROJW, dht, o, projw);
         const Tensor d_qkv = attention_backward(*a, qkv, table, AttentionSaved{v[11], v[12], v[19]}, o, d_o, ask[TABLE], out[TABLE]);
         out[X] = norm_backward(through(QKVW, d_qkv, x1, qkvw), x, stats1, g1, dh, out[G1], out[B1]);

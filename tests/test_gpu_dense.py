@@ -306,3 +306,26 @@ def test_dense_backward_of_few_rows_in_one_launch(N, P, K, dtype, out, factor):
     dw.fill_(float("nan"))
     _lib.check(lib.sswin_dense_backward_small(CODE[dtype], CODE[out], epi, _ptr(dy), _ptr(x), _ptr(w), N, P, K, _ptr(f), _ptr(dx), _ptr(dw), None, _stream()))
     assert torch.equal(dw, dw2)
+
+
+@pytest.mark.parametrize("N,D", [(1, 16), (33, 192), (5, 80), (5000, 96)])
+@pytest.mark.parametrize("kind", [torch.float16, torch.bfloat16], ids=["fp16", "bf16"])
+def test_layer_norm_backward_with_a_16_bit_copy(N, D, kind):
+    """dx in dy's type beside fp32 dx: the rounding of the same values, and nothing else changes."""
+    from sparseswin3d_amd import _lib
+    lib = _lib.load()
+    gen = torch.Generator().manual_seed(N + D)
+    x, dres, g, dy = _rand(gen, N, D), _rand(gen, N, D), _rand(gen, D, spread=1), _rand(gen, N, D, dtype=kind)
+    stats = torch.stack([x.mean(1), (x.var(1, unbiased=False) + 1e-5).rsqrt()]).contiguous()
+    nb = lib.sswin_layer_norm_backward_workspace_bytes(0, N, D)
+    results = []
+    for with_copy in (True, False):
+        ws = torch.empty(nb, dtype=torch.uint8, device="cuda")
+        dx, dg, db = (torch.full(s, float("nan"), device="cuda") for s in ((N, D), (D,), (D,)))
+        copy = torch.full((N, D), float("nan"), dtype=kind, device="cuda") if with_copy else None
+        _lib.check(lib.sswin_layer_norm_backward_copy(0, CODE[kind], _ptr(dy), _ptr(x), _ptr(stats), N, D, _ptr(g), _ptr(dres), _ptr(dx), _ptr(copy), _ptr(dg),
+                                                      _ptr(db), _ptr(ws), nb, _stream()))
+        results.append((dx, dg, db))
+        if with_copy:
+            assert torch.equal(copy, dx.to(kind))
+    assert all(torch.equal(a, b) for a, b in zip(*results))
