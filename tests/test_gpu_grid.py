@@ -159,3 +159,24 @@ def test_shift_masks_are_kept_per_shape():
     assert len(layers._MASKS) == 8
     again = layers.compute_mask([10, 10, 10], [5, 5, 5], [2, 2, 2], "cuda")        # dropped meanwhile: built anew
     assert again is not a and torch.equal(again, a)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16], ids=["fp32", "fp16", "bf16"])
+def test_pooling_in_pieces_of_four_channels_equals_the_wide_one(dtype):
+    """Rows of 24 channels take 16-byte pieces in every type, rows of 12 pieces of four channels in the 16-bit ones: the same sums
+    per channel, in windows of up to 27 voxels (counts that are no multiple of the rows in flight)."""
+    from sparseswin3d_amd.layers import _PoolWindows, downsample_plan
+    from sparseswin3d_amd.window_attention import SparseVoxelTensor
+    rng = np.random.default_rng(11)
+    grid = (19, 14, 9)
+    c4 = _coords(rng, 2, grid, 3000)
+    feats = torch.from_numpy(rng.standard_normal((len(c4), 24)).astype(np.float32)).to(dtype).cuda()
+    plan = downsample_plan(SparseVoxelTensor(feats, torch.from_numpy(c4).cuda(), grid, 2), 3)[0]
+    for mean in (True, False):
+        rows, grads = [], []
+        for x in (feats.clone().requires_grad_(True), feats[:, :12].contiguous().requires_grad_(True)):
+            out = _PoolWindows.apply(x, plan, mean)
+            out.backward(torch.linspace(-2, 2, 24, device="cuda")[:x.shape[1]].to(dtype).expand(out.shape).contiguous())
+            rows.append(out.detach()[:, :12])
+            grads.append(x.grad[:, :12])
+        assert torch.equal(*rows) and torch.equal(*grads)
