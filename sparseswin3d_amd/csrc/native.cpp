@@ -105,6 +105,10 @@ struct Plan : torch::CustomClassHolder {
     int H = 0;
     bool order_only = false;
     std::shared_ptr<SharedEvent> event;
+    // allocated; its kernels are in the stream; its totals are decoded; its totals failed their check, which every later use
+    // reports again (a plan stays in its view's cache, and the tables of a failed one are not filled)
+    enum State { FRESH, QUEUED, DONE, FAILED } state = FRESH;
+    std::string failure;
     int64_t G = 0, windows = 0, A = 0, c_max = 0, buckets[4] = {0, 0, 0, 0}, oversize = 0;
 
     Plan(const Tensor& ind, int64_t batch, int64_t positions, int64_t heads, bool with_tasks, bool order) {
@@ -128,25 +132,37 @@ struct Plan : torch::CustomClassHolder {
     }
 
     void finish() {
-        if (!event) return;
-        if (PyGILState_Check()) {
-            py::gil_scoped_release nogil;
-            wait();
-        } else {
-            wait();
+        if (state == DONE) return;
+        TORCH_CHECK(state != FRESH, "token plan: its kernels were not launched");
+        if (state == QUEUED) {
+            if (PyGILState_Check()) {
+                py::gil_scoped_release nogil;
+                wait();
+            } else {
+                wait();
+            }
+            decode();
         }
-        event.reset();
-        Tensor t = std::move(totals);
-        int64_t* v = t.data_ptr<int64_t>();
+        TORCH_CHECK(state == DONE, failure);
+    }
+    void decode() {
+        int64_t* v = totals.data_ptr<int64_t>();
         const int rc = N > 0 ? sswin_token_plan_totals(v, H, g_cap) : 0;
         if (rc == 0) {
             G = v[0], windows = v[1], A = v[2], c_max = v[3], oversize = v[8];
             for (int b = 0; b < 4; ++b) buckets[b] = v[4 + b];
+        } else {
+            failure = sswin_last_error();
         }
-        give_pinned(std::move(t));
+        state = rc == 0 ? DONE : FAILED;
+        event.reset();
+        give_pinned(std::move(totals));
         ws = Tensor();
         indices = Tensor();
-        TORCH_CHECK(rc == 0, sswin_last_error());
+    }
+    const Plan& decoded() const {
+        TORCH_CHECK(state == DONE, state == FAILED ? failure : "token plan: the totals are there after finish()");
+        return *this;
     }
     void wait() const { TORCH_CHECK(hipEventSynchronize(event->event) == hipSuccess, "token plan: the stream failed"); }
 };
@@ -174,7 +190,7 @@ void enqueue_plans(const std::vector<PlanPtr>& plans) {
     }
     auto event = std::make_shared<SharedEvent>();
     TORCH_CHECK(hipEventRecord(event->event, static_cast<hipStream_t>(s)) == hipSuccess, "hipEventRecord failed");
-    for (const PlanPtr& p : plans) p->event = event;
+    for (const PlanPtr& p : plans) p->event = event, p->state = Plan::QUEUED;
 }
 
 // (batch, d, h, w) -> (window slot, position) of the padded grid rolled by -shift
@@ -811,12 +827,12 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         .def_readonly("B", &Plan::B)
         .def_readonly("g_cap", &Plan::g_cap)
         .def_readonly("order_only", &Plan::order_only)
-        .def_readonly("G", &Plan::G)
-        .def_readonly("windows", &Plan::windows)
-        .def_readonly("A", &Plan::A)
-        .def_readonly("c_max", &Plan::c_max)
-        .def_readonly("oversize_groups", &Plan::oversize)
-        .def_property_readonly("buckets", [](const Plan& p) { return std::vector<int64_t>(p.buckets, p.buckets + 4); });
+        .def_property_readonly("G", [](const Plan& p) { return p.decoded().G; })
+        .def_property_readonly("windows", [](const Plan& p) { return p.decoded().windows; })
+        .def_property_readonly("A", [](const Plan& p) { return p.decoded().A; })
+        .def_property_readonly("c_max", [](const Plan& p) { return p.decoded().c_max; })
+        .def_property_readonly("oversize_groups", [](const Plan& p) { return p.decoded().oversize; })
+        .def_property_readonly("buckets", [](const Plan& p) { return std::vector<int64_t>(p.decoded().buckets, p.buckets + 4); });
     m.def("enqueue_plans", &enqueue_plans);
     m.def("window_indices", &window_indices);
     m.def("window_coords", &window_coords);

@@ -145,6 +145,45 @@ def test_token_plan_rejects_bad_indices():
     assert tp.G == len(np.unique(good[:, 0])) * H
 
 
+@pytest.mark.parametrize("dim,heads,path", [(96, 3, "resident"), (48, 3, "flash"), (96, 3, "fused"), (96, 3, "operators")])
+@pytest.mark.parametrize("bad,what", [([40, 3], "outside"), (None, "distinct")], ids=["outside", "twice"])
+def test_failed_plan_is_refused_on_every_use(dim, heads, path, bad, what):
+    """A plan whose totals failed their check stays in its view's cache: every later call on the view reports it again."""
+    from sparseswin3d_amd.window_attention import SparseVoxelTensor
+    attn = _modules(dim, heads, torch.float32)
+    set_path(attn, path if path != "flash" else "operators")
+    attn.fused, attn.resident = path != "operators", None if path == "flash" else attn.resident
+    good = random_window_indices(np.random.default_rng(5), 40, 125, 900)
+    ind = np.concatenate([good[:400], np.array([bad or good[17]], np.int32), good[400:]])
+    x = SparseVoxelTensor(torch.randn(len(ind), dim, device="cuda"), torch.from_numpy(ind).cuda(), (125,), 40)
+    x.plan_cache = {}
+    for _ in range(3):
+        with pytest.raises(RuntimeError, match=what):
+            attn(x, None)
+        with pytest.raises(RuntimeError, match=what), torch.no_grad():
+            attn(x, None)
+    plan = x.plan_cache[heads]
+    with pytest.raises(RuntimeError, match=what):
+        plan.finish()
+    with pytest.raises(RuntimeError, match=what):
+        plan.G
+
+
+def test_failed_merge_plan_is_refused_on_every_use():
+    from sparseswin3d_amd.fused import TokenPlan
+    from sparseswin3d_amd.layers import PoolDownsample
+    from sparseswin3d_amd.window_attention import SparseVoxelTensor
+    c4 = torch.tensor([[0, 1, 2, 3], [0, 4, 4, 4], [0, 1, 2, 3]], dtype=torch.int32, device="cuda")
+    pool = PoolDownsample(32).cuda()
+    x = SparseVoxelTensor(torch.randn(3, 32, device="cuda"), c4, (6, 6, 6), 1)
+    plan, = TokenPlan.batch([pool.plan_request(x)])
+    with pytest.raises(RuntimeError, match="finish"):
+        plan.windows                                              # not decoded yet
+    for _ in range(3):
+        with pytest.raises(RuntimeError, match="distinct"):
+            pool(x, plan)
+
+
 def _modules(dim, heads, dtype):
     from sparseswin3d_amd.window_attention import WindowAttentionSparse
     torch.manual_seed(0)
