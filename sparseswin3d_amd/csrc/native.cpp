@@ -15,6 +15,7 @@
 #include <hip/hip_runtime.h>
 
 #include <array>
+#include <atomic>
 #include <mutex>
 #include <optional>
 #include <string>
@@ -107,7 +108,9 @@ struct Plan : torch::CustomClassHolder {
     std::shared_ptr<SharedEvent> event;
     // allocated; its kernels are in the stream; its totals are decoded; its totals failed their check, which every later use
     // reports again (a plan stays in its view's cache, and the tables of a failed one are not filled)
-    enum State { FRESH, QUEUED, DONE, FAILED } state = FRESH;
+    enum State { FRESH, QUEUED, DONE, FAILED };
+    std::atomic<int> state{FRESH};
+    std::mutex mutex;                        // of the step from QUEUED to DONE or FAILED
     std::string failure;
     int64_t G = 0, windows = 0, A = 0, c_max = 0, buckets[4] = {0, 0, 0, 0}, oversize = 0;
 
@@ -131,16 +134,23 @@ struct Plan : torch::CustomClassHolder {
         if (event) (void)hipEventSynchronize(event->event);              // the kernels still write into totals
     }
 
+    // Any number of threads may ask: the first one waits and decodes, the others wait for it.  The lock is taken without the GIL
+    // only, so that a thread that holds the lock can never wait for one that holds the GIL.
     void finish() {
-        if (state == DONE) return;
-        TORCH_CHECK(state != FRESH, "token plan: its kernels were not launched");
-        if (state == QUEUED) {
+        if (state.load(std::memory_order_acquire) != DONE) {
             if (PyGILState_Check()) {
                 py::gil_scoped_release nogil;
-                wait();
+                complete();
             } else {
-                wait();
+                complete();
             }
+        }
+    }
+    void complete() {
+        std::lock_guard<std::mutex> lock(mutex);
+        TORCH_CHECK(state != FRESH, "token plan: its kernels were not launched");
+        if (state == QUEUED) {
+            TORCH_CHECK(hipEventSynchronize(event->event) == hipSuccess, "token plan: the stream failed");
             decode();
         }
         TORCH_CHECK(state == DONE, failure);
@@ -154,17 +164,17 @@ struct Plan : torch::CustomClassHolder {
         } else {
             failure = sswin_last_error();
         }
-        state = rc == 0 ? DONE : FAILED;
         event.reset();
         give_pinned(std::move(totals));
         ws = Tensor();
         indices = Tensor();
+        state.store(rc == 0 ? DONE : FAILED, std::memory_order_release);
     }
     const Plan& decoded() const {
-        TORCH_CHECK(state == DONE, state == FAILED ? failure : "token plan: the totals are there after finish()");
+        const int now = state.load(std::memory_order_acquire);
+        TORCH_CHECK(now == DONE, now == FAILED ? failure : "token plan: the totals are there after finish()");
         return *this;
     }
-    void wait() const { TORCH_CHECK(hipEventSynchronize(event->event) == hipSuccess, "token plan: the stream failed"); }
 };
 using PlanPtr = c10::intrusive_ptr<Plan>;
 

@@ -184,6 +184,41 @@ def test_failed_merge_plan_is_refused_on_every_use():
             pool(x, plan)
 
 
+@pytest.mark.parametrize("bad", [False, True])
+def test_plan_shared_by_threads(bad):
+    """Threads that meet at one deferred plan: one of them decodes it, all get its result (or its failure)."""
+    import threading
+    from sparseswin3d_amd.window_attention import SparseVoxelTensor, prefetch_plans
+    attn = _modules(96, 3, torch.float32)
+    ind = random_window_indices(np.random.default_rng(7), 4000, 125, 60000)
+    feats = torch.randn(len(ind), 96, device="cuda")
+    with torch.no_grad():
+        want = attn(SparseVoxelTensor(feats, torch.from_numpy(ind).cuda(), (125,), 4000), None).features
+    if bad:
+        ind[-1] = ind[0]
+    ind = torch.from_numpy(ind).cuda()
+    for _ in range(10):
+        x = SparseVoxelTensor(feats, ind, (125,), 4000)
+        prefetch_plans([(attn, x)])
+        gate, results = threading.Barrier(8), []
+
+        def work():
+            gate.wait()
+            try:
+                with torch.no_grad():
+                    results.append(attn(x, None).features)
+            except RuntimeError as e:
+                results.append(str(e))
+
+        threads = [threading.Thread(target=work) for _ in range(8)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+        assert len(results) == 8
+        assert all("distinct" in r if bad else torch.equal(r, want) for r in results)
+
+
 def _modules(dim, heads, dtype):
     from sparseswin3d_amd.window_attention import WindowAttentionSparse
     torch.manual_seed(0)
