@@ -178,29 +178,48 @@ struct Plan : torch::CustomClassHolder {
 };
 using PlanPtr = c10::intrusive_ptr<Plan>;
 
-// Launch allocated plans, four per library call; they share one event.
+// Launch allocated plans, four per library call; they share one event.  Where a call fails, the plans of the calls before it
+// are in the stream and can be used, and no plan gives up the memory its kernels may still write before the event.
 void enqueue_plans(const std::vector<PlanPtr>& plans) {
     if (plans.empty()) return;
     const Tensor& like = plans[0]->indices;
+    for (const PlanPtr& p : plans) {
+        TORCH_CHECK(p->state == Plan::FRESH, "TokenPlan: launched already");
+        TORCH_CHECK(p->indices.device() == like.device(), "TokenPlan.batch: all index sets must live on one device");
+    }
     c10::hip::HIPGuardMasqueradingAsCUDA guard(like.device());
     void* s = current_stream(like);
+    auto event = std::make_shared<SharedEvent>();
+    auto record = [&](size_t queued, size_t failed, const char* why) {       // [0, queued) launched, [queued, failed) perhaps in part
+        const bool ok = hipEventRecord(event->event, static_cast<hipStream_t>(s)) == hipSuccess;
+        if (!ok) (void)hipStreamSynchronize(static_cast<hipStream_t>(s));
+        for (size_t i = 0; i < failed; ++i) {
+            Plan& p = *plans[i];
+            if (ok) p.event = event;
+            if (!ok || i >= queued) p.failure = ok ? why : "hipEventRecord failed";
+            p.state = ok && i < queued ? Plan::QUEUED : Plan::FAILED;
+        }
+        TORCH_CHECK(ok || queued < failed, "hipEventRecord failed");
+    };
     for (size_t k = 0; k < plans.size(); k += 4) {
         sswin_token_plan_desc d[4];
         const int m = (int)std::min<size_t>(4, plans.size() - k);
         for (int i = 0; i < m; ++i) {
             Plan& p = *plans[k + i];
-            TORCH_CHECK(p.indices.device() == like.device(), "TokenPlan.batch: all index sets must live on one device");
             d[i] = sswin_token_plan_desc{};
             d[i].indices = i32(p.indices), d[i].N = p.N, d[i].B = (int32_t)p.B, d[i].n = (int32_t)p.n, d[i].H = p.H;
             d[i].flags = (p.order_only ? SSWIN_PLAN_ORDER_ONLY : 0) | SSWIN_PLAN_TOTALS_DIRECT;
             d[i].tokens = i32(p.tokens), d[i].plan = i32(p.plan), d[i].g_cap = p.g_cap, d[i].tasks = i32(p.tasks);
             d[i].totals_out = p.totals.data_ptr<int64_t>(), d[i].ws = p.ws.data_ptr(), d[i].ws_bytes = (size_t)p.ws.numel();
         }
-        RUN(sswin_token_plan_batch(d, m, s));
+        try {
+            RUN(sswin_token_plan_batch(d, m, s));
+        } catch (...) {
+            record(k, k + m, "token plan: its launch failed");
+            throw;
+        }
     }
-    auto event = std::make_shared<SharedEvent>();
-    TORCH_CHECK(hipEventRecord(event->event, static_cast<hipStream_t>(s)) == hipSuccess, "hipEventRecord failed");
-    for (const PlanPtr& p : plans) p->event = event, p->state = Plan::QUEUED;
+    record(plans.size(), plans.size(), "");
 }
 
 // (batch, d, h, w) -> (window slot, position) of the padded grid rolled by -shift

@@ -219,6 +219,31 @@ def test_plan_shared_by_threads(bad):
         assert all("distinct" in r if bad else torch.equal(r, want) for r in results)
 
 
+def test_plans_launched_before_a_refused_call_stay_usable():
+    """Six plans are two library calls; the second one is refused on the host (more heads than it takes).  The first four are
+    in the stream: they can be finished, and their totals are not freed under the kernels that write them."""
+    from sparseswin3d_amd import _lib
+    native = _lib.native()
+    rng = np.random.default_rng(3)
+    sets = [random_window_indices(rng, 900, 125, 20000 + 500 * k) for k in range(6)]
+    for drop in (True, False):
+        plans = [native.Plan(torch.from_numpy(i).cuda(), 900, 125, 300 if k == 5 else 3, True, False) for k, i in enumerate(sets)]
+        with pytest.raises(RuntimeError, match="bad sizes in plan 1"):
+            native.enqueue_plans(plans)
+        with pytest.raises(RuntimeError, match="launched already"):
+            native.enqueue_plans(plans[:1])
+        for p in plans[4:]:
+            for _ in range(2):
+                with pytest.raises(RuntimeError, match="launch failed"):
+                    p._finish()
+        if drop:
+            del plans, p                                          # in flight
+            continue
+        for p, i in zip(plans[:4], sets):
+            p._finish()
+            assert (p.G, p.N) == (3 * len(np.unique(i[:, 0])), len(i))
+
+
 def _modules(dim, heads, dtype):
     from sparseswin3d_amd.window_attention import WindowAttentionSparse
     torch.manual_seed(0)
