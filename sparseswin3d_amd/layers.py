@@ -235,6 +235,14 @@ def _plain(*modules) -> bool:
     return all(type(m) in (nn.LayerNorm, nn.Linear, nn.GELU) for m in modules) and _unhooked(*modules)
 
 
+def _passes(drop) -> bool:
+    """A dropout that leaves its input as it is.  Each module obeys its own ``training``: one that was put back in train mode acts
+    in an eval model as well."""
+    kind = type(drop)
+    return kind is nn.Identity or (kind is nn.Dropout and (not drop.training or drop.p == 0)) or \
+        (kind is DropPath and (not drop.training or drop.drop_prob == 0))
+
+
 def _norm_fits(norm, features) -> bool:
     """``norm`` is a LayerNorm over the rows of ``features`` with gain and offset in the types the kernels take."""
     return type(norm) is nn.LayerNorm and norm.weight is not None and norm.bias is not None and len(norm.normalized_shape) == 1 \
@@ -415,11 +423,10 @@ class SwinTransformerBlock(nn.Module):
     def _fused_arguments(self, x):
         """The compute dtype where the whole block runs as one autograd node, else None: LayerNorm, the fused attention path, GELU, and no dropout that is switched on."""
         attn, mlp, f = self.attn, self.mlp, x.features
-        if self.training and (mlp.drop1.p > 0 or mlp.drop2.p > 0 or attn.proj_drop.p > 0 or
-                              (type(self.drop_path) is not nn.Identity and self.drop_path.drop_prob > 0)):
+        if type(mlp) is not MLP or type(attn) is not WindowAttentionSparse or \
+                not (_passes(mlp.drop1) and _passes(mlp.drop2) and _passes(attn.proj_drop) and _passes(self.drop_path)):
             return None
-        if type(mlp) is not MLP or type(mlp.fn) is not nn.GELU or mlp.fn.approximate != "none" or \
-                type(attn) is not WindowAttentionSparse or not _unhooked(attn, mlp) or not _plain(self.norm1, self.norm2, attn.qkv, attn.proj, mlp.linear1, mlp.linear2, mlp.fn):
+        if type(mlp.fn) is not nn.GELU or mlp.fn.approximate != "none" or not _unhooked(attn, mlp) or not _plain(self.norm1, self.norm2, attn.qkv, attn.proj, mlp.linear1, mlp.linear2, mlp.fn):
             return None
         if not (x.indices.is_cuda and x.indices.dtype == torch.int32 and x.indices.shape[0] > 0 and attn.num_heads < 256):
             return None
