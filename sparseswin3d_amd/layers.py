@@ -21,7 +21,7 @@ from torch.autograd.function import once_differentiable
 
 from . import _lib
 from .fused import attention_path
-from .window_attention import WindowAttentionSparse, _token_plan, prefetch_plans, replace_feature, tall_linear
+from .window_attention import WindowAttentionSparse, _token_plan, prefetch_plans, replace_feature, tall_linear, unhooked
 
 _DTYPE_CODE = {torch.float32: 0, torch.float16: 1, torch.bfloat16: 2}
 
@@ -226,13 +226,9 @@ def downsample_plan(x, factor: int = 2, plan=None):
     return plan, coords, [e // f for e in dims]
 
 
-def _unhooked(*modules) -> bool:
-    return not any(m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks for m in modules)
-
-
 def _plain(*modules) -> bool:
     """Modules of exactly these types without hooks: calling them is applying their parameters."""
-    return all(type(m) in (nn.LayerNorm, nn.Linear, nn.GELU) for m in modules) and _unhooked(*modules)
+    return all(type(m) in (nn.LayerNorm, nn.Linear, nn.GELU) for m in modules) and unhooked(*modules)
 
 
 def _passes(drop) -> bool:
@@ -421,12 +417,15 @@ class SwinTransformerBlock(nn.Module):
         return replace_feature(x, self.drop_path(self.mlp(x.features)))
 
     def _fused_arguments(self, x):
-        """The compute dtype where the whole block runs as one autograd node, else None: LayerNorm, the fused attention path, GELU, and no dropout that is switched on."""
+        """The compute dtype where the whole block runs as one autograd node, else None: LayerNorm, the fused attention path, GELU,
+        no dropout that is switched on, and nothing that a call of one of the modules passed by would run besides."""
         attn, mlp, f = self.attn, self.mlp, x.features
-        if type(mlp) is not MLP or type(attn) is not WindowAttentionSparse or \
-                not (_passes(mlp.drop1) and _passes(mlp.drop2) and _passes(attn.proj_drop) and _passes(self.drop_path)):
+        if type(self) is not SwinTransformerBlock or type(mlp) is not MLP or type(attn) is not WindowAttentionSparse or \
+                not self.__dict__.keys().isdisjoint(("forward_part1", "forward_part2", "window_view")):
             return None
-        if type(mlp.fn) is not nn.GELU or mlp.fn.approximate != "none" or not _unhooked(attn, mlp) or not _plain(self.norm1, self.norm2, attn.qkv, attn.proj, mlp.linear1, mlp.linear2, mlp.fn):
+        drops = mlp.drop1, mlp.drop2, attn.proj_drop, self.drop_path
+        if not all(map(_passes, drops)) or type(mlp.fn) is not nn.GELU or mlp.fn.approximate != "none" or \
+                not _plain(self.norm1, self.norm2, attn.qkv, attn.proj, mlp.linear1, mlp.linear2, mlp.fn) or not unhooked(attn, mlp, *drops):
             return None
         if not (x.indices.is_cuda and x.indices.dtype == torch.int32 and x.indices.shape[0] > 0 and attn.num_heads < 256):
             return None

@@ -687,6 +687,18 @@ def relative_position_index_3d(window_size: Sequence[int]) -> torch.Tensor:
     return rel.sum(-1)
 
 
+def unhooked(*modules) -> bool:
+    """Calling these modules is running their class's ``forward`` and nothing else: no hooks, their own or global ones, and no
+    ``forward`` set on an instance."""
+    if nn.modules.module._has_any_global_hook():
+        return False
+    for m in modules:
+        d = m.__dict__
+        if d["_forward_hooks"] or d["_forward_pre_hooks"] or d["_backward_hooks"] or d["_backward_pre_hooks"] or "forward" in d:
+            return False
+    return True
+
+
 class WindowAttentionSparse(nn.Module):
     """Window multi-head self attention with relative position bias on sparse windows.
 
@@ -754,8 +766,7 @@ class WindowAttentionSparse(nn.Module):
             return None
         autocast = torch.is_autocast_enabled("cuda")
         # under autocast the projections are called as modules (tall_linear), which may be anything
-        if autocast and any(type(m) is not nn.Linear or m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks
-                            for m in (self.qkv, self.proj)):
+        if autocast and not (type(self.qkv) is nn.Linear and type(self.proj) is nn.Linear and unhooked(self.qkv, self.proj)):
             return None
         dtype = torch.get_autocast_dtype("cuda") if autocast else features.dtype
         weight = self.qkv.weight.dtype

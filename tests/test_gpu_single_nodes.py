@@ -76,6 +76,42 @@ INSIDE = ["attn", "mlp", "attn.proj_drop", "mlp.drop1", "mlp.drop2", "drop_path"
 CALLED = [p for p in INSIDE if p not in ("attn.qkv", "attn.proj", "mlp.linear1", "mlp.linear2")]
 
 
+@pytest.mark.parametrize("path", CALLED)
+def test_hooks_inside_a_block_run(path):
+    layer, run, feats = _stage_pieces(96, 3, 5, torch.float32, False, 5)
+    plain = run(feats)
+    m = _of(layer.blocks[0], path)
+    calls = []
+    for register in (m.register_forward_hook, m.register_forward_pre_hook):
+        calls.clear()
+        handle = register(lambda *a: calls.append(1))
+        y = run(feats)
+        handle.remove()
+        assert len(calls) == (2 if path == "drop_path" else 1)    # both branches
+        assert torch.allclose(y, plain, rtol=1e-4, atol=1e-5)
+    calls.clear()
+    handle = m.register_full_backward_hook(lambda *a: calls.append(1))
+    if path != "attn":                                            # a view goes in and comes out: no tensors, no backward hook
+        run(feats.clone().requires_grad_(True)).sum().backward()
+        assert calls
+    handle.remove()
+
+
+@pytest.mark.parametrize("register", [nn.modules.module.register_module_forward_hook, nn.modules.module.register_module_forward_pre_hook,
+                                      nn.modules.module.register_module_full_backward_hook], ids=["forward", "forward_pre", "backward"])
+def test_global_module_hooks_see_the_modules_of_a_block_and_a_merge(register):
+    layer, run, feats = _stage_pieces(96, 3, 5, torch.float32, True, 5)
+    seen = set()
+    handle = register(lambda m, *a: seen.add(id(m)) and None)
+    try:
+        run(feats.clone().requires_grad_(True)).sum().backward()
+    finally:
+        handle.remove()
+    blk = layer.blocks[0]
+    for m in [_of(blk, p) for p in CALLED if p != "attn"] + [layer.downsample.norm]:
+        assert id(m) in seen, type(m)
+
+
 @pytest.mark.parametrize("training", [True, False], ids=["train", "eval"])
 @pytest.mark.parametrize("path", ["drop_path", "attn.proj_drop", "mlp.drop1", "mlp.drop2"])
 def test_other_types_in_place_of_dropout_run(path, training):
@@ -88,3 +124,45 @@ def test_other_types_in_place_of_dropout_run(path, training):
     assert not torch.allclose(run(feats), plain, rtol=1e-3, atol=1e-3)
     setattr(owner, name, nn.Identity())
     assert torch.allclose(run(feats), plain, rtol=1e-4, atol=1e-5)
+
+
+@pytest.mark.parametrize("what", ["forward_part1", "forward_part2", "window_view"])
+@pytest.mark.parametrize("how", ["subclass", "instance"])
+def test_overridden_parts_of_a_block_run(what, how):
+    from sparseswin3d_amd.layers import SwinTransformerBlock
+    layer, run, feats = _stage_pieces(96, 3, 5, torch.float32, False, 5)
+    plain = run(feats)
+    calls = []
+    original = getattr(SwinTransformerBlock, what)
+
+    def replaced(self, *a):
+        calls.append(1)
+        return original(self, *a)
+
+    blk = layer.blocks[0]
+    if how == "subclass":
+        blk.__class__ = type("Other", (SwinTransformerBlock,), {what: replaced})
+    else:
+        object.__setattr__(blk, what, replaced.__get__(blk))
+    y = run(feats)
+    assert len(calls) >= (2 if what == "window_view" else 1)      # the stage asks for the view once itself
+    assert torch.allclose(y, plain, rtol=1e-4, atol=1e-5)
+
+
+@pytest.mark.parametrize("path", CALLED)
+def test_forward_replaced_on_an_instance_runs(path):
+    layer, run, feats = _stage_pieces(96, 3, 5, torch.float32, False, 5)
+    m = _of(layer.blocks[0], path)
+    calls, original = [], m.forward
+    m.forward = lambda *a, **k: (calls.append(1), original(*a, **k))[1]
+    run(feats)
+    assert calls
+
+
+def test_merge_modules_replaced_on_an_instance_run():
+    layer, run, feats = _stage_pieces(96, 3, 5, torch.float32, True, 5)
+    norm, calls = layer.downsample.norm, []
+    original = norm.forward
+    norm.forward = lambda x: (calls.append(1), original(x))[1]
+    run(feats)
+    assert calls == [1]
