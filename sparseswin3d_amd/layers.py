@@ -242,7 +242,7 @@ def _passes(drop) -> bool:
 def _norm_fits(norm, features) -> bool:
     """``norm`` is a LayerNorm over the rows of ``features`` with gain and offset in the types the kernels take."""
     return type(norm) is nn.LayerNorm and norm.weight is not None and norm.bias is not None and len(norm.normalized_shape) == 1 \
-        and norm.normalized_shape[0] == features.shape[1] and norm.weight.dtype == features.dtype \
+        and norm.normalized_shape[0] == features.shape[1] and norm.weight.dtype == norm.bias.dtype == features.dtype \
         and _lib.native().norm_supported(features)
 
 
@@ -432,7 +432,7 @@ class SwinTransformerBlock(nn.Module):
         weight = attn.qkv.weight
         dtype = _fused_dtype(f, weight)
         if dtype is None or not (_norm_fits(self.norm1, f) and _norm_fits(self.norm2, f)) or \
-                any(m.weight.dtype != weight.dtype for m in (attn.proj, mlp.linear1, mlp.linear2)):
+                any(p is not None and p.dtype != weight.dtype for m in (attn.qkv, attn.proj, mlp.linear1, mlp.linear2) for p in (m.weight, m.bias)):
             return None
         return dtype
 

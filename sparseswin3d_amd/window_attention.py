@@ -769,10 +769,12 @@ class WindowAttentionSparse(nn.Module):
         if autocast and not (type(self.qkv) is nn.Linear and type(self.proj) is nn.Linear and unhooked(self.qkv, self.proj)):
             return None
         dtype = torch.get_autocast_dtype("cuda") if autocast else features.dtype
-        weight = self.qkv.weight.dtype
-        if dtype not in fused._DTYPE_CODE or weight not in (dtype, torch.float32) or self.proj.weight.dtype != weight:
+        params = [p.dtype for m in (self.qkv, self.proj) for p in (m.weight, m.bias) if p is not None]
+        if dtype not in fused._DTYPE_CODE or any(p != params[0] for p in params):
             return None
-        if features.dtype != dtype and not autocast:
+        # outside autocast operands of one type, inside what autocast would cast; anything else is the layers' own error
+        if params[0] != dtype and not (autocast and params[0] == torch.float32) or \
+                (features.dtype != dtype and not (autocast and features.dtype in fused._DTYPE_CODE)):
             return None
         ti = self._table_index(n)
         if n > 384 if ti is not None else n * n * 4 > 64 * 1024:

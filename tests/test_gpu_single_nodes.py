@@ -166,3 +166,34 @@ def test_merge_modules_replaced_on_an_instance_run():
     norm.forward = lambda x: (calls.append(1), original(x))[1]
     run(feats)
     assert calls == [1]
+
+
+@pytest.mark.parametrize("x,w", [(torch.bfloat16, torch.float32), (torch.float16, torch.float32), (torch.float32, torch.float16), (torch.float64, torch.float32)])
+@pytest.mark.parametrize("grad", [True, False], ids=["grad", "no_grad"])
+def test_features_and_weights_of_different_types_are_refused(x, w, grad):
+    """Outside autocast a dense layer refuses operands of two types, as nn.Linear does, and does not round the weights; inside
+    float64 features stay refused."""
+    from sparseswin3d_amd.window_attention import SparseVoxelTensor, WindowAttentionSparse
+    torch.manual_seed(0)
+    attn = WindowAttentionSparse(96, 3, (5, 5, 5), qkv_bias=True).cuda().to(w)
+    ind = torch.from_numpy(random_window_indices(np.random.default_rng(0), 40, 125, 700)).cuda()
+    feats = torch.randn(700, 96, device="cuda").to(x)
+    with torch.set_grad_enabled(grad), pytest.raises(RuntimeError, match="dtype"):
+        attn(SparseVoxelTensor(feats, ind, (125,), 40), None)
+    if x == torch.float64:
+        with torch.set_grad_enabled(grad), torch.autocast("cuda", dtype=torch.float16), pytest.raises(RuntimeError, match="dtype"):
+            attn(SparseVoxelTensor(feats, ind, (125,), 40), None)
+    layer, run, _ = _stage_pieces(96, 3, 5, w, True, 7)
+    with torch.set_grad_enabled(grad), pytest.raises(RuntimeError):
+        run(torch.randn(3000, 96, device="cuda").to(x))
+
+
+@pytest.mark.parametrize("path", ["attn.qkv.bias", "attn.proj.bias", "mlp.linear1.bias", "mlp.linear2.bias", "norm1.bias", "norm2.bias", "attn.proj.weight"])
+def test_parameters_of_another_type_are_refused(path):
+    """One parameter of a fp32 block left in bf16: refused by the layer it belongs to, not rounded or widened on the way."""
+    layer, run, feats = _stage_pieces(96, 3, 5, torch.float32, False, 7)
+    owner, _, name = path.rpartition(".")
+    m = _of(layer.blocks[0], owner)
+    m._parameters[name] = nn.Parameter(m._parameters[name].detach().bfloat16())
+    with pytest.raises(RuntimeError):
+        run(feats)
