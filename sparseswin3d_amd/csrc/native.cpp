@@ -394,6 +394,10 @@ DenseGrads dense_backward(const Tensor& dy, const Tensor& x, const Tensor& w_in,
 // row normalisation
 // ------------------------------------------------------------------------------------------
 Tensor norm_forward(const Tensor& x, const Tensor& gamma_in, const Tensor& beta_in, double eps, ScalarType out, Tensor* stats) {
+    TORCH_CHECK(x.dim() == 2 && gamma_in.dim() == 1 && gamma_in.size(0) == x.size(1) && beta_in.sizes() == gamma_in.sizes() &&
+                    gamma_in.scalar_type() == x.scalar_type() && beta_in.scalar_type() == x.scalar_type(),
+                "a norm with a gain of ", gamma_in.sizes(), " ", gamma_in.scalar_type(), " and an offset of ", beta_in.sizes(), " ", beta_in.scalar_type(),
+                " on rows of ", x.sizes(), " ", x.scalar_type());
     const Tensor gamma = ready(gamma_in), beta = ready(beta_in);
     Tensor y = at::empty(x.sizes(), x.options().dtype(out));
     if (stats) *stats = at::empty({2, x.size(0)}, x.options().dtype(at::kFloat));
@@ -727,6 +731,7 @@ struct MergeNode : torch::autograd::Function<MergeNode> {
                           ScalarType type) {
         NoAutocast off;
         plan->finish();
+        TORCH_CHECK(x_in.dim() == 2 && x_in.size(0) == plan->N, "merge: rows of ", x_in.sizes(), " for a plan of ", plan->N, " voxels");
         const Tensor x = ready(x_in);
         const int64_t M = plan->windows, D = x.size(1);
         Tensor pooled = at::empty({M, D}, x.options()), stats;

@@ -175,6 +175,8 @@ class _PoolWindows(Function):
 
     @staticmethod
     def forward(ctx, features, plan, mean):
+        if features.dim() != 2 or features.shape[0] != plan.N:
+            raise RuntimeError(f"pooling rows of {list(features.shape)} with a plan of {plan.N} voxels")
         features = features.contiguous()
         M, channels = plan.windows, features.shape[1]
         out = torch.empty((M, channels), dtype=features.dtype, device=features.device)

@@ -197,3 +197,31 @@ def test_parameters_of_another_type_are_refused(path):
     m._parameters[name] = nn.Parameter(m._parameters[name].detach().bfloat16())
     with pytest.raises(RuntimeError):
         run(feats)
+
+
+@pytest.mark.parametrize("single", [True, False], ids=["node", "composed"])
+@pytest.mark.parametrize("grad", [True, False], ids=["grad", "no_grad"])
+def test_merge_refuses_rows_that_are_not_its_voxels(single, grad, monkeypatch):
+    from sparseswin3d_amd import layers
+    from sparseswin3d_amd.window_attention import SparseVoxelTensor
+    if not single:
+        monkeypatch.setattr(layers, "_fused_dtype", lambda *a: None)
+    pool = layers.PoolDownsample(32).cuda()
+    cells = np.random.default_rng(0).choice(20 ** 3, size=900, replace=False)
+    c4 = torch.from_numpy(np.stack([0 * cells, *np.unravel_index(cells, (20, 20, 20))], 1).astype(np.int32)).cuda()
+    with torch.set_grad_enabled(grad):
+        for n in (899, 901, 1, 0):
+            with pytest.raises(RuntimeError, match="900 voxels"):
+                pool(SparseVoxelTensor(torch.randn(n, 32, device="cuda"), c4, (20, 20, 20), 1))
+        pool(SparseVoxelTensor(torch.randn(900, 32, device="cuda"), c4, (20, 20, 20), 1))
+
+
+@pytest.mark.parametrize("owner", ["block", "merge"])
+@pytest.mark.parametrize("name", ["weight", "bias"])
+@pytest.mark.parametrize("size", [48, 192])
+def test_norm_parameters_of_another_size_are_refused(owner, name, size):
+    layer, run, feats = _stage_pieces(96, 3, 5, torch.float32, True, 7)
+    norm = layer.blocks[0].norm2 if owner == "block" else layer.downsample.norm
+    norm._parameters[name] = nn.Parameter(torch.ones(size, device="cuda"))
+    with pytest.raises(RuntimeError):
+        run(feats)
