@@ -293,6 +293,12 @@ template <size_t COUNT> std::array<Tensor, COUNT> in_type(const std::array<Tenso
     return out;
 }
 
+// the kernels take pointers: a parameter or plan left on another device has to stop here
+void same_device(const Tensor& x, std::initializer_list<const Tensor*> others) {
+    for (const Tensor* t : others)
+        TORCH_CHECK(!t->defined() || t->device() == x.device(), "all tensors of a call have to be on the same device: found ", x.device(), " and ", t->device());
+}
+
 // x [N, K], w [P, K] -> last step of x w^T + b
 Tensor dense(const Tensor& x, const Tensor& w_in, const Tensor& b_in, int epilogue = SSWIN_DENSE_PLAIN, const Tensor& extra = Tensor(),
              Tensor* slope = nullptr, std::optional<ScalarType> out_type = std::nullopt) {
@@ -448,6 +454,10 @@ Tensor attention_forward(Attention& a, const Tensor& qkv, const Tensor& bias, At
     tp.finish();
     TORCH_CHECK(qkv.dim() == 2 && qkv.size(0) == tp.N && qkv.size(1) % (3 * a.H) == 0 && tp.H == a.H && tp.n == a.n, "attention: qkv of ", qkv.sizes(),
                 " for a plan of ", tp.N, " tokens in windows of ", tp.n, " and ", tp.H, " heads");
+    TORCH_CHECK(!tp.order_only && (!a.resident || tp.tasks.defined()), "attention: the plan was made without what the attention reads");
+    same_device(qkv, {&bias, &a.mask, &a.code, &tp.tokens});
+    TORCH_CHECK(!a.code.defined() || (a.code.numel() == a.n && a.code.scalar_type() == at::kInt && a.code.is_contiguous()), "attention: position codes of ",
+                a.code.sizes());
     TORCH_CHECK(a.code.defined() ? bias.dim() == 2 && bias.size(1) == a.H : bias.dim() == 3 && bias.size(0) == a.H && bias.size(1) == a.n && bias.size(2) == a.n,
                 "attention: bias of ", bias.sizes());
     TORCH_CHECK(!a.mask.defined() || (a.mask.dim() == 2 && a.mask.size(0) > 0 && a.mask.size(1) == a.n), "attention: mask of ", a.mask.sizes());
@@ -629,6 +639,7 @@ struct ModuleNode : torch::autograd::Function<ModuleNode> {
                           const Tensor& proj_w, const OptTensor& proj_bias, AttentionPtr a, ScalarType type) {
         NoAutocast off;
         const Tensor qkv_b = or_undefined(qkv_bias), proj_b = or_undefined(proj_bias);
+        same_device(x_in, {&qkv_w, &qkv_b, &proj_w, &proj_b});
         const Tensor x = ready(x_in.to(type));
         const auto w = in_type<4>({qkv_w, qkv_b, proj_w, proj_b}, type);
         const Tensor qkv = dense(x, w[0], w[1]);
@@ -669,7 +680,10 @@ struct BlockNode : torch::autograd::Function<BlockNode> {
                           ScalarType type) {
         NoAutocast off;
         Tensor p[PARAMS];
-        for (size_t i = 0; i < which.size(); ++i) p[which[i]] = given[i];
+        for (size_t i = 0; i < which.size(); ++i) {
+            p[which[i]] = given[i];
+            same_device(p[X], {&p[which[i]]});
+        }
         const Tensor x = ready(p[X]);
         const ScalarType stream_type = x.scalar_type();                  // of the residual stream
         const ScalarType params_type = p[QKVW].scalar_type();
@@ -732,6 +746,7 @@ struct MergeNode : torch::autograd::Function<MergeNode> {
         NoAutocast off;
         plan->finish();
         TORCH_CHECK(x_in.dim() == 2 && x_in.size(0) == plan->N, "merge: rows of ", x_in.sizes(), " for a plan of ", plan->N, " voxels");
+        same_device(x_in, {&gamma, &beta, &w, &plan->tokens});
         const Tensor x = ready(x_in);
         const int64_t M = plan->windows, D = x.size(1);
         Tensor pooled = at::empty({M, D}, x.options()), stats;

@@ -175,8 +175,8 @@ class _PoolWindows(Function):
 
     @staticmethod
     def forward(ctx, features, plan, mean):
-        if features.dim() != 2 or features.shape[0] != plan.N:
-            raise RuntimeError(f"pooling rows of {list(features.shape)} with a plan of {plan.N} voxels")
+        if features.dim() != 2 or features.shape[0] != plan.N or features.device != plan.device:
+            raise RuntimeError(f"pooling rows of {list(features.shape)} on {features.device} with a plan of {plan.N} voxels on {plan.device}")
         features = features.contiguous()
         M, channels = plan.windows, features.shape[1]
         out = torch.empty((M, channels), dtype=features.dtype, device=features.device)

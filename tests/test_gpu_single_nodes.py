@@ -225,3 +225,35 @@ def test_norm_parameters_of_another_size_are_refused(owner, name, size):
     norm._parameters[name] = nn.Parameter(torch.ones(size, device="cuda"))
     with pytest.raises(RuntimeError):
         run(feats)
+
+
+@pytest.mark.parametrize("path", ["blocks.0.norm1.weight", "blocks.0.attn.qkv.weight", "blocks.0.attn.proj.bias", "blocks.1.norm2.bias", "blocks.1.mlp.linear1.weight",
+                                  "downsample.norm.weight", "downsample.reduction.weight"])
+@pytest.mark.parametrize("grad", [True, False], ids=["grad", "no_grad"])
+def test_parameters_on_another_device_are_refused(path, grad):
+    layer, run, feats = _stage_pieces(96, 3, 5, torch.float32, True, 7)
+    owner, _, name = path.rpartition(".")
+    m = layer
+    for part in owner.split("."):
+        m = m._modules[part]
+    m._parameters[name] = nn.Parameter(m._parameters[name].detach().cpu())
+    with torch.set_grad_enabled(grad), pytest.raises(RuntimeError, match="same device"):
+        run(feats)
+
+
+def test_attention_refuses_masks_and_plans_it_cannot_read():
+    from sparseswin3d_amd.fused import BiasTableIndex, TokenPlan, fused_window_attention
+    from sparseswin3d_amd.window_attention import SparseVoxelTensor, WindowAttentionSparse, relative_position_index_3d
+    attn = WindowAttentionSparse(96, 3, (5, 5, 5), qkv_bias=True).cuda()
+    ind = torch.from_numpy(random_window_indices(np.random.default_rng(0), 40, 125, 700)).cuda()
+    feats = torch.randn(700, 96, device="cuda")
+    with pytest.raises(RuntimeError, match="same device"):
+        attn(SparseVoxelTensor(feats, ind, (125,), 40), torch.zeros(40, 125, dtype=torch.int8))
+    ti = BiasTableIndex.build(relative_position_index_3d((5, 5, 5)).cuda(), 729)
+    qkv, table = torch.randn(700, 3, 3, 32, device="cuda"), torch.randn(729, 3, device="cuda")
+    for kw in (dict(tasks=False), dict(tasks=True, order_only=True), dict(tasks=False, order_only=True)):
+        with pytest.raises(RuntimeError, match="without what"):
+            fused_window_attention(qkv, table, ind, None, 40, 125, 0.2, plan=TokenPlan(ind, 40, 125, 3, **kw), table_index=ti)
+    small = BiasTableIndex.build(relative_position_index_3d((4, 4, 4)).cuda(), 343)
+    with pytest.raises(RuntimeError, match="position codes"):
+        fused_window_attention(qkv, table, ind, None, 40, 125, 0.2, table_index=small)
