@@ -513,8 +513,8 @@ def _split_linear_forward(x: torch.Tensor, weight: torch.Tensor, bias):
     """``x @ W^T + b`` through the library's matrix-core kernel for fp32 (operands split into bf16
     pieces, fp32 accuracy), or None when the shape or dtype is outside what that kernel takes."""
     if not (x.is_cuda and x.dtype == torch.float32 and weight.dtype == torch.float32 and x.dim() == 2
-            and x.shape[0] > 0 and weight.device == x.device
-            and (bias is None or (bias.dtype == torch.float32 and bias.device == x.device))):
+            and x.shape[0] > 0 and weight.device == x.device and weight.dim() == 2 and weight.shape[1] == x.shape[1]
+            and (bias is None or (bias.dtype == torch.float32 and bias.device == x.device and bias.shape == weight.shape[:1]))):
         return None
     import ctypes as C
     from . import _lib

@@ -206,3 +206,15 @@ def test_module_projection_matches_library_gemm():
     torch.testing.assert_close(x.grad.double(), xr.grad, rtol=1e-5, atol=1e-5)
     torch.testing.assert_close(layer.weight.grad.double(), ref_layer.weight.grad, rtol=1e-5, atol=2e-4)
     torch.testing.assert_close(layer.bias.grad.double(), ref_layer.bias.grad, rtol=1e-5, atol=2e-4)
+
+
+def test_rows_and_biases_that_do_not_fit_the_layer_are_refused():
+    """Shapes the layer does not fit reach nn.Linear's own check instead of a kernel."""
+    from sparseswin3d_amd.window_attention import tall_linear
+    layer = torch.nn.Linear(96, 288).cuda()
+    assert tall_linear(torch.randn(500, 96, device="cuda"), layer).shape == (500, 288)
+    with pytest.raises(RuntimeError):
+        tall_linear(torch.randn(500, 48, device="cuda"), layer)
+    layer.bias = torch.nn.Parameter(torch.zeros(384, device="cuda"))
+    with pytest.raises(RuntimeError):
+        tall_linear(torch.randn(500, 96, device="cuda"), layer)
