@@ -139,9 +139,15 @@ struct Block {
 
 // The blocks that start in the 32 ranks of a chunk, one after the other.  Lane l holds what is known of rank r0 + l (a block
 // may reach 31 ranks past its chunk); all of it is requested together, before the bias table is waited for.
+//
+// Values that are not finite: 0 x inf is NaN, so one of them in a row that takes part with P = 0 (another window of a merged block,
+// the repeated rows behind a window's end) or in a product with the identity would spread.  The kernels look at a block's results:
+// where one is NaN the block is done again, and the rest of the chunk after it, one window at a time with columns read lane by
+// lane and nothing behind the end.  Finite tokens pay one comparison a block.
 struct Blocks {
     int r0, T, c, voxel;
-    uint32_t word, starts;
+    uint32_t word, starts, before;
+    bool careful;
     __device__ __forceinline__ Blocks(const Args& g, int64_t chunk) {
         r0 = (int)(chunk * 32);
         const int r = r0 + (int)(threadIdx.x & 63), at = (int)(r < g.N ? r : g.N - 1);
@@ -153,11 +159,19 @@ struct Blocks {
     __device__ __forceinline__ void begin(const Args& g) {
         const int lane = threadIdx.x & 63, r = r0 + lane;
         starts = (uint32_t)__ballot(lane < 32 && r < g.N && ((r - T) & 31) == 0);
+        careful = false;
+    }
+    // the block next() returned last once more, if a sum of its results is NaN
+    __device__ __forceinline__ bool again(float sum) {
+        if (careful || !__any(sum != sum)) return false;
+        starts = before;
+        return careful = true;
     }
     // of the block's own token s * 16 + l % 16 (the last one again behind it)
     __device__ __forceinline__ int slot(const Block& b, int s) const { return b.a - r0 + min(s * 16 + (int)(threadIdx.x & 15), b.len - 1); }
     __device__ __forceinline__ bool next(Block& b) {
         if (!starts) return false;
+        before = starts;
         int j = __builtin_ctz(starts);
         starts &= starts - 1;
         const int T0 = __builtin_amdgcn_readlane(T, j), c0 = __builtin_amdgcn_readlane(c, j);
@@ -170,7 +184,7 @@ struct Blocks {
             return true;
         }
         // small windows that follow each other share a block as long as they fit
-        while (starts) {
+        while (starts && !careful) {
             j = __builtin_ctz(starts);
             const int cn = __builtin_amdgcn_readlane(c, j);
             if (cn >= 32 || b.to - b.a + cn > 32) break;
@@ -188,6 +202,15 @@ __device__ __forceinline__ float across(float v, bool maximum) {         // over
     v = maximum ? fmaxf(v, o) : v + o;
     o = __shfl_xor(v, 32, 64);
     return maximum ? fmaxf(v, o) : v + o;
+}
+
+template <int NB> __device__ __forceinline__ float sum_of(const f32x4 (&o)[2][NB]) {
+    float t = 0.f;
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+#pragma unroll
+        for (int c = 0; c < NB; ++c) t += (o[s][c][0] + o[s][c][1]) + (o[s][c][2] + o[s][c][3]);
+    return t;
 }
 
 // Workgroup -> head and first chunk: the heads of the same tokens follow each other on one XCD, whose L2 holds their rows
@@ -217,7 +240,7 @@ template <typename T, int HD> struct Rows {
         for (int b = 0; b < NB; ++b) f[b].load(base + (__umul24(v, pitch) + col + b * 16));
     }
     // fp32 column operand: lane (channel 16 b + l % 16, slots = the tokens 4 (l / 16) + j with voxels v[j])
-    __device__ __forceinline__ void column(const int (&v)[4], const Frag<T> (&rows)[NB], Frag<float> (&f)[NB]) const {
+    __device__ __forceinline__ void column(const int (&v)[4], const Frag<T> (&rows)[NB], Frag<float> (&f)[NB], bool careful) const {
         if constexpr (sizeof(T) == 4) {
 #pragma unroll
             for (int b = 0; b < NB; ++b)
@@ -231,7 +254,27 @@ template <typename T, int HD> struct Rows {
             const Frag<T> id = packed<T>(one);
 #pragma unroll
             for (int b = 0; b < NB; ++b) f[b].v = mma(rows[b], id, f32x4{0.f, 0.f, 0.f, 0.f});
+            if (careful) {                                               // the product spreads what is not finite over its row
+                const int l16 = threadIdx.x & 15, quad = (threadIdx.x & 63) >> 4;
+#pragma unroll
+                for (int b = 0; b < NB; ++b) {
+                    const uint2 w = __builtin_bit_cast(uint2, rows[b].v);
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        const int from = (l16 >> 2) * 16 + quad * 4 + j; // holds channels 4 (l16 / 4) .. + 3 of token 4 quad + j
+                        const uint32_t lo = __shfl(w.x, from, 64), hi = __shfl(w.y, from, 64), pair = l16 & 2 ? hi : lo;
+                        f[b].v[j] = to_acc(__builtin_bit_cast(T, (uint16_t)(l16 & 1 ? pair >> 16 : pair)));
+                    }
+                }
+            }
         }
+    }
+    // clears the slots behind the window's end: they hold its last token again, with P = 0
+    static __device__ __forceinline__ void clear(int last, Frag<float> (&f)[NB]) {
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) f[b].v[j] = (int)((threadIdx.x & 63) >> 4) * 4 + j > last ? 0.f : f[b].v[j];
     }
 };
 
@@ -291,10 +334,11 @@ __device__ __forceinline__ float score(float acc, float scale2, uint32_t pq, uin
 }
 
 // ------------------------------------------------------------------------------------------
-// forward: own = queries
+// forward: own = queries.  fp32: three wavefronts per SIMD, which heads of 32 channels miss by one register (two are spilled;
+// 84 742 tokens, windows of 7^3, 3 heads of 32: 74.7 us)
 // ------------------------------------------------------------------------------------------
 template <typename T, int HD>
-__global__ __launch_bounds__(WAVES * 64) void flash_forward_kernel(Args g, int64_t groups) {
+__global__ __launch_bounds__(WAVES * 64, sizeof(T) == 4 ? 3 : 1) void flash_forward_kernel(Args g, int64_t groups) {
     constexpr int NB = HD / 16;
     extern __shared__ float table[];
     int h;
@@ -333,7 +377,7 @@ __global__ __launch_bounds__(WAVES * 64) void flash_forward_kernel(Args g, int64
         uint32_t w_next[4];
         auto request = [&]() {
             k_rows.row((uint32_t)ahead.row, k_next);
-            if constexpr (sizeof(T) == 4) v_rows.column(ahead.v, v_next, v_next);
+            if constexpr (sizeof(T) == 4) v_rows.column(ahead.v, v_next, v_next, false);
             else v_rows.row((uint32_t)ahead.row, v_next);
 #pragma unroll
             for (int j = 0; j < 4; ++j) w_next[j] = ahead.w[j];
@@ -356,8 +400,9 @@ __global__ __launch_bounds__(WAVES * 64) void flash_forward_kernel(Args g, int64
                 for (int c = 0; c < NB; ++c) vt[c] = v[c];
             } else {
                 const int none[4] = {0, 0, 0, 0};
-                v_rows.column(none, v, vt);
+                v_rows.column(none, v, vt, blocks.careful);
             }
+            if (blocks.careful && last < 15) v_rows.clear(last, vt);
             auto tile = [&](auto fast_tag) {
                 constexpr bool FAST = decltype(fast_tag)::value;
 #pragma unroll
@@ -399,6 +444,7 @@ __global__ __launch_bounds__(WAVES * 64) void flash_forward_kernel(Args g, int64
             if (last >= 15 && !general) tile(std::true_type{});
             else tile(std::false_type{});
         }
+        if (blocks.again(sum_of(o))) continue;
 #pragma unroll
         for (int s = 0; s < 2; ++s) {
             if (s >= subs) break;
@@ -483,7 +529,8 @@ __global__ __launch_bounds__(WAVES * 64) void flash_backward_q_kernel(Args g, in
             Frag<float> kt[NB];
             k_rows.row((uint32_t)step.row, k);
             v_rows.row((uint32_t)step.row, v);
-            k_rows.column(step.v, k, kt);
+            k_rows.column(step.v, k, kt, blocks.careful);
+            if (blocks.careful && last < 15) k_rows.clear(last, kt);
             if (last >= 16) ahead.load(g, k0 + 16, b.to);
             auto tile = [&](auto fast_tag) {
                 constexpr bool FAST = decltype(fast_tag)::value;
@@ -498,8 +545,8 @@ __global__ __launch_bounds__(WAVES * 64) void flash_backward_q_kernel(Args g, in
 #pragma unroll
                     for (int j = 0; j < 4; ++j) {
                         float x = score<FAST>(acc[j], scale2, pq[s], step.w[j], table);
-                        if (!FAST && quad * 4 + j > last) x = -INFINITY;
                         ds[j] = __builtin_amdgcn_exp2f(x) * dp[j];
+                        if (!FAST && quad * 4 + j > last) ds[j] = 0.f;
                     }
                     if (g.ds && s * 16 + l16 < b.len) {                  // four neighbours of a row of dS per lane
                         float* row = g.ds + at[s] + k0 + quad * 4;
@@ -519,6 +566,7 @@ __global__ __launch_bounds__(WAVES * 64) void flash_backward_q_kernel(Args g, in
             if (last >= 15 && !general) tile(std::true_type{});
             else tile(std::false_type{});
         }
+        if (blocks.again(sum_of(dq))) continue;
 #pragma unroll
         for (int s = 0; s < 2; ++s) {
             if (s * 16 + l16 < b.len) {
@@ -583,7 +631,7 @@ __global__ __launch_bounds__(WAVES * 64) void flash_backward_kv_kernel(Args g, i
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
                     const int64_t r = h * g.N + q0 + min(quad * 4 + j, last);
-                    lse[j] = quad * 4 + j <= last ? g.lse[r] : INFINITY;   // rows past the end: P = 0
+                    lse[j] = g.lse[r];
                     delta[j] = g.delta[r];
                 }
             }
@@ -591,8 +639,12 @@ __global__ __launch_bounds__(WAVES * 64) void flash_backward_kv_kernel(Args g, i
             Frag<float> qt[NB], dot[NB];
             q_rows.row((uint32_t)step.row, q);
             do_rows.row((uint32_t)step.row, d_o);
-            q_rows.column(step.v, q, qt);
-            do_rows.column(step.v, d_o, dot);
+            q_rows.column(step.v, q, qt, blocks.careful);
+            do_rows.column(step.v, d_o, dot, blocks.careful);
+            if (blocks.careful && last < 15) {
+                q_rows.clear(last, qt);
+                do_rows.clear(last, dot);
+            }
             if (last >= 16) ahead.load(g, q0 + 16, b.to);
             const f32x4 a0 = lse * -unscale, d0 = -delta;               // what the accumulators start from
             auto tile = [&](auto fast_tag) {
@@ -606,7 +658,9 @@ __global__ __launch_bounds__(WAVES * 64) void flash_backward_kv_kernel(Args g, i
 #pragma unroll
                     for (int j = 0; j < 4; ++j) {
                         p[j] = __builtin_amdgcn_exp2f(score<FAST>(acc[j], scale2, step.w[j] + (uint32_t)g.offset4, pk[s], table));
+                        if (!FAST && quad * 4 + j > last) p[j] = 0.f;
                         ds[j] = p[j] * dp[j];
+                        if (!FAST && quad * 4 + j > last) ds[j] = 0.f;
                     }
                     const Frag<float> pf = {p}, df = {ds};
 #pragma unroll
@@ -616,6 +670,7 @@ __global__ __launch_bounds__(WAVES * 64) void flash_backward_kv_kernel(Args g, i
             if (last >= 15 && !general) tile(std::true_type{});
             else tile(std::false_type{});
         }
+        if (blocks.again(sum_of(dk) + sum_of(dv))) continue;
 #pragma unroll
         for (int s = 0; s < 2; ++s) {
             if (s * 16 + l16 < b.len) {

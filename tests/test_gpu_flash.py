@@ -94,3 +94,64 @@ def test_flash_fp16_gradients_outside_the_range_of_fp16():
         got.append(x.grad.double())
     assert torch.isfinite(got[1]).all()
     assert ((got[0] - got[1]).norm() / got[1].norm()).item() < 1e-3     # an ulp of fp16 at most
+
+
+def _float64(qkv, table, index, ind, scale, up):
+    """Output and gradients of qkv in float64, window by window; what is not finite stays where the formulas put it."""
+    N, _, H, hd = qkv.shape
+    x, t, d_o = qkv.double().cpu(), table.double().cpu(), up.double().cpu().view(N, H, hd)
+    out, d = torch.empty(N, H, hd, dtype=torch.float64), torch.empty_like(x)
+    for w in ind[:, 0].unique():
+        rows = (ind[:, 0] == w).nonzero()[:, 0]
+        pos = ind[rows, 1].long()
+        for h in range(H):
+            q, k, v = (x[rows, i, h] for i in range(3))
+            s = scale * (q @ k.T) + t[index[pos][:, pos], h]
+            e = torch.exp(s - s.amax(1, keepdim=True).clamp_min(0))
+            p = e / (e.sum(1, keepdim=True) + 1e-8)
+            o, g = p @ v, d_o[rows, h]
+            ds = p * (g @ v.T - (g * o).sum(1, keepdim=True))
+            out[rows, h] = o
+            d[rows, 0, h], d[rows, 1, h], d[rows, 2, h] = scale * ds @ k, scale * ds.T @ q, p.T @ g
+    return out.view(N, -1), d
+
+
+@pytest.mark.parametrize("which", ["q", "k", "v", "dO"])
+@pytest.mark.parametrize("value", [float("inf"), float("nan")], ids=["inf", "nan"])
+@pytest.mark.parametrize("hd,dtype", [(16, torch.float32), (32, torch.float32), (16, torch.float16), (32, torch.bfloat16)],
+                         ids=["16-fp32", "32-fp32", "16-fp16", "32-bf16"])
+def test_flash_keeps_what_is_not_finite_where_it_belongs(which, value, hd, dtype):
+    """One channel of one token of a few windows is not finite: other windows keep their results, whichever windows share a block
+    with them, and inside the window infinities and NaN stand where float64 has them.  Bounds of finite values: as above, per
+    result (5 x the norm's bound, at a norm of one token's row)."""
+    from sparseswin3d_amd import _lib
+    from sparseswin3d_amd.fused import BiasTableIndex, TokenPlan
+    from sparseswin3d_amd.window_attention import relative_position_index_3d
+    counts, n, H = [3, 1, 2, 5, 31, 1, 7, 9, 15, 17, 1, 2, 4, 33, 40, 3, 3, 64, 100, 2, 2, 200], 343, 2
+    index = relative_position_index_3d((7, 7, 7))
+    ti = BiasTableIndex.build(index.cuda(), 13 ** 3)
+    ind = torch.from_numpy(ragged_window_indices(np.random.default_rng(hd), counts, n))
+    torch.manual_seed(hd)
+    qkv, up = torch.randn(len(ind), 3, H, hd).to(dtype), torch.randn(len(ind), H * hd).to(dtype)
+    table = torch.randn(13 ** 3, H) * 0.3
+    hit = [int((ind[:, 0] == w).nonzero()[-1]) for w in (3, 6, 13, 15, 18, 21)]
+    for r in hit:
+        if which == "dO":
+            up[r, hd + 3] = value                                 # of head 1
+        else:
+            qkv[r, "qkv".index(which), 1, 3] = value
+    x = qkv.cuda().requires_grad_(True)
+    plan = TokenPlan(ind.cuda(), len(counts), n, H)
+    out = _lib.native().attention(x, table.cuda(), plan.native, None, ti.code, ti.offset0, n, hd ** -0.5, "flash")
+    out.backward(up.cuda())
+    ref = _float64(qkv, table, index, ind, hd ** -0.5, up)
+    tol = {torch.float32: 1e-4, torch.float16: 5e-3, torch.bfloat16: 3e-2}[dtype]
+    for got, want, what in zip((out.detach(), x.grad), ref, ("out", "d qkv")):
+        got = got.double().cpu()
+        finite = want.isfinite()
+        assert got[finite].isfinite().all(), what
+        assert ((got - want)[finite].abs() <= tol * (1 + want[finite].abs())).all(), what
+        assert torch.equal(got[want.isinf()], want[want.isinf()]), what
+        assert not got[want.isnan()].isfinite().any(), what
+    if which != "dO":
+        assert not torch.isfinite(out).all()
