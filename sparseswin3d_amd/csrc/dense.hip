@@ -4,7 +4,8 @@
 //
 // Products run on the 16-bit matrix cores with fp32 accumulation.  fp32 operands are split exactly into three bf16
 // pieces (x = h + m + l by truncation and exact subtraction) and a product is the sum of the six piece products that
-// weigh at least 2^-16 of the leading one; what is dropped is below 2^-23 of the product.
+// weigh at least 2^-16 of the leading one; what is dropped is below 2^-23 of the product.  Infinities and NaN give what they give
+// in plain fp32 (plain_products below).
 //
 // dense_rows_kernel (fp32): a workgroup of WM wavefronts owns BM = 32 MT WM rows and 96 columns.  Both operands pass through
 // registers, where they are split, into LDS in matrix operand order, [row tile][plane][lane] pieces of 16 bytes, so that every
@@ -84,6 +85,36 @@ __device__ __forceinline__ void planes_of(const float (&v)[8], u32x4 (&out)[Op<T
 #pragma unroll
         for (int q = 0; q < 4; ++q) out[0][q] = pack2<T>(v[2 * q], v[2 * q + 1]);
     }
+}
+
+// Pieces of an infinity hold a NaN, and so does every result one takes part in, as do pieces whose sums leave the range: fp32
+// results that come out NaN are formed again from the operands in plain fp32, in the order of the reduction, until they are
+// NaN there as well.
+__device__ __forceinline__ bool nan_among(const f32x4& v) {
+    const float t = (v[0] + v[1]) + (v[2] + v[3]);                       // infinities of both signs too: formed again for nothing
+    return t != t;
+}
+// sum over i < n of a[i a_step] b[i b_step + e b_next], e < 4; four steps of the reduction in flight
+__device__ __forceinline__ f32x4 plain_products(const float* a, int64_t a_step, const float* b, int64_t b_step, int64_t b_next, int64_t n) {
+    f32x4 s = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+    for (int64_t i0 = 0; i0 < n && (s[0] == s[0] || s[1] == s[1] || s[2] == s[2] || s[3] == s[3]); i0 += 4) {
+        float v[4];
+        f32x4 w[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int64_t i = i0 + q < n ? i0 + q : n - 1;
+            v[q] = a[i * a_step];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) w[q][e] = b[i * b_step + e * b_next];
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            if (i0 + q < n)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) s[e] = fmaf(v[q], w[q][e], s[e]);
+    }
+    return s;
 }
 
 // ------------------------------------------------------------------------------------------
@@ -297,6 +328,21 @@ __global__ __launch_bounds__(WM * 64) __attribute__((amdgpu_waves_per_eu(OCC, OC
             for (int r = 0; r < 16; ++r) mine[acc_row(r, half) * PITCH + j * 32 + l32] = acc[i][j][r];
         __builtin_amdgcn_wave_barrier();
         constexpr int PIECES = 32 * (BN / 4) / 64;
+        f32x4 any = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) any[r & 3] += acc[i][j][r];
+        if (__any(nan_among(any))) {
+#pragma unroll 1
+            for (int q = 0; q < PIECES; ++q) {
+                const int e = q * 64 + lane, rr = e / (BN / 4), cc = (e % (BN / 4)) * 4;
+                f32x4* v = reinterpret_cast<f32x4*>(mine + rr * PITCH + cc);
+                if (r0 + rr < N && col0 + cc < P && nan_among(*v))
+                    *v = plain_products(x + (r0 + rr) * K, 1, w + (DOWN ? col0 + cc : (int64_t)(col0 + cc) * K), DOWN ? P : 1, DOWN ? 1 : K, K);
+            }
+            __builtin_amdgcn_wave_barrier();
+        }
         Second4<float, float, EPI> second[PIECES];
 #pragma unroll
         for (int q = 0; q < PIECES; ++q) {
@@ -722,6 +768,9 @@ __device__ __forceinline__ void small_tile(int block, const T* __restrict__ x, i
         f32x4 v = *reinterpret_cast<const f32x4*>(&sums[0][rr * 36 + cc]);
 #pragma unroll
         for (int q = 1; q < SMALL_WAVES; ++q) v += *reinterpret_cast<const f32x4*>(&sums[q][rr * 36 + cc]);
+        if constexpr (PL == 3)
+            if (__builtin_expect(in && nan_among(v), 0))
+                v = plain_products(x + (row0 + rr) * K, 1, w + (DOWN ? col0 + cc : (int64_t)(col0 + cc) * K), DOWN ? P : 1, DOWN ? 1 : K, K);
         if (in) finish4<T, TO, EPI>(ep, row0 + rr, col0 + cc, P, v, second);
     }
 }
@@ -888,6 +937,7 @@ __global__ __launch_bounds__(WM * WN * 64) __attribute__((amdgpu_waves_per_eu(OC
         }
     }
     float* pw = part_w + chunk * (int64_t)P * K;
+    f32x4 any = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int i = 0; i < MT; ++i)
 #pragma unroll
@@ -896,7 +946,17 @@ __global__ __launch_bounds__(WM * WN * 64) __attribute__((amdgpu_waves_per_eu(OC
             for (int r = 0; r < 16; ++r) {
                 const int p = p0 + (wm * MT + i) * 32 + acc_row(r, half), k = k0 + (wn * NT + j) * 32 + l32;
                 if (p < P && k < K) pw[(int64_t)p * K + k] = acc[i][j][r];
+                any[r & 3] += acc[i][j][r];
             }
+    if (__builtin_expect(nan_among(any), 0)) {                              // those of this lane that are NaN, read back where they were stored
+#pragma unroll 1
+        for (int e = 0; e < MT * NT * 16; ++e) {
+            const int p = p0 + (wm * MT + e / (NT * 16)) * 32 + acc_row(e & 15, half), k = k0 + (wn * NT + e / 16 % NT) * 32 + l32;
+            if (p >= P || k >= K) continue;
+            const float v = pw[(int64_t)p * K + k];
+            if (v != v) pw[(int64_t)p * K + k] = plain_products(dy + begin * P + p, P, x + begin * K + k, K, 0, end - begin)[0];
+        }
+    }
     if (sums_here) {
         // unit u holds rows of chunk u / (BM / 2) of its column pair: the chunks of a pair are added in order
         __syncthreads();
@@ -967,6 +1027,8 @@ __device__ __forceinline__ void wgrad_small_tile(int block, const T* __restrict_
 #pragma unroll
         for (int q = 1; q < SMALL_WAVES; ++q) v += *reinterpret_cast<const f32x4*>(&sums[q][rr * 36 + cc]);
         if (p0 + rr < P && k0 + cc < K) {
+            if constexpr (PL == 3)
+                if (__builtin_expect(nan_among(v), 0)) v = plain_products(dy + p0 + rr, P, x + k0 + cc, K, 1, N);
             Vec4<TO> o;
 #pragma unroll
             for (int e = 0; e < 4; ++e) o.v[e] = from_acc<TO>(v[e]);

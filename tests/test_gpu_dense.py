@@ -329,3 +329,72 @@ def test_layer_norm_backward_with_a_16_bit_copy(N, D, kind):
         if with_copy:
             assert torch.equal(copy, dx.to(kind))
     assert all(torch.equal(a, b) for a, b in zip(*results))
+
+
+# the tiled kernel (half a step of the reduction and whole ones), the few-rows one; weight gradients: few rows and each tile shape
+EXACT_ROWS = [(20000, 48, 96), (20000, 16, 112), (300, 384, 208), (33, 96, 96), (20001, 144, 48)]
+EXACT_WGRAD = [(900, 144, 48), (9001, 208, 192), (20001, 48, 208), (30001, 64, 48), (40001, 144, 48), (9000, 208, 96)]
+
+
+def _same_class(got, ref, scale, what):
+    """Finite where float64 is (to the bound of the file), the same infinities, NaN where float64 has NaN."""
+    got = got.double()
+    finite = ref.isfinite()
+    assert got[finite].isfinite().all(), what
+    assert ((got - ref)[finite].abs() <= 1e-6 * scale[finite] + 1e-30).all(), what
+    assert torch.equal(got[ref.isinf()], ref[ref.isinf()]), what
+    assert got[ref.isnan()].isnan().all(), what
+
+
+@pytest.mark.parametrize("N,K,P", EXACT_ROWS)
+@pytest.mark.parametrize("value", [float("inf"), float("-inf"), float("nan"), 3.4028234e38])
+@pytest.mark.parametrize("where", ["rows", "weight"])
+def test_dense_fp32_of_values_that_are_not_finite(N, K, P, value, where):
+    """An infinity, a NaN or the largest number in a few places: the results that depend on them are those of plain fp32
+    arithmetic.  (Rows or columns of the largest number are scaled down, so that the result is in range.)"""
+    from sparseswin3d_amd import _lib
+    lib = _lib.load()
+    gen = torch.Generator().manual_seed(N + K)
+    for transposed in (0, 1):
+        rows, cols = (P, K) if transposed else (K, P)             # of the reduction and the result
+        x, w = torch.randn(N, rows, generator=gen), torch.randn(P, K, generator=gen)
+        if abs(value) < float("inf"):
+            x, w = x * 2.0 ** -10, w * 2.0 ** -10
+        for r, c in ((0, 1), (N // 2, rows - 1), (N - 1, 0)):
+            if where == "rows":
+                x[r, c] = value
+            elif transposed:
+                w[c, r % K] = value
+            else:
+                w[r % P, c] = value
+        x[N // 3] = 0                                              # 0 x inf
+        x, w = x.cuda(), w.cuda()
+        y, _ = _forward(lib, _lib, x, w, None, transposed, PLAIN, None, torch.float32)
+        wd = w.double() if transposed else w.double().T
+        ref, scale = x.double() @ wd, x.double().abs() @ wd.abs()
+        _same_class(y, ref, scale, f"transposed {transposed}")
+        assert (abs(value) < float("inf")) == bool(ref.isfinite().all())
+
+
+@pytest.mark.parametrize("N,P,K", EXACT_WGRAD)
+@pytest.mark.parametrize("value", [float("inf"), float("nan"), 3.4028234e38])
+@pytest.mark.parametrize("where", ["dy", "x"])
+def test_dense_fp32_weight_gradient_of_values_that_are_not_finite(N, P, K, value, where):
+    from sparseswin3d_amd import _lib
+    lib = _lib.load()
+    gen = torch.Generator().manual_seed(N + K)
+    dy, x = torch.randn(N, P, generator=gen), torch.randn(N, K, generator=gen)
+    if abs(value) < float("inf"):
+        dy, x = dy * 2.0 ** -12, x * 2.0 ** -12
+    t = dy if where == "dy" else x
+    for r, c in ((0, 1), (N // 2, t.shape[1] - 1), (N - 1, 7)):
+        t[r, c] = value
+        (x if where == "dy" else dy)[r, :5] = 0
+    dy, x = dy.cuda(), x.cuda()
+    dw, db = torch.empty(P, K, device="cuda"), torch.empty(P, device="cuda")
+    nb = lib.sswin_dense_weight_grad_workspace_bytes(0, N, P, K)
+    ws = torch.empty(max(nb, 1), dtype=torch.uint8, device="cuda")
+    _lib.check(lib.sswin_dense_weight_grad(0, 0, _ptr(dy), _ptr(x), N, P, K, _ptr(dw), _ptr(db), _ptr(ws), nb, _stream()))
+    d, v = dy.double(), x.double()
+    _same_class(dw, d.T @ v, d.abs().T @ v.abs(), "dW")
+    _same_class(db, d.sum(0), d.abs().sum(0), "db")
