@@ -21,7 +21,7 @@ from torch.autograd.function import once_differentiable
 
 from . import _lib
 from .fused import attention_path
-from .window_attention import WindowAttentionSparse, _token_plan, prefetch_plans, replace_feature, tall_linear, unhooked
+from .window_attention import WindowAttentionSparse, _token_plan, prefetch_plans, param, replace_feature, tall_linear, unhooked
 
 _DTYPE_CODE = {torch.float32: 0, torch.float16: 1, torch.bfloat16: 2}
 
@@ -230,7 +230,13 @@ def downsample_plan(x, factor: int = 2, plan=None):
 
 def _plain(*modules) -> bool:
     """Modules of exactly these types without hooks: calling them is applying their parameters."""
-    return all(type(m) in (nn.LayerNorm, nn.Linear, nn.GELU) for m in modules) and unhooked(*modules)
+    for m in modules:
+        if type(m) not in _PLAIN_TYPES:
+            return False
+    return unhooked(*modules)
+
+
+_PLAIN_TYPES = frozenset((nn.LayerNorm, nn.Linear, nn.GELU))
 
 
 def _passes(drop) -> bool:
@@ -241,11 +247,16 @@ def _passes(drop) -> bool:
         (kind is DropPath and (not drop.training or drop.drop_prob == 0))
 
 
-def _norm_fits(norm, features) -> bool:
-    """``norm`` is a LayerNorm over the rows of ``features`` with gain and offset in the types the kernels take."""
-    return type(norm) is nn.LayerNorm and norm.weight is not None and norm.bias is not None and len(norm.normalized_shape) == 1 \
-        and norm.normalized_shape[0] == features.shape[1] and norm.weight.dtype == norm.bias.dtype == features.dtype \
-        and _lib.native().norm_supported(features)
+def _norms_fit(features, *norms) -> bool:
+    """Each of ``norms`` is a LayerNorm over the rows of ``features`` with gain and offset in the types the kernels take."""
+    width, dtype = features.shape[1], features.dtype
+    for norm in norms:
+        if type(norm) is not nn.LayerNorm or norm.normalized_shape != (width,):
+            return False
+        for p in (param(norm, "weight"), param(norm, "bias")):
+            if p is None or p.dtype != dtype:
+                return False
+    return _lib.native().norm_supported(features)
 
 
 def _fused_dtype(features, weight):
@@ -283,7 +294,7 @@ class PoolDownsample(nn.Module):
     def forward(self, x, plan=None):
         plan, coords, shape = downsample_plan(x, 2, plan)
         dtype = _fused_dtype(x.features, self.reduction.weight) if _plain(self.norm, self.reduction) else None
-        if dtype is not None and _norm_fits(self.norm, x.features) and self.reduction.bias is None:
+        if dtype is not None and _norms_fit(x.features, self.norm) and self.reduction.bias is None:
             # pooling, norm and the dense layer in one autograd node
             features = _lib.native().merge(x.features, self.norm.weight, self.norm.bias, self.reduction.weight, plan.native, self.norm.eps,
                                            dtype)
@@ -343,6 +354,10 @@ class DropPath(nn.Module):
         if keep > 0.0 and self.scale_by_keep:
             mask.div_(keep)
         return x * mask
+
+
+# what a block would look up on itself, were it set on the instance
+_BLOCK_PARTS = ("attn", "mlp", "norm1", "norm2", "drop_path", "forward_part1", "forward_part2", "window_view")
 
 
 class SwinTransformerBlock(nn.Module):
@@ -419,39 +434,52 @@ class SwinTransformerBlock(nn.Module):
         return replace_feature(x, self.drop_path(self.mlp(x.features)))
 
     def _fused_arguments(self, x):
-        """The compute dtype where the whole block runs as one autograd node, else None: LayerNorm, the fused attention path, GELU,
-        no dropout that is switched on, and nothing that a call of one of the modules passed by would run besides."""
-        attn, mlp, f = self.attn, self.mlp, x.features
-        if type(self) is not SwinTransformerBlock or type(mlp) is not MLP or type(attn) is not WindowAttentionSparse or \
-                not self.__dict__.keys().isdisjoint(("forward_part1", "forward_part2", "window_view")):
+        """(attention module, parameters in the compiled block's order, compute dtype) where the whole block runs as one autograd
+        node, else None: LayerNorm, the fused attention path, GELU, no dropout that is switched on, and nothing that a call of one
+        of the modules passed by would run besides.  Submodules and parameters are taken from the modules' own dictionaries:
+        nn.Module's attribute access would be most of this function's time."""
+        if type(self) is not SwinTransformerBlock or not self.__dict__.keys().isdisjoint(_BLOCK_PARTS):
             return None
-        drops = mlp.drop1, mlp.drop2, attn.proj_drop, self.drop_path
-        if not all(map(_passes, drops)) or type(mlp.fn) is not nn.GELU or mlp.fn.approximate != "none" or \
-                not _plain(self.norm1, self.norm2, attn.qkv, attn.proj, mlp.linear1, mlp.linear2, mlp.fn) or not unhooked(attn, mlp, *drops):
+        parts = self._modules
+        attn, mlp, norm1, norm2, f = parts["attn"], parts["mlp"], parts["norm1"], parts["norm2"], x.features
+        if type(mlp) is not MLP or type(attn) is not WindowAttentionSparse:
             return None
-        if not (x.indices.is_cuda and x.indices.dtype == torch.int32 and x.indices.shape[0] > 0 and attn.num_heads < 256):
+        a, m = attn._modules, mlp._modules
+        qkv, proj, linear1, linear2, gelu = a["qkv"], a["proj"], m["linear1"], m["linear2"], m["fn"]
+        drops = m["drop1"], m["drop2"], a["proj_drop"], parts["drop_path"]
+        if not all(map(_passes, drops)) or type(gelu) is not nn.GELU or gelu.approximate != "none" or \
+                not _plain(norm1, norm2, qkv, proj, linear1, linear2, gelu) or not unhooked(attn, mlp, *drops):
             return None
-        weight = attn.qkv.weight
+        indices = x.indices
+        if not (indices.is_cuda and indices.dtype == torch.int32 and indices.shape[0] > 0 and attn.num_heads < 256):
+            return None
+        weight = param(qkv, "weight")
         dtype = _fused_dtype(f, weight)
-        if dtype is None or not (_norm_fits(self.norm1, f) and _norm_fits(self.norm2, f)) or \
-                any(p is not None and p.dtype != weight.dtype for m in (attn.qkv, attn.proj, mlp.linear1, mlp.linear2) for p in (m.weight, m.bias)):
+        if dtype is None or not _norms_fit(f, norm1, norm2):
             return None
-        return dtype
+        layers, kind = [], weight.dtype
+        for layer in (qkv, proj, linear1, linear2):
+            for name in ("weight", "bias"):
+                p = param(layer, name)
+                if p is not None and p.dtype != kind:
+                    return None
+                layers.append(p)
+        return attn, [f, param(norm1, "weight"), param(norm1, "bias"), layers[0], layers[1], attn.relative_position_bias_table, layers[2], layers[3],
+                      param(norm2, "weight"), param(norm2, "bias"), *layers[4:]], dtype
 
     def forward(self, x, mask_matrix):
-        dtype = self._fused_arguments(x)
-        if dtype is not None:
+        fused = self._fused_arguments(x)
+        if fused is not None:
+            attn, params, dtype = fused
             view, shifted = self._view_of(x)
-            attn, mlp, n = self.attn, self.mlp, view.spatial_shape[0]
+            n = view.spatial_shape[0]
             how = attn._fused_arguments(x.features, n)
             if how is not None and how[0] is not None:
                 ti = how[0]
                 plan = _token_plan(attn, view)
-                y = _lib.native().block(
-                    [x.features, self.norm1.weight, self.norm1.bias, attn.qkv.weight, attn.qkv.bias, attn.relative_position_bias_table,
-                     attn.proj.weight, attn.proj.bias, self.norm2.weight, self.norm2.bias, mlp.linear1.weight, mlp.linear1.bias,
-                     mlp.linear2.weight, mlp.linear2.bias], plan.native, mask_matrix if shifted else None, ti.code, ti.offset0, n,
-                    attn.num_heads, attn.scale, attention_path(attn.dim // attn.num_heads, n, ti, attn.resident), self.norm1.eps, self.norm2.eps, dtype)
+                norms = self._modules["norm1"], self._modules["norm2"]
+                y = _lib.native().block(params, plan.native, mask_matrix if shifted else None, ti.code, ti.offset0, n, attn.num_heads, attn.scale,
+                                        attention_path(attn.dim // attn.num_heads, n, ti, attn.resident), norms[0].eps, norms[1].eps, dtype)
                 return replace_feature(x, y)
         shortcut = x
         x = self.forward_part1(x, mask_matrix)

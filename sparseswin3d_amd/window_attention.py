@@ -700,6 +700,12 @@ def unhooked(*modules) -> bool:
     return True
 
 
+def param(module, name):
+    """``getattr(module, name)`` of a parameter, without nn.Module's attribute access where it is registered as one."""
+    p = module._parameters.get(name)
+    return p if p is not None else getattr(module, name)
+
+
 class WindowAttentionSparse(nn.Module):
     """Window multi-head self attention with relative position bias on sparse windows.
 
@@ -766,16 +772,19 @@ class WindowAttentionSparse(nn.Module):
         if not self.fused or features.dim() != 2:
             return None
         autocast = torch.is_autocast_enabled("cuda")
+        qkv, proj = (self._modules.get(k) or getattr(self, k) for k in ("qkv", "proj"))
         # under autocast the projections are called as modules (tall_linear), which may be anything
-        if autocast and not (type(self.qkv) is nn.Linear and type(self.proj) is nn.Linear and unhooked(self.qkv, self.proj)):
+        if autocast and not (type(qkv) is nn.Linear and type(proj) is nn.Linear and unhooked(qkv, proj)):
             return None
-        dtype = torch.get_autocast_dtype("cuda") if autocast else features.dtype
-        params = [p.dtype for m in (self.qkv, self.proj) for p in (m.weight, m.bias) if p is not None]
-        if dtype not in fused._DTYPE_CODE or any(p != params[0] for p in params):
-            return None
+        given = features.dtype
+        dtype = torch.get_autocast_dtype("cuda") if autocast else given
+        weight = param(qkv, "weight").dtype
+        for p in (param(qkv, "bias"), param(proj, "weight"), param(proj, "bias")):
+            if p is not None and p.dtype != weight:
+                return None
         # outside autocast operands of one type, inside what autocast would cast; anything else is the layers' own error
-        if params[0] != dtype and not (autocast and params[0] == torch.float32) or \
-                (features.dtype != dtype and not (autocast and features.dtype in fused._DTYPE_CODE)):
+        if dtype not in fused._DTYPE_CODE or (weight != dtype and not (autocast and weight == torch.float32)) or \
+                (given != dtype and not (autocast and given in fused._DTYPE_CODE)):
             return None
         ti = self._table_index(n)
         if n > 384 if ti is not None else n * n * 4 > 64 * 1024:
