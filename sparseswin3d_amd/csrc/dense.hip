@@ -3,7 +3,7 @@
 // product folded into its last step: bias, GELU and its derivative, the product with that derivative, the residual sum.
 //
 // Products run on the 16-bit matrix cores with fp32 accumulation.  fp32 operands are split exactly into three bf16
-// pieces (x = h + m + l by truncation and exact subtraction) and a product is the sum of the six piece products that
+// pieces (x = h + m + l, split2 below) and a product is the sum of the six piece products that
 // weigh at least 2^-16 of the leading one; what is dropped is below 2^-23 of the product.  Infinities and NaN give what they give
 // in plain fp32 (plain_products below).
 //
@@ -61,14 +61,21 @@ template <> struct Op<__hip_bfloat16> {
     }
 };
 
+// x = h + m + l exactly, h rounded to nearest (a carry of the half into the upper 16 bits), m and l cut off: with x of leading power
+// 1, |m| <= 2^-8 and |l| < 2^-16, so that the products left out (m l, l m, l l) stay below 2^-23.  Cutting h off as well, |m| < 2^-7
+// and |l| < 2^-15 with x's sign, they reach 2^-21 and add up (equal operands just below 1 + 2^-7: 7.9 x 2^-24 of the result, now
+// 2.0 x 2^-24).  The price is two additions a pair: 112 700 rows 48 -> 144 and 48 -> 48 together 48.1 -> 49.1 us, their weight
+// gradients 52.2 -> 53.6.  Rounding m as well (2^-24) costs twice that, v_cvt_pk_bf16_f32 in place of the integer forms 20 % of the
+// narrow weight gradients, the two missing products 15 % of the wide layers.  From 2^128 - 2^119 on h is infinite: see plain_products.
 __device__ __forceinline__ void split2(float x0, float x1, uint32_t& h, uint32_t& m, uint32_t& l) {
-    const uint32_t u0 = __builtin_bit_cast(uint32_t, x0), u1 = __builtin_bit_cast(uint32_t, x1);
-    const float r0 = x0 - __builtin_bit_cast(float, u0 & 0xffff0000u), r1 = x1 - __builtin_bit_cast(float, u1 & 0xffff0000u);
-    const uint32_t v0 = __builtin_bit_cast(uint32_t, r0), v1 = __builtin_bit_cast(uint32_t, r1);
-    const float s0 = r0 - __builtin_bit_cast(float, v0 & 0xffff0000u), s1 = r1 - __builtin_bit_cast(float, v1 & 0xffff0000u);
-    h = __builtin_amdgcn_perm(u1, u0, 0x07060302u);
-    m = __builtin_amdgcn_perm(v1, v0, 0x07060302u);
-    l = __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, s1), __builtin_bit_cast(uint32_t, s0), 0x07060302u);
+    auto bits = [](float v) { return __builtin_bit_cast(uint32_t, v); };
+    auto value = [](uint32_t v) { return __builtin_bit_cast(float, v & 0xffff0000u); };
+    auto upper = [](uint32_t hi, uint32_t lo) { return __builtin_amdgcn_perm(hi, lo, 0x07060302u); };
+    const uint32_t u0 = bits(x0) + 0x8000u, u1 = bits(x1) + 0x8000u;
+    const float r0 = x0 - value(u0), r1 = x1 - value(u1);
+    h = upper(u1, u0);
+    m = upper(bits(r1), bits(r0));
+    l = upper(bits(r1 - value(bits(r1))), bits(r0 - value(bits(r0))));
 }
 
 // eight fp32 values -> planes of T

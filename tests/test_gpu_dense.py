@@ -398,3 +398,35 @@ def test_dense_fp32_weight_gradient_of_values_that_are_not_finite(N, P, K, value
     d, v = dy.double(), x.double()
     _same_class(dw, d.T @ v, d.abs().T @ v.abs(), "dW")
     _same_class(db, d.sum(0), d.abs().sum(0), "db")
+
+
+@pytest.mark.parametrize("kind", ["rows", "few rows", "weight gradient", "weight gradient, few rows"])
+def test_dense_fp32_keeps_the_bits_of_single_products(kind):
+    """16 equal products of operands whose lower pieces are as large as they get (just below 1 + 2^-7; just below and above a
+    half-way point of the pieces).  What the piece products leave out is at most 2^-23 of each product; adding up the kept ones rounds
+    the result a few times more (the last additions: 2^-24 each): 2^-22 in all."""
+    from sparseswin3d_amd import _lib
+    lib = _lib.load()
+    ones = [1 + 2.0 ** -7 - 2.0 ** -15 - 2.0 ** -23, 1 + 2.0 ** -7 - 2.0 ** -23, 1 + 2.0 ** -8 + 2.0 ** -16 + 2.0 ** -23, 1 + 2.0 ** -8 + 2.0 ** -17,
+            1.9999999, 1 + 2.0 ** -8 - 2.0 ** -17 - 2.0 ** -23]
+    worst = 0.0
+    for a in ones:
+        for b in ones:
+            for sign in (1.0, -1.0):
+                ta, tb = torch.tensor(a, dtype=torch.float32), torch.tensor(b, dtype=torch.float32) * sign
+                exact = 16 * ta.double().item() * tb.double().item()
+                if kind in ("rows", "few rows"):
+                    x, w = ta.expand(20000 if kind == "rows" else 64, 16).contiguous().cuda(), tb.expand(112, 16).contiguous().cuda()
+                    y, _ = _forward(lib, _lib, x, w, None, 0, PLAIN, None, torch.float32)
+                else:
+                    N = 2000 if kind == "weight gradient" else 40
+                    d, v = torch.zeros(N, 112), torch.zeros(N, 208)
+                    d[8:24], v[8:24] = ta, tb
+                    d, v, y = d.cuda(), v.cuda(), torch.empty(112, 208, device="cuda")
+                    nb = lib.sswin_dense_weight_grad_workspace_bytes(0, N, 112, 208)
+                    ws = torch.empty(max(nb, 1), dtype=torch.uint8, device="cuda")
+                    _lib.check(lib.sswin_dense_weight_grad(0, 0, _ptr(d), _ptr(v), N, 112, 208, _ptr(y), None, _ptr(ws), nb, _stream()))
+                err = (y.double() - exact).abs().max().item() / abs(exact)
+                worst = max(worst, err)
+                assert err <= 2.0 ** -22, (a, b, sign, err * 2 ** 24)
+    print(f"{kind}: worst error {worst * 2 ** 24:.2f} x 2^-24")
