@@ -324,6 +324,34 @@ def operators_in_module(wl, reps=5):
     return {k: (sum(v) / len(v), len(v) / reps) for k, v in acc.items()}
 
 
+def _ptr(t):
+    return C.c_void_p(t.data_ptr() if t is not None else 0)
+
+
+# the block products of the path with the attention matrix in memory, one launch each
+def _tokens_to_sq(tp, dtype, epilogue, a, a_stride, a_col0, b, b_stride, b_col0, hd, scale, bias, mask, out, rows):
+    from sparseswin3d_amd import _lib
+    _lib.check(_lib.load().sswin_fused_tokens_to_sq(
+        DTYPE_CODE[dtype], 1 if epilogue else 0, _ptr(tp.plan), tp.g_cap, tp.G, _ptr(tp.tokens), tp.N, tp.H, hd,
+        _ptr(a), a_stride, a_col0, _ptr(b), b_stride, b_col0, C.c_float(scale), _ptr(bias), tp.n, _ptr(mask),
+        0 if mask is None else mask.shape[0], _ptr(out), _ptr(rows), _lib.stream_handle(tp.device)))
+
+
+def _sq_to_tokens(tp, dtype, a_kmajor, sq, b, b_stride, b_col0, o, o_stride, o_col0, hd, scale):
+    from sparseswin3d_amd import _lib
+    _lib.check(_lib.load().sswin_fused_sq_to_tokens(
+        DTYPE_CODE[dtype], 1 if a_kmajor else 0, _ptr(tp.plan), tp.g_cap, tp.G, _ptr(tp.tokens), tp.N, tp.H, hd,
+        _ptr(sq), _ptr(b), b_stride, b_col0, _ptr(o), o_stride, o_col0, C.c_float(scale), _lib.stream_handle(tp.device)))
+
+
+def _score_grad(tp, dtype, d_o, do_stride, do_col0, v, v_stride, v_col0, o, o_stride, o_col0, hd, p, ds):
+    """dS = P (dO V^T - D), D_i = dO_i . O_i: the product dP and the softmax backward in one launch."""
+    from sparseswin3d_amd import _lib
+    _lib.check(_lib.load().sswin_fused_score_grad(
+        DTYPE_CODE[dtype], _ptr(tp.plan), tp.g_cap, tp.G, _ptr(tp.tokens), tp.N, tp.H, hd, tp.c_max, _ptr(d_o), do_stride,
+        do_col0, _ptr(v), v_stride, v_col0, _ptr(o), o_stride, o_col0, _ptr(p), _ptr(ds), _lib.stream_handle(tp.device)))
+
+
 def kernel_table(wl, reps=20, only=None):
     """Time every operator's kernels alone on the first block's tensors (regular windows).  The operator
     and fused paths are timed for fp32 tokens only; the window-resident kernels in the workload's dtype."""
@@ -437,7 +465,7 @@ def kernel_table(wl, reps=20, only=None):
             ("bias + mask add, one pass [A]", lambda: ops.group_add_table_bias_mask(s_val, row_pos, gp, b["n"], table_o, ti_o.code, ti_o.offset0, mask), 2 * s * A + 8 * G, 1),
             ("bias + mask add from a gathered [H,n,n] bias", lambda: ops.group_add_bias_mask(s_val, row_pos, gp, b["n"], bias_d, mask), 2 * s * A + 8 * G, 0),
             # what the module's backward calls: with a token plan at hand the batches are dealt from its descriptors
-            ("bias table gradient (batches from the token plan)", lambda: F._bias_gradient(tp, H, g_s, (torch.float32, (n_table_o, H)), ti_o), 4 * A, int(dealt_o)),
+            ("bias table gradient (batches from the token plan)", lambda: F._bias_gradient(tp, g_s, (torch.float32, (n_table_o, H)), ti_o), 4 * A, int(dealt_o)),
             ("bias table gradient from the product's groups", lambda: ops.group_bias_table_grad(g_s, row_pos, gp, H, b["n"], ti_o.code, ti_o.offset0, n_table_o), 4 * A, int(not dealt_o)),
             ("softmax rows from the group sizes [A]", lambda: ops.softmax_rows_from_counts(c, A), 4 * A + 12 * G, 1),
             ("flatten_indices [3,A] (generic softmax rows)", lambda: ops.flatten_indices(s_idx[:3], s_shape[:3]), 16 * A, 0),
@@ -473,16 +501,16 @@ def kernel_table(wl, reps=20, only=None):
         bg_ws = torch.empty(int(bg_bytes), dtype=torch.uint8, device=dev)
         f_entries = [
             ("fused token plan, one of a stage's two", staged_plan, 28 * N + 20 * tp.G, 1),
-            ("fused S=QK^T+bias+mask", lambda: F._tokens_to_sq(tp, dt, True, qkv_c, 3 * D, 0, qkv_c, 3 * D, D, hd, 0.17, bias, mask, s_f, None), 8 * E + 4 * A, 1),
+            ("fused S=QK^T+bias+mask", lambda: _tokens_to_sq(tp, dt, True, qkv_c, 3 * D, 0, qkv_c, 3 * D, D, hd, 0.17, bias, mask, s_f, None), 8 * E + 4 * A, 1),
             ("fused softmax fwd (rows from the group table)", lambda: F._group_softmax(tp, False, s_f, None, p_f), 8 * A, 1),
-            ("fused O=PV", lambda: F._sq_to_tokens(tp, dt, False, p_val, qkv_c, 3 * D, 2 * D, out_f, D, 0, hd, 1.0), 4 * A + 8 * E, 1),
-            ("fused dS=P(dO V^T - dO.O)", lambda: F._score_grad(tp, dt, out_f, D, 0, qkv_c, 3 * D, 2 * D, out_f, D, 0, hd, p_val, s_f), 12 * E + 8 * A, 1),
-            ("fused dP=dO V^T (the product alone)", lambda: F._tokens_to_sq(tp, dt, False, out_f, D, 0, qkv_c, 3 * D, 2 * D, hd, 1.0, None, None, s_f, None), 8 * E + 4 * A, 0),
-            ("fused dV=P^T dO", lambda: F._sq_to_tokens(tp, dt, True, p_val, out_f, D, 0, dqkv, 3 * D, 2 * D, hd, 1.0), 4 * A + 8 * E, 1),
+            ("fused O=PV", lambda: _sq_to_tokens(tp, dt, False, p_val, qkv_c, 3 * D, 2 * D, out_f, D, 0, hd, 1.0), 4 * A + 8 * E, 1),
+            ("fused dS=P(dO V^T - dO.O)", lambda: _score_grad(tp, dt, out_f, D, 0, qkv_c, 3 * D, 2 * D, out_f, D, 0, hd, p_val, s_f), 12 * E + 8 * A, 1),
+            ("fused dP=dO V^T (the product alone)", lambda: _tokens_to_sq(tp, dt, False, out_f, D, 0, qkv_c, 3 * D, 2 * D, hd, 1.0, None, None, s_f, None), 8 * E + 4 * A, 0),
+            ("fused dV=P^T dO", lambda: _sq_to_tokens(tp, dt, True, p_val, out_f, D, 0, dqkv, 3 * D, 2 * D, hd, 1.0), 4 * A + 8 * E, 1),
             ("fused softmax bwd (rows from the group table; alone)", lambda: F._group_softmax(tp, True, p_val, g_s, p_f), 12 * A, 0),
-            ("fused dQ=dS K", lambda: F._sq_to_tokens(tp, dt, False, g_s, qkv_c, 3 * D, D, dqkv, 3 * D, 0, hd, 0.17), 4 * A + 8 * E, 1),
-            ("fused dK=dS^T Q", lambda: F._sq_to_tokens(tp, dt, True, g_s, qkv_c, 3 * D, 0, dqkv, 3 * D, D, hd, 0.17), 4 * A + 8 * E, 1),
-            ("fused bias table grad", lambda: F._bias_gradient(tp, H, g_s, (torch.float32, (n_table, H)), ti), 4 * A, 1),
+            ("fused dQ=dS K", lambda: _sq_to_tokens(tp, dt, False, g_s, qkv_c, 3 * D, D, dqkv, 3 * D, 0, hd, 0.17), 4 * A + 8 * E, 1),
+            ("fused dK=dS^T Q", lambda: _sq_to_tokens(tp, dt, True, g_s, qkv_c, 3 * D, 0, dqkv, 3 * D, D, hd, 0.17), 4 * A + 8 * E, 1),
+            ("fused bias table grad", lambda: F._bias_gradient(tp, g_s, (torch.float32, (n_table, H)), ti), 4 * A, 1),
             ("fused bias grad [H,n,n]", lambda: _lib.check(lib.sswin_fused_bias_grad(ptr(tp.plan), tp.g_cap, tp.G, ptr(tp.tokens), tp.N, H, b["n"], ptr(g_s), ptr(dbias), ptr(bg_ws), bg_bytes, stream)), 4 * A, 0),
         ]
 

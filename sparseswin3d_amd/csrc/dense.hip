@@ -1105,16 +1105,6 @@ __global__ __launch_bounds__(256) void dense_wgrad_sum_kernel(const float* __res
 // ------------------------------------------------------------------------------------------
 // launches
 // ------------------------------------------------------------------------------------------
-static int device_cus() {
-    static int cached = 0;
-    if (!cached) {
-        int dev = 0, n = 0;
-        if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
-        cached = n;
-    }
-    return cached;
-}
-
 template <typename F> static int allow_lds(F* kernel, size_t bytes) {
     if (bytes > 64 * 1024)
         SSWIN_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));

@@ -505,30 +505,31 @@ Tensor attention_forward(Attention& a, const Tensor& qkv, const Tensor& bias, At
     return out;
 }
 
-// gradient of the bias (of the table where positions are coded) from dS, one [c x c] block per group
-Tensor bias_gradient(const Attention& a, const Tensor& d_s, const Tensor& bias) {
-    Plan& tp = *a.plan;
+// gradient of the [H, n, n] bias, or of the [rows, H] table where positions are coded, from dS, one [c x c] block per group
+Tensor bias_gradient(Plan& tp, int H, int n, const Tensor& code, int offset0, const Tensor& d_s, at::IntArrayRef sizes, ScalarType type) {
     void* s = current_stream(d_s);
     Tensor out;
-    if (!a.code.defined()) {
-        out = at::zeros(bias.sizes(), d_s.options());
-        const size_t nb = sswin_fused_bias_grad_workspace_bytes(tp.G, a.H, a.n);
+    if (!code.defined()) {
+        out = at::zeros(sizes, d_s.options());
+        const size_t nb = sswin_fused_bias_grad_workspace_bytes(tp.G, H, n);
         Tensor ws = bytes(nb, d_s);
-        RUN(sswin_fused_bias_grad(i32(tp.plan), tp.g_cap, tp.G, i32(tp.tokens), tp.N, a.H, a.n, f32(d_s), f32(out), ptr(ws), nb, s));
-        return out.to(bias.scalar_type());
+        RUN(sswin_fused_bias_grad(i32(tp.plan), tp.g_cap, tp.G, i32(tp.tokens), tp.N, H, n, f32(d_s), f32(out), ptr(ws), nb, s));
+        return out.to(type);
     }
-    const int rows = (int)bias.size(0);
-    out = at::empty(bias.sizes(), d_s.options());
-    const size_t nb = sswin_bias_table_grad_workspace_bytes(tp.G, a.H, rows);
+    const int rows = (int)sizes[0];
+    out = at::empty(sizes, d_s.options());
+    const size_t nb = sswin_bias_table_grad_workspace_bytes(tp.G, H, rows);
     Tensor ws = bytes(nb, d_s);
-    if (tp.tasks.defined() && a.n <= 128 && tp.buckets[0] + tp.buckets[1] + tp.buckets[2] + tp.buckets[3] == tp.G)
+    if (tp.tasks.defined() && n <= 128 && tp.buckets[0] + tp.buckets[1] + tp.buckets[2] + tp.buckets[3] == tp.G)
         // every group has a task descriptor: the batches of dS are dealt evenly from the descriptor lists
-        RUN(sswin_bias_table_grad_tasks(i32(tp.tasks), tp.g_cap, tp.buckets, tp.G, i32(tp.tokens), tp.N, a.H, a.n, i32(a.code), a.offset0, rows, f32(d_s),
+        RUN(sswin_bias_table_grad_tasks(i32(tp.tasks), tp.g_cap, tp.buckets, tp.G, i32(tp.tokens), tp.N, H, n, i32(code), offset0, rows, f32(d_s),
                                         f32(out), ptr(ws), nb, s));
     else
-        RUN(sswin_bias_table_grad(i32(tp.plan), tp.g_cap, tp.G, i32(tp.tokens), tp.N, a.H, a.n, i32(a.code), a.offset0, rows, f32(d_s), f32(out), ptr(ws),
-                                  nb, s));
-    return out.to(bias.scalar_type());
+        RUN(sswin_bias_table_grad(i32(tp.plan), tp.g_cap, tp.G, i32(tp.tokens), tp.N, H, n, i32(code), offset0, rows, f32(d_s), f32(out), ptr(ws), nb, s));
+    return out.to(type);
+}
+Tensor bias_gradient(const Attention& a, const Tensor& d_s, const Tensor& bias) {
+    return bias_gradient(*a.plan, a.H, a.n, a.code, a.offset0, d_s, bias.sizes(), bias.scalar_type());
 }
 
 Tensor attention_backward(const Attention& a, const Tensor& qkv, const Tensor& bias, const AttentionSaved& saved, const Tensor& out, const Tensor& d_out,
@@ -839,6 +840,20 @@ Tensor merge(const Tensor& x, const Tensor& gamma, const Tensor& beta, const Ten
     return MergeNode::apply(x, gamma, beta, w, plan, eps, type);
 }
 
+// the bias gradient alone: dS of a plan's groups, as the operators' product lays it out
+Tensor plan_bias_gradient(const PlanPtr& plan, const Tensor& d_s, const OptTensor& code, int64_t offset0, const std::vector<int64_t>& sizes, ScalarType type) {
+    plan->finish();
+    c10::hip::HIPGuardMasqueradingAsCUDA guard(d_s.device());
+    const Tensor c = or_undefined(code);
+    TORCH_CHECK(!plan->order_only && d_s.scalar_type() == at::kFloat && d_s.is_contiguous() && d_s.numel() >= plan->A, "bias gradient: dS of ", d_s.sizes(),
+                " for a plan of ", plan->A, " scores");
+    TORCH_CHECK(c.defined() ? sizes.size() == 2 && sizes[1] == plan->H && c.numel() == plan->n && c.scalar_type() == at::kInt && c.is_contiguous()
+                            : sizes == std::vector<int64_t>({plan->H, plan->n, plan->n}),
+                "bias gradient: a bias of ", sizes, " for ", plan->H, " heads and windows of ", plan->n);
+    same_device(d_s, {&c, &plan->tokens});
+    return bias_gradient(*plan, plan->H, (int)plan->n, c, (int)offset0, d_s, sizes, type);
+}
+
 Tensor window_coords(const PlanPtr& plan, const std::vector<int64_t>& dims, const std::vector<int64_t>& window) {
     plan->finish();
     c10::hip::HIPGuardMasqueradingAsCUDA guard(plan->plan.device());
@@ -885,6 +900,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("enqueue_plans", &enqueue_plans);
     m.def("window_indices", &window_indices);
     m.def("window_coords", &window_coords);
+    m.def("bias_gradient", &plan_bias_gradient);
     m.def("attention", &attention);
     m.def("attention_module", &attention_module);
     m.def("block", &block);

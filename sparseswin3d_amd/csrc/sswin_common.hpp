@@ -144,6 +144,15 @@ __device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) {
     return __builtin_bit_cast(uint32_t, pair{(__bf16)lo, (__bf16)hi});
 }
 
+// compute units of the current device (asked once: all devices of a host are of one kind)
+inline int device_cus() {
+    static const int cus = [] {
+        int dev = 0, n = 0;
+        return hipGetDevice(&dev) == hipSuccess && hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0 ? n : 256;
+    }();
+    return cus;
+}
+
 // Zeros by a kernel instead of hipMemsetAsync: callers may capture these entry points into a HIP graph, and memset
 // nodes have given wrong results on replays of a captured graph.
 template <typename T>

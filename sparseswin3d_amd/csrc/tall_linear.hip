@@ -9,8 +9,9 @@
 // up fp32 accuracy: every fp32 operand is split exactly into three bf16 pieces (x = h + m + l, 8 + 8 +
 // 8 significant bits, by truncation and exact subtraction) and a product is the sum of the six
 // piece products whose weight is at least 2^-16 of the leading one (hh, hm, mh, mm, hl, lh), all
-// accumulated in fp32 by v_mfma_f32_32x32x16_bf16.  What is dropped (ml, lm, ll) is below 2^-23 of
-// the product, i.e. at the level of fp32 rounding itself.  Inputs are taken to be finite (the pieces
+// accumulated in fp32 by v_mfma_f32_32x32x16_bf16.  What is dropped (ml, lm, ll) is below 2^-21 of the
+// product (m < 2^-7 and l < 2^-15 of the leading power, with the sign of the value), about 2^-24 of it for operands
+// of evenly spread bits, i.e. at the level of fp32 rounding itself.  Inputs are taken to be finite (the pieces
 // of an infinity are infinity and NaN).
 //
 // Common layout of the row-streaming kernels (forward, input gradient): a workgroup owns one group of
@@ -771,14 +772,6 @@ static int staged_lds_bytes(int ksteps) {
     return ksteps * 9 * 64 * (int)sizeof(tl_u32x4) + 8 * 32 * (ksteps * 16 + 4) * (int)sizeof(float);
 }
 
-static int device_cus() {
-    int dev = 0, n = 0;
-    if (hipGetDevice(&dev) == hipSuccess && hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess &&
-        n > 0)
-        return n;
-    return 256;
-}
-
 namespace sswin {
 namespace dense {
 template <bool TRANSPOSED, int EPI>
@@ -879,13 +872,7 @@ int sswin_tall_linear_forward(const float* x, int64_t N, int K, const float* w, 
     SSWIN_CHECK(((uintptr_t)x % 16) == 0 && ((uintptr_t)w % 16) == 0, "tall_linear_forward: x and w must be 16-byte aligned");
     hipStream_t s = static_cast<hipStream_t>(stream);
     const int groups = P / TL_COLS, ksteps = K / 16;
-    int cus = 256;
-    {
-        int dev = 0, n = 0;
-        if (hipGetDevice(&dev) == hipSuccess &&
-            hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0)
-            cus = n;
-    }
+    const int cus = device_cus();
     static bool configured = false;
     if (!configured) {
         const int max_lds = TL_MAX_K / 16 * 9 * 64 * (int)sizeof(tl_u32x4);

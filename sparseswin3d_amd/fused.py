@@ -1,5 +1,5 @@
-"""Fused window attention: one autograd Function around the token-plan and the fused MFMA
-block products of ``libsswin3d.so``.
+"""Fused window attention: token plans and the call into the compiled host path (``csrc/native.cpp``), which runs the
+attention, or the attention with the two dense layers around it, as one autograd node.
 
 Numerically this is the same computation as the operator-by-operator composition in
 :mod:`sparseswin3d_amd.window_attention` (reference ``sparse_swin/swin3d_base.py:654-675``):
@@ -8,8 +8,8 @@ Numerically this is the same computation as the operator-by-operator composition
 
 but Q, K, V token rows are read straight from the dense ``qkv`` tensor through the token order
 and the output is written straight into voxel order, so the sorted COO copies, the bias/mask
-gather passes, the permute and the un-sort never exist.  The attention values S and P are still
-materialised in HBM (P is needed by the backward pass).
+gather passes, the permute and the un-sort never exist.  Three families of kernels (:func:`attention_path`): two keep the
+attention matrix in registers and form it again in the backward pass, the block products keep P in memory.
 """
 from __future__ import annotations
 
@@ -18,7 +18,6 @@ import ctypes as C
 import torch
 
 from . import _lib
-from . import custom_ops as ops
 
 _DTYPE_CODE = {torch.float32: 0, torch.float16: 1, torch.bfloat16: 2}
 
@@ -30,10 +29,10 @@ def _ptr(t):
 class TokenPlan:
     """Token order and per-group table of one set of (window, pos) voxel indices.
 
-    With ``defer=True`` the constructor only enqueues the kernels and the copy of the totals;
+    With ``defer=True`` the constructor only enqueues the kernels, the last of which writes the totals to pinned memory;
     work enqueued afterwards (the qkv projection) overlaps the host round trip, and
     :meth:`finish` waits for the totals when they are needed.  :meth:`finish` raises if an index
-    lies outside ``[0, batch_size) x [0, n)`` or a (window, pos) pair occurs twice.
+    lies outside ``[0, batch_size) x [0, n)`` or a (window, pos) pair occurs twice, and so does every later use of the plan.
 
     ``tokens``, ``plan`` and ``tasks`` are the device tables of ``sswin_token_plan``; ``tasks``: group descriptors of the
     window-resident kernels, bucketed by ceil(c / 32), and behind them the token records, one per window and tile of 32
@@ -80,30 +79,6 @@ for _name in ("tokens", "plan", "tasks", "device", "N", "H", "n", "B", "g_cap", 
     setattr(TokenPlan, _name, property(lambda self, _name=_name: getattr(self.native, _name)))
 
 
-def _tokens_to_sq(tp, dtype, epilogue, a, a_stride, a_col0, b, b_stride, b_col0, hd, scale, bias, mask, out, rows):
-    lib = _lib.load()
-    stream = _lib.stream_handle(tp.device)
-    _lib.check(lib.sswin_fused_tokens_to_sq(
-        _DTYPE_CODE[dtype], 1 if epilogue else 0, _ptr(tp.plan), tp.g_cap, tp.G, _ptr(tp.tokens), tp.N, tp.H, hd,
-        _ptr(a), a_stride, a_col0, _ptr(b), b_stride, b_col0, C.c_float(scale), _ptr(bias), tp.n, _ptr(mask),
-        0 if mask is None else mask.shape[0], _ptr(out), _ptr(rows), stream))
-
-
-def _sq_to_tokens(tp, dtype, a_kmajor, sq, b, b_stride, b_col0, o, o_stride, o_col0, hd, scale):
-    lib = _lib.load()
-    stream = _lib.stream_handle(tp.device)
-    _lib.check(lib.sswin_fused_sq_to_tokens(
-        _DTYPE_CODE[dtype], 1 if a_kmajor else 0, _ptr(tp.plan), tp.g_cap, tp.G, _ptr(tp.tokens), tp.N, tp.H, hd,
-        _ptr(sq), _ptr(b), b_stride, b_col0, _ptr(o), o_stride, o_col0, C.c_float(scale), stream))
-
-
-def _score_grad(tp, dtype, d_o, do_stride, do_col0, v, v_stride, v_col0, o, o_stride, o_col0, hd, p, ds):
-    """dS = P (dO V^T - D), D_i = dO_i . O_i: the product dP and the softmax backward in one launch."""
-    _lib.check(_lib.load().sswin_fused_score_grad(
-        _DTYPE_CODE[dtype], _ptr(tp.plan), tp.g_cap, tp.G, _ptr(tp.tokens), tp.N, tp.H, hd, tp.c_max, _ptr(d_o), do_stride,
-        do_col0, _ptr(v), v_stride, v_col0, _ptr(o), o_stride, o_col0, _ptr(p), _ptr(ds), _lib.stream_handle(tp.device)))
-
-
 def _group_softmax(tp, backward, x_or_y, grad, out):
     """Row softmax (or its backward) over the [c x c] blocks of the plan's groups; ``out`` may be one of the inputs."""
     _lib.check(_lib.load().sswin_group_softmax(
@@ -111,34 +86,12 @@ def _group_softmax(tp, backward, x_or_y, grad, out):
         _lib.stream_handle(tp.device)))
 
 
-def _bias_gradient(tp, H, d_s, bias_meta, table_index):
+def _bias_gradient(tp, d_s, bias_meta, table_index):
     """Gradient of the [H, n, n] bias, or of the [rows, H] table when ``table_index`` is given, from dS
     (one [c x c] block per group)."""
-    lib = _lib.load()
-    d = d_s.device
-    bias_dtype, bias_shape = bias_meta
-    stream = _lib.stream_handle(d)
-    if table_index is None:
-        d_bias32 = torch.zeros(bias_shape, dtype=torch.float32, device=d)
-        nbytes = lib.sswin_fused_bias_grad_workspace_bytes(tp.G, H, tp.n)
-        ws = torch.empty(int(nbytes), dtype=torch.uint8, device=d)
-        _lib.check(lib.sswin_fused_bias_grad(_ptr(tp.plan), tp.g_cap, tp.G, _ptr(tp.tokens), tp.N, H, tp.n,
-                                             _ptr(d_s), _ptr(d_bias32), _ptr(ws), nbytes, stream))
-    else:
-        rows = bias_shape[0]
-        d_bias32 = torch.empty(bias_shape, dtype=torch.float32, device=d)
-        nbytes = lib.sswin_bias_table_grad_workspace_bytes(tp.G, H, rows)
-        ws = torch.empty(int(nbytes), dtype=torch.uint8, device=d)
-        if tp.tasks is not None and tp.n <= 128 and sum(tp.bucket_counts) == tp.G:
-            # every group has a task descriptor: the batches of dS are dealt evenly from the descriptor lists
-            _lib.check(lib.sswin_bias_table_grad_tasks(_ptr(tp.tasks), tp.g_cap, tp.bucket_counts, tp.G, _ptr(tp.tokens), tp.N,
-                                                       H, tp.n, _ptr(table_index.code), table_index.offset0, rows,
-                                                       _ptr(d_s), _ptr(d_bias32), _ptr(ws), nbytes, stream))
-        else:
-            _lib.check(lib.sswin_bias_table_grad(_ptr(tp.plan), tp.g_cap, tp.G, _ptr(tp.tokens), tp.N, H, tp.n,
-                                                 _ptr(table_index.code), table_index.offset0, rows, _ptr(d_s),
-                                                 _ptr(d_bias32), _ptr(ws), nbytes, stream))
-    return d_bias32.to(bias_dtype)
+    dtype, shape = bias_meta
+    code, offset0 = (None, 0) if table_index is None else (table_index.code, table_index.offset0)
+    return _lib.native().bias_gradient(tp.native, d_s, code, offset0, list(shape), dtype)
 
 
 class BiasTableIndex:
@@ -199,10 +152,6 @@ def attention_path(head_dim: int, n: int, table_index, resident=None) -> str:
     if resident is None and head_dim in (16, 32) and table_index is not None and table_index.ascending:
         return "flash"
     return "products"
-
-
-def supports_resident(qkv: torch.Tensor, n: int) -> bool:
-    return supports(qkv, n) and qkv.shape[-1] == 32 and n <= 128
 
 
 def supports(qkv: torch.Tensor, n: int, table: bool = False) -> bool:

@@ -433,8 +433,7 @@ class _GroupBiasMask(Function):
             if tp is not None and tp.H == num_heads and tp.A == grad.numel():
                 # the values of the product lie in the plan's group order: the fused path's table gradient applies
                 # as it is (batches dealt from the task descriptors where every window has one)
-                d_table = fused._bias_gradient(tp, num_heads, grad.float().contiguous(), (table_dtype, (table_rows, num_heads)),
-                                               table_index)
+                d_table = fused._bias_gradient(tp, grad.float().contiguous(), (table_dtype, (table_rows, num_heads)), table_index)
             else:
                 d_table = ops.group_bias_table_grad(grad.float(), idx, gp, num_heads, n, table_index.code,
                                                     table_index.offset0, table_rows).to(table_dtype)
