@@ -257,3 +257,49 @@ def test_attention_refuses_masks_and_plans_it_cannot_read():
     small = BiasTableIndex.build(relative_position_index_3d((4, 4, 4)).cuda(), 343)
     with pytest.raises(RuntimeError, match="position codes"):
         fused_window_attention(qkv, table, ind, None, 40, 125, 0.2, table_index=small)
+
+
+@pytest.mark.parametrize("dim,heads,window,mode", [(96, 3, 5, "fp32"), (48, 3, 7, "fp32"), (48, 3, 7, "amp"), (192, 6, 5, "bf16")])
+def test_nodes_on_other_streams(dim, heads, window, mode):
+    """A stage with its merge on a stream of its own, and on two streams at once from two threads: the bits of the default stream
+    (sums are added in a fixed order everywhere)."""
+    import threading
+    layer, run, feats = _stage_pieces(dim, heads, window, torch.bfloat16 if mode == "bf16" else torch.float32, True, 11)
+    up = torch.randn(4096, 2 * dim, device="cuda")
+
+    def once(x):
+        with torch.autocast("cuda", dtype=torch.float16, enabled=mode == "amp"):
+            y = run(x)
+        grads = torch.autograd.grad(y, [x, *layer.parameters()], up[:y.shape[0]].to(y.dtype))
+        with torch.no_grad(), torch.autocast("cuda", dtype=torch.float16, enabled=mode == "amp"):
+            return [y.detach(), run(x), *grads]
+
+    want = once(feats.clone().requires_grad_(True))
+    torch.cuda.synchronize()
+    results, errors = {}, []
+
+    def work(k, gate=None):
+        try:
+            stream = torch.cuda.Stream()
+            stream.wait_stream(torch.cuda.default_stream())
+            with torch.cuda.stream(stream):
+                x = feats.clone().requires_grad_(True)
+                if gate is not None:
+                    gate.wait()
+                for r in range(3):
+                    results[k, r] = once(x)
+            stream.synchronize()
+        except Exception as e:                                    # noqa: BLE001  (told to the main thread)
+            errors.append(e)
+
+    work(0)
+    gate = threading.Barrier(2)
+    threads = [threading.Thread(target=work, args=(k, gate)) for k in (1, 2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors, errors
+    assert len(results) == 9
+    for got in results.values():
+        assert all(torch.equal(a, b) for a, b in zip(got, want))
