@@ -593,6 +593,35 @@ def kernel_table(wl, reps=20, only=None):
     if not resident_ok:
         r_entries = r_entries[:2]
 
+    # ---- the flash kernels (what the step runs for heads of 16, and for heads of 32 in windows of more than 128 positions) ----
+    fl_entries = []
+    if ti is not None and F.attention_path(hd, b["n"], ti) == "flash":
+        words = torch.empty(2 * N, dtype=torch.int32, device=dev)
+        table_fl = wl["blocks"][0]["attn"].relative_position_bias_table.detach().float().contiguous()
+        delta = torch.empty(H * N, device=dev)
+
+        def fl_tokens():
+            _lib.check(lib.sswin_flash_tokens(ptr(tp.plan), tp.g_cap, tp.G, ptr(tp.tokens), N, H, b["n"], ptr(ti.code), mask_p, nmw, ptr(words),
+                                              C.c_void_p(words.data_ptr() + 4 * N), stream))
+
+        def fl_fwd():
+            _lib.check(lib.sswin_flash_forward(code, ptr(tp.tokens), ptr(words), N, H, hd, b["n"], ptr(qkv_r), C.c_float(0.17), ptr(table_fl), n_table,
+                                               ti.offset0, ptr(out_r), ptr(lse), stream))
+
+        def fl_bwd():
+            _lib.check(lib.sswin_flash_backward(code, ptr(tp.tokens), ptr(words), C.c_void_p(words.data_ptr() + 4 * N), N, H, hd, b["n"], ptr(qkv_r),
+                                                C.c_float(0.17), ptr(table_fl), n_table, ti.offset0, ptr(out_r), ptr(lse), ptr(up_r), ptr(dqkv_r),
+                                                ptr(delta), ptr(ds_r), stream))
+
+        fl_tokens()
+        fl_fwd()                                  # lse and out_r must hold a real forward for the backward timings
+        fl_entries = [
+            ("flash token words", fl_tokens, 28 * N, 1),
+            ("flash forward", fl_fwd, 16 * Er + 4 * H * N, 1, 4 * A * hd),
+            ("flash backward (dQ,dK,dV,dS; two launches)", fl_bwd, 32 * Er + 4 * A + 4 * H * N, 1, 10 * A * hd),
+            ("flash bias table grad", r_table_grad, 4 * A, 1),
+        ]
+
     def measure(items, path):
         rows_ = []
         for name, fn, nbytes, calls, *flops in items:
@@ -609,7 +638,7 @@ def kernel_table(wl, reps=20, only=None):
         src = torch.empty(CALIBRATION_BYTES // 4, dtype=torch.float32, device=dev).normal_()
         dst = torch.empty_like(src)
         names = [o for o in only.split(",") if o]
-        picked = [e for e in r_entries + f_entries + entries + (projection_entries(wl) if code == 0 else [])
+        picked = [e for e in r_entries + fl_entries + f_entries + entries + (projection_entries(wl) if code == 0 else [])
                   if any(o in e[0] for o in names)]
         for name, fn, nbytes, calls, *_ in picked:
             log(f"profiling {name}: {reps} launches, algorithmic bytes {nbytes}")
@@ -620,7 +649,7 @@ def kernel_table(wl, reps=20, only=None):
         torch.cuda.synchronize()
         log(f"calibration copy: {reps} launches of {CALIBRATION_BYTES} bytes read and written")
         return [], sizes
-    table = measure(r_entries, "resident")
+    table = measure(r_entries, "resident") + measure(fl_entries, "flash")
     if code == 0:
         op_rows = measure(entries, "operators")
         # the same launches inside a module call: what the path's summary is made of
@@ -650,6 +679,7 @@ def module_times(wl, reps=10):
     from sparseswin3d_amd.window_attention import SparseVoxelTensor
     if wl["dtype"] != torch.float32:
         return {}
+    from sparseswin3d_amd.fused import attention_path
     b = wl["blocks"][0]
     attn = b["attn"]
     keep = (attn.fused, attn.resident)
@@ -662,9 +692,11 @@ def module_times(wl, reps=10):
 
     out = {}
     hd = wl["dim"] // wl["heads"]
-    for name, fused_, resident in (("resident", True, True), ("fused", True, False), ("operators", False, None)):
+    for name, fused_, resident in (("resident", True, True), ("flash", True, None), ("fused", True, False), ("operators", False, None)):
         if name == "resident" and (hd != 32 or b["stats"]["c_max"] > 128):
             continue                                          # the resident kernels do not take this shape
+        if name == "flash" and attention_path(hd, b["n"], attn._table_index(b["n"])) != "flash":
+            continue
         attn.fused, attn.resident = fused_, resident
         out[name] = round(event_time_ms(once, reps), 4)
     attn.fused, attn.resident = keep
@@ -1001,7 +1033,7 @@ def main():
     # library call (a few extra steps after the timed region, so the events do not perturb `value`)
     from sparseswin3d_amd import _lib
     _lib.launch_timer = []
-    _lib.launch_timer_only = {"sswin_window_attention_forward", "sswin_window_attention_backward"}
+    _lib.launch_timer_only = {"sswin_window_attention_forward", "sswin_window_attention_backward", "sswin_flash_forward", "sswin_flash_backward"}
     for _ in range(max(3, min(10, args.steps))):
         run_step(wl)
     torch.cuda.synchronize()
@@ -1023,7 +1055,7 @@ def main():
         titles = {"stage": "-- index glue of one stage (window indices, mask, stride-2 merge) --",
                   "projections": "-- qkv and proj layers of one attention call (dense [N, C] GEMMs) --"}
         scope = {"stage": "once per stage", "projections": "one attention fwd+bwd"}
-        for path in ("resident", "fused", "operators", "stage", "projections"):
+        for path in ("resident", "flash", "fused", "operators", "stage", "projections"):
             rows_ = [r for r in table if r["path"] == path]
             if not rows_:
                 continue
@@ -1045,15 +1077,15 @@ def main():
                                      frac_alone=round(alg / alone / 1e6 / HBM_PEAK_GBPS, 4))
             log(f"{path} kernels, {scope.get(path, 'one attention fwd+bwd')}: {ms_:.3f} ms for {alg / 1e6:.1f} MB algorithmic "
                 f"= {alg / ms_ / 1e6:.1f} GB/s = {100 * alg / ms_ / 1e6 / HBM_PEAK_GBPS:.2f}% of HBM peak")
-        # the step runs the window-resident path: its slowest kernel is the dominant one
+        # the slowest kernel of the path the step runs is the dominant one
         # (the token plan is a sequence of small launches, not a kernel)
-        # the path the step runs (the module's own choice): resident where its kernels apply, else fused
-        run_path = "resident" if any(r["kernel"] == "resident forward" for r in table) else "fused"
+        # the path the step runs (the module's own choice): resident where its kernels apply, else flash, else fused
+        run_path = next((p for p in ("resident", "flash") if any(r["kernel"] == f"{p} forward" for r in table)), "fused")
         dom = max((r for r in table if r["path"] == run_path and "token plan" not in r["kernel"] and "token_plan" not in r["kernel"]),
                   key=lambda r: r.get("ms_in_module", r["ms"]) * r["calls"])
         # its duration inside the step (events above) is what the roofline entry uses; the same
         # launch repeated back to back on its own (the table) runs 10-20 % slower
-        step_ms = in_step.get("window_attention_backward") if "backward (dQ,dK,dV,dS)" in dom["kernel"] else None
+        step_ms = in_step.get("flash_backward" if run_path == "flash" else "window_attention_backward") if "backward (dQ,dK,dV,dS" in dom["kernel"] else None
         ms = step_ms or dom.get("ms_in_module") or dom["ms"]
         gbps = dom["algorithmic_bytes"] / ms / 1e6
         traffic, traffic_note = measured_traffic(wl["name"], dom["kernel"])
