@@ -441,12 +441,13 @@ class SwinTransformerBlock(nn.Module):
         if type(self) is not SwinTransformerBlock or not self.__dict__.keys().isdisjoint(_BLOCK_PARTS):
             return None
         parts = self._modules
-        attn, mlp, norm1, norm2, f = parts["attn"], parts["mlp"], parts["norm1"], parts["norm2"], x.features
+        attn, mlp, norm1, norm2, f = parts.get("attn"), parts.get("mlp"), parts.get("norm1"), parts.get("norm2"), x.features
         if type(mlp) is not MLP or type(attn) is not WindowAttentionSparse:
             return None
         a, m = attn._modules, mlp._modules
-        qkv, proj, linear1, linear2, gelu = a["qkv"], a["proj"], m["linear1"], m["linear2"], m["fn"]
-        drops = m["drop1"], m["drop2"], a["proj_drop"], parts["drop_path"]
+        # what is no module (a function as activation) is not among them
+        qkv, proj, linear1, linear2, gelu = a.get("qkv"), a.get("proj"), m.get("linear1"), m.get("linear2"), m.get("fn")
+        drops = m.get("drop1"), m.get("drop2"), a.get("proj_drop"), parts.get("drop_path")
         if not all(map(_passes, drops)) or type(gelu) is not nn.GELU or gelu.approximate != "none" or \
                 not _plain(norm1, norm2, qkv, proj, linear1, linear2, gelu) or not unhooked(attn, mlp, *drops):
             return None

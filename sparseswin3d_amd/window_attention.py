@@ -701,7 +701,8 @@ def unhooked(*modules) -> bool:
 
 def param(module, name):
     """``getattr(module, name)`` of a parameter, without nn.Module's attribute access where it is registered as one."""
-    p = module._parameters.get(name)
+    registered = getattr(module, "_parameters", None)
+    p = registered.get(name) if registered else None
     return p if p is not None else getattr(module, name)
 
 

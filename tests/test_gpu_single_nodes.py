@@ -303,3 +303,23 @@ def test_nodes_on_other_streams(dim, heads, window, mode):
     assert len(results) == 9
     for got in results.values():
         assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+def test_functions_in_place_of_modules_run():
+    """An activation given as a function, a norm that is a function: parts of a block that are no modules."""
+    from sparseswin3d_amd.layers import MLP
+    layer, run, feats = _stage_pieces(96, 3, 5, torch.float32, False, 5)
+    plain = run(feats)
+    blk = layer.blocks[0]
+    mlp = MLP(96, 384, act=torch.nn.functional.gelu).cuda()
+    mlp.load_state_dict(blk.mlp.state_dict())
+    blk.mlp = mlp
+    assert torch.allclose(run(feats), plain, rtol=1e-4, atol=1e-5)
+    norm = blk.norm1
+    del blk.norm1
+    blk.norm1 = lambda x: torch.nn.functional.layer_norm(x, (96,), norm.weight, norm.bias, norm.eps)
+    assert torch.allclose(run(feats), plain, rtol=1e-4, atol=1e-5)
+    norm2, blk2 = layer.blocks[1].norm2, layer.blocks[1]
+    del blk2.norm2
+    blk2.norm2 = lambda x: torch.nn.functional.layer_norm(x, (96,), norm2.weight, norm2.bias, norm2.eps)
+    assert torch.allclose(run(feats), plain, rtol=1e-4, atol=1e-5)
