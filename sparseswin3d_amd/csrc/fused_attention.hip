@@ -1178,8 +1178,10 @@ constexpr int RPBT_U = 16;                                      // steps of a ba
 // slot is never copied: a copy would wait for its loads).
 //
 // Which batches a wavefront adds (BY_TASKS):
-//   false: from the group table.  A slice of wavefronts takes every wslices-th window and deals the batches of its
-//          windows among its rsplit members (each member walks over all windows of the slice).
+//   false: from the group table, in plan order, cut into runs of equal cost (run_cut): a row of dS of a window of c tokens
+//          counts c + 16, so the start of window k is known from the prefix sums the table holds, and every wavefront finds
+//          its first and last row by itself.  (Dealing every 85th window to eight wavefronts instead, the fullest held
+//          twice the mean: windows of 7^3, 112 700 voxels 51.2 us, 219 000 voxels 78.5; in runs 39.9 and 69.2.)
 //   true:  from the task descriptors of a token plan, which list the groups by their number of 32-token tiles
 //          (fused TokenPlan, windows of at most 128 tokens).  The batches of a head, numbered bucket by bucket (16, 9,
 //          4 or 1 per group), are cut into Q runs of equal length, one per wavefront of the head (consecutive
@@ -1194,12 +1196,35 @@ struct BatchList {
     int total;               // batches of a head
 };
 
+// Cost of the rows in front of window k, and the row (of a multiple of eight in its window) at which a cost is reached: lanes
+// look at 64 windows at a time, each round leaves the windows between two of them (10 000 windows: three rounds).
+constexpr int RUN_ROW = 16;
+__device__ __forceinline__ int64_t run_start(const FusedGroups& gt, int64_t k, int H) {
+    return gt.sq[k * H] / H + (int64_t)gt.T[k * H] * RUN_ROW;
+}
+struct RunCut {
+    int window, row;
+};
+__device__ __forceinline__ RunCut run_cut(const FusedGroups& gt, int64_t windows, int H, int64_t cost) {
+    int64_t lo = 0, count = windows;                            // the window lies in [lo, lo + count)
+    while (count > 1) {
+        const int64_t step = (count + 63) / 64, k = lo + (threadIdx.x & 63) * step;
+        const int in_front = __popcll(__ballot(k < lo + count && run_start(gt, k, H) <= cost));   // the first of them always is
+        const int64_t end = lo + count;
+        lo += (in_front - 1) * step;
+        count = min(step, end - lo);
+    }
+    const int c = gt.c[lo * H];
+    const int64_t row = (cost - run_start(gt, lo, H)) / (c + RUN_ROW);
+    return {__builtin_amdgcn_readfirstlane((int)lo), __builtin_amdgcn_readfirstlane(row >= c ? c : (int)row & ~7)};
+}
+
 template <bool BY_TASKS>
 __global__ __launch_bounds__(256) void rpb_table_partial_kernel(FusedGroups gt, BatchList bl, const int32_t* __restrict__ tok_pos,
                                                                 int H, const int32_t* __restrict__ code, int n,
                                                                 int offset0, int rows, int rows_pad,
                                                                 const float* __restrict__ ds, int64_t windows,
-                                                                int wslices, int rsplit, float* __restrict__ partial) {
+                                                                int slices, float* __restrict__ partial) {
     extern __shared__ __attribute__((aligned(16))) float rpbt_lds[];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int half = lane >> 5, l32 = lane & 31;
@@ -1207,23 +1232,24 @@ __global__ __launch_bounds__(256) void rpb_table_partial_kernel(FusedGroups gt, 
     for (int e = threadIdx.x; e < n; e += 256) code_lds[e] = code[e];
     __syncthreads();
     const int64_t p = (int64_t)blockIdx.x * 4 + wave;           // wavefront id = h * slices + sl
-    const int slices = wslices * rsplit;                        // a multiple of four: the wavefronts of a workgroup share a head
-    if (p >= (int64_t)slices * H) return;                       // (the whole workgroup then)
+    if (p >= (int64_t)slices * H) return;                       // slices: a multiple of four, the wavefronts of a workgroup share a head
     const int h = (int)(p / slices);
     const int64_t sl = p % slices;
-    const int64_t ws = sl % wslices;                            // windows ws, ws + wslices, ...
-    const int rs = (int)(sl / wslices);                         // which of the rsplit wavefronts of this window slice
     float* tables = rpbt_lds + wave * 2 * rows_pad;
     float* mine = tables + half * rows_pad;
     for (int e = l32; e < rows; e += 32) mine[e] = 0.f;
 
-    // A slice takes every wslices-th window (crowded windows are neighbours in plan order, so dealing them out
-    // evens the load); the batches of its windows are dealt to the rsplit wavefronts of the slice.
-    // The headers of 64 windows of the slice at a time sit in the lanes (lane l: the l-th of them).
-    int hw_c = 0, hw_T = 0, hw_sq = 0, hw_ch = 0, hw_ib = 0;
+    // The headers of 64 windows (BY_TASKS: batches) of the run at a time sit in the lanes.
+    int hw_c = 0, hw_T = 0, hw_sq = 0, hw_ch = 0, hw_ib = 0, hw_end = 0;
     const int per_wave = BY_TASKS ? (bl.total + slices - 1) / slices : 0;   // a wavefront's run of consecutive batches
+    RunCut from = {0, 0}, to = {0, 0};                          // its run of rows
+    if constexpr (!BY_TASKS) {
+        const int64_t g = (windows - 1) * H, c = gt.c[g], total = run_start(gt, windows - 1, H) + c * (c + RUN_ROW);
+        from = run_cut(gt, windows, H, total * sl / slices);
+        to = run_cut(gt, windows, H, total * (sl + 1) / slices);
+    }
     auto load_headers = [&](int m_first) __attribute__((always_inline)) {
-        hw_c = 0;
+        hw_c = hw_end = hw_ib = 0;
         if constexpr (BY_TASKS) {
             // batch number sl * per_wave + m_first + lane of head h -> bucket, group inside it, chunk and row block
             const int64_t f64 = sl * per_wave + m_first + lane;
@@ -1240,83 +1266,58 @@ __global__ __launch_bounds__(256) void rpb_table_partial_kernel(FusedGroups gt, 
                 hw_c = d.y & 0xff;
                 hw_sq = d.w;
                 hw_ib = (rem / nb) * 32;
+                hw_end = hw_c;
                 hw_ch = rem - (rem / nb) * nb;
             }
         } else {
-            const int64_t k = ws + ((int64_t)m_first + lane) * wslices;
-            if (k < windows) {
+            const int64_t k = from.window + m_first + lane;
+            if (k < windows && k <= to.window) {
                 const int64_t g = k * H + h;
                 hw_c = gt.c[g];
                 hw_T = gt.T[g];
                 hw_sq = gt.sq[g];
+                hw_ib = k == from.window ? from.row : 0;        // rows [hw_ib, hw_end)
+                hw_end = k == to.window ? min(to.row, hw_c) : hw_c;
             }
         }
     };
     constexpr int BR = 2 * RPBT_U;                              // rows of a batch
     struct Cursor {
-        int m, m0, rot, c, T, sq, ch, ib;
+        int m, m0, c, T, sq, ch, ib, end;
         bool valid;
     };
-    // The batches of a window, numbered chunk by chunk inside a block of BR rows, then block by block, are dealt to
-    // the rsplit wavefronts of the slice: this one takes the numbers rot, rot + rsplit, ...; rot moves on by one
-    // with every window.  A count of chunks beyond the window's chunks carries into the row blocks.
-    auto carry = [&](Cursor cur) __attribute__((always_inline)) -> Cursor {
-        const int nch = (cur.c + 31) >> 5;
-        if (nch <= 1) {
-            cur.ib += BR * cur.ch;
-            cur.ch = 0;
-        } else {
-            while (cur.ch >= nch) {
-                cur.ch -= nch;
-                cur.ib += BR;
-            }
-        }
-        return cur;
-    };
-    // first batch of window cur.m and after among the 64 windows whose headers are loaded, or none.  (Loading
-    // headers here, inside the pipeline, would put a wait for all loads in flight on every path.)
+    // first batch of window cur.m and after among the 64 windows whose headers are loaded, or none: a batch nobody adds, at a
+    // safe address.  (Loading headers here, inside the pipeline, would put a wait for all loads in flight on every path.)
     auto seek = [&](Cursor cur) __attribute__((always_inline)) -> Cursor {
-        if constexpr (BY_TASKS) {
-            // the batch of lane cur.m - cur.m0, or none (a lane without a batch holds c = 0)
+        for (;; ++cur.m) {
             const int at = cur.m - cur.m0;
-            const int c_at = at < 64 ? __builtin_amdgcn_readlane(hw_c, at & 63) : 0;
-            if (c_at == 0) return Cursor{cur.m, cur.m0, 0, 1, 0, 0, 0, 0, false};
-            return Cursor{cur.m, cur.m0, 0, c_at, __builtin_amdgcn_readlane(hw_T, at & 63), __builtin_amdgcn_readlane(hw_sq, at & 63),
-                          __builtin_amdgcn_readlane(hw_ch, at & 63), __builtin_amdgcn_readlane(hw_ib, at & 63), true};
-        }
-        for (;;) {
-            if (cur.m - cur.m0 == 64)                           // a batch nobody adds, at a safe address
-                return Cursor{cur.m, cur.m0, cur.rot, 1, 0, 0, 0, 0, false};
-            cur.c = __builtin_amdgcn_readlane(hw_c, cur.m - cur.m0);
-            cur.ch = cur.rot;
-            cur.ib = 0;
-            cur = carry(cur);
-            if (cur.ib < cur.c) {
-                cur.T = __builtin_amdgcn_readlane(hw_T, cur.m - cur.m0);
-                cur.sq = __builtin_amdgcn_readlane(hw_sq, cur.m - cur.m0);
-                return cur;
-            }
-            ++cur.m;
-            cur.rot = cur.rot + 1 == rsplit ? 0 : cur.rot + 1;
+            cur.c = at < 64 ? __builtin_amdgcn_readlane(hw_c, at & 63) : 0;
+            if (cur.c == 0) return Cursor{cur.m, cur.m0, 1, 0, 0, 0, 0, 1, false};   // behind the last header
+            cur.ib = __builtin_amdgcn_readlane(hw_ib, at);
+            cur.end = __builtin_amdgcn_readlane(hw_end, at);
+            if (!BY_TASKS && cur.ib >= cur.end) continue;       // none of the window's rows are in the run
+            cur.ch = BY_TASKS ? __builtin_amdgcn_readlane(hw_ch, at) : 0;
+            cur.T = __builtin_amdgcn_readlane(hw_T, at);
+            cur.sq = __builtin_amdgcn_readlane(hw_sq, at);
+            return cur;
         }
     };
+    // chunk by chunk inside a block of BR rows, then block by block
     auto advance = [&](Cursor cur) __attribute__((always_inline)) -> Cursor {
         if (!cur.valid) return cur;
-        if constexpr (BY_TASKS) {
-            ++cur.m;
-            return seek(cur);
+        if constexpr (!BY_TASKS) {
+            if (++cur.ch * 32 < cur.c) return cur;
+            cur.ch = 0;
+            cur.ib += BR;
+            if (cur.ib < cur.end) return cur;
         }
-        cur.ch += rsplit;
-        cur = carry(cur);
-        if (cur.ib < cur.c) return cur;
         ++cur.m;
-        cur.rot = cur.rot + 1 == rsplit ? 0 : cur.rot + 1;
         return seek(cur);
     };
     struct Slot {
         float v[RPBT_U];
         int pj, pi;         // positions of this lane's column and of row ib + 2 (lane & 15) + half
-        int c, ch, ib;
+        int c, ch, ib, end;
         bool valid;
     };
     const uint32_t table_off = (uint32_t)((wave * 2 + half) * rows_pad) * 4u;   // byte offset of this half's table
@@ -1328,6 +1329,7 @@ __global__ __launch_bounds__(256) void rpb_table_partial_kernel(FusedGroups gt, 
         s.c = cur.c;
         s.ch = cur.ch;
         s.ib = cur.ib;
+        s.end = cur.end;
         const uint32_t j = (uint32_t)(cur.ch * 32 + l32);
         const uint32_t jc = j < c ? j : 0u;
         const float* src = ds + cur.sq;
@@ -1348,14 +1350,13 @@ __global__ __launch_bounds__(256) void rpb_table_partial_kernel(FusedGroups gt, 
     // of them) hands every lane the code of its half's row.  Dead rows and columns carry codes that put the byte
     // offset beyond the table, as a table row below zero does: those entries land in a spare row, without a branch.
     auto consume = [&](const Slot& s) __attribute__((always_inline)) {
-        const int c = s.c;
-        const bool jlive = s.ch * 32 + l32 < c;
-        const bool rlive = s.ib + 2 * (lane & 15) + half < c;
+        const bool jlive = s.ch * 32 + l32 < s.c;
+        const bool rlive = s.ib + 2 * (lane & 15) + half < s.end;
         const int cjb = jlive ? (code_lds[s.pj] - offset0) * 4 : -(1 << 30);
         const int crow4 = rlive ? code_lds[s.pi] * 4 : (1 << 30);
         static_steps<0, RPBT_U>([&](auto uc) __attribute__((always_inline)) {
             constexpr int u = decltype(uc)::value;
-            if (s.ib + 2 * u >= c) return false;
+            if (s.ib + 2 * u >= s.end) return false;
             const int ci4 = __builtin_amdgcn_update_dpp(0, crow4, 0x150 + u, 0xf, 0xf, false);   // row_newbcast:u
             const uint32_t rel = (uint32_t)(ci4 - cjb);          // table row times four; negative or dead: huge
             const uint32_t off = (rel < trash_rel ? rel : trash_rel) + table_off;
@@ -1364,10 +1365,9 @@ __global__ __launch_bounds__(256) void rpb_table_partial_kernel(FusedGroups gt, 
             return true;
         });
     };
-    int rot = rs;
-    for (int m0 = 0; BY_TASKS ? m0 < per_wave && sl * per_wave + m0 < bl.total : ws + (int64_t)m0 * wslices < windows; m0 += 64) {
+    for (int m0 = 0; BY_TASKS ? m0 < per_wave && sl * per_wave + m0 < bl.total : from.window + m0 <= to.window; m0 += 64) {
         load_headers(m0);
-        Cursor cur = seek(Cursor{m0, m0, rot, 1, 0, 0, 0, 0, true});
+        Cursor cur = seek(Cursor{m0, m0, 0, 0, 0, 0, 0, 0, true});
         Slot sa, sb, sc;
         issue(sa, cur);
         cur = advance(cur);
@@ -1387,7 +1387,6 @@ __global__ __launch_bounds__(256) void rpb_table_partial_kernel(FusedGroups gt, 
             cur = advance(cur);
             consume(sc);
         }
-        rot = cur.rot;
     }
     // the eight tables of the workgroup (four wavefronts, two halves each) are one head's: summed here in a fixed
     // order, so a quarter of the partial tables reaches memory and the reduction
@@ -1797,10 +1796,8 @@ int sswin_fused_bias_grad(const int32_t* plan, int64_t g_cap, int64_t G, const i
     return launch_ok("fused bias gradient");
 }
 
-// slices = window slices x wavefronts per window slice.  About 3072 wavefronts (three per SIMD: what a
-// wavefront waits for is its own chain of LDS read-add-writes, so a few of them share a SIMD well), eight per
-// window slice: the batches of a crowded window (up to 3 x 3 of them for 89 tokens) spread over all eight.
-// Measured on cfg2 (the two launches): 2048 wavefronts / 4 per slice 0.038 ms, 3072 / 8 0.036, 4096 / 8 0.040.
+// Wavefronts of a head, each with a run of rows or batches of equal cost.  About 3072 in all (three per SIMD: what a
+// wavefront waits for is its own chain of LDS read-add-writes, so a few of them share a SIMD well).
 // A table of more than 1 664 rows (windows of 7^3 positions: 2 197) leaves room for two workgroups per compute unit
 // only, a larger one for one: the launch then holds 2 048 or 1 024 wavefronts, so that all of them are resident at once
 // (3 072 wavefronts on two workgroups per unit ran as one full round and a half-empty second one).
@@ -1808,20 +1805,14 @@ static size_t table_grad_lds(int table_rows, int n) {
     const int rows_pad = (table_rows + 31) / 32 * 32 + 32;  // 32 spare rows
     return (size_t)8 * rows_pad * sizeof(float) + (size_t)n * sizeof(int32_t);
 }
-static void table_grad_slices(int64_t windows, int H, int table_rows, int* wslices, int* rsplit) {
-    constexpr int64_t PER_SLICE = 8;
+static int table_grad_slices(int64_t windows, int H, int table_rows) {
     const int64_t resident = std::max<int64_t>(1, std::min<int64_t>(3, (int64_t)(160 * 1024) / (int64_t)table_grad_lds(table_rows, 384)));
-    const int64_t WAVES = 1024 * resident;
-    const int64_t want = std::max<int64_t>(1, WAVES / (std::max(H, 1) * PER_SLICE));
-    *wslices = (int)std::min<int64_t>(want, std::max<int64_t>(1, windows));
-    *rsplit = (int)PER_SLICE;
+    const int64_t want = std::min<int64_t>(1024 * resident / std::max(H, 1), 8 * std::max<int64_t>(1, windows));
+    return (int)std::max<int64_t>(8, want / 4 * 4);             // whole workgroups per head
 }
 
 size_t sswin_bias_table_grad_workspace_bytes(int64_t G, int H, int table_rows) {
-    const int64_t windows = H > 0 ? G / H : 0;
-    int wslices, rsplit;
-    table_grad_slices(windows, H, table_rows, &wslices, &rsplit);
-    return (size_t)wslices * rsplit * H * table_rows * sizeof(float) + 256;
+    return (size_t)table_grad_slices(H > 0 ? G / H : 0, H, table_rows) * H * table_rows * sizeof(float) + 256;
 }
 
 // the two launches of the table gradient; bl == nullptr: batches from the group table
@@ -1830,16 +1821,12 @@ static int launch_table_grad(const FusedGroups& gt, const BatchList* bl, int64_t
                              size_t ws_bytes, hipStream_t s) {
     SSWIN_CHECK(ws_bytes >= sswin_bias_table_grad_workspace_bytes(G, H, table_rows), "bias_table_grad: workspace too small");
     const int64_t windows = G / H;
-    int wslices, rsplit;
-    table_grad_slices(windows, H, table_rows, &wslices, &rsplit);
+    int slices = table_grad_slices(windows, H, table_rows);
     if (bl) {
         // dealt batches: a wavefront should have about six of them before it is worth its table (small inputs: 22 000
         // voxels 18.5 -> 15 us with half the wavefronts; more wavefronts than the walking kernel's never paid)
-        const int per_head = (int)std::max<int64_t>(32, std::min<int64_t>((int64_t)wslices * rsplit, bl->total / 6));
-        wslices = (per_head + 3) / 4 * 4;                          // whole workgroups per head
-        rsplit = 1;
+        slices = (int)std::min<int64_t>(slices, std::max<int64_t>(32, bl->total / 6 / 4 * 4));
     }
-    const int slices = wslices * rsplit;
     float* partial = static_cast<float*>(ws);
     const int64_t waves = (int64_t)slices * H;
     const int rows_pad = (table_rows + 31) / 32 * 32 + 32;  // 32 spare rows
@@ -1857,10 +1844,10 @@ static int launch_table_grad(const FusedGroups& gt, const BatchList* bl, int64_t
     const dim3 grid((unsigned)((waves + 3) / 4));
     if (bl)
         hipLaunchKernelGGL(rpb_table_partial_kernel<true>, grid, dim3(256), lds, s, gt, *bl, tokens + 3 * N, H,
-                           code, n, offset0, table_rows, rows_pad, ds, windows, wslices, rsplit, partial);
+                           code, n, offset0, table_rows, rows_pad, ds, windows, slices, partial);
     else
         hipLaunchKernelGGL(rpb_table_partial_kernel<false>, grid, dim3(256), lds, s, gt, BatchList{}, tokens + 3 * N, H,
-                           code, n, offset0, table_rows, rows_pad, ds, windows, wslices, rsplit, partial);
+                           code, n, offset0, table_rows, rows_pad, ds, windows, slices, partial);
     hipLaunchKernelGGL(rpb_table_reduce_kernel, dim3((unsigned)((table_rows + 15) / 16), (unsigned)H), dim3(1024), 0, s,
                        partial, slices / 4, table_rows, H, d_table);
     return launch_ok("bias table gradient");
