@@ -462,6 +462,17 @@ int sswin_dense_forward(int dtype, int out_dtype, int transposed, int epilogue, 
  * rounded to nearest: the parameters of a block under mixed precision. */
 enum { SSWIN_CAST_PARTS = 8 };
 int sswin_cast_parts(int dtype, const void* const* src, const int64_t* sizes, int count, void* dst, void* stream);
+/* The feed-forward part of a block as one launch: y [N, D] = GELU(x w1^T + b1) w2^T + b2 + residual for x [N, D], w1 [hidden, D],
+ * w2 [D, hidden] (biases and residual, of y's type, may be null).  act and slope [N, hidden] of x's type receive GELU's value and
+ * derivative, or are both null.  Backward: du [N, hidden] = (dy w2) * slope, dx [N, D] = du w1.  fp32: 96 channels; 16 bit: 48, 96 or
+ * 192; hidden a multiple of 64 (fp32: 32) up to 1024; at least 32 rows.  All pointers 16-byte aligned. */
+int sswin_mlp_supported(int dtype, int64_t N, int D, int hidden);
+int sswin_mlp_preferred(int dtype, int64_t N, int D, int hidden);   /* supported, and ahead of the two layers */
+size_t sswin_mlp_workspace_bytes(int dtype, int D, int hidden, int backward);
+int sswin_mlp_forward(int dtype, int out_dtype, const void* x, int64_t N, int D, int hidden, const void* w1, const void* b1, const void* w2, const void* b2,
+                      const void* residual, void* y, void* act, void* slope, void* ws, size_t ws_bytes, void* stream);
+int sswin_mlp_backward(int dtype, const void* dy, int64_t N, int D, int hidden, const void* w1, const void* w2, const void* slope, void* du, void* dx, void* ws,
+                       size_t ws_bytes, void* stream);
 /* scratch for long reductions over few rows (shares of the reduction added in a fixed order); with less the call runs without */
 size_t sswin_dense_forward_workspace_bytes(int dtype, int64_t N, int K, int P);
 /* dw [P, K] = dy^T x and db [P] = column sums of dy (or null) for dy [N, P], x [N, K] of dtype; dw, db of out_dtype (dtype or

@@ -84,6 +84,11 @@ SIGNATURES = {
     "sswin_tall_linear_weight_grad_workspace_bytes": (_sz, [_i64, _i32, _i32]),
     "sswin_tall_linear_weight_grad": (_i32, [_vp, _vp, _i64, _i32, _i32, _vp, _vp, _vp, _sz, _vp]),
     "sswin_dense_supported": (_i32, [_i32, _i32, _i32]),
+    "sswin_mlp_supported": (_i32, [_i32, _i64, _i32, _i32]),
+    "sswin_mlp_preferred": (_i32, [_i32, _i64, _i32, _i32]),
+    "sswin_mlp_workspace_bytes": (_sz, [_i32, _i32, _i32, _i32]),
+    "sswin_mlp_forward": (_i32, [_i32, _i32, _vp, _i64, _i32, _i32, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _sz, _vp]),
+    "sswin_mlp_backward": (_i32, [_i32, _vp, _i64, _i32, _i32, _vp, _vp, _vp, _vp, _vp, _vp, _sz, _vp]),
     "sswin_cast_parts": (_i32, [_i32, _vp, _vp, _i32, _vp, _vp]),
     "sswin_dense_forward": (_i32, [_i32, _i32, _i32, _i32, _vp, _i64, _i32, _vp, _vp, _i32, _vp, _vp, _vp, _vp, _sz, _vp]),
     "sswin_dense_forward_workspace_bytes": (_sz, [_i32, _i64, _i32, _i32]),
@@ -114,7 +119,7 @@ SIGNATURES = {
                                                _vp, _i64, _i32, _vp, _i64, _i32, _vp, _i64, _i32, _vp, _i32, _vp]),
 }
 
-ABI_VERSION = 33
+ABI_VERSION = 34
 _lib = None
 
 # A list turns on timing of the library's launches: every call that takes a stream is bracketed by events on that

@@ -1,0 +1,420 @@
+// The feed-forward part of a block (sparse_swin/swin3d_base.py:700-706, 851-873) as one launch: both of its layers, the
+// step between them and what follows the second one.
+//   forward    g = GELU(x W1^T + b1), y = g W2^T + b2 + residual     (g and the derivative of GELU stored for the backward)
+//   backward   du = (dy W2) * slope, dx = du W1                      (du stored for the weight gradients)
+// Both are y = step(x A^T) B^T with A [hidden, D] and B [D, hidden]: A = W1, B = W2 forward, A = W2^T, B = W1^T backward.
+//
+// As two launches of dense.hip the hidden rows (4 D values a token) are written and read back between the layers and every
+// launch is bound by that traffic; inference does not need them in memory at all.  Here a wavefront owns 32 tokens.  Products are
+// formed transposed, z^T [hidden, tokens] = A x^T, so that an accumulator lane holds one token: with the rows of A permuted
+// (hidden_of) its 16 values of a 32-wide hidden tile are two runs of eight neighbours, which is the operand of the second product
+// y^T += B z^T in place.  No exchange between lanes, no round through LDS.  x stays in registers for the whole launch (96 channels:
+// 24 registers, as three pieces of fp32 72), y accumulates in registers, A and B pass from L2 into LDS a step of 32 hidden
+// channels at a time, the next step in flight, shared by the wavefronts of the workgroup.  What is stored or read per hidden value (g,
+// slope, du) goes through a tile of LDS per wavefront, so that it is touched in runs of 64 or 128 bytes (16 bits straight from
+// the accumulators, runs of 32 bytes: 225 000 rows fp16 48 channels 95 us, through the tile 69).
+//
+// Microseconds, two launches and one.  225 700 rows fp32 96 channels: forward 318 and 273, backward 277 and 251 (traffic alone at copy
+// rate 187 and 170; without the matrix instructions 205 and 212: rounds of 256 workgroups, the last one partly full).  fp16 48
+// channels, 225 000 rows: 89 and 69, 55 and 43 (55 and 38).  bf16 96 channels, inference, 112 700 rows: 66 and 46 (13; GELU on the
+// vector units 21).
+#include <algorithm>
+#include <type_traits>
+
+#include "dense_epilogue.hpp"
+#include "dense_operand.hpp"
+#include "mfma_block.hpp"
+#include "sswin_common.hpp"
+
+namespace sswin {
+namespace dense {
+
+struct MlpArgs {
+    const void* x;             // [N, D]
+    int64_t N;
+    int hidden;
+    const uint16_t* a;         // [planes][hidden, D]
+    const uint16_t* b;         // [planes][D, hidden]
+    const void* bias_a;        // [hidden] or null
+    const void* bias_b;        // [D] or null
+    const void* factor;        // backward: slope [N, hidden]
+    const void* residual;      // forward: [N, D] of y's type, or null
+    void* h;                   // g or du [N, hidden]
+    void* slope;               // forward: [N, hidden]
+    void* y;                   // [N, D]
+};
+
+constexpr int MLP_LDS = 160 * 1024;
+enum { MLP_INFER, MLP_TRAIN, MLP_BACKWARD };
+
+// row of the hidden tile (of an output tile) that is put into row i of the operand: accumulator register 8 s + e of half h is
+// then row 16 s + 8 h + e
+__device__ __forceinline__ int hidden_of(int i) { return (i & 0x13) | (i & 4) << 1 | (i & 8) >> 1; }
+
+// 16 bytes a lane, counted by the waits of the kernel below.  The registers of a store this wide may not be written by the next
+// instruction, which the compiler sees to for its own stores only.
+__device__ __forceinline__ void store_counted(void* p, const u32x4& v) {
+    asm volatile("global_store_dwordx4 %0, %1, off\n\ts_nop 1" ::"v"(p), "v"(v) : "memory");
+}
+
+template <typename T> __device__ __forceinline__ void planes_at(const T* p, u32x4 (&x)[Op<T>::PL]) {
+    if constexpr (Op<T>::PL == 3) {
+        const f32x4 lo = *reinterpret_cast<const f32x4*>(p), hi = *reinterpret_cast<const f32x4*>(p + 4);
+        const float v[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+        planes_of<T>(v, x);
+    } else {
+        x[0] = *reinterpret_cast<const u32x4*>(p);
+    }
+}
+
+// 32 hidden values (or columns of y) of a wavefront's 32 tokens in LDS, so that memory is touched in runs of a row: rows of ROW
+// 16-byte pieces, the pieces of a row exchanged by its number.  Own side: the lane's token; memory side: slots in their order.
+template <typename T> struct HiddenTile {
+    static constexpr int VALUES = 16 / (int)sizeof(T), ROW = 32 / VALUES, PIECES = 32 * ROW, MOVES = PIECES / 64, STEP_ROWS = 64 / ROW;
+    static __device__ __forceinline__ int slot(int r, int piece) { return r * ROW + (piece ^ (ROW == 8 ? r & 7 : r >> 1 & 3)); }
+    // row and first column of this lane's slot of the first 64; the same column in the others
+    static __device__ __forceinline__ int mem_row() { return (threadIdx.x & 63) / ROW; }
+    static __device__ __forceinline__ int mem_col() {
+        const int r = mem_row(), s = (threadIdx.x & 63) % ROW;
+        return (slot(r, s) - r * ROW) * VALUES;
+    }
+    // the values 16 s + 8 half .. + 7 of the own token
+    static __device__ __forceinline__ void put(u32x4* tile, int s, const float (&v)[8]) {
+        const int half = (threadIdx.x & 63) >> 5, l32 = threadIdx.x & 31;
+        if constexpr (sizeof(T) == 4) {
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+                tile[slot(l32, s * 4 + half * 2 + h)] = __builtin_bit_cast(u32x4, f32x4{v[4 * h], v[4 * h + 1], v[4 * h + 2], v[4 * h + 3]});
+        } else {
+            u32x4 p[1];
+            planes_of<T>(v, p);
+            tile[slot(l32, s * 2 + half)] = p[0];
+        }
+    }
+    static __device__ __forceinline__ void get(const u32x4* tile, int s, float (&v)[8]) {
+        const int half = (threadIdx.x & 63) >> 5, l32 = threadIdx.x & 31;
+        if constexpr (sizeof(T) == 4) {
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const f32x4 p = __builtin_bit_cast(f32x4, tile[slot(l32, s * 4 + half * 2 + h)]);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[4 * h + e] = p[e];
+            }
+        } else {
+            const Vec8<T> p = __builtin_bit_cast(Vec8<T>, tile[slot(l32, s * 2 + half)]);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v[e] = to_acc(p.q[e / 4].v[e % 4]);
+        }
+    }
+};
+
+// the step between the layers on eight hidden values
+template <typename T, int MODE>
+__device__ __forceinline__ void between(const f32x16& z, int s, const float* bias, const u32x4* tile, float (&v)[8], float (&u)[8]) {
+    if constexpr (MODE == MLP_BACKWARD) {
+        HiddenTile<T>::get(tile, s, u);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = z[s * 8 + e] * u[e];
+    } else {
+        const f32x4* const b8 = reinterpret_cast<const f32x4*>(bias + s * 16 + ((threadIdx.x & 63) >> 5) * 8);
+        const f32x4 b[2] = {b8[0], b8[1]};
+#pragma unroll
+        for (int e = 0; e < 8; ++e) gelu_and_slope<sizeof(T) == 4>(z[s * 8 + e] + b[e / 4][e % 4], v[e], u[e]);
+    }
+}
+
+// y of a wavefront's 32 tokens from row0 on, 32 columns at a time through a tile of fp32 values
+template <typename TO, int D, int MODE>
+__device__ __forceinline__ void store_y(const MlpArgs& g, const f32x16 (&y)[(D + 31) / 32], int64_t row0, const float* bias, u32x4* tile) {
+    using Y = HiddenTile<float>;
+#pragma unroll
+    for (int j = 0; j < (D + 31) / 32; ++j) {
+        const int col = j * 32 + Y::mem_col();
+        const bool in = D % 32 == 0 || col < D;
+        const int64_t at = (row0 + Y::mem_row()) * D + col;
+        Vec4<TO> r[4];
+        if (MODE != MLP_BACKWARD && g.residual && in)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) r[i] = *reinterpret_cast<const Vec4<TO>*>(static_cast<const TO*>(g.residual) + at + i * 8 * D);
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            float v[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v[e] = y[j][s * 8 + e];
+            Y::put(tile, s, v);
+        }
+        __builtin_amdgcn_wave_barrier();
+        if (in)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const f32x4 v = __builtin_bit_cast(f32x4, tile[i * 64 + (threadIdx.x & 63)]);
+                float o[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    o[e] = v[e];
+                    if constexpr (MODE != MLP_BACKWARD) {
+                        o[e] += bias[col + e];
+                        if (g.residual) o[e] += to_acc(r[i].v[e]);
+                    }
+                }
+                *reinterpret_cast<Vec4<TO>*>(static_cast<TO*>(g.y) + at + i * 8 * D) = pack4<TO>(o);
+            }
+    }
+}
+template <typename T> __device__ __forceinline__ void stage_biases(const MlpArgs& g, int D, float* bias) {
+    for (int e = threadIdx.x; e < g.hidden; e += (int)blockDim.x) bias[e] = g.bias_a ? to_acc(static_cast<const T*>(g.bias_a)[e]) : 0.f;
+    for (int e = threadIdx.x; e < D; e += (int)blockDim.x) bias[g.hidden + e] = g.bias_b ? to_acc(static_cast<const T*>(g.bias_b)[e]) : 0.f;
+}
+// a last ragged tile is moved back to end at row N, tiles behind it repeat it: rows stored twice hold the same bits
+__device__ __forceinline__ int64_t tile_row(int64_t t, int64_t N) { return t * 32 + 32 <= N ? t * 32 : N - 32; }
+
+// A step is 32 hidden channels.  The wait for the next step's A and B leaves the stores of this step in flight; it counts them, so they
+// are inline assembly.  fp32 inputs are taken to be finite, as by the first layer's own kernel (tall_linear.hip).
+template <typename T, int D, int MODE, int WAVES> struct MlpLds {
+    static constexpr int PIECES = Op<T>::PL * (D / 16 + 2 * ((D + 31) / 32));   // of 64 x 16 bytes, a step's A and B
+    // of 16 bytes, a wavefront's tiles: two of hidden values, at least one of y.  Inference: y leaves through the place of A and B
+    // where it is large enough
+    static constexpr bool SHARED = MODE == MLP_INFER && WAVES * 256 <= 2 * PIECES * 64;
+    static constexpr int OWN = SHARED ? 0 : std::max(256, 2 * HiddenTile<T>::PIECES);
+    static size_t bytes(int hidden) { return (size_t)2 * PIECES * 1024 + (size_t)(hidden + D) * 4 + (size_t)WAVES * OWN * 16; }
+};
+template <typename T, typename TO, int D, int MODE, int WAVES, int OCC>
+__global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(OCC, OCC))) void mlp_kernel(MlpArgs g) {
+    using L = MlpLds<T, D, MODE, WAVES>;
+    using H = HiddenTile<T>;
+    constexpr int PL = Op<T>::PL, KS = D / 16, CT = (D + 31) / 32, PA = KS * PL, PIECES = L::PIECES;
+    constexpr int STORES = MODE == MLP_INFER ? 0 : MODE == MLP_TRAIN ? 2 * H::MOVES : H::MOVES;
+    extern __shared__ __attribute__((aligned(16))) u32x4 lds[];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, half = lane >> 5, l32 = lane & 31;
+    float* const bias = reinterpret_cast<float*>(lds + 2 * PIECES * 64); // [hidden] and [D]
+    u32x4* const tiles = L::SHARED ? lds + wave * 256 : lds + 2 * PIECES * 64 + (g.hidden + D) / 4 + wave * L::OWN;
+    const int64_t row0 = tile_row((int64_t)blockIdx.x * WAVES + wave, g.N), plane = (int64_t)g.hidden * D;
+    const uint32_t lane_a = (uint32_t)(hidden_of(l32) * D + half * 8);
+    auto request = [&](int step) {
+        const uint32_t to = lds_address(lds) + (uint32_t)(step & 1) * PIECES * 1024;
+#pragma unroll
+        for (int q = 0; q < (PIECES + WAVES - 1) / WAVES; ++q) {
+            const int p = q * WAVES + wave, r = p - PA;                  // uniform in the wavefront
+            if (PIECES % WAVES != 0 && p >= PIECES) break;
+            const uint16_t* from;
+            if (p < PA) from = g.a + p % PL * plane + (int64_t)step * 32 * D + p / PL * 16 + lane_a;
+            else from = g.b + r % PL * plane + (int64_t)min(r / PL % CT * 32 + hidden_of(l32), D - 1) * g.hidden + step * 32 + r / (PL * CT) * 16 + half * 8;
+            copy_to_lds(from, to + (uint32_t)p * 1024);
+        }
+    };
+    const int steps = g.hidden / 32;
+    request(0);
+    if constexpr (MODE != MLP_BACKWARD) stage_biases<T>(g, D, bias);
+    u32x4 x[KS][PL];
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) planes_at<T>(static_cast<const T*>(g.x) + (row0 + l32) * D + ks * 16 + half * 8, x[ks]);
+    const int64_t mem = (row0 + H::mem_row()) * g.hidden + H::mem_col();
+    auto load_tile = [&](int step) {                                     // of slope
+#pragma unroll
+        for (int i = 0; i < H::MOVES; ++i)
+            copy_to_lds(static_cast<const T*>(g.factor) + mem + (int64_t)i * H::STEP_ROWS * g.hidden + step * 32,
+                        lds_address(tiles + (step & 1) * H::PIECES + i * 64));
+    };
+    auto store_tile = [&](const u32x4* tile, void* to, int step) {
+        u32x4 v[H::MOVES];
+#pragma unroll
+        for (int i = 0; i < H::MOVES; ++i) v[i] = tile[i * 64 + lane];
+#pragma unroll
+        for (int i = 0; i < H::MOVES; ++i) store_counted(static_cast<T*>(to) + mem + (int64_t)i * H::STEP_ROWS * g.hidden + step * 32, v[i]);
+    };
+    f32x16 y[CT];
+#pragma unroll
+    for (int j = 0; j < CT; ++j) y[j] = f32x16{0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+    if constexpr (MODE == MLP_BACKWARD) load_tile(0);
+    wait_copies<0>();
+    if (PL == 3 && wave < WAVES / 2) __builtin_amdgcn_s_setprio(1);      // the two wavefronts of a SIMD at different places of a step
+    for (int step = 0; step < steps; ++step) {
+        block_barrier();                                                 // this buffer is there, the other one is free
+        if (step + 1 < steps) {
+            request(step + 1);
+            if constexpr (MODE == MLP_BACKWARD) load_tile(step + 1);
+        }
+        u32x4* const tile = tiles + (MODE == MLP_BACKWARD ? (step & 1) * H::PIECES : 0);   // du takes the place of its slope
+        const u32x4* const pieces = lds + (step & 1) * PIECES * 64 + lane;
+        // z^T: the pieces of A are read a slice of 16 channels ahead of its products
+        f32x16 z = f32x16{0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+        u32x4 a[2][PL];
+#pragma unroll
+        for (int q = 0; q < PL; ++q) a[0][q] = pieces[q * 64];
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+            if (ks + 1 < KS)
+#pragma unroll
+                for (int q = 0; q < PL; ++q) a[(ks + 1) & 1][q] = pieces[((ks + 1) * PL + q) * 64];
+#pragma unroll
+            for (int p = 0; p < Op<T>::NP; ++p) z = Op<T>::mfma(a[ks & 1][Op<T>::PA[p]], x[ks][Op<T>::PB[p]], z);
+            __builtin_amdgcn_sched_group_barrier(0x100, PL, 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, Op<T>::NP, 0);
+        }
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            float v[8], u[8];
+            between<T, MODE>(z, s, bias + step * 32, tile, v, u);
+            if constexpr (MODE != MLP_INFER) H::put(tile, s, v);
+            if constexpr (MODE == MLP_TRAIN) H::put(tile + H::PIECES, s, u);
+            u32x4 h[PL], w[2][PL];
+            planes_of<T>(v, h);
+            auto read = [&](int j) {
+#pragma unroll
+                for (int q = 0; q < PL; ++q) w[j & 1][q] = pieces[(PA + (s * CT + j) * PL + q) * 64];
+            };
+            read(0);
+#pragma unroll
+            for (int j = 0; j < CT; ++j) {
+                if (j + 1 < CT) read(j + 1);
+#pragma unroll
+                for (int p = 0; p < Op<T>::NP; ++p) y[j] = Op<T>::mfma(w[j & 1][Op<T>::PA[p]], h[Op<T>::PB[p]], y[j]);
+            }
+        }
+        if constexpr (MODE != MLP_INFER) {
+            __builtin_amdgcn_wave_barrier();
+            store_tile(tile, g.h, step);
+            if constexpr (MODE == MLP_TRAIN) store_tile(tile + H::PIECES, g.slope, step);
+            __builtin_amdgcn_wave_barrier();
+        }
+        if (step + 1 < steps) wait_copies<STORES>();                     // all but the stores of this step
+    }
+    if constexpr (L::SHARED) block_barrier();                    // A and B have been read
+    store_y<TO, D, MODE>(g, y, row0, bias + g.hidden, tiles);
+}
+
+// A and B as the kernel reads them: fp32 weights as planes of their pieces, weights of the backward turned.  A thread per pair of
+// neighbours of a row.
+template <typename T>
+__global__ __launch_bounds__(256) void mlp_weights_kernel(const T* __restrict__ wa, const T* __restrict__ wb, bool turned, int D, int hidden,
+                                                          uint16_t* __restrict__ a, uint16_t* __restrict__ b) {
+    constexpr int PL = Op<T>::PL;
+    const int64_t pairs = (int64_t)D * hidden / 2, i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= 2 * pairs) return;
+    const bool second = i >= pairs;
+    const int64_t e = (second ? i - pairs : i) * 2;
+    const int cols = second ? hidden : D, rows = second ? D : hidden;    // of the result
+    const int64_t r = e / cols, c = e % cols;
+    const T* w = second ? wb : wa;
+    const T v0 = turned ? w[c * rows + r] : w[e], v1 = turned ? w[(c + 1) * rows + r] : w[e + 1];
+    uint16_t* to = (second ? b : a) + e;
+    if constexpr (PL == 3) {
+        uint32_t p[3];
+        split2(v0, v1, p[0], p[1], p[2]);
+#pragma unroll
+        for (int q = 0; q < 3; ++q) *reinterpret_cast<uint32_t*>(to + q * 2 * pairs) = p[q];
+    } else {
+        *reinterpret_cast<uint32_t*>(to) = (uint32_t)__builtin_bit_cast(uint16_t, v0) | (uint32_t)__builtin_bit_cast(uint16_t, v1) << 16;
+    }
+}
+
+template <typename K> static int allow_all_lds(K* k) {
+    SSWIN_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, MLP_LDS));
+    return 0;
+}
+template <typename T, typename TO, int D, int MODE, int WAVES, int OCC> static int launch_mlp_as(const MlpArgs& g, hipStream_t s) {
+    auto* k = mlp_kernel<T, TO, D, MODE, WAVES, OCC>;
+    static const int configured = allow_all_lds(k);
+    if (configured) return configured;
+    hipLaunchKernelGGL(k, dim3((unsigned)((g.N + WAVES * 32 - 1) / (WAVES * 32))), dim3(WAVES * 64), (MlpLds<T, D, MODE, WAVES>::bytes(g.hidden)), s, g);
+    return launch_ok("mlp");
+}
+template <typename T, typename TO, int MODE> static int launch_mlp(const MlpArgs& g, int D, hipStream_t s) {
+    // wavefronts per SIMD: what the registers allow without spilling
+    if constexpr (std::is_same<T, float>::value) return launch_mlp_as<T, TO, 96, MODE, 8, 2>(g, s);
+    else if (D == 48) return launch_mlp_as<T, TO, 48, MODE, 4, 4>(g, s);
+    else return launch_mlp_as<T, TO, 96, MODE, 4, MODE == MLP_INFER ? 4 : 3>(g, s);
+}
+
+template <typename T>
+static int launch_weights(const void* wa, const void* wb, bool turned, int D, int hidden, uint16_t* a, uint16_t* b, hipStream_t s) {
+    hipLaunchKernelGGL((mlp_weights_kernel<T>), dim3((unsigned)(((int64_t)D * hidden + 255) / 256)), dim3(256), 0, s, static_cast<const T*>(wa),
+                       static_cast<const T*>(wb), turned, D, hidden, a, b);
+    return launch_ok("mlp weights");
+}
+
+}  // namespace dense
+}  // namespace sswin
+
+using namespace sswin;
+using namespace sswin::dense;
+
+static int mlp_check(const char* what, int dtype, int64_t N, int D, int hidden, size_t ws_bytes, const void* ws, bool backward) {
+    SSWIN_CHECK(sswin_mlp_supported(dtype, N, D, hidden), "%s: %lld rows of %d channels, %d hidden, of type %d are not supported", what, (long long)N, D, hidden,
+                dtype);
+    SSWIN_CHECK(ws_bytes >= sswin_mlp_workspace_bytes(dtype, D, hidden, backward) && (uintptr_t)ws % 16 == 0, "%s: the workspace is too small or not aligned", what);
+    return 0;
+}
+
+extern "C" {
+
+int sswin_mlp_supported(int dtype, int64_t N, int D, int hidden) {
+    if (N < 32 || N >= (1ll << 31) || hidden < 64 || hidden % 32 != 0) return 0;
+    if (dtype == SSWIN_F32) return D == 96 && hidden <= 1024;
+    if (dtype != SSWIN_F16 && dtype != SSWIN_BF16) return 0;
+    return (D == 48 || D == 96) && hidden <= 1024;
+}
+
+// Where one launch is ahead of two.  16 bit: from 8192 rows on (8000 rows fp16 48 channels, forward and backward 25.0 -> 22.3 us, 4000
+// rows 17.6 -> 21.5; bf16 96 channels, inference, 19.8 -> 18.4 and 13.3 -> 18.3).  fp32: a round of workgroups on all compute units
+// takes about 62 us forward and backward alike, however full it is, so the rounds have to be three quarters full (60 000 rows 156 ->
+// 138 us, 90 000 (1.4 rounds) 238 -> 239, 112 700 309 -> 255, 225 700 595 -> 529).
+int sswin_mlp_preferred(int dtype, int64_t N, int D, int hidden) {
+    if (!sswin_mlp_supported(dtype, N, D, hidden)) return 0;
+    if (dtype != SSWIN_F32) return N >= 8192;
+    const int64_t blocks = (N + 255) / 256, cus = device_cus();
+    return blocks * 4 >= (blocks + cus - 1) / cus * cus * 3;
+}
+
+size_t sswin_mlp_workspace_bytes(int dtype, int D, int hidden, int backward) {
+    const size_t plane = (size_t)D * hidden * 2;
+    return dtype == SSWIN_F32 ? 6 * plane : backward ? 2 * plane : 0;
+}
+
+int sswin_mlp_forward(int dtype, int out_dtype, const void* x, int64_t N, int D, int hidden, const void* w1, const void* b1, const void* w2, const void* b2,
+                      const void* residual, void* y, void* act, void* slope, void* ws, size_t ws_bytes, void* stream) {
+    if (int rc = mlp_check("mlp_forward", dtype, N, D, hidden, ws_bytes, ws, false)) return rc;
+    SSWIN_CHECK(x && w1 && w2 && y && (!act == !slope) && (ws || dtype != SSWIN_F32), "mlp_forward: null pointer");
+    SSWIN_CHECK(((uintptr_t)x | (uintptr_t)w1 | (uintptr_t)b1 | (uintptr_t)w2 | (uintptr_t)b2 | (uintptr_t)residual | (uintptr_t)y | (uintptr_t)act |
+                 (uintptr_t)slope) % 16 == 0, "mlp_forward: pointers must be 16-byte aligned");
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    const uint16_t *a = static_cast<const uint16_t*>(w1), *b = static_cast<const uint16_t*>(w2);
+    if (dtype == SSWIN_F32) {
+        uint16_t* planes = static_cast<uint16_t*>(ws);
+        a = planes, b = planes + (size_t)3 * D * hidden;
+        if (int rc = launch_weights<float>(w1, w2, false, D, hidden, planes, planes + (size_t)3 * D * hidden, s)) return rc;
+    }
+    const MlpArgs g = {x, N, hidden, a, b, b1, b2, nullptr, residual, act, slope, y};
+#define MLP_RUN(T, TO) return act ? launch_mlp<T, TO, MLP_TRAIN>(g, D, s) : launch_mlp<T, TO, MLP_INFER>(g, D, s)
+    if (dtype == SSWIN_F32 && out_dtype == SSWIN_F32) MLP_RUN(float, float);
+    if (dtype == SSWIN_F16 && out_dtype == SSWIN_F16) MLP_RUN(__half, __half);
+    if (dtype == SSWIN_F16 && out_dtype == SSWIN_F32) MLP_RUN(__half, float);
+    if (dtype == SSWIN_BF16 && out_dtype == SSWIN_BF16) MLP_RUN(__hip_bfloat16, __hip_bfloat16);
+    if (dtype == SSWIN_BF16 && out_dtype == SSWIN_F32) MLP_RUN(__hip_bfloat16, float);
+#undef MLP_RUN
+    return fail("mlp_forward: operands of type %d with a result of type %d are not supported", dtype, out_dtype);
+}
+
+int sswin_mlp_backward(int dtype, const void* dy, int64_t N, int D, int hidden, const void* w1, const void* w2, const void* slope, void* du, void* dx, void* ws,
+                       size_t ws_bytes, void* stream) {
+    if (int rc = mlp_check("mlp_backward", dtype, N, D, hidden, ws_bytes, ws, true)) return rc;
+    SSWIN_CHECK(dy && w1 && w2 && slope && du && dx && ws, "mlp_backward: null pointer");
+    SSWIN_CHECK(((uintptr_t)dy | (uintptr_t)w1 | (uintptr_t)w2 | (uintptr_t)slope | (uintptr_t)du | (uintptr_t)dx) % 16 == 0,
+                "mlp_backward: pointers must be 16-byte aligned");
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    uint16_t *a = static_cast<uint16_t*>(ws), *b = a + sswin_mlp_workspace_bytes(dtype, D, hidden, 1) / 4;
+    const MlpArgs g = {dy, N, hidden, a, b, nullptr, nullptr, slope, nullptr, du, nullptr, dx};
+#define MLP_RUN(T)                                                                     \
+    do {                                                                               \
+        if (int rc = launch_weights<T>(w2, w1, true, D, hidden, a, b, s)) return rc;   \
+        return launch_mlp<T, T, MLP_BACKWARD>(g, D, s);                                \
+    } while (0)
+    if (dtype == SSWIN_F32) MLP_RUN(float);
+    if (dtype == SSWIN_F16) MLP_RUN(__half);
+    MLP_RUN(__hip_bfloat16);
+#undef MLP_RUN
+}
+
+}  // extern "C"

@@ -396,6 +396,47 @@ DenseGrads dense_backward(const Tensor& dy, const Tensor& x, const Tensor& w_in,
     return g;
 }
 
+// both layers of the feed-forward part as one launch, where that is ahead: x [N, D], w1 [hidden, D], w2 [D, hidden]
+bool mlp_takes(const Tensor& x, const Tensor& w1, const Tensor& w2) {
+    return w1.dim() == 2 && w2.dim() == 2 && w1.size(1) == x.size(1) && w2.size(0) == x.size(1) && w2.size(1) == w1.size(0) &&
+           w1.scalar_type() == x.scalar_type() && w2.scalar_type() == x.scalar_type() &&
+           sswin_mlp_preferred(code_of(x.scalar_type()), x.size(0), (int)x.size(1), (int)w1.size(0));
+}
+Tensor mlp_workspace(const Tensor& x, const Tensor& w1, bool backward, size_t& nb) {
+    nb = sswin_mlp_workspace_bytes(code_of(x.scalar_type()), (int)x.size(1), (int)w1.size(0), backward);
+    return nb ? bytes(nb, x) : Tensor();
+}
+Tensor feed_forward(const Tensor& x, const Tensor& w1_in, const Tensor& b1_in, const Tensor& w2_in, const Tensor& b2_in, const Tensor& residual, Tensor* act,
+                    Tensor* slope) {
+    auto bias_of = [&](const Tensor& b, int64_t n) { return !b.defined() || (b.dim() == 1 && b.size(0) == n && b.scalar_type() == x.scalar_type()); };
+    const int64_t N = x.size(0), D = x.size(1);
+    if (mlp_takes(x, w1_in, w2_in) && bias_of(b1_in, w1_in.size(0)) && bias_of(b2_in, D) && residual.dim() == 2 && residual.sizes() == x.sizes()) {
+        const Tensor w1 = ready(w1_in), b1 = ready(b1_in), w2 = ready(w2_in), b2 = ready(b2_in);
+        const int64_t hidden = w1.size(0);
+        Tensor y = at::empty(x.sizes(), residual.options());
+        if (act) *act = at::empty({N, hidden}, x.options()), *slope = at::empty({N, hidden}, x.options());
+        size_t nb;
+        const Tensor ws = mlp_workspace(x, w1, false, nb);
+        RUN(sswin_mlp_forward(code_of(x.scalar_type()), code_of(residual.scalar_type()), ptr(x), N, (int)D, (int)hidden, ptr(w1), ptr(b1), ptr(w2), ptr(b2),
+                              ptr(residual), ptr(y), act ? ptr(*act) : nullptr, act ? ptr(*slope) : nullptr, ptr(ws), nb, current_stream(x)));
+        return y;
+    }
+    const Tensor g = dense(x, w1_in, b1_in, SSWIN_DENSE_GELU, Tensor(), slope);
+    if (act) *act = g;
+    return dense(g, w2_in, b2_in, SSWIN_DENSE_RESIDUAL, residual, nullptr, residual.scalar_type());
+}
+// dy [N, D] -> du [N, hidden] = (dy w2) slope and dx = du w1
+std::pair<Tensor, Tensor> feed_forward_dx(const Tensor& dy, const Tensor& w1_in, const Tensor& w2_in, const Tensor& slope) {
+    const Tensor w1 = ready(w1_in), w2 = ready(w2_in);
+    const int64_t N = dy.size(0), D = dy.size(1), hidden = w1.size(0);
+    Tensor du = at::empty({N, hidden}, dy.options()), dx = at::empty({N, D}, dy.options());
+    size_t nb;
+    const Tensor ws = mlp_workspace(dy, w1, true, nb);
+    RUN(sswin_mlp_backward(code_of(dy.scalar_type()), ptr(dy), N, (int)D, (int)hidden, ptr(w1), ptr(w2), ptr(slope), ptr(du), ptr(dx), ptr(ws), nb,
+                           current_stream(dy)));
+    return {du, dx};
+}
+
 // ------------------------------------------------------------------------------------------
 // row normalisation
 // ------------------------------------------------------------------------------------------
@@ -696,8 +737,8 @@ struct BlockNode : torch::autograd::Function<BlockNode> {
         const Tensor o = attention_forward(*a, qkv, p[TABLE], saved);
         const Tensor h = dense(o, w[2], w[3], SSWIN_DENSE_RESIDUAL, x, nullptr, stream_type);
         const Tensor x2 = norm_forward(h, p[G2], p[B2], eps2, type, ctx ? &stats2 : nullptr);
-        const Tensor g = dense(x2, w[4], w[5], SSWIN_DENSE_GELU, Tensor(), ctx ? &slope : nullptr);
-        Tensor y = dense(g, w[6], w[7], SSWIN_DENSE_RESIDUAL, h, nullptr, stream_type);
+        Tensor g;
+        Tensor y = feed_forward(x2, w[4], w[5], w[6], w[7], h, ctx ? &g : nullptr, ctx ? &slope : nullptr);
         if (ctx) {
             ctx->save_for_backward({x, p[G1], w[0], p[TABLE], w[2], p[G2], w[4], w[6], stats1, x1, qkv, saved.bias32, saved.aux, o, h, stats2, x2, g,
                                     slope, saved.words});
@@ -727,9 +768,17 @@ struct BlockNode : torch::autograd::Function<BlockNode> {
             out[w] = r.dw, out[w + 1] = r.db;
             return r.dx;
         };
-        const Tensor du = through(W2, dyt, g, w2, SSWIN_DENSE_SCALE, slope);
+        Tensor d_x2;
+        if (mlp_takes(x2, w1, w2)) {
+            const auto [du, dx] = feed_forward_dx(dyt, w1, w2, slope);
+            if (ask[W2] || ask[C2]) std::tie(out[W2], out[C2]) = dense_dw(dyt, g, ask[C2], wt);
+            if (ask[W1] || ask[C1]) std::tie(out[W1], out[C1]) = dense_dw(du, x2, ask[C1], wt);
+            d_x2 = dx;
+        } else {
+            d_x2 = through(W1, through(W2, dyt, g, w2, SSWIN_DENSE_SCALE, slope), x2, w1);
+        }
         Tensor dht;                                                      // dh in the layers' type
-        const Tensor dh = norm_backward(through(W1, du, x2, w1), h, stats2, g2, dy, out[G2], out[B2], &dht);
+        const Tensor dh = norm_backward(d_x2, h, stats2, g2, dy, out[G2], out[B2], &dht);
         const Tensor d_o = through(PROJW, dht, o, projw);
         const Tensor d_qkv = attention_backward(*a, qkv, table, AttentionSaved{v[11], v[12], v[19]}, o, d_o, ask[TABLE], out[TABLE]);
         out[X] = norm_backward(through(QKVW, d_qkv, x1, qkvw), x, stats1, g1, dh, out[G1], out[B1]);

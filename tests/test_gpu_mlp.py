@@ -1,0 +1,105 @@
+"""GPU parity of the feed-forward part as one launch (``sswin_mlp_*``) against float64 arithmetic on the same inputs, and against
+the two layers it stands for.
+
+Bounds: a hidden value carries the error of its product (2e-6 of the sum of the absolute products, two chains of an fp32 GEMM) and of
+GELU (4e-7 of the value's own size, 1e-6 near 0), rounded to the layers' type; the second layer adds its own, and passes on that of the
+hidden values through the absolute weights."""
+import ctypes as C
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+CODE = {torch.float32: 0, torch.float16: 1, torch.bfloat16: 2}
+ROUND = {torch.float32: 0.0, torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8}
+
+
+def _ptr(t):
+    return C.c_void_p(t.data_ptr() if t is not None else None)
+
+
+def _stream():
+    return C.c_void_p(torch.cuda.current_stream().cuda_stream)
+
+
+def _empty(shape, dtype):
+    return torch.full(shape, float("nan"), dtype=dtype, device="cuda")
+
+
+def _workspace(lib, x, hidden, backward):
+    nb = lib.sswin_mlp_workspace_bytes(CODE[x.dtype], x.shape[1], hidden, backward)
+    return torch.empty(max(nb, 16), dtype=torch.uint8, device="cuda"), nb
+
+
+def _check(got, ref, bound, what):
+    assert not torch.isnan(got).any(), what
+    err = (got.double() - ref).abs()
+    assert (err <= bound).all(), f"{what}: {(err / bound).max().item():.2f} of the bound"
+
+
+def _gelu(u):
+    phi = 0.5 * torch.special.erfc(-u * 0.5 ** 0.5)
+    return u * phi, phi + u * torch.exp(-0.5 * u * u) * 0.3989422804014327
+
+
+# 32 rows, one more, parts of a workgroup, several workgroups with a ragged last tile; one and several steps of the hidden channels
+SIZES = [(torch.float32, 96, 384), (torch.float32, 96, 64), (torch.float16, 48, 192), (torch.bfloat16, 96, 384), (torch.float16, 96, 128), (torch.float16, 48, 64)]
+
+
+@pytest.mark.parametrize("N", [32, 33, 129, 3001, 140001])
+@pytest.mark.parametrize("dtype,D,hidden", SIZES, ids=lambda v: str(v).split(".")[-1])
+def test_mlp_against_float64(dtype, D, hidden, N):
+    from sparseswin3d_amd import _lib
+    lib = _lib.load()
+    gen = torch.Generator().manual_seed(N + D)
+    rand = lambda *s, std=1.0: (torch.randn(*s, generator=gen) * std).to(dtype).cuda()
+    x, w1, b1, w2, b2 = rand(N, D), rand(hidden, D, std=D ** -0.5), rand(hidden, std=0.5), rand(D, hidden, std=hidden ** -0.5), rand(D)
+    round_ = ROUND[dtype]
+    x64, w1d, w2d = x.double(), w1.double(), w2.double()
+    u = x64 @ w1d.t() + b1.double()
+    scale = x64.abs() @ w1d.abs().t() + b1.double().abs()
+    g64, d64 = _gelu(u)
+    g_err = 2e-6 * scale + 1e-6 + round_ * g64.abs() + (2.0 ** -24 if dtype == torch.float16 else 0)
+    d_err = 2e-6 * scale + 1e-6 + round_ * d64.abs() + (2.0 ** -24 if dtype == torch.float16 else 0)
+    for out in ([dtype] if dtype == torch.float32 else [dtype, torch.float32]):
+        res = torch.randn(N, D, generator=gen).to(out).cuda()
+        y64 = g64 @ w2d.t() + b2.double() + res.double()
+        y_err = g_err @ w2d.abs().t() + 2e-6 * (g64.abs() @ w2d.abs().t() + b2.double().abs() + res.double().abs()) + ROUND[out] * y64.abs()
+        for train in (True, False):
+            y, g, d = _empty((N, D), out), _empty((N, hidden), dtype) if train else None, _empty((N, hidden), dtype) if train else None
+            ws, nb = _workspace(lib, x, hidden, 0)
+            _lib.check(lib.sswin_mlp_forward(CODE[dtype], CODE[out], _ptr(x), N, D, hidden, _ptr(w1), _ptr(b1), _ptr(w2), _ptr(b2), _ptr(res), _ptr(y),
+                                             _ptr(g), _ptr(d), _ptr(ws), nb, _stream()))
+            _check(y, y64, y_err, f"y {out} train {train}")
+            if train:
+                _check(g, g64, g_err, "act")
+                _check(d, d64, d_err, "slope")
+    # without biases and residual
+    y = _empty((N, D), dtype)
+    ws, nb = _workspace(lib, x, hidden, 0)
+    _lib.check(lib.sswin_mlp_forward(CODE[dtype], CODE[dtype], _ptr(x), N, D, hidden, _ptr(w1), None, _ptr(w2), None, None, _ptr(y), None, None, _ptr(ws), nb,
+                                     _stream()))
+    g0 = _gelu(x64 @ w1d.t())[0]
+    bound = 2e-6 * (x64.abs() @ w1d.abs().t()) + 1e-6 + round_ * g0.abs() + (2.0 ** -24 if dtype == torch.float16 else 0)
+    y0 = g0 @ w2d.t()
+    _check(y, y0, bound @ w2d.abs().t() + 2e-6 * (g0.abs() @ w2d.abs().t()) + round_ * y0.abs(), "y without biases")
+
+    dy, slope = rand(N, D), d64.to(dtype)
+    du64 = (dy.double() @ w2d) * slope.double()
+    du_err = 2e-6 * (dy.double().abs() @ w2d.abs()) * slope.double().abs() + round_ * du64.abs() + (2.0 ** -24 if dtype == torch.float16 else 1e-30)
+    dx64 = du64 @ w1d
+    dx_err = du_err @ w1d.abs() + 2e-6 * (du64.abs() @ w1d.abs()) + round_ * dx64.abs() + (2.0 ** -24 if dtype == torch.float16 else 0)
+    du, dx = _empty((N, hidden), dtype), _empty((N, D), dtype)
+    ws, nb = _workspace(lib, x, hidden, 1)
+    _lib.check(lib.sswin_mlp_backward(CODE[dtype], _ptr(dy), N, D, hidden, _ptr(w1), _ptr(w2), _ptr(slope), _ptr(du), _ptr(dx), _ptr(ws), nb, _stream()))
+    _check(du, du64, du_err, "du")
+    _check(dx, dx64, dx_err, "dx")
+
+
+def test_mlp_refuses_what_it_does_not_take():
+    from sparseswin3d_amd import _lib
+    lib = _lib.load()
+    for dtype, n, d, hidden in [(0, 31, 96, 384), (0, 64, 48, 192), (0, 64, 96, 400), (2, 64, 96, 32), (2, 64, 96, 100), (2, 64, 112, 448), (2, 64, 192, 768), (2, 64, 96, 1056), (3, 64, 96, 384)]:
+        assert not lib.sswin_mlp_supported(dtype, n, d, hidden)
+        assert lib.sswin_mlp_backward(dtype, None, n, d, hidden, None, None, None, None, None, None, 1 << 30, None) != 0
