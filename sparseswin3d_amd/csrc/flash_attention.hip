@@ -24,9 +24,13 @@
 // carries {4 code, mask region, window} in one word, so one subtraction gives the table address and whether mask or window
 // differ.
 //
-// 112 700 voxels, windows of 7^3, 3 heads of 16 (27 million scores): fp32 forward 63 us, backward 212 us (the store of dS 36 of
-// them).  219 000 voxels, fp16: forward 84 us, backward 292 (72 and 273 with P and dS rounded to fp16, which loses the operators'
-// precision).  The block products with the attention matrix in memory take 195 and 258 us (112 700 voxels, fp32).  The vector ALU is
+// Backward: with dS asked for (the bias table's gradient needs it) the key side forms scores, P and dS, sums dV and dK and stores
+// dS, and the query side is dQ = dS K from the stored dS; before, both sides formed them and the query side stored.
+//
+// 112 700 voxels, windows of 7^3, 3 heads of 16 (27 million scores): fp32 forward 63 us, backward 212 us, now 178 (D 11, key side 125,
+// dQ 42).  219 000 voxels, fp16: forward 84 us, backward 296, now 285 (14, 180, 91; dS is 217 MB written and read again).  dQ waits for
+// memory, 15 us a wavefront of four 32 x 32 pieces; rows of dS padded to 64 bytes, rows read by neighbouring
+// lanes and exchanged, voxels kept in lanes change it by less than 3 %.  The block products with the attention matrix in memory take 195 and 258 us (112 700 voxels, fp32).  The vector ALU is
 // busy for half of a launch, the fp32 matrix instructions (which occupy it) for another quarter; leaving out the bias reads, the
 // exponentials or the row loads one by one changes the forward by less than 3 %, the rows of the backward by 15 %.
 #include <math.h>
@@ -462,7 +466,7 @@ __global__ __launch_bounds__(WAVES * 64, sizeof(T) == 4 ? 3 : 1) void flash_forw
 }
 
 // ------------------------------------------------------------------------------------------
-// backward, own = queries: D = dO . O, dQ = scale dS K, dS stored for the bias gradient
+// backward, own = queries: D = dO . O, dQ = scale dS K, where nobody asks for dS
 // ------------------------------------------------------------------------------------------
 template <typename T, int HD>
 __global__ __launch_bounds__(WAVES * 64) void flash_backward_q_kernel(Args g, int64_t groups) {
@@ -487,7 +491,6 @@ __global__ __launch_bounds__(WAVES * 64) void flash_backward_q_kernel(Args g, in
         Frag<T> q[2][NB], d_o[2][NB];
         uint32_t pq[2];
         int vq[2];
-        int64_t at[2];         // first value of the query's row of dS, less its window's first rank
         float lse[2], delta[2];
         f32x4 dq[2][NB];
         Step<T> ahead;
@@ -498,10 +501,6 @@ __global__ __launch_bounds__(WAVES * 64) void flash_backward_q_kernel(Args g, in
             vq[s] = __shfl(blocks.voxel, blocks.slot(b, s), 64);
             pq[s] = __shfl(blocks.word, blocks.slot(b, s), 64) + (uint32_t)g.offset4;
             lse[s] = g.lse[h * g.N + r];
-            if (g.ds) {
-                const int c = __shfl(blocks.c, blocks.slot(b, s), 64), T0 = __shfl(blocks.T, blocks.slot(b, s), 64);
-                at[s] = (int64_t)g.tok_sq[r] * g.H + (int64_t)h * c * c + (int64_t)(r - T0) * c - T0;
-            }
         }
 #pragma unroll
         for (int s = 0; s < 2; ++s) {
@@ -548,16 +547,6 @@ __global__ __launch_bounds__(WAVES * 64) void flash_backward_q_kernel(Args g, in
                         ds[j] = __builtin_amdgcn_exp2f(x) * dp[j];
                         if (!FAST && quad * 4 + j > last) ds[j] = 0.f;
                     }
-                    if (g.ds && s * 16 + l16 < b.len) {                  // four neighbours of a row of dS per lane
-                        float* row = g.ds + at[s] + k0 + quad * 4;
-                        if (FAST || (last >= 15 && !b.merged)) {
-                            *reinterpret_cast<f32x4_any*>(row) = ds;
-                        } else {
-#pragma unroll
-                            for (int j = 0; j < 4; ++j)
-                                if (quad * 4 + j <= last && !((pq[s] ^ step.w[j]) >> 23)) row[j] = ds[j];
-                        }
-                    }
                     const Frag<float> dst = {ds};
 #pragma unroll
                     for (int c = 0; c < NB; ++c) dq[s][c] = mma(kt[c], dst, dq[s][c]);
@@ -579,9 +568,138 @@ __global__ __launch_bounds__(WAVES * 64) void flash_backward_q_kernel(Args g, in
 }
 
 // ------------------------------------------------------------------------------------------
-// backward, own = keys: dV = P^T dO, dK = scale dS^T Q
+// backward from a stored dS: D = dO . O in front of the key side, dQ = scale dS K behind it
 // ------------------------------------------------------------------------------------------
+template <typename T, int HD> __global__ __launch_bounds__(256) void flash_delta_kernel(Args g) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;           // heads of a token side by side
+    if (i >= g.N * g.H) return;
+    const int64_t r = i / g.H, h = i - r * g.H, at = ((int64_t)g.order[r] * g.H + h) * HD;
+    const T* const a = static_cast<const T*>(g.dout) + at;
+    const T* const b = static_cast<const T*>(g.out) + at;
+    Frag<T> x[HD / 4], y[HD / 4];
+#pragma unroll
+    for (int q = 0; q < HD / 4; ++q) x[q].load(a + q * 4), y[q].load(b + q * 4);
+    float part[4] = {0.f, 0.f, 0.f, 0.f};                                // summed as four lanes of the query side would
+#pragma unroll
+    for (int q = 0; q < HD / 4; ++q)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            part[q & 3] = fmaf(to_acc(reinterpret_cast<const T*>(&x[q].v)[j]), to_acc(reinterpret_cast<const T*>(&y[q].v)[j]), part[q & 3]);
+    g.delta[h * g.N + r] = (part[0] + part[1]) + (part[2] + part[3]);
+}
+
+// own = queries
 template <typename T, int HD>
+__global__ __launch_bounds__(WAVES * 64) void flash_dq_kernel(Args g, int64_t groups) {
+    constexpr int NB = HD / 16;
+    int h;
+    int64_t first;
+    place(g.H, groups, h, first);
+    const int lane = threadIdx.x & 63, l16 = lane & 15, quad = lane >> 4;
+    const int64_t chunk = first + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (chunk * 32 >= g.N) return;
+    Blocks blocks(g, chunk);
+    blocks.begin(g);
+    const int64_t D = (int64_t)g.H * HD;
+    const Rows<T, HD> k_rows(g.qkv, 3 * D, D + h * HD);
+    Block b;
+    while (blocks.next(b)) {
+        int vq[2];
+        uint32_t at[2];        // first value of the query's row of dS, less its window's first rank (modulo 2^32: places are below 2^31)
+        f32x4 dq[2][NB];
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            const int r = b.a + min(s * 16 + l16, b.len - 1), c = __shfl(blocks.c, blocks.slot(b, s), 64), T0 = __shfl(blocks.T, blocks.slot(b, s), 64);
+            vq[s] = __shfl(blocks.voxel, blocks.slot(b, s), 64);
+            at[s] = (uint32_t)(g.tok_sq[r] * g.H + h * c * c + (r - T0) * c) - (uint32_t)T0;
+#pragma unroll
+            for (int c2 = 0; c2 < NB; ++c2) dq[s][c2] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+        // 32 keys at a time, whole lines of dS, the next 32 in flight
+        struct Tile {
+            f32x4 ds[2][2];
+            Frag<T> k[2][NB];                                            // 16 bits: rows, fp32: columns
+        };
+        struct Keys {
+            int v[2][sizeof(T) == 4 ? 4 : 1];                            // voxels of the lane's slots, or of its row
+        };
+        auto keys = [&](int k0, Keys& t) {
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int j = 0; j < (sizeof(T) == 4 ? 4 : 1); ++j) t.v[i][j] = g.order[min(k0 + i * 16 + (sizeof(T) == 4 ? quad * 4 + j : l16), b.to - 1)];
+        };
+        auto request = [&](int k0, const Keys& from, Tile& t) {
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                if constexpr (sizeof(T) == 4) k_rows.column(from.v[i], t.k[i], t.k[i], false);
+                else k_rows.row((uint32_t)from.v[i][0], t.k[i]);
+            }
+            if (b.to - k0 >= 32 && !b.merged) {
+#pragma unroll
+                for (int s = 0; s < 2; ++s)
+#pragma unroll
+                    for (int i = 0; i < 2; ++i) t.ds[i][s] = *reinterpret_cast<const f32x4_any*>(g.ds + (at[s] + (uint32_t)(k0 + i * 16 + quad * 4)));
+            } else {                                                     // the window's own tokens
+#pragma unroll
+                for (int s = 0; s < 2; ++s) {
+                    const int T0 = __shfl(blocks.T, blocks.slot(b, s), 64), end = T0 + __shfl(blocks.c, blocks.slot(b, s), 64);
+#pragma unroll
+                    for (int i = 0; i < 2; ++i)
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) {
+                            const int r = k0 + i * 16 + quad * 4 + j;
+                            t.ds[i][s][j] = r >= T0 && r < end ? g.ds[at[s] + (uint32_t)r] : 0.f;
+                        }
+                }
+            }
+        };
+        Tile tile;
+        Keys next;
+        keys(b.from, next);
+        request(b.from, next, tile);
+        if (b.to - b.from > 32) keys(b.from + 32, next);
+        for (int k0 = b.from; k0 < b.to; k0 += 32) {
+            const Tile now = tile;
+            if (b.to - k0 > 32) request(k0 + 32, next, tile);
+            if (b.to - k0 > 64) keys(k0 + 64, next);
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const int last = b.to - 1 - k0 - i * 16;
+                if (last < 0) break;
+                Frag<float> kt[NB];
+                if constexpr (sizeof(T) == 4) {
+#pragma unroll
+                    for (int c = 0; c < NB; ++c) kt[c] = now.k[i][c];
+                } else {
+                    const int none[4] = {0, 0, 0, 0};
+                    k_rows.column(none, now.k[i], kt, blocks.careful);
+                }
+                if (blocks.careful && last < 15) k_rows.clear(last, kt);
+#pragma unroll
+                for (int s = 0; s < 2; ++s) {
+                    const Frag<float> ds = {now.ds[i][s]};
+#pragma unroll
+                    for (int c = 0; c < NB; ++c) dq[s][c] = mma(kt[c], ds, dq[s][c]);
+                }
+            }
+        }
+        if (blocks.again(sum_of(dq))) continue;
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            if (s * 16 + l16 < b.len) {
+                T* row = static_cast<T*>(g.dqkv) + (int64_t)vq[s] * 3 * D + h * HD + quad * 4;
+#pragma unroll
+                for (int c = 0; c < NB; ++c) store4<T>(row + c * 16, dq[s][c] * g.scale);
+            }
+        }
+    }
+}
+
+// ------------------------------------------------------------------------------------------
+// backward, own = keys: dV = P^T dO, dK = scale dS^T Q; STORE: dS for the bias gradient and for dQ
+// ------------------------------------------------------------------------------------------
+template <typename T, int HD, bool STORE>
 __global__ __launch_bounds__(WAVES * 64) void flash_backward_kv_kernel(Args g, int64_t groups) {
     constexpr int NB = HD / 16;
     extern __shared__ float table[];
@@ -604,6 +722,8 @@ __global__ __launch_bounds__(WAVES * 64) void flash_backward_kv_kernel(Args g, i
         Frag<T> k[2][NB], v[2][NB];
         uint32_t pk[2];
         int vk[2];
+        uint32_t at[2];        // first value of the key's column of dS, less its window's first rank times the row's length
+        int width[2];          // of a row of dS
         f32x4 dk[2][NB], dv[2][NB];
         Step<T> ahead;
         ahead.load(g, b.from, b.to);
@@ -611,6 +731,11 @@ __global__ __launch_bounds__(WAVES * 64) void flash_backward_kv_kernel(Args g, i
         for (int s = 0; s < 2; ++s) {
             vk[s] = __shfl(blocks.voxel, blocks.slot(b, s), 64);
             pk[s] = __shfl(blocks.word, blocks.slot(b, s), 64);
+            if constexpr (STORE) {
+                const int r = b.a + min(s * 16 + l16, b.len - 1), T0 = __shfl(blocks.T, blocks.slot(b, s), 64);
+                width[s] = __shfl(blocks.c, blocks.slot(b, s), 64);
+                at[s] = (uint32_t)(g.tok_sq[r] * g.H + h * width[s] * width[s] + r - T0) - (uint32_t)T0 * (uint32_t)width[s];
+            }
         }
 #pragma unroll
         for (int s = 0; s < 2; ++s) {
@@ -662,6 +787,14 @@ __global__ __launch_bounds__(WAVES * 64) void flash_backward_kv_kernel(Args g, i
                         ds[j] = p[j] * dp[j];
                         if (!FAST && quad * 4 + j > last) ds[j] = 0.f;
                     }
+                    if constexpr (STORE) {
+                        if (s * 16 + l16 < b.len) {                      // four rows of dS, sixteen neighbours of each per store
+                            const uint32_t to = at[s] + (uint32_t)(q0 + quad * 4) * (uint32_t)width[s];
+#pragma unroll
+                            for (int j = 0; j < 4; ++j)
+                                if (FAST || (quad * 4 + j <= last && !((pk[s] ^ step.w[j]) >> 23))) g.ds[to + (uint32_t)(j * width[s])] = ds[j];
+                        }
+                    }
                     const Frag<float> pf = {p}, df = {ds};
 #pragma unroll
                     for (int c = 0; c < NB; ++c) dv[s][c] = mma(dot[c], pf, dv[s][c]), dk[s][c] = mma(qt[c], df, dk[s][c]);
@@ -685,11 +818,23 @@ __global__ __launch_bounds__(WAVES * 64) void flash_backward_kv_kernel(Args g, i
     }
 }
 
-template <typename K> static int launch(K kernel, const Args& g, hipStream_t s, const char* what) {
+template <typename K> static int launch(K kernel, const Args& g, hipStream_t s, const char* what, bool table = true) {
     const int64_t groups = (g.N + 32 * WAVES - 1) / (32 * WAVES);
     SSWIN_CHECK(groups * g.H < (1ll << 31), "%s: too many tokens", what);
-    hipLaunchKernelGGL(kernel, dim3((unsigned)(groups * g.H)), dim3(WAVES * 64), (size_t)g.rows * sizeof(float), s, g, groups);
+    hipLaunchKernelGGL(kernel, dim3((unsigned)(groups * g.H)), dim3(WAVES * 64), table ? (size_t)g.rows * sizeof(float) : 0, s, g, groups);
     return launch_ok(what);
+}
+
+// With dS asked for, the query side reads what the key side has stored instead of forming scores, exponentials and dP again.
+template <typename T, int HD> static int launch_backward(const Args& g, hipStream_t s) {
+    if (!g.ds) {
+        if (int rc = launch(flash_backward_q_kernel<T, HD>, g, s, "flash_backward, queries")) return rc;
+        return launch(flash_backward_kv_kernel<T, HD, false>, g, s, "flash_backward, keys");
+    }
+    hipLaunchKernelGGL((flash_delta_kernel<T, HD>), dim3((unsigned)((g.N * g.H + 255) / 256)), dim3(256), 0, s, g);
+    if (int rc = launch_ok("flash_backward, delta")) return rc;
+    if (int rc = launch(flash_backward_kv_kernel<T, HD, true>, g, s, "flash_backward, keys")) return rc;
+    return launch(flash_dq_kernel<T, HD>, g, s, "flash_backward, queries", false);
 }
 
 }  // namespace flash
@@ -739,6 +884,7 @@ int sswin_flash_forward(int dtype, const int32_t* tokens, const int32_t* word, i
     if (dtype == SSWIN_F32) return FLASH(flash_forward_kernel, float);
     if (dtype == SSWIN_F16) return FLASH(flash_forward_kernel, __half);
     return FLASH(flash_forward_kernel, __hip_bfloat16);
+#undef FLASH
 }
 
 int sswin_flash_backward(int dtype, const int32_t* tokens, const int32_t* word, const int32_t* tok_sq, int64_t N, int H, int hd, int n, const void* qkv, float scale,
@@ -753,15 +899,9 @@ int sswin_flash_backward(int dtype, const int32_t* tokens, const int32_t* word, 
     g.N = N, g.H = H, g.rows = rows, g.offset4 = offset0 * 4, g.scale = scale, g.table = table, g.qkv = qkv, g.out = const_cast<void*>(out);
     g.lse = const_cast<float*>(lse), g.dout = dout, g.delta = delta, g.dqkv = dqkv, g.ds = ds, g.tok_sq = tok_sq;
     hipStream_t s = static_cast<hipStream_t>(stream);
-    int rc;
-    if (dtype == SSWIN_F32) rc = FLASH(flash_backward_q_kernel, float);
-    else if (dtype == SSWIN_F16) rc = FLASH(flash_backward_q_kernel, __half);
-    else rc = FLASH(flash_backward_q_kernel, __hip_bfloat16);
-    if (rc) return rc;
-    if (dtype == SSWIN_F32) return FLASH(flash_backward_kv_kernel, float);
-    if (dtype == SSWIN_F16) return FLASH(flash_backward_kv_kernel, __half);
-    return FLASH(flash_backward_kv_kernel, __hip_bfloat16);
-#undef FLASH
+    if (dtype == SSWIN_F32) return hd == 16 ? launch_backward<float, 16>(g, s) : launch_backward<float, 32>(g, s);
+    if (dtype == SSWIN_F16) return hd == 16 ? launch_backward<__half, 16>(g, s) : launch_backward<__half, 32>(g, s);
+    return hd == 16 ? launch_backward<__hip_bfloat16, 16>(g, s) : launch_backward<__hip_bfloat16, 32>(g, s);
 }
 
 }  // extern "C"
