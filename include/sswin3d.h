@@ -392,6 +392,9 @@ int sswin_bias_from_table(const float* table, int table_rows, int H, const int32
 /* The same from a table of fp32, fp16 or bf16 values. */
 int sswin_bias_from_typed_table(int dtype, const void* table, int table_rows, int H, const int32_t* code, int offset0, int n,
                                 float* bias, void* stream);
+/* The same into [2, H, n, n]: the bias and behind it the bias turned, [H, key, query]. */
+int sswin_bias_pair_from_typed_table(int dtype, const void* table, int table_rows, int H, const int32_t* code, int offset0, int n,
+                                float* bias, void* stream);
 
 /* Gradient of the relative position bias table itself (swin3d_base.py:624-652 gathers the
  * [H,n,n] bias from a [(2w-1)^3, H] table by relative_position_index; autograd scatters back with
@@ -548,6 +551,28 @@ int sswin_window_attention_forward(int dtype, const int32_t* tasks, int64_t g_ca
  * group exchange their partial dS K through LDS) and only the larger groups have query-side tasks.
  * Asynchronous. */
 int sswin_window_attention_backward(int dtype, const int32_t* tasks, int64_t g_cap,
+                                    const int64_t* bucket_counts, const int32_t* tokens, int64_t N,
+                                    int H, int hd, const void* q_base, int64_t q_stride, int q_col0,
+                                    const void* k_base, int64_t k_stride, int k_col0,
+                                    const void* v_base, int64_t v_stride, int v_col0, float scale,
+                                    const float* bias, int n, const int8_t* mask, int n_mask_windows,
+                                    const void* o_base, int64_t o_stride, int o_col0,
+                                    const void* do_base, int64_t do_stride, int do_col0,
+                                    const float* lse, void* dq_base, int64_t dq_stride, int dq_col0,
+                                    void* dk_base, int64_t dk_stride, int dk_col0, void* dv_base,
+                                    int64_t dv_stride, int dv_col0, float* ds_out, int sides,
+                                    void* stream);
+/* The same with bias [2, H, n, n]: as above, and behind it turned (key, query), which the kernels whose lanes hold queries read in
+ * whole lines (sswin_bias_pair_from_typed_table). */
+int sswin_window_attention_forward_pair(int dtype, const int32_t* tasks, int64_t g_cap,
+                                   const int64_t* bucket_counts, const int32_t* tokens, int64_t N,
+                                   int H, int hd, const void* q_base, int64_t q_stride, int q_col0,
+                                   const void* k_base, int64_t k_stride, int k_col0,
+                                   const void* v_base, int64_t v_stride, int v_col0, float scale,
+                                   const float* bias, int n, const int8_t* mask, int n_mask_windows,
+                                   void* o_base, int64_t o_stride, int o_col0, float* lse,
+                                   void* stream);
+int sswin_window_attention_backward_pair(int dtype, const int32_t* tasks, int64_t g_cap,
                                     const int64_t* bucket_counts, const int32_t* tokens, int64_t N,
                                     int H, int hd, const void* q_base, int64_t q_stride, int q_col0,
                                     const void* k_base, int64_t k_stride, int k_col0,

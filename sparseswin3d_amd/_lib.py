@@ -73,6 +73,7 @@ SIGNATURES = {
     "sswin_column_sum": (_i32, [_vp, _i32, _i64, _i32, _vp, _vp, _sz, _vp]),
     "sswin_bias_from_table": (_i32, [_vp, _i32, _i32, _vp, _i32, _i32, _vp, _vp]),
     "sswin_bias_from_typed_table": (_i32, [_i32, _vp, _i32, _i32, _vp, _i32, _i32, _vp, _vp]),
+    "sswin_bias_pair_from_typed_table": (_i32, [_i32, _vp, _i32, _i32, _vp, _i32, _i32, _vp, _vp]),
     "sswin_bias_table_grad_workspace_bytes": (_sz, [_i64, _i32, _i32]),
     "sswin_bias_table_grad": (_i32, [_vp, _i64, _i64, _vp, _i64, _i32, _i32, _vp, _i32, _i32, _vp, _vp, _vp, _sz, _vp]),
     "sswin_bias_table_grad_tasks": (_i32, [_vp, _i64, _vp, _i64, _vp, _i64, _i32, _i32, _vp, _i32, _i32, _vp, _vp, _vp, _sz,
@@ -113,7 +114,14 @@ SIGNATURES = {
     "sswin_window_attention_forward": (_i32, [_i32, _vp, _i64, _vp, _vp, _i64, _i32, _i32,
                                               _vp, _i64, _i32, _vp, _i64, _i32, _vp, _i64, _i32, C.c_float,
                                               _vp, _i32, _vp, _i32, _vp, _i64, _i32, _vp, _vp]),
+    "sswin_window_attention_forward_pair": (_i32, [_i32, _vp, _i64, _vp, _vp, _i64, _i32, _i32,
+                                              _vp, _i64, _i32, _vp, _i64, _i32, _vp, _i64, _i32, C.c_float,
+                                              _vp, _i32, _vp, _i32, _vp, _i64, _i32, _vp, _vp]),
     "sswin_window_attention_backward": (_i32, [_i32, _vp, _i64, _vp, _vp, _i64, _i32, _i32,
+                                               _vp, _i64, _i32, _vp, _i64, _i32, _vp, _i64, _i32, C.c_float,
+                                               _vp, _i32, _vp, _i32, _vp, _i64, _i32, _vp, _i64, _i32, _vp,
+                                               _vp, _i64, _i32, _vp, _i64, _i32, _vp, _i64, _i32, _vp, _i32, _vp]),
+    "sswin_window_attention_backward_pair": (_i32, [_i32, _vp, _i64, _vp, _vp, _i64, _i32, _i32,
                                                _vp, _i64, _i32, _vp, _i64, _i32, _vp, _i64, _i32, C.c_float,
                                                _vp, _i32, _vp, _i32, _vp, _i64, _i32, _vp, _i64, _i32, _vp,
                                                _vp, _i64, _i32, _vp, _i64, _i32, _vp, _i64, _i32, _vp, _i32, _vp]),

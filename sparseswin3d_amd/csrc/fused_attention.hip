@@ -1149,13 +1149,17 @@ __global__ __launch_bounds__(256) void rpb_grad_reduce_kernel(const float* __res
 template <typename T>
 __global__ __launch_bounds__(256) void rpb_gather_kernel(const T* __restrict__ table, int rows, int H,
                                                          const int32_t* __restrict__ code, int offset0, int n,
-                                                         float* __restrict__ bias) {
+                                                         float* __restrict__ bias, bool pair) {
     const int e = blockIdx.x * 256 + threadIdx.x;
     if (e >= n * n) return;
     const int p = e / n, q = e - p * n;
-    const unsigned r = (unsigned)(code[p] - code[q] + offset0);
+    const unsigned r = (unsigned)(code[p] - code[q] + offset0), turned = (unsigned)(code[q] - code[p] + offset0);
+    auto entry = [&](unsigned row, int h) { return row < (unsigned)rows ? to_acc(table[(int64_t)row * H + h]) : 0.f; };
     // a workgroup per head (up to 24 heads one after the other: 5.1 us on average in a backbone, now 4.1)
-    for (int h = blockIdx.y; h < H; h += gridDim.y) bias[(int64_t)h * n * n + e] = r < (unsigned)rows ? to_acc(table[(int64_t)r * H + h]) : 0.f;
+    for (int h = blockIdx.y; h < H; h += gridDim.y) {
+        bias[(int64_t)h * n * n + e] = entry(r, h);
+        if (pair) bias[(int64_t)(H + h) * n * n + e] = entry(turned, h);
+    }
 }
 
 constexpr int RPBT_MAX_ROWS = 4096;
@@ -1912,22 +1916,29 @@ int sswin_bias_from_table(const float* table, int table_rows, int H, const int32
     return sswin_bias_from_typed_table(SSWIN_F32, table, table_rows, H, code, offset0, n, bias, stream);
 }
 
-int sswin_bias_from_typed_table(int dtype, const void* table, int table_rows, int H, const int32_t* code, int offset0, int n, float* bias,
-                                void* stream) {
+static int bias_from_typed_table(int dtype, const void* table, int table_rows, int H, const int32_t* code, int offset0, int n, float* bias, bool pair,
+                                 void* stream) {
     SSWIN_CHECK(table_rows > 0 && H > 0 && n > 0 && n <= 4096, "bias_from_table: bad sizes");
     SSWIN_CHECK(table && code && bias, "bias_from_table: null pointer");
     const dim3 grid((unsigned)((n * n + 255) / 256), (unsigned)std::min(H, 65535)), block(256);
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (dtype == SSWIN_F32)
-        hipLaunchKernelGGL(rpb_gather_kernel<float>, grid, block, 0, s, static_cast<const float*>(table), table_rows, H, code, offset0, n, bias);
+        hipLaunchKernelGGL(rpb_gather_kernel<float>, grid, block, 0, s, static_cast<const float*>(table), table_rows, H, code, offset0, n, bias, pair);
     else if (dtype == SSWIN_F16)
-        hipLaunchKernelGGL(rpb_gather_kernel<__half>, grid, block, 0, s, static_cast<const __half*>(table), table_rows, H, code, offset0, n, bias);
+        hipLaunchKernelGGL(rpb_gather_kernel<__half>, grid, block, 0, s, static_cast<const __half*>(table), table_rows, H, code, offset0, n, bias, pair);
     else if (dtype == SSWIN_BF16)
         hipLaunchKernelGGL(rpb_gather_kernel<__hip_bfloat16>, grid, block, 0, s, static_cast<const __hip_bfloat16*>(table), table_rows, H, code, offset0, n,
-                           bias);
+                           bias, pair);
     else
         return fail("bias_from_table: a table of type %d", dtype);
     return launch_ok("bias_from_table");
+}
+
+int sswin_bias_from_typed_table(int dtype, const void* table, int table_rows, int H, const int32_t* code, int offset0, int n, float* bias, void* stream) {
+    return bias_from_typed_table(dtype, table, table_rows, H, code, offset0, n, bias, false, stream);
+}
+int sswin_bias_pair_from_typed_table(int dtype, const void* table, int table_rows, int H, const int32_t* code, int offset0, int n, float* bias, void* stream) {
+    return bias_from_typed_table(dtype, table, table_rows, H, code, offset0, n, bias, true, stream);
 }
 
 }  // extern "C"

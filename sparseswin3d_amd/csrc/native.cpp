@@ -60,15 +60,16 @@ struct Timed {
         if (g_recorder) py::reinterpret_borrow<py::object>(g_recorder)(name, before);
     }
 };
-#define RUN(call)                                             \
+#define RUN_NAMED(name, call)                                 \
     do {                                                      \
         int rc_;                                              \
         {                                                     \
-            Timed timed_(#call);                              \
+            Timed timed_(name);                               \
             rc_ = call;                                       \
         }                                                     \
         TORCH_CHECK(rc_ == 0, sswin_last_error());            \
     } while (0)
+#define RUN(call) RUN_NAMED(#call, call)
 
 Tensor bytes(size_t n, const Tensor& like) { return at::empty({(int64_t)n}, like.options().dtype(at::kByte)); }
 
@@ -523,8 +524,15 @@ Tensor attention_forward(Attention& a, const Tensor& qkv, const Tensor& bias, At
     if (a.code.defined()) {
         const ScalarType kind = bias.scalar_type();
         const Tensor table = (kind == at::kHalf || kind == at::kBFloat16 ? bias : bias.to(at::kFloat)).contiguous();
-        saved.bias32 = at::empty({a.H, a.n, a.n}, fopt);
-        RUN(sswin_bias_from_typed_table(code_of(table.scalar_type()), ptr(table), (int)table.size(0), a.H, i32(a.code), a.offset0, a.n, f32(saved.bias32), s));
+        if (a.resident) {                                                // as [query, key] and turned
+            saved.bias32 = at::empty({2, a.H, a.n, a.n}, fopt);
+            RUN(sswin_bias_pair_from_typed_table(code_of(table.scalar_type()), ptr(table), (int)table.size(0), a.H, i32(a.code), a.offset0, a.n,
+                                                 f32(saved.bias32), s));
+        } else {
+            saved.bias32 = at::empty({a.H, a.n, a.n}, fopt);
+            RUN(sswin_bias_from_typed_table(code_of(table.scalar_type()), ptr(table), (int)table.size(0), a.H, i32(a.code), a.offset0, a.n,
+                                            f32(saved.bias32), s));
+        }
     } else {
         saved.bias32 = bias.to(at::kFloat).contiguous();
     }
@@ -532,9 +540,10 @@ Tensor attention_forward(Attention& a, const Tensor& qkv, const Tensor& bias, At
     const int8_t* mask = a.mask.defined() ? a.mask.data_ptr<int8_t>() : nullptr;
     if (a.resident) {
         saved.aux = at::empty({std::max<int64_t>(a.H * N, 1)}, fopt);
-        RUN(sswin_window_attention_forward(dt, i32(tp.tasks), tp.g_cap, tp.buckets, i32(tp.tokens), N, a.H, hd, ptr(qkv), 3 * D, 0, ptr(qkv), 3 * D, (int)D,
-                                           ptr(qkv), 3 * D, (int)(2 * D), (float)a.scale, f32(saved.bias32), a.n, mask, a.regions(), ptr(out), D, 0,
-                                           f32(saved.aux), s));
+        const auto run = saved.bias32.dim() == 4 ? sswin_window_attention_forward_pair : sswin_window_attention_forward;
+        RUN_NAMED("sswin_window_attention_forward", run(dt, i32(tp.tasks), tp.g_cap, tp.buckets, i32(tp.tokens), N, a.H, hd, ptr(qkv), 3 * D, 0, ptr(qkv),
+                                                        3 * D, (int)D, ptr(qkv), 3 * D, (int)(2 * D), (float)a.scale, f32(saved.bias32), a.n, mask,
+                                                        a.regions(), ptr(out), D, 0, f32(saved.aux), s));
         return out;
     }
     Tensor p = saved.aux = at::empty({tp.A}, fopt);
@@ -591,10 +600,11 @@ Tensor attention_backward(const Attention& a, const Tensor& qkv, const Tensor& b
     if (a.resident) {
         const int8_t* mask = a.mask.defined() ? a.mask.data_ptr<int8_t>() : nullptr;
         Tensor d_s = want_bias ? at::empty({std::max<int64_t>(tp.A, 1)}, fopt) : Tensor();
-        RUN(sswin_window_attention_backward(dt, i32(tp.tasks), tp.g_cap, tp.buckets, i32(tp.tokens), N, a.H, hd, ptr(qkv), 3 * D, 0, ptr(qkv), 3 * D, (int)D,
-                                            ptr(qkv), 3 * D, (int)(2 * D), (float)a.scale, f32(saved.bias32), a.n, mask, a.regions(), ptr(out), D, 0,
-                                            ptr(d_out), D, 0, f32(saved.aux), ptr(d_qkv), 3 * D, 0, ptr(d_qkv), 3 * D, (int)D, ptr(d_qkv), 3 * D,
-                                            (int)(2 * D), f32(d_s), 3, s));
+        const auto run = saved.bias32.dim() == 4 ? sswin_window_attention_backward_pair : sswin_window_attention_backward;
+        RUN_NAMED("sswin_window_attention_backward", run(dt, i32(tp.tasks), tp.g_cap, tp.buckets, i32(tp.tokens), N, a.H, hd, ptr(qkv), 3 * D, 0, ptr(qkv),
+                                                         3 * D, (int)D, ptr(qkv), 3 * D, (int)(2 * D), (float)a.scale, f32(saved.bias32), a.n, mask,
+                                                         a.regions(), ptr(out), D, 0, ptr(d_out), D, 0, f32(saved.aux), ptr(d_qkv), 3 * D, 0, ptr(d_qkv),
+                                                         3 * D, (int)D, ptr(d_qkv), 3 * D, (int)(2 * D), f32(d_s), 3, s));
         if (want_bias) d_bias = bias_gradient(a, d_s, bias);
         return d_qkv;
     }

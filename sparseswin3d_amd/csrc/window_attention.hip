@@ -126,8 +126,8 @@ __device__ __forceinline__ void fwd_task(const WAttnCommon& a, const GroupCtx& g
     const float qscale = a.scale * LOG2E;                    // scores are kept in units of log 2
 #pragma unroll
     for (int s = 0; s < 16; ++s) qb[s] *= qscale;
-    const char* bias_h = reinterpret_cast<const char*>(a.bias + (int64_t)h * a.n * a.n);
-    const uint32_t brow = (uint32_t)(pos_i * a.n) * 4u;
+    const BiasOfQueries bias(a, h);
+    const uint32_t bias_q = (uint32_t)pos_i * bias.q_step;
 
     float m = 0.f;                                           // the operator's max(0, rowmax)
     float l = 0.f;                                           // this lane half's share of the row sum
@@ -137,7 +137,7 @@ __device__ __forceinline__ void fwd_task(const WAttnCommon& a, const GroupCtx& g
     // rk, rv hold the K and V rows of key tile t (requested by the caller), ki its indices.
     auto tile_step = [&](auto first_tag, const int t, const KIdx& ki) {
         constexpr bool FIRST = decltype(first_tag)::value;
-        uint32_t pk = (uint32_t)ki.pos * 4u;
+        uint32_t pk = (uint32_t)ki.pos * bias.k_step;
         if (MASK) pk |= (uint32_t)mrow[ki.pos] << 16;
         __builtin_amdgcn_wave_barrier();
         table_put(tab_key, l32, pk);
@@ -150,7 +150,7 @@ __device__ __forceinline__ void fwd_task(const WAttnCommon& a, const GroupCtx& g
         float bv[16];
 #pragma unroll
         for (int r = 0; r < 16; ++r)
-            bv[r] = *reinterpret_cast<const float*>(bias_h + (brow + (MASK ? (pkr[r] & 0xffffu) : pkr[r])));
+            bv[r] = *reinterpret_cast<const float*>(bias.base + (bias_q + (MASK ? (pkr[r] & 0xffffu) : pkr[r])));
         float ka[16];
         tile_get_rows(tile_x, l32, half, ka);
         // S^T tile: rows = keys, columns = queries
@@ -273,7 +273,8 @@ __device__ __forceinline__ void fwd_task_small(const WAttnCommon& a, const Group
         rk[v] = *reinterpret_cast<const u32x4_a*>(kbase + (__umul24(vr, kpitch) + off));
         rv[v] = *reinterpret_cast<const u32x4_a*>(vbase + (__umul24(vr, vpitch) + off));
     }
-    uint32_t pk = (uint32_t)pos * 4u;
+    const BiasOfQueries bias(a, h);
+    uint32_t pk = (uint32_t)pos * bias.k_step;
     if (MASK) pk |= (uint32_t)reg << 16;
     __builtin_amdgcn_wave_barrier();
     if (sl == 0) tab_key[col] = pk;
@@ -289,11 +290,10 @@ __device__ __forceinline__ void fwd_task_small(const WAttnCommon& a, const Group
     // bias gathers first: keys 4 sl .. 4 sl + 3 of query col
     const u32x4_a pkq = *reinterpret_cast<const u32x4_a*>(tab_key + 4 * sl);
     const uint32_t pkr[4] = {pkq.x, pkq.y, pkq.z, pkq.w};
-    const char* bias_h = reinterpret_cast<const char*>(a.bias + (int64_t)h * a.n * a.n);
-    const uint32_t brow = (uint32_t)(pos * a.n) * 4u;
+    const uint32_t bias_q = (uint32_t)pos * bias.q_step;
     float bv[4];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) bv[r] = *reinterpret_cast<const float*>(bias_h + (brow + (MASK ? (pkr[r] & 0xffffu) : pkr[r])));
+    for (int r = 0; r < 4; ++r) bv[r] = *reinterpret_cast<const float*>(bias.base + (bias_q + (MASK ? (pkr[r] & 0xffffu) : pkr[r])));
     float qb[8], ka[8];
     {
         const f32x4_a* pq = reinterpret_cast<const f32x4_a*>(tile_x + col * TILE_LD + 8 * sl);
@@ -446,8 +446,8 @@ __device__ __forceinline__ void bwd_q_task(const WAttnCommon& a, int64_t task, f
     const float qscale = a.scale * LOG2E;
 #pragma unroll
     for (int s = 0; s < 16; ++s) qb[s] *= qscale;
-    const char* bias_h = reinterpret_cast<const char*>(a.bias + (int64_t)h * a.n * a.n);
-    const uint32_t brow = (uint32_t)(pos_i * a.n) * 4u;
+    const BiasOfQueries bias(a, h);
+    const uint32_t bias_q = (uint32_t)pos_i * bias.q_step;
 
     f32x16 dq = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
 #pragma unroll 1
@@ -457,7 +457,7 @@ __device__ __forceinline__ void bwd_q_task(const WAttnCommon& a, int64_t task, f
         RowLoad<T> rk, rv;
         rows_load<T>(kbase, kpitch, vox_j, lane, rk);
         rows_load<T>(vbase, vpitch, vox_j, lane, rv);
-        uint32_t pk = (uint32_t)pos_j * 4u;
+        uint32_t pk = (uint32_t)pos_j * bias.k_step;
         if (MASK) pk |= (uint32_t)mrow[pos_j] << 16;
         if (t + 1 < nt) {                                    // indices of the next key tile, a tile ahead
             const int2 e = token_entry(a, rec0 + t + 1, l32);
@@ -477,7 +477,7 @@ __device__ __forceinline__ void bwd_q_task(const WAttnCommon& a, int64_t task, f
         float bv[16];
 #pragma unroll
         for (int r = 0; r < 16; ++r)
-            bv[r] = *reinterpret_cast<const float*>(bias_h + (brow + (MASK ? (pkr[r] & 0xffffu) : pkr[r])));
+            bv[r] = *reinterpret_cast<const float*>(bias.base + (bias_q + (MASK ? (pkr[r] & 0xffffu) : pkr[r])));
         f32x16 St = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
         f32x16 dPt = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
         mma_slots<T, 0, 16>(ka, qb, St);
@@ -1120,7 +1120,7 @@ static bool legacy_kernels(int dtype) {
 }
 
 static WAttnCommon make_common(const int32_t* tasks, int64_t g_cap, const int64_t* counts, const int32_t* tokens,
-                               int64_t N, int H, int n, float scale, const float* bias, const int8_t* mask, int nmw) {
+                               int64_t N, int H, int n, float scale, const float* bias, bool pair, const int8_t* mask, int nmw) {
     WAttnCommon a;
     a.tasks = reinterpret_cast<const int4*>(tasks);
     a.g_cap = g_cap;
@@ -1135,6 +1135,7 @@ static WAttnCommon make_common(const int32_t* tasks, int64_t g_cap, const int64_
     a.n = n;
     a.scale = scale;
     a.bias = bias;
+    a.bias_t = pair ? bias + (int64_t)H * n * n : nullptr;
     a.mask = mask;
     a.nmw = nmw;
     return a;
@@ -1165,17 +1166,13 @@ static int check_common(const char* who, int dtype, const int32_t* tasks, int64_
 
 using namespace sswin;
 
-extern "C" {
-
-int sswin_window_attention_forward(int dtype, const int32_t* tasks, int64_t g_cap, const int64_t* bucket_counts,
-                                   const int32_t* tokens, int64_t N, int H, int hd, const void* q_base,
-                                   int64_t q_stride, int q_col0, const void* k_base, int64_t k_stride, int k_col0,
-                                   const void* v_base, int64_t v_stride, int v_col0, float scale, const float* bias,
-                                   int n, const int8_t* mask, int n_mask_windows, void* o_base, int64_t o_stride,
-                                   int o_col0, float* lse, void* stream) {
+static int attention_forward(bool pair, int dtype, const int32_t* tasks, int64_t g_cap, const int64_t* bucket_counts,
+                             const int32_t* tokens, int64_t N, int H, int hd, const void* q_base, int64_t q_stride,
+                             int q_col0, const void* k_base, int64_t k_stride, int k_col0, const void* v_base, int64_t
+                             v_stride, int v_col0, float scale, const float* bias, int n, const int8_t* mask, int
+                             n_mask_windows, void* o_base, int64_t o_stride, int o_col0, float* lse, void* stream) {
     int64_t total = 0;
-    if (check_common("window_attention_forward", dtype, tasks, g_cap, bucket_counts, tokens, N, H, hd, bias, n, mask,
-                     n_mask_windows, &total))
+    if (check_common("window_attention_forward", dtype, tasks, g_cap, bucket_counts, tokens, N, H, hd, bias, n, mask, n_mask_windows, &total))
         return 1;
     if (total == 0) return 0;
     SSWIN_CHECK(q_base && k_base && v_base && o_base && lse, "window_attention_forward: null pointer");
@@ -1184,7 +1181,7 @@ int sswin_window_attention_forward(int dtype, const int32_t* tasks, int64_t g_ca
         check_tensor("window_attention_forward", "v", v_base, v_stride, v_col0, N, H, dtype) ||
         check_tensor("window_attention_forward", "o", o_base, o_stride, o_col0, N, H, dtype))
         return 1;
-    const WAttnCommon a = make_common(tasks, g_cap, bucket_counts, tokens, N, H, n, scale, bias, mask, n_mask_windows);
+    const WAttnCommon a = make_common(tasks, g_cap, bucket_counts, tokens, N, H, n, scale, bias, pair, mask, n_mask_windows);
     const TokenTensor32 q{q_base, q_stride, q_col0}, k{k_base, k_stride, k_col0}, v{v_base, v_stride, v_col0},
         o{o_base, o_stride, o_col0};
     hipStream_t s = static_cast<hipStream_t>(stream);
@@ -1200,15 +1197,14 @@ int sswin_window_attention_forward(int dtype, const int32_t* tasks, int64_t g_ca
     }
 }
 
-int sswin_window_attention_backward(int dtype, const int32_t* tasks, int64_t g_cap, const int64_t* bucket_counts,
-                                    const int32_t* tokens, int64_t N, int H, int hd, const void* q_base,
-                                    int64_t q_stride, int q_col0, const void* k_base, int64_t k_stride, int k_col0,
-                                    const void* v_base, int64_t v_stride, int v_col0, float scale, const float* bias,
-                                    int n, const int8_t* mask, int n_mask_windows, const void* o_base,
-                                    int64_t o_stride, int o_col0, const void* do_base, int64_t do_stride,
-                                    int do_col0, const float* lse, void* dq_base, int64_t dq_stride, int dq_col0,
-                                    void* dk_base, int64_t dk_stride, int dk_col0, void* dv_base, int64_t dv_stride,
-                                    int dv_col0, float* ds_out, int sides, void* stream) {
+static int attention_backward(bool pair, int dtype, const int32_t* tasks, int64_t g_cap, const int64_t* bucket_counts,
+                              const int32_t* tokens, int64_t N, int H, int hd, const void* q_base, int64_t q_stride,
+                              int q_col0, const void* k_base, int64_t k_stride, int k_col0, const void* v_base,
+                              int64_t v_stride, int v_col0, float scale, const float* bias, int n, const int8_t* mask,
+                              int n_mask_windows, const void* o_base, int64_t o_stride, int o_col0, const void*
+                              do_base, int64_t do_stride, int do_col0, const float* lse, void* dq_base, int64_t
+                              dq_stride, int dq_col0, void* dk_base, int64_t dk_stride, int dk_col0, void* dv_base,
+                              int64_t dv_stride, int dv_col0, float* ds_out, int sides, void* stream) {
     int64_t total = 0;
     if (check_common("window_attention_backward", dtype, tasks, g_cap, bucket_counts, tokens, N, H, hd, bias, n, mask,
                      n_mask_windows, &total))
@@ -1231,7 +1227,7 @@ int sswin_window_attention_backward(int dtype, const int32_t* tasks, int64_t g_c
                             check_tensor(who, "dv", dv_base, dv_stride, dv_col0, N, H, dtype)))
             return 1;
     }
-    const WAttnCommon a = make_common(tasks, g_cap, bucket_counts, tokens, N, H, n, scale, bias, mask, n_mask_windows);
+    const WAttnCommon a = make_common(tasks, g_cap, bucket_counts, tokens, N, H, n, scale, bias, pair, mask, n_mask_windows);
     const TokenTensor32 q{q_base, q_stride, q_col0}, k{k_base, k_stride, k_col0}, v{v_base, v_stride, v_col0},
         o{o_base, o_stride, o_col0}, d_o{do_base, do_stride, do_col0}, dq{dq_base, dq_stride, dq_col0},
         dk{dk_base, dk_stride, dk_col0}, dv{dv_base, dv_stride, dv_col0};
@@ -1246,6 +1242,53 @@ int sswin_window_attention_backward(int dtype, const int32_t* tasks, int64_t g_c
         case SSWIN_BF16: return run_backward<__hip_bfloat16>(a, q, k, v, o, d_o, lse, dq, dk, dv, ds_out, sides, s);
         default: return fail("window_attention_backward: unsupported token dtype %d", dtype);
     }
+}
+
+extern "C" {
+
+int sswin_window_attention_forward(int dtype, const int32_t* tasks, int64_t g_cap, const int64_t* bucket_counts,
+                                   const int32_t* tokens, int64_t N, int H, int hd, const void* q_base,
+                                   int64_t q_stride, int q_col0, const void* k_base, int64_t k_stride, int k_col0,
+                                   const void* v_base, int64_t v_stride, int v_col0, float scale, const float* bias,
+                                   int n, const int8_t* mask, int n_mask_windows, void* o_base, int64_t o_stride,
+                                   int o_col0, float* lse, void* stream) {
+    return attention_forward(false, dtype, tasks, g_cap, bucket_counts, tokens, N, H, hd, q_base, q_stride, q_col0, k_base, k_stride,
+                k_col0, v_base, v_stride, v_col0, scale, bias, n, mask, n_mask_windows, o_base, o_stride, o_col0, lse, stream);
+}
+int sswin_window_attention_forward_pair(int dtype, const int32_t* tasks, int64_t g_cap, const int64_t* bucket_counts,
+                                   const int32_t* tokens, int64_t N, int H, int hd, const void* q_base,
+                                   int64_t q_stride, int q_col0, const void* k_base, int64_t k_stride, int k_col0,
+                                   const void* v_base, int64_t v_stride, int v_col0, float scale, const float* bias,
+                                   int n, const int8_t* mask, int n_mask_windows, void* o_base, int64_t o_stride,
+                                   int o_col0, float* lse, void* stream) {
+    return attention_forward(true, dtype, tasks, g_cap, bucket_counts, tokens, N, H, hd, q_base, q_stride, q_col0, k_base, k_stride, k_col0,
+                v_base, v_stride, v_col0, scale, bias, n, mask, n_mask_windows, o_base, o_stride, o_col0, lse, stream);
+}
+int sswin_window_attention_backward(int dtype, const int32_t* tasks, int64_t g_cap, const int64_t* bucket_counts,
+                                    const int32_t* tokens, int64_t N, int H, int hd, const void* q_base,
+                                    int64_t q_stride, int q_col0, const void* k_base, int64_t k_stride, int k_col0,
+                                    const void* v_base, int64_t v_stride, int v_col0, float scale, const float* bias,
+                                    int n, const int8_t* mask, int n_mask_windows, const void* o_base,
+                                    int64_t o_stride, int o_col0, const void* do_base, int64_t do_stride,
+                                    int do_col0, const float* lse, void* dq_base, int64_t dq_stride, int dq_col0,
+                                    void* dk_base, int64_t dk_stride, int dk_col0, void* dv_base, int64_t dv_stride,
+                                    int dv_col0, float* ds_out, int sides, void* stream) {
+    return attention_backward(false, dtype, tasks, g_cap, bucket_counts, tokens, N, H, hd, q_base, q_stride, q_col0, k_base, k_stride,
+                k_col0, v_base, v_stride, v_col0, scale, bias, n, mask, n_mask_windows, o_base, o_stride, o_col0, do_base, do_stride,
+                do_col0, lse, dq_base, dq_stride, dq_col0, dk_base, dk_stride, dk_col0, dv_base, dv_stride, dv_col0, ds_out, sides, stream);
+}
+int sswin_window_attention_backward_pair(int dtype, const int32_t* tasks, int64_t g_cap, const int64_t* bucket_counts,
+                                    const int32_t* tokens, int64_t N, int H, int hd, const void* q_base,
+                                    int64_t q_stride, int q_col0, const void* k_base, int64_t k_stride, int k_col0,
+                                    const void* v_base, int64_t v_stride, int v_col0, float scale, const float* bias,
+                                    int n, const int8_t* mask, int n_mask_windows, const void* o_base,
+                                    int64_t o_stride, int o_col0, const void* do_base, int64_t do_stride,
+                                    int do_col0, const float* lse, void* dq_base, int64_t dq_stride, int dq_col0,
+                                    void* dk_base, int64_t dk_stride, int dk_col0, void* dv_base, int64_t dv_stride,
+                                    int dv_col0, float* ds_out, int sides, void* stream) {
+    return attention_backward(true, dtype, tasks, g_cap, bucket_counts, tokens, N, H, hd, q_base, q_stride, q_col0, k_base, k_stride,
+                k_col0, v_base, v_stride, v_col0, scale, bias, n, mask, n_mask_windows, o_base, o_stride, o_col0, do_base, do_stride,
+                do_col0, lse, dq_base, dq_stride, dq_col0, dk_base, dk_stride, dk_col0, dv_base, dv_stride, dv_col0, ds_out, sides, stream);
 }
 
 }  // extern "C"

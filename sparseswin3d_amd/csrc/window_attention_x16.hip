@@ -352,8 +352,8 @@ __device__ __forceinline__ void fwd_task(const WAttnCommon& a, const GroupCtx& g
     uint32_t vox_j = (uint32_t)e_k0.x;
     int pos_j = e_k0.y;
     const int reg_i = MASK ? mrow[pos_i] : 0;
-    const char* bias_h = reinterpret_cast<const char*>(a.bias + (int64_t)h * a.n * a.n);
-    const uint32_t brow = (uint32_t)(pos_i * a.n) * 4u;
+    const BiasOfQueries bias(a, h);
+    const uint32_t bias_q = (uint32_t)pos_i * bias.q_step;
     RowLoad<T> rk, rv, rq;
     Op qR;
     int aQ = 0;
@@ -378,7 +378,7 @@ __device__ __forceinline__ void fwd_task(const WAttnCommon& a, const GroupCtx& g
         rows_load<T>(vbase, vpitch, vox_j, lane, rv);
         if (t + 1 < nt) load_kidx(t + 1, vox_n, pos_n);      // the indices of the next tile, a tile ahead
         __builtin_amdgcn_wave_barrier();
-        table_put(tab_key, l32, (uint32_t)pos_j * 4u | (uint32_t)reg_k << 16);
+        table_put(tab_key, l32, (uint32_t)pos_j * bias.k_step | (uint32_t)reg_k << 16);
         __builtin_amdgcn_wave_barrier();
         float bv[16];
         uint32_t differ = 0;                                  // bit r: regions of the query and the key differ
@@ -387,7 +387,7 @@ __device__ __forceinline__ void fwd_task(const WAttnCommon& a, const GroupCtx& g
             table_get(tab_key, hf, pkr);
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
-                bv[r] = *reinterpret_cast<const float*>(bias_h + (brow + (MASK ? (pkr[r] & 0xffffu) : pkr[r])));
+                bv[r] = *reinterpret_cast<const float*>(bias.base + (bias_q + (MASK ? (pkr[r] & 0xffffu) : pkr[r])));
                 if (MASK) differ |= ((int)(pkr[r] >> 16) != reg_i ? 1u : 0u) << r;
             }
         }
@@ -533,8 +533,8 @@ __device__ __forceinline__ void bwd_q_task(const WAttnCommon& a, int64_t task, f
         doR = read_R<T>(tile_x, l32, hf);
     }
     const float D = u2f(tab_D.get(l32));
-    const char* bias_h = reinterpret_cast<const char*>(a.bias + (int64_t)h * a.n * a.n);
-    const uint32_t brow = (uint32_t)(pos_i * a.n) * 4u;
+    const BiasOfQueries bias(a, h);
+    const uint32_t bias_q = (uint32_t)pos_i * bias.q_step;
 
     f32x16 dq = zero16();
     int xq = 0;
@@ -555,7 +555,7 @@ __device__ __forceinline__ void bwd_q_task(const WAttnCommon& a, int64_t task, f
             pos_n = e.y;
         }
         __builtin_amdgcn_wave_barrier();
-        table_put(tab_key, l32, (uint32_t)pos_j * 4u | (uint32_t)reg_k << 16);
+        table_put(tab_key, l32, (uint32_t)pos_j * bias.k_step | (uint32_t)reg_k << 16);
         __builtin_amdgcn_wave_barrier();
         float bv[16];
         uint32_t differ = 0;                                  // bit r: regions of the query and the key differ
@@ -564,7 +564,7 @@ __device__ __forceinline__ void bwd_q_task(const WAttnCommon& a, int64_t task, f
             table_get(tab_key, hf, pkr);
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
-                bv[r] = *reinterpret_cast<const float*>(bias_h + (brow + (MASK ? (pkr[r] & 0xffffu) : pkr[r])));
+                bv[r] = *reinterpret_cast<const float*>(bias.base + (bias_q + (MASK ? (pkr[r] & 0xffffu) : pkr[r])));
                 if (MASK) differ |= ((int)(pkr[r] >> 16) != reg_i ? 1u : 0u) << r;
             }
         }
