@@ -713,110 +713,68 @@ __global__ __launch_bounds__(SMALL_WAVES * 64) void dense_small_kernel(const T* 
 }
 
 // ------------------------------------------------------------------------------------------
-// dW [P, K] = dY^T X, db [P] = column sums of dY.  A workgroup owns BM x BN of dW for one chunk of rows.  Operands are requested
-// two steps of 16 rows ahead: with one, a step waited for memory (8500 cycles of which 1150 are products; 219 000 rows 384 -> 96:
-// 190 us, with two 146; 35 569 rows 192 -> 576 and 192 -> 192 60 and 48).
+// dW [P, K] = dY^T X, db [P] = column sums of dY.  A workgroup owns BM x BN of dW for one chunk of rows; WK groups of its wavefronts
+// take 16 rows of a step each, and their sums are added through LDS at the end.
+// Bound by the splitting into planes (120 vector instructions a wavefront and step) next to the products.  Therefore:
+//   12 wavefronts a compute unit in one workgroup, which also writes one partial sum (two workgroups of 6 do not fit next to each
+//   other: 219 000 rows 384 -> 96 150 us, one of 12 with two row groups 121, four wavefronts of 64 x 96 before 155);
+//   one unit of 8 x 2 values a lane at most, and the next step's splitting between this step's products, without a branch (with two
+//   units on some wavefronts every one splits twice: 96 -> 384 rows 207 us, now 118);
+//   rows requested two steps ahead, with waits that count (the loop waited for everything it had requested: a branch stood
+//   between).
 // ------------------------------------------------------------------------------------------
-template <int WM, int WN, int MT, int NT, int OCC>
-__global__ __launch_bounds__(WM * WN * 64) __attribute__((amdgpu_waves_per_eu(OCC, OCC))) void dense_wgrad_kernel(
+template <int WM, int WN, int WK, int MT, int NT, int OCC>
+__global__ __launch_bounds__(WM * WN * WK * 64) __attribute__((amdgpu_waves_per_eu(OCC, OCC))) void dense_wgrad_kernel(
     const float* __restrict__ dy, const float* __restrict__ x, int64_t N, int P, int K, int tiles_p, int tiles_k, int64_t rows_per_chunk,
     float* __restrict__ part_w, float* __restrict__ part_b) {
-    constexpr int PL = 3, BK = 16, KC = BK / 8;
-    constexpr int BM = WM * MT * 32, BN = WN * NT * 32, THREADS = WM * WN * 64;
-    constexpr int A_UNITS = BM / 2 * KC, UA = (A_UNITS + THREADS - 1) / THREADS;
-    constexpr int B_UNITS = BN / 2 * KC, UB = (B_UNITS + THREADS - 1) / THREADS;
+    constexpr int PL = 3, BK = 16 * WK, WAVES = WM * WN;                 // waves of a row part
+    constexpr int BM = WM * MT * 32, BN = WN * NT * 32, THREADS = WK * WAVES * 64;
+    // A unit is 8 rows of two columns; a wavefront takes 64 units of dY or 64 of X
+    constexpr int A_UNITS = BM, B_UNITS = BN, A_WAVES = (A_UNITS + 63) / 64, B_WAVES = (B_UNITS + 63) / 64;
+    static_assert(A_WAVES + B_WAVES <= WAVES, "a unit for every lane at most");
     constexpr int A_LDS = BM / 32 * PL * 64, B_LDS = BN / 32 * PL * 64, BUF = A_LDS + B_LDS;
-    extern __shared__ __attribute__((aligned(16))) u32x4 lds[];
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, half = lane >> 5, l32 = lane & 31;
+    extern __shared__ __attribute__((aligned(16))) u32x4 lds[];          // [buffer 2][row part][dY, X][32 columns][plane][lane]
+    const int id = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wave = id % WAVES, part = id / WAVES, lane = threadIdx.x & 63, half = lane >> 5, l32 = lane & 31;
     const int wm = wave / WN, wn = wave % WN;
     int tile;
     int64_t chunk;
     block_of(tiles_p * tiles_k, tile, chunk);
     const int p0 = (tile / tiles_k) * BM, k0 = (tile % tiles_k) * BN;
+    u32x4* planes = lds + part * BUF;
     const int64_t begin = chunk * rows_per_chunk, end = begin + rows_per_chunk < N ? begin + rows_per_chunk : N;
-    const bool sums_here = part_b && k0 == 0;
 
-    Down ra[2][UA], rx[2][UB];                                           // of the next two steps
-    float bs[UA][2];
+    // Lanes without a unit of their own read, split and store the last one again: no branch, so that the waits can count the loads and
+    // the splitting can go between the products
+    const bool of_a = wave < A_WAVES;
+    const int own = (of_a ? wave : min(wave - A_WAVES, B_WAVES - 1)) * 64 + lane, unit = min(own, (of_a ? A_UNITS : B_UNITS) - 1);
+    const int pairs = of_a ? BM / 2 : BN / 2, eight = unit / pairs, column = unit % pairs * 2, first_row = part * 16 + eight * 8;
+    const int pitch = of_a ? P : K;
+    const float* rows = of_a ? dy : x;
+    const uint32_t from = (uint32_t)(first_row * pitch + (of_a ? min(p0 + column, P - 2) : min(k0 + column, K - 2)));
+    u32x4* to = planes + (of_a ? 0 : A_LDS) + (column >> 5) * PL * 64 + eight * 32 + (column & 31);
+
+    Down raw[2];                                                         // of the next two steps
+    float bs[2] = {0.f, 0.f};
+    auto request = [&](int slot, int64_t n0) {                           // a step of whole rows
 #pragma unroll
-    for (int i = 0; i < UA; ++i) bs[i][0] = bs[i][1] = 0.f;
-    uint32_t oa[UA], ox[UB];
-#pragma unroll
-    for (int i = 0; i < UA; ++i) {
-        const int u = min((int)threadIdx.x + i * THREADS, A_UNITS - 1);
-        oa[i] = (uint32_t)((u / (BM / 2)) * 8 * P + min(p0 + (u % (BM / 2)) * 2, P - 2));
-    }
-#pragma unroll
-    for (int i = 0; i < UB; ++i) {
-        const int u = min((int)threadIdx.x + i * THREADS, B_UNITS - 1);
-        ox[i] = (uint32_t)((u / (BN / 2)) * 8 * K + min(k0 + (u % (BN / 2)) * 2, K - 2));
-    }
-    // 16 whole rows.  Lanes without a unit read the last one again: no branch around the loads, so that the waits can count them
-    auto request = [&](int slot, int64_t n0) {
-        const float* yb = dy + n0 * P;
-        const float* xb = x + n0 * K;
-#pragma unroll
-        for (int i = 0; i < UA; ++i)
-#pragma unroll
-            for (int e = 0; e < 8; ++e) ra[slot][i].load(e, yb + e * P + oa[i]);
-#pragma unroll
-        for (int i = 0; i < UB; ++i)
-#pragma unroll
-            for (int e = 0; e < 8; ++e) rx[slot][i].load(e, xb + e * K + ox[i]);
+        for (int e = 0; e < 8; ++e) raw[slot].load(e, rows + (n0 + e) * pitch + from);
     };
     auto request_end = [&](int slot, int64_t n0) {                       // zeros past the last row
-        const float* yb = dy + n0 * P;
-        const float* xb = x + n0 * K;
-        const int left = (int)(end - n0);
+        const int64_t left = end - n0 - first_row;
 #pragma unroll
-        for (int i = 0; i < UA; ++i) {
-            const int n = min((int)threadIdx.x + i * THREADS, A_UNITS - 1) / (BM / 2) * 8;
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                if (n + e < left) ra[slot][i].load(e, yb + e * P + oa[i]);
-                else ra[slot][i].zero(e);
-            }
-        }
-#pragma unroll
-        for (int i = 0; i < UB; ++i) {
-            const int n = min((int)threadIdx.x + i * THREADS, B_UNITS - 1) / (BN / 2) * 8;
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                if (n + e < left) rx[slot][i].load(e, xb + e * K + ox[i]);
-                else rx[slot][i].zero(e);
-            }
+        for (int e = 0; e < 8; ++e) {
+            if (e < left) raw[slot].load(e, rows + (n0 + e) * pitch + from);
+            else raw[slot].zero(e);
         }
     };
-    auto put = [&](u32x4* base, int tiles, int row, int c, const u32x4 (&p)[PL]) {
-        u32x4* dst = base + (((c >> 1) * tiles + (row >> 5)) * PL) * 64 + (c & 1) * 32 + (row & 31);
+    auto store = [&](int slot) {
 #pragma unroll
-        for (int q = 0; q < PL; ++q) dst[q * 64] = p[q];
-    };
-    auto store = [&](int slot, u32x4* buf) {
+        for (int h = 0; h < 2; ++h) {
+            u32x4 p[PL];
+            raw[slot].planes(h, p);
+            bs[h] += raw[slot].sum(h);
 #pragma unroll
-        for (int i = 0; i < UA; ++i) {
-            const int u = threadIdx.x + i * THREADS, pair = u % (BM / 2), c = u / (BM / 2);
-            if (A_UNITS % THREADS == 0 || u < A_UNITS) {
-#pragma unroll
-                for (int h = 0; h < 2; ++h) {
-                    u32x4 p[PL];
-                    ra[slot][i].planes(h, p);
-                    put(buf, BM / 32, pair * 2 + h, c, p);
-                    if (sums_here) bs[i][h] += ra[slot][i].sum(h);
-                }
-            }
-        }
-#pragma unroll
-        for (int i = 0; i < UB; ++i) {
-            const int u = threadIdx.x + i * THREADS, pair = u % (BN / 2), c = u / (BN / 2);
-            if (B_UNITS % THREADS == 0 || u < B_UNITS) {
-#pragma unroll
-                for (int h = 0; h < 2; ++h) {
-                    u32x4 p[PL];
-                    rx[slot][i].planes(h, p);
-                    put(buf + A_LDS, BN / 32, pair * 2 + h, c, p);
-                }
-            }
+            for (int q = 0; q < PL; ++q) to[slot * WK * BUF + h + q * 64] = p[q];
         }
     };
     f32x16 acc[MT][NT];
@@ -827,34 +785,45 @@ __global__ __launch_bounds__(WM * WN * 64) __attribute__((amdgpu_waves_per_eu(OC
     const int nk = (int)((end - begin + BK - 1) / BK), whole = (int)((end - begin) / BK);
     request_end(0, begin);
     if (nk > 1) request_end(1, begin + BK);
-    store(0, lds);
+    store(0);
+    if (nk > 2) request_end(0, begin + 2 * BK);
     auto products = [&](int slot) {
-        const u32x4* buf = lds + slot * BUF;
-        u32x4 a[MT][PL], b[NT][PL];
+        const u32x4* buf = planes + slot * WK * BUF;
+        u32x4 a[MT][PL];
 #pragma unroll
         for (int i = 0; i < MT; ++i)
 #pragma unroll
             for (int q = 0; q < PL; ++q) a[i][q] = buf[((wm * MT + i) * PL + q) * 64 + lane];
 #pragma unroll
-        for (int j = 0; j < NT; ++j)
+        for (int j = 0; j < NT; ++j) {
+            u32x4 b[PL];
 #pragma unroll
-            for (int q = 0; q < PL; ++q) b[j][q] = buf[A_LDS + ((wn * NT + j) * PL + q) * 64 + lane];
+            for (int q = 0; q < PL; ++q) b[q] = buf[A_LDS + ((wn * NT + j) * PL + q) * 64 + lane];
 #pragma unroll
-        for (int p = 0; p < Op<float>::NP; ++p)
+            for (int p = 0; p < Op<float>::NP; ++p)
 #pragma unroll
-            for (int i = 0; i < MT; ++i)
-#pragma unroll
-                for (int j = 0; j < NT; ++j) acc[i][j] = Op<float>::mfma(a[i][Op<float>::PA[p]], b[j][Op<float>::PB[p]], acc[i][j]);
-        __builtin_amdgcn_sched_barrier(0);                               // the next operands' splitting stays behind the products
+                for (int i = 0; i < MT; ++i) acc[i][j] = Op<float>::mfma(a[i][Op<float>::PA[p]], b[Op<float>::PB[p]], acc[i][j]);
+        }
     };
+    // Step kb multiplies its planes and splits the rows of kb + 1, requested two steps before; those of kb + 3 are requested then
     int kb = 0;
-    for (; kb + 3 < whole; kb += 2) {
+    constexpr int MFMAS = Op<float>::NP * MT * NT;
+    for (; kb + 4 < whole; kb += 2) {
 #pragma unroll
         for (int slot = 0; slot < 2; ++slot) {
             __syncthreads();
-            request(slot, begin + (int64_t)(kb + slot + 2) * BK);
             products(slot);
-            store(slot ^ 1, lds + (slot ^ 1) * BUF);
+            store(slot ^ 1);
+            request(slot ^ 1, begin + (int64_t)(kb + slot + 3) * BK);
+#pragma unroll
+            for (int g = 0; g < MFMAS; ++g) {                            // the splitting between the products
+                if (g == 0) __builtin_amdgcn_sched_group_barrier(0x100, (MT + 1) * PL, 0);
+                if (g % (Op<float>::NP * MT) == 1 && g / (Op<float>::NP * MT) + 1 < NT) __builtin_amdgcn_sched_group_barrier(0x100, PL, 0);
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x002, (120 + MFMAS - 1) / MFMAS, 0);
+                if (g >= MFMAS - 6) __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
         }
     }
     for (; kb < nk; kb += 2) {
@@ -862,46 +831,58 @@ __global__ __launch_bounds__(WM * WN * 64) __attribute__((amdgpu_waves_per_eu(OC
         for (int slot = 0; slot < 2; ++slot) {
             if (kb + slot >= nk) break;
             __syncthreads();
-            if (kb + slot + 2 < nk) request_end(slot, begin + (int64_t)(kb + slot + 2) * BK);
             products(slot);
-            if (kb + slot + 1 < nk) store(slot ^ 1, lds + (slot ^ 1) * BUF);
+            if (kb + slot + 1 < nk) store(slot ^ 1);
+            if (kb + slot + 3 < nk) request_end(slot ^ 1, begin + (int64_t)(kb + slot + 3) * BK);
         }
     }
-    float* pw = part_w + chunk * (int64_t)P * K;
-    f32x4 any = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int i = 0; i < MT; ++i)
+    for (int q = 1; q < WK; ++q) {                                       // the sums of the other row parts, in order, onto those of part 0
+        float* red = reinterpret_cast<float*>(lds) + wave * 64 + lane;
+        __syncthreads();
+        if (part == q) {
 #pragma unroll
-        for (int j = 0; j < NT; ++j)
+            for (int e = 0; e < MT * NT * 16; ++e) red[e * WAVES * 64] = acc[e / (NT * 16)][e / 16 % NT][e & 15];
+        }
+        __syncthreads();
+        if (part == 0) {
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int p = p0 + (wm * MT + i) * 32 + acc_row(r, half), k = k0 + (wn * NT + j) * 32 + l32;
-                if (p < P && k < K) pw[(int64_t)p * K + k] = acc[i][j][r];
-                any[r & 3] += acc[i][j][r];
-            }
-    if (__builtin_expect(nan_among(any), 0)) {                              // those of this lane that are NaN, read back where they were stored
+            for (int e = 0; e < MT * NT * 16; ++e) acc[e / (NT * 16)][e / 16 % NT][e & 15] += red[e * WAVES * 64];
+        }
+    }
+    if (part == 0) {
+        float* pw = part_w + chunk * (int64_t)P * K;
+        f32x4 any = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+            for (int j = 0; j < NT; ++j)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const int p = p0 + (wm * MT + i) * 32 + acc_row(r, half), k = k0 + (wn * NT + j) * 32 + l32;
+                    if (p < P && k < K) pw[(int64_t)p * K + k] = acc[i][j][r];
+                    any[r & 3] += acc[i][j][r];
+                }
+        if (__builtin_expect(nan_among(any), 0)) {                              // those of this lane that are NaN, read back where they were stored
 #pragma unroll 1
-        for (int e = 0; e < MT * NT * 16; ++e) {
-            const int p = p0 + (wm * MT + e / (NT * 16)) * 32 + acc_row(e & 15, half), k = k0 + (wn * NT + e / 16 % NT) * 32 + l32;
-            if (p >= P || k >= K) continue;
-            const float v = pw[(int64_t)p * K + k];
-            if (v != v) pw[(int64_t)p * K + k] = plain_products(dy + begin * P + p, P, x + begin * K + k, K, 0, end - begin)[0];
+            for (int e = 0; e < MT * NT * 16; ++e) {
+                const int p = p0 + (wm * MT + e / (NT * 16)) * 32 + acc_row(e & 15, half), k = k0 + (wn * NT + e / 16 % NT) * 32 + l32;
+                if (p >= P || k >= K) continue;
+                const float v = pw[(int64_t)p * K + k];
+                if (v != v) pw[(int64_t)p * K + k] = plain_products(dy + begin * P + p, P, x + begin * K + k, K, 0, end - begin)[0];
+            }
         }
     }
-    if (sums_here) {
-        // unit u holds rows of chunk u / (BM / 2) of its column pair: the chunks of a pair are added in order
+    if (part_b && k0 == 0) {
+        // unit u of dY holds 8 rows u / (BM / 2) of its column pair: those of a pair are added in order
         __syncthreads();
         float* red = reinterpret_cast<float*>(lds);
-#pragma unroll
-        for (int i = 0; i < UA; ++i) {
-            const int u = threadIdx.x + i * THREADS;
-            if (A_UNITS % THREADS == 0 || u < A_UNITS) red[u * 2] = bs[i][0], red[u * 2 + 1] = bs[i][1];
-        }
+        if (of_a && own == unit) red[(part * A_UNITS + unit) * 2] = bs[0], red[(part * A_UNITS + unit) * 2 + 1] = bs[1];
         __syncthreads();
         for (int c = threadIdx.x; c < BM; c += THREADS) {
             float s = 0.f;
 #pragma unroll
-            for (int q = 0; q < KC; ++q) s += red[(q * (BM / 2) + c / 2) * 2 + (c & 1)];
+            for (int q = 0; q < 2 * WK; ++q) s += red[(q * (BM / 2) + c / 2) * 2 + (c & 1)];
             if (p0 + c < P) part_b[chunk * P + p0 + c] = s;
         }
     }
@@ -1168,9 +1149,11 @@ static WgradPlan wgrad_plan(int64_t N, int P, int K, int bk, int bm, int bn, int
 // rows up to which one launch of 32 x 32 tiles beats row chunks and their sums (284 rows 384 -> 1152: 19 us in chunks)
 constexpr int64_t WGRAD_SMALL_ROWS = 1024;
 // Tiles of dW.  fp32: by the columns it has, since a tile wider than dW works on copies of its last columns.
-//   128 x 192 from 192 columns of X on (35 569 rows 192 -> 576: 91 and 78 us with 96 x 96), 64 x 192 where dY has at most 64;
-//   192 x 64 and 64 x 64 up to 64 columns of X (112 700 rows 48 -> 144 and 48 -> 48: 32 and 20 us, 39 on average with 96 x 96);
-//   96 x 96 between, with more workgroups per compute unit.
+//   from 192 columns of X on 128 x 192, and 96 x 192 where that takes no more tiles (35 569 rows 192 -> 576: 64 us, with 96 x 192 61
+//   but sums a fifth longer and 8 % more rounding; before 71; 192 -> 768 73 and 78, before 82; 192 -> 192 with 96 x 192 30, before
+//   39; 768 -> 192 78, before 97); 64 x 192 where dY has at most 64 (112 700 rows 192 -> 48: 35 us, before 40);
+//   192 x 64 and 64 x 64 up to 64 columns of X (112 700 rows 48 -> 144 and 48 -> 48: 36 and 21 us, before 39 and 26);
+//   128 x 96 between (75 000 rows 144 -> 144: 55 us, with 96 x 96 before 64).
 // 16 bit: 96 x 96 (219 000 rows 96 -> 288: 39 us; 192 x 192 tiles 58, 192 x 96 44); 192 x 192 where dW has at least 48 such tiles
 //   and the rows are many, so that half the bytes pass from L2 (8119 rows 768 -> 2304: 69 us and 57, 768 -> 3072 80 and 61;
 //   2000 rows 768 -> 2304 25 and 26; 9000 rows 384 -> 1536 30 either way).
@@ -1182,9 +1165,9 @@ static WgradTile wgrad_tile(int dtype, int64_t N, int P, int K) {
         if (N >= 4096 && P % 192 == 0 && K % 192 == 0 && (int64_t)P * K >= 48 * 192 * 192) return {192, 192, 1};
         return {96, 96, 3};
     }
-    if (K >= 192) return P <= 64 ? WgradTile{64, 192, 2} : WgradTile{128, 192, 2};
-    if (K <= 64) return P <= 64 ? WgradTile{64, 64, 4} : WgradTile{192, 64, 2};
-    return {96, 96, 4};
+    if (K >= 192) return P <= 64 ? WgradTile{64, 192, 2} : (P + 127) / 128 < (P + 95) / 96 ? WgradTile{128, 192, 1} : WgradTile{96, 192, 1};
+    if (K <= 64) return P <= 64 ? WgradTile{64, 64, 3} : WgradTile{192, 64, 1};
+    return {128, 96, 1};
 }
 static WgradPlan wgrad_plan(int dtype, int64_t N, int P, int K) {
     const WgradTile t = wgrad_tile(dtype, N, P, K);
@@ -1211,6 +1194,16 @@ static int launch_wgrad_as(F* k, int threads, size_t lds, const WgradPlan& pl, c
     return launch_ok("dense weight gradient, sums");
 }
 
+// fp32: `parts` row groups of two buffers of (column tiles) x 3 planes
+template <auto* KERNEL, typename TO>
+static int launch_wgrad_f32(int waves, int parts, const WgradTile& t, const WgradPlan& pl, const void* dy, const void* x, int64_t N, int P, int K, void* dw,
+                            void* db, float* ws, hipStream_t s) {
+    const size_t lds = 2 * (size_t)parts * ((t.bm + t.bn) / 32) * 3 * 1024;
+    static const hipError_t configured = hipFuncSetAttribute(reinterpret_cast<const void*>(KERNEL), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    SSWIN_HIP(configured);
+    return launch_wgrad_as<float, TO>(KERNEL, waves * 64, lds, pl, dy, x, N, P, K, dw, db, ws, s);
+}
+
 template <typename T, typename TO>
 static int launch_wgrad(const void* dy, const void* x, int64_t N, int P, int K, void* dw, void* db, float* ws, hipStream_t s) {
     if (N <= WGRAD_SMALL_ROWS) {
@@ -1222,12 +1215,12 @@ static int launch_wgrad(const void* dy, const void* x, int64_t N, int P, int K, 
     if constexpr (Op<T>::PL == 3) {
         const WgradPlan pl = wgrad_plan(SSWIN_F32, N, P, K);
         const WgradTile t = wgrad_tile(SSWIN_F32, N, P, K);
-        const size_t lds = 2 * (size_t)((t.bm + t.bn) / 32) * 3 * 1024;                                  // two buffers of (row tiles) x 3 planes
-        if (t.bm == 128) return launch_wgrad_as<T, TO>(dense_wgrad_kernel<2, 2, 2, 3, 2>, 256, lds, pl, dy, x, N, P, K, dw, db, ws, s);
-        if (t.bn == 192) return launch_wgrad_as<T, TO>(dense_wgrad_kernel<2, 2, 1, 3, 2>, 256, lds, pl, dy, x, N, P, K, dw, db, ws, s);
-        if (t.bm == 192) return launch_wgrad_as<T, TO>(dense_wgrad_kernel<3, 1, 2, 2, 2>, 192, lds, pl, dy, x, N, P, K, dw, db, ws, s);
-        if (t.bm == 64) return launch_wgrad_as<T, TO>(dense_wgrad_kernel<2, 1, 1, 2, 3>, 128, lds, pl, dy, x, N, P, K, dw, db, ws, s);
-        return launch_wgrad_as<T, TO>(dense_wgrad_kernel<3, 1, 1, 3, 3>, 192, lds, pl, dy, x, N, P, K, dw, db, ws, s);
+        if (t.bm == 128 && t.bn == 192) return launch_wgrad_f32<dense_wgrad_kernel<2, 3, 2, 2, 2, 3>, TO>(12, 2, t, pl, dy, x, N, P, K, dw, db, ws, s);
+        if (t.bm == 96) return launch_wgrad_f32<dense_wgrad_kernel<3, 2, 2, 1, 3, 3>, TO>(12, 2, t, pl, dy, x, N, P, K, dw, db, ws, s);
+        if (t.bn == 192) return launch_wgrad_f32<dense_wgrad_kernel<2, 2, 1, 1, 3, 2>, TO>(4, 1, t, pl, dy, x, N, P, K, dw, db, ws, s);
+        if (t.bm == 192) return launch_wgrad_f32<dense_wgrad_kernel<6, 1, 2, 1, 2, 3>, TO>(12, 2, t, pl, dy, x, N, P, K, dw, db, ws, s);
+        if (t.bm == 64) return launch_wgrad_f32<dense_wgrad_kernel<2, 1, 2, 1, 2, 3>, TO>(4, 2, t, pl, dy, x, N, P, K, dw, db, ws, s);
+        return launch_wgrad_f32<dense_wgrad_kernel<4, 1, 3, 1, 3, 3>, TO>(12, 3, t, pl, dy, x, N, P, K, dw, db, ws, s);
     } else {
         constexpr size_t lds = 3 * 2 * 32 * 192;                         // three stages of two tiles of 32 x 96
         const WgradPlan pl = wgrad_plan(SSWIN_F16, N, P, K);

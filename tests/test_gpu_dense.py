@@ -105,6 +105,22 @@ def test_dense_weight_gradient(N, P, K, dtype, out):
     assert torch.equal(results[0][0], results[1][0]) and torch.equal(results[0][1], results[1][1])       # fixed order of the sums
 
 
+@pytest.mark.parametrize("N", [1025, 1033, 1057, 4111])
+@pytest.mark.parametrize("P,K", [(96, 384), (112, 192), (128, 208), (400, 192), (64, 192), (192, 64), (80, 48), (64, 64), (16, 16), (144, 144), (48, 80)])
+def test_fp32_weight_gradient_at_the_edges_of_its_tiles(N, P, K):
+    """Every tile of dW, with columns that end inside one and rows that end inside the row groups of a step."""
+    from sparseswin3d_amd import _lib
+    lib = _lib.load()
+    gen = torch.Generator().manual_seed(N + P + K)
+    dy, x = _rand(gen, N, P), _rand(gen, N, K)
+    dw, db = (torch.full(s, float("nan"), device="cuda") for s in ((P, K), (P,)))
+    nb = lib.sswin_dense_weight_grad_workspace_bytes(0, N, P, K)
+    ws = torch.empty(nb, dtype=torch.uint8, device="cuda")
+    _lib.check(lib.sswin_dense_weight_grad(0, 0, _ptr(dy), _ptr(x), N, P, K, _ptr(dw), _ptr(db), _ptr(ws), nb, _stream()))
+    _check(dw, dy.double().T @ x.double(), dy.double().abs().T @ x.double().abs(), torch.float32, "dW")
+    _check(db, dy.double().sum(0), dy.double().abs().sum(0), torch.float32, "db")
+
+
 @pytest.mark.parametrize("sizes", [(8,), (96 * 288, 288, 96 * 96, 96, 8, 16, 2056, 24)])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_cast_parts(sizes, dtype):
