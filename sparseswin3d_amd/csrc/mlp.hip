@@ -14,8 +14,8 @@
 // slope, du) goes through a tile of LDS per wavefront, so that it is touched in runs of 64 or 128 bytes (16 bits straight from
 // the accumulators, runs of 32 bytes: 225 000 rows fp16 48 channels 95 us, through the tile 69).
 //
-// Microseconds, two launches and one.  225 700 rows fp32 96 channels: forward 318 and 273, backward 277 and 251 (traffic alone at copy
-// rate 187 and 170; without the matrix instructions 205 and 212: rounds of 256 workgroups, the last one partly full).  fp16 48
+// Microseconds, two launches and one.  225 700 rows fp32 96 channels: forward 326 and 275, backward 294 and 246 (traffic alone at copy
+// rate 187 and 170; the matrix instructions alone about 120 at the clock they run at on such data).  fp16 48
 // channels, 225 000 rows: 89 and 69, 55 and 43 (55 and 38).  bf16 96 channels, inference, 112 700 rows: 66 and 46 (13; GELU on the
 // vector units 21).
 #include <algorithm>
@@ -42,6 +42,8 @@ struct MlpArgs {
     void* h;                   // g or du [N, hidden]
     void* slope;               // forward: [N, hidden]
     void* y;                   // [N, D]
+    int64_t full;              // workgroups whose wavefronts all have 32 tokens; in those behind them the first `some` have
+    int some;
 };
 
 constexpr int MLP_LDS = 160 * 1024;
@@ -189,7 +191,8 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(OCC,
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, half = lane >> 5, l32 = lane & 31;
     float* const bias = reinterpret_cast<float*>(lds + 2 * PIECES * 64); // [hidden] and [D]
     u32x4* const tiles = L::SHARED ? lds + wave * 256 : lds + 2 * PIECES * 64 + (g.hidden + D) / 4 + wave * L::OWN;
-    const int64_t row0 = tile_row((int64_t)blockIdx.x * WAVES + wave, g.N), plane = (int64_t)g.hidden * D;
+    const int64_t behind = (int64_t)blockIdx.x - g.full, row0 = tile_row(behind < 0 ? (int64_t)blockIdx.x * WAVES + wave : g.full * WAVES + behind * g.some + wave, g.N);
+    const int64_t plane = (int64_t)g.hidden * D;
     const uint32_t lane_a = (uint32_t)(hidden_of(l32) * D + half * 8);
     auto request = [&](int step) {
         const uint32_t to = lds_address(lds) + (uint32_t)(step & 1) * PIECES * 1024;
@@ -206,6 +209,16 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(OCC,
     const int steps = g.hidden / 32;
     request(0);
     if constexpr (MODE != MLP_BACKWARD) stage_biases<T>(g, D, bias);
+    if (behind >= 0 && wave >= g.some) {                                 // without tokens: only brings A and B
+        wait_copies<0>();
+        for (int step = 0; step < steps; ++step) {
+            block_barrier();
+            if (step + 1 < steps) request(step + 1);
+            wait_copies<0>();
+        }
+        if constexpr (L::SHARED) block_barrier();
+        return;
+    }
     u32x4 x[KS][PL];
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) planes_at<T>(static_cast<const T*>(g.x) + (row0 + l32) * D + ks * 16 + half * 8, x[ks]);
@@ -314,11 +327,18 @@ template <typename K> static int allow_all_lds(K* k) {
     SSWIN_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, MLP_LDS));
     return 0;
 }
-template <typename T, typename TO, int D, int MODE, int WAVES, int OCC> static int launch_mlp_as(const MlpArgs& g, hipStream_t s) {
+template <typename T, typename TO, int D, int MODE, int WAVES, int OCC> static int launch_mlp_as(MlpArgs g, hipStream_t s) {
     auto* k = mlp_kernel<T, TO, D, MODE, WAVES, OCC>;
     static const int configured = allow_all_lds(k);
     if (configured) return configured;
-    hipLaunchKernelGGL(k, dim3((unsigned)((g.N + WAVES * 32 - 1) / (WAVES * 32))), dim3(WAVES * 64), (MlpLds<T, D, MODE, WAVES>::bytes(g.hidden)), s, g);
+    // One workgroup of 8 wavefronts fills a compute unit: the tokens behind the last full round are dealt to all of them, so that fewer
+    // wavefronts share a SIMD there.  (Smaller workgroups need no rule.)
+    const int64_t tiles = (g.N + 31) / 32, cus = device_cus();
+    g.full = WAVES == 8 ? tiles / (WAVES * cus) * cus : tiles / WAVES;
+    const int64_t rest = tiles - g.full * WAVES;
+    g.some = WAVES == 8 ? (int)((rest + cus - 1) / cus) : WAVES;
+    const int64_t blocks = g.full + (rest ? (rest + g.some - 1) / g.some : 0);
+    hipLaunchKernelGGL(k, dim3((unsigned)blocks), dim3(WAVES * 64), (MlpLds<T, D, MODE, WAVES>::bytes(g.hidden)), s, g);
     return launch_ok("mlp");
 }
 template <typename T, typename TO, int MODE> static int launch_mlp(const MlpArgs& g, int D, hipStream_t s) {
@@ -358,14 +378,13 @@ int sswin_mlp_supported(int dtype, int64_t N, int D, int hidden) {
 }
 
 // Where one launch is ahead of two.  16 bit: from 8192 rows on (8000 rows fp16 48 channels, forward and backward 25.0 -> 22.3 us, 4000
-// rows 17.6 -> 21.5; bf16 96 channels, inference, 19.8 -> 18.4 and 13.3 -> 18.3).  fp32: a round of workgroups on all compute units
-// takes about 62 us forward and backward alike, however full it is, so the rounds have to be three quarters full (60 000 rows 156 ->
-// 138 us, 90 000 (1.4 rounds) 238 -> 239, 112 700 309 -> 255, 225 700 595 -> 529).
+// rows 17.6 -> 21.5; bf16 96 channels, inference, 19.8 -> 18.4 and 13.3 -> 18.3).  fp32: a wavefront takes about 42 us forward and 35
+// backward alone on its SIMD, 75 and 67 with a second one, so from three wavefronts a compute unit on (forward and backward of 8192
+// rows 60 -> 78 us, 16 384 86 -> 85, 24 576 98 -> 91, 32 768 116 -> 100, 65 536 180 -> 145, 81 920 240 -> 228, 225 700 621 -> 521).
 int sswin_mlp_preferred(int dtype, int64_t N, int D, int hidden) {
     if (!sswin_mlp_supported(dtype, N, D, hidden)) return 0;
     if (dtype != SSWIN_F32) return N >= 8192;
-    const int64_t blocks = (N + 255) / 256, cus = device_cus();
-    return blocks * 4 >= (blocks + cus - 1) / cus * cus * 3;
+    return N > 2 * 32 * (int64_t)device_cus();
 }
 
 size_t sswin_mlp_workspace_bytes(int dtype, int D, int hidden, int backward) {
@@ -386,7 +405,7 @@ int sswin_mlp_forward(int dtype, int out_dtype, const void* x, int64_t N, int D,
         a = planes, b = planes + (size_t)3 * D * hidden;
         if (int rc = launch_weights<float>(w1, w2, false, D, hidden, planes, planes + (size_t)3 * D * hidden, s)) return rc;
     }
-    const MlpArgs g = {x, N, hidden, a, b, b1, b2, nullptr, residual, act, slope, y};
+    const MlpArgs g = {x, N, hidden, a, b, b1, b2, nullptr, residual, act, slope, y, 0, 0};
 #define MLP_RUN(T, TO) return act ? launch_mlp<T, TO, MLP_TRAIN>(g, D, s) : launch_mlp<T, TO, MLP_INFER>(g, D, s)
     if (dtype == SSWIN_F32 && out_dtype == SSWIN_F32) MLP_RUN(float, float);
     if (dtype == SSWIN_F16 && out_dtype == SSWIN_F16) MLP_RUN(__half, __half);
@@ -405,7 +424,7 @@ int sswin_mlp_backward(int dtype, const void* dy, int64_t N, int D, int hidden, 
                 "mlp_backward: pointers must be 16-byte aligned");
     hipStream_t s = static_cast<hipStream_t>(stream);
     uint16_t *a = static_cast<uint16_t*>(ws), *b = a + sswin_mlp_workspace_bytes(dtype, D, hidden, 1) / 4;
-    const MlpArgs g = {dy, N, hidden, a, b, nullptr, nullptr, slope, nullptr, du, nullptr, dx};
+    const MlpArgs g = {dy, N, hidden, a, b, nullptr, nullptr, slope, nullptr, du, nullptr, dx, 0, 0};
 #define MLP_RUN(T)                                                                     \
     do {                                                                               \
         if (int rc = launch_weights<T>(w2, w1, true, D, hidden, a, b, s)) return rc;   \

@@ -103,3 +103,11 @@ def test_mlp_refuses_what_it_does_not_take():
     for dtype, n, d, hidden in [(0, 31, 96, 384), (0, 64, 48, 192), (0, 64, 96, 400), (2, 64, 96, 32), (2, 64, 96, 100), (2, 64, 112, 448), (2, 64, 192, 768), (2, 64, 96, 1056), (3, 64, 96, 384)]:
         assert not lib.sswin_mlp_supported(dtype, n, d, hidden)
         assert lib.sswin_mlp_backward(dtype, None, n, d, hidden, None, None, None, None, None, None, 1 << 30, None) != 0
+
+
+# behind the last full round of workgroups of 256 rows the tiles of 32 are dealt to all compute units: none, one, two and seven a
+# workgroup, after no, one and two rounds
+@pytest.mark.parametrize("rounds,tiles,extra", [(1, 0, 0), (0, 1, 1), (0, 2, -1), (1, 1, 31), (1, 7, 0), (2, 0, 1)])
+def test_mlp_last_round(rounds, tiles, extra):
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    test_mlp_against_float64(torch.float32, 96, 64, 32 * cus * (8 * rounds + tiles) + extra)
