@@ -1077,6 +1077,8 @@ template <typename T, typename TO, int EPI, bool DOWN>
 static int launch_forward(const void* x, int64_t N, int K, const void* w, int P, const Epilogue& ep, float* ws, size_t ws_bytes, hipStream_t s) {
     const T* xp = static_cast<const T*>(x);
     const T* wp = static_cast<const T*>(w);
+    if constexpr (Op<T>::PL == 1 && EPI == EPI_NONE && !DOWN)
+        if (rows_once_takes(N, K, P)) return rows_once<T>(xp, N, K, wp, static_cast<const T*>(ep.bias), P, static_cast<T*>(ep.y), s);
     const int64_t few_blocks = (N + 31) / 32 * ((P + 31) / 32);
     Cut cut = cut_of(Op<T>::PL == 3 ? SSWIN_F32 : SSWIN_F16, N, K, P);
     if (cut.few && few_blocks < (1ll << 31)) {

@@ -298,6 +298,108 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(OCC,
     store_y<TO, D, MODE>(g, y, row0, bias + g.hidden, tiles);
 }
 
+// ------------------------------------------------------------------------------------------
+// y [N, P] = x [N, D] W^T + b for 16-bit rows and few input channels, the first half of the kernel above: a wavefront keeps its
+// 32 tokens of x in registers and forms y^T 32 columns at a time, so that a row of x is read once and by one workgroup (the tiles of
+// dense.hip read it once per 96 columns of y, and start anew for each).  Bound by the stores of y.  W passes through LDS a step of 32 columns at a time.
+// ------------------------------------------------------------------------------------------
+// CT tiles of 32 columns a step; OWN: 16-byte pieces of a wavefront's 32 x 32 CT results
+template <int D, int CT, int WAVES> struct RowsOnceLds {
+    static constexpr int PIECES = D / 16 * CT, OWN = CT * 128;
+    static size_t bytes(int P) { return (size_t)2 * PIECES * 1024 + (size_t)WAVES * OWN * 16 + (size_t)(P + CT * 32 - 1) / (CT * 32) * CT * 128; }
+};
+template <typename T, int D, int CT, int WAVES, int OCC>
+__global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(OCC, OCC))) void rows_once_kernel(const T* __restrict__ x, int64_t N,
+                                                                                                     const T* __restrict__ w, const T* __restrict__ b, int P,
+                                                                                                     T* __restrict__ y) {
+    using L = RowsOnceLds<D, CT, WAVES>;
+    using H = HiddenTile<typename std::conditional<CT == 2, float, T>::type>;                             // rows of 64 or 128 bytes
+    constexpr int KS = D / 16, PIECES = L::PIECES;
+    extern __shared__ __attribute__((aligned(16))) u32x4 lds[];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, half = lane >> 5, l32 = lane & 31;
+    u32x4* const tile = lds + 2 * PIECES * 64 + wave * L::OWN;
+    float* const bias = reinterpret_cast<float*>(lds + 2 * PIECES * 64 + WAVES * L::OWN);
+    const int64_t row0 = tile_row((int64_t)blockIdx.x * WAVES + wave, N);
+    const int steps = (P + CT * 32 - 1) / (CT * 32);
+    auto request = [&](int step) {
+#pragma unroll
+        for (int q = 0; q < (PIECES + WAVES - 1) / WAVES; ++q) {
+            const int p = q * WAVES + wave;                              // uniform in the wavefront
+            if (PIECES % WAVES != 0 && p >= PIECES) break;
+            copy_to_lds(w + (int64_t)min((step * CT + p / KS) * 32 + hidden_of(l32), P - 1) * D + p % KS * 16 + half * 8,
+                        lds_address(lds) + (uint32_t)((step & 1) * PIECES + p) * 1024);
+        }
+    };
+    request(0);
+    for (int e = threadIdx.x; e < steps * CT * 32; e += WAVES * 64) bias[e] = b && e < P ? to_acc(b[e]) : 0.f;
+    u32x4 rows[KS];
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) rows[ks] = *reinterpret_cast<const u32x4*>(x + (row0 + l32) * D + ks * 16 + half * 8);
+    const int col = H::mem_col() * (CT == 2 ? 2 : 1);                    // pieces of eight values either way
+    const int64_t mem = (row0 + H::mem_row()) * P + col;
+    wait_copies<0>();
+    for (int step = 0; step < steps; ++step) {
+        block_barrier();                                                 // this buffer is there, the other one is free
+        if (step + 1 < steps) request(step + 1);
+        const u32x4* const pieces = lds + (step & 1) * PIECES * 64 + lane;
+        f32x16 z[CT];
+#pragma unroll
+        for (int t = 0; t < CT; ++t) {
+            z[t] = f32x16{0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) z[t] = Op<T>::mfma(pieces[(t * KS + ks) * 64], rows[ks], z[t]);
+        }
+#pragma unroll
+        for (int t = 0; t < CT; ++t)
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+                const f32x4* const b8 = reinterpret_cast<const f32x4*>(bias + (step * CT + t) * 32 + s * 16 + half * 8);
+                const f32x4 b01[2] = {b8[0], b8[1]};
+                float v[8];
+#pragma unroll
+                for (int e = 0; e < 8; ++e) v[e] = z[t][s * 8 + e] + b01[e / 4][e % 4];
+                u32x4 p[1];
+                planes_of<T>(v, p);
+                tile[H::slot(l32, t * 4 + s * 2 + half)] = p[0];
+            }
+        __builtin_amdgcn_wave_barrier();
+        u32x4 out[H::MOVES];
+#pragma unroll
+        for (int i = 0; i < H::MOVES; ++i) out[i] = tile[i * 64 + lane];
+        if (step * CT * 32 + col < P)                                    // 16 columns at least: the stores are counted
+#pragma unroll
+            for (int i = 0; i < H::MOVES; ++i) store_counted(y + mem + (int64_t)i * H::STEP_ROWS * P + step * CT * 32, out[i]);
+        __builtin_amdgcn_wave_barrier();
+        if (step + 1 < steps) wait_copies<H::MOVES>();                   // all but the stores of this step
+    }
+}
+template <typename K> static int allow_all_lds(K* k) {
+    SSWIN_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, MLP_LDS));
+    return 0;
+}
+template <typename T, int D, int CT, int WAVES, int OCC> static int launch_rows_once(const T* x, int64_t N, const T* w, const T* b, int P, T* y, hipStream_t s) {
+    auto* k = rows_once_kernel<T, D, CT, WAVES, OCC>;
+    static const int configured = allow_all_lds(k);
+    if (configured) return configured;
+    hipLaunchKernelGGL(k, dim3((unsigned)((N + WAVES * 32 - 1) / (WAVES * 32))), dim3(WAVES * 64), (RowsOnceLds<D, CT, WAVES>::bytes(P)), s, x, N, w, b, P, y);
+    return launch_ok("rows once");
+}
+// The rows from which this is ahead of the tiles of dense.hip (microseconds, tiles and here).  bf16 96 -> 288: 8000 rows 7.0 and 8.0,
+// 16 000 12.0 and 8.8, 112 700 23.1 and 17.5, 445 000 108 and 83 (67 at copy rate).  fp16 48 -> 144: 4000 4.0 and 4.6, 8000 4.9 and 4.8,
+// 225 000 25.0 and 19.1 (17).  bf16 192 -> 576: 37 000 22.7 and 24.2, 50 000 28.5 and 25.3, 147 000 64.7 and 55.2 (44): with fewer rows a
+// compute unit has too few workgroups to hide where each one starts.  With GELU 192 -> 768 loses up to 100 000 rows.
+bool rows_once_takes(int64_t N, int D, int P) {
+    return N < (1ll << 31) && P <= 2048 && ((D == 48 && N >= 8000) || (D == 96 && N >= 16000) || (D == 192 && N >= 50000));
+}
+// 64 columns a step (runs of 128 bytes), with 192 channels 32, for the place their pieces of W take; 445 000 rows 96 -> 288: 92 us with 32
+template <typename T> int rows_once(const T* x, int64_t N, int D, const T* w, const T* b, int P, T* y, hipStream_t s) {
+    if (D == 48) return launch_rows_once<T, 48, 2, 4, 5>(x, N, w, b, P, y, s);
+    if (D == 96) return launch_rows_once<T, 96, 2, 8, 4>(x, N, w, b, P, y, s);
+    return launch_rows_once<T, 192, 1, 8, 4>(x, N, w, b, P, y, s);
+}
+template int rows_once<__half>(const __half*, int64_t, int, const __half*, const __half*, int, __half*, hipStream_t);
+template int rows_once<__hip_bfloat16>(const __hip_bfloat16*, int64_t, int, const __hip_bfloat16*, const __hip_bfloat16*, int, __hip_bfloat16*, hipStream_t);
+
 // A and B as the kernel reads them: fp32 weights as planes of their pieces, weights of the backward turned.  A thread per pair of
 // neighbours of a row.
 template <typename T>
@@ -323,10 +425,6 @@ __global__ __launch_bounds__(256) void mlp_weights_kernel(const T* __restrict__ 
     }
 }
 
-template <typename K> static int allow_all_lds(K* k) {
-    SSWIN_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, MLP_LDS));
-    return 0;
-}
 template <typename T, typename TO, int D, int MODE, int WAVES, int OCC> static int launch_mlp_as(MlpArgs g, hipStream_t s) {
     auto* k = mlp_kernel<T, TO, D, MODE, WAVES, OCC>;
     static const int configured = allow_all_lds(k);

@@ -84,6 +84,22 @@ def test_dense_forward_and_input_gradient(N, K, P, dtype, out):
     _check(y, pre + extra.double(), mag + extra.double().abs(), out, "residual")
 
 
+# rows at the line from which x is read once and in its last, moved tile; columns that end inside a step of 64 or 32
+@pytest.mark.parametrize("K,N", [(48, 7999), (48, 8000), (48, 8001), (48, 8095), (96, 16000), (96, 16257), (192, 50000), (192, 50017)])
+@pytest.mark.parametrize("P", [16, 48, 64, 144, 240])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=["fp16", "bf16"])
+def test_dense_forward_that_reads_its_rows_once(K, N, P, dtype):
+    from sparseswin3d_amd import _lib
+    lib = _lib.load()
+    gen = torch.Generator().manual_seed(N + 3 * K + 7 * P)
+    x, w, b = _rand(gen, N, K, dtype=dtype), (_rand(gen, P, K, spread=1) / K ** 0.5).to(dtype), _rand(gen, P, dtype=dtype)
+    pre, mag = x.double() @ w.double().T, x.double().abs() @ w.double().abs().T
+    for bias in (b, None):
+        add = 0 if bias is None else bias.double()
+        y, _ = _forward(lib, _lib, x, w, bias, 0, PLAIN, None, dtype)
+        _check(y, pre + add, mag + abs(add), dtype, "plain")
+
+
 @pytest.mark.parametrize("N,P,K", [(1, 16, 16), (17, 144, 48), (1024, 96, 96), (1025, 48, 208), (1100, 288, 96), (9001, 208, 192), (70001, 48, 144),
                                    (2000, 16, 16), (30001, 64, 48), (40001, 144, 48), (1100, 400, 64), (3003, 64, 400), (4501, 2304, 768)])
 @pytest.mark.parametrize("dtype,out", [(torch.float32, torch.float32), (torch.bfloat16, torch.bfloat16), (torch.float16, torch.float32)],
