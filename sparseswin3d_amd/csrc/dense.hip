@@ -1057,8 +1057,10 @@ static int launch_rows16(const T* x, int64_t N, int K, const T* w, int P, int ks
 
 // How a product is cut.
 //   few rows: 32 x 32 tiles while the workgroups of the larger tiles would leave most of the chip idle.  fp32: below 150 tiles of
-//     128 x 96.  16 bit: the tiles' own time grows with the reduction, so the line is tiles x K: 500 rows 768 -> 768 (24 576)
-//     7.8 us against 12.2, 1364 rows 768 -> 768 (67 584) 15.5 against 12.6, 2000 rows 1152 -> 384 (73 728) 15.5 against 13.8.
+//     128 x 96.  16 bit: their time grows with tiles x K, that of the larger tiles starts at 6 us and grows with K: 500 rows
+//     768 -> 768 (24 576) 7.8 us against 12.2, 1364 rows (67 584) 15.5 against 12.6; 2000 rows 384 -> 384 (24 576) 7.4 and 9.7, 4000
+//     (49 152) 12.7 and 10.0; 6000 rows 192 -> 192 (18 048) 7.2 and 7.1, 16 000 (48 000) 14.2 and 7.8; 24 000 rows 96 -> 96 with a
+//     residual (18 048) 8.3 and 8.7, 60 000 (45 024) 16.3 and 12.7; 60 000 rows 48 -> 48, input gradient (22 512) 14.6 and 8.1.
 //   ksplit (16 bit): shares of the reduction, each at least 576 long, while the tiles alone do not fill the chip: 1364 rows
 //     3072 -> 768 (88 tiles) 36 us with one share, 24 with two, 23 with four; 2729 rows (176 tiles) 37, 33 and 36.
 struct Cut {
@@ -1068,7 +1070,7 @@ struct Cut {
 static Cut cut_of(int dtype, int64_t N, int K, int P) {
     const int64_t tiles = (N + 127) / 128 * ((P + 95) / 96);
     if (dtype == SSWIN_F32) return {tiles < 150, 1};
-    if (tiles * K <= 50000) return {true, 1};
+    if (tiles * K <= std::min(50000, 12000 + 50 * K)) return {true, 1};
     const int64_t shares = std::min<int64_t>({4, 400 / tiles, K / 576});
     return {false, (int)std::max<int64_t>(shares, 1)};
 }
@@ -1319,8 +1321,9 @@ int sswin_cast_parts(int dtype, const void* const* src, const int64_t* sizes, in
 }
 
 int sswin_dense_backward_small_supported(int dtype, int64_t N, int P, int K) {
-    // where both gradients would take their few-rows kernels
-    return N > 0 && N <= WGRAD_SMALL_ROWS && sswin_dense_supported(dtype, P, K) && cut_of(dtype, N, P, K).few;
+    // where both gradients would take their few-rows kernels; 16 bit: also where dX alone would not, since it saves a launch
+    if (N <= 0 || N > WGRAD_SMALL_ROWS || !sswin_dense_supported(dtype, P, K)) return 0;
+    return dtype == SSWIN_F32 ? cut_of(dtype, N, P, K).few : (N + 127) / 128 * ((K + 95) / 96) * P <= 50000;
 }
 
 int sswin_dense_backward_small(int dtype, int out_dtype, int epilogue, const void* dy, const void* x, const void* w, int64_t N, int P, int K,

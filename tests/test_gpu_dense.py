@@ -100,6 +100,22 @@ def test_dense_forward_that_reads_its_rows_once(K, N, P, dtype):
         _check(y, pre + add, mag + abs(add), dtype, "plain")
 
 
+# 16 bit: the last rows of the few-rows kernel and the first of the tiles behind it, with a residual and as an input gradient
+@pytest.mark.parametrize("N", [5376, 5377])
+def test_dense_forward_where_the_tiles_take_over(N):
+    from sparseswin3d_amd import _lib
+    lib = _lib.load()
+    K, P, dtype = 288, 144, torch.bfloat16                               # 42 row tiles x 2 x 288 = 24 192, 43: 24 768; the line: 26 400
+    gen = torch.Generator().manual_seed(N)
+    for n in (N, N + 384, N + 512):                                      # 45 row tiles: 25 920, 46: 26 496
+        x, w, b, extra = _rand(gen, n, K, dtype=dtype), (_rand(gen, P, K, spread=1) / K ** 0.5).to(dtype), _rand(gen, P, dtype=dtype), _rand(gen, n, P, dtype=dtype)
+        pre, mag = x.double() @ w.double().T, x.double().abs() @ w.double().abs().T
+        y, _ = _forward(lib, _lib, x, w, b, 0, RESIDUAL, extra, dtype)
+        _check(y, pre + b.double() + extra.double(), mag + b.double().abs() + extra.double().abs(), dtype, "residual")
+        dx, _ = _forward(lib, _lib, x, w.T.contiguous(), None, 1, PLAIN, None, dtype)
+        _check(dx, pre, mag, dtype, "input gradient")
+
+
 @pytest.mark.parametrize("N,P,K", [(1, 16, 16), (17, 144, 48), (1024, 96, 96), (1025, 48, 208), (1100, 288, 96), (9001, 208, 192), (70001, 48, 144),
                                    (2000, 16, 16), (30001, 64, 48), (40001, 144, 48), (1100, 400, 64), (3003, 64, 400), (4501, 2304, 768)])
 @pytest.mark.parametrize("dtype,out", [(torch.float32, torch.float32), (torch.bfloat16, torch.bfloat16), (torch.float16, torch.float32)],
