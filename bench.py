@@ -520,6 +520,7 @@ def kernel_table(wl, reps=20, only=None):
     # ---- the window-resident kernels (what the step runs for heads of 32 channels), in the workload's dtype ----
     qkv_r = qkv.reshape(N, 3 * D).to(tdt).contiguous()
     bias_r = torch.randn(H, b["n"], b["n"], device=dev)
+    bias_r = torch.stack([bias_r, bias_r.transpose(1, 2)]).contiguous()  # and turned, as the step has it
     out_r = torch.empty(N, D, device=dev, dtype=tdt)
     dqkv_r = torch.empty_like(qkv_r)
     ds_r = torch.empty(A, device=dev)
@@ -531,9 +532,9 @@ def kernel_table(wl, reps=20, only=None):
     Er = es * E // 4                                         # E in units of four bytes of token values
 
     def r_fwd():
-        _lib.check(lib.sswin_window_attention_forward(code, ptr(tp.tasks), tp.g_cap, tp.bucket_counts, ptr(tp.tokens), N, H,
-                                                      hd, *qa, C.c_float(0.17), ptr(bias_r), b["n"], mask_p, nmw,
-                                                      ptr(out_r), D, 0, ptr(lse), stream))
+        _lib.check(lib.sswin_window_attention_forward_pair(code, ptr(tp.tasks), tp.g_cap, tp.bucket_counts, ptr(tp.tokens), N, H,
+                                                           hd, *qa, C.c_float(0.17), ptr(bias_r), b["n"], mask_p, nmw,
+                                                           ptr(out_r), D, 0, ptr(lse), stream))
 
     # The step asks for all gradients at once (sides = 3): one launch in which groups of at most
     # 64 tokens get dQ from their key-side tasks and only the larger groups have query-side tasks.
@@ -546,7 +547,7 @@ def kernel_table(wl, reps=20, only=None):
 
     def r_bwd(sides, counts=None):
         counts = tp.bucket_counts if counts is None else (C.c_int64 * 4)(*counts)
-        return lambda: _lib.check(lib.sswin_window_attention_backward(
+        return lambda: _lib.check(lib.sswin_window_attention_backward_pair(
             code, ptr(tp.tasks), tp.g_cap, counts, ptr(tp.tokens), N, H, hd, *qa, C.c_float(0.17), ptr(bias_r),
             b["n"], mask_p, nmw, ptr(out_r), D, 0, ptr(up_r), D, 0, ptr(lse), *da, ptr(ds_r), sides, stream))
 
@@ -931,10 +932,10 @@ def trace_summary(dirs, out_name, command):
         if not paths:
             sys.exit(f"no *kernel_stats.csv under {d}")
         rows = list(csv.DictReader(open(paths[0])))
-        # one backward launch per attention call: the resident kernels', the flash kernels' query side or, on the fused path, the
+        # one backward launch per attention call: the resident kernels', the flash kernels' key side or, on the fused path, the
         # score gradient's
         bwd = sum(int(r["Calls"]) for r in rows if "_bwd_all_kernel" in r["Name"]) or \
-            sum(int(r["Calls"]) for r in rows if "flash_backward_q_kernel" in r["Name"]) or \
+            sum(int(r["Calls"]) for r in rows if "flash_backward_kv_kernel" in r["Name"]) or \
             sum(int(r["Calls"]) for r in rows if "fused_sq_kernel<" in r["Name"] and ", 2>" in r["Name"])
         steps = max(bwd // 2, 1)
         if bwd == 0:                                 # the forward-only encoder: four attention launches per pass
