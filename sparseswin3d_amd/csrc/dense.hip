@@ -3,9 +3,9 @@
 // product folded into its last step: bias, GELU and its derivative, the product with that derivative, the residual sum.
 //
 // Products run on the 16-bit matrix cores with fp32 accumulation.  fp32 operands are split exactly into three bf16
-// pieces (x = h + m + l, split2 below) and a product is the sum of the six piece products that
+// pieces (x = h + m + l, split2 of dense_operand.hpp) and a product is the sum of the six piece products that
 // weigh at least 2^-16 of the leading one; what is dropped is below 2^-23 of the product.  Infinities and NaN give what they give
-// in plain fp32 (plain_products below).
+// in plain fp32 (plain_products).
 //
 // dense_rows_kernel (fp32): a workgroup of WM wavefronts owns BM = 32 MT WM rows and 96 columns.  Both operands pass through
 // registers, where they are split, into LDS in matrix operand order, [row tile][plane][lane] pieces of 16 bytes, so that every
@@ -29,36 +29,6 @@
 
 namespace sswin {
 namespace dense {
-
-// Pieces of an infinity hold a NaN, and so does every result one takes part in, as do pieces whose sums leave the range: fp32
-// results that come out NaN are formed again from the operands in plain fp32, in the order of the reduction, until they are
-// NaN there as well.
-__device__ __forceinline__ bool nan_among(const f32x4& v) {
-    const float t = (v[0] + v[1]) + (v[2] + v[3]);                       // infinities of both signs too: formed again for nothing
-    return t != t;
-}
-// sum over i < n of a[i a_step] b[i b_step + e b_next], e < 4; four steps of the reduction in flight
-__device__ __forceinline__ f32x4 plain_products(const float* a, int64_t a_step, const float* b, int64_t b_step, int64_t b_next, int64_t n) {
-    f32x4 s = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll 1
-    for (int64_t i0 = 0; i0 < n && (s[0] == s[0] || s[1] == s[1] || s[2] == s[2] || s[3] == s[3]); i0 += 4) {
-        float v[4];
-        f32x4 w[4];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const int64_t i = i0 + q < n ? i0 + q : n - 1;
-            v[q] = a[i * a_step];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) w[q][e] = b[i * b_step + e * b_next];
-        }
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-            if (i0 + q < n)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) s[e] = fmaf(v[q], w[q][e], s[e]);
-    }
-    return s;
-}
 
 // ------------------------------------------------------------------------------------------
 // Raw values of a unit on their way from memory to LDS.

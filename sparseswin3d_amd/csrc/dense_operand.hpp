@@ -76,6 +76,36 @@ __device__ __forceinline__ void planes_of(const float (&v)[8], u32x4 (&out)[Op<T
     }
 }
 
+// Pieces of an infinity hold a NaN, and so does every result one takes part in, as do pieces whose sums leave the range: fp32
+// results that come out NaN are formed again from the operands in plain fp32, in the order of the reduction, until they are
+// NaN there as well.
+__device__ __forceinline__ bool nan_among(const f32x4& v) {
+    const float t = (v[0] + v[1]) + (v[2] + v[3]);                       // infinities of both signs too: formed again for nothing
+    return t != t;
+}
+// sum over i < n of a[i a_step] b[i b_step + e b_next], e < 4; four steps of the reduction in flight
+__device__ __forceinline__ f32x4 plain_products(const float* a, int64_t a_step, const float* b, int64_t b_step, int64_t b_next, int64_t n) {
+    f32x4 s = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+    for (int64_t i0 = 0; i0 < n && (s[0] == s[0] || s[1] == s[1] || s[2] == s[2] || s[3] == s[3]); i0 += 4) {
+        float v[4];
+        f32x4 w[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int64_t i = i0 + q < n ? i0 + q : n - 1;
+            v[q] = a[i * a_step];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) w[q][e] = b[i * b_step + e * b_next];
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            if (i0 + q < n)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) s[e] = fmaf(v[q], w[q][e], s[e]);
+    }
+    return s;
+}
+
 // 64 lanes x 16 bytes: lane l's piece lands at lds + 16 l
 __device__ __forceinline__ void copy_to_lds(const void* src, uint32_t lds) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(src) : "memory", "m0");

@@ -35,6 +35,7 @@ struct MlpArgs {
     int hidden;
     const uint16_t* a;         // [planes][hidden, D]
     const uint16_t* b;         // [planes][D, hidden]
+    const float *wa, *wb;      // fp32: what the pieces are of, forward [hidden, D] and [D, hidden], backward turned
     const void* bias_a;        // [hidden] or null
     const void* bias_b;        // [D] or null
     const void* factor;        // backward: slope [N, hidden]
@@ -171,8 +172,75 @@ template <typename T> __device__ __forceinline__ void stage_biases(const MlpArgs
 // a last ragged tile is moved back to end at row N, tiles behind it repeat it: rows stored twice hold the same bits
 __device__ __forceinline__ int64_t tile_row(int64_t t, int64_t N) { return t * 32 + 32 <= N ? t * 32 : N - 32; }
 
+// fp32: y where the pieces left NaN, again in plain fp32 as in dense.hip (plain_products), and the hidden values before it with what is
+// stored of them.  A hidden value that came out NaN makes every y of its token NaN, so y alone tells, once a launch.  Inference has
+// no hidden values in memory and forms all of these tokens again.
+template <int D, int MODE> __device__ __forceinline__ void plain_rows(const MlpArgs& g, int64_t row0, const float* bias, u32x4* tile, f32x16 (&y)[(D + 31) / 32]) {
+    constexpr int CT = (D + 31) / 32;
+    using H = HiddenTile<float>;
+    const int half = (threadIdx.x & 63) >> 5, l32 = threadIdx.x & 31;
+    const int64_t row = row0 + l32;
+    f32x16 p[CT];
+#pragma unroll
+    for (int j = 0; j < CT; ++j) p[j] = f32x16{0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+    wait_copies<0>();                                                    // the stores of this wavefront, read here
+#pragma unroll 1
+    for (int k0 = 0; k0 < g.hidden; k0 += 32) {
+#pragma unroll 1
+        for (int c = 0; c < 4; ++c) {
+            const int k = k0 + half * 16 + c * 4;
+            f32x4* const stored = reinterpret_cast<f32x4*>(static_cast<float*>(g.h) + row * g.hidden + k);
+            f32x4 v;
+            if (MODE != MLP_INFER) v = *stored;
+            if (MODE == MLP_INFER || nan_among(v)) {
+                const float* const x = static_cast<const float*>(g.x) + row * D;
+                f32x4 u;
+                if constexpr (MODE == MLP_BACKWARD) {
+                    v = plain_products(x, 1, g.wa + k, g.hidden, 1, D);
+                    u = *reinterpret_cast<const f32x4*>(static_cast<const float*>(g.factor) + row * g.hidden + k);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) v[e] *= u[e];
+                } else {
+                    v = plain_products(x, 1, g.wa + (int64_t)k * D, 1, D, D);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        float act, slope;
+                        gelu_and_slope<true>(v[e] + bias[k + e], act, slope);
+                        v[e] = act, u[e] = slope;
+                    }
+                }
+                if (MODE != MLP_INFER) *stored = v;
+                if (MODE == MLP_TRAIN) *reinterpret_cast<f32x4*>(static_cast<float*>(g.slope) + row * g.hidden + k) = u;
+            }
+            tile[H::slot(l32, half * 4 + c)] = __builtin_bit_cast(u32x4, v);
+        }
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll 1
+        for (int c = 0; c < 8; ++c) {
+            const f32x4 v = __builtin_bit_cast(f32x4, tile[H::slot(l32, c)]);
+#pragma unroll 1
+            for (int e = 0; e < 4; ++e) {
+                const int k = k0 + c * 4 + e;
+                const float f = e == 0 ? v[0] : e == 1 ? v[1] : e == 2 ? v[2] : v[3];
+#pragma unroll
+                for (int j = 0; j < CT; ++j)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) {
+                        const int col = j * 32 + r / 8 * 16 + half * 8 + r % 8;
+                        p[j][r] = fmaf(f, MODE == MLP_BACKWARD ? g.wb[(int64_t)k * D + col] : g.wb[(int64_t)col * g.hidden + k], p[j][r]);
+                    }
+            }
+        }
+        __builtin_amdgcn_wave_barrier();
+    }
+#pragma unroll
+    for (int j = 0; j < CT; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) y[j][r] = y[j][r] == y[j][r] ? y[j][r] : p[j][r];
+}
+
 // A step is 32 hidden channels.  The wait for the next step's A and B leaves the stores of this step in flight; it counts them, so they
-// are inline assembly.  fp32 inputs are taken to be finite, as by the first layer's own kernel (tall_linear.hip).
+// are inline assembly.
 template <typename T, int D, int MODE, int WAVES> struct MlpLds {
     static constexpr int PIECES = Op<T>::PL * (D / 16 + 2 * ((D + 31) / 32));   // of 64 x 16 bytes, a step's A and B
     // of 16 bytes, a wavefront's tiles: two of hidden values, at least one of y.  Inference: y leaves through the place of A and B
@@ -295,6 +363,14 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(OCC,
         if (step + 1 < steps) wait_copies<STORES>();                     // all but the stores of this step
     }
     if constexpr (L::SHARED) block_barrier();                    // A and B have been read
+    if constexpr (PL == 3) {
+        f32x4 any = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < CT; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) any[r & 3] += y[j][r];
+        if (__any(nan_among(any))) plain_rows<D, MODE>(g, row0, bias, tiles, y);
+    }
     store_y<TO, D, MODE>(g, y, row0, bias + g.hidden, tiles);
 }
 
@@ -503,7 +579,7 @@ int sswin_mlp_forward(int dtype, int out_dtype, const void* x, int64_t N, int D,
         a = planes, b = planes + (size_t)3 * D * hidden;
         if (int rc = launch_weights<float>(w1, w2, false, D, hidden, planes, planes + (size_t)3 * D * hidden, s)) return rc;
     }
-    const MlpArgs g = {x, N, hidden, a, b, b1, b2, nullptr, residual, act, slope, y, 0, 0};
+    const MlpArgs g = {x, N, hidden, a, b, static_cast<const float*>(w1), static_cast<const float*>(w2), b1, b2, nullptr, residual, act, slope, y, 0, 0};
 #define MLP_RUN(T, TO) return act ? launch_mlp<T, TO, MLP_TRAIN>(g, D, s) : launch_mlp<T, TO, MLP_INFER>(g, D, s)
     if (dtype == SSWIN_F32 && out_dtype == SSWIN_F32) MLP_RUN(float, float);
     if (dtype == SSWIN_F16 && out_dtype == SSWIN_F16) MLP_RUN(__half, __half);
@@ -522,7 +598,7 @@ int sswin_mlp_backward(int dtype, const void* dy, int64_t N, int D, int hidden, 
                 "mlp_backward: pointers must be 16-byte aligned");
     hipStream_t s = static_cast<hipStream_t>(stream);
     uint16_t *a = static_cast<uint16_t*>(ws), *b = a + sswin_mlp_workspace_bytes(dtype, D, hidden, 1) / 4;
-    const MlpArgs g = {dy, N, hidden, a, b, nullptr, nullptr, slope, nullptr, du, nullptr, dx, 0, 0};
+    const MlpArgs g = {dy, N, hidden, a, b, static_cast<const float*>(w2), static_cast<const float*>(w1), nullptr, nullptr, slope, nullptr, du, nullptr, dx, 0, 0};
 #define MLP_RUN(T)                                                                     \
     do {                                                                               \
         if (int rc = launch_weights<T>(w2, w1, true, D, hidden, a, b, s)) return rc;   \

@@ -111,3 +111,58 @@ def test_mlp_refuses_what_it_does_not_take():
 def test_mlp_last_round(rounds, tiles, extra):
     cus = torch.cuda.get_device_properties(0).multi_processor_count
     test_mlp_against_float64(torch.float32, 96, 64, 32 * cus * (8 * rounds + tiles) + extra)
+
+
+def _same_class(got, ref, bound, what):
+    """Finite where float64 is (to the bound), the same infinities, NaN where float64 has NaN."""
+    got, finite = got.double(), ref.isfinite()
+    assert got[finite].isfinite().all(), what
+    assert ((got - ref)[finite].abs() <= bound[finite]).all(), what
+    assert torch.equal(got[ref.isinf()], ref[ref.isinf()]), what
+    assert got[ref.isnan()].isnan().all(), what
+
+
+@pytest.mark.parametrize("N,hidden", [(33, 64), (3001, 384), (16500, 64)])
+@pytest.mark.parametrize("value", [float("inf"), float("-inf"), float("nan"), 3.4028234e38])
+@pytest.mark.parametrize("where", ["rows", "w1", "b1", "w2", "slope"])
+def test_mlp_fp32_of_values_that_are_not_finite(N, hidden, value, where):
+    """An infinity, a NaN or the largest number in a few places: hidden values, results and gradients are those of plain fp32
+    arithmetic, as where the two layers run one by one.  (Everything else is small where the largest number is, so that results are in
+    range.)  Bounds of finite results: as above."""
+    from sparseswin3d_amd import _lib
+    lib = _lib.load()
+    D, gen = 96, torch.Generator().manual_seed(N)
+    small = 2.0 ** -10 if abs(value) < float("inf") else 1.0
+    rand = lambda *s, std=1.0: torch.randn(*s, generator=gen) * std * small
+    x, w1, b1, w2, dy, slope = rand(N, D), rand(hidden, D, std=D ** -0.5), rand(hidden), rand(D, hidden, std=hidden ** -0.5), rand(N, D), rand(N, hidden)
+    for t in {"rows": (x, dy), "w1": (w1,), "b1": (b1,), "w2": (w2,), "slope": (slope,)}[where]:
+        if t.dim() == 1:
+            t[hidden // 2 + 3] = value
+        else:
+            t[1, 0], t[t.shape[0] // 2, t.shape[1] - 1] = value, value
+    x[N // 3], dy[N // 3] = 0, 0                                   # 0 x inf
+    x, w1, b1, w2, dy, slope = (t.cuda() for t in (x, w1, b1, w2, dy, slope))
+    w1d, w2d = w1.double(), w2.double()
+    u, scale = x.double() @ w1d.t() + b1.double(), x.double().abs() @ w1d.abs().t() + b1.double().abs()
+    g64, d64 = _gelu(u)
+    err = 2e-6 * scale + 1e-6
+    y64, y_err = g64 @ w2d.t(), err @ w2d.abs().t() + 2e-6 * (g64.abs() @ w2d.abs().t())
+    for train in (True, False):
+        y, g, d = _empty((N, D), torch.float32), *((_empty((N, hidden), torch.float32) if train else None) for _ in range(2))
+        ws, nb = _workspace(lib, x, hidden, 0)
+        _lib.check(lib.sswin_mlp_forward(0, 0, _ptr(x), N, D, hidden, _ptr(w1), _ptr(b1), _ptr(w2), None, None, _ptr(y), _ptr(g), _ptr(d), _ptr(ws), nb, _stream()))
+        _same_class(y, y64, y_err, f"y train {train}")
+        if train:
+            _same_class(g, g64, err, "act")
+            _same_class(d, d64, err, "slope")
+    if where == "b1":
+        return
+    du64 = (dy.double() @ w2d) * slope.double()
+    du_err = 2e-6 * (dy.double().abs() @ w2d.abs()) * slope.double().abs() + 1e-30
+    dx64, dx_err = du64 @ w1d, du_err @ w1d.abs() + 2e-6 * (du64.abs() @ w1d.abs())
+    du, dx = _empty((N, hidden), torch.float32), _empty((N, D), torch.float32)
+    ws, nb = _workspace(lib, x, hidden, 1)
+    _lib.check(lib.sswin_mlp_backward(0, _ptr(dy), N, D, hidden, _ptr(w1), _ptr(w2), _ptr(slope), _ptr(du), _ptr(dx), _ptr(ws), nb, _stream()))
+    _same_class(du, du64, du_err, "du")
+    _same_class(dx, dx64, dx_err, "dx")
+    assert (abs(value) < float("inf")) == bool(y64.isfinite().all() and dx64.isfinite().all() if where != "slope" else dx64.isfinite().all())
