@@ -946,7 +946,8 @@ __global__ __launch_bounds__(SMALL_WAVES * 64) void dense_backward_small_kernel(
 // out[e] = sum over chunks of part[chunk][e] for the weights and the bias behind each other; a block takes 4 EL outputs,
 // CL = 256 / EL threads share four of them, each adds every CL-th chunk in order, the CL sums in a fixed tree.
 // EL = 16; 4 from 256 chunks on, where small layers leave the chip idle and the sums one after the other take the time
-// (1024 chunks of 144 x 48 and 48 x 48: 16.8 us on average, with 4 6.8); 64 up to 16 chunks, where most of 16 threads have none
+// (1024 chunks of 144 x 48 and 48 x 48: 16.8 us on average, with 4 6.8), and for small fp32 layers from 150 (with the sums of 235
+// chunks 144 x 48 21.4 -> 18.9 us and 2 % less rounding, 250 of 96 x 144 30.4 -> 29.1; 192 x 192 and 96 x 384 lose 4 us); 64 up to 16 chunks, where most of 16 threads have none
 // (weight gradients of 2000 and 8119 rows 768 -> 2304: 35.5 -> 24.7 us and 73.0 -> 68.6)
 template <typename TO, int EL>
 __global__ __launch_bounds__(256) void dense_wgrad_sum_kernel(const float* __restrict__ part_w, const float* __restrict__ part_b, int chunks,
@@ -1108,12 +1109,12 @@ struct WgradPlan {
     int tiles_p, tiles_k, chunks;
     int64_t rows;
 };
-static WgradPlan wgrad_plan(int64_t N, int P, int K, int bk, int bm, int bn, int per_cu) {
+static WgradPlan wgrad_plan(int64_t N, int P, int K, int bk, int min_rows, int bm, int bn, int per_cu) {
     WgradPlan p;
     p.tiles_p = (P + bm - 1) / bm;
     p.tiles_k = (K + bn - 1) / bn;
     const int64_t want = std::max<int64_t>(1, (int64_t)per_cu * device_cus() / ((int64_t)p.tiles_p * p.tiles_k));
-    int64_t rows = std::max<int64_t>((N + want - 1) / want, 4 * bk);
+    int64_t rows = std::max<int64_t>((N + want - 1) / want, min_rows);
     rows = (rows + bk - 1) / bk * bk;
     p.rows = rows;
     p.chunks = (int)((N + rows - 1) / rows);
@@ -1123,29 +1124,38 @@ static WgradPlan wgrad_plan(int64_t N, int P, int K, int bk, int bm, int bn, int
 // rows up to which one launch of 32 x 32 tiles beats row chunks and their sums (284 rows 384 -> 1152: 19 us in chunks)
 constexpr int64_t WGRAD_SMALL_ROWS = 1024;
 // Tiles of dW.  fp32: by the columns it has, since a tile wider than dW works on copies of its last columns.
-//   from 192 columns of X on 128 x 192, and 96 x 192 where that takes no more tiles (35 569 rows 192 -> 576: 64 us, with 96 x 192 61
-//   but sums a fifth longer and 8 % more rounding; before 71; 192 -> 768 73 and 78, before 82; 192 -> 192 with 96 x 192 30, before
-//   39; 768 -> 192 78, before 97); 64 x 192 where dY has at most 64 (112 700 rows 192 -> 48: 35 us, before 40);
-//   192 x 64 and 64 x 64 up to 64 columns of X (112 700 rows 48 -> 144 and 48 -> 48: 36 and 21 us, before 39 and 26);
-//   128 x 96 between (75 000 rows 144 -> 144: 55 us, with 96 x 96 before 64).
+//   from 97 columns of X on 128 x 192, and 96 x 192 where that takes no more tiles (35 569 rows 192 -> 576: 64 us, with 96 x 192 61
+//   but sums a fifth longer and 8 % more rounding; 192 -> 768 73, 192 -> 192 30, 768 -> 192 78; 75 000 rows 144 -> 144: 48 us, in tiles
+//   of 128 x 96 56); 64 x 192 where dY has at most 64 (112 700 rows 192 -> 48: 37 us; 112 -> 48 31, in tiles of 128 x 96 46);
+//   192 x 64 and 64 x 64 up to 64 columns of X (112 700 rows 48 -> 144 and 48 -> 48: 36 and 19 us);
+//   128 x 96 between (75 000 rows 80 -> 112: 27 us).
+// Rows of a sum (one row group of one chunk) decide the rounding as well: the matrix instructions do not round to nearest, what
+// they leave is of one sign and grows with the number of sums, everything else with their length.  Relative error against float64
+// of 30 000 rows 48 -> 48: sums of 32 rows 2.5e-7, of 64 2.1e-7; of 112 700 rows 144 -> 144: of 587 rows 5.7e-7, of 448 5.1e-7.
+//   A sum has at least 64 rows.  Below 6144 rows (three row groups: 3072) sums are few, and shorter ones fill the chip: 4097 rows
+//   48 -> 48 9.2 us and 1.3e-7, in sums of 64 rows 10.5 and 1.4e-7; but 6000 rows 80 -> 80 14.4 and 1.7e-7, 16.4 and 1.5e-7.
+//   Tiles of 128 x 96 take two workgroups a compute unit where one would make sums longer than 128 rows and than tiles of 96 x 96
+//   with four had: 112 700 rows 80 -> 80 34 us and 3.5e-7, with two 41 and 3.4e-7; 225 700 rows 53 and 5.5e-7, 62 and 4.5e-7.
 // 16 bit: 96 x 96 (219 000 rows 96 -> 288: 39 us; 192 x 192 tiles 58, 192 x 96 44); 192 x 192 where dW has at least 48 such tiles
 //   and the rows are many, so that half the bytes pass from L2 (8119 rows 768 -> 2304: 69 us and 57, 768 -> 3072 80 and 61;
 //   2000 rows 768 -> 2304 25 and 26; 9000 rows 384 -> 1536 30 either way).
 struct WgradTile {
-    int bm, bn, per_cu;
+    int bm, bn, per_cu, parts;                                           // fp32: row groups of a workgroup
 };
 static WgradTile wgrad_tile(int dtype, int64_t N, int P, int K) {
     if (dtype != SSWIN_F32) {
-        if (N >= 4096 && P % 192 == 0 && K % 192 == 0 && (int64_t)P * K >= 48 * 192 * 192) return {192, 192, 1};
-        return {96, 96, 3};
+        if (N >= 4096 && P % 192 == 0 && K % 192 == 0 && (int64_t)P * K >= 48 * 192 * 192) return {192, 192, 1, 1};
+        return {96, 96, 3, 1};
     }
-    if (K >= 192) return P <= 64 ? WgradTile{64, 192, 2} : (P + 127) / 128 < (P + 95) / 96 ? WgradTile{128, 192, 1} : WgradTile{96, 192, 1};
-    if (K <= 64) return P <= 64 ? WgradTile{64, 64, 3} : WgradTile{192, 64, 1};
-    return {128, 96, 1};
+    const int tall = (P + 127) / 128, low = (P + 95) / 96;
+    if (K > 96) return P <= 64 ? WgradTile{64, 192, 2, 1} : tall < low ? WgradTile{128, 192, 1, 2} : WgradTile{96, 192, 1, 2};
+    if (K <= 64) return P <= 64 ? WgradTile{64, 64, 2, 2} : WgradTile{192, 64, 1, 2};
+    return {128, 96, 4 * tall <= 3 * low || N * tall <= (int64_t)3 * 128 * device_cus() ? 1 : 2, 3};
 }
 static WgradPlan wgrad_plan(int dtype, int64_t N, int P, int K) {
     const WgradTile t = wgrad_tile(dtype, N, P, K);
-    return wgrad_plan(N, P, K, dtype == SSWIN_F32 ? 16 : 32, t.bm, t.bn, t.per_cu);
+    if (dtype != SSWIN_F32) return wgrad_plan(N, P, K, 32, 128, t.bm, t.bn, t.per_cu);
+    return wgrad_plan(N, P, K, 16, N < (t.parts == 2 ? 6144 : 3072) ? 64 : 64 * t.parts, t.bm, t.bn, t.per_cu);
 }
 
 template <typename T, typename TO, typename F>
@@ -1156,10 +1166,11 @@ static int launch_wgrad_as(F* k, int threads, size_t lds, const WgradPlan& pl, c
                        P, K, pl.tiles_p, pl.tiles_k, pl.rows, ws, db ? part_b : nullptr);
     if (int rc = launch_ok("dense weight gradient")) return rc;
     const int64_t PK = (int64_t)P * K;
+    const bool narrow = pl.chunks >= 256 || (sizeof(T) == 4 && pl.chunks >= 150 && PK <= 16384);
     if (pl.chunks <= 16)
         hipLaunchKernelGGL((dense_wgrad_sum_kernel<TO, 64>), dim3((unsigned)((PK + P + 255) / 256)), dim3(256), 0, s, ws, part_b, pl.chunks, PK, P,
                            static_cast<TO*>(dw), static_cast<TO*>(db));
-    else if (pl.chunks >= 256)
+    else if (narrow)
         hipLaunchKernelGGL((dense_wgrad_sum_kernel<TO, 4>), dim3((unsigned)((PK + P + 15) / 16)), dim3(256), 0, s, ws, part_b, pl.chunks, PK, P,
                            static_cast<TO*>(dw), static_cast<TO*>(db));
     else
@@ -1168,11 +1179,11 @@ static int launch_wgrad_as(F* k, int threads, size_t lds, const WgradPlan& pl, c
     return launch_ok("dense weight gradient, sums");
 }
 
-// fp32: `parts` row groups of two buffers of (column tiles) x 3 planes
+// fp32: row groups of two buffers of (column tiles) x 3 planes
 template <auto* KERNEL, typename TO>
-static int launch_wgrad_f32(int waves, int parts, const WgradTile& t, const WgradPlan& pl, const void* dy, const void* x, int64_t N, int P, int K, void* dw,
+static int launch_wgrad_f32(int waves, const WgradTile& t, const WgradPlan& pl, const void* dy, const void* x, int64_t N, int P, int K, void* dw,
                             void* db, float* ws, hipStream_t s) {
-    const size_t lds = 2 * (size_t)parts * ((t.bm + t.bn) / 32) * 3 * 1024;
+    const size_t lds = 2 * (size_t)t.parts * ((t.bm + t.bn) / 32) * 3 * 1024;
     static const hipError_t configured = hipFuncSetAttribute(reinterpret_cast<const void*>(KERNEL), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     SSWIN_HIP(configured);
     return launch_wgrad_as<float, TO>(KERNEL, waves * 64, lds, pl, dy, x, N, P, K, dw, db, ws, s);
@@ -1189,12 +1200,12 @@ static int launch_wgrad(const void* dy, const void* x, int64_t N, int P, int K, 
     if constexpr (Op<T>::PL == 3) {
         const WgradPlan pl = wgrad_plan(SSWIN_F32, N, P, K);
         const WgradTile t = wgrad_tile(SSWIN_F32, N, P, K);
-        if (t.bm == 128 && t.bn == 192) return launch_wgrad_f32<dense_wgrad_kernel<2, 3, 2, 2, 2, 3>, TO>(12, 2, t, pl, dy, x, N, P, K, dw, db, ws, s);
-        if (t.bm == 96) return launch_wgrad_f32<dense_wgrad_kernel<3, 2, 2, 1, 3, 3>, TO>(12, 2, t, pl, dy, x, N, P, K, dw, db, ws, s);
-        if (t.bn == 192) return launch_wgrad_f32<dense_wgrad_kernel<2, 2, 1, 1, 3, 2>, TO>(4, 1, t, pl, dy, x, N, P, K, dw, db, ws, s);
-        if (t.bm == 192) return launch_wgrad_f32<dense_wgrad_kernel<6, 1, 2, 1, 2, 3>, TO>(12, 2, t, pl, dy, x, N, P, K, dw, db, ws, s);
-        if (t.bm == 64) return launch_wgrad_f32<dense_wgrad_kernel<2, 1, 2, 1, 2, 3>, TO>(4, 2, t, pl, dy, x, N, P, K, dw, db, ws, s);
-        return launch_wgrad_f32<dense_wgrad_kernel<4, 1, 3, 1, 3, 3>, TO>(12, 3, t, pl, dy, x, N, P, K, dw, db, ws, s);
+        if (t.bm == 128 && t.bn == 192) return launch_wgrad_f32<dense_wgrad_kernel<2, 3, 2, 2, 2, 3>, TO>(12, t, pl, dy, x, N, P, K, dw, db, ws, s);
+        if (t.bm == 96) return launch_wgrad_f32<dense_wgrad_kernel<3, 2, 2, 1, 3, 3>, TO>(12, t, pl, dy, x, N, P, K, dw, db, ws, s);
+        if (t.bn == 192) return launch_wgrad_f32<dense_wgrad_kernel<2, 2, 1, 1, 3, 2>, TO>(4, t, pl, dy, x, N, P, K, dw, db, ws, s);
+        if (t.bm == 192) return launch_wgrad_f32<dense_wgrad_kernel<6, 1, 2, 1, 2, 3>, TO>(12, t, pl, dy, x, N, P, K, dw, db, ws, s);
+        if (t.bm == 64) return launch_wgrad_f32<dense_wgrad_kernel<2, 1, 2, 1, 2, 3>, TO>(4, t, pl, dy, x, N, P, K, dw, db, ws, s);
+        return launch_wgrad_f32<dense_wgrad_kernel<4, 1, 3, 1, 3, 3>, TO>(12, t, pl, dy, x, N, P, K, dw, db, ws, s);
     } else {
         constexpr size_t lds = 3 * 2 * 32 * 192;                         // three stages of two tiles of 32 x 96
         const WgradPlan pl = wgrad_plan(SSWIN_F16, N, P, K);

@@ -448,6 +448,30 @@ def test_dense_fp32_weight_gradient_of_values_that_are_not_finite(N, P, K, value
     _same_class(db, d.sum(0), d.abs().sum(0), "db")
 
 
+# each tile shape where its sums are shortest or longest for their number; relative error of dW against float64 (2-norms).  The
+# bounds are a twentieth above what tiles of 96 x 96 (64 x 64 up to 64 columns) with sums of at least 64 rows give there, averaged over
+# as many inputs.
+ROUNDING = [(14000, 80, 80, 1.78e-7), (30000, 48, 48, 2.12e-7), (20000, 144, 48, 1.90e-7), (30000, 144, 48, 2.13e-7), (112700, 144, 144, 5.08e-7),
+            (112700, 96, 144, 3.85e-7), (14000, 240, 112, 1.90e-7)]
+
+
+@pytest.mark.parametrize("N,P,K,error", ROUNDING)
+def test_dense_fp32_weight_gradient_rounding(N, P, K, error):
+    from sparseswin3d_amd import _lib
+    lib = _lib.load()
+    errors = []
+    for seed in range(3):
+        gen = torch.Generator(device="cuda").manual_seed(seed)
+        dy, x = torch.randn(N, P, generator=gen, device="cuda"), torch.randn(N, K, generator=gen, device="cuda")
+        dw = torch.empty(P, K, device="cuda")
+        nb = lib.sswin_dense_weight_grad_workspace_bytes(0, N, P, K)
+        ws = torch.empty(nb, dtype=torch.uint8, device="cuda")
+        _lib.check(lib.sswin_dense_weight_grad(0, 0, _ptr(dy), _ptr(x), N, P, K, _ptr(dw), None, _ptr(ws), nb, _stream()))
+        ref = dy.double().T @ x.double()
+        errors.append(((dw.double() - ref).norm() / ref.norm()).item())
+    assert sum(errors) / 3 <= 1.05 * error, [f"{e:.3e}" for e in errors]
+
+
 @pytest.mark.parametrize("kind", ["rows", "few rows", "weight gradient", "weight gradient, few rows"])
 def test_dense_fp32_keeps_the_bits_of_single_products(kind):
     """16 equal products of operands whose lower pieces are as large as they get (just below 1 + 2^-7; just below and above a
