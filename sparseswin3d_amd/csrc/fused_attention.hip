@@ -1203,23 +1203,24 @@ struct BatchList {
 // Cost of the rows in front of window k, and the row (of a multiple of eight in its window) at which a cost is reached: lanes
 // look at 64 windows at a time, each round leaves the windows between two of them (10 000 windows: three rounds).
 constexpr int RUN_ROW = 16;
-__device__ __forceinline__ int64_t run_start(const FusedGroups& gt, int64_t k, int H) {
-    return gt.sq[k * H] / H + (int64_t)gt.T[k * H] * RUN_ROW;
+// token_rows: rows that T counts for a token, 1 in a token plan and H in the plan of a product, whose groups have rows of their own
+__device__ __forceinline__ int64_t run_start(const FusedGroups& gt, int64_t k, int H, int token_rows) {
+    return gt.sq[k * H] / H + (int64_t)(gt.T[k * H] / token_rows) * RUN_ROW;
 }
 struct RunCut {
     int window, row;
 };
-__device__ __forceinline__ RunCut run_cut(const FusedGroups& gt, int64_t windows, int H, int64_t cost) {
+__device__ __forceinline__ RunCut run_cut(const FusedGroups& gt, int64_t windows, int H, int token_rows, int64_t cost) {
     int64_t lo = 0, count = windows;                            // the window lies in [lo, lo + count)
     while (count > 1) {
         const int64_t step = (count + 63) / 64, k = lo + (threadIdx.x & 63) * step;
-        const int in_front = __popcll(__ballot(k < lo + count && run_start(gt, k, H) <= cost));   // the first of them always is
+        const int in_front = __popcll(__ballot(k < lo + count && run_start(gt, k, H, token_rows) <= cost));   // the first of them always is
         const int64_t end = lo + count;
         lo += (in_front - 1) * step;
         count = min(step, end - lo);
     }
     const int c = gt.c[lo * H];
-    const int64_t row = (cost - run_start(gt, lo, H)) / (c + RUN_ROW);
+    const int64_t row = (cost - run_start(gt, lo, H, token_rows)) / (c + RUN_ROW);
     return {__builtin_amdgcn_readfirstlane((int)lo), __builtin_amdgcn_readfirstlane(row >= c ? c : (int)row & ~7)};
 }
 
@@ -1228,7 +1229,7 @@ __global__ __launch_bounds__(256) void rpb_table_partial_kernel(FusedGroups gt, 
                                                                 int H, const int32_t* __restrict__ code, int n,
                                                                 int offset0, int rows, int rows_pad,
                                                                 const float* __restrict__ ds, int64_t windows,
-                                                                int slices, float* __restrict__ partial) {
+                                                                int token_rows, int slices, float* __restrict__ partial) {
     extern __shared__ __attribute__((aligned(16))) float rpbt_lds[];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int half = lane >> 5, l32 = lane & 31;
@@ -1248,9 +1249,9 @@ __global__ __launch_bounds__(256) void rpb_table_partial_kernel(FusedGroups gt, 
     const int per_wave = BY_TASKS ? (bl.total + slices - 1) / slices : 0;   // a wavefront's run of consecutive batches
     RunCut from = {0, 0}, to = {0, 0};                          // its run of rows
     if constexpr (!BY_TASKS) {
-        const int64_t g = (windows - 1) * H, c = gt.c[g], total = run_start(gt, windows - 1, H) + c * (c + RUN_ROW);
-        from = run_cut(gt, windows, H, total * sl / slices);
-        to = run_cut(gt, windows, H, total * (sl + 1) / slices);
+        const int64_t g = (windows - 1) * H, c = gt.c[g], total = run_start(gt, windows - 1, H, token_rows) + c * (c + RUN_ROW);
+        from = run_cut(gt, windows, H, token_rows, total * sl / slices);
+        to = run_cut(gt, windows, H, token_rows, total * (sl + 1) / slices);
     }
     auto load_headers = [&](int m_first) __attribute__((always_inline)) {
         hw_c = hw_end = hw_ib = 0;
@@ -1848,10 +1849,10 @@ static int launch_table_grad(const FusedGroups& gt, const BatchList* bl, int64_t
     const dim3 grid((unsigned)((waves + 3) / 4));
     if (bl)
         hipLaunchKernelGGL(rpb_table_partial_kernel<true>, grid, dim3(256), lds, s, gt, *bl, tokens + 3 * N, H,
-                           code, n, offset0, table_rows, rows_pad, ds, windows, slices, partial);
+                           code, n, offset0, table_rows, rows_pad, ds, windows, N ? 1 : H, slices, partial);
     else
         hipLaunchKernelGGL(rpb_table_partial_kernel<false>, grid, dim3(256), lds, s, gt, BatchList{}, tokens + 3 * N, H,
-                           code, n, offset0, table_rows, rows_pad, ds, windows, slices, partial);
+                           code, n, offset0, table_rows, rows_pad, ds, windows, N ? 1 : H, slices, partial);
     hipLaunchKernelGGL(rpb_table_reduce_kernel, dim3((unsigned)((table_rows + 15) / 16), (unsigned)H), dim3(1024), 0, s,
                        partial, slices / 4, table_rows, H, d_table);
     return launch_ok("bias table gradient");

@@ -489,8 +489,7 @@ def test_bias_table_gradient(mix, H):
     rng = np.random.default_rng(len(mix) + H)
     mixes = {"tiny": [1, 2, 3, 1, 5, 4], "mixed": [1, 40, 2, 125, 0, 0, 17, 32, 90, 3, 3, 3, 3, 64, 65, 70],
              "full": [125, 124, 100, 7], "many": list(rng.integers(0, 60, size=700)),
-             # more than 64 windows per window slice of the kernel (128 slices for three heads): a wavefront
-             # fetches window headers more than once
+             # more windows than wavefronts: runs of several small windows
              "crowd": list(rng.integers(0, 5, size=9000))}
     counts = [int(c) for c in mixes[mix]]
     n, rows = 125, 729
@@ -534,6 +533,64 @@ def test_bias_table_gradient(mix, H):
         res.append(o)
     close(res[0].cpu().numpy(), ref, 1e-5, "d table, batches from the task descriptors", mag=mag)
     assert torch.equal(res[0], res[1])
+
+
+@pytest.mark.parametrize("rows_of", ["tokens", "groups"])
+def test_bias_table_gradient_runs(rows_of):
+    """Runs of more than 64 windows, so that a wavefront fetches window headers more than once and runs end inside windows of a
+    later fetch; from a token plan and from the plan of a product, where every group has rows of its own.  The partial table of a
+    workgroup shows how many entries its four runs hold: a row of a window of c tokens counts c + 16, runs are of equal cost and are
+    cut at every eighth row."""
+    import ctypes as C
+    from sparseswin3d_amd import _lib
+    from sparseswin3d_amd.fused import BiasTableIndex, _ptr
+    from sparseswin3d_amd.window_attention import relative_position_index_3d
+    rng = np.random.default_rng(7)
+    n, rows, H = 125, 729, 24
+    counts = np.array(([1] * 90 + [60]) * 120 + [60] * 60)
+    G, sq = len(counts) * H, counts.astype(np.int64) ** 2
+    pos = [np.sort(rng.choice(n, size=c, replace=False)).astype(np.int32) for c in counts]
+    c_g = np.repeat(counts, H)
+    first = np.repeat(np.cumsum(counts) - counts, H) if rows_of == "tokens" else np.cumsum(c_g) - c_g
+    plan = np.stack([c_g, first, np.cumsum(np.repeat(sq, H)) - np.repeat(sq, H), np.repeat(np.arange(len(counts)), H),
+                     np.tile(np.arange(H), len(counts))]).astype(np.int32)
+    if rows_of == "tokens":
+        N = int(counts.sum())
+        table = np.zeros((5, N), np.int32)
+        table[3] = np.concatenate(pos)
+    else:
+        N, table = 0, np.concatenate([np.tile(p, H) for p in pos])
+    plan, table = torch.from_numpy(plan).cuda(), torch.from_numpy(table).cuda()
+    rel = relative_position_index_3d((5, 5, 5))
+    ti = BiasTableIndex.build(rel.cuda(), rows)
+    lib = _lib.load()
+    nbytes = lib.sswin_bias_table_grad_workspace_bytes(G, H, rows)
+    ws = torch.empty(int(nbytes), dtype=torch.uint8, device="cuda")
+    stream = C.c_void_p(torch.cuda.current_stream().cuda_stream)
+
+    def gradient(ds):
+        out = torch.full((rows, H), float("nan"), device="cuda")
+        _lib.check(lib.sswin_bias_table_grad(_ptr(plan), G, G, _ptr(table), N, H, n, _ptr(ti.code), ti.offset0, rows, _ptr(ds), _ptr(out),
+                                             _ptr(ws), nbytes, stream))
+        return out
+    ds = rng.standard_normal(int(sq.sum()) * H).astype(np.float32)
+    got = gradient(torch.from_numpy(ds).cuda())
+    ref, mag, at = np.zeros((rows, H)), np.zeros((rows, H)), 0
+    for c, p in zip(counts, pos):
+        block = ds[at:at + H * c * c].reshape(H, c * c).T.astype(np.float64)
+        at += H * c * c
+        index = rel.numpy()[p][:, p].reshape(-1)
+        np.add.at(ref, index, block)
+        np.add.at(mag, index, np.abs(block))
+    close(got.cpu().numpy(), ref, 1e-5, "d table", mag=mag)
+
+    gradient(torch.ones(len(ds), device="cuda"))
+    slices = (int(nbytes) - 256) // (4 * H * rows)               # wavefronts of a head, four a partial table
+    assert (counts > 0).sum() / slices > 64
+    held = ws[:(int(nbytes) - 256) // 4].view(torch.float32).view(H, slices // 4, rows).double().sum(-1)
+    assert held.sum() == len(ds)
+    cost = int((counts * (counts + 16)).sum()) / slices
+    assert held.max() <= 4 * cost + 8 * (counts.max() + 16)
 
 
 def test_bias_from_table_matches_the_gather():
