@@ -467,8 +467,9 @@ enum { SSWIN_CAST_PARTS = 8 };
 int sswin_cast_parts(int dtype, const void* const* src, const int64_t* sizes, int count, void* dst, void* stream);
 /* The feed-forward part of a block as one launch: y [N, D] = GELU(x w1^T + b1) w2^T + b2 + residual for x [N, D], w1 [hidden, D],
  * w2 [D, hidden] (biases and residual, of y's type, may be null).  act and slope [N, hidden] of x's type receive GELU's value and
- * derivative, or are both null.  Backward: du [N, hidden] = (dy w2) * slope, dx [N, D] = du w1.  fp32: 96 channels; 16 bit: 48, 96 or
- * 192; hidden a multiple of 64 (fp32: 32) up to 1024; at least 32 rows.  All pointers 16-byte aligned. */
+ * derivative, or are both null.  Backward: du [N, hidden] = (dy w2) * slope, dx [N, D] = du w1.  fp32: 96 channels; 16 bit: 48 or 96;
+ * hidden a multiple of 32, 64 to 1024; at least 32 rows.  All pointers 16-byte aligned; y, act and slope may not overlap x or residual,
+ * du and dx not dy or slope. */
 int sswin_mlp_supported(int dtype, int64_t N, int D, int hidden);
 int sswin_mlp_preferred(int dtype, int64_t N, int D, int hidden);   /* supported, and ahead of the two layers */
 size_t sswin_mlp_workspace_bytes(int dtype, int D, int hidden, int backward);

@@ -19,6 +19,7 @@
 // channels, 225 000 rows: 89 and 69, 55 and 43 (55 and 38).  bf16 96 channels, inference, 112 700 rows: 66 and 46 (13; GELU on the
 // vector units 21).
 #include <algorithm>
+#include <initializer_list>
 #include <type_traits>
 
 #include "dense_epilogue.hpp"
@@ -542,6 +543,19 @@ static int mlp_check(const char* what, int dtype, int64_t N, int D, int hidden, 
     return 0;
 }
 
+// The last tile of 32 rows is moved back and read again where other wavefronts may already have stored: results lie apart from rows read
+struct Rows {
+    const void* p;
+    size_t bytes;
+};
+static bool apart(std::initializer_list<Rows> results, std::initializer_list<Rows> inputs) {
+    for (const Rows& r : results)
+        for (const Rows& i : inputs)
+            if (r.p && i.p && (uintptr_t)r.p < (uintptr_t)i.p + i.bytes && (uintptr_t)i.p < (uintptr_t)r.p + r.bytes) return false;
+    return true;
+}
+static size_t value_size(int dtype) { return dtype == SSWIN_F32 ? 4 : 2; }
+
 extern "C" {
 
 int sswin_mlp_supported(int dtype, int64_t N, int D, int hidden) {
@@ -572,6 +586,8 @@ int sswin_mlp_forward(int dtype, int out_dtype, const void* x, int64_t N, int D,
     SSWIN_CHECK(x && w1 && w2 && y && (!act == !slope) && (ws || dtype != SSWIN_F32), "mlp_forward: null pointer");
     SSWIN_CHECK(((uintptr_t)x | (uintptr_t)w1 | (uintptr_t)b1 | (uintptr_t)w2 | (uintptr_t)b2 | (uintptr_t)residual | (uintptr_t)y | (uintptr_t)act |
                  (uintptr_t)slope) % 16 == 0, "mlp_forward: pointers must be 16-byte aligned");
+    const size_t rows = (size_t)N * D * value_size(dtype), out_rows = (size_t)N * D * value_size(out_dtype), inner = (size_t)N * hidden * value_size(dtype);
+    SSWIN_CHECK(apart({{y, out_rows}, {act, inner}, {slope, inner}}, {{x, rows}, {residual, out_rows}}), "mlp_forward: results may not overlap x or residual");
     hipStream_t s = static_cast<hipStream_t>(stream);
     const uint16_t *a = static_cast<const uint16_t*>(w1), *b = static_cast<const uint16_t*>(w2);
     if (dtype == SSWIN_F32) {
@@ -596,6 +612,8 @@ int sswin_mlp_backward(int dtype, const void* dy, int64_t N, int D, int hidden, 
     SSWIN_CHECK(dy && w1 && w2 && slope && du && dx && ws, "mlp_backward: null pointer");
     SSWIN_CHECK(((uintptr_t)dy | (uintptr_t)w1 | (uintptr_t)w2 | (uintptr_t)slope | (uintptr_t)du | (uintptr_t)dx) % 16 == 0,
                 "mlp_backward: pointers must be 16-byte aligned");
+    const size_t rows = (size_t)N * D * value_size(dtype), inner = (size_t)N * hidden * value_size(dtype);
+    SSWIN_CHECK(apart({{du, inner}, {dx, rows}}, {{dy, rows}, {slope, inner}}), "mlp_backward: results may not overlap dy or slope");
     hipStream_t s = static_cast<hipStream_t>(stream);
     uint16_t *a = static_cast<uint16_t*>(ws), *b = a + sswin_mlp_workspace_bytes(dtype, D, hidden, 1) / 4;
     const MlpArgs g = {dy, N, hidden, a, b, static_cast<const float*>(w2), static_cast<const float*>(w1), nullptr, nullptr, slope, nullptr, du, nullptr, dx, 0, 0};

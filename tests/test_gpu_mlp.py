@@ -105,6 +105,26 @@ def test_mlp_refuses_what_it_does_not_take():
         assert lib.sswin_mlp_backward(dtype, None, n, d, hidden, None, None, None, None, None, None, 1 << 30, None) != 0
 
 
+def test_mlp_refuses_results_over_rows_it_reads():
+    """The last rows are read twice: a result in the place of an input would change them in between.  Refused on the host."""
+    from sparseswin3d_amd import _lib
+    lib = _lib.load()
+    N, D, hidden = 65, 48, 192
+    rows = lambda width, dtype=torch.float16: torch.zeros(N, width, dtype=dtype, device="cuda")
+    x, y, w1, w2, act, slope = rows(D), rows(D), torch.zeros(hidden, D, device="cuda").half(), torch.zeros(D, hidden, device="cuda").half(), rows(hidden), rows(hidden)
+    ws, nb = _workspace(lib, x, hidden, 1)
+    wide = torch.zeros(N + 64, D, dtype=torch.float16, device="cuda")
+    forward = lambda x, residual, y, act, slope: lib.sswin_mlp_forward(1, 1, _ptr(x), N, D, hidden, _ptr(w1), None, _ptr(w2), None, _ptr(residual), _ptr(y), _ptr(act),
+                                                                       _ptr(slope), None, 0, _stream())
+    backward = lambda dy, slope, du, dx: lib.sswin_mlp_backward(1, _ptr(dy), N, D, hidden, _ptr(w1), _ptr(w2), _ptr(slope), _ptr(du), _ptr(dx), _ptr(ws), nb, _stream())
+    for args in [(x, y, y, None, None), (x, None, x, None, None), (wide, None, wide[64:], None, None), (wide[64:], None, wide, None, None), (act, None, y, act, slope),
+                 (slope, None, y, act, slope)]:
+        assert forward(*args) != 0 and b"overlap" in lib.sswin_last_error()
+    for args in [(x, slope, act, x), (x, slope, slope, y), (act, slope, act, y)]:
+        assert backward(*args) != 0 and b"overlap" in lib.sswin_last_error()
+    assert forward(x, None, y, act, slope) == 0 and backward(x, slope, act, y) == 0
+
+
 # behind the last full round of workgroups of 256 rows the tiles of 32 are dealt to all compute units: none, one, two and seven a
 # workgroup, after no, one and two rounds
 @pytest.mark.parametrize("rounds,tiles,extra", [(1, 0, 0), (0, 1, 1), (0, 2, -1), (1, 1, 31), (1, 7, 0), (2, 0, 1)])
