@@ -540,7 +540,7 @@ Tensor attention_forward(Attention& a, const Tensor& qkv, const Tensor& bias, At
     const int8_t* mask = a.mask.defined() ? a.mask.data_ptr<int8_t>() : nullptr;
     if (a.resident) {
         saved.aux = at::empty({std::max<int64_t>(a.H * N, 1)}, fopt);
-        const auto run = saved.bias32.dim() == 4 ? sswin_window_attention_forward_pair : sswin_window_attention_forward;
+        const auto run = a.code.defined() ? sswin_window_attention_forward_pair : sswin_window_attention_forward;
         RUN_NAMED("sswin_window_attention_forward", run(dt, i32(tp.tasks), tp.g_cap, tp.buckets, i32(tp.tokens), N, a.H, hd, ptr(qkv), 3 * D, 0, ptr(qkv),
                                                         3 * D, (int)D, ptr(qkv), 3 * D, (int)(2 * D), (float)a.scale, f32(saved.bias32), a.n, mask,
                                                         a.regions(), ptr(out), D, 0, f32(saved.aux), s));
@@ -600,7 +600,9 @@ Tensor attention_backward(const Attention& a, const Tensor& qkv, const Tensor& b
     if (a.resident) {
         const int8_t* mask = a.mask.defined() ? a.mask.data_ptr<int8_t>() : nullptr;
         Tensor d_s = want_bias ? at::empty({std::max<int64_t>(tp.A, 1)}, fopt) : Tensor();
-        const auto run = saved.bias32.dim() == 4 ? sswin_window_attention_backward_pair : sswin_window_attention_backward;
+        const bool pair = a.code.defined();                              // as the forward stored it
+        TORCH_CHECK(saved.bias32.numel() == (pair ? 2 : 1) * (int64_t)a.H * a.n * a.n, "attention: a saved bias of ", saved.bias32.sizes());
+        const auto run = pair ? sswin_window_attention_backward_pair : sswin_window_attention_backward;
         RUN_NAMED("sswin_window_attention_backward", run(dt, i32(tp.tasks), tp.g_cap, tp.buckets, i32(tp.tokens), N, a.H, hd, ptr(qkv), 3 * D, 0, ptr(qkv),
                                                          3 * D, (int)D, ptr(qkv), 3 * D, (int)(2 * D), (float)a.scale, f32(saved.bias32), a.n, mask,
                                                          a.regions(), ptr(out), D, 0, ptr(d_out), D, 0, f32(saved.aux), ptr(d_qkv), 3 * D, 0, ptr(d_qkv),

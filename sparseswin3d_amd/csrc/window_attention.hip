@@ -1167,10 +1167,10 @@ static int check_common(const char* who, int dtype, const int32_t* tasks, int64_
 using namespace sswin;
 
 static int attention_forward(bool pair, int dtype, const int32_t* tasks, int64_t g_cap, const int64_t* bucket_counts,
-                             const int32_t* tokens, int64_t N, int H, int hd, const void* q_base, int64_t q_stride,
-                             int q_col0, const void* k_base, int64_t k_stride, int k_col0, const void* v_base, int64_t
-                             v_stride, int v_col0, float scale, const float* bias, int n, const int8_t* mask, int
-                             n_mask_windows, void* o_base, int64_t o_stride, int o_col0, float* lse, void* stream) {
+                             const int32_t* tokens, int64_t N, int H, int hd, const void* q_base, int64_t q_stride, int q_col0,
+                             const void* k_base, int64_t k_stride, int k_col0, const void* v_base, int64_t v_stride, int v_col0,
+                             float scale, const float* bias, int n, const int8_t* mask, int n_mask_windows, void* o_base,
+                             int64_t o_stride, int o_col0, float* lse, void* stream) {
     int64_t total = 0;
     if (check_common("window_attention_forward", dtype, tasks, g_cap, bucket_counts, tokens, N, H, hd, bias, n, mask, n_mask_windows, &total))
         return 1;
@@ -1198,13 +1198,12 @@ static int attention_forward(bool pair, int dtype, const int32_t* tasks, int64_t
 }
 
 static int attention_backward(bool pair, int dtype, const int32_t* tasks, int64_t g_cap, const int64_t* bucket_counts,
-                              const int32_t* tokens, int64_t N, int H, int hd, const void* q_base, int64_t q_stride,
-                              int q_col0, const void* k_base, int64_t k_stride, int k_col0, const void* v_base,
-                              int64_t v_stride, int v_col0, float scale, const float* bias, int n, const int8_t* mask,
-                              int n_mask_windows, const void* o_base, int64_t o_stride, int o_col0, const void*
-                              do_base, int64_t do_stride, int do_col0, const float* lse, void* dq_base, int64_t
-                              dq_stride, int dq_col0, void* dk_base, int64_t dk_stride, int dk_col0, void* dv_base,
-                              int64_t dv_stride, int dv_col0, float* ds_out, int sides, void* stream) {
+                              const int32_t* tokens, int64_t N, int H, int hd, const void* q_base, int64_t q_stride, int q_col0,
+                              const void* k_base, int64_t k_stride, int k_col0, const void* v_base, int64_t v_stride, int v_col0,
+                              float scale, const float* bias, int n, const int8_t* mask, int n_mask_windows, const void* o_base,
+                              int64_t o_stride, int o_col0, const void* do_base, int64_t do_stride, int do_col0, const float* lse,
+                              void* dq_base, int64_t dq_stride, int dq_col0, void* dk_base, int64_t dk_stride, int dk_col0,
+                              void* dv_base, int64_t dv_stride, int dv_col0, float* ds_out, int sides, void* stream) {
     int64_t total = 0;
     if (check_common("window_attention_backward", dtype, tasks, g_cap, bucket_counts, tokens, N, H, hd, bias, n, mask,
                      n_mask_windows, &total))

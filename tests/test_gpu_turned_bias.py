@@ -36,3 +36,24 @@ def test_attention_from_the_table_equals_attention_from_the_bias(window, counts,
         results.append((out.detach(), x.grad))
     for a, b in zip(*results):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("coded", [True, False], ids=["table", "bias"])
+def test_a_saved_bias_of_another_size_is_refused(coded):
+    """The backward reads one or two biases by whether positions are coded: a hook on saved tensors that gives back the other number
+    is an error, in front of the launch."""
+    from sparseswin3d_amd import _lib
+    from sparseswin3d_amd.fused import BiasTableIndex, TokenPlan
+    from sparseswin3d_amd.window_attention import relative_position_index_3d
+    n, H, hd, rows = 27, 3, 32, 125
+    ind = torch.from_numpy(ragged_window_indices(np.random.default_rng(0), [3, 27], n)).cuda()
+    ti = BiasTableIndex.build(relative_position_index_3d((3, 3, 3)).cuda(), rows)
+    bias = torch.randn(rows, H, device="cuda") if coded else torch.randn(H, n, n, device="cuda")
+
+    def other(t):
+        return t[0] if coded and t.dim() == 4 else torch.stack([t, t]) if not coded and t.shape == (H, n, n) else t
+    x = torch.randn(len(ind), 3, H, hd, device="cuda", requires_grad=True)
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t, other):
+        out = _lib.native().attention(x, bias, TokenPlan(ind, 2, n, H).native, None, ti.code if coded else None, ti.offset0, n, hd ** -0.5, "resident")
+    with pytest.raises(RuntimeError, match="saved bias"):
+        out.backward(torch.ones_like(out))
