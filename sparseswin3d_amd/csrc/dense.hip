@@ -1045,6 +1045,7 @@ static Cut cut_of(int dtype, int64_t N, int K, int P) {
     const int64_t shares = std::min<int64_t>({4, 400 / tiles, K / 576});
     return {false, (int)std::max<int64_t>(shares, 1)};
 }
+bool few_rows(int dtype, int64_t N, int K, int P) { return cut_of(dtype, N, K, P).few; }
 
 template <typename T, typename TO, int EPI, bool DOWN>
 static int launch_forward(const void* x, int64_t N, int K, const void* w, int P, const Epilogue& ep, float* ws, size_t ws_bytes, hipStream_t s) {

@@ -143,6 +143,8 @@ __device__ __forceinline__ void finish8(const Epilogue& ep, int64_t row, int col
 
 // fp32 layers of 96 reduction channels and a multiple of 96 outputs (tall_linear.hip): x [N >= 32, 96], all of Wop in LDS
 int staged_layer_96(const float* x, int64_t N, const float* w, int P, bool transposed, int epilogue, const Epilogue& ep, hipStream_t s);
+// whether a layer of N rows, K -> P, takes the kernel for few rows, whose wavefronts share the reduction (dense.hip)
+bool few_rows(int dtype, int64_t N, int K, int P);
 // 16-bit layers of 48, 96 or 192 reduction channels without a last step: x read once (mlp.hip)
 bool rows_once_takes(int64_t N, int D, int P);
 template <typename T> int rows_once(const T* x, int64_t N, int D, const T* w, const T* b, int P, T* y, hipStream_t s);

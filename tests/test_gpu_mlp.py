@@ -133,6 +133,38 @@ def test_mlp_last_round(rounds, tiles, extra):
     test_mlp_against_float64(torch.float32, 96, 64, 32 * cus * (8 * rounds + tiles) + extra)
 
 
+@pytest.mark.parametrize("N", [16385, 17001, 19072, 19073, 32768])
+def test_mlp_fp32_sums_no_less_exactly_than_two_layers(N):
+    """Where the launch is preferred, its error against float64 (2-norms) is at most that of the layers it stands for, up to 2 % for the
+    spread of the inputs: they sum few rows in eight parts."""
+    from sparseswin3d_amd import _lib
+    lib = _lib.load()
+    D, hidden, gen = 96, 384, torch.Generator().manual_seed(N)
+    assert lib.sswin_mlp_preferred(0, N, D, hidden) == (N > 19072)      # 149 tiles of 128 rows: few rows
+    if N <= 19072:
+        return
+    rand = lambda *s, std=1.0: (torch.randn(*s, generator=gen) * std).cuda()
+    x, w1, w2, dy, slope = rand(N, D), rand(hidden, D, std=D ** -0.5), rand(D, hidden, std=hidden ** -0.5), rand(N, D), rand(N, hidden)
+    empty = lambda width: _empty((N, width), torch.float32)
+    y, dx, du, act, y2, dx2, du2 = empty(D), empty(D), empty(hidden), empty(hidden), empty(D), empty(D), empty(hidden)
+    nb = max(lib.sswin_mlp_workspace_bytes(0, D, hidden, 1), lib.sswin_mlp_workspace_bytes(0, D, hidden, 0), lib.sswin_dense_forward_workspace_bytes(0, N, hidden, D),
+             lib.sswin_dense_forward_workspace_bytes(0, N, D, hidden), 16)
+    ws = torch.empty(nb, dtype=torch.uint8, device="cuda")
+    layer = lambda turned, epilogue, a, k, w, p, extra, out: _lib.check(lib.sswin_dense_forward(0, 0, turned, epilogue, _ptr(a), N, k, _ptr(w), None, p, _ptr(extra), _ptr(out),
+                                                                                              None, _ptr(ws), nb, _stream()))
+    layer(0, 1, x, D, w1, hidden, None, act)                              # GELU
+    layer(0, 0, act, hidden, w2, D, None, y2)
+    layer(1, 3, dy, D, w2, hidden, slope, du2)                            # times the slope
+    layer(1, 0, du2, hidden, w1, D, None, dx2)
+    _lib.check(lib.sswin_mlp_forward(0, 0, _ptr(x), N, D, hidden, _ptr(w1), None, _ptr(w2), None, None, _ptr(y), None, None, _ptr(ws), nb, _stream()))
+    _lib.check(lib.sswin_mlp_backward(0, _ptr(dy), N, D, hidden, _ptr(w1), _ptr(w2), _ptr(slope), _ptr(du), _ptr(dx), _ptr(ws), nb, _stream()))
+    y64 = _gelu(x.double() @ w1.double().t())[0] @ w2.double().t()
+    dx64 = ((dy.double() @ w2.double()) * slope.double()) @ w1.double()
+    for one, two, ref, what in ((y, y2, y64, "y"), (dx, dx2, dx64, "dx")):
+        errors = [((t.double() - ref).norm() / ref.norm()).item() for t in (one, two)]
+        assert errors[0] <= 1.02 * errors[1], (what, errors)
+
+
 def _same_class(got, ref, bound, what):
     """Finite where float64 is (to the bound), the same infinities, NaN where float64 has NaN."""
     got, finite = got.double(), ref.isfinite()
