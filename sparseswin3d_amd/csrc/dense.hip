@@ -1052,7 +1052,8 @@ static int launch_forward(const void* x, int64_t N, int K, const void* w, int P,
     const T* xp = static_cast<const T*>(x);
     const T* wp = static_cast<const T*>(w);
     if constexpr (Op<T>::PL == 1 && EPI == EPI_NONE && !DOWN)
-        if (rows_once_takes(N, K, P)) return rows_once<T>(xp, N, K, wp, static_cast<const T*>(ep.bias), P, static_cast<T*>(ep.y), s);
+        // not in place: its last tile reads rows again that another wavefront may have stored
+        if (rows_once_takes(N, K, P) && ep.y != x) return rows_once<T>(xp, N, K, wp, static_cast<const T*>(ep.bias), P, static_cast<T*>(ep.y), s);
     const int64_t few_blocks = (N + 31) / 32 * ((P + 31) / 32);
     Cut cut = cut_of(Op<T>::PL == 3 ? SSWIN_F32 : SSWIN_F16, N, K, P);
     if (cut.few && few_blocks < (1ll << 31)) {

@@ -100,6 +100,19 @@ def test_dense_forward_that_reads_its_rows_once(K, N, P, dtype):
         _check(y, pre + add, mag + abs(add), dtype, "plain")
 
 
+# a result in the place of its rows, where one workgroup of a tile holds them whole (96 columns at most, more rows than the few-rows kernel takes)
+@pytest.mark.parametrize("K", [48, 96])
+def test_dense_forward_in_place(K):
+    from sparseswin3d_amd import _lib
+    lib = _lib.load()
+    N, dtype = 140001, torch.float16
+    gen = torch.Generator().manual_seed(K)
+    x, w, b = _rand(gen, N, K, dtype=dtype), (_rand(gen, K, K, spread=1) / K ** 0.5).to(dtype), _rand(gen, K, dtype=dtype)
+    ref, mag = x.double() @ w.double().T + b.double(), x.double().abs() @ w.double().abs().T + b.double().abs()
+    _lib.check(lib.sswin_dense_forward(1, 1, 0, PLAIN, _ptr(x), N, K, _ptr(w), _ptr(b), K, None, _ptr(x), None, None, 0, _stream()))
+    _check(x, ref, mag, dtype, "in place")
+
+
 # 16 bit: the last rows of the few-rows kernel and the first of the tiles behind it, with a residual and as an input gradient
 @pytest.mark.parametrize("N", [5376, 5377])
 def test_dense_forward_where_the_tiles_take_over(N):
