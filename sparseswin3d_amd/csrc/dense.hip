@@ -1028,24 +1028,44 @@ static int launch_rows16(const T* x, int64_t N, int K, const T* w, int P, int ks
 
 // How a product is cut.
 //   few rows: 32 x 32 tiles while the workgroups of the larger tiles would leave most of the chip idle.  fp32: below 150 tiles of
-//     128 x 96.  16 bit: their time grows with tiles x K, that of the larger tiles starts at 6 us and grows with K: 500 rows
-//     768 -> 768 (24 576) 7.8 us against 12.2, 1364 rows (67 584) 15.5 against 12.6; 2000 rows 384 -> 384 (24 576) 7.4 and 9.7, 4000
-//     (49 152) 12.7 and 10.0; 6000 rows 192 -> 192 (18 048) 7.2 and 7.1, 16 000 (48 000) 14.2 and 7.8; 24 000 rows 96 -> 96 with a
-//     residual (18 048) 8.3 and 8.7, 60 000 (45 024) 16.3 and 12.7; 60 000 rows 48 -> 48, input gradient (22 512) 14.6 and 8.1.
+//     128 x 96.  16 bit: see few_line.
 //   ksplit (16 bit): shares of the reduction, each at least 576 long, while the tiles alone do not fill the chip: 1364 rows
 //     3072 -> 768 (88 tiles) 36 us with one share, 24 with two, 23 with four; 2729 rows (176 tiles) 37, 33 and 36.
 struct Cut {
     bool few;
     int ksplit;
 };
-static Cut cut_of(int dtype, int64_t N, int K, int P) {
+constexpr int64_t FEW_MOST = 50000;
+static Cut cut_of(int dtype, int64_t N, int K, int P, int64_t line = FEW_MOST) {
     const int64_t tiles = (N + 127) / 128 * ((P + 95) / 96);
     if (dtype == SSWIN_F32) return {tiles < 150, 1};
-    if (tiles * K <= std::min(50000, 12000 + 50 * K)) return {true, 1};
+    if (tiles * K <= line) return {true, 1};
     const int64_t shares = std::min<int64_t>({4, 400 / tiles, K / 576});
     return {false, (int)std::max<int64_t>(shares, 1)};
 }
 bool few_rows(int dtype, int64_t N, int K, int P) { return cut_of(dtype, N, K, P).few; }
+
+// 16 bit: tiles x K up to which few rows are ahead.  Their time grows with it, that of the larger tiles starts at 6 us with the input
+// gradient, at 7 to 9 with a layer, and grows with K.  Microseconds of a bf16 launch, few rows and tiles:
+//   input gradient: 288 -> 96, 11 776 rows (26 496) 9.3 and 7.5; 192 -> 192, 7296 (21 888) 9.4 and 6.3; 48 -> 48, 38 528 (14 448) 10.3 and 7.2;
+//   layers of whole steps of 64 channels: 192 -> 192, 7296 rows (21 888) 7.8 and 6.7; 384 -> 384, 2816 (33 792) 9.5 and 8.3; with GELU
+//     later: 192 -> 768, 1920 rows (23 040) 8.5 and 9.3, 2688 (32 256) 10.0 and 9.9;
+//   up to 96 channels: 48 -> 48 with a residual, 57 216 rows (21 456) 9.1 and 9.3, 76 160 (28 560) 11.9 and 9.5; with GELU 96 -> 384, 9984
+//     (29 952) 11.0 and 13.0, 14 336 (43 008) 14.7 and 13.7; with fp32
+//     results 96 -> 96, 39 936 (29 952) 10.7 and 11.5, 48 768 (36 576) 13.1 and 12.4;
+//   others, whose last step is ragged in the tiles: 144 -> 144, 19 328 rows (43 488) 9.2 and 9.8; 240 -> 240, 5120 (28 800) 5.5 and 7.7;
+//     480 -> 480, 2560 (48 000) 8.0 and 9.7; and fewer than 96 columns, which a tile does not use: 192 -> 48, 18 048 (27 072) 6.6 and 6.9.
+// fp32 results of 16-bit rows show how they were summed (16-bit results differ by a rounding and have the same error, 2.1e-4 fp16 and
+// 1.7e-3 bf16): with tiles only where their error against float64 is no larger, fp16 192 -> 192 5.3e-8 either way, but 288 -> 288
+// 5.4e-8 and 5.9e-8, and behind 512 tiles, where a tile is summed in one part, 96 -> 96 4.8e-8 and 5.2e-8.
+static int64_t few_line(int64_t N, int K, int P, int epi, bool down, bool wide) {
+    if (wide && (K > 192 || (N + 127) / 128 * ((P + 95) / 96) > 512)) return FEW_MOST;
+    if (down) return std::min<int64_t>(FEW_MOST, 12000 + 50 * K);
+    if (P < 96 && K > 48) return FEW_MOST;
+    if (K % 64 == 0) return std::min<int64_t>(FEW_MOST, (epi == EPI_GELU ? 22000 : 12000) + 50 * K);
+    if (K <= 96) return epi == EPI_GELU ? 40000 : wide ? 35000 : 25000;
+    return FEW_MOST;
+}
 
 template <typename T, typename TO, int EPI, bool DOWN>
 static int launch_forward(const void* x, int64_t N, int K, const void* w, int P, const Epilogue& ep, float* ws, size_t ws_bytes, hipStream_t s) {
@@ -1055,7 +1075,7 @@ static int launch_forward(const void* x, int64_t N, int K, const void* w, int P,
         // not in place: its last tile reads rows again that another wavefront may have stored
         if (rows_once_takes(N, K, P) && ep.y != x) return rows_once<T>(xp, N, K, wp, static_cast<const T*>(ep.bias), P, static_cast<T*>(ep.y), s);
     const int64_t few_blocks = (N + 31) / 32 * ((P + 31) / 32);
-    Cut cut = cut_of(Op<T>::PL == 3 ? SSWIN_F32 : SSWIN_F16, N, K, P);
+    Cut cut = cut_of(Op<T>::PL == 3 ? SSWIN_F32 : SSWIN_F16, N, K, P, few_line(N, K, P, EPI, DOWN, sizeof(T) < sizeof(TO)));
     if (cut.few && few_blocks < (1ll << 31)) {
         hipLaunchKernelGGL((dense_small_kernel<T, TO, EPI, DOWN>), dim3((unsigned)few_blocks), dim3(SMALL_WAVES * 64), 0, s, xp, N, K, wp, P,
                            (P + 31) / 32, ep);

@@ -100,6 +100,26 @@ def test_dense_forward_that_reads_its_rows_once(K, N, P, dtype):
         _check(y, pre + add, mag + abs(add), dtype, "plain")
 
 
+# 16 bit: on either side of the line up to which a layer takes the few-rows kernel: whole steps of 64 channels with and without GELU, up to 96
+# channels, ragged steps, fewer than 96 columns
+@pytest.mark.parametrize("K,P,epi,rows", [(192, 192, PLAIN, 56), (192, 768, GELU, 20), (96, 96, RESIDUAL, 260), (96, 384, GELU, 104), (144, 144, PLAIN, 173), (192, 48, RESIDUAL, 260)])
+def test_dense_forward_around_the_lines_of_few_rows(K, P, epi, rows):
+    from sparseswin3d_amd import _lib
+    lib = _lib.load()
+    dtype = torch.bfloat16
+    gen = torch.Generator().manual_seed(K + 3 * P)
+    for N in (rows * 128, rows * 128 + 1):
+        x, w, b, extra = _rand(gen, N, K, dtype=dtype), (_rand(gen, P, K, spread=1) / K ** 0.5).to(dtype), _rand(gen, P, dtype=dtype), _rand(gen, N, P, dtype=dtype)
+        y, _ = _forward(lib, _lib, x, w, b, 0, epi, extra if epi == RESIDUAL else None, dtype)
+        pre = x.double() @ w.double().T + b.double()
+        mag = x.double().abs() @ w.double().abs().T + b.double().abs()
+        if epi == GELU:
+            pre, mag = pre * 0.5 * (1 + torch.erf(pre / 2 ** 0.5)), 1.13 * mag + pre.abs()
+        elif epi == RESIDUAL:
+            pre, mag = pre + extra.double(), mag + extra.double().abs()
+        _check(y, pre, mag, dtype, f"{N} rows")
+
+
 # a result in the place of its rows, where one workgroup of a tile holds them whole (96 columns at most, more rows than the few-rows kernel takes)
 @pytest.mark.parametrize("K", [48, 96])
 def test_dense_forward_in_place(K):
@@ -483,6 +503,20 @@ def test_dense_fp32_weight_gradient_rounding(N, P, K, error):
         ref = dy.double().T @ x.double()
         errors.append(((dw.double() - ref).norm() / ref.norm()).item())
     assert sum(errors) / 3 <= 1.05 * error, [f"{e:.3e}" for e in errors]
+
+
+# fp32 results of 16-bit rows: 2-norm of the error over that of the result, as the kernel for few rows has it (5.4, 5.5, 4.85 and 5.4e-8, three
+# inputs within 1 %); the tiles give 6.0, 6.5 and 5.2e-8 for the first three, and 5.4e-8 for the last, where they are taken
+@pytest.mark.parametrize("N,K,P,error", [(7296, 288, 288, 5.6e-8), (4096, 384, 384, 5.65e-8), (65920, 96, 96, 5.0e-8), (16384, 192, 192, 5.55e-8)])
+def test_dense_fp32_results_of_16_bit_rows_rounding(N, K, P, error):
+    from sparseswin3d_amd import _lib
+    lib = _lib.load()
+    gen = torch.Generator(device="cuda").manual_seed(N + K)
+    rand = lambda *s: torch.randn(*s, generator=gen, device="cuda")
+    x, w, b, extra = rand(N, K).half(), (rand(P, K) * K ** -0.5).half(), rand(P).half(), rand(N, P)
+    y, _ = _forward(lib, _lib, x, w, b, 0, RESIDUAL, extra, torch.float32)
+    ref = x.double() @ w.double().T + b.double() + extra.double()
+    assert (y.double() - ref).norm() <= error * ref.norm()
 
 
 @pytest.mark.parametrize("kind", ["rows", "few rows", "weight gradient", "weight gradient, few rows"])
