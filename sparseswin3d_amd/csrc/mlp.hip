@@ -566,14 +566,16 @@ int sswin_mlp_supported(int dtype, int64_t N, int D, int hidden) {
 }
 
 // Where one launch is ahead of two.  16 bit: from 8192 rows on (fp16 48 channels with an fp32 residual, forward and backward: 8000 rows
-// 33.4 -> 23.5 us; bf16 96 channels, 8000 rows 41.8 -> 40.0, inference 20.4 -> 18.5, 4000 rows 33.9 -> 38.4 and 16.3 -> 18.2).  fp32: a
+// 33.4 -> 23.5 us; bf16 96 channels, 8000 rows 41.8 -> 40.0, inference 20.4 -> 18.5, 4000 rows 33.9 -> 38.4 and 16.3 -> 18.2); a wavefront's
+// time grows with the hidden channels, that of the two layers' tiles with all of their work, so with more than 384 later (bf16 96 channels,
+// forward and backward, 768 hidden: 20 000 rows 66 -> 76, 50 000 114 -> 91; 1024 hidden 8192 57 -> 91, 50 000 142 -> 121).  fp32: a
 // wavefront takes about 46 us forward and 34 backward alone on its SIMD, so from three wavefronts a compute unit on (forward and
 // backward of 8192 rows 60 -> 80 us, 16 384 88 -> 89, 24 576 101 -> 93, 32 768 116 -> 101, 65 536 189 -> 152, 81 920 248 -> 241, 225 700
 // 633 -> 543), and only behind the rows up to which the second layer is one of few rows: there eight wavefronts share its sums, and
 // their error against float64 is 1.2e-7 of y and 2.3e-7 of dx, here 1.9e-7 and 3.3e-7; in larger tiles 1.9e-7 and 3.6e-7.
 int sswin_mlp_preferred(int dtype, int64_t N, int D, int hidden) {
     if (!sswin_mlp_supported(dtype, N, D, hidden)) return 0;
-    if (dtype != SSWIN_F32) return N >= 8192;
+    if (dtype != SSWIN_F32) return N >= (hidden <= 384 ? 8192 : 32 * hidden);
     return N > 2 * 32 * (int64_t)device_cus() && !few_rows(dtype, N, hidden, D);
 }
 

@@ -105,6 +105,15 @@ def test_mlp_refuses_what_it_does_not_take():
         assert lib.sswin_mlp_backward(dtype, None, n, d, hidden, None, None, None, None, None, None, 1 << 30, None) != 0
 
 
+def test_mlp_is_preferred_later_with_many_hidden_channels():
+    """A wavefront's time grows with the hidden channels: 16 bit, beyond 384 of them the two layers are ahead up to 32 rows a channel."""
+    from sparseswin3d_amd import _lib
+    lib = _lib.load()
+    for d, hidden, rows in [(48, 192, 8192), (96, 384, 8192), (48, 384, 8192), (96, 416, 13312), (96, 768, 24576), (48, 1024, 32768)]:
+        for dtype in (1, 2):
+            assert lib.sswin_mlp_preferred(dtype, rows, d, hidden) and not lib.sswin_mlp_preferred(dtype, rows - 1, d, hidden)
+
+
 def test_mlp_refuses_results_over_rows_it_reads():
     """The last rows are read twice: a result in the place of an input would change them in between.  Refused on the host."""
     from sparseswin3d_amd import _lib
