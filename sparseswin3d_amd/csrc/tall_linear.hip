@@ -700,12 +700,17 @@ __global__ __launch_bounds__(WG_WAVES * 64) __attribute__((amdgpu_waves_per_eu(3
     };
     // Step s multiplies the planes of s and splits the rows of s + 1, requested two steps before; the rows of s + 3 are requested as
     // soon as those are split.
-    fetch_end(0, 0);
-    fetch_end(1, 1);
-    take(0, 0);
-    fetch_end(2, 0);
-    int s = 0;
     const int whole = (int)((row_end - row_begin) / WG_STEP_ROWS);
+    // the first three: rows checked one by one only where a step ends the chunk (1500 rows 96 -> 96 9.0 us, now 8.5)
+    auto fetch_any = [&](int s, int slot) {
+        if (s < whole) fetch(s, slot);
+        else if (s < steps) fetch_end(s, slot);
+    };
+    fetch_any(0, 0);
+    fetch_any(1, 1);
+    take(0, 0);
+    fetch_any(2, 0);
+    int s = 0;
     for (; s + 4 < whole; s += 2) {
 #pragma unroll
         for (int k = 0; k < 2; ++k) {
