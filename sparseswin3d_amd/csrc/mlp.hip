@@ -14,10 +14,10 @@
 // slope, du) goes through a tile of LDS per wavefront, so that it is touched in runs of 64 or 128 bytes (16 bits straight from
 // the accumulators, runs of 32 bytes: 225 000 rows fp16 48 channels 95 us, through the tile 69).
 //
-// Microseconds, two launches and one.  225 700 rows fp32 96 channels: forward 326 and 275, backward 294 and 246 (traffic alone at copy
-// rate 187 and 170; the matrix instructions alone about 120 at the clock they run at on such data).  fp16 48
-// channels, 225 000 rows: 89 and 69, 55 and 43 (55 and 38).  bf16 96 channels, inference, 112 700 rows: 66 and 46 (13; GELU on the
-// vector units 21).
+// Microseconds, two launches and one.  225 700 rows fp32 96 channels: forward 339 and 294, inference 296 and 219, backward 285 and 248 (traffic
+// alone at copy rate 187 and 170 for the first and last; the matrix cores are busy for 32 and 39 % of the launch, 190 000 cycles a SIMD).
+// fp16 48 channels, 225 000 rows: 89 and 69, 55 and 43 (55 and 38).  bf16 96 channels, inference, 112 700 rows: 65 and 45 (13; GELU on
+// the vector units 21).
 #include <algorithm>
 #include <initializer_list>
 #include <type_traits>
