@@ -90,18 +90,6 @@ template <> __device__ __forceinline__ float half_of<__hip_bfloat16>(uint32_t w,
 // that lanes which hold the chunks of one row write to different banks
 __device__ __forceinline__ int swz(int chunk) { return (chunk & 1) * 4 | (chunk & 2); }
 
-// workgroups b, b + 8, b + 16 ... share an XCD and its L2: the column blocks of one row block are dealt to such workgroups
-__device__ __forceinline__ void block_of(int groups, int& cg, int64_t& rb) {
-    const int b = blockIdx.x, chunk = 8 * groups, full = gridDim.x / chunk * chunk;
-    if (b < full) {
-        cg = (b / 8) % groups;
-        rb = b / chunk * 8 + b % 8;
-    } else {
-        cg = (b - full) % groups;
-        rb = full / groups + (b - full) / groups;
-    }
-}
-
 // ------------------------------------------------------------------------------------------
 // y [N, P] = last step of x [N, K] Wop, Wop [K, P] = W^T of W [P, K] (DOWN = false) or W [K, P] itself (DOWN = true)
 // ------------------------------------------------------------------------------------------

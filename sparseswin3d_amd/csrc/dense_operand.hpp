@@ -76,6 +76,104 @@ __device__ __forceinline__ void planes_of(const float (&v)[8], u32x4 (&out)[Op<T
     }
 }
 
+// fp32 values as two fp16 pieces, h rounded to nearest and l, 2^11 times what is left of it, also rounded: x 2^e = h + l 2^-11 to 2^-23 of
+// the power of two above x, so three products of 11 bits each take the place of six of 8: (h,h), and (l,h) (h,l) into sums of their own, for
+// their factor.  Half the matrix instructions, two thirds of the operand bytes and half the vector instructions.  What is lost: a bit of a
+// quarter of the values (6e-8 of a result, with l l); what is won: the matrix instructions do not round their sums to nearest, and
+// (h,h) is one of them a step, in place of six.  fp16 has five bits of exponent, so rows (and columns) are scaled by a power of two that
+// takes their largest value below 2^15; values down to 2^-25 of the largest keep all bits, since l is of h's size, and smaller ones are off by at
+// most 2^-50 of it.  Infinities and NaN leave NaN, as above.
+struct Pairs {
+    static constexpr float LOW = 0.00048828125f;                         // 2^-11
+    static __device__ __forceinline__ f32x16 mfma(const u32x4& a, const u32x4& b, const f32x16& c) {
+        return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8_t, a), __builtin_bit_cast(f16x8_t, b), c, 0, 0, 0);
+    }
+};
+__device__ __forceinline__ void split_pairs(const float (&v)[8], float scale, u32x4 (&out)[2]) {
+    typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const float a = v[2 * q], b = v[2 * q + 1];
+        f16x2 h = {(_Float16)(a * scale), (_Float16)(b * scale)};
+        asm("" : "+v"(h));                                               // (or each half is converted again for its rest)
+        const f16x2 l = {(_Float16)(fmaf(a, scale, -(float)h[0]) * 2048.f), (_Float16)(fmaf(b, scale, -(float)h[1]) * 2048.f)};
+        out[0][q] = __builtin_bit_cast(uint32_t, h);
+        out[1][q] = __builtin_bit_cast(uint32_t, l);
+    }
+}
+// exponent E with |v| < 2^E; of zero far below that of any value.  (Infinities and NaN: 0.)
+__device__ __forceinline__ int exponent_above(float most) { return most == 0.f ? -200 : __builtin_amdgcn_frexp_expf(most); }
+// scales stay normal numbers: rows of values below 2^-105 have fewer bits
+constexpr int PAIRS_MOST_SCALE = 120;
+__device__ __forceinline__ float power_of_two(int e) { return __builtin_amdgcn_ldexpf(1.f, e); }
+__device__ __forceinline__ float largest(const float (&v)[8]) {
+    float m = fabsf(v[0]);
+#pragma unroll
+    for (int e = 1; e < 8; ++e) m = fmaxf(m, fabsf(v[e]));
+    return m;
+}
+// of a lane and the one 32 lanes away
+__device__ __forceinline__ float largest_of_halves(float m) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, m), __builtin_bit_cast(uint32_t, m), false, false);
+    return fmaxf(__builtin_bit_cast(float, (uint32_t)r[0]), __builtin_bit_cast(float, (uint32_t)r[1]));
+}
+
+// Pieces of the columns [32 tile, 32 tile + 32) of Wop [K, P] (W [P, K] turned, or with DOWN W [K, P] itself), a scale per column, by a workgroup of
+// WAVES wavefronts: put(column, step of 16 channels, half of it, pieces); columns past the last repeat it.  Returns the exponent of the
+// scale of the lane's column, to all.
+template <bool DOWN, int WAVES, typename PUT>
+__device__ __forceinline__ int pairs_of_columns(const float* __restrict__ w, int K, int P, int tile, PUT put) {
+    constexpr int KEPT = 4;                                              // steps of a wavefront in registers: 64 WAVES channels are read once
+    __shared__ float most[WAVES][32];
+    const int wave = threadIdx.x >> 6, half = (threadIdx.x & 63) >> 5, l32 = threadIdx.x & 31;
+    const int col = min(tile * 32 + l32, P - 1), steps = K / 16;
+    auto load = [&](int ks, float (&v)[8]) {
+        const int k = ks * 16 + half * 8;
+        if constexpr (DOWN) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v[e] = w[(int64_t)(k + e) * P + col];
+        } else {
+            const f32x4* src = reinterpret_cast<const f32x4*>(w + (int64_t)col * K + k);
+            const f32x4 a = src[0], b = src[1];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v[e] = e < 4 ? a[e] : b[e - 4];
+        }
+    };
+    float kept[KEPT][8], m = 0.f;
+#pragma unroll
+    for (int i = 0; i < KEPT; ++i)
+        if (wave + i * WAVES < steps) load(wave + i * WAVES, kept[i]);
+#pragma unroll
+    for (int i = 0; i < KEPT; ++i)
+        if (wave + i * WAVES < steps) m = fmaxf(m, largest(kept[i]));
+    for (int ks = wave + KEPT * WAVES; ks < steps; ks += WAVES) {
+        float v[8];
+        load(ks, v);
+        m = fmaxf(m, largest(v));
+    }
+    m = largest_of_halves(m);
+    if (half == 0) most[wave][l32] = m;
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < WAVES; ++q) m = fmaxf(m, most[q][l32]);
+    const int e = min(15 - exponent_above(m), PAIRS_MOST_SCALE);
+    const float scale = power_of_two(e);
+    u32x4 p[2];
+#pragma unroll
+    for (int i = 0; i < KEPT; ++i)
+        if (wave + i * WAVES < steps) {
+            split_pairs(kept[i], scale, p);
+            put(tile * 32 + l32, wave + i * WAVES, half, p);
+        }
+    for (int ks = wave + KEPT * WAVES; ks < steps; ks += WAVES) {
+        float v[8];
+        load(ks, v);
+        split_pairs(v, scale, p);
+        put(tile * 32 + l32, ks, half, p);
+    }
+    return e;
+}
+
 // Pieces of an infinity hold a NaN, and so does every result one takes part in, as do pieces whose sums leave the range: fp32
 // results that come out NaN are formed again from the operands in plain fp32, in the order of the reduction, until they are
 // NaN there as well.
@@ -106,12 +204,31 @@ __device__ __forceinline__ f32x4 plain_products(const float* a, int64_t a_step, 
     return s;
 }
 
+// a last ragged tile is moved back to end at row N, tiles behind it repeat it: rows stored twice hold the same bits
+__device__ __forceinline__ int64_t tile_row(int64_t t, int64_t N) { return t * 32 + 32 <= N ? t * 32 : N - 32; }
+// workgroups b, b + 8, b + 16 ... share an XCD and its L2: the column blocks of one row block are dealt to such workgroups
+__device__ __forceinline__ void block_of(int groups, int& cg, int64_t& rb) {
+    const int b = blockIdx.x, chunk = 8 * groups, full = gridDim.x / chunk * chunk;
+    if (b < full) {
+        cg = (b / 8) % groups;
+        rb = b / chunk * 8 + b % 8;
+    } else {
+        cg = (b - full) % groups;
+        rb = full / groups + (b - full) / groups;
+    }
+}
+
 // 64 lanes x 16 bytes: lane l's piece lands at lds + 16 l
 __device__ __forceinline__ void copy_to_lds(const void* src, uint32_t lds) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(src) : "memory", "m0");
 }
 __device__ __forceinline__ uint32_t lds_address(const void* p) {
     return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)p;
+}
+// 16 bytes a lane, counted by the waits that follow.  The registers of a store this wide may not be written by the next
+// instruction, which the compiler sees to for its own stores only.
+__device__ __forceinline__ void store_counted(void* p, const u32x4& v) {
+    asm volatile("global_store_dwordx4 %0, %1, off\n\ts_nop 1" ::"v"(p), "v"(v) : "memory");
 }
 template <int N> __device__ __forceinline__ void wait_copies() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
 __device__ __forceinline__ void block_barrier() {

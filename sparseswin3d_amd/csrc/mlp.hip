@@ -9,13 +9,19 @@
 // formed transposed, z^T [hidden, tokens] = A x^T, so that an accumulator lane holds one token: with the rows of A permuted
 // (hidden_of) its 16 values of a 32-wide hidden tile are two runs of eight neighbours, which is the operand of the second product
 // y^T += B z^T in place.  No exchange between lanes, no round through LDS.  x stays in registers for the whole launch (96 channels:
-// 24 registers, as three pieces of fp32 72), y accumulates in registers, A and B pass from L2 into LDS a step of 32 hidden
+// 24 registers, as two pieces of fp32 48), y accumulates in registers, A and B pass from L2 into LDS a step of 32 hidden
 // channels at a time, the next step in flight, shared by the wavefronts of the workgroup.  What is stored or read per hidden value (g,
 // slope, du) goes through a tile of LDS per wavefront, so that it is touched in runs of 64 or 128 bytes (16 bits straight from
 // the accumulators, runs of 32 bytes: 225 000 rows fp16 48 channels 95 us, through the tile 69).
 //
-// Microseconds, two launches and one.  225 700 rows fp32 96 channels: forward 339 and 294, inference 296 and 219, backward 285 and 248 (traffic
-// alone at copy rate 187 and 170 for the first and last; the matrix cores are busy for 32 and 39 % of the launch, 190 000 cycles a SIMD).
+// fp32 operands are pairs of fp16 (Pairs of dense_operand.hpp).  A scale per row of x, found when the row is loaded, and per row of A and
+// B, found by the launch that splits them; the hidden values' scale follows the largest of the token so far, and since a token's
+// results lie in its own lanes, dropping it is a product a register.
+//
+// Microseconds, two launches (of three bf16 pieces) and one.  225 700 rows fp32 96 channels: forward 339 and 267, inference 296 and 189, backward
+// 285 and 199 (with three pieces here 308, 227 and 245; traffic alone at copy rate 187 and 170 for the first and last).  Error against float64 (2-norms) of
+// y 1.0e-7, three pieces 1.8e-7, of dx 1.9e-7 and 3.4e-7.  What bounds fp32 now: the stores of training, GELU on the vector units (about 26
+// instructions of 45 a hidden value) and the products, of which two wavefronts a SIMD cover two thirds with each other.
 // fp16 48 channels, 225 000 rows: 89 and 69, 55 and 43 (55 and 38).  bf16 96 channels, inference, 112 700 rows: 65 and 45 (13; GELU on
 // the vector units 21).
 #include <algorithm>
@@ -36,6 +42,7 @@ struct MlpArgs {
     int hidden;
     const uint16_t* a;         // [planes][hidden, D]
     const uint16_t* b;         // [planes][D, hidden]
+    const int *ea, *eb;        // fp32: exponents of the scales of their rows
     const float *wa, *wb;      // fp32: what the pieces are of, forward [hidden, D] and [D, hidden], backward turned
     const void* bias_a;        // [hidden] or null
     const void* bias_b;        // [D] or null
@@ -55,19 +62,29 @@ enum { MLP_INFER, MLP_TRAIN, MLP_BACKWARD };
 // then row 16 s + 8 h + e
 __device__ __forceinline__ int hidden_of(int i) { return (i & 0x13) | (i & 4) << 1 | (i & 8) >> 1; }
 
-// 16 bytes a lane, counted by the waits of the kernel below.  The registers of a store this wide may not be written by the next
-// instruction, which the compiler sees to for its own stores only.
-__device__ __forceinline__ void store_counted(void* p, const u32x4& v) {
-    asm volatile("global_store_dwordx4 %0, %1, off\n\ts_nop 1" ::"v"(p), "v"(v) : "memory");
-}
+template <typename T> constexpr int MLP_PL = sizeof(T) == 4 ? 2 : 1;     // planes of an operand
 
-template <typename T> __device__ __forceinline__ void planes_at(const T* p, u32x4 (&x)[Op<T>::PL]) {
-    if constexpr (Op<T>::PL == 3) {
-        const f32x4 lo = *reinterpret_cast<const f32x4*>(p), hi = *reinterpret_cast<const f32x4*>(p + 4);
-        const float v[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-        planes_of<T>(v, x);
+// a wavefront's rows as operands; the exponent of the scale of the lane's row (fp32)
+template <typename T, int KS> __device__ __forceinline__ int load_rows(const T* p, u32x4 (&x)[KS][MLP_PL<T>]) {
+    if constexpr (sizeof(T) == 4) {
+        float v[KS][8], m = 0.f;
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+            const f32x4 lo = *reinterpret_cast<const f32x4*>(p + ks * 16), hi = *reinterpret_cast<const f32x4*>(p + ks * 16 + 4);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v[ks][e] = e < 4 ? lo[e] : hi[e - 4];
+        }
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) m = fmaxf(m, largest(v[ks]));
+        const int e = min(15 - exponent_above(largest_of_halves(m)), PAIRS_MOST_SCALE);
+        const float scale = power_of_two(e);
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) split_pairs(v[ks], scale, x[ks]);
+        return e;
     } else {
-        x[0] = *reinterpret_cast<const u32x4*>(p);
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) x[ks][0] = *reinterpret_cast<const u32x4*>(p + ks * 16);
+        return 0;
     }
 }
 
@@ -170,9 +187,6 @@ template <typename T> __device__ __forceinline__ void stage_biases(const MlpArgs
     for (int e = threadIdx.x; e < g.hidden; e += (int)blockDim.x) bias[e] = g.bias_a ? to_acc(static_cast<const T*>(g.bias_a)[e]) : 0.f;
     for (int e = threadIdx.x; e < D; e += (int)blockDim.x) bias[g.hidden + e] = g.bias_b ? to_acc(static_cast<const T*>(g.bias_b)[e]) : 0.f;
 }
-// a last ragged tile is moved back to end at row N, tiles behind it repeat it: rows stored twice hold the same bits
-__device__ __forceinline__ int64_t tile_row(int64_t t, int64_t N) { return t * 32 + 32 <= N ? t * 32 : N - 32; }
-
 // fp32: y where the pieces left NaN, again in plain fp32 as in dense.hip (plain_products), and the hidden values before it with what is
 // stored of them.  A hidden value that came out NaN makes every y of its token NaN, so y alone tells, once a launch.  Inference has
 // no hidden values in memory and forms all of these tokens again.
@@ -243,23 +257,25 @@ template <int D, int MODE> __device__ __forceinline__ void plain_rows(const MlpA
 // A step is 32 hidden channels.  The wait for the next step's A and B leaves the stores of this step in flight; it counts them, so they
 // are inline assembly.
 template <typename T, int D, int MODE, int WAVES> struct MlpLds {
-    static constexpr int PIECES = Op<T>::PL * (D / 16 + 2 * ((D + 31) / 32));   // of 64 x 16 bytes, a step's A and B
+    static constexpr int PIECES = MLP_PL<T> * (D / 16 + 2 * ((D + 31) / 32));   // of 64 x 16 bytes, a step's A and B
     // of 16 bytes, a wavefront's tiles: two of hidden values, at least one of y.  Inference: y leaves through the place of A and B
     // where it is large enough
     static constexpr bool SHARED = MODE == MLP_INFER && WAVES * 256 <= 2 * PIECES * 64;
     static constexpr int OWN = SHARED ? 0 : std::max(256, 2 * HiddenTile<T>::PIECES);
-    static size_t bytes(int hidden) { return (size_t)2 * PIECES * 1024 + (size_t)(hidden + D) * 4 + (size_t)WAVES * OWN * 16; }
+    static constexpr int PER_CHANNEL = sizeof(T) == 4 ? 2 : 1;           // its bias, and fp32 the exponent of its scale
+    static size_t bytes(int hidden) { return (size_t)2 * PIECES * 1024 + (size_t)(hidden + D) * 4 * PER_CHANNEL + (size_t)WAVES * OWN * 16; }
 };
 template <typename T, typename TO, int D, int MODE, int WAVES, int OCC>
 __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(OCC, OCC))) void mlp_kernel(MlpArgs g) {
     using L = MlpLds<T, D, MODE, WAVES>;
     using H = HiddenTile<T>;
-    constexpr int PL = Op<T>::PL, KS = D / 16, CT = (D + 31) / 32, PA = KS * PL, PIECES = L::PIECES;
+    constexpr int PL = MLP_PL<T>, KS = D / 16, CT = (D + 31) / 32, PA = KS * PL, PIECES = L::PIECES;
     constexpr int STORES = MODE == MLP_INFER ? 0 : MODE == MLP_TRAIN ? 2 * H::MOVES : H::MOVES;
     extern __shared__ __attribute__((aligned(16))) u32x4 lds[];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, half = lane >> 5, l32 = lane & 31;
     float* const bias = reinterpret_cast<float*>(lds + 2 * PIECES * 64); // [hidden] and [D]
-    u32x4* const tiles = L::SHARED ? lds + wave * 256 : lds + 2 * PIECES * 64 + (g.hidden + D) / 4 + wave * L::OWN;
+    int* const exps = reinterpret_cast<int*>(bias + g.hidden + D);       // fp32: the same
+    u32x4* const tiles = L::SHARED ? lds + wave * 256 : lds + 2 * PIECES * 64 + (g.hidden + D) * L::PER_CHANNEL / 4 + wave * L::OWN;
     const int64_t behind = (int64_t)blockIdx.x - g.full, row0 = tile_row(behind < 0 ? (int64_t)blockIdx.x * WAVES + wave : g.full * WAVES + behind * g.some + wave, g.N);
     const int64_t plane = (int64_t)g.hidden * D;
     const uint32_t lane_a = (uint32_t)(hidden_of(l32) * D + half * 8);
@@ -278,6 +294,8 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(OCC,
     const int steps = g.hidden / 32;
     request(0);
     if constexpr (MODE != MLP_BACKWARD) stage_biases<T>(g, D, bias);
+    if constexpr (PL == 2)
+        for (int c = threadIdx.x; c < g.hidden + D; c += WAVES * 64) exps[c] = c < g.hidden ? g.ea[c] : g.eb[c - g.hidden];
     if (behind >= 0 && wave >= g.some) {                                 // without tokens: only brings A and B
         wait_copies<0>();
         for (int step = 0; step < steps; ++step) {
@@ -289,8 +307,7 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(OCC,
         return;
     }
     u32x4 x[KS][PL];
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) planes_at<T>(static_cast<const T*>(g.x) + (row0 + l32) * D + ks * 16 + half * 8, x[ks]);
+    const int ex = load_rows<T, KS>(static_cast<const T*>(g.x) + (row0 + l32) * D + half * 8, x);
     const int64_t mem = (row0 + H::mem_row()) * g.hidden + H::mem_col();
     auto load_tile = [&](int step) {                                     // of slope
 #pragma unroll
@@ -305,12 +322,14 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(OCC,
 #pragma unroll
         for (int i = 0; i < H::MOVES; ++i) store_counted(static_cast<T*>(to) + mem + (int64_t)i * H::STEP_ROWS * g.hidden + step * 32, v[i]);
     };
-    f32x16 y[CT];
+    f32x16 y[CT], y_low[PL == 2 ? CT : 1];
 #pragma unroll
-    for (int j = 0; j < CT; ++j) y[j] = f32x16{0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+    for (int j = 0; j < CT; ++j) y[j] = y_low[PL == 2 ? j : 0] = f32x16{0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+    int eh = 300;                                                        // fp32: exponent of the scale of the row's hidden values
+    float hidden_scale = 0.f;
     if constexpr (MODE == MLP_BACKWARD) load_tile(0);
     wait_copies<0>();
-    if (PL == 3 && wave < WAVES / 2) __builtin_amdgcn_s_setprio(1);      // the two wavefronts of a SIMD at different places of a step
+    if (PL == 2 && wave < WAVES / 2) __builtin_amdgcn_s_setprio(1);      // the two wavefronts of a SIMD at different places of a step
     for (int step = 0; step < steps; ++step) {
         block_barrier();                                                 // this buffer is there, the other one is free
         if (step + 1 < steps) {
@@ -320,7 +339,7 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(OCC,
         u32x4* const tile = tiles + (MODE == MLP_BACKWARD ? (step & 1) * H::PIECES : 0);   // du takes the place of its slope
         const u32x4* const pieces = lds + (step & 1) * PIECES * 64 + lane;
         // z^T: the pieces of A are read a slice of 16 channels ahead of its products
-        f32x16 z = f32x16{0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+        f32x16 z = f32x16{0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0}, z_low = z;
         u32x4 a[2][PL];
 #pragma unroll
         for (int q = 0; q < PL; ++q) a[0][q] = pieces[q * 64];
@@ -330,19 +349,34 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(OCC,
             if (ks + 1 < KS)
 #pragma unroll
                 for (int q = 0; q < PL; ++q) a[(ks + 1) & 1][q] = pieces[((ks + 1) * PL + q) * 64];
-#pragma unroll
-            for (int p = 0; p < Op<T>::NP; ++p) z = Op<T>::mfma(a[ks & 1][Op<T>::PA[p]], x[ks][Op<T>::PB[p]], z);
+            if constexpr (PL == 2) {
+                z_low = Pairs::mfma(a[ks & 1][1], x[ks][0], z_low);
+                z = Pairs::mfma(a[ks & 1][0], x[ks][0], z);
+                z_low = Pairs::mfma(a[ks & 1][0], x[ks][1], z_low);
+            } else {
+                z = Op<T>::mfma(a[ks & 1][0], x[ks][0], z);
+            }
             __builtin_amdgcn_sched_group_barrier(0x100, PL, 0);
-            __builtin_amdgcn_sched_group_barrier(0x008, Op<T>::NP, 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, PL == 2 ? 3 : 1, 0);
         }
+        if constexpr (PL == 2) {
 #pragma unroll
-        for (int s = 0; s < 2; ++s) {
-            float v[8], u[8];
+            for (int s = 0; s < 2; ++s) {
+                const int4* const e8 = reinterpret_cast<const int4*>(exps + step * 32 + s * 16 + half * 8);
+                const int4 lo = e8[0], hi = e8[1];
+                const int ew[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+#pragma unroll
+                for (int e = 0; e < 8; ++e) z[s * 8 + e] = __builtin_amdgcn_ldexpf(fmaf(z_low[s * 8 + e], Pairs::LOW, z[s * 8 + e]), -(ex + ew[e]));
+            }
+        }
+        auto step_between = [&](int s, float (&v)[8]) {
+            float u[8];
             between<T, MODE>(z, s, bias + step * 32, tile, v, u);
             if constexpr (MODE != MLP_INFER) H::put(tile, s, v);
             if constexpr (MODE == MLP_TRAIN) H::put(tile + H::PIECES, s, u);
-            u32x4 h[PL], w[2][PL];
-            planes_of<T>(v, h);
+        };
+        auto second_layer = [&](int s, const u32x4 (&h)[PL]) {
+            u32x4 w[2][PL];
             auto read = [&](int j) {
 #pragma unroll
                 for (int q = 0; q < PL; ++q) w[j & 1][q] = pieces[(PA + (s * CT + j) * PL + q) * 64];
@@ -351,8 +385,43 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(OCC,
 #pragma unroll
             for (int j = 0; j < CT; ++j) {
                 if (j + 1 < CT) read(j + 1);
+                if constexpr (PL == 2) {
+                    y_low[j] = Pairs::mfma(w[j & 1][1], h[0], y_low[j]);
+                    y[j] = Pairs::mfma(w[j & 1][0], h[0], y[j]);
+                    y_low[j] = Pairs::mfma(w[j & 1][0], h[1], y_low[j]);
+                } else {
+                    y[j] = Op<T>::mfma(w[j & 1][0], h[0], y[j]);
+                }
+            }
+        };
+        u32x4 h[PL];
+        if constexpr (PL == 2) {
+            float v[2][8];
+            step_between(0, v[0]);
+            step_between(1, v[1]);
+            // the scale follows the largest value seen: where a step's would leave fp16's range it drops, and the sums with it
+            const int above = exponent_above(largest_of_halves(fmaxf(largest(v[0]), largest(v[1]))));
+            if (__any(above + eh > 15)) {
+                const int now = above + eh > 15 ? min(11 - above, PAIRS_MOST_SCALE) : eh;
+                const float factor = power_of_two(now - eh);
+                eh = now, hidden_scale = power_of_two(now);
 #pragma unroll
-                for (int p = 0; p < Op<T>::NP; ++p) y[j] = Op<T>::mfma(w[j & 1][Op<T>::PA[p]], h[Op<T>::PB[p]], y[j]);
+                for (int j = 0; j < CT; ++j)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) y[j][r] *= factor, y_low[j][r] *= factor;
+            }
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+                split_pairs(v[s], hidden_scale, h);
+                second_layer(s, h);
+            }
+        } else {
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+                float v[8];
+                step_between(s, v);
+                planes_of<T>(v, h);
+                second_layer(s, h);
             }
         }
         if constexpr (MODE != MLP_INFER) {
@@ -364,12 +433,16 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(OCC,
         if (step + 1 < steps) wait_copies<STORES>();                     // all but the stores of this step
     }
     if constexpr (L::SHARED) block_barrier();                    // A and B have been read
-    if constexpr (PL == 3) {
+    if constexpr (PL == 2) {
         f32x4 any = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int j = 0; j < CT; ++j)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) any[r & 3] += y[j][r];
+            for (int r = 0; r < 16; ++r) {
+                const int ew = exps[g.hidden + j * 32 + r / 8 * 16 + half * 8 + r % 8];
+                y[j][r] = __builtin_amdgcn_ldexpf(fmaf(y_low[j][r], Pairs::LOW, y[j][r]), -(eh + ew));
+                any[r & 3] += y[j][r];
+            }
         if (__any(nan_among(any))) plain_rows<D, MODE>(g, row0, bias, tiles, y);
     }
     store_y<TO, D, MODE>(g, y, row0, bias + g.hidden, tiles);
@@ -477,12 +550,10 @@ template <typename T> int rows_once(const T* x, int64_t N, int D, const T* w, co
 template int rows_once<__half>(const __half*, int64_t, int, const __half*, const __half*, int, __half*, hipStream_t);
 template int rows_once<__hip_bfloat16>(const __hip_bfloat16*, int64_t, int, const __hip_bfloat16*, const __hip_bfloat16*, int, __hip_bfloat16*, hipStream_t);
 
-// A and B as the kernel reads them: fp32 weights as planes of their pieces, weights of the backward turned.  A thread per pair of
-// neighbours of a row.
+// A and B of the backward, weights turned, 16 bit: a thread per pair of neighbours of a row
 template <typename T>
-__global__ __launch_bounds__(256) void mlp_weights_kernel(const T* __restrict__ wa, const T* __restrict__ wb, bool turned, int D, int hidden,
-                                                          uint16_t* __restrict__ a, uint16_t* __restrict__ b) {
-    constexpr int PL = Op<T>::PL;
+__global__ __launch_bounds__(256) void mlp_weights_kernel(const T* __restrict__ wa, const T* __restrict__ wb, int D, int hidden, uint16_t* __restrict__ a,
+                                                          uint16_t* __restrict__ b) {
     const int64_t pairs = (int64_t)D * hidden / 2, i = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (i >= 2 * pairs) return;
     const bool second = i >= pairs;
@@ -490,16 +561,21 @@ __global__ __launch_bounds__(256) void mlp_weights_kernel(const T* __restrict__ 
     const int cols = second ? hidden : D, rows = second ? D : hidden;    // of the result
     const int64_t r = e / cols, c = e % cols;
     const T* w = second ? wb : wa;
-    const T v0 = turned ? w[c * rows + r] : w[e], v1 = turned ? w[(c + 1) * rows + r] : w[e + 1];
-    uint16_t* to = (second ? b : a) + e;
-    if constexpr (PL == 3) {
-        uint32_t p[3];
-        split2(v0, v1, p[0], p[1], p[2]);
+    const T v0 = w[c * rows + r], v1 = w[(c + 1) * rows + r];
+    *reinterpret_cast<uint32_t*>((second ? b : a) + e) = (uint32_t)__builtin_bit_cast(uint16_t, v0) | (uint32_t)__builtin_bit_cast(uint16_t, v1) << 16;
+}
+// fp32: the pieces of both, and the exponents of their rows' scales; a workgroup per 32 rows
+template <bool TURNED>
+__global__ __launch_bounds__(512) void mlp_pairs_kernel(const float* __restrict__ wa, const float* __restrict__ wb, int D, int hidden, uint16_t* __restrict__ a,
+                                                        uint16_t* __restrict__ b, int* __restrict__ ea, int* __restrict__ eb) {
+    const bool second = (int)blockIdx.x >= hidden / 32;
+    const int tile = second ? (int)blockIdx.x - hidden / 32 : (int)blockIdx.x, rows = second ? D : hidden, cols = second ? hidden : D;
+    uint16_t* const to = second ? b : a;
+    const int e = pairs_of_columns<TURNED, 8>(second ? wb : wa, cols, rows, tile, [&](int row, int ks, int half, const u32x4 (&p)[2]) {
 #pragma unroll
-        for (int q = 0; q < 3; ++q) *reinterpret_cast<uint32_t*>(to + q * 2 * pairs) = p[q];
-    } else {
-        *reinterpret_cast<uint32_t*>(to) = (uint32_t)__builtin_bit_cast(uint16_t, v0) | (uint32_t)__builtin_bit_cast(uint16_t, v1) << 16;
-    }
+        for (int q = 0; q < 2; ++q) *reinterpret_cast<u32x4*>(to + (int64_t)q * D * hidden + (int64_t)row * cols + ks * 16 + half * 8) = p[q];
+    });
+    if (threadIdx.x < 32) (second ? eb : ea)[tile * 32 + threadIdx.x] = e;
 }
 
 template <typename T, typename TO, int D, int MODE, int WAVES, int OCC> static int launch_mlp_as(MlpArgs g, hipStream_t s) {
@@ -523,10 +599,20 @@ template <typename T, typename TO, int MODE> static int launch_mlp(const MlpArgs
     else return launch_mlp_as<T, TO, 96, MODE, 4, MODE == MLP_INFER ? 4 : 3>(g, s);
 }
 
-template <typename T>
-static int launch_weights(const void* wa, const void* wb, bool turned, int D, int hidden, uint16_t* a, uint16_t* b, hipStream_t s) {
-    hipLaunchKernelGGL((mlp_weights_kernel<T>), dim3((unsigned)(((int64_t)D * hidden + 255) / 256)), dim3(256), 0, s, static_cast<const T*>(wa),
-                       static_cast<const T*>(wb), turned, D, hidden, a, b);
+// fp32: two planes of A, two of B, then the exponents of their rows
+template <typename T> static int launch_weights(MlpArgs& g, const void* wa, const void* wb, bool turned, int D, int hidden, void* ws, hipStream_t s) {
+    uint16_t *a = static_cast<uint16_t*>(ws), *b = a + (size_t)MLP_PL<T> * D * hidden;
+    g.a = a, g.b = b;
+    if constexpr (sizeof(T) == 4) {
+        int *ea = reinterpret_cast<int*>(b + (size_t)2 * D * hidden), *eb = ea + hidden;
+        g.ea = ea, g.eb = eb;
+        const dim3 grid((unsigned)((hidden + D) / 32));
+        auto* k = turned ? mlp_pairs_kernel<true> : mlp_pairs_kernel<false>;
+        hipLaunchKernelGGL(k, grid, dim3(512), 0, s, static_cast<const float*>(wa), static_cast<const float*>(wb), D, hidden, a, b, ea, eb);
+    } else {
+        hipLaunchKernelGGL((mlp_weights_kernel<T>), dim3((unsigned)(((int64_t)D * hidden + 255) / 256)), dim3(256), 0, s, static_cast<const T*>(wa),
+                           static_cast<const T*>(wb), D, hidden, a, b);
+    }
     return launch_ok("mlp weights");
 }
 
@@ -569,10 +655,9 @@ int sswin_mlp_supported(int dtype, int64_t N, int D, int hidden) {
 // 33.4 -> 23.5 us; bf16 96 channels, 8000 rows 41.8 -> 40.0, inference 20.4 -> 18.5, 4000 rows 33.9 -> 38.4 and 16.3 -> 18.2); a wavefront's
 // time grows with the hidden channels, that of the two layers' tiles with all of their work, so with more than 384 later (bf16 96 channels,
 // forward and backward, 768 hidden: 20 000 rows 66 -> 76, 50 000 114 -> 91; 1024 hidden 8192 57 -> 91, 50 000 142 -> 121).  fp32: a
-// wavefront takes about 46 us forward and 34 backward alone on its SIMD, so from three wavefronts a compute unit on (forward and
-// backward of 8192 rows 60 -> 80 us, 16 384 88 -> 89, 24 576 101 -> 93, 32 768 116 -> 101, 65 536 189 -> 152, 81 920 248 -> 241, 225 700
-// 633 -> 543), and only behind the rows up to which the second layer is one of few rows: there eight wavefronts share its sums, and
-// their error against float64 is 1.2e-7 of y and 2.3e-7 of dx, here 1.9e-7 and 3.3e-7; in larger tiles 1.9e-7 and 3.6e-7.
+// wavefront takes about 44 us forward and 30 backward alone on its SIMD, so from three wavefronts a compute unit on (forward and
+// backward of 8192 rows 60 -> 80 us, 16 384 88 -> 89, as three bf16 pieces; 24 576 101 -> 76, 225 700 633 -> 466), and only behind the rows up to
+// which the second layer is one of few rows.
 int sswin_mlp_preferred(int dtype, int64_t N, int D, int hidden) {
     if (!sswin_mlp_supported(dtype, N, D, hidden)) return 0;
     if (dtype != SSWIN_F32) return N >= (hidden <= 384 ? 8192 : 32 * hidden);
@@ -581,7 +666,7 @@ int sswin_mlp_preferred(int dtype, int64_t N, int D, int hidden) {
 
 size_t sswin_mlp_workspace_bytes(int dtype, int D, int hidden, int backward) {
     const size_t plane = (size_t)D * hidden * 2;
-    return dtype == SSWIN_F32 ? 6 * plane : backward ? 2 * plane : 0;
+    return dtype == SSWIN_F32 ? 4 * plane + (size_t)(hidden + D) * sizeof(int) : backward ? 2 * plane : 0;
 }
 
 int sswin_mlp_forward(int dtype, int out_dtype, const void* x, int64_t N, int D, int hidden, const void* w1, const void* b1, const void* w2, const void* b2,
@@ -593,13 +678,10 @@ int sswin_mlp_forward(int dtype, int out_dtype, const void* x, int64_t N, int D,
     const size_t rows = (size_t)N * D * value_size(dtype), out_rows = (size_t)N * D * value_size(out_dtype), inner = (size_t)N * hidden * value_size(dtype);
     SSWIN_CHECK(apart({{y, out_rows}, {act, inner}, {slope, inner}}, {{x, rows}, {residual, out_rows}}), "mlp_forward: results may not overlap x or residual");
     hipStream_t s = static_cast<hipStream_t>(stream);
-    const uint16_t *a = static_cast<const uint16_t*>(w1), *b = static_cast<const uint16_t*>(w2);
-    if (dtype == SSWIN_F32) {
-        uint16_t* planes = static_cast<uint16_t*>(ws);
-        a = planes, b = planes + (size_t)3 * D * hidden;
-        if (int rc = launch_weights<float>(w1, w2, false, D, hidden, planes, planes + (size_t)3 * D * hidden, s)) return rc;
-    }
-    const MlpArgs g = {x, N, hidden, a, b, static_cast<const float*>(w1), static_cast<const float*>(w2), b1, b2, nullptr, residual, act, slope, y, 0, 0};
+    MlpArgs g = {x, N, hidden, static_cast<const uint16_t*>(w1), static_cast<const uint16_t*>(w2), nullptr, nullptr, static_cast<const float*>(w1),
+                 static_cast<const float*>(w2), b1, b2, nullptr, residual, act, slope, y, 0, 0};
+    if (dtype == SSWIN_F32)
+        if (int rc = launch_weights<float>(g, w1, w2, false, D, hidden, ws, s)) return rc;
 #define MLP_RUN(T, TO) return act ? launch_mlp<T, TO, MLP_TRAIN>(g, D, s) : launch_mlp<T, TO, MLP_INFER>(g, D, s)
     if (dtype == SSWIN_F32 && out_dtype == SSWIN_F32) MLP_RUN(float, float);
     if (dtype == SSWIN_F16 && out_dtype == SSWIN_F16) MLP_RUN(__half, __half);
@@ -619,12 +701,12 @@ int sswin_mlp_backward(int dtype, const void* dy, int64_t N, int D, int hidden, 
     const size_t rows = (size_t)N * D * value_size(dtype), inner = (size_t)N * hidden * value_size(dtype);
     SSWIN_CHECK(apart({{du, inner}, {dx, rows}}, {{dy, rows}, {slope, inner}}), "mlp_backward: results may not overlap dy or slope");
     hipStream_t s = static_cast<hipStream_t>(stream);
-    uint16_t *a = static_cast<uint16_t*>(ws), *b = a + sswin_mlp_workspace_bytes(dtype, D, hidden, 1) / 4;
-    const MlpArgs g = {dy, N, hidden, a, b, static_cast<const float*>(w2), static_cast<const float*>(w1), nullptr, nullptr, slope, nullptr, du, nullptr, dx, 0, 0};
-#define MLP_RUN(T)                                                                     \
-    do {                                                                               \
-        if (int rc = launch_weights<T>(w2, w1, true, D, hidden, a, b, s)) return rc;   \
-        return launch_mlp<T, T, MLP_BACKWARD>(g, D, s);                                \
+    MlpArgs g = {dy, N, hidden, nullptr, nullptr, nullptr, nullptr, static_cast<const float*>(w2), static_cast<const float*>(w1), nullptr, nullptr, slope,
+                 nullptr, du, nullptr, dx, 0, 0};
+#define MLP_RUN(T)                                                                      \
+    do {                                                                                \
+        if (int rc = launch_weights<T>(g, w2, w1, true, D, hidden, ws, s)) return rc;   \
+        return launch_mlp<T, T, MLP_BACKWARD>(g, D, s);                                 \
     } while (0)
     if (dtype == SSWIN_F32) MLP_RUN(float);
     if (dtype == SSWIN_F16) MLP_RUN(__half);

@@ -174,6 +174,38 @@ def test_mlp_fp32_sums_no_less_exactly_than_two_layers(N):
         assert errors[0] <= 1.02 * errors[1], (what, errors)
 
 
+@pytest.mark.parametrize("span", [20, -20])
+@pytest.mark.parametrize("N,hidden", [(33, 64), (3001, 384)])
+def test_mlp_fp32_scales(N, hidden, span):
+    """fp32 operands are split into fp16 pieces, scaled by row: rows of any size; hidden values that grow or fall by 2^20 over the hidden
+    channels, met by weights that fall or grow as much, so that each counts the same; rows whose first hidden values are zero.  Bounds as
+    above: the sums of absolute products."""
+    from sparseswin3d_amd import _lib
+    lib = _lib.load()
+    D, gen = 96, torch.Generator().manual_seed(N)
+    rand = lambda *s, std=1.0: torch.randn(*s, generator=gen) * std
+    ramp = torch.exp2(torch.linspace(-span / 2, span / 2, hidden).round())
+    size = torch.exp2(torch.randint(-60, 61, (N, 1), generator=gen).float())
+    dy, w1, w2, slope = rand(N, D) * size, rand(hidden, D) / ramp[:, None], rand(D, hidden), rand(N, hidden) * ramp
+    slope[N // 2, :hidden - 5] = 0
+    dy, w1, w2, slope = (t.cuda() for t in (dy, w1, w2, slope))
+    du64 = (dy.double() @ w2.double()) * slope.double()
+    du_err = 2e-6 * (dy.double().abs() @ w2.double().abs()) * slope.double().abs()
+    dx_err = du_err @ w1.double().abs() + 2e-6 * (du64.abs() @ w1.double().abs())
+    du, dx = _empty((N, hidden), torch.float32), _empty((N, D), torch.float32)
+    ws, nb = _workspace(lib, dy, hidden, 1)
+    _lib.check(lib.sswin_mlp_backward(0, _ptr(dy), N, D, hidden, _ptr(w1), _ptr(w2), _ptr(slope), _ptr(du), _ptr(dx), _ptr(ws), nb, _stream()))
+    _check(du, du64, du_err + 1e-30, "du")
+    _check(dx, du64 @ w1.double(), dx_err + 1e-30, "dx")
+    x, w1, w2 = dy / size.cuda() * torch.exp2(torch.randint(-8, 9, (N, 1), generator=gen).float()).cuda(), w1 * ramp[:, None].cuda() ** 2, w2 / ramp.cuda()
+    g64 = _gelu(x.double() @ w1.double().t())[0]
+    g_err = 2e-6 * (x.double().abs() @ w1.double().abs().t()) + 1e-6 * g64.abs().clamp(max=1)
+    y = _empty((N, D), torch.float32)
+    ws, nb = _workspace(lib, x, hidden, 0)
+    _lib.check(lib.sswin_mlp_forward(0, 0, _ptr(x), N, D, hidden, _ptr(w1), None, _ptr(w2), None, None, _ptr(y), None, None, _ptr(ws), nb, _stream()))
+    _check(y, g64 @ w2.double().t(), g_err @ w2.double().abs().t() + 2e-6 * (g64.abs() @ w2.double().abs().t()) + 1e-30, "y")
+
+
 def _same_class(got, ref, bound, what):
     """Finite where float64 is (to the bound), the same infinities, NaN where float64 has NaN."""
     got, finite = got.double(), ref.isfinite()
