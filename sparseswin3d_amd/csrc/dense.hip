@@ -7,6 +7,7 @@
 // weigh at least 2^-16 of the leading one; what is dropped is below 2^-23 of the product.  Infinities and NaN give what they give
 // in plain fp32 (plain_products).
 //
+// (dense_pairs.hip: layers of at least 96 reduction channels, with a workspace, as two fp16 pieces.)
 // dense_rows_kernel (fp32): a workgroup of WM wavefronts owns BM = 32 MT WM rows and 96 columns.  Both operands pass through
 // registers, where they are split, into LDS in matrix operand order, [row tile][plane][lane] pieces of 16 bytes, so that every
 // operand read is one conflict-free 16-byte read per lane; 32 columns of the reduction at a time, the next 32 in flight
@@ -1072,6 +1073,9 @@ static int launch_forward(const void* x, int64_t N, int K, const void* w, int P,
     if constexpr (Op<T>::PL == 3) {
         // 96 channels: the kernel that keeps Wop in LDS (219 000 rows, 96 -> 288: 89 us against 120 here, with a residual 133 and 202)
         if (K == 96 && P % 96 == 0) return staged_layer_96(xp, N, wp, P, DOWN, EPI, ep, s);
+        // fp16 pairs, from the reductions on whose sums come out as exactly: error against float64 (2-norms) with 96 channels 7.8e-8 and
+        // 1.0e-7 here, 144 1.1e-7 and 1.75e-7 (turned); 48 channels of three bf16 pieces 6.9e-8, of pairs 7.1e-8 and more
+        if (pairs_takes(K) && ws_bytes >= pairs_workspace_bytes(K, P)) return pairs_layer<EPI, DOWN>(xp, N, K, wp, P, ep, ws, s);
         // wavefronts per SIMD: what the registers allow without spilling (four: forward equal, input gradient 89 us against 40)
         return launch_rows<EPI, DOWN, 4, 1, 3>(xp, N, K, wp, P, ep, s);
     } else {
@@ -1258,6 +1262,7 @@ int sswin_dense_supported(int dtype, int P, int K) {
 size_t sswin_dense_forward_workspace_bytes(int dtype, int64_t N, int K, int P) {
     if (N <= 0 || !sswin_dense_supported(dtype, P, K)) return 0;
     const Cut c = cut_of(dtype, N, K, P);
+    if (dtype == SSWIN_F32) return c.few || !pairs_takes(K) || (K == 96 && P % 96 == 0) ? 0 : pairs_workspace_bytes(K, P);
     return c.ksplit > 1 ? (size_t)c.ksplit * N * P * sizeof(float) : 0;
 }
 

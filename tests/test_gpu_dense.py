@@ -481,6 +481,63 @@ def test_dense_fp32_weight_gradient_of_values_that_are_not_finite(N, P, K, value
     _same_class(db, d.sum(0), d.abs().sum(0), "db")
 
 
+# fp32 layers of at least 96 reduction channels (pairs of fp16): whole steps of 32 and a last one of 16, columns that end inside a tile, several
+# column blocks; one row past a workgroup's
+PAIRS = [(19201, 96, 112), (20001, 144, 48), (20001, 208, 304), (9601, 576, 192)]
+
+
+@pytest.mark.parametrize("N,K,P", PAIRS)
+@pytest.mark.parametrize("value", [float("inf"), float("nan"), 3.4028234e38])
+def test_dense_fp32_pairs_of_values_that_are_not_finite(N, K, P, value):
+    for where in ("rows", "weight"):
+        test_dense_fp32_of_values_that_are_not_finite(N, K, P, value, where)
+
+
+@pytest.mark.parametrize("span", [20, -20])
+@pytest.mark.parametrize("N,K,P", PAIRS)
+def test_dense_fp32_pairs_scales(N, K, P, span):
+    """The pieces are scaled by row and by column: rows and columns of any size, values that grow or fall by 2^20 along the reduction and
+    meet weights that do the opposite, so that each product counts the same; rows that begin with zeros.  Bound: the file's."""
+    from sparseswin3d_amd import _lib
+    lib = _lib.load()
+    gen = torch.Generator().manual_seed(K + P)
+    two = lambda lo, hi, *s: torch.exp2(torch.randint(lo, hi + 1, s, generator=gen).float())
+    for transposed in (0, 1):
+        rows, cols = (P, K) if transposed else (K, P)             # of the reduction and the result
+        ramp = torch.exp2(torch.linspace(-span / 2, span / 2, rows).round())
+        x, wt = torch.randn(N, rows, generator=gen) * ramp * two(-40, 40, N, 1), torch.randn(cols, rows, generator=gen) / ramp * two(-40, 40, cols, 1)
+        x[N // 2, :rows - 8] = 0
+        x[N // 3] = 0
+        x, w = x.cuda(), (wt.T.contiguous() if transposed else wt).cuda()
+        y, _ = _forward(lib, _lib, x, w, None, transposed, PLAIN, None, torch.float32)
+        wd = wt.double().cuda()
+        _check(y, x.double() @ wd.T, x.double().abs() @ wd.abs().T, torch.float32, f"transposed {transposed}")
+
+
+# 2-norm of the error over that of the result, a twentieth above what was measured (three bf16 pieces: 2.0, 1.75, 2.5 and 6.0e-7)
+@pytest.mark.parametrize("N,K,P,transposed,error", [(35569, 192, 192, 0, 1.27e-7), (20000, 48, 144, 1, 1.17e-7), (19201, 96, 288, 1, 1.43e-7), (9000, 384, 1536, 1, 2.75e-7)])
+def test_dense_fp32_pairs_rounding(N, K, P, transposed, error):
+    from sparseswin3d_amd import _lib
+    lib = _lib.load()
+    gen = torch.Generator(device="cuda").manual_seed(N + K)
+    rows = P if transposed else K
+    x, w = torch.randn(N, rows, generator=gen, device="cuda"), torch.randn(P, K, generator=gen, device="cuda") * rows ** -0.5
+    y, _ = _forward(lib, _lib, x, w, None, transposed, PLAIN, None, torch.float32)
+    ref = x.double() @ (w.double() if transposed else w.double().T)
+    assert (y.double() - ref).norm() <= error * ref.norm()
+
+
+def test_dense_fp32_without_a_workspace():
+    from sparseswin3d_amd import _lib
+    lib = _lib.load()
+    gen = torch.Generator().manual_seed(5)
+    N, K, P = 20001, 208, 144
+    x, w, y = _rand(gen, N, K), _rand(gen, P, K, spread=1), torch.full((N, P), float("nan"), device="cuda")
+    assert lib.sswin_dense_forward_workspace_bytes(0, N, K, P) > 0
+    _lib.check(lib.sswin_dense_forward(0, 0, 0, PLAIN, _ptr(x), N, K, _ptr(w), None, P, None, _ptr(y), None, None, 0, _stream()))
+    _check(y, x.double() @ w.double().T, x.double().abs() @ w.double().abs().T, torch.float32, "plain")
+
+
 # each tile shape where its sums are shortest or longest for their number; relative error of dW against float64 (2-norms).  The
 # bounds are a twentieth above what tiles of 96 x 96 (64 x 64 up to 64 columns) with sums of at least 64 rows give there, averaged over
 # as many inputs.
