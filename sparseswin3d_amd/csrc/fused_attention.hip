@@ -38,7 +38,7 @@ constexpr int FUSED_GROUPS_PER_WG = 4;
 // ------------------------------------------------------------------------------------------
 // token plan
 //
-// Five phases, no sort:
+// Five phases, no sort (small scenes: all of them by one workgroup, tp_small_kernel):
 //   1. clear the presence bitmap (W = ceil(n/32) words per window slot) and the counters
 //   2. one atomicOr per voxel (indices outside [0,B) x [0,n) are counted and skipped)
 //   3. per block of 256 window slots: sums of (tokens, tokens^2, non-empty windows, windows per
@@ -314,61 +314,70 @@ __device__ __forceinline__ void tp_phase_tokens(const TokenPlanArgs& a, int64_t 
     }
 }
 
-// per voxel -> source voxel by token rank, and the token records
-__device__ __forceinline__ void tp_phase_rank(const TokenPlanArgs& a, int64_t gtid, int64_t gthreads) {
+// voxel v -> source voxel by token rank, and the token records.  Its rank and its window's first rank and size (all: the bitmap is there)
+struct TpRank {
+    int T, c, r;
+};
+__device__ __forceinline__ TpRank tp_rank_voxel(const TokenPlanArgs& a, int64_t v, const int2& wp) {
     const int W = a.W;
     const int64_t N = a.N;
-    int32_t* order = a.tokens;
-    // the totals are complete since the windows phase
-    if (gtid < 8 && a.host_totals) __hip_atomic_store(a.host_totals + gtid, a.totals[gtid], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-    for (int64_t v = gtid; v < N; v += gthreads) {
-        const int2 wp = *reinterpret_cast<const int2*>(a.ind + 2 * v);
-        if ((unsigned)wp.x >= (unsigned)a.B || (unsigned)wp.y >= (unsigned)a.n) continue;   // counted in phase 2
-        const int T = a.win_T[wp.x];
-        const int word = wp.y >> 5;
-        const uint32_t below_mask = (1u << (wp.y & 31)) - 1u;
-        int below = 0, c = 0;
-        if (W == 4) {
-            const uint4 q = *reinterpret_cast<const uint4*>(a.bits + (int64_t)wp.x * 4);
-            const uint32_t b[4] = {q.x, q.y, q.z, q.w};
+    const int T = a.win_T[wp.x];
+    const int word = wp.y >> 5;
+    const uint32_t below_mask = (1u << (wp.y & 31)) - 1u;
+    int below = 0, c = 0;
+    if (W == 4) {
+        const uint4 q = *reinterpret_cast<const uint4*>(a.bits + (int64_t)wp.x * 4);
+        const uint32_t b[4] = {q.x, q.y, q.z, q.w};
 #pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                const int pc = __popc(b[k]);
-                c += pc;
-                below += k < word ? pc : (k == word ? __popc(b[k] & below_mask) : 0);
-            }
-        } else {
-            for (int k = 0; k < W; ++k) {
-                const uint32_t x = a.bits[(int64_t)wp.x * W + k];
-                const int pc = __popc(x);
-                c += pc;
-                below += k < word ? pc : (k == word ? __popc(x & below_mask) : 0);
+        for (int k = 0; k < 4; ++k) {
+            const int pc = __popc(b[k]);
+            c += pc;
+            below += k < word ? pc : (k == word ? __popc(b[k] & below_mask) : 0);
+        }
+    } else {
+        for (int k = 0; k < W; ++k) {
+            const uint32_t x = a.bits[(int64_t)wp.x * W + k];
+            const int pc = __popc(x);
+            c += pc;
+            below += k < word ? pc : (k == word ? __popc(x & below_mask) : 0);
+        }
+    }
+    const int r = T + below;
+    if (r < N) {                                                // duplicates cannot push a rank past the end, but stay inside anyway
+        a.tokens[r] = (int32_t)v;
+    }
+    if (a.recs != nullptr) {
+        // Token records of the window-resident kernels: one record of 32 {voxel, pos} entries per (window, tile
+        // of 32 tokens), at the position of the tile's task inside its bucket, so that a task finds its tokens
+        // from its own number, in the same round trip as its group descriptor.  The entries behind the last
+        // token of a window repeat that token (what the kernels feed their padding rows with).
+        const int32_t wr = a.win_rec[wp.x];
+        if (wr >= 0) {
+            const int b = wr >> 28, nt = b + 1;
+            const int32_t* counters = tp_counters(a);
+            int64_t first = 0;                                   // records of the buckets of more tiles come first
+            for (int bb = 3; bb > b; --bb) first += (int64_t)(counters[bb] / a.H) * (bb + 1);
+            const int64_t rec = first + (int64_t)(wr & 0x0fffffff) * nt + (below >> 5);
+            if (rec < a.rec_cap && below < c) {
+                const int2 entry = make_int2((int)v, wp.y);
+                a.recs[rec * 32 + (below & 31)] = entry;
+                if (below == c - 1)
+                    for (int k = (below & 31) + 1; k < 32; ++k) a.recs[rec * 32 + k] = entry;
             }
         }
-        const int r = T + below;
-        if (r < N) {                                            // duplicates cannot push a rank past the end, but stay inside anyway
-            order[r] = (int32_t)v;
-        }
-        if (a.recs != nullptr) {
-            // Token records of the window-resident kernels: one record of 32 {voxel, pos} entries per (window, tile
-            // of 32 tokens), at the position of the tile's task inside its bucket, so that a task finds its tokens
-            // from its own number, in the same round trip as its group descriptor.  The entries behind the last
-            // token of a window repeat that token (what the kernels feed their padding rows with).
-            const int32_t wr = a.win_rec[wp.x];
-            if (wr >= 0) {
-                const int b = wr >> 28, nt = b + 1;
-                const int32_t* counters = tp_counters(a);
-                int64_t first = 0;                               // records of the buckets of more tiles come first
-                for (int bb = 3; bb > b; --bb) first += (int64_t)(counters[bb] / a.H) * (bb + 1);
-                const int64_t rec = first + (int64_t)(wr & 0x0fffffff) * nt + (below >> 5);
-                if (rec < a.rec_cap && below < c) {
-                    const int2 entry = make_int2((int)v, wp.y);
-                    a.recs[rec * 32 + (below & 31)] = entry;
-                    if (below == c - 1)
-                        for (int k = (below & 31) + 1; k < 32; ++k) a.recs[rec * 32 + k] = entry;
-                }
-            }
-        }
+    }
+    return {T, c, r};
+}
+__device__ __forceinline__ bool tp_in_range(const TokenPlanArgs& a, const int2& wp) { return (unsigned)wp.x < (unsigned)a.B && (unsigned)wp.y < (unsigned)a.n; }
+// the totals are complete since the windows phase
+__device__ __forceinline__ void tp_totals_to_host(const TokenPlanArgs& a, int64_t gtid) {
+    if (gtid < 8 && a.host_totals) __hip_atomic_store(a.host_totals + gtid, a.totals[gtid], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+__device__ __forceinline__ void tp_phase_rank(const TokenPlanArgs& a, int64_t gtid, int64_t gthreads) {
+    tp_totals_to_host(a, gtid);
+    for (int64_t v = gtid; v < a.N; v += gthreads) {
+        const int2 wp = *reinterpret_cast<const int2*>(a.ind + 2 * v);
+        if (tp_in_range(a, wp)) (void)tp_rank_voxel(a, v, wp);  // others were counted in phase 2
     }
 }
 
@@ -406,6 +415,137 @@ __global__ __launch_bounds__(256) void tp_rank_kernel(TokenPlanBatch b, int voxe
         tp_phase_rank(b.p[blockIdx.y], (int64_t)blockIdx.x * 256 + threadIdx.x, (int64_t)voxel_blocks * 256);
     else
         tp_phase_tokens(b.p[blockIdx.y], (int64_t)(blockIdx.x - voxel_blocks) * 256 + threadIdx.x, (int64_t)(gridDim.x - voxel_blocks) * 256);
+}
+
+// The whole plan of a small scene by one workgroup, its bitmap and what follows from it in LDS.  The five launches take 3 to 5 us each
+// whatever the size, and a stage's first block waits for the totals the last of them sends; here a voxel more is work of one compute unit.
+// Two plans from their enqueueing until their totals are there, five launches and one (us): 294 voxels 43 and 30; 1364 in 147 windows of 5^3, 12
+// heads 45 and 34; 2048 in 200 windows 46 and 40, in 800 windows (9600 rows of groups) 49 and 49; 3000 and 4096 in 800 windows 48 and 53, 49 and 60.
+constexpr int TP_SMALL_THREADS = 1024, TP_SMALL_ITEMS = 4, TP_SMALL_OWN = 2;   // window slots and voxels of a thread
+constexpr int64_t TP_SMALL_VOXELS = TP_SMALL_THREADS * TP_SMALL_OWN, TP_SMALL_WORDS = 8192, TP_SMALL_SLOTS = TP_SMALL_THREADS * TP_SMALL_ITEMS;
+constexpr int64_t TP_SMALL_GROUPS = 8192;
+
+// The windows phase with all running sums in 32 bits, and the H rows of a window written by neighbouring threads
+__device__ __forceinline__ void tp_small_windows(const TokenPlanArgs& a, int4* list, uint32_t (*sums)[TP_SMALL_THREADS / 64], int32_t* most) {
+    constexpr int S = 5, WAVES = TP_SMALL_THREADS / 64;                  // c; c * c; windows of 1 and 2 tiles; of 3 and 4; of more, non-empty ones
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, w0 = (int)threadIdx.x * TP_SMALL_ITEMS;
+    int c[TP_SMALL_ITEMS], cmax = 0;
+    uint32_t before[S] = {0, 0, 0, 0, 0}, own[S];
+    auto add = [](uint32_t (&to)[S], int c) {
+        const int b = tp_bucket(c);
+        to[0] += c, to[1] += c * c;
+        to[2] += b == 0 ? 1u : b == 1 ? 1u << 16 : 0u;
+        to[3] += b == 2 ? 1u : b == 3 ? 1u << 16 : 0u;
+        to[4] += (b == 4 ? 1u : 0u) | (c > 0 ? 1u << 16 : 0u);
+    };
+#pragma unroll
+    for (int u = 0; u < TP_SMALL_ITEMS; ++u) {
+        c[u] = w0 + u < a.B ? tp_window_count(a.bits, w0 + u, a.W) : 0;
+        cmax = max(cmax, c[u]);
+        add(before, c[u]);
+    }
+#pragma unroll
+    for (int k = 0; k < S; ++k) own[k] = before[k];
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1)
+#pragma unroll
+        for (int k = 0; k < S; ++k) {
+            const uint32_t t = __shfl_up(before[k], d, 64);
+            before[k] += lane >= d ? t : 0u;
+        }
+    const int wm = wave_max_i32(cmax);
+    if (lane == 63) {
+#pragma unroll
+        for (int k = 0; k < S; ++k) sums[k][wave] = before[k];
+        most[wave] = wm;
+    }
+    __syncthreads();
+    uint32_t all[S];
+    cmax = 0;
+#pragma unroll
+    for (int k = 0; k < S; ++k) before[k] -= own[k], all[k] = 0;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) {
+#pragma unroll
+        for (int k = 0; k < S; ++k) {
+            before[k] += w < wave ? sums[k][w] : 0u;
+            all[k] += sums[k][w];
+        }
+        cmax = max(cmax, most[w]);
+    }
+    if (threadIdx.x == 0) {
+        int32_t* const counters = tp_counters(a);
+        a.totals[0] = all[4] >> 16;
+        a.totals[1] = (int64_t)all[0] | (int64_t)all[1] << 32;
+#pragma unroll
+        for (int b = 0; b < 5; ++b) counters[b] = (int32_t)(all[2 + b / 2] >> (b & 1) * 16 & 0xffffu) * a.H;
+        counters[TPC_CMAX] = cmax;
+    }
+#pragma unroll
+    for (int u = 0; u < TP_SMALL_ITEMS; ++u) {
+        if (w0 + u < a.B) {
+            const int k = (int)(before[4] >> 16), b = tp_bucket(c[u]);
+            const uint32_t slot = b < 0 || b > 3 ? 0u : before[2 + b / 2] >> (b & 1) * 16 & 0xffffu;
+            a.win_T[w0 + u] = (int)before[0];
+            const bool live = c[u] > 0 && ((int64_t)k + 1) * a.H <= a.g_cap;
+            const bool task = a.tasks != nullptr && live && b < 4 && (int64_t)(slot + 1) * a.H <= a.g_cap;
+            a.win_rec[w0 + u] = task ? (int32_t)((uint32_t)b << 28 | slot) : -1;
+            if (live) list[k] = make_int4(w0 + u, c[u], (int)before[0], (int)before[1]);
+        }
+        add(before, c[u]);
+    }
+    __syncthreads();
+    const int rows = (int)min((int64_t)(all[4] >> 16) * a.H, a.g_cap / a.H * a.H);
+    for (int g = threadIdx.x; g < rows; g += TP_SMALL_THREADS) {
+        const int k = g / a.H, h = g - k * a.H;
+        const int4 e = list[k];
+        const int32_t sq = (int32_t)((uint32_t)e.w * a.H + (uint32_t)h * e.y * e.y);
+        a.plan[g] = e.y;
+        a.plan[a.g_cap + g] = e.z;
+        a.plan[2 * a.g_cap + g] = sq;
+        a.plan[3 * a.g_cap + g] = e.x;
+        a.plan[4 * a.g_cap + g] = h;
+        const int32_t rec = a.win_rec[e.x];
+        if (rec >= 0) a.tasks[(int64_t)(rec >> 28) * a.g_cap + (int64_t)(rec & 0x0fffffff) * a.H + h] = make_int4(e.z, e.y | h << 8, e.x, sq);
+    }
+}
+
+__global__ __launch_bounds__(TP_SMALL_THREADS) void tp_small_kernel(TokenPlanBatch b) {
+    __shared__ __attribute__((aligned(16))) uint32_t bits[TP_SMALL_WORDS];
+    __shared__ int32_t win_T[TP_SMALL_SLOTS], win_rec[TP_SMALL_SLOTS];
+    __shared__ int4 list[TP_SMALL_SLOTS];
+    __shared__ uint32_t sums[5][TP_SMALL_THREADS / 64];
+    __shared__ int32_t most[TP_SMALL_THREADS / 64];
+    __shared__ int64_t totals[8];
+    TokenPlanArgs a = b.p[blockIdx.y];
+    int64_t* const totals_out = a.totals;
+    a.bits = bits, a.win_T = win_T, a.win_rec = win_rec, a.totals = totals;
+    int2 wp[TP_SMALL_OWN];                                               // of this thread's voxels; the range check fails for those behind the last
+#pragma unroll
+    for (int u = 0; u < TP_SMALL_OWN; ++u) {
+        const int v = u * TP_SMALL_THREADS + (int)threadIdx.x;
+        wp[u] = v < a.N ? *reinterpret_cast<const int2*>(a.ind + 2 * v) : make_int2(-1, -1);
+    }
+    tp_phase_clear(a, threadIdx.x, TP_SMALL_THREADS);
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < TP_SMALL_OWN; ++u) {
+        if (tp_in_range(a, wp[u])) atomicOr(&bits[wp[u].x * a.W + (wp[u].y >> 5)], 1u << (wp[u].y & 31));
+        else if (u * TP_SMALL_THREADS + (int)threadIdx.x < a.N) atomicAdd(&tp_counters(a)[TPC_RANGE], 1);
+    }
+    __syncthreads();
+    tp_small_windows(a, list, sums, most);
+    tp_totals_to_host(a, threadIdx.x);
+#pragma unroll
+    for (int u = 0; u < TP_SMALL_OWN; ++u)
+        if (tp_in_range(a, wp[u])) {
+            const TpRank t = tp_rank_voxel(a, u * TP_SMALL_THREADS + (int)threadIdx.x, wp[u]);
+            if (!a.order_only && t.r < a.N) {
+                int32_t* const token = a.tokens + a.N + t.r;
+                token[0] = t.T, token[a.N] = t.c, token[2 * a.N] = wp[u].y, token[3 * a.N] = wp[u].x;
+            }
+        }
+    if (threadIdx.x < 8 && !a.host_totals) totals_out[threadIdx.x] = totals[threadIdx.x];
 }
 
 // ------------------------------------------------------------------------------------------
@@ -1573,7 +1713,14 @@ static int token_plan_args(const int32_t* indices, int64_t N, int B, int n, int 
     return 0;
 }
 
-// The five launches for `count` plans (1..TP_MAX_BATCH) and the copies of their raw totals to the host.
+// raw totals: the caller decodes them with sswin_token_plan_totals once the copies have landed
+static int token_plan_totals_to_host(const TokenPlanArgs* args, int64_t* const* totals_out, int count, hipStream_t s) {
+    for (int k = 0; k < count; ++k)
+        if (!args[k].host_totals) SSWIN_HIP(hipMemcpyAsync(totals_out[k], args[k].totals, 8 * sizeof(int64_t), hipMemcpyDeviceToHost, s));
+    return 0;
+}
+
+// The launches for `count` plans (1..TP_MAX_BATCH) and the copies of their raw totals to the host.
 static int token_plan_launch(const TokenPlanArgs* args, int64_t* const* totals_out, int count, hipStream_t s) {
     TokenPlanBatch b;
     size_t words = 0, token_words = 0;
@@ -1586,6 +1733,15 @@ static int token_plan_launch(const TokenPlanArgs* args, int64_t* const* totals_o
         if (!args[k].order_only) token_words = std::max(token_words, (size_t)args[k].B * args[k].W);
         voxels = std::max(voxels, args[k].N);
         blocks = std::max(blocks, args[k].blocks);
+    }
+    bool small = true;
+    for (int k = 0; k < count; ++k)
+        small = small && args[k].N <= TP_SMALL_VOXELS && (int64_t)args[k].B * args[k].W <= TP_SMALL_WORDS && args[k].B <= TP_SMALL_SLOTS &&
+                std::min<int64_t>(args[k].N, args[k].B) * args[k].H <= TP_SMALL_GROUPS;
+    if (small) {
+        hipLaunchKernelGGL(tp_small_kernel, dim3(1, (unsigned)count), dim3(TP_SMALL_THREADS), 0, s, b);
+        if (launch_ok("token plan")) return 1;
+        return token_plan_totals_to_host(args, totals_out, count, s);
     }
     // all plans of a launch share the slots per thread: four as soon as one of them has that many window slots
     int64_t slots = 0;
@@ -1611,10 +1767,7 @@ static int token_plan_launch(const TokenPlanArgs* args, int64_t* const* totals_o
     const unsigned word_blocks = (unsigned)std::max<size_t>(1, std::min<size_t>((token_words * 4 + 255) / 256, 8192));
     hipLaunchKernelGGL(tp_rank_kernel, dim3(nb + word_blocks, y), dim3(256), 0, s, b, (int)nb);
     if (launch_ok("token plan")) return 1;
-    // raw totals: the caller decodes them with sswin_token_plan_totals once the copies have landed
-    for (int k = 0; k < count; ++k)
-        if (!args[k].host_totals) SSWIN_HIP(hipMemcpyAsync(totals_out[k], args[k].totals, 8 * sizeof(int64_t), hipMemcpyDeviceToHost, s));
-    return 0;
+    return token_plan_totals_to_host(args, totals_out, count, s);
 }
 
 int sswin_token_plan(const int32_t* indices, int64_t N, int B, int n, int H, int32_t* tokens,

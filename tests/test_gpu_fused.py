@@ -55,6 +55,39 @@ def test_token_plan_closed_forms(case):
     np.testing.assert_array_equal(tp.plan.view(5, -1)[:, :tp.G].cpu().numpy(), plan)
 
 
+# the plans one workgroup makes, and the first ones it does not: voxels, words of the bitmap, window slots, rows of groups; one and
+# several words a window, five of them with tokens in more than one thread's slots
+@pytest.mark.parametrize("B,n,H,N", [(66, 125, 3, 2048), (66, 125, 3, 2049), (4096, 8, 1, 2048), (4097, 8, 1, 2048), (744, 343, 3, 1500), (745, 343, 3, 1500),
+                                     (682, 125, 12, 1900), (683, 125, 12, 1900), (5, 343, 2, 1600), (3, 33, 255, 40), (1, 1, 1, 1)])
+def test_token_plan_of_small_scenes(B, n, H, N):
+    from sparseswin3d_amd.fused import TokenPlan
+    ind = random_window_indices(np.random.default_rng(B + N), B, n, N)
+    tokens, plan, A, c_max = _closed_form_plan(ind, n, H)
+    G = plan.shape[1]
+    dev = torch.from_numpy(ind).cuda()
+    full, lean = TokenPlan.batch([(dev, B, n, H), (dev, B, n, H, False, True)])
+    for tp in (full, lean):
+        tp.finish()
+        assert (tp.G, tp.A, tp.c_max) == (G, A, c_max)
+        np.testing.assert_array_equal(tp.plan.view(5, -1)[:, :G].cpu().numpy(), plan)
+    np.testing.assert_array_equal(full.tokens.view(5, -1).cpu().numpy(), tokens)
+    np.testing.assert_array_equal(lean.tokens.cpu().numpy(), tokens[0])
+    # descriptors of each bucket in window order, head by head; records: the bucket of four tiles first
+    desc = full.tasks[:16 * full.g_cap].view(4, full.g_cap, 4).cpu().numpy()
+    tiles = np.where(plan[0] <= 128, (plan[0] + 31) // 32, 0)
+    first = 0
+    for k in (4, 3, 2, 1):
+        rows = plan[:, tiles == k]
+        assert int(full.bucket_counts[k - 1]) == rows.shape[1]
+        np.testing.assert_array_equal(desc[k - 1, :rows.shape[1]], np.stack([rows[1], rows[0] | rows[4] << 8, rows[3], rows[2]], 1))
+        for c, T in rows[:2, ::H].T:
+            for tile in range(k):
+                ranks = T + np.minimum(32 * tile + np.arange(32), c - 1)
+                rec = full.tasks[16 * full.g_cap + 64 * first:16 * full.g_cap + 64 * (first + 1)].view(32, 2).cpu().numpy()
+                np.testing.assert_array_equal(rec, np.stack([tokens[0, ranks], tokens[3, ranks]], 1))
+                first += 1
+
+
 def test_token_plans_in_one_batch_equal_single_plans():
     """Several plans built by shared launches (different voxel counts, window counts, window sizes, head counts,
     one of them empty, one without task descriptors) hold the same bits as plans built one by one; a bad index in
