@@ -1083,6 +1083,10 @@ static int launch_forward(const void* x, int64_t N, int K, const void* w, int P,
         const int64_t rows = (N + 127) / 128, tiles = rows * ((P + 95) / 96) * cut.ksplit;
         // long reductions into many columns: fewest bytes through LDS (8119 rows, 768 -> 3072: 57 us against 70 with the next two)
         if (K >= 384 && P % 192 == 0 && rows * (P / 192) >= 512) return launch_rows16<T, TO, EPI, DOWN, 64, 2, 2, 1, 2, 2, 2>(xp, N, K, wp, P, 1, ws, ep, s);
+        // one workgroup a compute unit and a long reduction: three blocks on their way instead of one, since nothing else hides a block's
+        // way from L2 (inside a backbone, weights not in L2: 7888 rows 1536 -> 384 28.2 us, now 20.8, five blocks of LDS 22.0; 1364 rows 768 -> 768 17.1 and
+        // 14.5; 7888 rows 384 -> 384 13.5 either way, again and again on one input 9.3 and 9.6)
+        if (tiles <= device_cus() && K >= 768) return launch_rows16<T, TO, EPI, DOWN, 64, 4, 1, 2, 1, 4, 2>(xp, N, K, wp, P, cut.ksplit, ws, ep, s);
         // up to two workgroups a compute unit: eight wavefronts each (8119 rows, 1536 -> 384: 22 us against 30), above that five
         // workgroups of four, whose loads and stores overlap (219 000 rows, 96 -> 288: 44 us against 80)
         if (tiles <= 512) return launch_rows16<T, TO, EPI, DOWN, 64, 4, 1, 2, 1, 2, 4>(xp, N, K, wp, P, cut.ksplit, ws, ep, s);

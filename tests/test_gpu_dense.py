@@ -120,6 +120,14 @@ def test_dense_forward_around_the_lines_of_few_rows(K, P, epi, rows):
         _check(y, pre, mag, dtype, f"{N} rows")
 
 
+# 16 bit, at most a workgroup a compute unit and a reduction of 768 and more: whole blocks of 64, a ragged last one, rows past a tile
+@pytest.mark.parametrize("N,K,P", [(2048, 768, 768), (2113, 784, 768), (768, 1552, 1536), (7889, 1536, 384)])
+@pytest.mark.parametrize("dtype,out", [(torch.bfloat16, torch.bfloat16), (torch.float16, torch.float16), (torch.float16, torch.float32)])
+def test_dense_forward_of_long_reductions(N, K, P, dtype, out):
+    test_dense_forward_and_input_gradient(N, K, P, dtype, out)
+    test_dense_forward_and_input_gradient(N, P, K, dtype, out)
+
+
 # a result in the place of its rows, where one workgroup of a tile holds them whole (96 columns at most, more rows than the few-rows kernel takes)
 @pytest.mark.parametrize("K", [48, 96])
 def test_dense_forward_in_place(K):
