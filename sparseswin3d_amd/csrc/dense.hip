@@ -1071,8 +1071,12 @@ static int launch_forward(const void* x, int64_t N, int K, const void* w, int P,
         return launch_ok("dense, few rows");
     }
     if constexpr (Op<T>::PL == 3) {
-        // 96 channels: the kernel that keeps Wop in LDS (219 000 rows, 96 -> 288: 89 us against 120 here, with a residual 133 and 202)
-        if (K == 96 && P % 96 == 0) return staged_layer_96(xp, N, wp, P, DOWN, EPI, ep, s);
+        // 96 channels: the kernels that keep Wop in LDS
+        if (K == 96 && P % 96 == 0) {
+            int rc = 0;
+            if (pairs_held<EPI, DOWN>(xp, N, wp, P, ep, s, rc)) return rc;
+            return staged_layer_96(xp, N, wp, P, DOWN, ep, s);
+        }
         // fp16 pairs, from the reductions on whose sums come out as exactly: error against float64 (2-norms) with 96 channels 7.8e-8 and
         // 1.0e-7 here, 144 1.1e-7 and 1.75e-7 (turned); 48 channels of three bf16 pieces 6.9e-8, of pairs 7.1e-8 and more
         if (pairs_takes(K) && ws_bytes >= pairs_workspace_bytes(K, P)) return pairs_layer<EPI, DOWN>(xp, N, K, wp, P, ep, ws, s);

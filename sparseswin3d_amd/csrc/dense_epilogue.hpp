@@ -141,14 +141,17 @@ __device__ __forceinline__ void finish8(const Epilogue& ep, int64_t row, int col
     *reinterpret_cast<Vec8<TO>*>(static_cast<TO*>(ep.y) + at) = y;
 }
 
-// fp32 layers of 96 reduction channels and a multiple of 96 outputs (tall_linear.hip): x [N >= 32, 96], all of Wop in LDS
-int staged_layer_96(const float* x, int64_t N, const float* w, int P, bool transposed, int epilogue, const Epilogue& ep, hipStream_t s);
+// fp32 layers of 96 reduction channels and a multiple of 96 outputs with a second operand (tall_linear.hip): x [N >= 32, 96], all of Wop in LDS;
+// a residual, or turned a factor
+int staged_layer_96(const float* x, int64_t N, const float* w, int P, bool transposed, const Epilogue& ep, hipStream_t s);
 // whether a layer of N rows, K -> P, takes the kernel for few rows, whose wavefronts share the reduction (dense.hip)
 bool few_rows(int dtype, int64_t N, int K, int P);
 // fp32 layers as fp16 pairs (dense_pairs.hip), W's pieces in ws
 inline bool pairs_takes(int K) { return K >= 96; }
 size_t pairs_workspace_bytes(int K, int P);
 template <int EPI, bool DOWN> int pairs_layer(const float* x, int64_t N, int K, const float* w, int P, const Epilogue& ep, void* ws, hipStream_t s);
+// the same for 96 reduction channels and a multiple of 96 outputs, without a workspace; false where staged_layer_96 is ahead (rc untouched)
+template <int EPI, bool DOWN> bool pairs_held(const float* x, int64_t N, const float* w, int P, const Epilogue& ep, hipStream_t s, int& rc);
 // 16-bit layers of 48, 96 or 192 reduction channels without a last step: x read once (mlp.hip)
 bool rows_once_takes(int64_t N, int D, int P);
 template <typename T> int rows_once(const T* x, int64_t N, int D, const T* w, const T* b, int P, T* y, hipStream_t s);

@@ -18,6 +18,8 @@
 // splitting one step ahead between the products at two wavefronts a SIMD (45 -> 57, 126 -> 146), rows kept in registers for all columns (45 -> 49 to 55).
 #include <stdint.h>
 
+#include <algorithm>
+
 #include "dense_epilogue.hpp"
 #include "dense_operand.hpp"
 #include "mfma_block.hpp"
@@ -221,6 +223,158 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
         }
 }
 
+// ------------------------------------------------------------------------------------------
+// 96 reduction channels: a workgroup of 8 wavefronts a compute unit splits its 32 CT columns of W itself, keeps their pieces in LDS and walks over the
+// rows, 32 a wavefront, the next 32 in flight.  A row's 96 values fit a lane as pieces (48 registers), so that its scale is that of its
+// largest value and it is split once for all of the columns.  Bound by the traffic, and by what a launch takes until its pieces are there (5 us).
+// The loops over the columns are unrolled: with a count the compiler does not know it waits for all stores where the next rows are used (CT = 9 in a
+// loop 42 us where three workgroups of 96 columns take 39; unrolled, 36 registers are spilled and 50).
+// Three bf16 pieces before, microseconds: 112 700 rows 96 -> 288 44.2 and 39.0, 96 -> 96 21.1 and 18.8 (turned 21.1 and 18.6), 20 000 rows 96 -> 288 12.6 and 12.4,
+// 96 -> 96 10.2 and 7.6; 225 700 rows 96 -> 288 87.3 and 86.6.  Error against float64 (2-norms) 1.13e-7 and 0.81e-7, turned 1.50e-7 and 1.04e-7.
+// ------------------------------------------------------------------------------------------
+constexpr int HELD_K = 96, HELD_KS = HELD_K / 16, HELD_WAVES = 8;
+template <int EPI, bool DOWN, int CT>
+__global__ __launch_bounds__(HELD_WAVES * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) void pairs_held_kernel(
+    const float* __restrict__ x, int64_t N, const float* __restrict__ w, int P, int groups, int64_t row_tiles, Epilogue ep) {
+    constexpr int K = HELD_K, KS = HELD_KS;
+    extern __shared__ __attribute__((aligned(16))) u32x4 lds[];          // pieces [column tile][16 channels][piece][lane], a tile a wavefront
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, half = lane >> 5, l32 = lane & 31;
+    int cg;
+    int64_t slot;
+    block_of(groups, cg, slot);
+    const int col0 = cg * CT * 32;
+    u32x4* const tile = lds + CT * KS * 128 + wave * 256;                // [32 rows][8 pieces], the pieces of a row exchanged by its number
+    int* const exps = reinterpret_cast<int*>(lds + CT * KS * 128 + HELD_WAVES * 256);
+    float* const bias = reinterpret_cast<float*>(exps + CT * 32);
+    const int64_t first = slot * HELD_WAVES + wave, stride = (int64_t)(gridDim.x / groups) * HELD_WAVES;
+
+    const int mem_row = lane >> 3, mem_piece = (lane & 7) ^ mem_row;     // of 8 rows x 32 columns, that this lane moves
+    f32x4 next[3][4];
+    auto fetch = [&](int64_t t) {                                        // rows past the end repeat the last one
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int64_t row = t * 32 + i * 8 + mem_row;
+            const float* const from = x + (row < N ? row : N - 1) * K + mem_piece * 4;
+#pragma unroll
+            for (int c = 0; c < 3; ++c) next[c][i] = *reinterpret_cast<const f32x4*>(from + c * 32);
+        }
+    };
+    if (first < row_tiles) fetch(first);
+    if (const int c = wave; c < CT) {
+        const int col = col0 + c * 32 + l32;
+        float v[KS][8], m = 0.f;
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+            const int k = ks * 16 + half * 8;
+            if constexpr (DOWN) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) v[ks][e] = w[(int64_t)(k + e) * P + col];
+            } else {
+                const f32x4* const src = reinterpret_cast<const f32x4*>(w + (int64_t)col * K + k);
+                const f32x4 a = src[0], b = src[1];
+#pragma unroll
+                for (int e = 0; e < 8; ++e) v[ks][e] = e < 4 ? a[e] : b[e - 4];
+            }
+        }
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) m = fmaxf(m, largest(v[ks]));
+        const int e = min(15 - exponent_above(largest_of_halves(m)), PAIRS_MOST_SCALE);
+        const float scale = power_of_two(e);
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+            u32x4 p[2];
+            split_pairs(v[ks], scale, p);
+            lds[((c * KS + ks) * 2 + 0) * 64 + lane] = p[0];
+            lds[((c * KS + ks) * 2 + 1) * 64 + lane] = p[1];
+        }
+        if (half == 0) {
+            exps[c * 32 + l32] = e;
+            bias[c * 32 + l32] = ep.bias ? static_cast<const float*>(ep.bias)[col] : 0.f;
+        }
+    }
+    block_barrier();
+    const Epilogue after = {nullptr, ep.extra, ep.y, ep.slope};          // the bias is added before
+    for (int64_t t = first; t < row_tiles; t += stride) {
+        float v[KS][8], m = 0.f;
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int i = 0; i < 4; ++i) tile[(i * 8 + mem_row) * 8 + (lane & 7)] = __builtin_bit_cast(u32x4, next[c][i]);
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int q = 0; q < 2; ++q) {
+                    const f32x4 p = __builtin_bit_cast(f32x4, tile[l32 * 8 + ((h * 4 + half * 2 + q) ^ (l32 & 7))]);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) v[c * 2 + h][q * 4 + e] = p[e];
+                }
+        }
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) m = fmaxf(m, largest(v[ks]));
+        const int e = min(15 - exponent_above(largest_of_halves(m)), PAIRS_MOST_SCALE);
+        const float scale = power_of_two(e);
+        u32x4 b[KS][2];
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) split_pairs(v[ks], scale, b[ks]);
+        if (t + stride < row_tiles) fetch(t + stride);
+        const int64_t r0 = t * 32 + mem_row;
+#pragma unroll
+        for (int c = 0; c < CT; ++c) {
+            const int col = col0 + c * 32 + mem_piece * 4;
+            Second4<float, float, EPI> second[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                if (r0 + q * 8 < N) second[q].load(ep, r0 + q * 8, col, P);
+            const u32x4* const pieces = lds + c * KS * 128 + lane;
+            f32x16 acc = f32x16{0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0}, low = acc;
+            u32x4 a[2][2];
+#pragma unroll
+            for (int q = 0; q < 2; ++q) a[0][q] = pieces[q * 64];
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) {
+                if (ks + 1 < KS)
+#pragma unroll
+                    for (int q = 0; q < 2; ++q) a[(ks + 1) & 1][q] = pieces[((ks + 1) * 2 + q) * 64];
+                low = Pairs::mfma(a[ks & 1][1], b[ks][0], low);
+                acc = Pairs::mfma(a[ks & 1][0], b[ks][0], acc);
+                low = Pairs::mfma(a[ks & 1][0], b[ks][1], low);
+            }
+            f32x4 any = {0.f, 0.f, 0.f, 0.f};
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int at = c * 32 + q * 8 + half * 4;
+                const int4 ew = *reinterpret_cast<const int4*>(exps + at);
+                const f32x4 add = *reinterpret_cast<const f32x4*>(bias + at);
+                const int ec[4] = {ew.x, ew.y, ew.z, ew.w};
+                f32x4 s;
+#pragma unroll
+                for (int u = 0; u < 4; ++u) s[u] = __builtin_amdgcn_ldexpf(fmaf(low[q * 4 + u], Pairs::LOW, acc[q * 4 + u]), -(e + ec[u])) + add[u];
+                any += s;
+                tile[l32 * 8 + ((q * 2 + half) ^ (l32 & 7))] = __builtin_bit_cast(u32x4, s);
+            }
+            __builtin_amdgcn_wave_barrier();
+            if (__any(nan_among(any))) {
+#pragma unroll 1
+                for (int q = 0; q < 4; ++q) {
+                    f32x4 s = __builtin_bit_cast(f32x4, tile[q * 64 + lane]);
+                    if (r0 + q * 8 < N && nan_among(s))
+                        s = plain_products(x + (r0 + q * 8) * K, 1, w + (DOWN ? col : (int64_t)col * K), DOWN ? P : 1, DOWN ? 1 : K, K) +
+                            *reinterpret_cast<const f32x4*>(bias + (col - col0));
+                    tile[q * 64 + lane] = __builtin_bit_cast(u32x4, s);
+                }
+                __builtin_amdgcn_wave_barrier();
+            }
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                if (r0 + q * 8 < N)
+                    finish4<float, float, EPI>(after, r0 + q * 8, col, P, __builtin_bit_cast(f32x4, tile[q * 64 + lane]), second[q]);
+        }
+    }
+}
+
 static int pairs_tiles(int P) { return (P + 95) / 96 * 3; }
 size_t pairs_workspace_bytes(int K, int P) { return (size_t)pairs_tiles(P) * (pairs_ksteps(K) * 2048 + 128); }
 
@@ -236,11 +390,38 @@ template <int EPI, bool DOWN> int pairs_layer(const float* x, int64_t N, int K, 
     hipLaunchKernelGGL((pairs_rows_kernel<EPI, DOWN>), dim3((unsigned)blocks), dim3(256), 0, s, x, N, K, planes, exps, w, P, groups, ep);
     return launch_ok("dense, pairs");
 }
+template <int EPI, bool DOWN, int CT> static int launch_held(const float* x, int64_t N, const float* w, int P, const Epilogue& ep, hipStream_t s) {
+    auto* k = pairs_held_kernel<EPI, DOWN, CT>;
+    constexpr int LDS = CT * (HELD_KS * 2048 + 256) + HELD_WAVES * 4096;
+    static const hipError_t configured = hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
+    SSWIN_HIP(configured);
+    const int groups = P / 32 / CT;
+    const int64_t row_tiles = (N + 31) / 32, slots = std::min<int64_t>((row_tiles + HELD_WAVES - 1) / HELD_WAVES, std::max(1, device_cus() / groups));
+    hipLaunchKernelGGL(k, dim3((unsigned)(slots * groups)), dim3(HELD_WAVES * 64), LDS, s, x, N, w, P, groups, row_tiles, ep);
+    return launch_ok("dense, pairs of 96 channels");
+}
+// False where tall_linear.hip is ahead: its kernel requests a second operand when the products are done, here it stands behind the next
+// rows, and in front of them there are no registers for it (112 700 rows 96 -> 96 with a residual: 21.2 us there, 23.3 here, in front 32).
+template <int EPI, bool DOWN> bool pairs_held(const float* x, int64_t N, const float* w, int P, const Epilogue& ep, hipStream_t s, int& rc) {
+    const int64_t workgroups = (N + HELD_WAVES * 32 - 1) / (HELD_WAVES * 32) * (P / 96);   // of 96 columns
+    // few of them: 32 columns (7000 rows 96 -> 288, 84 workgroups: 10.1 us with 96 columns, 8.0 with 32; 36 000 96 -> 96, 141: 12.4 and 11.1; 28 000 96 -> 192,
+    // 220: 11.2 and 12.9).  Not in place, where other workgroups read the rows.
+    const bool few = workgroups * 8 <= device_cus() * 5 && ep.y != x;
+    if (Second4<float, float, EPI>::USED && !few) return false;
+    if constexpr (Second4<float, float, EPI>::USED) rc = launch_held<EPI, DOWN, 1>(x, N, w, P, ep, s);
+    else rc = few ? launch_held<EPI, DOWN, 1>(x, N, w, P, ep, s) : launch_held<EPI, DOWN, 3>(x, N, w, P, ep, s);
+    return true;
+}
 template int pairs_layer<EPI_NONE, false>(const float*, int64_t, int, const float*, int, const Epilogue&, void*, hipStream_t);
 template int pairs_layer<EPI_GELU, false>(const float*, int64_t, int, const float*, int, const Epilogue&, void*, hipStream_t);
 template int pairs_layer<EPI_RESIDUAL, false>(const float*, int64_t, int, const float*, int, const Epilogue&, void*, hipStream_t);
 template int pairs_layer<EPI_NONE, true>(const float*, int64_t, int, const float*, int, const Epilogue&, void*, hipStream_t);
 template int pairs_layer<EPI_SCALE, true>(const float*, int64_t, int, const float*, int, const Epilogue&, void*, hipStream_t);
+template bool pairs_held<EPI_NONE, false>(const float*, int64_t, const float*, int, const Epilogue&, hipStream_t, int&);
+template bool pairs_held<EPI_GELU, false>(const float*, int64_t, const float*, int, const Epilogue&, hipStream_t, int&);
+template bool pairs_held<EPI_RESIDUAL, false>(const float*, int64_t, const float*, int, const Epilogue&, hipStream_t, int&);
+template bool pairs_held<EPI_NONE, true>(const float*, int64_t, const float*, int, const Epilogue&, hipStream_t, int&);
+template bool pairs_held<EPI_SCALE, true>(const float*, int64_t, const float*, int, const Epilogue&, hipStream_t, int&);
 
 }  // namespace dense
 }  // namespace sswin

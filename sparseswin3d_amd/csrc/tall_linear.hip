@@ -19,7 +19,7 @@
 // (it splits them itself when it starts); its waves walk over 32-row tiles.  Per 16-wide k step a
 // lane holds 8 fp32 of X (row l % 32, k group l / 32), splits them, and feeds 3 column tiles x 6
 // products.  Kernels, by shape:
-//   tall_linear_forward_staged_kernel   K <= 96 (also dX of a 96-column dY, W read transposed)
+//   tall_linear_forward_staged_kernel   K <= 96 (96 with a residual; dX of a 96-column dY times a factor, W read transposed)
 //   tall_linear_forward_kernel          96 < K <= 192
 //   tall_linear_wide_kernel             dX for 192..288 columns of dY: all of W on the CU
 //   tall_linear_chunked_kernel          dX for more columns of dY: W in chunks of 96 rows
@@ -204,11 +204,11 @@ constexpr int TL_STAGED_MAX_KS = 6;
 // SMALL: fewer than 32 rows in all (one ragged tile, guarded).  Otherwise a last ragged tile is moved
 // back to end at row N: it recomputes a few rows of its neighbour (same inputs, same arithmetic, the
 // same bits stored twice) and every tile takes the unguarded path.
-// EPI: what follows the product (dense_epilogue.hpp), applied where the accumulators are stored
+// EPI: a residual or factor that follows the product (dense_epilogue.hpp), applied where the accumulators are stored
 template <int KS, bool SMALL, bool TRANSPOSED = false, int EPI = dense::EPI_NONE>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void tall_linear_forward_staged_kernel(
     const float* __restrict__ x, int64_t N, const float* __restrict__ w, int groups, const float* __restrict__ bias,
-    float* __restrict__ y, int P, int64_t row_tiles, const float* __restrict__ extra = nullptr, float* __restrict__ slope = nullptr) {
+    float* __restrict__ y, int P, int64_t row_tiles, const float* __restrict__ extra = nullptr) {
     constexpr int K = KS * 16, PITCH = K + 4, C4 = K / 4, NI = 2 * KS;   // 16-byte chunks per row; loads per lane and tile
     extern __shared__ __attribute__((aligned(16))) tl_u32x4 w_s[];      // [k step][tile][plane][lane], then the X tiles
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;   // wave: a scalar
@@ -318,21 +318,16 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
             for (int q = 0; q < 12; ++q) {                               // piece q * 64 + lane of 32 rows x 24 pieces
                 at[q] = (uint32_t)(((q * 64 + lane) / 24) * P + ((q * 64 + lane) % 24) * 4);
-                if constexpr (EPI == dense::EPI_RESIDUAL || EPI == dense::EPI_SCALE)
-                    second[q] = *reinterpret_cast<const tl_f32x4*>(extra + tile_at + at[q]);
+                second[q] = *reinterpret_cast<const tl_f32x4*>(extra + tile_at + at[q]);
             }
 #pragma unroll
             for (int q = 0; q < 12; ++q) {
                 const tl_f32x4 v = *reinterpret_cast<const tl_f32x4*>(xs + ((q * 64 + lane) / 24) * PITCH + ((q * 64 + lane) % 24) * 4);
-                tl_f32x4 o, d;
+                tl_f32x4 o;
+                float slope;
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    float s = 0.f;
-                    o[e] = dense::finish1<EPI>(v[e], EPI == dense::EPI_GELU ? 0.f : second[q][e], s);
-                    d[e] = s;
-                }
+                for (int e = 0; e < 4; ++e) o[e] = dense::finish1<EPI>(v[e], second[q][e], slope);
                 *reinterpret_cast<tl_f32x4*>(y + tile_at + at[q]) = o;
-                if (EPI == dense::EPI_GELU && slope) *reinterpret_cast<tl_f32x4*>(slope + tile_at + at[q]) = d;
             }
         }
     }
@@ -825,16 +820,11 @@ static int launch_staged_96(const float* x, int64_t N, const float* w, int P, co
     const int64_t row_tiles = (N + 31) / 32;
     const int64_t per_group = std::min<int64_t>((row_tiles + 7) / 8, std::max<int64_t>(1, device_cus() / groups));
     hipLaunchKernelGGL(k, dim3((unsigned)(per_group * groups)), dim3(512), staged_lds_bytes(6), s, x, N, w, groups,
-                       static_cast<const float*>(ep.bias), static_cast<float*>(ep.y), P, row_tiles, static_cast<const float*>(ep.extra),
-                       static_cast<float*>(ep.slope));
+                       static_cast<const float*>(ep.bias), static_cast<float*>(ep.y), P, row_tiles, static_cast<const float*>(ep.extra));
     return launch_ok("staged layer");
 }
-int staged_layer_96(const float* x, int64_t N, const float* w, int P, bool transposed, int epilogue, const Epilogue& ep, hipStream_t s) {
-    if (transposed)
-        return epilogue == EPI_SCALE ? launch_staged_96<true, EPI_SCALE>(x, N, w, P, ep, s) : launch_staged_96<true, EPI_NONE>(x, N, w, P, ep, s);
-    if (epilogue == EPI_GELU) return launch_staged_96<false, EPI_GELU>(x, N, w, P, ep, s);
-    if (epilogue == EPI_RESIDUAL) return launch_staged_96<false, EPI_RESIDUAL>(x, N, w, P, ep, s);
-    return launch_staged_96<false, EPI_NONE>(x, N, w, P, ep, s);
+int staged_layer_96(const float* x, int64_t N, const float* w, int P, bool transposed, const Epilogue& ep, hipStream_t s) {
+    return transposed ? launch_staged_96<true, EPI_SCALE>(x, N, w, P, ep, s) : launch_staged_96<false, EPI_RESIDUAL>(x, N, w, P, ep, s);
 }
 }  // namespace dense
 }  // namespace sswin
@@ -890,9 +880,10 @@ int sswin_tall_linear_input_grad(const float* dy, int64_t N, int P, const float*
     hipStream_t s = static_cast<hipStream_t>(stream);
     const int cus = device_cus();
     if (P == 96 && N >= 32) {
-        // 96 channels of dY: the staged kernel of the forward with W read transposed
         SSWIN_CHECK(((uintptr_t)w % 16) == 0, "tall_linear_input_grad: w must be 16-byte aligned");
-        return dense::staged_layer_96(dy, N, w, K, true, dense::EPI_NONE, dense::Epilogue{nullptr, nullptr, dx, nullptr}, s);
+        int rc = 0;
+        dense::pairs_held<dense::EPI_NONE, true>(dy, N, w, K, dense::Epilogue{nullptr, nullptr, dx, nullptr}, s, rc);
+        return rc;
     }
     return launch_chunked<true>(dy, N, P, w, nullptr, K, dx, cus, s, "tall_linear_input_grad");
 }

@@ -492,6 +492,8 @@ def test_dense_fp32_weight_gradient_of_values_that_are_not_finite(N, P, K, value
 # fp32 layers of at least 96 reduction channels (pairs of fp16): whole steps of 32 and a last one of 16, columns that end inside a tile, several
 # column blocks; one row past a workgroup's
 PAIRS = [(19201, 96, 112), (20001, 144, 48), (20001, 208, 304), (9601, 576, 192)]
+# 96 channels (turned: 96 columns) and a multiple of 96 outputs: 32 or 96 columns a workgroup, one and several tiles of rows a wavefront
+PAIRS += [(6401, 96, 288), (13825, 96, 288), (19233, 96, 96), (90001, 96, 96), (30001, 288, 96)]
 
 
 @pytest.mark.parametrize("N,K,P", PAIRS)
@@ -520,6 +522,12 @@ def test_dense_fp32_pairs_scales(N, K, P, span):
         y, _ = _forward(lib, _lib, x, w, None, transposed, PLAIN, None, torch.float32)
         wd = wt.double().cuda()
         _check(y, x.double() @ wd.T, x.double().abs() @ wd.abs().T, torch.float32, f"transposed {transposed}")
+
+
+# the last steps of 96 channels, on either side of the rows from which a workgroup takes 96 columns
+@pytest.mark.parametrize("N,K,P", [(6400, 96, 288), (13633, 96, 288), (21761, 288, 96), (41217, 96, 96)])
+def test_dense_fp32_pairs_of_96_channels(N, K, P):
+    test_dense_forward_and_input_gradient(N, K, P, torch.float32, torch.float32)
 
 
 # 2-norm of the error over that of the result, a twentieth above what was measured (three bf16 pieces: 2.0, 1.75, 2.5 and 6.0e-7)
