@@ -500,7 +500,9 @@ int sswin_dense_backward_small(int dtype, int out_dtype, int epilogue, const voi
  *   ids or null.
  * forward: lse fp32 [H, N] for the backward.
  * backward: dqkv; ds (or null) = gradient of the scores in the groups' [c x c] blocks, for sswin_bias_table_grad; delta fp32 [H, N]
- *   scratch. */
+ *   scratch.
+ * The same with `order` (int32 [sswin_flash_order_ints], 0: not worth one; or null): which 32 tokens are worked on first.  sswin_flash_tokens_ordered
+ *   writes it, forward and backward read it; results do not depend on it. */
 int sswin_flash_supported(int dtype, int64_t N, int H, int hd, int rows);
 int sswin_flash_tokens(const int32_t* plan, int64_t g_cap, int64_t groups, const int32_t* tokens, int64_t N, int H, int n,
                        const int32_t* code, const int8_t* mask, int nmw, int32_t* word, int32_t* tok_sq, void* stream);
@@ -509,6 +511,14 @@ int sswin_flash_forward(int dtype, const int32_t* tokens, const int32_t* word, i
 int sswin_flash_backward(int dtype, const int32_t* tokens, const int32_t* word, const int32_t* tok_sq, int64_t N, int H, int hd, int n,
                          const void* qkv, float scale, const float* table, int rows, int offset0, const void* out, const float* lse,
                          const void* dout, void* dqkv, float* delta, float* ds, void* stream);
+size_t sswin_flash_order_ints(int64_t N, int H);
+int sswin_flash_tokens_ordered(const int32_t* plan, int64_t g_cap, int64_t groups, const int32_t* tokens, int64_t N, int H, int n, const int32_t* code,
+                               const int8_t* mask, int nmw, int32_t* word, int32_t* tok_sq, int32_t* order, void* stream);
+int sswin_flash_forward_ordered(int dtype, const int32_t* tokens, const int32_t* word, const int32_t* order, int64_t N, int H, int hd, int n,
+                                const void* qkv, float scale, const float* table, int rows, int offset0, void* out, float* lse, void* stream);
+int sswin_flash_backward_ordered(int dtype, const int32_t* tokens, const int32_t* word, const int32_t* tok_sq, const int32_t* order, int64_t N, int H,
+                                 int hd, int n, const void* qkv, float scale, const float* table, int rows, int offset0, const void* out,
+                                 const float* lse, const void* dout, void* dqkv, float* delta, float* ds, void* stream);
 
 /* nn.LayerNorm over rows of D values (swin3d_base.py:706, 722).  x of x_dtype; y of y_dtype (x_dtype, or a 16-bit type for
  * fp32 x); gamma, beta fp32 for fp32 x, else of x_dtype.  stats: fp32 [2][N] mean and reciprocal deviation for the backward, or

@@ -102,6 +102,10 @@ SIGNATURES = {
     "sswin_flash_forward": (_i32, [_i32, _vp, _vp, _i64, _i32, _i32, _i32, _vp, C.c_float, _vp, _i32, _i32, _vp, _vp, _vp]),
     "sswin_flash_backward": (_i32, [_i32, _vp, _vp, _vp, _i64, _i32, _i32, _i32, _vp, C.c_float, _vp, _i32, _i32, _vp, _vp, _vp, _vp, _vp,
                                     _vp, _vp]),
+    "sswin_flash_order_ints": (_sz, [_i64, _i32]),
+    "sswin_flash_tokens_ordered": (_i32, [_vp, _i64, _i64, _vp, _i64, _i32, _i32, _vp, _vp, _i32, _vp, _vp, _vp, _vp]),
+    "sswin_flash_forward_ordered": (_i32, [_i32, _vp, _vp, _vp, _i64, _i32, _i32, _i32, _vp, C.c_float, _vp, _i32, _i32, _vp, _vp, _vp]),
+    "sswin_flash_backward_ordered": (_i32, [_i32, _vp, _vp, _vp, _vp, _i64, _i32, _i32, _i32, _vp, C.c_float, _vp, _i32, _i32, _vp, _vp, _vp, _vp, _vp, _vp, _vp]),
     "sswin_layer_norm_supported": (_i32, [_i32, _i32]),
     "sswin_layer_norm_forward": (_i32, [_i32, _i32, _vp, _i64, _i32, _vp, _vp, C.c_float, _vp, _vp, _vp]),
     "sswin_layer_norm_backward_workspace_bytes": (_sz, [_i32, _i64, _i32]),

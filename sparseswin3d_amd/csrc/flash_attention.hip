@@ -27,8 +27,8 @@
 // Backward: with dS asked for (the bias table's gradient needs it) the key side forms scores, P and dS, sums dV and dK and stores
 // dS, and the query side is dQ = dS K from the stored dS; before, both sides formed them and the query side stored.
 //
-// 112 700 voxels, windows of 7^3, 3 heads of 16 (27 million scores): fp32 forward 63 us, backward 212 us, now 178 (D 11, key side 125,
-// dQ 42).  219 000 voxels, fp16: forward 84 us, backward 296, now 285 (14, 180, 91; dS is 217 MB written and read again).  dQ waits for
+// 112 700 voxels, windows of 7^3, 3 heads of 16 (27 million scores): fp32 forward 56 us, backward 172 (D 11, key side 117,
+// dQ 43; 63 and 178 with the work taken by rank).  225 700 voxels, fp16: forward 80 us, backward 285 (14, 180, 91; dS is 217 MB written and read again).  dQ waits for
 // memory, 15 us a wavefront of four 32 x 32 pieces; rows of dS padded to 64 bytes, rows read by neighbouring
 // lanes and exchanged, voxels kept in lanes change it by less than 3 %.  The block products with the attention matrix in memory take 195 and 258 us (112 700 voxels, fp32).  The vector ALU is
 // busy for half of a launch, the fp32 matrix instructions (which occupy it) for another quarter; leaving out the bias reads, the
@@ -52,6 +52,7 @@ constexpr float MASKED = -100.f * LOG2E;       // what sp_add_mask adds, in unit
 constexpr int WAVES = 4;
 constexpr int MAX_ROWS = 4096;
 constexpr int64_t MAX_TOKENS = 1 << 24;    // row numbers are multiplied in 24 bits
+constexpr int TOKENS_WAVES = 16, ORDER_THREADS = TOKENS_WAVES * 64, ORDER_CLASSES = 16, ORDER_MOST = 12288, ORDER_WINDOWS = 16384;
 
 // four reduction slots of one operand row
 template <typename T> struct Frag;
@@ -108,15 +109,71 @@ struct Args {
     void* dqkv;                // [N, 3 H hd]
     float* ds;                 // [c x c] blocks of the groups, or null
     const int32_t* tok_sq;     // sum of c * c over the windows before r's
+    const int32_t* work;       // chunks in the order they are taken, or null: by their ranks
 };
 
+// The chunks by descending work, those of equal work by their ranks (a window's stay together), by one workgroup.  A chunk's work follows from its window's
+// size, 1 to 22 steps, and the four wavefronts of a workgroup hold their place until the last is done: taken by their ranks, 61 to 69 %
+// of the places are in use, by descending work 89 to 97 % (simulated on the rooms of 112 700 and 225 700 voxels; 69 % measured).
+// 112 700 voxels fp32: forward 62.8 -> 56.0 us, key side 126.9 -> 117.3, dQ 42.9 either way (by rank behind an ordered key side 45.9); 225 700 fp16: forward
+// 89.4 -> 79.5, key side 182 -> 180.  The launch for the words takes 7.2 and 10.3 us with the order, 5.0 and 5.5 without.
+// The work is summed over the windows (their table is short; 7055 chunks of the token rows take one workgroup 40 us): a step of 16 tokens of the window counts
+// two, three with a second sub-tile, a block two more; windows of less than 32 tokens, which share blocks, count by their tokens.
+__device__ __forceinline__ void order_chunks(const int32_t* __restrict__ plan, int64_t g_cap, int64_t windows, int H, int64_t N, int32_t* __restrict__ work) {
+    __shared__ uint32_t cost[ORDER_MOST / 2];                            // two chunks each
+    __shared__ uint16_t place[ORDER_CLASSES * ORDER_THREADS];            // [class][thread]
+    __shared__ int sums[TOKENS_WAVES];
+    const int chunks = (int)((N + 31) / 32), t = threadIdx.x;
+    if (windows > ORDER_WINDOWS) {
+        for (int i = t; i < chunks; i += ORDER_THREADS) work[i] = i;
+        return;
+    }
+    for (int i = t; i < (chunks + 1) / 2; i += ORDER_THREADS) cost[i] = 0;
+    __syncthreads();
+    auto add = [&](int rank, int v) { atomicAdd(&cost[rank >> 6], (uint32_t)v << (rank >> 1 & 16)); };
+    for (int k = t; k < (int)windows; k += ORDER_THREADS) {
+        const int c = plan[(int64_t)k * H], T = plan[g_cap + (int64_t)k * H];
+        if (c < 32) add(T, (c + 7) / 8);
+        else
+            for (int j = 0; j < c; j += 32) add(T + j, (c + 15) / 16 * (c - j > 16 ? 3 : 2) + 2);
+    }
+    __syncthreads();
+    auto kind = [&](int i) { return ORDER_CLASSES - 1 - min((int)(cost[i >> 1] >> ((i & 1) * 16) & 0xffffu) / 4, ORDER_CLASSES - 1); };
+    for (int k = 0; k < ORDER_CLASSES; ++k) place[k * ORDER_THREADS + t] = 0;
+    __syncthreads();
+    const int per = (chunks + ORDER_THREADS - 1) / ORDER_THREADS, begin = min(t * per, chunks), end = min(begin + per, chunks);
+    for (int i = begin; i < end; ++i) ++place[kind(i) * ORDER_THREADS + t];
+    __syncthreads();
+    // sums in front, classes first; a thread adds 16 neighbours
+    int own = 0;
+    for (int k = 0; k < ORDER_CLASSES; ++k) own += place[t * ORDER_CLASSES + k];
+    int before = own;
+    for (int o = 1; o < 64; o <<= 1) {
+        const int v = __shfl_up(before, o, 64);
+        if ((t & 63) >= o) before += v;
+    }
+    if ((t & 63) == 63) sums[t >> 6] = before;
+    __syncthreads();
+    before -= own;
+    for (int w = 0; w < t >> 6; ++w) before += sums[w];
+    for (int k = 0; k < ORDER_CLASSES; ++k) {
+        const int n = place[t * ORDER_CLASSES + k];
+        place[t * ORDER_CLASSES + k] = (uint16_t)before;
+        before += n;
+    }
+    __syncthreads();
+    for (int i = begin; i < end; ++i) work[place[kind(i) * ORDER_THREADS + t]++] = i;
+}
+
 // What a token contributes to the table index, mask and window comparisons, one word per rank, and the sum of c * c over
-// the windows before its own; a wavefront per window
-__global__ __launch_bounds__(256) void flash_tokens_kernel(const int32_t* __restrict__ plan, int64_t g_cap, int64_t windows, int H,
-                                                           const int32_t* __restrict__ tok_pos, const int32_t* __restrict__ code,
-                                                           const int8_t* __restrict__ mask, int nmw, int n, uint32_t* __restrict__ word,
-                                                           int32_t* __restrict__ tok_sq) {
-    const int64_t k = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+// the windows before its own; a wavefront per window.  The first workgroup finds the chunks' order, if it is asked for.
+__global__ __launch_bounds__(ORDER_THREADS) void flash_tokens_kernel(const int32_t* __restrict__ plan, int64_t g_cap, int64_t windows, int H,
+                                                                     const int32_t* __restrict__ tok_pos, int64_t N, const int32_t* __restrict__ code,
+                                                                     const int8_t* __restrict__ mask, int nmw, int n, uint32_t* __restrict__ word,
+                                                                     int32_t* __restrict__ tok_sq, int32_t* __restrict__ work) {
+    int64_t block = blockIdx.x;
+    if (work && block-- == 0) return order_chunks(plan, g_cap, windows, H, N, work);
+    const int64_t k = block * TOKENS_WAVES + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     if (k >= windows) return;
     const int64_t g = k * H;                                             // the window's first group (head 0)
     const int c = plan[g], T = plan[g_cap + g], sq = plan[2 * g_cap + g] / H, w = plan[3 * g_cap + g];
@@ -230,6 +287,8 @@ __device__ __forceinline__ void place(int H, int64_t groups, int& h, int64_t& fi
         first = (groups / 8 * 8 + i % rest) * WAVES;
     }
 }
+
+__device__ __forceinline__ int64_t chunk_of(const Args& g, int64_t at) { return g.work && at * 32 < g.N ? g.work[at] : at; }
 
 template <typename T, int HD> struct Rows {
     static constexpr int NB = HD / 16;
@@ -349,7 +408,7 @@ __global__ __launch_bounds__(WAVES * 64, sizeof(T) == 4 ? 3 : 1) void flash_forw
     int64_t first;
     place(g.H, groups, h, first);
     const int lane = threadIdx.x & 63, l16 = lane & 15, quad = lane >> 4;
-    const int64_t chunk = first + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t chunk = chunk_of(g, first + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6));
     Blocks blocks(g, chunk * 32 < g.N ? chunk : 0);
     stage_table(g, h, table);
     if (chunk * 32 >= g.N) return;
@@ -476,7 +535,7 @@ __global__ __launch_bounds__(WAVES * 64) void flash_backward_q_kernel(Args g, in
     int64_t first;
     place(g.H, groups, h, first);
     const int lane = threadIdx.x & 63, l16 = lane & 15, quad = lane >> 4;
-    const int64_t chunk = first + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t chunk = chunk_of(g, first + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6));
     Blocks blocks(g, chunk * 32 < g.N ? chunk : 0);
     stage_table(g, h, table);
     if (chunk * 32 >= g.N) return;
@@ -596,7 +655,7 @@ __global__ __launch_bounds__(WAVES * 64) void flash_dq_kernel(Args g, int64_t gr
     int64_t first;
     place(g.H, groups, h, first);
     const int lane = threadIdx.x & 63, l16 = lane & 15, quad = lane >> 4;
-    const int64_t chunk = first + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t chunk = chunk_of(g, first + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6));
     if (chunk * 32 >= g.N) return;
     Blocks blocks(g, chunk);
     blocks.begin(g);
@@ -707,7 +766,7 @@ __global__ __launch_bounds__(WAVES * 64) void flash_backward_kv_kernel(Args g, i
     int64_t first;
     place(g.H, groups, h, first);
     const int lane = threadIdx.x & 63, l16 = lane & 15, quad = lane >> 4;
-    const int64_t chunk = first + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t chunk = chunk_of(g, first + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6));
     Blocks blocks(g, chunk * 32 < g.N ? chunk : 0);
     stage_table(g, h, table);
     if (chunk * 32 >= g.N) return;
@@ -859,26 +918,37 @@ int sswin_flash_supported(int dtype, int64_t N, int H, int hd, int rows) {
            N * 3 * H * hd < (1ll << 32);
 }
 
-int sswin_flash_tokens(const int32_t* plan, int64_t g_cap, int64_t groups, const int32_t* tokens, int64_t N, int H, int n, const int32_t* code,
-                       const int8_t* mask, int nmw, int32_t* word, int32_t* tok_sq, void* stream) {
+// Below, all wavefronts find a place at once (three a SIMD), and above, one workgroup is a while about it and the last places weigh little
+size_t sswin_flash_order_ints(int64_t N, int H) {
+    const int64_t chunks = (N + 31) / 32;
+    return chunks <= ORDER_MOST && chunks * H > 12 * (int64_t)device_cus() ? (size_t)chunks : 0;
+}
+
+int sswin_flash_tokens_ordered(const int32_t* plan, int64_t g_cap, int64_t groups, const int32_t* tokens, int64_t N, int H, int n, const int32_t* code,
+                               const int8_t* mask, int nmw, int32_t* word, int32_t* tok_sq, int32_t* order, void* stream) {
     SSWIN_CHECK(N >= 0 && n > 0 && H > 0 && groups >= 0 && groups <= g_cap && groups % H == 0, "flash_tokens: bad sizes");
     if (N == 0 || groups == 0) return 0;
     SSWIN_CHECK(plan && tokens && code && word && (!mask || nmw > 0), "flash_tokens: null pointer");
+    SSWIN_CHECK(!order || (N + 31) / 32 <= ORDER_MOST, "flash_tokens: an order of %lld tokens", (long long)N);
     const int64_t windows = groups / H;
-    hipLaunchKernelGGL(flash_tokens_kernel, dim3((unsigned)((windows + 3) / 4)), dim3(256), 0, static_cast<hipStream_t>(stream), plan, g_cap, windows, H,
-                       tokens + 3 * N, code, mask, nmw, n, reinterpret_cast<uint32_t*>(word), tok_sq);
+    hipLaunchKernelGGL(flash_tokens_kernel, dim3((unsigned)((windows + TOKENS_WAVES - 1) / TOKENS_WAVES + (order ? 1 : 0))), dim3(ORDER_THREADS), 0,
+                       static_cast<hipStream_t>(stream), plan, g_cap, windows, H, tokens + 3 * N, N, code, mask, nmw, n, reinterpret_cast<uint32_t*>(word), tok_sq, order);
     return launch_ok("flash_tokens");
 }
+int sswin_flash_tokens(const int32_t* plan, int64_t g_cap, int64_t groups, const int32_t* tokens, int64_t N, int H, int n, const int32_t* code,
+                       const int8_t* mask, int nmw, int32_t* word, int32_t* tok_sq, void* stream) {
+    return sswin_flash_tokens_ordered(plan, g_cap, groups, tokens, N, H, n, code, mask, nmw, word, tok_sq, nullptr, stream);
+}
 
-int sswin_flash_forward(int dtype, const int32_t* tokens, const int32_t* word, int64_t N, int H, int hd, int n, const void* qkv, float scale, const float* table,
-                        int rows, int offset0, void* out, float* lse, void* stream) {
+int sswin_flash_forward_ordered(int dtype, const int32_t* tokens, const int32_t* word, const int32_t* order, int64_t N, int H, int hd, int n, const void* qkv,
+                                float scale, const float* table, int rows, int offset0, void* out, float* lse, void* stream) {
     if (int rc = flash_check("flash_forward", dtype, N, H, hd, n, rows, offset0)) return rc;
     if (N == 0) return 0;
     SSWIN_CHECK(tokens && word && qkv && table && out && lse, "flash_forward: null pointer");
     SSWIN_CHECK(((uintptr_t)qkv | (uintptr_t)out) % 16 == 0, "flash_forward: pointers must be 16-byte aligned");
     Args g = {};
     g.order = tokens, g.tok_T = tokens + N, g.tok_c = tokens + 2 * N, g.word = reinterpret_cast<const uint32_t*>(word);
-    g.N = N, g.H = H, g.rows = rows, g.offset4 = offset0 * 4, g.scale = scale, g.table = table, g.qkv = qkv, g.out = out, g.lse = lse;
+    g.N = N, g.H = H, g.rows = rows, g.offset4 = offset0 * 4, g.scale = scale, g.table = table, g.qkv = qkv, g.out = out, g.lse = lse, g.work = order;
     hipStream_t s = static_cast<hipStream_t>(stream);
 #define FLASH(K, T) (hd == 16 ? launch(K<T, 16>, g, s, #K) : launch(K<T, 32>, g, s, #K))
     if (dtype == SSWIN_F32) return FLASH(flash_forward_kernel, float);
@@ -887,9 +957,14 @@ int sswin_flash_forward(int dtype, const int32_t* tokens, const int32_t* word, i
 #undef FLASH
 }
 
-int sswin_flash_backward(int dtype, const int32_t* tokens, const int32_t* word, const int32_t* tok_sq, int64_t N, int H, int hd, int n, const void* qkv, float scale,
-                         const float* table, int rows, int offset0, const void* out, const float* lse, const void* dout, void* dqkv, float* delta, float* ds,
-                         void* stream) {
+int sswin_flash_forward(int dtype, const int32_t* tokens, const int32_t* word, int64_t N, int H, int hd, int n, const void* qkv, float scale, const float* table,
+                        int rows, int offset0, void* out, float* lse, void* stream) {
+    return sswin_flash_forward_ordered(dtype, tokens, word, nullptr, N, H, hd, n, qkv, scale, table, rows, offset0, out, lse, stream);
+}
+
+int sswin_flash_backward_ordered(int dtype, const int32_t* tokens, const int32_t* word, const int32_t* tok_sq, const int32_t* order, int64_t N, int H, int hd, int n,
+                                 const void* qkv, float scale, const float* table, int rows, int offset0, const void* out, const float* lse, const void* dout,
+                                 void* dqkv, float* delta, float* ds, void* stream) {
     if (int rc = flash_check("flash_backward", dtype, N, H, hd, n, rows, offset0)) return rc;
     if (N == 0) return 0;
     SSWIN_CHECK(tokens && word && qkv && table && out && lse && dout && dqkv && delta && (!ds || tok_sq), "flash_backward: null pointer");
@@ -897,11 +972,16 @@ int sswin_flash_backward(int dtype, const int32_t* tokens, const int32_t* word, 
     Args g = {};
     g.order = tokens, g.tok_T = tokens + N, g.tok_c = tokens + 2 * N, g.word = reinterpret_cast<const uint32_t*>(word);
     g.N = N, g.H = H, g.rows = rows, g.offset4 = offset0 * 4, g.scale = scale, g.table = table, g.qkv = qkv, g.out = const_cast<void*>(out);
-    g.lse = const_cast<float*>(lse), g.dout = dout, g.delta = delta, g.dqkv = dqkv, g.ds = ds, g.tok_sq = tok_sq;
+    g.lse = const_cast<float*>(lse), g.dout = dout, g.delta = delta, g.dqkv = dqkv, g.ds = ds, g.tok_sq = tok_sq, g.work = order;
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (dtype == SSWIN_F32) return hd == 16 ? launch_backward<float, 16>(g, s) : launch_backward<float, 32>(g, s);
     if (dtype == SSWIN_F16) return hd == 16 ? launch_backward<__half, 16>(g, s) : launch_backward<__half, 32>(g, s);
     return hd == 16 ? launch_backward<__hip_bfloat16, 16>(g, s) : launch_backward<__hip_bfloat16, 32>(g, s);
+}
+int sswin_flash_backward(int dtype, const int32_t* tokens, const int32_t* word, const int32_t* tok_sq, int64_t N, int H, int hd, int n, const void* qkv, float scale,
+                         const float* table, int rows, int offset0, const void* out, const float* lse, const void* dout, void* dqkv, float* delta, float* ds,
+                         void* stream) {
+    return sswin_flash_backward_ordered(dtype, tokens, word, tok_sq, nullptr, N, H, hd, n, qkv, scale, table, rows, offset0, out, lse, dout, dqkv, delta, ds, stream);
 }
 
 }  // extern "C"

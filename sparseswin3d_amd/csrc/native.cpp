@@ -488,7 +488,7 @@ using AttentionPtr = c10::intrusive_ptr<Attention>;
 
 struct AttentionSaved {
     Tensor bias32, aux;     // bias or table; log-sum-exp of every attention row, or P
-    Tensor words;           // flash: int32 [2, N] token words and window offsets
+    Tensor words;           // flash: int32 token words [N], window offsets [N], and the order of the work where there is one
 };
 
 Tensor attention_forward(Attention& a, const Tensor& qkv, const Tensor& bias, AttentionSaved& saved) {
@@ -512,13 +512,16 @@ Tensor attention_forward(Attention& a, const Tensor& qkv, const Tensor& bias, At
     const auto fopt = qkv.options().dtype(at::kFloat);
     if (a.flash) {
         const Tensor table32 = saved.bias32 = bias.to(at::kFloat).contiguous();
-        saved.words = at::empty({2, N}, tp.tokens.options());
+        const int64_t ordered = (int64_t)sswin_flash_order_ints(N, a.H);
+        saved.words = at::empty({2 * N + ordered}, tp.tokens.options());
+        int32_t* const order = ordered ? i32(saved.words) + 2 * N : nullptr;
         saved.aux = at::empty({a.H, N}, fopt);
         Tensor o = at::empty({N, D}, qkv.options());
-        RUN(sswin_flash_tokens(i32(tp.plan), tp.g_cap, tp.G, i32(tp.tokens), N, a.H, a.n, i32(a.code), a.mask.defined() ? a.mask.data_ptr<int8_t>() : nullptr,
-                               a.regions(), i32(saved.words), i32(saved.words) + N, s));
-        RUN(sswin_flash_forward(dt, i32(tp.tokens), i32(saved.words), N, a.H, hd, a.n, ptr(qkv), (float)a.scale, f32(table32), (int)table32.size(0), a.offset0,
-                                ptr(o), f32(saved.aux), s));
+        RUN_NAMED("sswin_flash_tokens", sswin_flash_tokens_ordered(i32(tp.plan), tp.g_cap, tp.G, i32(tp.tokens), N, a.H, a.n, i32(a.code),
+                                                                   a.mask.defined() ? a.mask.data_ptr<int8_t>() : nullptr, a.regions(), i32(saved.words),
+                                                                   i32(saved.words) + N, order, s));
+        RUN_NAMED("sswin_flash_forward", sswin_flash_forward_ordered(dt, i32(tp.tokens), i32(saved.words), order, N, a.H, hd, a.n, ptr(qkv), (float)a.scale,
+                                                                     f32(table32), (int)table32.size(0), a.offset0, ptr(o), f32(saved.aux), s));
         return o;
     }
     if (a.code.defined()) {
@@ -592,8 +595,10 @@ Tensor attention_backward(const Attention& a, const Tensor& qkv, const Tensor& b
     const auto fopt = qkv.options().dtype(at::kFloat);
     if (a.flash) {
         Tensor d_s = want_bias ? at::empty({std::max<int64_t>(tp.A, 1)}, fopt) : Tensor(), delta = at::empty({a.H, N}, fopt);
-        RUN(sswin_flash_backward(dt, i32(tp.tokens), i32(saved.words), i32(saved.words) + N, N, a.H, hd, a.n, ptr(qkv), (float)a.scale, f32(saved.bias32),
-                                 (int)saved.bias32.size(0), a.offset0, ptr(out), f32(saved.aux), ptr(d_out), ptr(d_qkv), f32(delta), f32(d_s), s));
+        RUN_NAMED("sswin_flash_backward", sswin_flash_backward_ordered(dt, i32(tp.tokens), i32(saved.words), i32(saved.words) + N,
+                                                                       saved.words.numel() > 2 * N ? i32(saved.words) + 2 * N : nullptr, N, a.H, hd, a.n, ptr(qkv),
+                                                                       (float)a.scale, f32(saved.bias32), (int)saved.bias32.size(0), a.offset0, ptr(out),
+                                                                       f32(saved.aux), ptr(d_out), ptr(d_qkv), f32(delta), f32(d_s), s));
         if (want_bias) d_bias = bias_gradient(a, d_s, bias);
         return d_qkv;
     }

@@ -155,3 +155,53 @@ def test_flash_keeps_what_is_not_finite_where_it_belongs(which, value, hd, dtype
         assert not got[want.isnan()].isfinite().any(), what
     if which != "dO":
         assert not torch.isfinite(out).all()
+
+
+# chunks of 32 tokens: one, some threads without any, several a thread, the most an order holds; windows that fill, span and share
+# chunks; more windows than an order takes, which leaves the chunks as they are
+@pytest.mark.parametrize("N,sizes", [(1, "all"), (32, "all"), (33, "all"), (1000, "all"), (34001, "all"), (12288 * 32, "all"), (40000, "small")])
+def test_flash_order_of_the_work(N, sizes):
+    """The order holds every chunk once, by descending work, and results have the bits they have without one."""
+    import ctypes as C
+    from sparseswin3d_amd import _lib
+    from sparseswin3d_amd.fused import BiasTableIndex, TokenPlan
+    from sparseswin3d_amd.window_attention import relative_position_index_3d
+    lib, H, n = _lib.load(), 1, 343
+    rng = np.random.default_rng(N)
+    counts, left = [], N
+    while left:
+        counts.append(int(min(rng.choice([1, 5, 20, 31, 32, 33, 64, 100, 250, 343] if sizes == "all" else [1, 2, 3]), left)))
+        left -= counts[-1]
+    ind = torch.from_numpy(ragged_window_indices(rng, counts, n)).cuda()
+    ti = BiasTableIndex.build(relative_position_index_3d((7, 7, 7)).cuda(), 2197)
+    plan = TokenPlan(ind, len(counts), n, H).native
+    plan._finish()
+    ptr = lambda t: C.c_void_p(t.data_ptr())
+    stream = C.c_void_p(torch.cuda.current_stream().cuda_stream)
+    qkv, d_o, table = torch.randn(N, 48).cuda(), torch.randn(N, 16).cuda(), torch.randn(2197, H).cuda()
+    chunks, got = (N + 31) // 32, []
+    assert lib.sswin_flash_order_ints(N, 3) == (chunks if 3 * chunks > 12 * torch.cuda.get_device_properties(0).multi_processor_count else 0)
+    for order in (None, torch.full((chunks,), -1, dtype=torch.int32, device="cuda")):
+        words = torch.empty(2 * N, dtype=torch.int32, device="cuda")
+        out, lse, d_qkv, delta = torch.empty(N, 16).cuda(), torch.empty(H, N).cuda(), torch.empty(N, 48).cuda(), torch.empty(H, N).cuda()
+        d_s, o, sq = torch.empty(max(plan.A, 1)).cuda(), None if order is None else ptr(order), C.c_void_p(words.data_ptr() + 4 * N)
+        _lib.check(lib.sswin_flash_tokens_ordered(ptr(plan.plan), plan.g_cap, plan.G, ptr(plan.tokens), N, H, n, ptr(ti.code), None, 0, ptr(words), sq, o, stream))
+        _lib.check(lib.sswin_flash_forward_ordered(0, ptr(plan.tokens), ptr(words), o, N, H, 16, n, ptr(qkv), 0.25, ptr(table), 2197, ti.offset0, ptr(out), ptr(lse),
+                                                   stream))
+        _lib.check(lib.sswin_flash_backward_ordered(0, ptr(plan.tokens), ptr(words), sq, o, N, H, 16, n, ptr(qkv), 0.25, ptr(table), 2197, ti.offset0, ptr(out),
+                                                    ptr(lse), ptr(d_o), ptr(d_qkv), ptr(delta), ptr(d_s), stream))
+        got.append((words, out, lse, d_qkv, d_s[:plan.A]))
+    assert all(torch.equal(a, b) for a, b in zip(*got))
+    assert torch.equal(order.sort()[0].cpu(), torch.arange(chunks, dtype=torch.int32))
+    cost, T = np.zeros(chunks, dtype=np.int64), 0
+    for c in counts:                                               # steps of 16 over the window: two, three with a second sub-tile, two a block
+        if c < 32:
+            cost[T // 32] += (c + 7) // 8
+        else:
+            for j in range(0, c, 32):
+                cost[(T + j) // 32] += (c + 15) // 16 * (3 if c - j > 16 else 2) + 2
+        T += c
+    assert np.array_equal(order.cpu().numpy(), np.argsort(15 - np.minimum(cost // 4, 15), kind="stable") if len(counts) <= 16384 else np.arange(chunks))
+    with pytest.raises(RuntimeError):
+        big = 12288 * 32 + 1
+        _lib.check(lib.sswin_flash_tokens_ordered(ptr(plan.plan), plan.g_cap, plan.G, ptr(plan.tokens), big, H, n, ptr(ti.code), None, 0, ptr(words), sq, o, stream))
