@@ -158,6 +158,22 @@ def test_tall_linear_input_grad(N, P, K):
     assert ((dx.double() - ref).abs() / scale).max().item() < TOL
 
 
+@pytest.mark.parametrize("N", [32, 3001, 30001])
+def test_tall_linear_input_grad_at_any_address(N):
+    """96 columns of dY: results that do not start at 16 bytes."""
+    from sparseswin3d_amd import _lib
+    lib = _lib.load()
+    gen = torch.Generator(device="cuda").manual_seed(N)
+    dy, w = torch.randn(N, 96, generator=gen, device="cuda"), torch.randn(96, 192, generator=gen, device="cuda")
+    ref, mag = dy.double() @ w.double(), dy.double().abs() @ w.double().abs()
+    room = torch.full((N * 192 + 4,), float("nan"), device="cuda")
+    for at in range(4):
+        dx = room[at:at + N * 192]
+        _lib.check(lib.sswin_tall_linear_input_grad(C.c_void_p(dy.data_ptr()), N, 96, C.c_void_p(w.data_ptr()), 192, C.c_void_p(dx.data_ptr()),
+                                                    C.c_void_p(torch.cuda.current_stream().cuda_stream)))
+        assert ((dx.view(N, 192).double() - ref).abs() <= TOL * mag).all(), at
+
+
 def test_tall_linear_input_grad_unsupported_shapes():
     from sparseswin3d_amd import _lib
     lib = _lib.load()
