@@ -1071,15 +1071,18 @@ static int launch_forward(const void* x, int64_t N, int K, const void* w, int P,
         return launch_ok("dense, few rows");
     }
     if constexpr (Op<T>::PL == 3) {
+        // In place only dense_rows_kernel, which has read a row's values and formed what came out NaN again before it stores the first column: the
+        // kernels of pairs store 32 columns at a time, that of tall_linear.hip reads rows of the last tile twice.
+        const bool apart = ep.y != x;
         // 96 channels: the kernels that keep Wop in LDS
-        if (K == 96 && P % 96 == 0) {
+        if (apart && K == 96 && P % 96 == 0) {
             int rc = 0;
             if (pairs_held<EPI, DOWN>(xp, N, wp, P, ep, s, rc)) return rc;
             return staged_layer_96(xp, N, wp, P, DOWN, ep, s);
         }
         // fp16 pairs, from the reductions on whose sums come out as exactly: error against float64 (2-norms) with 96 channels 7.8e-8 and
         // 1.0e-7 here, 144 1.1e-7 and 1.75e-7 (turned); 48 channels of three bf16 pieces 6.9e-8, of pairs 7.1e-8 and more
-        if (pairs_takes(K) && ws_bytes >= pairs_workspace_bytes(K, P)) return pairs_layer<EPI, DOWN>(xp, N, K, wp, P, ep, ws, s);
+        if (apart && pairs_takes(K) && ws_bytes >= pairs_workspace_bytes(K, P)) return pairs_layer<EPI, DOWN>(xp, N, K, wp, P, ep, ws, s);
         // wavefronts per SIMD: what the registers allow without spilling (four: forward equal, input gradient 89 us against 40)
         return launch_rows<EPI, DOWN, 4, 1, 3>(xp, N, K, wp, P, ep, s);
     } else {

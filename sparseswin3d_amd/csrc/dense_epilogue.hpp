@@ -146,7 +146,7 @@ __device__ __forceinline__ void finish8(const Epilogue& ep, int64_t row, int col
 int staged_layer_96(const float* x, int64_t N, const float* w, int P, bool transposed, const Epilogue& ep, hipStream_t s);
 // whether a layer of N rows, K -> P, takes the kernel for few rows, whose wavefronts share the reduction (dense.hip)
 bool few_rows(int dtype, int64_t N, int K, int P);
-// fp32 layers as fp16 pairs (dense_pairs.hip), W's pieces in ws
+// fp32 layers as fp16 pairs (dense_pairs.hip), W's pieces in ws; y and x apart, here and below
 inline bool pairs_takes(int K) { return K >= 96; }
 size_t pairs_workspace_bytes(int K, int P);
 template <int EPI, bool DOWN> int pairs_layer(const float* x, int64_t N, int K, const float* w, int P, const Epilogue& ep, void* ws, hipStream_t s);

@@ -405,8 +405,8 @@ template <int EPI, bool DOWN, int CT> static int launch_held(const float* x, int
 template <int EPI, bool DOWN> bool pairs_held(const float* x, int64_t N, const float* w, int P, const Epilogue& ep, hipStream_t s, int& rc) {
     const int64_t workgroups = (N + HELD_WAVES * 32 - 1) / (HELD_WAVES * 32) * (P / 96);   // of 96 columns
     // few of them: 32 columns (7000 rows 96 -> 288, 84 workgroups: 10.1 us with 96 columns, 8.0 with 32; 36 000 96 -> 96, 141: 12.4 and 11.1; 28 000 96 -> 192,
-    // 220: 11.2 and 12.9).  Not in place, where other workgroups read the rows.
-    const bool few = workgroups * 8 <= device_cus() * 5 && ep.y != x;
+    // 220: 11.2 and 12.9)
+    const bool few = workgroups * 8 <= device_cus() * 5;
     if (Second4<float, float, EPI>::USED && !few) return false;
     if constexpr (Second4<float, float, EPI>::USED) rc = launch_held<EPI, DOWN, 1>(x, N, w, P, ep, s);
     else rc = few ? launch_held<EPI, DOWN, 1>(x, N, w, P, ep, s) : launch_held<EPI, DOWN, 3>(x, N, w, P, ep, s);

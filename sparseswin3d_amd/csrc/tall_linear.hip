@@ -882,8 +882,8 @@ int sswin_tall_linear_input_grad(const float* dy, int64_t N, int P, const float*
     if (P == 96 && N >= 32) {
         SSWIN_CHECK(((uintptr_t)w % 16) == 0, "tall_linear_input_grad: w must be 16-byte aligned");
         int rc = 0;
-        // which stores dX in 16-byte pieces
-        if ((uintptr_t)dx % 16 == 0 && dense::pairs_held<dense::EPI_NONE, true>(dy, N, w, K, dense::Epilogue{nullptr, nullptr, dx, nullptr}, s, rc)) return rc;
+        // which stores dX in 16-byte pieces, and not in the place of dY
+        if ((uintptr_t)dx % 16 == 0 && dx != dy && dense::pairs_held<dense::EPI_NONE, true>(dy, N, w, K, dense::Epilogue{nullptr, nullptr, dx, nullptr}, s, rc)) return rc;
     }
     return launch_chunked<true>(dy, N, P, w, nullptr, K, dx, cus, s, "tall_linear_input_grad");
 }

@@ -141,6 +141,35 @@ def test_dense_forward_in_place(K):
     _check(x, ref, mag, dtype, "in place")
 
 
+# fp32 in place with values that are not finite, whose results are formed again from rows that lie where results go; 32 and 96 columns a
+# workgroup where the rows lie apart, a ragged last tile.  Up to 48 channels, 96, and with a workspace for pieces that in place has no use for
+@pytest.mark.parametrize("N,K", [(19201, 96), (30001, 96), (140001, 48)])
+@pytest.mark.parametrize("epi", [PLAIN, RESIDUAL])
+@pytest.mark.parametrize("where", ["finite", "weight", "rows"])
+def test_dense_fp32_forward_in_place(N, K, epi, where):
+    from sparseswin3d_amd import _lib
+    lib = _lib.load()
+    for transposed in (0, 1):
+        if transposed and epi == RESIDUAL:
+            continue
+        gen = torch.Generator().manual_seed(N + K)
+        x, w, extra = torch.randn(N, K, generator=gen), torch.randn(K, K, generator=gen), torch.randn(N, K, generator=gen).cuda()
+        if where == "weight":
+            w[(K - 8, 40) if transposed else (40, K - 8)] = float("inf")
+        elif where == "rows":
+            x[N // 2, 40], x[N - 1, 3] = float("inf"), float("nan")
+        x, w = x.cuda(), w.cuda()
+        wd = w.double() if transposed else w.double().T
+        ref, scale = x.double() @ wd, x.double().abs() @ wd.abs()
+        if epi == RESIDUAL:
+            ref, scale = ref + extra.double(), scale + extra.double().abs()
+        ws = torch.empty(1 << 20, dtype=torch.uint8, device="cuda")
+        _lib.check(lib.sswin_dense_forward(0, 0, transposed, epi, _ptr(x), N, K, _ptr(w), None, K, _ptr(extra) if epi == RESIDUAL else None, _ptr(x), None,
+                                           _ptr(ws), ws.numel(), _stream()))
+        _same_class(x, ref, scale, f"transposed {transposed}")
+        assert ref.isfinite().all() == (where == "finite")
+
+
 # 16 bit: the last rows of the few-rows kernel and the first of the tiles behind it, with a residual and as an input gradient
 @pytest.mark.parametrize("N", [5376, 5377])
 def test_dense_forward_where_the_tiles_take_over(N):

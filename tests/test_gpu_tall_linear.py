@@ -174,6 +174,22 @@ def test_tall_linear_input_grad_at_any_address(N):
         assert ((dx.view(N, 192).double() - ref).abs() <= TOL * mag).all(), at
 
 
+@pytest.mark.parametrize("N", [3001, 30001])
+def test_tall_linear_input_grad_in_place(N):
+    """dX in the place of dY (96 -> 96); an infinity in W reaches its own column only."""
+    from sparseswin3d_amd import _lib
+    lib = _lib.load()
+    gen = torch.Generator(device="cuda").manual_seed(N)
+    for value in (1.0, float("inf")):
+        dy, w = torch.randn(N, 96, generator=gen, device="cuda"), torch.randn(96, 96, generator=gen, device="cuda")
+        ref, mag = dy.double() @ w.double(), dy.double().abs() @ w.double().abs()
+        w[88, 40] = value * w[88, 40]
+        _lib.check(lib.sswin_tall_linear_input_grad(C.c_void_p(dy.data_ptr()), N, 96, C.c_void_p(w.data_ptr()), 96, C.c_void_p(dy.data_ptr()),
+                                                    C.c_void_p(torch.cuda.current_stream().cuda_stream)))
+        good = ((dy.double() - ref).abs() <= TOL * mag).all(0)
+        assert good.sum() == (96 if value == 1 else 95) and good[40] == (value == 1), value
+
+
 def test_tall_linear_input_grad_unsupported_shapes():
     from sparseswin3d_amd import _lib
     lib = _lib.load()
