@@ -478,7 +478,8 @@ int sswin_mlp_forward(int dtype, int out_dtype, const void* x, int64_t N, int D,
 int sswin_mlp_backward(int dtype, const void* dy, int64_t N, int D, int hidden, const void* w1, const void* w2, const void* slope, void* du, void* dx, void* ws,
                        size_t ws_bytes, void* stream);
 /* scratch for long reductions over few rows (shares of the reduction added in a fixed order), and for the pieces of fp32 weights; with
- * less the call runs without */
+ * less, or a null pointer, the call runs without.  16-byte aligned; written by every call that is given one, so calls on several streams
+ * need one each. */
 size_t sswin_dense_forward_workspace_bytes(int dtype, int64_t N, int K, int P);
 /* dw [P, K] = dy^T x and db [P] = column sums of dy (or null) for dy [N, P], x [N, K] of dtype; dw, db of out_dtype (dtype or
  * fp32).  Partial sums over row chunks are added in a fixed order: the same bits on every run. */

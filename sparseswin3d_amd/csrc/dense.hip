@@ -1291,6 +1291,7 @@ int sswin_dense_forward(int dtype, int out_dtype, int transposed, int epilogue, 
                 "dense_forward: pointers must be 16-byte aligned");
     const Epilogue ep = {bias, extra, y, slope};
     SSWIN_CHECK(((uintptr_t)ws) % 16 == 0, "dense_forward: the workspace must be 16-byte aligned");
+    if (!ws) ws_bytes = 0;                                               // whatever size goes with a null pointer
     float* f = static_cast<float*>(ws);
     hipStream_t s = static_cast<hipStream_t>(stream);
     const bool down = transposed != 0;

@@ -583,6 +583,19 @@ def test_dense_fp32_without_a_workspace():
     _check(y, x.double() @ w.double().T, x.double().abs() @ w.double().abs().T, torch.float32, "plain")
 
 
+# a null workspace with a size beside it: fp32 with pieces of W, 16 bit with shares of the reduction
+@pytest.mark.parametrize("N,K,P,dtype", [(20001, 208, 144, torch.float32), (1364, 3072, 768, torch.bfloat16)])
+def test_dense_null_workspace_with_a_size(N, K, P, dtype):
+    from sparseswin3d_amd import _lib
+    lib = _lib.load()
+    gen = torch.Generator().manual_seed(5)
+    x, w, y = _rand(gen, N, K, dtype=dtype), (_rand(gen, P, K, spread=1) / K ** 0.5).to(dtype), torch.full((N, P), float("nan"), dtype=dtype, device="cuda")
+    nb = lib.sswin_dense_forward_workspace_bytes(CODE[dtype], N, K, P)
+    assert nb > 0
+    _lib.check(lib.sswin_dense_forward(CODE[dtype], CODE[dtype], 0, PLAIN, _ptr(x), N, K, _ptr(w), None, P, None, _ptr(y), None, None, nb, _stream()))
+    _check(y, x.double() @ w.double().T, x.double().abs() @ w.double().abs().T, dtype, "plain")
+
+
 # each tile shape where its sums are shortest or longest for their number; relative error of dW against float64 (2-norms).  The
 # bounds are a twentieth above what tiles of 96 x 96 (64 x 64 up to 64 columns) with sums of at least 64 rows give there, averaged over
 # as many inputs.
