@@ -456,7 +456,9 @@ int sswin_tall_linear_weight_grad(const float* dy, const float* x, int64_t N, in
  * (the input gradient of a layer with K outputs and P inputs; no bias).  x, w and bias: dtype; y: out_dtype (dtype, or fp32
  * with SSWIN_DENSE_RESIDUAL under mixed precision, where the residual stream is fp32).
  * epilogue SSWIN_DENSE_GELU: y = gelu(.), slope [N, P] = its derivative (or null); SSWIN_DENSE_RESIDUAL: y = . + extra [N, P]
- * of out_dtype; SSWIN_DENSE_SCALE (transposed only): y = . * extra [N, P] of dtype.  Accumulation in fp32. */
+ * of out_dtype; SSWIN_DENSE_SCALE (transposed only): y = . * extra [N, P] of dtype.  Accumulation in fp32.
+ * fp32 operands are split into pieces of 16 bits (three bf16, or two fp16 with a scale per row and column); either way the error of a result
+ * is bounded by the sum of the absolute products, as that of a plain fp32 sum is, whatever the range of values in a row or column. */
 enum { SSWIN_DENSE_PLAIN = 0, SSWIN_DENSE_GELU = 1, SSWIN_DENSE_RESIDUAL = 2, SSWIN_DENSE_SCALE = 3 };
 int sswin_dense_supported(int dtype, int P, int K);
 int sswin_dense_forward(int dtype, int out_dtype, int transposed, int epilogue, const void* x, int64_t N, int K, const void* w,

@@ -1,5 +1,5 @@
-// Operands of the matrix instructions of the dense layers (dense.hip, mlp.hip): fp32 values as three bf16 pieces, 16-bit values
-// as they are, and the copies from memory to LDS that pass no register.
+// Operands of the matrix instructions of the dense layers (dense.hip, dense_pairs.hip, mlp.hip): fp32 values as three bf16 pieces or two
+// fp16 pieces, 16-bit values as they are, and the copies from memory to LDS that pass no register.
 #pragma once
 
 #include <stdint.h>
@@ -78,11 +78,17 @@ __device__ __forceinline__ void planes_of(const float (&v)[8], u32x4 (&out)[Op<T
 
 // fp32 values as two fp16 pieces, h rounded to nearest and l, 2^11 times what is left of it, also rounded: x 2^e = h + l 2^-11 to 2^-23 of
 // the power of two above x, so three products of 11 bits each take the place of six of 8: (h,h), and (l,h) (h,l) into sums of their own, for
-// their factor.  Half the matrix instructions, two thirds of the operand bytes and half the vector instructions.  What is lost: a bit of a
+// their factor (published as error-corrected half-precision products: Ootomo and Yokota, "Recovering single precision accuracy from Tensor
+// Cores while surpassing the FP32 theoretical peak performance", 2022; here with a scale per row and column).
+// Half the matrix instructions, two thirds of the operand bytes and half the vector instructions.  What is lost: a bit of a
 // quarter of the values (6e-8 of a result, with l l); what is won: the matrix instructions do not round their sums to nearest, and
-// (h,h) is one of them a step, in place of six.  fp16 has five bits of exponent, so rows (and columns) are scaled by a power of two that
-// takes their largest value below 2^15; values down to 2^-25 of the largest keep all bits, since l is of h's size, and smaller ones are off by at
-// most 2^-50 of it.  Infinities and NaN leave NaN, as above.
+// (h,h) is one of them a step, in place of six.  Infinities and NaN leave NaN, as above.
+// fp16 has five bits of exponent, so rows (and columns) are scaled by a power of two: fixed, so that the largest value lies in [2^14, 2^15), or
+// following the largest value so far, which then lies above 2^12 (pairs_rows_kernel, hidden values of mlp_kernel).  Scaled values
+// from 2^-13 on keep all bits, since l is of h's size: down to 2^-27 of the row's largest, 2^-25 of the largest so far.  Smaller ones are off by up to
+// 2^-36, so a sum of K products, each with a factor below 2^15, by up to K 2^-20.  Sums of at least PAIRS_SMALL are therefore right to K 2^-26 of themselves, a
+// quarter of what K roundings of plain fp32 may add up to; smaller ones, unless row or column is all zeros, are formed again in plain fp32
+// (normally distributed operands: one in 2^20 and fewer).
 struct Pairs {
     static constexpr float LOW = 0.00048828125f;                         // 2^-11
     static __device__ __forceinline__ f32x16 mfma(const u32x4& a, const u32x4& b, const f32x16& c) {
@@ -101,16 +107,30 @@ __device__ __forceinline__ void split_pairs(const float (&v)[8], float scale, u3
         out[1][q] = __builtin_bit_cast(uint32_t, l);
     }
 }
+constexpr float PAIRS_SMALL = 64.f;
 // exponent E with |v| < 2^E; of zero far below that of any value.  (Infinities and NaN: 0.)
 __device__ __forceinline__ int exponent_above(float most) { return most == 0.f ? -200 : __builtin_amdgcn_frexp_expf(most); }
-// scales stay normal numbers: rows of values below 2^-105 have fewer bits
-constexpr int PAIRS_MOST_SCALE = 120;
+// Exponent of the scale of a row whose largest value lies below 2^above.  Scales stay normal numbers; exponents above PAIRS_MOST_SCALE
+// say that the row (so far) is all zeros.
+constexpr int PAIRS_MOST_SCALE = 120, PAIRS_ZEROS = 121, PAIRS_ZEROS_SO_FAR = 200;
+__device__ __forceinline__ int pairs_scale(int above) { return above == -200 ? PAIRS_ZEROS : min(15 - above, PAIRS_MOST_SCALE); }
+// The same where it follows the largest value: from e on to a step whose values lie below 2^above (above + e > 15: they would leave fp16's range)
+__device__ __forceinline__ int pairs_scale_after(int above, int e) { return above + e > 15 ? min(13 - above, PAIRS_MOST_SCALE) : e; }
 __device__ __forceinline__ float power_of_two(int e) { return __builtin_amdgcn_ldexpf(1.f, e); }
 __device__ __forceinline__ float largest(const float (&v)[8]) {
     float m = fabsf(v[0]);
 #pragma unroll
     for (int e = 1; e < 8; ++e) m = fmaxf(m, fabsf(v[e]));
     return m;
+}
+// The least value that is not zero, as a number that grows with it (0xffffffff: none so far), and whether pieces of that scale lose bits of it
+__device__ __forceinline__ uint32_t least_nonzero(const float (&v)[8], uint32_t m) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) m = min(m, (__builtin_bit_cast(uint32_t, v[e]) << 1) - 1u);
+    return m;
+}
+__device__ __forceinline__ bool pairs_lose(uint32_t least, float scale) {
+    return least != 0xffffffffu && __builtin_bit_cast(float, (least + 1u) >> 1) * scale < 0x1p-13f;
 }
 // of a lane and the one 32 lanes away
 __device__ __forceinline__ float largest_of_halves(float m) {
@@ -120,11 +140,13 @@ __device__ __forceinline__ float largest_of_halves(float m) {
 
 // Pieces of the columns [32 tile, 32 tile + 32) of Wop [K, P] (W [P, K] turned, or with DOWN W [K, P] itself), a scale per column, by a workgroup of
 // WAVES wavefronts: put(column, step of 16 channels, half of it, pieces); columns past the last repeat it.  Returns the exponent of the
-// scale of the lane's column, to all.
-template <bool DOWN, int WAVES, typename PUT>
+// scale of the lane's column, to all; with LOST, PAIRS_LOST more where the pieces lose bits.
+constexpr int PAIRS_LOST = 1024;
+template <bool DOWN, int WAVES, bool LOST, typename PUT>
 __device__ __forceinline__ int pairs_of_columns(const float* __restrict__ w, int K, int P, int tile, PUT put) {
     constexpr int KEPT = 4;                                              // steps of a wavefront in registers: 64 WAVES channels are read once
     __shared__ float most[WAVES][32];
+    __shared__ uint32_t leasts[LOST ? WAVES : 1][32];
     const int wave = threadIdx.x >> 6, half = (threadIdx.x & 63) >> 5, l32 = threadIdx.x & 31;
     const int col = min(tile * 32 + l32, P - 1), steps = K / 16;
     auto load = [&](int ks, float (&v)[8]) {
@@ -140,23 +162,35 @@ __device__ __forceinline__ int pairs_of_columns(const float* __restrict__ w, int
         }
     };
     float kept[KEPT][8], m = 0.f;
+    uint32_t least = 0xffffffffu;
+    auto see = [&](const float (&v)[8]) {
+        m = fmaxf(m, largest(v));
+        if constexpr (LOST) least = least_nonzero(v, least);
+    };
 #pragma unroll
     for (int i = 0; i < KEPT; ++i)
         if (wave + i * WAVES < steps) load(wave + i * WAVES, kept[i]);
 #pragma unroll
     for (int i = 0; i < KEPT; ++i)
-        if (wave + i * WAVES < steps) m = fmaxf(m, largest(kept[i]));
+        if (wave + i * WAVES < steps) see(kept[i]);
     for (int ks = wave + KEPT * WAVES; ks < steps; ks += WAVES) {
         float v[8];
         load(ks, v);
-        m = fmaxf(m, largest(v));
+        see(v);
     }
     m = largest_of_halves(m);
-    if (half == 0) most[wave][l32] = m;
+    if constexpr (LOST) least = min(least, (uint32_t)__shfl_xor((int)least, 32, 64));
+    if (half == 0) {
+        most[wave][l32] = m;
+        if constexpr (LOST) leasts[wave][l32] = least;
+    }
     __syncthreads();
 #pragma unroll
-    for (int q = 0; q < WAVES; ++q) m = fmaxf(m, most[q][l32]);
-    const int e = min(15 - exponent_above(m), PAIRS_MOST_SCALE);
+    for (int q = 0; q < WAVES; ++q) {
+        m = fmaxf(m, most[q][l32]);
+        if constexpr (LOST) least = min(least, leasts[q][l32]);
+    }
+    const int e = pairs_scale(exponent_above(m));
     const float scale = power_of_two(e);
     u32x4 p[2];
 #pragma unroll
@@ -171,7 +205,7 @@ __device__ __forceinline__ int pairs_of_columns(const float* __restrict__ w, int
         split_pairs(v, scale, p);
         put(tile * 32 + l32, ks, half, p);
     }
-    return e;
+    return LOST && pairs_lose(least, scale) ? e + PAIRS_LOST : e;
 }
 
 // Pieces of an infinity hold a NaN, and so does every result one takes part in, as do pieces whose sums leave the range: fp32
@@ -203,6 +237,33 @@ __device__ __forceinline__ f32x4 plain_products(const float* a, int64_t a_step, 
     }
     return s;
 }
+
+__device__ __forceinline__ float wave_sum(float v) {
+    v = row16_sum(v);
+    v += __shfl_xor(v, 16, 64);
+    return v + __shfl_xor(v, 32, 64);
+}
+// the smaller of |a| and |b|, NaN where one is; whether results of a row whose scale's exponent is e, the least of them as it left the products, are NaN
+// or small
+__device__ __forceinline__ float least_size(float a, float b) { return __builtin_elementwise_minimum(fabsf(a), fabsf(b)); }
+__device__ __forceinline__ bool nan_or_small(float least, int e) { return e <= PAIRS_MOST_SCALE ? !(least >= PAIRS_SMALL) : least != least; }
+// sum over i < n of a[i] b[i b_step], by a wavefront (a, b uniform), to all its lanes
+__device__ __forceinline__ float wave_product(const float* a, const float* b, int64_t b_step, int n) {
+    float s = 0.f;
+#pragma unroll 1
+    for (int i = threadIdx.x & 63; i < n; i += 64) s = fmaf(a[i], b[i * b_step], s);
+    return wave_sum(s);
+}
+// again(lane, bit) for every bit set in the lanes' masks, by the wavefront together: a result formed again takes it 2 us, by a lane alone some 20
+template <typename F> __device__ __forceinline__ void for_each_small(uint32_t mask, F again) {
+    while (const uint64_t lanes = __ballot(mask != 0)) {
+        const int owner = __builtin_ctzll(lanes);
+        again(owner, __builtin_ctz((uint32_t)__builtin_amdgcn_readlane((int)mask, owner)));
+        if ((int)(threadIdx.x & 63) == owner) mask &= mask - 1;
+    }
+}
+// more of them, by lane, than one by one pays for
+__device__ __forceinline__ bool many_small(uint32_t mask) { return __popcll(__ballot(mask != 0)) > 8; }
 
 // a last ragged tile is moved back to end at row N, tiles behind it repeat it: rows stored twice hold the same bits
 __device__ __forceinline__ int64_t tile_row(int64_t t, int64_t N) { return t * 32 + 32 <= N ? t * 32 : N - 32; }

@@ -40,7 +40,7 @@ __global__ __launch_bounds__(DOWN ? 1024 : 256) void pairs_weights_kernel(const 
     const int ksteps = pairs_ksteps(K);
     auto at = [&](int col, int ks, int half) { return planes + ((int64_t)(col >> 5) * ksteps + ks) * 128 + half * 32 + (col & 31); };
     if constexpr (DOWN) {
-        const int e = pairs_of_columns<true, 16>(w, K, P, blockIdx.x, [&](int col, int ks, int half, const u32x4 (&p)[2]) {
+        const int e = pairs_of_columns<true, 16, false>(w, K, P, blockIdx.x, [&](int col, int ks, int half, const u32x4 (&p)[2]) {
             u32x4* dst = at(col, ks, half);
             dst[0] = p[0];
             dst[64] = p[1];
@@ -71,7 +71,7 @@ __global__ __launch_bounds__(DOWN ? 1024 : 256) void pairs_weights_kernel(const 
         }
         m = largest_of_halves(row16_max(m));
         m = fmaxf(m, __shfl_xor(m, 16, 64));
-        const int e = min(15 - exponent_above(m), PAIRS_MOST_SCALE);
+        const int e = pairs_scale(exponent_above(m));
         const float scale = power_of_two(e);
         auto put = [&](int i, const float (&v)[8]) {
             u32x4 p[2];
@@ -91,6 +91,22 @@ __global__ __launch_bounds__(DOWN ? 1024 : 256) void pairs_weights_kernel(const 
         if (ksteps > K / 16 && lane < 4) at(col, K / 16, lane >> 1)[(lane & 1) * 64] = u32x4{0, 0, 0, 0};
         if (lane == 0) exps[col] = e;
     }
+}
+
+// The results of a wavefront's tile of 32 x 32 whose bits are set in `mask` (of lane l, register r: row l % 32, column 8 (r / 4) + 4 (l / 32) + r % 4)
+// from product(row, column), or marked with NaN if they are many
+template <typename F> __device__ __forceinline__ void small_again(u32x4* tile, uint32_t mask, F product) {
+    const int lane = threadIdx.x & 63;
+    auto at = [&](int l, int r) { return reinterpret_cast<float*>(tile + (l & 31) * 8 + ((r / 4 * 2 + (l >> 5)) ^ (l & 7))) + r % 4; };
+    if (many_small(mask)) {
+        for (; mask; mask &= mask - 1) *at(lane, __builtin_ctz(mask)) = NAN;
+    } else {
+        for_each_small(mask, [&](int owner, int r) {
+            const float v = product(owner & 31, r / 4 * 8 + (owner >> 5) * 4 + r % 4);
+            if (lane == owner) *at(lane, r) = v;
+        });
+    }
+    __builtin_amdgcn_wave_barrier();
 }
 
 template <int EPI, bool DOWN>
@@ -132,7 +148,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
     request_x(0);
 
     f32x16 acc[NT], low[NT];                                             // (h,h); (l,h) and (h,l)
-    int e = 300;                                                         // exponent of the row's scale
+    int e = PAIRS_ZEROS_SO_FAR;                                          // exponent of the row's scale
     float scale = 0.f;
 #pragma unroll
     for (int j = 0; j < NT; ++j) acc[j] = low[j] = f32x16{0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
@@ -152,8 +168,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");               // read, so that the next step may come in its place
         if (step + 1 < steps) request_x(step + 1);
         const int above = exponent_above(largest_of_halves(fmaxf(largest(v[0]), largest(v[1]))));
-        if (__any(above + e > 15)) {                                     // first step, or 16 times larger than what had been seen
-            const int now = above + e > 15 ? min(11 - above, PAIRS_MOST_SCALE) : e;
+        if (__any(above + e > 15)) {                                     // first step, or 4 times larger than what had been seen
+            const int now = pairs_scale_after(above, e);
             const float factor = power_of_two(now - e);
             e = now, scale = power_of_two(now);
 #pragma unroll
@@ -189,7 +205,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
 #pragma unroll
             for (int q = 0; q < 4; ++q)
                 if (r0 + q * 8 < N && col < P) second[q].load(ep, r0 + q * 8, col, P);
-            f32x4 any = {0.f, 0.f, 0.f, 0.f};
+            float least = INFINITY;
             __builtin_amdgcn_wave_barrier();
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
@@ -197,15 +213,29 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
                 const int c[4] = {ew.x, ew.y, ew.z, ew.w};
                 f32x4 t;
 #pragma unroll
-                for (int u = 0; u < 4; ++u) t[u] = __builtin_amdgcn_ldexpf(fmaf(low[j][q * 4 + u], Pairs::LOW, acc[j][q * 4 + u]), -(e + c[u]));
-                any += t;
+                for (int u = 0; u < 4; ++u) {
+                    const float s = fmaf(low[j][q * 4 + u], Pairs::LOW, acc[j][q * 4 + u]);
+                    least = least_size(least, s);
+                    t[u] = __builtin_amdgcn_ldexpf(s, -(e + c[u]));
+                }
                 tile[l32 * 8 + ((q * 2 + half) ^ (l32 & 7))] = __builtin_bit_cast(u32x4, t);
             }
             __builtin_amdgcn_wave_barrier();
             f32x4 y[4];
 #pragma unroll
             for (int q = 0; q < 4; ++q) y[q] = __builtin_bit_cast(f32x4, tile[q * 64 + lane]);
-            if (__any(nan_among(any))) {
+            if (__any(nan_or_small(least, e))) {
+                uint32_t mask = 0;
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const int at = col0 + j * 32 + r / 4 * 8 + half * 4 + r % 4;
+                    if (fabsf(fmaf(low[j][r], Pairs::LOW, acc[j][r])) < PAIRS_SMALL && at < P && exps[at] <= PAIRS_MOST_SCALE) mask |= 1u << r;
+                }
+                if (e > PAIRS_MOST_SCALE || row0 + l32 >= N) mask = 0;
+                small_again(tile, mask, [&](int r32, int c32) {
+                    const int at = col0 + j * 32 + c32;
+                    return wave_product(x + (row0 + r32) * K, w + (DOWN ? at : (int64_t)at * K), DOWN ? P : 1, K);
+                });
 #pragma unroll 1
                 for (int q = 0; q < 4; ++q) {
                     f32x4 t = __builtin_bit_cast(f32x4, tile[q * 64 + lane]);
@@ -278,7 +308,7 @@ __global__ __launch_bounds__(HELD_WAVES * 64) __attribute__((amdgpu_waves_per_eu
         }
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) m = fmaxf(m, largest(v[ks]));
-        const int e = min(15 - exponent_above(largest_of_halves(m)), PAIRS_MOST_SCALE);
+        const int e = pairs_scale(exponent_above(largest_of_halves(m)));
         const float scale = power_of_two(e);
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) {
@@ -313,7 +343,7 @@ __global__ __launch_bounds__(HELD_WAVES * 64) __attribute__((amdgpu_waves_per_eu
         }
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) m = fmaxf(m, largest(v[ks]));
-        const int e = min(15 - exponent_above(largest_of_halves(m)), PAIRS_MOST_SCALE);
+        const int e = pairs_scale(exponent_above(largest_of_halves(m)));
         const float scale = power_of_two(e);
         u32x4 b[KS][2];
 #pragma unroll
@@ -341,7 +371,7 @@ __global__ __launch_bounds__(HELD_WAVES * 64) __attribute__((amdgpu_waves_per_eu
                 acc = Pairs::mfma(a[ks & 1][0], b[ks][0], acc);
                 low = Pairs::mfma(a[ks & 1][0], b[ks][1], low);
             }
-            f32x4 any = {0.f, 0.f, 0.f, 0.f};
+            float least = INFINITY;
             __builtin_amdgcn_wave_barrier();
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
@@ -351,12 +381,24 @@ __global__ __launch_bounds__(HELD_WAVES * 64) __attribute__((amdgpu_waves_per_eu
                 const int ec[4] = {ew.x, ew.y, ew.z, ew.w};
                 f32x4 s;
 #pragma unroll
-                for (int u = 0; u < 4; ++u) s[u] = __builtin_amdgcn_ldexpf(fmaf(low[q * 4 + u], Pairs::LOW, acc[q * 4 + u]), -(e + ec[u])) + add[u];
-                any += s;
+                for (int u = 0; u < 4; ++u) {
+                    const float p = fmaf(low[q * 4 + u], Pairs::LOW, acc[q * 4 + u]);
+                    least = least_size(least, p);
+                    s[u] = __builtin_amdgcn_ldexpf(p, -(e + ec[u])) + add[u];
+                }
                 tile[l32 * 8 + ((q * 2 + half) ^ (l32 & 7))] = __builtin_bit_cast(u32x4, s);
             }
             __builtin_amdgcn_wave_barrier();
-            if (__any(nan_among(any))) {
+            if (__any(nan_or_small(least, e))) {
+                uint32_t mask = 0;
+#pragma unroll
+                for (int r = 0; r < 16; ++r)
+                    if (fabsf(fmaf(low[r], Pairs::LOW, acc[r])) < PAIRS_SMALL && exps[c * 32 + r / 4 * 8 + half * 4 + r % 4] <= PAIRS_MOST_SCALE) mask |= 1u << r;
+                if (e > PAIRS_MOST_SCALE || t * 32 + l32 >= N) mask = 0;
+                small_again(tile, mask, [&](int r32, int c32) {
+                    const int at = col0 + c * 32 + c32;
+                    return wave_product(x + (t * 32 + r32) * K, w + (DOWN ? at : (int64_t)at * K), DOWN ? P : 1, K) + bias[c * 32 + c32];
+                });
 #pragma unroll 1
                 for (int q = 0; q < 4; ++q) {
                     f32x4 s = __builtin_bit_cast(f32x4, tile[q * 64 + lane]);

@@ -17,6 +17,8 @@
 // fp32 operands are pairs of fp16 (Pairs of dense_operand.hpp).  A scale per row of x, found when the row is loaded, and per row of A and
 // B, found by the launch that splits them; the hidden values' scale follows the largest of the token so far, and since a token's
 // results lie in its own lanes, dropping it is a product a register.
+// Small results are formed again (PAIRS_SMALL): hidden values where the wavefront's rows of x or any row of A have lost bits, which is
+// known before the first step (225 700 rows, inference 178 -> 184 us; looked for in every step 190), values of y always.
 //
 // Microseconds, two launches (of three bf16 pieces) and one.  225 700 rows fp32 96 channels: forward 339 and 267, inference 296 and 189, backward
 // 285 and 199 (with three pieces here 308, 227 and 245; traffic alone at copy rate 187 and 170 for the first and last).  Error against float64 (2-norms) of
@@ -64,8 +66,8 @@ __device__ __forceinline__ int hidden_of(int i) { return (i & 0x13) | (i & 4) <<
 
 template <typename T> constexpr int MLP_PL = sizeof(T) == 4 ? 2 : 1;     // planes of an operand
 
-// a wavefront's rows as operands; the exponent of the scale of the lane's row (fp32)
-template <typename T, int KS> __device__ __forceinline__ int load_rows(const T* p, u32x4 (&x)[KS][MLP_PL<T>]) {
+// a wavefront's rows as operands; the exponent of the scale of the lane's row (fp32), and whether the pieces lose bits of its part of it
+template <typename T, int KS> __device__ __forceinline__ int load_rows(const T* p, u32x4 (&x)[KS][MLP_PL<T>], bool& lost) {
     if constexpr (sizeof(T) == 4) {
         float v[KS][8], m = 0.f;
 #pragma unroll
@@ -76,8 +78,12 @@ template <typename T, int KS> __device__ __forceinline__ int load_rows(const T* 
         }
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) m = fmaxf(m, largest(v[ks]));
-        const int e = min(15 - exponent_above(largest_of_halves(m)), PAIRS_MOST_SCALE);
+        const int e = pairs_scale(exponent_above(largest_of_halves(m)));
         const float scale = power_of_two(e);
+        uint32_t least = 0xffffffffu;
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) least = least_nonzero(v[ks], least);
+        lost = pairs_lose(least, scale);
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) split_pairs(v[ks], scale, x[ks]);
         return e;
@@ -254,6 +260,51 @@ template <int D, int MODE> __device__ __forceinline__ void plain_rows(const MlpA
         for (int r = 0; r < 16; ++r) y[j][r] = y[j][r] == y[j][r] ? y[j][r] : p[j][r];
 }
 
+// The small ones among a tile's values (PAIRS_SMALL; register 8 s + e of half h is row 16 s + 8 h + e, the lane's token column), of scales ex and exps, from
+// product(token, row); true: they are many, and marked with NaN, which makes their tokens those of plain_rows.
+template <typename F> __device__ __forceinline__ bool small_again(f32x16& z, int ex, const int* exps, F product) {
+    const int lane = threadIdx.x & 63;
+    uint32_t mask = 0;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        const int ew = exps[r / 8 * 16 + (lane >> 5) * 8 + r % 8];
+        if (ew <= PAIRS_MOST_SCALE && fabsf(__builtin_amdgcn_ldexpf(z[r], ex + ew)) < PAIRS_SMALL) mask |= 1u << r;
+    }
+    if (ex > PAIRS_MOST_SCALE) mask = 0;
+    if (many_small(mask)) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) z[r] = mask >> r & 1 ? NAN : z[r];
+        return true;
+    }
+    for_each_small(mask, [&](int owner, int bit) {
+        const float v = product(owner & 31, bit / 8 * 16 + (owner >> 5) * 8 + bit % 8);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) z[r] = lane == owner && bit == r ? v : z[r];
+    });
+    return false;
+}
+// y of one token and column in plain fp32, without its bias, by the wavefront: from the hidden values in memory, or formed again
+template <int D, int MODE> __device__ __forceinline__ float one_output(const MlpArgs& g, int64_t row, int col, const float* bias) {
+    const float* const w = g.wb + (MODE == MLP_BACKWARD ? col : (int64_t)col * g.hidden);
+    if constexpr (MODE != MLP_INFER) return wave_product(static_cast<const float*>(g.h) + row * g.hidden, w, MODE == MLP_BACKWARD ? D : 1, g.hidden);
+    const float* const x = static_cast<const float*>(g.x) + row * D;
+    float y = 0.f;
+#pragma unroll 1
+    for (int k = threadIdx.x & 63; k < g.hidden; k += 64) {
+        const f32x4* const a = reinterpret_cast<const f32x4*>(g.wa + (int64_t)k * D);
+        float z = 0.f, act, slope;
+#pragma unroll 4
+        for (int i = 0; i < D / 4; ++i) {
+            const f32x4 v = a[i];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) z = fmaf(x[i * 4 + e], v[e], z);
+        }
+        gelu_and_slope<true>(z + bias[k], act, slope);
+        y = fmaf(act, w[k], y);
+    }
+    return wave_sum(y);
+}
+
 // A step is 32 hidden channels.  The wait for the next step's A and B leaves the stores of this step in flight; it counts them, so they
 // are inline assembly.
 template <typename T, int D, int MODE, int WAVES> struct MlpLds {
@@ -263,7 +314,8 @@ template <typename T, int D, int MODE, int WAVES> struct MlpLds {
     static constexpr bool SHARED = MODE == MLP_INFER && WAVES * 256 <= 2 * PIECES * 64;
     static constexpr int OWN = SHARED ? 0 : std::max(256, 2 * HiddenTile<T>::PIECES);
     static constexpr int PER_CHANNEL = sizeof(T) == 4 ? 2 : 1;           // its bias, and fp32 the exponent of its scale
-    static size_t bytes(int hidden) { return (size_t)2 * PIECES * 1024 + (size_t)(hidden + D) * 4 * PER_CHANNEL + (size_t)WAVES * OWN * 16; }
+    static constexpr int FLAGS = sizeof(T) == 4 ? (WAVES + 3) / 4 : 0;   // 16-byte pieces with one a wavefront
+    static size_t bytes(int hidden) { return (size_t)2 * PIECES * 1024 + (size_t)(hidden + D) * 4 * PER_CHANNEL + FLAGS * 16 + (size_t)WAVES * OWN * 16; }
 };
 template <typename T, typename TO, int D, int MODE, int WAVES, int OCC>
 __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(OCC, OCC))) void mlp_kernel(MlpArgs g) {
@@ -275,7 +327,8 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(OCC,
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, half = lane >> 5, l32 = lane & 31;
     float* const bias = reinterpret_cast<float*>(lds + 2 * PIECES * 64); // [hidden] and [D]
     int* const exps = reinterpret_cast<int*>(bias + g.hidden + D);       // fp32: the same
-    u32x4* const tiles = L::SHARED ? lds + wave * 256 : lds + 2 * PIECES * 64 + (g.hidden + D) * L::PER_CHANNEL / 4 + wave * L::OWN;
+    int* const lost_ab = exps + g.hidden + D;                            // fp32: whether a wavefront has seen rows of A (1) and B (2) that lose bits
+    u32x4* const tiles = L::SHARED ? lds + wave * 256 : lds + 2 * PIECES * 64 + (g.hidden + D) * L::PER_CHANNEL / 4 + L::FLAGS + wave * L::OWN;
     const int64_t behind = (int64_t)blockIdx.x - g.full, row0 = tile_row(behind < 0 ? (int64_t)blockIdx.x * WAVES + wave : g.full * WAVES + behind * g.some + wave, g.N);
     const int64_t plane = (int64_t)g.hidden * D;
     const uint32_t lane_a = (uint32_t)(hidden_of(l32) * D + half * 8);
@@ -294,10 +347,18 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(OCC,
     const int steps = g.hidden / 32;
     request(0);
     if constexpr (MODE != MLP_BACKWARD) stage_biases<T>(g, D, bias);
-    if constexpr (PL == 2)
-        for (int c = threadIdx.x; c < g.hidden + D; c += WAVES * 64) exps[c] = c < g.hidden ? g.ea[c] : g.eb[c - g.hidden];
+    if constexpr (PL == 2) {
+        bool seen_a = false, seen_b = false;
+        for (int c = threadIdx.x; c < g.hidden + D; c += WAVES * 64) {
+            const int e = c < g.hidden ? g.ea[c] : g.eb[c - g.hidden], cut = e >= PAIRS_LOST / 2 ? PAIRS_LOST : 0;
+            exps[c] = e - cut;
+            seen_a |= cut && c < g.hidden, seen_b |= cut && c >= g.hidden;
+        }
+        lost_ab[wave] = (__any(seen_a) ? 1 : 0) | (__any(seen_b) ? 2 : 0);
+    }
     if (behind >= 0 && wave >= g.some) {                                 // without tokens: only brings A and B
         wait_copies<0>();
+        if constexpr (PL == 2) block_barrier();
         for (int step = 0; step < steps; ++step) {
             block_barrier();
             if (step + 1 < steps) request(step + 1);
@@ -307,7 +368,8 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(OCC,
         return;
     }
     u32x4 x[KS][PL];
-    const int ex = load_rows<T, KS>(static_cast<const T*>(g.x) + (row0 + l32) * D + half * 8, x);
+    bool lost = false;
+    const int ex = load_rows<T, KS>(static_cast<const T*>(g.x) + (row0 + l32) * D + half * 8, x, lost);
     const int64_t mem = (row0 + H::mem_row()) * g.hidden + H::mem_col();
     auto load_tile = [&](int step) {                                     // of slope
 #pragma unroll
@@ -325,125 +387,161 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(OCC,
     f32x16 y[CT], y_low[PL == 2 ? CT : 1];
 #pragma unroll
     for (int j = 0; j < CT; ++j) y[j] = y_low[PL == 2 ? j : 0] = f32x16{0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-    int eh = 300;                                                        // fp32: exponent of the scale of the row's hidden values
+    int eh = PAIRS_ZEROS_SO_FAR;                                         // fp32: exponent of the scale of the row's hidden values
     float hidden_scale = 0.f;
     if constexpr (MODE == MLP_BACKWARD) load_tile(0);
     wait_copies<0>();
+    int ab = 0;
+    if constexpr (PL == 2) {
+        block_barrier();
+#pragma unroll
+        for (int w = 0; w < WAVES; ++w) ab |= lost_ab[w];
+        lost = __any(lost || (ab & 1));                                  // results of operands that lose no bits may be small
+    }
+    float least_hidden = INFINITY;
     if (PL == 2 && wave < WAVES / 2) __builtin_amdgcn_s_setprio(1);      // the two wavefronts of a SIMD at different places of a step
-    for (int step = 0; step < steps; ++step) {
-        block_barrier();                                                 // this buffer is there, the other one is free
-        if (step + 1 < steps) {
-            request(step + 1);
-            if constexpr (MODE == MLP_BACKWARD) load_tile(step + 1);
-        }
-        u32x4* const tile = tiles + (MODE == MLP_BACKWARD ? (step & 1) * H::PIECES : 0);   // du takes the place of its slope
-        const u32x4* const pieces = lds + (step & 1) * PIECES * 64 + lane;
-        // z^T: the pieces of A are read a slice of 16 channels ahead of its products
-        f32x16 z = f32x16{0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0}, z_low = z;
-        u32x4 a[2][PL];
-#pragma unroll
-        for (int q = 0; q < PL; ++q) a[0][q] = pieces[q * 64];
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-            if (ks + 1 < KS)
-#pragma unroll
-                for (int q = 0; q < PL; ++q) a[(ks + 1) & 1][q] = pieces[((ks + 1) * PL + q) * 64];
-            if constexpr (PL == 2) {
-                z_low = Pairs::mfma(a[ks & 1][1], x[ks][0], z_low);
-                z = Pairs::mfma(a[ks & 1][0], x[ks][0], z);
-                z_low = Pairs::mfma(a[ks & 1][0], x[ks][1], z_low);
-            } else {
-                z = Op<T>::mfma(a[ks & 1][0], x[ks][0], z);
+    // twice in the code, since a branch for small hidden values in the loop costs 3 % where there are none
+    auto run = [&](auto small) {
+        for (int step = 0; step < steps; ++step) {
+            block_barrier();                                                 // this buffer is there, the other one is free
+            if (step + 1 < steps) {
+                request(step + 1);
+                if constexpr (MODE == MLP_BACKWARD) load_tile(step + 1);
             }
-            __builtin_amdgcn_sched_group_barrier(0x100, PL, 0);
-            __builtin_amdgcn_sched_group_barrier(0x008, PL == 2 ? 3 : 1, 0);
-        }
-        if constexpr (PL == 2) {
+            u32x4* const tile = tiles + (MODE == MLP_BACKWARD ? (step & 1) * H::PIECES : 0);   // du takes the place of its slope
+            const u32x4* const pieces = lds + (step & 1) * PIECES * 64 + lane;
+            // z^T: the pieces of A are read a slice of 16 channels ahead of its products
+            f32x16 z = f32x16{0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0}, z_low = z;
+            u32x4 a[2][PL];
 #pragma unroll
-            for (int s = 0; s < 2; ++s) {
-                const int4* const e8 = reinterpret_cast<const int4*>(exps + step * 32 + s * 16 + half * 8);
-                const int4 lo = e8[0], hi = e8[1];
-                const int ew[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+            for (int q = 0; q < PL; ++q) a[0][q] = pieces[q * 64];
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                for (int e = 0; e < 8; ++e) z[s * 8 + e] = __builtin_amdgcn_ldexpf(fmaf(z_low[s * 8 + e], Pairs::LOW, z[s * 8 + e]), -(ex + ew[e]));
-            }
-        }
-        auto step_between = [&](int s, float (&v)[8]) {
-            float u[8];
-            between<T, MODE>(z, s, bias + step * 32, tile, v, u);
-            if constexpr (MODE != MLP_INFER) H::put(tile, s, v);
-            if constexpr (MODE == MLP_TRAIN) H::put(tile + H::PIECES, s, u);
-        };
-        auto second_layer = [&](int s, const u32x4 (&h)[PL]) {
-            u32x4 w[2][PL];
-            auto read = [&](int j) {
+            for (int ks = 0; ks < KS; ++ks) {
+                if (ks + 1 < KS)
 #pragma unroll
-                for (int q = 0; q < PL; ++q) w[j & 1][q] = pieces[(PA + (s * CT + j) * PL + q) * 64];
-            };
-            read(0);
-#pragma unroll
-            for (int j = 0; j < CT; ++j) {
-                if (j + 1 < CT) read(j + 1);
+                    for (int q = 0; q < PL; ++q) a[(ks + 1) & 1][q] = pieces[((ks + 1) * PL + q) * 64];
                 if constexpr (PL == 2) {
-                    y_low[j] = Pairs::mfma(w[j & 1][1], h[0], y_low[j]);
-                    y[j] = Pairs::mfma(w[j & 1][0], h[0], y[j]);
-                    y_low[j] = Pairs::mfma(w[j & 1][0], h[1], y_low[j]);
+                    z_low = Pairs::mfma(a[ks & 1][1], x[ks][0], z_low);
+                    z = Pairs::mfma(a[ks & 1][0], x[ks][0], z);
+                    z_low = Pairs::mfma(a[ks & 1][0], x[ks][1], z_low);
                 } else {
-                    y[j] = Op<T>::mfma(w[j & 1][0], h[0], y[j]);
+                    z = Op<T>::mfma(a[ks & 1][0], x[ks][0], z);
+                }
+                __builtin_amdgcn_sched_group_barrier(0x100, PL, 0);
+                __builtin_amdgcn_sched_group_barrier(0x008, PL == 2 ? 3 : 1, 0);
+            }
+            if constexpr (PL == 2) {
+#pragma unroll
+                for (int s = 0; s < 2; ++s) {
+                    const int4* const e8 = reinterpret_cast<const int4*>(exps + step * 32 + s * 16 + half * 8);
+                    const int4 lo = e8[0], hi = e8[1];
+                    const int ew[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) z[s * 8 + e] = __builtin_amdgcn_ldexpf(fmaf(z_low[s * 8 + e], Pairs::LOW, z[s * 8 + e]), -(ex + ew[e]));
+                }
+                if constexpr (decltype(small)::value)
+                    small_again(z, ex, exps + step * 32, [&](int l, int c) {
+                        const int k = step * 32 + c;
+                        return wave_product(static_cast<const float*>(g.x) + (row0 + l) * D, g.wa + (MODE == MLP_BACKWARD ? k : (int64_t)k * D),
+                                            MODE == MLP_BACKWARD ? g.hidden : 1, D);
+                    });
+            }
+            auto step_between = [&](int s, float (&v)[8]) {
+                float u[8];
+                between<T, MODE>(z, s, bias + step * 32, tile, v, u);
+                if constexpr (MODE != MLP_INFER) H::put(tile, s, v);
+                if constexpr (MODE == MLP_TRAIN) H::put(tile + H::PIECES, s, u);
+            };
+            auto second_layer = [&](int s, const u32x4 (&h)[PL]) {
+                u32x4 w[2][PL];
+                auto read = [&](int j) {
+#pragma unroll
+                    for (int q = 0; q < PL; ++q) w[j & 1][q] = pieces[(PA + (s * CT + j) * PL + q) * 64];
+                };
+                read(0);
+#pragma unroll
+                for (int j = 0; j < CT; ++j) {
+                    if (j + 1 < CT) read(j + 1);
+                    if constexpr (PL == 2) {
+                        y_low[j] = Pairs::mfma(w[j & 1][1], h[0], y_low[j]);
+                        y[j] = Pairs::mfma(w[j & 1][0], h[0], y[j]);
+                        y_low[j] = Pairs::mfma(w[j & 1][0], h[1], y_low[j]);
+                    } else {
+                        y[j] = Op<T>::mfma(w[j & 1][0], h[0], y[j]);
+                    }
+                }
+            };
+            u32x4 h[PL];
+            if constexpr (PL == 2) {
+                float v[2][8];
+                step_between(0, v[0]);
+                step_between(1, v[1]);
+                // the scale follows the largest value seen: where a step's would leave fp16's range it drops, and the sums with it
+                const int above = exponent_above(largest_of_halves(fmaxf(largest(v[0]), largest(v[1]))));
+                if constexpr (MODE == MLP_INFER)
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) least_hidden = least_size(least_hidden, v[e / 8][e % 8]);
+                if (__any(above + eh > 15)) {
+                    const int now = pairs_scale_after(above, eh);
+                    const float factor = power_of_two(now - eh);
+                    eh = now, hidden_scale = power_of_two(now);
+#pragma unroll
+                    for (int j = 0; j < CT; ++j)
+#pragma unroll
+                        for (int r = 0; r < 16; ++r) y[j][r] *= factor, y_low[j][r] *= factor;
+                }
+#pragma unroll
+                for (int s = 0; s < 2; ++s) {
+                    split_pairs(v[s], hidden_scale, h);
+                    second_layer(s, h);
+                }
+            } else {
+#pragma unroll
+                for (int s = 0; s < 2; ++s) {
+                    float v[8];
+                    step_between(s, v);
+                    planes_of<T>(v, h);
+                    second_layer(s, h);
                 }
             }
-        };
-        u32x4 h[PL];
-        if constexpr (PL == 2) {
-            float v[2][8];
-            step_between(0, v[0]);
-            step_between(1, v[1]);
-            // the scale follows the largest value seen: where a step's would leave fp16's range it drops, and the sums with it
-            const int above = exponent_above(largest_of_halves(fmaxf(largest(v[0]), largest(v[1]))));
-            if (__any(above + eh > 15)) {
-                const int now = above + eh > 15 ? min(11 - above, PAIRS_MOST_SCALE) : eh;
-                const float factor = power_of_two(now - eh);
-                eh = now, hidden_scale = power_of_two(now);
-#pragma unroll
-                for (int j = 0; j < CT; ++j)
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) y[j][r] *= factor, y_low[j][r] *= factor;
+            if constexpr (MODE != MLP_INFER) {
+                __builtin_amdgcn_wave_barrier();
+                store_tile(tile, g.h, step);
+                if constexpr (MODE == MLP_TRAIN) store_tile(tile + H::PIECES, g.slope, step);
+                __builtin_amdgcn_wave_barrier();
             }
-#pragma unroll
-            for (int s = 0; s < 2; ++s) {
-                split_pairs(v[s], hidden_scale, h);
-                second_layer(s, h);
-            }
-        } else {
-#pragma unroll
-            for (int s = 0; s < 2; ++s) {
-                float v[8];
-                step_between(s, v);
-                planes_of<T>(v, h);
-                second_layer(s, h);
-            }
+            if (step + 1 < steps) wait_copies<STORES>();                     // all but the stores of this step
         }
-        if constexpr (MODE != MLP_INFER) {
-            __builtin_amdgcn_wave_barrier();
-            store_tile(tile, g.h, step);
-            if constexpr (MODE == MLP_TRAIN) store_tile(tile + H::PIECES, g.slope, step);
-            __builtin_amdgcn_wave_barrier();
-        }
-        if (step + 1 < steps) wait_copies<STORES>();                     // all but the stores of this step
-    }
+    };
+    if (lost) run(std::true_type());
+    else run(std::false_type());
     if constexpr (L::SHARED) block_barrier();                    // A and B have been read
     if constexpr (PL == 2) {
-        f32x4 any = {0.f, 0.f, 0.f, 0.f};
+        float least = INFINITY;
 #pragma unroll
         for (int j = 0; j < CT; ++j)
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
                 const int ew = exps[g.hidden + j * 32 + r / 8 * 16 + half * 8 + r % 8];
-                y[j][r] = __builtin_amdgcn_ldexpf(fmaf(y_low[j][r], Pairs::LOW, y[j][r]), -(eh + ew));
-                any[r & 3] += y[j][r];
+                const float t = fmaf(y_low[j][r], Pairs::LOW, y[j][r]);
+                least = least_size(least, t);
+                y[j][r] = __builtin_amdgcn_ldexpf(t, -(eh + ew));
             }
-        if (__any(nan_among(any))) plain_rows<D, MODE>(g, row0, bias, tiles, y);
+        // Inference has no hidden values in memory, and forms 2500 to 60 000 again for a small result: only where one of them may have lost bits
+        bool look = nan_or_small(least, eh);
+        if constexpr (MODE == MLP_INFER) {
+            least_hidden = fminf(least_hidden, __shfl_xor(least_hidden, 32, 64));      // the token's others
+            look = look && (least != least || (ab & 2) || __builtin_amdgcn_ldexpf(least_hidden, eh) < 0x1p-13f);
+        }
+        if (__any(look)) {
+            wait_copies<0>();                                            // the hidden values stored by this wavefront are read
+            bool nan = __any(least != least);
+#pragma unroll
+            for (int j = 0; j < CT; ++j)
+                nan |= small_again(y[j], eh, exps + g.hidden + j * 32, [&](int l, int c) { return one_output<D, MODE>(g, row0 + l, j * 32 + c, bias); });
+            if (nan) plain_rows<D, MODE>(g, row0, bias, tiles, y);
+        }
     }
     store_y<TO, D, MODE>(g, y, row0, bias + g.hidden, tiles);
 }
@@ -571,7 +669,7 @@ __global__ __launch_bounds__(512) void mlp_pairs_kernel(const float* __restrict_
     const bool second = (int)blockIdx.x >= hidden / 32;
     const int tile = second ? (int)blockIdx.x - hidden / 32 : (int)blockIdx.x, rows = second ? D : hidden, cols = second ? hidden : D;
     uint16_t* const to = second ? b : a;
-    const int e = pairs_of_columns<TURNED, 8>(second ? wb : wa, cols, rows, tile, [&](int row, int ks, int half, const u32x4 (&p)[2]) {
+    const int e = pairs_of_columns<TURNED, 8, true>(second ? wb : wa, cols, rows, tile, [&](int row, int ks, int half, const u32x4 (&p)[2]) {
 #pragma unroll
         for (int q = 0; q < 2; ++q) *reinterpret_cast<u32x4*>(to + (int64_t)q * D * hidden + (int64_t)row * cols + ks * 16 + half * 8) = p[q];
     });

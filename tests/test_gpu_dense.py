@@ -553,6 +553,39 @@ def test_dense_fp32_pairs_scales(N, K, P, span):
         _check(y, x.double() @ wd.T, x.double().abs() @ wd.abs().T, torch.float32, f"transposed {transposed}")
 
 
+@pytest.mark.parametrize("span", [40, -40, 70])
+@pytest.mark.parametrize("N,K,P", PAIRS)
+def test_dense_fp32_pairs_scales_that_the_pieces_do_not_span(N, K, P, span):
+    """Every result is small against what its row and column hold: all of them formed again."""
+    test_dense_fp32_pairs_scales(N, K, P, span)
+
+
+@pytest.mark.parametrize("power", [30, 36, 48])
+@pytest.mark.parametrize("N,K,P", PAIRS)
+def test_dense_fp32_pairs_of_a_channel_above_the_rest(N, K, P, power):
+    """A channel 2^power above the others of its rows that meets zeros in some columns, whose results are those of the other channels: few
+    results of a tile (the rows of a tile but one, one column), many (a block of rows that all have it); a row and a column of zeros."""
+    from sparseswin3d_amd import _lib
+    lib = _lib.load()
+    gen = torch.Generator().manual_seed(K + P + power)
+    for transposed in (0, 1):
+        rows, cols = (P, K) if transposed else (K, P)             # of the reduction and the result
+        x, wt = torch.randn(N, rows, generator=gen), torch.randn(cols, rows, generator=gen)
+        c = rows - 5
+        x[7, c] = x[N // 2, c] = x[N - 1, c] = 2.0 ** power
+        x[64:128, c] = -2.0 ** power
+        x[9], wt[5] = 0, 0
+        wt[3, c] = wt[cols - 1, c] = 0
+        wt[cols // 2] *= 2.0 ** -power                            # one large weight in a column, met by zeros
+        wt[cols // 2, 1] = 1
+        x[N // 3:N // 3 + 3, 1] = 0
+        x, w = x.cuda(), (wt.T.contiguous() if transposed else wt).cuda()
+        wd = wt.double().cuda()
+        for extra in (None, torch.zeros(N, cols, device="cuda") if transposed == 0 else torch.ones(N, cols, device="cuda")):
+            y, _ = _forward(lib, _lib, x, w, None, transposed, PLAIN if extra is None else SCALE if transposed else RESIDUAL, extra, torch.float32)
+            _check(y, x.double() @ wd.T, x.double().abs() @ wd.abs().T, torch.float32, f"transposed {transposed}")
+
+
 # the last steps of 96 channels, on either side of the rows from which a workgroup takes 96 columns
 @pytest.mark.parametrize("N,K,P", [(6400, 96, 288), (13633, 96, 288), (21761, 288, 96), (41217, 96, 96)])
 def test_dense_fp32_pairs_of_96_channels(N, K, P):

@@ -206,6 +206,60 @@ def test_mlp_fp32_scales(N, hidden, span):
     _check(y, g64 @ w2.double().t(), g_err @ w2.double().abs().t() + 2e-6 * (g64.abs() @ w2.double().abs().t()) + 1e-30, "y")
 
 
+@pytest.mark.parametrize("span", [40, -40, 60])
+@pytest.mark.parametrize("N,hidden", [(33, 64), (3001, 384)])
+def test_mlp_fp32_scales_that_the_pieces_do_not_span(N, hidden, span):
+    test_mlp_fp32_scales(N, hidden, span)
+
+
+@pytest.mark.parametrize("power", [30, 40])
+@pytest.mark.parametrize("where", ["token", "tokens", "weight", "ramp"])
+@pytest.mark.parametrize("N,hidden", [(33, 64), (3001, 384)])
+def test_mlp_fp32_of_a_channel_above_the_rest(N, hidden, where, power):
+    """A channel of a token 2^power above its others, seen by one hidden channel alone, and that by all columns but some: hidden values and
+    results that are small against what their rows hold, in one token of a tile or in most.  A weight of a hidden channel as much above its others, met
+    by zeros in a few tokens; channels of a token that grow by as much and meet weights that fall, or fall and meet weights that grow."""
+    from sparseswin3d_amd import _lib
+    lib = _lib.load()
+    D, gen = 96, torch.Generator().manual_seed(N + power)
+    rand = lambda *s: torch.randn(*s, generator=gen)
+    x, wa, wb = rand(N, D), rand(hidden, D), rand(D, hidden)      # forward: w1 and w2, backward: w2^T and w1^T
+    if where == "weight":
+        wa[hidden - 7, 17] = 2.0 ** power
+        x[N // 2, 17] = x[5, 17] = 0
+    elif where == "ramp":
+        ramp = torch.exp2(torch.linspace(-power, power, D).round() * (1 if hidden == 64 else -1))
+        x, wa = x * ramp, wa / ramp
+    else:
+        x[0 if where == "tokens" else N // 2:N - 3 if where == "tokens" else N // 2 + 1, 17] = 2.0 ** power
+        wa[:, 17], wa[hidden - 7, 17] = 0, 1
+    wb[::5, hidden - 7] = 0
+    wa[11], wb[20], x[N - 1] = 0, 0, 0
+    slope = (rand(N, hidden) * 0.5 + 0.5).cuda()
+    x, wa, wb = x.cuda(), wa.cuda(), wb.cuda()
+    z64, mag = x.double() @ wa.double().t(), x.double().abs() @ wa.double().abs().t()
+    g64, s64 = _gelu(z64)
+    g_err = 2e-6 * mag + 1e-6 * g64.abs().clamp(max=1)
+    y_err = g_err @ wb.double().abs().t() + 2e-6 * (g64.abs() @ wb.double().abs().t()) + 1e-30
+    ws, nb = _workspace(lib, x, hidden, 0)
+    for train in (False, True):
+        y, act, slope_out = _empty((N, D), torch.float32), _empty((N, hidden), torch.float32), _empty((N, hidden), torch.float32)
+        _lib.check(lib.sswin_mlp_forward(0, 0, _ptr(x), N, D, hidden, _ptr(wa), None, _ptr(wb), None, None, _ptr(y), _ptr(act) if train else None,
+                                         _ptr(slope_out) if train else None, _ptr(ws), nb, _stream()))
+        _check(y, g64 @ wb.double().t(), y_err, f"y, training {train}")
+    _check(act, g64, g_err + 1e-30, "act")
+    _check(slope_out, s64, 2e-6 * mag + 1e-6, "slope")
+    du64 = z64 * slope.double()
+    du_err = 2e-6 * mag * slope.double().abs()
+    dx_err = du_err @ wb.double().abs().t() + 2e-6 * (du64.abs() @ wb.double().abs().t())
+    w2, w1 = wa.t().contiguous(), wb.t().contiguous()
+    du, dx = _empty((N, hidden), torch.float32), _empty((N, D), torch.float32)
+    ws, nb = _workspace(lib, x, hidden, 1)
+    _lib.check(lib.sswin_mlp_backward(0, _ptr(x), N, D, hidden, _ptr(w1), _ptr(w2), _ptr(slope), _ptr(du), _ptr(dx), _ptr(ws), nb, _stream()))
+    _check(du, du64, du_err + 1e-30, "du")
+    _check(dx, du64 @ wb.double().t(), dx_err + 1e-30, "dx")
+
+
 def _same_class(got, ref, bound, what):
     """Finite where float64 is (to the bound), the same infinities, NaN where float64 has NaN."""
     got, finite = got.double(), ref.isfinite()
