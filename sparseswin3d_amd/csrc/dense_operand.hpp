@@ -246,6 +246,11 @@ __device__ __forceinline__ float wave_sum(float v) {
 // the smaller of |a| and |b|, NaN where one is; whether results of a row whose scale's exponent is e, the least of them as it left the products, are NaN
 // or small
 __device__ __forceinline__ float least_size(float a, float b) { return __builtin_elementwise_minimum(fabsf(a), fabsf(b)); }
+__device__ __forceinline__ float wave_least(float v) {
+#pragma unroll
+    for (int m = 32; m; m >>= 1) v = least_size(v, __shfl_xor(v, m, 64));
+    return v;
+}
 __device__ __forceinline__ bool nan_or_small(float least, int e) { return e <= PAIRS_MOST_SCALE ? !(least >= PAIRS_SMALL) : least != least; }
 // sum over i < n of a[i] b[i b_step], by a wavefront (a, b uniform), to all its lanes
 __device__ __forceinline__ float wave_product(const float* a, const float* b, int64_t b_step, int n) {

@@ -20,8 +20,8 @@
 // Small results are formed again (PAIRS_SMALL): hidden values where the wavefront's rows of x or any row of A have lost bits, which is
 // known before the first step (225 700 rows, inference 178 -> 184 us; looked for in every step 190), values of y always.
 //
-// Microseconds, two launches (of three bf16 pieces) and one.  225 700 rows fp32 96 channels: forward 339 and 267, inference 296 and 189, backward
-// 285 and 199 (with three pieces here 308, 227 and 245; traffic alone at copy rate 187 and 170 for the first and last).  Error against float64 (2-norms) of
+// Microseconds, two launches (of three bf16 pieces) and one.  225 700 rows fp32 96 channels: forward 339 and 264, inference 296 and 184, backward
+// 285 and 200 (with three pieces here 308, 227 and 245; traffic alone at copy rate 187 and 170 for the first and last).  Error against float64 (2-norms) of
 // y 1.0e-7, three pieces 1.8e-7, of dx 1.9e-7 and 3.4e-7.  What bounds fp32 now: the stores of training, GELU on the vector units (about 26
 // instructions of 45 a hidden value) and the products, of which two wavefronts a SIMD cover two thirds with each other.
 // fp16 48 channels, 225 000 rows: 89 and 69, 55 and 43 (55 and 38).  bf16 96 channels, inference, 112 700 rows: 65 and 45 (13; GELU on
@@ -195,7 +195,7 @@ template <typename T> __device__ __forceinline__ void stage_biases(const MlpArgs
 }
 // fp32: y where the pieces left NaN, again in plain fp32 as in dense.hip (plain_products), and the hidden values before it with what is
 // stored of them.  A hidden value that came out NaN makes every y of its token NaN, so y alone tells, once a launch.  Inference has
-// no hidden values in memory and forms all of these tokens again.
+// no hidden values in memory and forms all of these tokens again; so does training for y, for the same bits.
 template <int D, int MODE> __device__ __forceinline__ void plain_rows(const MlpArgs& g, int64_t row0, const float* bias, u32x4* tile, f32x16 (&y)[(D + 31) / 32]) {
     constexpr int CT = (D + 31) / 32;
     using H = HiddenTile<float>;
@@ -213,7 +213,8 @@ template <int D, int MODE> __device__ __forceinline__ void plain_rows(const MlpA
             f32x4* const stored = reinterpret_cast<f32x4*>(static_cast<float*>(g.h) + row * g.hidden + k);
             f32x4 v;
             if (MODE != MLP_INFER) v = *stored;
-            if (MODE == MLP_INFER || nan_among(v)) {
+            const bool nan = MODE != MLP_INFER && nan_among(v);
+            if (MODE != MLP_BACKWARD || nan) {
                 const float* const x = static_cast<const float*>(g.x) + row * D;
                 f32x4 u;
                 if constexpr (MODE == MLP_BACKWARD) {
@@ -230,8 +231,8 @@ template <int D, int MODE> __device__ __forceinline__ void plain_rows(const MlpA
                         v[e] = act, u[e] = slope;
                     }
                 }
-                if (MODE != MLP_INFER) *stored = v;
-                if (MODE == MLP_TRAIN) *reinterpret_cast<f32x4*>(static_cast<float*>(g.slope) + row * g.hidden + k) = u;
+                if (nan) *stored = v;
+                if (MODE == MLP_TRAIN && nan) *reinterpret_cast<f32x4*>(static_cast<float*>(g.slope) + row * g.hidden + k) = u;
             }
             tile[H::slot(l32, half * 4 + c)] = __builtin_bit_cast(u32x4, v);
         }
@@ -283,10 +284,10 @@ template <typename F> __device__ __forceinline__ bool small_again(f32x16& z, int
     });
     return false;
 }
-// y of one token and column in plain fp32, without its bias, by the wavefront: from the hidden values in memory, or formed again
+// y of one token and column in plain fp32, without its bias, by the wavefront: from du in memory, or from hidden values formed again
 template <int D, int MODE> __device__ __forceinline__ float one_output(const MlpArgs& g, int64_t row, int col, const float* bias) {
     const float* const w = g.wb + (MODE == MLP_BACKWARD ? col : (int64_t)col * g.hidden);
-    if constexpr (MODE != MLP_INFER) return wave_product(static_cast<const float*>(g.h) + row * g.hidden, w, MODE == MLP_BACKWARD ? D : 1, g.hidden);
+    if constexpr (MODE == MLP_BACKWARD) return wave_product(static_cast<const float*>(g.h) + row * g.hidden, w, D, g.hidden);
     const float* const x = static_cast<const float*>(g.x) + row * D;
     float y = 0.f;
 #pragma unroll 1
@@ -528,18 +529,28 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(OCC,
                 least = least_size(least, t);
                 y[j][r] = __builtin_amdgcn_ldexpf(t, -(eh + ew));
             }
-        // Inference has no hidden values in memory, and forms 2500 to 60 000 again for a small result: only where one of them may have lost bits
-        bool look = nan_or_small(least, eh);
-        if constexpr (MODE == MLP_INFER) {
-            least_hidden = fminf(least_hidden, __shfl_xor(least_hidden, 32, 64));      // the token's others
-            look = look && (least != least || (ab & 2) || __builtin_amdgcn_ldexpf(least_hidden, eh) < 0x1p-13f);
-        }
-        if (__any(look)) {
+        bool small = nan_or_small(least, eh);
+        if (__any(small)) {
             wait_copies<0>();                                            // the hidden values stored by this wavefront are read
+            // In inference a value of y takes its hidden values again, 13 us: only where one of them, or of B, has lost bits.  The same in training,
+            // so that both give the same bits.
+            if constexpr (MODE != MLP_BACKWARD) {
+                if constexpr (MODE == MLP_INFER) least_hidden = fminf(least_hidden, __shfl_xor(least_hidden, 32, 64));      // the token's others
+                else
+                    for_each_small(small ? 1u : 0u, [&](int owner, int) {
+                        const float* const h = static_cast<const float*>(g.h) + (row0 + (owner & 31)) * g.hidden;
+                        float m = INFINITY;
+                        for (int k = lane; k < g.hidden; k += 64) m = least_size(m, h[k]);
+                        m = wave_least(m);
+                        if (lane == owner) least_hidden = m;
+                    });
+                small = small && ((ab & 2) || __builtin_amdgcn_ldexpf(least_hidden, eh) < 0x1p-13f);
+            }
             bool nan = __any(least != least);
 #pragma unroll
             for (int j = 0; j < CT; ++j)
-                nan |= small_again(y[j], eh, exps + g.hidden + j * 32, [&](int l, int c) { return one_output<D, MODE>(g, row0 + l, j * 32 + c, bias); });
+                nan |= small_again(y[j], small ? eh : PAIRS_ZEROS, exps + g.hidden + j * 32,
+                                   [&](int l, int c) { return one_output<D, MODE>(g, row0 + l, j * 32 + c, bias); });
             if (nan) plain_rows<D, MODE>(g, row0, bias, tiles, y);
         }
     }
@@ -754,7 +765,7 @@ int sswin_mlp_supported(int dtype, int64_t N, int D, int hidden) {
 // time grows with the hidden channels, that of the two layers' tiles with all of their work, so with more than 384 later (bf16 96 channels,
 // forward and backward, 768 hidden: 20 000 rows 66 -> 76, 50 000 114 -> 91; 1024 hidden 8192 57 -> 91, 50 000 142 -> 121).  fp32: a
 // wavefront takes about 44 us forward and 30 backward alone on its SIMD, so from three wavefronts a compute unit on (forward and
-// backward of 8192 rows 60 -> 80 us, 16 384 88 -> 89, as three bf16 pieces; 24 576 101 -> 76, 225 700 633 -> 466), and only behind the rows up to
+// backward of 8192 rows 60 -> 80 us, 16 384 88 -> 89, as three bf16 pieces; 24 576 101 -> 78, 225 700 633 -> 464), and only behind the rows up to
 // which the second layer is one of few rows.
 int sswin_mlp_preferred(int dtype, int64_t N, int D, int hidden) {
     if (!sswin_mlp_supported(dtype, N, D, hidden)) return 0;

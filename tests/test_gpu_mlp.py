@@ -206,6 +206,29 @@ def test_mlp_fp32_scales(N, hidden, span):
     _check(y, g64 @ w2.double().t(), g_err @ w2.double().abs().t() + 2e-6 * (g64.abs() @ w2.double().abs().t()) + 1e-30, "y")
 
 
+def test_mlp_fp32_inference_has_the_bits_of_training():
+    """Rows enough for results that are small by chance, with and without weights that lose bits."""
+    from sparseswin3d_amd import _lib
+    lib = _lib.load()
+    N, D, hidden, gen = 100003, 96, 384, torch.Generator(device="cuda").manual_seed(3)
+    rand = lambda *s: torch.randn(*s, generator=gen, device="cuda")
+    x, w1, w2, b1, b2, res = rand(N, D), rand(hidden, D) * D ** -0.5, rand(D, hidden) * hidden ** -0.5, rand(hidden) * 0.1, rand(D) * 0.1, rand(N, D)
+    ws, nb = _workspace(lib, x, hidden, 0)
+    for k in range(3):
+        if k == 1:
+            w2[5, 7] = w1[9, 3] = 1e-12
+        elif k == 2:
+            b1[11] = 1e7                                          # a hidden channel above the rest, so that the others lose bits
+            w2[:, 11] *= 1e-7
+        ys = []
+        for train in (False, True):
+            y, act, slope = _empty((N, D), torch.float32), _empty((N, hidden), torch.float32), _empty((N, hidden), torch.float32)
+            _lib.check(lib.sswin_mlp_forward(0, 0, _ptr(x), N, D, hidden, _ptr(w1), _ptr(b1), _ptr(w2), _ptr(b2), _ptr(res), _ptr(y), _ptr(act) if train else None,
+                                             _ptr(slope) if train else None, _ptr(ws), nb, _stream()))
+            ys.append(y)
+        assert torch.equal(*ys), k
+
+
 @pytest.mark.parametrize("span", [40, -40, 60])
 @pytest.mark.parametrize("N,hidden", [(33, 64), (3001, 384)])
 def test_mlp_fp32_scales_that_the_pieces_do_not_span(N, hidden, span):
@@ -242,11 +265,14 @@ def test_mlp_fp32_of_a_channel_above_the_rest(N, hidden, where, power):
     g_err = 2e-6 * mag + 1e-6 * g64.abs().clamp(max=1)
     y_err = g_err @ wb.double().abs().t() + 2e-6 * (g64.abs() @ wb.double().abs().t()) + 1e-30
     ws, nb = _workspace(lib, x, hidden, 0)
+    ys = []
     for train in (False, True):
         y, act, slope_out = _empty((N, D), torch.float32), _empty((N, hidden), torch.float32), _empty((N, hidden), torch.float32)
         _lib.check(lib.sswin_mlp_forward(0, 0, _ptr(x), N, D, hidden, _ptr(wa), None, _ptr(wb), None, None, _ptr(y), _ptr(act) if train else None,
                                          _ptr(slope_out) if train else None, _ptr(ws), nb, _stream()))
         _check(y, g64 @ wb.double().t(), y_err, f"y, training {train}")
+        ys.append(y)
+    assert torch.equal(*ys)                                       # inference has the bits of training
     _check(act, g64, g_err + 1e-30, "act")
     _check(slope_out, s64, 2e-6 * mag + 1e-6, "slope")
     du64 = z64 * slope.double()
