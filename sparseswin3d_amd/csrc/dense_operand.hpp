@@ -111,7 +111,7 @@ constexpr float PAIRS_SMALL = 64.f;
 // exponent E with |v| < 2^E; of zero far below that of any value.  (Infinities and NaN: 0.)
 __device__ __forceinline__ int exponent_above(float most) { return most == 0.f ? -200 : __builtin_amdgcn_frexp_expf(most); }
 // Exponent of the scale of a row whose largest value lies below 2^above.  Scales stay normal numbers; exponents above PAIRS_MOST_SCALE
-// say that the row (so far) is all zeros.
+// say that the row (so far) is all zeros; its scale is 2^PAIRS_MOST_SCALE or 0, never infinite, which would turn the zeros into NaN.
 constexpr int PAIRS_MOST_SCALE = 120, PAIRS_ZEROS = 121, PAIRS_ZEROS_SO_FAR = 200;
 __device__ __forceinline__ int pairs_scale(int above) { return above == -200 ? PAIRS_ZEROS : min(15 - above, PAIRS_MOST_SCALE); }
 // The same where it follows the largest value: from e on to a step whose values lie below 2^above (above + e > 15: they would leave fp16's range)

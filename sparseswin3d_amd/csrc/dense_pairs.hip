@@ -94,11 +94,13 @@ __global__ __launch_bounds__(DOWN ? 1024 : 256) void pairs_weights_kernel(const 
 }
 
 // The results of a wavefront's tile of 32 x 32 whose bits are set in `mask` (of lane l, register r: row l % 32, column 8 (r / 4) + 4 (l / 32) + r % 4)
-// from product(row, column), or marked with NaN if they are many
-template <typename F> __device__ __forceinline__ void small_again(u32x4* tile, uint32_t mask, F product) {
+// from product(row, column); true: they are many, and marked with NaN instead
+template <typename F> __device__ __forceinline__ bool small_again(u32x4* tile, uint32_t mask, F product) {
     const int lane = threadIdx.x & 63;
+    if (!__any(mask)) return false;
     auto at = [&](int l, int r) { return reinterpret_cast<float*>(tile + (l & 31) * 8 + ((r / 4 * 2 + (l >> 5)) ^ (l & 7))) + r % 4; };
-    if (many_small(mask)) {
+    const bool many = many_small(mask);
+    if (many) {
         for (; mask; mask &= mask - 1) *at(lane, __builtin_ctz(mask)) = NAN;
     } else {
         for_each_small(mask, [&](int owner, int r) {
@@ -107,6 +109,7 @@ template <typename F> __device__ __forceinline__ void small_again(u32x4* tile, u
         });
     }
     __builtin_amdgcn_wave_barrier();
+    return many;
 }
 
 template <int EPI, bool DOWN>
@@ -171,7 +174,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
         if (__any(above + e > 15)) {                                     // first step, or 4 times larger than what had been seen
             const int now = pairs_scale_after(above, e);
             const float factor = power_of_two(now - e);
-            e = now, scale = power_of_two(now);
+            e = now, scale = power_of_two(min(now, PAIRS_MOST_SCALE));     // (rows of zeros so far too)
 #pragma unroll
             for (int j = 0; j < NT; ++j)
 #pragma unroll
@@ -232,18 +235,20 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
                     if (fabsf(fmaf(low[j][r], Pairs::LOW, acc[j][r])) < PAIRS_SMALL && at < P && exps[at] <= PAIRS_MOST_SCALE) mask |= 1u << r;
                 }
                 if (e > PAIRS_MOST_SCALE || row0 + l32 >= N) mask = 0;
-                small_again(tile, mask, [&](int r32, int c32) {
+                const bool many = small_again(tile, mask, [&](int r32, int c32) {
                     const int at = col0 + j * 32 + c32;
                     return wave_product(x + (row0 + r32) * K, w + (DOWN ? at : (int64_t)at * K), DOWN ? P : 1, K);
                 });
+                if (__any(least != least) || many) {
 #pragma unroll 1
-                for (int q = 0; q < 4; ++q) {
-                    f32x4 t = __builtin_bit_cast(f32x4, tile[q * 64 + lane]);
-                    if (r0 + q * 8 < N && col < P && nan_among(t))
-                        t = plain_products(x + (r0 + q * 8) * K, 1, w + (DOWN ? col : (int64_t)col * K), DOWN ? P : 1, DOWN ? 1 : K, K);
-                    tile[q * 64 + lane] = __builtin_bit_cast(u32x4, t);
+                    for (int q = 0; q < 4; ++q) {
+                        f32x4 t = __builtin_bit_cast(f32x4, tile[q * 64 + lane]);
+                        if (r0 + q * 8 < N && col < P && nan_among(t))
+                            t = plain_products(x + (r0 + q * 8) * K, 1, w + (DOWN ? col : (int64_t)col * K), DOWN ? P : 1, DOWN ? 1 : K, K);
+                        tile[q * 64 + lane] = __builtin_bit_cast(u32x4, t);
+                    }
+                    __builtin_amdgcn_wave_barrier();
                 }
-                __builtin_amdgcn_wave_barrier();
 #pragma unroll
                 for (int q = 0; q < 4; ++q) y[q] = __builtin_bit_cast(f32x4, tile[q * 64 + lane]);
             }
@@ -259,8 +264,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
 // largest value and it is split once for all of the columns.  Bound by the traffic, and by what a launch takes until its pieces are there (5 us).
 // The loops over the columns are unrolled: with a count the compiler does not know it waits for all stores where the next rows are used (CT = 9 in a
 // loop 42 us where three workgroups of 96 columns take 39; unrolled, 36 registers are spilled and 50).
-// Three bf16 pieces before, microseconds: 112 700 rows 96 -> 288 44.2 and 39.0, 96 -> 96 21.1 and 18.8 (turned 21.1 and 18.6), 20 000 rows 96 -> 288 12.6 and 12.4,
-// 96 -> 96 10.2 and 7.6; 225 700 rows 96 -> 288 87.3 and 86.6.  Error against float64 (2-norms) 1.13e-7 and 0.81e-7, turned 1.50e-7 and 1.04e-7.
+// Three bf16 pieces before, microseconds: 112 700 rows 96 -> 288 44.2 and 41.0, 96 -> 96 21.1 and 19.3 (turned 21.1 and 20.1), 225 700 rows 96 -> 288 87.3 and
+// 87.5; with other rows and weights in each call 50 000 rows 96 -> 288 33.8 and 28.5, 96 -> 96 15.2 and 14.5 (turned 15.2 and 15.7), 20 000 rows 14.2 and 13.8,
+// 10.6 and 8.3 (turned 10.8 and 8.9).  Behind a plan, where clocks and caches are cold, the launches of 20 000 rows take 17.2 and 9.4.
+// Error against float64 (2-norms) 1.13e-7 and 0.81e-7, turned 1.50e-7 and 1.04e-7.  Not ahead: W's columns dealt to all wavefronts 16 channels at a time, their
+// maxima through LDS (6400 rows 96 -> 288 8.2 -> 8.5, 20 000 13.6 -> 14.5, 51 200 28.7 -> 29.7).
 // ------------------------------------------------------------------------------------------
 constexpr int HELD_K = 96, HELD_KS = HELD_K / 16, HELD_WAVES = 8;
 template <int EPI, bool DOWN, int CT>
@@ -395,19 +403,21 @@ __global__ __launch_bounds__(HELD_WAVES * 64) __attribute__((amdgpu_waves_per_eu
                 for (int r = 0; r < 16; ++r)
                     if (fabsf(fmaf(low[r], Pairs::LOW, acc[r])) < PAIRS_SMALL && exps[c * 32 + r / 4 * 8 + half * 4 + r % 4] <= PAIRS_MOST_SCALE) mask |= 1u << r;
                 if (e > PAIRS_MOST_SCALE || t * 32 + l32 >= N) mask = 0;
-                small_again(tile, mask, [&](int r32, int c32) {
+                const bool many = small_again(tile, mask, [&](int r32, int c32) {
                     const int at = col0 + c * 32 + c32;
                     return wave_product(x + (t * 32 + r32) * K, w + (DOWN ? at : (int64_t)at * K), DOWN ? P : 1, K) + bias[c * 32 + c32];
                 });
+                if (__any(least != least) || many) {
 #pragma unroll 1
-                for (int q = 0; q < 4; ++q) {
-                    f32x4 s = __builtin_bit_cast(f32x4, tile[q * 64 + lane]);
-                    if (r0 + q * 8 < N && nan_among(s))
-                        s = plain_products(x + (r0 + q * 8) * K, 1, w + (DOWN ? col : (int64_t)col * K), DOWN ? P : 1, DOWN ? 1 : K, K) +
-                            *reinterpret_cast<const f32x4*>(bias + (col - col0));
-                    tile[q * 64 + lane] = __builtin_bit_cast(u32x4, s);
+                    for (int q = 0; q < 4; ++q) {
+                        f32x4 s = __builtin_bit_cast(f32x4, tile[q * 64 + lane]);
+                        if (r0 + q * 8 < N && nan_among(s))
+                            s = plain_products(x + (r0 + q * 8) * K, 1, w + (DOWN ? col : (int64_t)col * K), DOWN ? P : 1, DOWN ? 1 : K, K) +
+                                *reinterpret_cast<const f32x4*>(bias + (col - col0));
+                        tile[q * 64 + lane] = __builtin_bit_cast(u32x4, s);
+                    }
+                    __builtin_amdgcn_wave_barrier();
                 }
-                __builtin_amdgcn_wave_barrier();
             }
 #pragma unroll
             for (int q = 0; q < 4; ++q)
@@ -446,8 +456,9 @@ template <int EPI, bool DOWN, int CT> static int launch_held(const float* x, int
 // rows, and in front of them there are no registers for it (112 700 rows 96 -> 96 with a residual: 21.2 us there, 23.3 here, in front 32).
 template <int EPI, bool DOWN> bool pairs_held(const float* x, int64_t N, const float* w, int P, const Epilogue& ep, hipStream_t s, int& rc) {
     const int64_t workgroups = (N + HELD_WAVES * 32 - 1) / (HELD_WAVES * 32) * (P / 96);   // of 96 columns
-    // few of them: 32 columns (7000 rows 96 -> 288, 84 workgroups: 10.1 us with 96 columns, 8.0 with 32; 36 000 96 -> 96, 141: 12.4 and 11.1; 28 000 96 -> 192,
-    // 220: 11.2 and 12.9)
+    // few of them: 32 columns.  With 32 and with 96, other rows and weights in each call: 84 workgroups (7000 rows 96 -> 288) 8.3 and 11.1 us, 120 11.2 and 11.6,
+    // 141 (36 000 rows 96 -> 96) 12.0 and 12.7, 160 (10 000 rows 96 -> 384) 11.8 and 12.0; 172 (22 000 rows 96 -> 192) 14.3 and 12.4, 196 15.3 and 13.1, 237
+    // 16.0 and 13.8
     const bool few = workgroups * 8 <= device_cus() * 5;
     if (Second4<float, float, EPI>::USED && !few) return false;
     if constexpr (Second4<float, float, EPI>::USED) rc = launch_held<EPI, DOWN, 1>(x, N, w, P, ep, s);

@@ -272,6 +272,7 @@ template <typename F> __device__ __forceinline__ bool small_again(f32x16& z, int
         if (ew <= PAIRS_MOST_SCALE && fabsf(__builtin_amdgcn_ldexpf(z[r], ex + ew)) < PAIRS_SMALL) mask |= 1u << r;
     }
     if (ex > PAIRS_MOST_SCALE) mask = 0;
+    if (!__any(mask)) return false;
     if (many_small(mask)) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) z[r] = mask >> r & 1 ? NAN : z[r];
@@ -486,7 +487,7 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(OCC,
                 if (__any(above + eh > 15)) {
                     const int now = pairs_scale_after(above, eh);
                     const float factor = power_of_two(now - eh);
-                    eh = now, hidden_scale = power_of_two(now);
+                    eh = now, hidden_scale = power_of_two(min(now, PAIRS_MOST_SCALE));
 #pragma unroll
                     for (int j = 0; j < CT; ++j)
 #pragma unroll

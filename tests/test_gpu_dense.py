@@ -586,6 +586,20 @@ def test_dense_fp32_pairs_of_a_channel_above_the_rest(N, K, P, power):
             _check(y, x.double() @ wd.T, x.double().abs() @ wd.abs().T, torch.float32, f"transposed {transposed}")
 
 
+@pytest.mark.parametrize("N,K,P", [(20001, 208, 304), (30001, 288, 96), (30001, 96, 288)])
+def test_dense_fp32_pairs_rows_that_begin_with_zeros(N, K, P):
+    """A row's results have the same bits whatever stands in the rows beside it: zeros at the beginning of every row or of some."""
+    from sparseswin3d_amd import _lib
+    lib = _lib.load()
+    gen = torch.Generator(device="cuda").manual_seed(K)
+    x, w = torch.randn(N, K, generator=gen, device="cuda"), torch.randn(P, K, generator=gen, device="cuda")
+    some, every = x.clone(), x
+    some[::3, :K // 2] = 0
+    every[:, :K // 2] = 0
+    a, b = (_forward(lib, _lib, t, w, None, 0, PLAIN, None, torch.float32)[0] for t in (some, every))
+    assert torch.equal(a[::3], b[::3])
+
+
 # the last steps of 96 channels, on either side of the rows from which a workgroup takes 96 columns
 @pytest.mark.parametrize("N,K,P", [(6400, 96, 288), (13633, 96, 288), (21761, 288, 96), (41217, 96, 96)])
 def test_dense_fp32_pairs_of_96_channels(N, K, P):

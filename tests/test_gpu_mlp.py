@@ -206,6 +206,25 @@ def test_mlp_fp32_scales(N, hidden, span):
     _check(y, g64 @ w2.double().t(), g_err @ w2.double().abs().t() + 2e-6 * (g64.abs() @ w2.double().abs().t()) + 1e-30, "y")
 
 
+def test_mlp_fp32_hidden_values_that_begin_with_zeros():
+    """A token's results have the same bits whatever stands beside it: zeros in the first hidden values of every token or of some."""
+    from sparseswin3d_amd import _lib
+    lib = _lib.load()
+    N, D, hidden, gen = 3001, 96, 384, torch.Generator(device="cuda").manual_seed(4)
+    rand = lambda *s: torch.randn(*s, generator=gen, device="cuda")
+    dy, w1, w2, slope = rand(N, D), rand(hidden, D), rand(D, hidden), rand(N, hidden)
+    some, every = slope.clone(), slope
+    some[::3, :100] = 0
+    every[:, :100] = 0
+    ws, nb = _workspace(lib, dy, hidden, 1)
+    dxs = []
+    for t in (some, every):
+        du, dx = _empty((N, hidden), torch.float32), _empty((N, D), torch.float32)
+        _lib.check(lib.sswin_mlp_backward(0, _ptr(dy), N, D, hidden, _ptr(w1), _ptr(w2), _ptr(t), _ptr(du), _ptr(dx), _ptr(ws), nb, _stream()))
+        dxs.append(dx[::3])
+    assert torch.equal(*dxs)
+
+
 def test_mlp_fp32_inference_has_the_bits_of_training():
     """Rows enough for results that are small by chance, with and without weights that lose bits."""
     from sparseswin3d_amd import _lib
