@@ -597,22 +597,24 @@ def kernel_table(wl, reps=20, only=None):
     # ---- the flash kernels (what the step runs for heads of 16, and for heads of 32 in windows of more than 128 positions) ----
     fl_entries = []
     if ti is not None and F.attention_path(hd, b["n"], ti) == "flash":
-        words = torch.empty(2 * N, dtype=torch.int32, device=dev)
+        n_order = lib.sswin_flash_order_ints(N, H)
+        words = torch.empty(2 * N + n_order, dtype=torch.int32, device=dev)
+        tok_sq, order = C.c_void_p(words.data_ptr() + 4 * N), C.c_void_p(words.data_ptr() + 8 * N) if n_order else None
         table_fl = wl["blocks"][0]["attn"].relative_position_bias_table.detach().float().contiguous()
         delta = torch.empty(H * N, device=dev)
 
         def fl_tokens():
-            _lib.check(lib.sswin_flash_tokens(ptr(tp.plan), tp.g_cap, tp.G, ptr(tp.tokens), N, H, b["n"], ptr(ti.code), mask_p, nmw, ptr(words),
-                                              C.c_void_p(words.data_ptr() + 4 * N), stream))
+            _lib.check(lib.sswin_flash_tokens_ordered(ptr(tp.plan), tp.g_cap, tp.G, ptr(tp.tokens), N, H, b["n"], ptr(ti.code), mask_p, nmw, ptr(words),
+                                                      tok_sq, order, stream))
 
         def fl_fwd():
-            _lib.check(lib.sswin_flash_forward(code, ptr(tp.tokens), ptr(words), N, H, hd, b["n"], ptr(qkv_r), C.c_float(0.17), ptr(table_fl), n_table,
-                                               ti.offset0, ptr(out_r), ptr(lse), stream))
+            _lib.check(lib.sswin_flash_forward_ordered(code, ptr(tp.tokens), ptr(words), order, N, H, hd, b["n"], ptr(qkv_r), C.c_float(0.17), ptr(table_fl),
+                                                       n_table, ti.offset0, ptr(out_r), ptr(lse), stream))
 
         def fl_bwd():
-            _lib.check(lib.sswin_flash_backward(code, ptr(tp.tokens), ptr(words), C.c_void_p(words.data_ptr() + 4 * N), N, H, hd, b["n"], ptr(qkv_r),
-                                                C.c_float(0.17), ptr(table_fl), n_table, ti.offset0, ptr(out_r), ptr(lse), ptr(up_r), ptr(dqkv_r),
-                                                ptr(delta), ptr(ds_r), stream))
+            _lib.check(lib.sswin_flash_backward_ordered(code, ptr(tp.tokens), ptr(words), tok_sq, order, N, H, hd, b["n"], ptr(qkv_r), C.c_float(0.17),
+                                                        ptr(table_fl), n_table, ti.offset0, ptr(out_r), ptr(lse), ptr(up_r), ptr(dqkv_r), ptr(delta), ptr(ds_r),
+                                                        stream))
 
         fl_tokens()
         fl_fwd()                                  # lse and out_r must hold a real forward for the backward timings
@@ -742,12 +744,25 @@ def stage_entries(wl):
 
 
 def projection_entries(wl):
-    """The qkv and proj nn.Linear of one attention call (fp32 on the bf16 matrix cores with split
-    operands), and the library GEMMs they replace (calls = 0)."""
+    """The qkv and proj nn.Linear of one attention call (fp32 on the matrix cores with split operands, through the entry points
+    that the modules call), and the library GEMMs they replace (calls = 0)."""
+    from sparseswin3d_amd import _lib
     from sparseswin3d_amd import window_attention as wa
+    lib = _lib.load()
     N, D = wl["N"], wl["dim"]
     dev = wl["feats"].device
     x = torch.randn(N, D, device=dev)
+    ptr = lambda t: None if t is None else C.c_void_p(t.data_ptr())
+
+    def dense(t, w, b, transposed):
+        """t [N, K] -> t w^T + b, or t w; result and workspace from the allocator, as in a module."""
+        K, P = w.shape if transposed else (w.shape[1], w.shape[0])
+        y, nb = torch.empty(N, P, device=dev), lib.sswin_dense_forward_workspace_bytes(0, N, K, P)
+        ws = torch.empty(nb, dtype=torch.uint8, device=dev) if nb else None
+        _lib.check(lib.sswin_dense_forward(0, 0, transposed, 0, ptr(t), N, K, ptr(w), ptr(b), P, None, ptr(y), None, ptr(ws), nb,
+                                           C.c_void_p(torch.cuda.current_stream().cuda_stream)))
+        return y
+
     entries = []
     for name, P in (("qkv", 3 * D), ("proj", D)):
         w = torch.randn(P, D, device=dev) * 0.1
@@ -755,11 +770,10 @@ def projection_entries(wl):
         dy = torch.randn(N, P, device=dev)
         io = 4 * N * (D + P)
         # what the module runs: this library's kernels where they take the shape (calls = 1), else the library GEMM
-        own_f = wa._split_linear_forward(x, w, b) is not None
+        own_f = own_x = bool(lib.sswin_dense_supported(0, P, D))
         own_w = wa._split_linear_weight_grad(dy, x, True)[0] is not None
-        own_x = wa._split_linear_input_grad(dy, w) is not None
         if own_f:
-            entries.append((f"{name} forward", (lambda w=w, b=b: wa._split_linear_forward(x, w, b)), io + 4 * P * D, 1))
+            entries.append((f"{name} forward", (lambda w=w, b=b: dense(x, w, b, 0)), io + 4 * P * D, 1))
         if own_w:
             entries.append((f"{name} weight+bias gradient", (lambda dy=dy: wa._split_linear_weight_grad(dy, x, True)), io + 4 * P * D, 1))
         def lib_dx(dy=dy, w=w):
@@ -767,7 +781,7 @@ def projection_entries(wl):
                 return dy @ w
 
         if own_x:
-            entries.append((f"{name} input gradient", (lambda dy=dy, w=w: wa._split_linear_input_grad(dy, w)), io + 4 * P * D, 1))
+            entries.append((f"{name} input gradient", (lambda dy=dy, w=w: dense(dy, w, None, 1)), io + 4 * P * D, 1))
 
         def lib_fwd(w=w, b=b):
             with wa._rocblas_gemm():
