@@ -435,7 +435,8 @@ int sswin_tall_linear_forward(const float* x, int64_t N, int K, const float* w, 
 
 /* dx[N,K] = dy[N,P] w[P,K]: input gradient of the same layers (autograd of nn.Linear,
  * swin3d_base.py:606-610).  fp32, P and K multiples of 96 (sswin_tall_linear_input_grad_supported
- * tells); same split-operand arithmetic as the forward.  dy 16-byte aligned.  Asynchronous. */
+ * tells).  Split operands as in the forward, except with P = 96, at least 32 rows and a dx that is 16-byte aligned and not dy: two
+ * fp16 pieces a value, as in sswin_dense_forward (results differ by a rounding).  dy 16-byte aligned.  Asynchronous. */
 int sswin_tall_linear_input_grad_supported(int P, int K);
 int sswin_tall_linear_input_grad(const float* dy, int64_t N, int P, const float* w, int K, float* dx,
                                  void* stream);

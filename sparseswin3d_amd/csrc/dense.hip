@@ -1082,6 +1082,8 @@ static int launch_forward(const void* x, int64_t N, int K, const void* w, int P,
         }
         // fp16 pairs, from the reductions on whose sums come out as exactly: error against float64 (2-norms) with 96 channels 7.8e-8 and
         // 1.0e-7 here, 144 1.1e-7 and 1.75e-7 (turned); 48 channels of three bf16 pieces 6.9e-8, of pairs 7.1e-8 and more
+        // The launch for W costs up to 2 us where tiles and reduction are few (three pieces and pairs, us): 9563 rows 112 -> 192 11.0 and 12.4, 4187 rows 144 -> 576
+        // 12.5 and 13.6, 32 700 rows 144 -> 48 turned 13.3 and 14.0, 16 300 rows 192 -> 192 15.0 and 15.4; from 288 reduction channels on pairs are ahead everywhere.
         if (apart && pairs_takes(K) && ws_bytes >= pairs_workspace_bytes(K, P)) return pairs_layer<EPI, DOWN>(xp, N, K, wp, P, ep, ws, s);
         // wavefronts per SIMD: what the registers allow without spilling (four: forward equal, input gradient 89 us against 40)
         return launch_rows<EPI, DOWN, 4, 1, 3>(xp, N, K, wp, P, ep, s);
@@ -1091,8 +1093,10 @@ static int launch_forward(const void* x, int64_t N, int K, const void* w, int P,
         // long reductions into many columns: fewest bytes through LDS (8119 rows, 768 -> 3072: 57 us against 70 with the next two)
         if (K >= 384 && P % 192 == 0 && rows * (P / 192) >= 512) return launch_rows16<T, TO, EPI, DOWN, 64, 2, 2, 1, 2, 2, 2>(xp, N, K, wp, P, 1, ws, ep, s);
         // one workgroup a compute unit and a long reduction: three blocks on their way instead of one, since nothing else hides a block's
-        // way from L2 (inside a backbone, weights not in L2: 7888 rows 1536 -> 384 28.2 us, now 20.8, five blocks of LDS 22.0; 1364 rows 768 -> 768 17.1 and
-        // 14.5; 7888 rows 384 -> 384 13.5 either way, again and again on one input 9.3 and 9.6)
+        // way from L2 (five blocks of LDS where this has four: 7888 rows 1536 -> 384 22.0 us and 20.8).  bf16, other rows and weights in each call, with one
+        // block and with three: 1364 rows 768 -> 768 14.7 and 11.6, 4000 rows 15.4 and 12.5, 8000 rows 768 -> 384 15.5 and 12.7, 7888 rows 1536 -> 384 28.2 and
+        // 21.8, 700 rows 1536 -> 1536 21.4 and 18.7, 3000 rows 1024 -> 512 18.0 and 13.8.  With more tiles than compute units it loses: 7000 rows
+        // 784 -> 400 (275) 19.9 and 25.0, 1364 rows 768 -> 3072 (352) 21.6 and 27.2.
         if (tiles <= device_cus() && K >= 768) return launch_rows16<T, TO, EPI, DOWN, 64, 4, 1, 2, 1, 4, 2>(xp, N, K, wp, P, cut.ksplit, ws, ep, s);
         // up to two workgroups a compute unit: eight wavefronts each (8119 rows, 1536 -> 384: 22 us against 30), above that five
         // workgroups of four, whose loads and stores overlap (219 000 rows, 96 -> 288: 44 us against 80)

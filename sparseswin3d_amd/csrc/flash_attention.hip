@@ -116,7 +116,7 @@ struct Args {
 // size, 1 to 22 steps, and the four wavefronts of a workgroup hold their place until the last is done: taken by their ranks, 61 to 69 %
 // of the places are in use, by descending work 89 to 97 % (simulated on the rooms of 112 700 and 225 700 voxels; 69 % measured).
 // 112 700 voxels fp32: forward 62.8 -> 56.0 us, key side 126.9 -> 117.3, dQ 42.9 either way (by rank behind an ordered key side 45.9); 225 700 fp16: forward
-// 89.4 -> 79.5, key side 182 -> 180.  The launch for the words takes 7.2 and 10.3 us with the order, 5.0 and 5.5 without.
+// 89.4 -> 79.5, key side 182 -> 180.  The launch for the words takes 6.4 and 9.1 us with the order, 4.2 and 4.4 without.
 // The work is summed over the windows (their table is short; 7055 chunks of the token rows take one workgroup 40 us): a step of 16 tokens of the window counts
 // two, three with a second sub-tile, a block two more; windows of less than 32 tokens, which share blocks, count by their tokens.
 __device__ __forceinline__ void order_chunks(const int32_t* __restrict__ plan, int64_t g_cap, int64_t windows, int H, int64_t N, int32_t* __restrict__ work) {
@@ -918,7 +918,10 @@ int sswin_flash_supported(int dtype, int64_t N, int H, int hd, int rows) {
            N * 3 * H * hd < (1ll << 32);
 }
 
-// Below, all wavefronts find a place at once (three a SIMD), and above, one workgroup is a while about it and the last places weigh little
+// Below, all wavefronts find a place at once (three a SIMD), and above, one workgroup is a while about it and the last places weigh little.
+// Words, forward and backward by rank and ordered, us (windows of 7^3, heads of 16; chunks x heads): fp32 1032 77 and 77, 1944 104 and 104, 2040 100 and 91,
+// 2964 115 and 111; 3462 147 and 141, 3966 165 and 148, 5940 185 and 157, 6978 188 and 168, 10 569 226 and 209, 13 968 400 and 356, 21 165 483 and 471;
+// fp16 1032 64 and 66, 1944 84 and 84, 2040 80 and 75, 2964 93 and 91; 3462 115 and 112, 3966 129 and 118, 5940 146 and 124, 10 569 173 and 161, 21 165 366 and 360.
 size_t sswin_flash_order_ints(int64_t N, int H) {
     const int64_t chunks = (N + 31) / 32;
     return chunks <= ORDER_MOST && chunks * H > 12 * (int64_t)device_cus() ? (size_t)chunks : 0;

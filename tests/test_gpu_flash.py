@@ -160,13 +160,14 @@ def test_flash_keeps_what_is_not_finite_where_it_belongs(which, value, hd, dtype
 # chunks of 32 tokens: one, some threads without any, several a thread, the most an order holds; windows that fill, span and share
 # chunks; more windows than an order takes, which leaves the chunks as they are
 @pytest.mark.parametrize("N,sizes", [(1, "all"), (32, "all"), (33, "all"), (1000, "all"), (34001, "all"), (12288 * 32, "all"), (40000, "small")])
-def test_flash_order_of_the_work(N, sizes):
+@pytest.mark.parametrize("H", [1, 3])
+def test_flash_order_of_the_work(N, sizes, H):
     """The order holds every chunk once, by descending work, and results have the bits they have without one."""
     import ctypes as C
     from sparseswin3d_amd import _lib
     from sparseswin3d_amd.fused import BiasTableIndex, TokenPlan
     from sparseswin3d_amd.window_attention import relative_position_index_3d
-    lib, H, n = _lib.load(), 1, 343
+    lib, n = _lib.load(), 343
     rng = np.random.default_rng(N)
     counts, left = [], N
     while left:
@@ -178,12 +179,13 @@ def test_flash_order_of_the_work(N, sizes):
     plan._finish()
     ptr = lambda t: C.c_void_p(t.data_ptr())
     stream = C.c_void_p(torch.cuda.current_stream().cuda_stream)
-    qkv, d_o, table = torch.randn(N, 48).cuda(), torch.randn(N, 16).cuda(), torch.randn(2197, H).cuda()
+    D = 16 * H
+    qkv, d_o, table = torch.randn(N, 3 * D).cuda(), torch.randn(N, D).cuda(), torch.randn(2197, H).cuda()
     chunks, got = (N + 31) // 32, []
-    assert lib.sswin_flash_order_ints(N, 3) == (chunks if 3 * chunks > 12 * torch.cuda.get_device_properties(0).multi_processor_count else 0)
+    assert lib.sswin_flash_order_ints(N, H) == (chunks if H * chunks > 12 * torch.cuda.get_device_properties(0).multi_processor_count else 0)
     for order in (None, torch.full((chunks,), -1, dtype=torch.int32, device="cuda")):
         words = torch.empty(2 * N, dtype=torch.int32, device="cuda")
-        out, lse, d_qkv, delta = torch.empty(N, 16).cuda(), torch.empty(H, N).cuda(), torch.empty(N, 48).cuda(), torch.empty(H, N).cuda()
+        out, lse, d_qkv, delta = torch.empty(N, D).cuda(), torch.empty(H, N).cuda(), torch.empty(N, 3 * D).cuda(), torch.empty(H, N).cuda()
         d_s, o, sq = torch.empty(max(plan.A, 1)).cuda(), None if order is None else ptr(order), C.c_void_p(words.data_ptr() + 4 * N)
         _lib.check(lib.sswin_flash_tokens_ordered(ptr(plan.plan), plan.g_cap, plan.G, ptr(plan.tokens), N, H, n, ptr(ti.code), None, 0, ptr(words), sq, o, stream))
         _lib.check(lib.sswin_flash_forward_ordered(0, ptr(plan.tokens), ptr(words), o, N, H, 16, n, ptr(qkv), 0.25, ptr(table), 2197, ti.offset0, ptr(out), ptr(lse),
