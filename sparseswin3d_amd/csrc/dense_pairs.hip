@@ -266,7 +266,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
 // loop 42 us where three workgroups of 96 columns take 39; unrolled, 36 registers are spilled and 50).
 // Three bf16 pieces before, microseconds: 112 700 rows 96 -> 288 44.2 and 41.0, 96 -> 96 21.1 and 19.3 (turned 21.1 and 20.1), 225 700 rows 96 -> 288 87.3 and
 // 87.5; with other rows and weights in each call 50 000 rows 96 -> 288 33.8 and 28.5, 96 -> 96 15.2 and 14.5 (turned 15.2 and 15.7), 20 000 rows 14.2 and 13.8,
-// 10.6 and 8.3 (turned 10.8 and 8.9).  Behind a plan, where clocks and caches are cold, the launches of 20 000 rows take 17.2 and 9.4.
+// 10.6 and 8.3 (turned 10.8 and 8.9).  Inside an attention module, where rows and weights come from memory, the launches of 20 000 rows take 17.0 and 9.3 (before 26.0 together).
 // Error against float64 (2-norms) 1.13e-7 and 0.81e-7, turned 1.50e-7 and 1.04e-7.  Not ahead: W's columns dealt to all wavefronts 16 channels at a time, their
 // maxima through LDS (6400 rows 96 -> 288 8.2 -> 8.5, 20 000 13.6 -> 14.5, 51 200 28.7 -> 29.7).
 // ------------------------------------------------------------------------------------------

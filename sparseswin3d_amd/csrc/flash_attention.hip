@@ -116,7 +116,7 @@ struct Args {
 // size, 1 to 22 steps, and the four wavefronts of a workgroup hold their place until the last is done: taken by their ranks, 61 to 69 %
 // of the places are in use, by descending work 89 to 97 % (simulated on the rooms of 112 700 and 225 700 voxels; 69 % measured).
 // 112 700 voxels fp32: forward 62.8 -> 56.0 us, key side 126.9 -> 117.3, dQ 42.9 either way (by rank behind an ordered key side 45.9); 225 700 fp16: forward
-// 89.4 -> 79.5, key side 182 -> 180.  The launch for the words takes 6.4 and 9.1 us with the order, 4.2 and 4.4 without.
+// 89.4 -> 79.5, key side 182 -> 180.  The launch for the words takes 6.4 and 9.1 us with the order, 4.2 and 4.4 without (alone; inside a module 7.4 and 10).
 // The work is summed over the windows (their table is short; 7055 chunks of the token rows take one workgroup 40 us): a step of 16 tokens of the window counts
 // two, three with a second sub-tile, a block two more; windows of less than 32 tokens, which share blocks, count by their tokens.
 __device__ __forceinline__ void order_chunks(const int32_t* __restrict__ plan, int64_t g_cap, int64_t windows, int H, int64_t N, int32_t* __restrict__ work) {
