@@ -597,32 +597,59 @@ def kernel_table(wl, reps=20, only=None):
     # ---- the flash kernels (what the step runs for heads of 16, and for heads of 32 in windows of more than 128 positions) ----
     fl_entries = []
     if ti is not None and F.attention_path(hd, b["n"], ti) == "flash":
-        n_order = lib.sswin_flash_order_ints(N, H)
-        words = torch.empty(2 * N + n_order, dtype=torch.int32, device=dev)
-        tok_sq, order = C.c_void_p(words.data_ptr() + 4 * N), C.c_void_p(words.data_ptr() + 8 * N) if n_order else None
         table_fl = wl["blocks"][0]["attn"].relative_position_bias_table.detach().float().contiguous()
-        delta = torch.empty(H * N, device=dev)
+        n_list = lib.sswin_flash_window_list_ints(code, N, H, hd, b["n"], n_table, tp.G // H)
+        if n_list:
+            # a wavefront a window and head; the bias-table gradient is summed in the backward's launch
+            words = torch.empty(N + n_list, dtype=torch.int32, device=dev)
+            work = C.c_void_p(words.data_ptr() + 4 * N)
+            d_table = torch.empty_like(table_fl)
+            fl_bytes = lib.sswin_flash_window_backward_workspace_bytes(N, H, n_table, tp.G // H)
+            fl_ws = torch.empty(fl_bytes, dtype=torch.uint8, device=dev)
+            groups = (ptr(tp.plan), tp.g_cap, tp.G, ptr(tp.tokens))
 
-        def fl_tokens():
-            _lib.check(lib.sswin_flash_tokens_ordered(ptr(tp.plan), tp.g_cap, tp.G, ptr(tp.tokens), N, H, b["n"], ptr(ti.code), mask_p, nmw, ptr(words),
-                                                      tok_sq, order, stream))
+            def fl_tokens():
+                _lib.check(lib.sswin_flash_window_tokens(*groups, N, H, b["n"], ptr(ti.code), mask_p, nmw, ptr(words), work, stream))
 
-        def fl_fwd():
-            _lib.check(lib.sswin_flash_forward_ordered(code, ptr(tp.tokens), ptr(words), order, N, H, hd, b["n"], ptr(qkv_r), C.c_float(0.17), ptr(table_fl),
-                                                       n_table, ti.offset0, ptr(out_r), ptr(lse), stream))
+            def fl_fwd():
+                _lib.check(lib.sswin_flash_window_forward(code, *groups, ptr(words), work, N, H, hd, b["n"], ptr(qkv_r), C.c_float(0.17), ptr(table_fl), n_table,
+                                                          ti.offset0, ptr(out_r), ptr(lse), stream))
 
-        def fl_bwd():
-            _lib.check(lib.sswin_flash_backward_ordered(code, ptr(tp.tokens), ptr(words), tok_sq, order, N, H, hd, b["n"], ptr(qkv_r), C.c_float(0.17),
-                                                        ptr(table_fl), n_table, ti.offset0, ptr(out_r), ptr(lse), ptr(up_r), ptr(dqkv_r), ptr(delta), ptr(ds_r),
-                                                        stream))
+            def fl_bwd():
+                _lib.check(lib.sswin_flash_window_backward(code, *groups, ptr(words), work, N, H, hd, b["n"], ptr(qkv_r), C.c_float(0.17), ptr(table_fl), n_table,
+                                                           ti.offset0, ptr(out_r), ptr(lse), ptr(up_r), ptr(dqkv_r), ptr(d_table), ptr(fl_ws), fl_bytes, stream))
+
+            backward_row = ("flash backward (dQ,dK,dV,dS summed by table row; three launches)", fl_bwd, 32 * Er + 4 * H * N, 1, 10 * A * hd)
+            more_rows = []
+        else:
+            n_order = lib.sswin_flash_order_ints(N, H)
+            words = torch.empty(2 * N + n_order, dtype=torch.int32, device=dev)
+            tok_sq, order = C.c_void_p(words.data_ptr() + 4 * N), C.c_void_p(words.data_ptr() + 8 * N) if n_order else None
+            delta = torch.empty(H * N, device=dev)
+
+            def fl_tokens():
+                _lib.check(lib.sswin_flash_tokens_ordered(ptr(tp.plan), tp.g_cap, tp.G, ptr(tp.tokens), N, H, b["n"], ptr(ti.code), mask_p, nmw, ptr(words),
+                                                          tok_sq, order, stream))
+
+            def fl_fwd():
+                _lib.check(lib.sswin_flash_forward_ordered(code, ptr(tp.tokens), ptr(words), order, N, H, hd, b["n"], ptr(qkv_r), C.c_float(0.17), ptr(table_fl),
+                                                           n_table, ti.offset0, ptr(out_r), ptr(lse), stream))
+
+            def fl_bwd():
+                _lib.check(lib.sswin_flash_backward_ordered(code, ptr(tp.tokens), ptr(words), tok_sq, order, N, H, hd, b["n"], ptr(qkv_r), C.c_float(0.17),
+                                                            ptr(table_fl), n_table, ti.offset0, ptr(out_r), ptr(lse), ptr(up_r), ptr(dqkv_r), ptr(delta),
+                                                            ptr(ds_r), stream))
+
+            backward_row = ("flash backward (dQ,dK,dV,dS; two launches)", fl_bwd, 32 * Er + 4 * A + 4 * H * N, 1, 10 * A * hd)
+            more_rows = [("flash bias table grad", r_table_grad, 4 * A, 1)]
 
         fl_tokens()
         fl_fwd()                                  # lse and out_r must hold a real forward for the backward timings
         fl_entries = [
             ("flash token words", fl_tokens, 28 * N, 1),
             ("flash forward", fl_fwd, 16 * Er + 4 * H * N, 1, 4 * A * hd),
-            ("flash backward (dQ,dK,dV,dS; two launches)", fl_bwd, 32 * Er + 4 * A + 4 * H * N, 1, 10 * A * hd),
-            ("flash bias table grad", r_table_grad, 4 * A, 1),
+            backward_row,
+            *more_rows,
         ]
 
     def measure(items, path):
@@ -946,10 +973,10 @@ def trace_summary(dirs, out_name, command):
         if not paths:
             sys.exit(f"no *kernel_stats.csv under {d}")
         rows = list(csv.DictReader(open(paths[0])))
-        # one backward launch per attention call: the resident kernels', the flash kernels' key side or, on the fused path, the
+        # one backward launch per attention call: the resident kernels', the flash kernels' (or their key side) or, on the fused path, the
         # score gradient's
         bwd = sum(int(r["Calls"]) for r in rows if "_bwd_all_kernel" in r["Name"]) or \
-            sum(int(r["Calls"]) for r in rows if "flash_backward_kv_kernel" in r["Name"]) or \
+            sum(int(r["Calls"]) for r in rows if "flash_backward_kv_kernel" in r["Name"] or "flash_window_backward_kernel" in r["Name"]) or \
             sum(int(r["Calls"]) for r in rows if "fused_sq_kernel<" in r["Name"] and ", 2>" in r["Name"])
         steps = max(bwd // 2, 1)
         if bwd == 0:                                 # the forward-only encoder: four attention launches per pass

@@ -524,6 +524,22 @@ int sswin_flash_backward_ordered(int dtype, const int32_t* tokens, const int32_t
                                  int hd, int n, const void* qkv, float scale, const float* table, int rows, int offset0, const void* out,
                                  const float* lse, const void* dout, void* dqkv, float* delta, float* ds, void* stream);
 
+/* The same attention for heads of 16 channels in windows of at most 384 positions, a wavefront per (window, head) and up to 96 tokens, with the
+ * gradient of the bias table in the backward's launch.  sswin_flash_window_list_ints: size of `list` (int32), 0 where a shape is not taken (then
+ * sswin_flash_* above).  plan, g_cap, groups: the token plan's group table.  sswin_flash_window_tokens writes word [N] (not that of sswin_flash_tokens)
+ * and list, to which the forward adds what its backward needs; d_table fp32 [rows, H] or null. */
+size_t sswin_flash_window_list_ints(int dtype, int64_t N, int H, int hd, int n, int rows, int64_t windows);
+int sswin_flash_window_tokens(const int32_t* plan, int64_t g_cap, int64_t groups, const int32_t* tokens, int64_t N, int H, int n, const int32_t* code,
+                              const int8_t* mask, int nmw, int32_t* word, int32_t* list, void* stream);
+int sswin_flash_window_forward(int dtype, const int32_t* plan, int64_t g_cap, int64_t groups, const int32_t* tokens, const int32_t* word,
+                               int32_t* list, int64_t N, int H, int hd, int n, const void* qkv, float scale, const float* table, int rows,
+                               int offset0, void* out, float* lse, void* stream);
+size_t sswin_flash_window_backward_workspace_bytes(int64_t N, int H, int rows, int64_t windows);
+int sswin_flash_window_backward(int dtype, const int32_t* plan, int64_t g_cap, int64_t groups, const int32_t* tokens, const int32_t* word,
+                                const int32_t* list, int64_t N, int H, int hd, int n, const void* qkv, float scale, const float* table, int rows,
+                                int offset0, const void* out, const float* lse, const void* dout, void* dqkv, float* d_table, void* ws,
+                                size_t ws_bytes, void* stream);
+
 /* nn.LayerNorm over rows of D values (swin3d_base.py:706, 722).  x of x_dtype; y of y_dtype (x_dtype, or a 16-bit type for
  * fp32 x); gamma, beta fp32 for fp32 x, else of x_dtype.  stats: fp32 [2][N] mean and reciprocal deviation for the backward, or
  * null.  sswin_layer_norm_supported: rows of whole 16-byte pieces, at most 8 x 64 of them.

@@ -102,6 +102,12 @@ SIGNATURES = {
     "sswin_flash_forward": (_i32, [_i32, _vp, _vp, _i64, _i32, _i32, _i32, _vp, C.c_float, _vp, _i32, _i32, _vp, _vp, _vp]),
     "sswin_flash_backward": (_i32, [_i32, _vp, _vp, _vp, _i64, _i32, _i32, _i32, _vp, C.c_float, _vp, _i32, _i32, _vp, _vp, _vp, _vp, _vp,
                                     _vp, _vp]),
+    "sswin_flash_window_list_ints": (_sz, [_i32, _i64, _i32, _i32, _i32, _i32, _i64]),
+    "sswin_flash_window_tokens": (_i32, [_vp, _i64, _i64, _vp, _i64, _i32, _i32, _vp, _vp, _i32, _vp, _vp, _vp]),
+    "sswin_flash_window_forward": (_i32, [_i32, _vp, _i64, _i64, _vp, _vp, _vp, _i64, _i32, _i32, _i32, _vp, C.c_float, _vp, _i32, _i32, _vp, _vp, _vp]),
+    "sswin_flash_window_backward_workspace_bytes": (_sz, [_i64, _i32, _i32, _i64]),
+    "sswin_flash_window_backward": (_i32, [_i32, _vp, _i64, _i64, _vp, _vp, _vp, _i64, _i32, _i32, _i32, _vp, C.c_float, _vp, _i32, _i32, _vp, _vp, _vp, _vp, _vp, _vp,
+                                           _sz, _vp]),
     "sswin_flash_order_ints": (_sz, [_i64, _i32]),
     "sswin_flash_tokens_ordered": (_i32, [_vp, _i64, _i64, _vp, _i64, _i32, _i32, _vp, _vp, _i32, _vp, _vp, _vp, _vp]),
     "sswin_flash_forward_ordered": (_i32, [_i32, _vp, _vp, _vp, _i64, _i32, _i32, _i32, _vp, C.c_float, _vp, _i32, _i32, _vp, _vp, _vp]),
@@ -131,7 +137,7 @@ SIGNATURES = {
                                                _vp, _i64, _i32, _vp, _i64, _i32, _vp, _i64, _i32, _vp, _i32, _vp]),
 }
 
-ABI_VERSION = 34
+ABI_VERSION = 35
 _lib = None
 
 # A list turns on timing of the library's launches: every call that takes a stream is bracketed by events on that

@@ -16,7 +16,7 @@ CSRC = os.path.join(HERE, "csrc")
 OUT = os.path.join(HERE, "libsswin3d.so")
 SOURCES = ["index_ops.hip", "plan.hip", "block_matmul.hip", "softmax.hip", "fused_attention.hip",
            "window_attention.hip", "window_attention_x16.hip", "column_sum.hip", "voxel_grid.hip", "tall_linear.hip",
-           "dense.hip", "dense_pairs.hip", "mlp.hip", "layer_norm.hip", "flash_attention.hip"]
+           "dense.hip", "dense_pairs.hip", "mlp.hip", "layer_norm.hip", "flash_attention.hip", "flash_window.hip"]
 ARCH = "gfx950"
 # packed FP32 instructions are switched off for all device code on purpose
 FLAGS = ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}",

@@ -1,0 +1,1007 @@
+// Window attention for heads of 16 channels in windows of up to 384 positions: a wavefront per (window, head) and up to 96 of the
+// window's tokens (WindowAttention.forward, sparse_swin/swin3d_base.py:654-675, from the projected qkv to the attention output, and
+// its backward with the gradient of the bias table in the same launch).  flash_attention.hip serves what these do not take: heads of 32
+// channels, more positions, heads or windows (sswin_flash_window_list_ints).
+//
+// Work: the windows by descending size (flash_window_tokens_kernel), dealt to as many workgroups as find a place at once; a workgroup keeps a
+// head's bias table, and in the backward the sums of its gradient, in LDS.  A window of up to KT tiles of 16 tokens is one wavefront's, one
+// of up to 2 KT tiles two wavefronts', larger ones take a workgroup of four.  All products are 16 x 16 tiles, laid out as in
+// flash_attention.hip: an accumulator is the operand of the next product over its rows.
+//
+// What this changes against blocks of 32 keys (flash_attention.hip): the scores of a window are formed once in the backward, not dS stored for dQ and for
+// the table's gradient (217 MB written and read twice with 225 700 tokens); rows are read once a window instead of once a block; P and dS meet
+// rows on the 16-bit matrix cores.  The table's gradient is summed by 64-bit integer additions in LDS, which take 10 clocks a wavefront's 64
+// (floating-point ones 180: what kept the sums out of the backward), and whose result does not depend on their order.
+//
+// Windows of 7^3, 3 heads of 16, us, blocks -> here: 112 700 tokens fp32 forward 56 -> 50, backward with the table's gradient 214 -> 115; 225 700 fp16 80 -> 75
+// and 348 -> 155; 8100 tokens in 50 nearly full windows, 24 heads, fp16: 66 and 129 here.  A tile takes a SIMD of the backward about 700 clocks (fp32) and 900
+// (fp16: 225 700 tokens), 300 of them instructions it issues: two wavefronts a SIMD, held there by their registers, wait for each other's rows,
+// transpositions and exponentials; a fourth of the time is in front of the first step of a window.
+#include <math.h>
+
+#include <algorithm>
+#include <type_traits>
+
+#include "flash_common.hpp"
+
+namespace sswin {
+namespace flash {
+namespace window {
+
+constexpr int HD = 16, WAVES = 4;
+constexpr int KT = 6, MOST = WAVES * KT;                                 // tiles of 16 tokens: of a wavefront in the backward, of a window
+constexpr int DELTA_BLOCKS = 1024, FORWARD_BLOCKS = 1024;
+constexpr int LIST_HEAD = 32, LIST_THREADS = 1024, LIST_WINDOWS = 16384;
+constexpr uint32_t INDEX = 0x7ffcu;                                      // of a difference of words: 4 row of the table
+constexpr int PITCH = 20, TURN = 16 * PITCH;                             // a 16 x 16 tile in LDS, values
+static_assert(MAX_ROWS * 4 <= 1 << 15, "codes and regions share a word");
+static_assert(MOST <= LIST_HEAD - 2, "the list's head counts windows by their tiles");
+
+struct Args {
+    const int32_t* plan;       // group table: [c | T | ..] of g_cap entries each, window k's groups at k H
+    int64_t g_cap;
+    const int32_t* order;      // voxel of token rank r
+    const uint32_t* word;      // 4 code | region << 15 | several regions in the window << 31 of token r
+    const int32_t* list;       // [t]: windows of more than t tiles; from LIST_HEAD on the windows, largest first
+    float* largest_v;          // [n_largest_v] largest |V| of the forward's workgroups
+    int n_largest_v;
+    int64_t N;
+    int windows, H, rows, offset4, per_head;
+    float scale;
+    const float* table;        // [rows, H]
+    const void* qkv;           // [N, 3 H hd] voxel rows
+    void* out;                 // [N, H hd]
+    float* lse;                // [H, N] by rank: offset + log2 of the row sum
+    // backward
+    const void* dout;          // [N, H hd]
+    const float* delta;        // [N, H]: dO . O
+    void* dqkv;                // [N, 3 H hd]
+    const float* largest;      // [n_largest] largest |dO| of some tokens
+    int n_largest;
+    float* partial;            // [H][per_head][rows] sums of dS by table row
+};
+
+// The windows by descending number of tiles, by one workgroup, and the word of every token, a wavefront per window.
+__device__ __forceinline__ void order_windows(const int32_t* __restrict__ plan, int windows, int H, int32_t* __restrict__ list) {
+    __shared__ uint16_t place[MOST * LIST_THREADS];                      // [class, most tiles first][thread]
+    __shared__ int sums[LIST_THREADS / 64];
+    const int t = threadIdx.x, per = (windows + LIST_THREADS - 1) / LIST_THREADS, begin = min(t * per, windows), end = min(begin + per, windows);
+    auto kind = [&](int k) { return MOST - max(1, min((plan[(int64_t)k * H] + 15) >> 4, MOST)); };
+    for (int k = 0; k < MOST; ++k) place[k * LIST_THREADS + t] = 0;
+    for (int k = begin; k < end; ++k) ++place[kind(k) * LIST_THREADS + t];
+    __syncthreads();
+    // sums in front, classes first; a thread adds MOST neighbours
+    int own = 0;
+    for (int k = 0; k < MOST; ++k) own += place[t * MOST + k];
+    int before = own;
+    for (int o = 1; o < 64; o <<= 1) {
+        const int v = __shfl_up(before, o, 64);
+        if ((t & 63) >= o) before += v;
+    }
+    if ((t & 63) == 63) sums[t >> 6] = before;
+    __syncthreads();
+    before -= own;
+    for (int w = 0; w < t >> 6; ++w) before += sums[w];
+    for (int k = 0; k < MOST; ++k) {
+        const int n = place[t * MOST + k];
+        place[t * MOST + k] = (uint16_t)before;
+        before += n;
+    }
+    __syncthreads();
+    // windows of more than t tiles: those in front of the class of t tiles
+    if (t < LIST_HEAD) list[t] = t >= MOST ? 0 : t == 0 ? windows : place[(MOST - t) * LIST_THREADS];
+    __syncthreads();
+    for (int k = begin; k < end; ++k) list[LIST_HEAD + place[kind(k) * LIST_THREADS + t]++] = k;
+}
+
+__global__ __launch_bounds__(LIST_THREADS) void flash_window_tokens_kernel(const int32_t* __restrict__ plan, int64_t g_cap, int windows, int H,
+                                                                           const int32_t* __restrict__ tok_pos, const int32_t* __restrict__ code,
+                                                                           const int8_t* __restrict__ mask, int nmw, int n, uint32_t* __restrict__ word,
+                                                                           int32_t* __restrict__ list) {
+    if (blockIdx.x == 0) return order_windows(plan, windows, H, list);
+    const int k = (int)(blockIdx.x - 1) * (LIST_THREADS / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (k >= windows) return;
+    const int64_t g = (int64_t)k * H;                                    // the window's first group (head 0)
+    const int c = plan[g], T = plan[g_cap + g], w = plan[3 * g_cap + g], lane = threadIdx.x & 63;
+    const int8_t* region = mask ? mask + (int64_t)(w % nmw) * n : nullptr;
+    uint32_t several = 0;
+    if (region) {
+        const int8_t r0 = region[tok_pos[T]];
+        bool differ = false;
+        for (int i = lane; i < c; i += 64) differ = differ || region[tok_pos[T + i]] != r0;
+        several = __any(differ) ? 0x80000000u : 0u;
+    }
+    for (int i = lane; i < c; i += 64) {
+        const int p = tok_pos[T + i];
+        word[T + i] = (uint32_t)code[p] * 4u | (region ? ((uint32_t)(uint8_t)region[p]) << 15 : 0u) | several;
+    }
+}
+
+// Workgroup -> head and place among the head's workgroups: the heads of the same windows follow each other on one XCD, whose L2 holds their rows
+__device__ __forceinline__ void place(int H, int& h, int& first) {
+    const int b = (int)blockIdx.x, y = b >> 3;
+    h = y % H;
+    first = y / H * 8 + (b & 7);
+}
+
+// The head's column of the bias table in units of log 2
+__device__ __forceinline__ void stage_table(const Args& g, int h, float* bias) {
+    constexpr int AT_ONCE = 9;                                           // of a thread, requested together: 13^3 rows
+    for (int r0 = threadIdx.x; r0 < g.rows; r0 += WAVES * 64 * AT_ONCE) {
+        float v[AT_ONCE];
+#pragma unroll
+        for (int i = 0; i < AT_ONCE; ++i) v[i] = g.table[(int64_t)min(r0 + i * WAVES * 64, g.rows - 1) * g.H + h];
+#pragma unroll
+        for (int i = 0; i < AT_ONCE; ++i)
+            if (r0 + i * WAVES * 64 < g.rows) bias[r0 + i * WAVES * 64] = v[i] * LOG2E;
+    }
+}
+
+// The pieces of work of a workgroup, as its wavefronts have them: every per_head-th of its head.  The largest windows come first, a workgroup
+// each; then those that two wavefronts hold, two at a time; then four at a time.  Lane l holds what is known of the l-th piece: list and plan are read
+// once, in front of the work.
+struct Task {
+    int team, rank, steps;     // wavefronts on the window, this one's number, tiles of the largest window among the workgroup's
+    int c, T, first, tiles;    // the window's tokens (0: nothing to do) and first rank, this wavefront's tiles
+};
+// TILES: of one wavefront; a window of up to 2 TILES has two, a larger one all four
+template <int TILES> struct Work {
+    int left, at;              // pieces not yet taken when the lanes were filled, lane of the next one
+    int u0, team, steps, c, T;
+    __device__ __forceinline__ void load(const Args& g) {
+        const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, u = u0 + lane * g.per_head;
+        const int big = g.list[2 * TILES], two = g.list[TILES], pairs = (two - big + 1) / 2, total = big + pairs + (g.windows - two + WAVES - 1) / WAVES;
+        left = u0 < total ? (total - u0 + g.per_head - 1) / g.per_head : 0;
+        at = team = steps = c = T = 0;
+        if (u >= total) return;
+        int from, end;
+        if (u < big) team = 4, from = u, end = big;
+        else if (u < big + pairs) team = 2, from = big + 2 * (u - big), end = two;
+        else team = 1, from = two + WAVES * (u - big - pairs), end = g.windows;
+        const int own = from + wave / team;
+        const int64_t head = (int64_t)g.list[LIST_HEAD + from] * g.H, group = (int64_t)g.list[LIST_HEAD + min(own, g.windows - 1)] * g.H;
+        steps = (g.plan[head] + 15) >> 4;
+        c = own < end ? g.plan[group] : 0;
+        T = g.plan[g.g_cap + group];
+    }
+    __device__ __forceinline__ Work(const Args& g, int first) {
+        u0 = first;
+        load(g);
+    }
+    __device__ __forceinline__ bool next(const Args& g, Task& t) {
+        if (at == 64) {
+            u0 += 64 * g.per_head;
+            load(g);
+        }
+        if (at >= left) return false;
+        t.team = __builtin_amdgcn_readlane(team, at);
+        t.steps = __builtin_amdgcn_readlane(steps, at);
+        t.c = __builtin_amdgcn_readlane(c, at);
+        t.T = __builtin_amdgcn_readlane(T, at);
+        ++at;
+        const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), all = (t.c + 15) >> 4, shift = t.team >> 1, share = all >> shift,
+                  more = all - (share << shift);
+        t.rank = wave & (t.team - 1);
+        t.tiles = share + (t.rank < more ? 1 : 0);
+        t.first = t.rank * share + min(t.rank, more);
+        return true;
+    }
+};
+
+__device__ __forceinline__ f32x4 widened(const Frag<float>& f) { return f.v; }
+__device__ __forceinline__ f32x4 widened(const Frag<__half>& f) { return f32x4{(float)f.v[0], (float)f.v[1], (float)f.v[2], (float)f.v[3]}; }
+__device__ __forceinline__ f32x4 widened(const Frag<__hip_bfloat16>& f) {
+    const uint2 w = __builtin_bit_cast(uint2, f.v);
+    return f32x4{__builtin_bit_cast(float, w.x << 16), __builtin_bit_cast(float, w.x & 0xffff0000u), __builtin_bit_cast(float, w.y << 16),
+                 __builtin_bit_cast(float, w.y & 0xffff0000u)};
+}
+
+// a 16 x 16 tile turned through LDS of the wavefront's own: lane (row l % 16, columns 4 (l / 16) + j) -> lane (rows 4 (l / 16) + j, column l % 16)
+__device__ __forceinline__ f32x4 turned(float* tile, const f32x4& v) {
+    const int l16 = threadIdx.x & 15, quad = (threadIdx.x & 63) >> 4;
+    *reinterpret_cast<f32x4*>(tile + l16 * PITCH + quad * 4) = v;
+    f32x4 r;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) r[j] = tile[(quad * 4 + j) * PITCH + l16];
+    return r;
+}
+
+// over the four lanes l % 16, to all of them
+template <typename F> __device__ __forceinline__ float across(float v, F&& f) {
+    const auto a = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(uint32_t, v), __builtin_bit_cast(uint32_t, v), false, false);
+    v = f(__builtin_bit_cast(float, (uint32_t)a[0]), __builtin_bit_cast(float, (uint32_t)a[1]));
+    const auto b = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, v), __builtin_bit_cast(uint32_t, v), false, false);
+    return f(__builtin_bit_cast(float, (uint32_t)b[0]), __builtin_bit_cast(float, (uint32_t)b[1]));
+}
+__device__ __forceinline__ float across_max(float v) {
+    return across(v, [](float a, float b) { return fmaxf(a, b); });
+}
+__device__ __forceinline__ float across_sum(float v) {
+    return across(v, [](float a, float b) { return a + b; });
+}
+
+// LDS by its address: a word of a query less one of a key is the address of their bias
+typedef __attribute__((address_space(3))) float LdsFloat;
+typedef __attribute__((address_space(3))) unsigned long long LdsLong;
+__device__ __forceinline__ uint32_t lds_address(const void* p) { return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)p; }
+__device__ __forceinline__ float lds_float(uint32_t at) { return *(const LdsFloat*)(uintptr_t)at; }
+
+// Arrays through buffer descriptors: a lane's 32 bits of offset and one of all lanes, no 64-bit addresses in vector registers, and what is read behind
+// an array's end is 0 (the clamps of the last step's rows).
+typedef __amdgpu_buffer_rsrc_t Buffer;
+template <typename V> __device__ __forceinline__ Buffer buffer(const V* p, int64_t count) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<V*>(p), 0, (int)(uint32_t)(count * (int64_t)sizeof(V)), 0x00020000);
+}
+__device__ __forceinline__ uint32_t load1(const Buffer& b, uint32_t lane_bytes, uint32_t bytes) {
+    return __builtin_amdgcn_raw_buffer_load_b32(b, lane_bytes, bytes, 0);
+}
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ u32x4 load4(const Buffer& b, uint32_t lane_bytes, uint32_t bytes) {
+    return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(b, lane_bytes, bytes, 0));
+}
+// rows of the voxels' tokens: four of a head's channels a lane
+template <typename T> struct Rows {
+    Buffer b;
+    uint32_t pitch, col, own;  // bytes: a row, the head's first channel, the lane's first channel in it
+    __device__ __forceinline__ Rows(const void* p, int64_t N, int pitch_, int col_)
+        : b(buffer(static_cast<const T*>(p), N * pitch_)), pitch((uint32_t)pitch_ * (uint32_t)sizeof(T)), col((uint32_t)col_ * (uint32_t)sizeof(T)),
+          own(((threadIdx.x & 63) >> 4) * (uint32_t)(4 * sizeof(T))) {}
+    __device__ __forceinline__ void row(int v, Frag<T>& f) const {
+        const uint32_t at = __umul24((uint32_t)v, pitch) + own;
+        if constexpr (sizeof(T) == 4) f.v = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(b, at, col, 0));
+        else f.v = __builtin_bit_cast(decltype(f.v), __builtin_amdgcn_raw_buffer_load_b64(b, at, col, 0));
+    }
+    __device__ __forceinline__ void store(int v, const f32x4& x) const {
+        const uint32_t at = __umul24((uint32_t)v, pitch) + own;
+        if constexpr (sizeof(T) == 4) __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, x), b, at, col, 0);
+        else __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, packed<T>(x).v), b, at, col, 0);
+    }
+};
+template <typename T> __device__ __forceinline__ void keep(bool live, Frag<T>& f) {
+    if (!live) f = Frag<T>{};
+}
+// the largest |x| of a row's four values, 0 if one of them is infinite
+__device__ __forceinline__ float largest_finite(const f32x4& v) {
+    const float m = fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3])));
+    return m < INFINITY ? m : 0.f;
+}
+__device__ __forceinline__ float largest_of_workgroup(float m, float* part) {
+    for (int o = 1; o < 64; o <<= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = m;
+    __syncthreads();
+    m = part[0];
+#pragma unroll
+    for (int w = 1; w < WAVES; ++w) m = fmaxf(m, part[w]);
+    return m;
+}
+// 0, or NaN if one of them is not finite
+__device__ __forceinline__ float not_finite(const f32x4& v) { return fmaf(v[0], 0.f, fmaf(v[1], 0.f, fmaf(v[2], 0.f, v[3] * 0.f))); }
+
+// ------------------------------------------------------------------------------------------
+// forward: a wavefront holds the queries of its tiles and walks over the window's keys, 16 at a time
+// ------------------------------------------------------------------------------------------
+constexpr int F_TILES = 4, F_RESIDENT = 3;                               // tiles of queries of a wavefront at a time; wavefronts a SIMD
+
+template <typename T> __global__ __launch_bounds__(WAVES * 64, F_RESIDENT) void flash_window_forward_kernel(Args g) {
+    extern __shared__ __attribute__((aligned(16))) char lds[];
+    const int lane = threadIdx.x & 63, l16 = lane & 15, quad = lane >> 4, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    float* const turn = reinterpret_cast<float*>(lds) + wave * TURN;
+    float* const bias = reinterpret_cast<float*>(lds) + WAVES * TURN;
+    const uint32_t bias_at = lds_address(bias);
+    int h, first;
+    place(g.H, h, first);
+    Work<F_TILES> work(g, first);
+    stage_table(g, h, bias);
+    __syncthreads();
+    const int D = g.H * HD;
+    const Rows<T> q_rows(g.qkv, g.N, 3 * D, h * HD), k_rows(g.qkv, g.N, 3 * D, D + h * HD), v_rows(g.qkv, g.N, 3 * D, 2 * D + h * HD), o_rows(g.out, g.N, D, h * HD);
+    const Buffer order = buffer(g.order, g.N), word = buffer(g.word, g.N);
+    const float scale2 = g.scale * LOG2E, unscale = 1.f / scale2;
+    float most = 0.f;
+    // F_TILES tiles of queries from tile `from` on; MASK: windows of several mask regions
+    auto run = [&](int c, int T0, int from, int count, auto masked_tag) __attribute__((always_inline)) {
+        constexpr bool MASK = decltype(masked_tag)::value;
+        constexpr uint32_t KEPT = MASK ? 0x7fffffffu : INDEX;            // of a word
+        const int all = (c + 15) >> 4;
+        struct Strip {                                                   // 16 keys
+            Frag<T> k, v;
+            u32x4 w;
+        };
+        auto voxel_of = [&](int s) { return (int)load1(order, l16 * 4, (T0 + s * 16) * 4); };
+        auto request = [&](int s, int voxel, Strip& x) {
+            k_rows.row(voxel, x.k);
+            v_rows.row(voxel, x.v);
+            x.w = load4(word, quad * 16, (T0 + s * 16) * 4);
+        };
+        Frag<T> q[F_TILES];
+        uint32_t pq[F_TILES];
+        int vq[F_TILES];
+        float offset[F_TILES], sum[F_TILES], top[F_TILES];
+        f32x4 o[F_TILES];
+        int voxel_ahead = voxel_of(0);
+#pragma unroll
+        for (int t = 0; t < F_TILES; ++t) {
+            offset[t] = sum[t] = 0.f, top[t] = -INFINITY;
+            o[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+            vq[t] = load1(order, l16 * 4, (T0 + (from + t) * 16) * 4);   // behind the window's end: some other token
+            pq[t] = (load1(word, l16 * 4, (T0 + (from + t) * 16) * 4) & KEPT) + (uint32_t)g.offset4 + (MASK ? 0 : bias_at);
+        }
+        Strip ahead;
+        request(0, voxel_ahead, ahead);
+        if (all > 1) voxel_ahead = voxel_of(1);
+#pragma unroll
+        for (int t = 0; t < F_TILES; ++t) q_rows.row(vq[t], q[t]);
+#pragma clang loop unroll(disable)
+        for (int s = 0; s < all; ++s) {
+            Strip now = ahead;
+            if (s + 1 < all) request(s + 1, voxel_ahead, ahead);
+            if (s + 2 < all) voxel_ahead = voxel_of(s + 2);
+            const int last = c - 1 - s * 16;
+            keep(l16 <= last, now.k), keep(l16 <= last, now.v);          // nothing behind the window's end
+            u32x4 wk;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) wk[j] = now.w[j] & KEPT;
+            const f32x4 vw = widened(now.v);
+            most = fmaxf(most, largest_finite(vw));
+            const Frag<float> vt = {turned(turn, vw)};
+            auto tiles = [&](auto from_tag) __attribute__((always_inline)) {
+                constexpr int FROM = decltype(from_tag)::value, COUNT = 2;   // two at a time: one's exponentials beside the other's products
+                float x[COUNT][4], xm[COUNT];
+                bool over = false;
+#pragma unroll
+                for (int i = 0; i < COUNT; ++i) {
+                    const int t = FROM + i;
+                    const float start = -offset[t] * unscale;            // the accumulator starts at minus the offset
+                    f32x4 acc = {start, start, start, start};
+                    acc = mma(now.k, q[t], acc);
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        const uint32_t d = pq[t] - wk[j];
+                        x[i][j] = fmaf(acc[j], scale2, lds_float(MASK ? (d & INDEX) + bias_at : d));
+                        if (MASK && d >> 15) x[i][j] += MASKED;
+                    }
+                    if (last < 15) {
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) x[i][j] = quad * 4 + j > last ? -INFINITY : x[i][j];
+                    }
+                    xm[i] = fmaxf(fmaxf(x[i][0], x[i][1]), fmaxf(x[i][2], x[i][3]));
+                    over = over || xm[i] > 10.f;
+                }
+                const bool move = s == 0 || __any(over);                 // the first tokens; later only by chance
+#pragma unroll
+                for (int i = 0; i < COUNT; ++i) {
+                    const int t = FROM + i;
+                    const float before = top[t];
+                    top[t] = fmaxf(before, xm[i]);
+                    if (move) {
+                        const float m = across_max(xm[i]);
+                        const bool fresh = across_max(before) == -INFINITY;
+                        const float by = m == -INFINITY ? 0.f : fresh ? m : fmaxf(0.f, m), f = fresh ? 0.f : __builtin_amdgcn_exp2f(-by);
+                        offset[t] += by;
+                        top[t] -= by;
+                        sum[t] *= f;
+                        o[t] *= f;
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) x[i][j] -= by;
+                    }
+                    f32x4 p;
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) p[j] = __builtin_amdgcn_exp2f(x[i][j]);
+                    sum[t] += (p[0] + p[1]) + (p[2] + p[3]);
+                    o[t] = mma(vt, Frag<float>{p}, o[t]);
+                }
+            };
+            tiles(std::integral_constant<int, 0>{});
+            if (count > 2) tiles(std::integral_constant<int, 2>{});
+        }
+#pragma unroll
+        for (int t = 0; t < F_TILES; ++t) {
+            if (t >= count) break;
+            // top: the row's maximum less the offset
+            const float z = across_sum(sum[t]) + 1e-8f * __builtin_amdgcn_exp2f(fmaxf(across_max(top[t]), -offset[t]));
+            const float inv = 1.f / z;
+            const int at = (from + t) * 16 + l16;
+            if (at < c) {
+                o_rows.store(vq[t], o[t] * inv);
+                if (quad == 0) g.lse[h * g.N + T0 + at] = offset[t] + __builtin_amdgcn_logf(z);
+            }
+        }
+    };
+    Task task;
+    while (work.next(g, task)) {
+        const int all = (task.c + 15) >> 4;
+        for (int from = task.rank * F_TILES; from < all; from += task.team * F_TILES) {
+            const int count = min(F_TILES, all - from);
+            if (g.word[task.T] >> 31) run(task.c, task.T, from, count, std::true_type{});
+            else run(task.c, task.T, from, count, std::false_type{});
+        }
+    }
+    __syncthreads();
+    const float m = largest_of_workgroup(most, bias);           // (the table has been read)
+    if (threadIdx.x == 0) g.largest_v[blockIdx.x] = m;
+}
+
+// ------------------------------------------------------------------------------------------
+// D = dO . O of every voxel and head, four lanes a head, and the largest |dO| (of what is finite) of a workgroup
+// ------------------------------------------------------------------------------------------
+template <typename T> __global__ __launch_bounds__(256) void flash_window_delta_kernel(const T* __restrict__ dout, const T* __restrict__ out, int64_t parts,
+                                                                                       float* __restrict__ delta, float* __restrict__ largest) {
+    __shared__ float part[4];
+    constexpr int AT_ONCE = 4;
+    float most = 0.f;
+    for (int64_t i0 = (int64_t)blockIdx.x * 256 + threadIdx.x; i0 < parts; i0 += (int64_t)gridDim.x * 256 * AT_ONCE) {
+        Frag<T> x[AT_ONCE], y[AT_ONCE];
+#pragma unroll
+        for (int k = 0; k < AT_ONCE; ++k) {
+            const int64_t i = min(i0 + (int64_t)gridDim.x * 256 * k, parts - 1);
+            x[k].load(dout + i * 4), y[k].load(out + i * 4);
+        }
+#pragma unroll
+        for (int k = 0; k < AT_ONCE; ++k) {
+            const int64_t i = i0 + (int64_t)gridDim.x * 256 * k;
+            const f32x4 a = widened(x[k]), b = widened(y[k]);
+            float dot = 0.f;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) dot = fmaf(a[j], b[j], dot);
+            dot += dpp_f32<0xB1>(dot);
+            dot += dpp_f32<0x4E>(dot);
+            most = fmaxf(most, largest_finite(a));
+            if (i < parts && (threadIdx.x & 3) == 0) delta[i >> 2] = dot;
+        }
+    }
+    const float m = largest_of_workgroup(most, part);
+    if (threadIdx.x == 0) largest[blockIdx.x] = m;
+}
+
+// The unit of the table's sums.  Integers, so that the result does not depend on the order of the additions.  |dS| <= |dP| + |D| <= 2 * 16 largest |dO| largest |V| (P of a row adds up to at most one, up to rounding) < 2^top; dS
+// in units of 2^(top - bits) is a whole number below 2^50, and N of them below 2^62.
+struct Unit {
+    int top, bits;
+    __device__ __forceinline__ Unit(float mo, float mv, int64_t N) {
+        const int eo = mo > 0.f ? (int)ilogbf(mo) : -149, ev = mv > 0.f ? (int)ilogbf(mv) : -149;
+        top = eo + ev + 8;
+        bits = min(50, 62 - (64 - __builtin_clzll((unsigned long long)N)));
+    }
+};
+
+// ------------------------------------------------------------------------------------------
+// Pieces.  P, dS and, of fp32 tokens, the rows are multiplied on the 16-bit matrix cores as x 2^e = h + l, h and l fp16 rounded to nearest, all
+// products of pieces kept but that of two l in dQ; sums are fp32.  22 bits of a value or 2^-25 in its scale, whichever is more, with fewer roundings of sums: error
+// against float64 (2-norms, windows of 7^3, fp32) dQ 5.4e-7 with fp32 products, 3.4e-7 here, dK 5.2 and 3.2, dV 5.0 and 3.0, table 5.2 and 4.1; 16-bit tokens: the
+// same to three digits.  A scale e is one of a wavefront: of K and V for the window, of Q and dO kept from step to step until a row no longer fits, when the
+// sums so far are scaled with it.  Rows too far below the largest for that, and windows in which something is not finite, are done with fp32 products
+// (How::exact), a whole window at a time.
+// ------------------------------------------------------------------------------------------
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+struct Pair {                  // x = h + l
+    f16x4 h, l;
+};
+__device__ __forceinline__ Pair split(const f32x4& x) {
+    typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+    struct Words { uint32_t a, b; };
+    Words h, l;
+    f16x2 h0 = {(_Float16)x[0], (_Float16)x[1]}, h1 = {(_Float16)x[2], (_Float16)x[3]};
+    asm("" : "+v"(h0), "+v"(h1));                                        // (or each half is converted again for its rest)
+    const f16x2 l0 = {(_Float16)fmaf(-1.f, (float)h0[0], x[0]), (_Float16)fmaf(-1.f, (float)h0[1], x[1])};
+    const f16x2 l1 = {(_Float16)fmaf(-1.f, (float)h1[0], x[2]), (_Float16)fmaf(-1.f, (float)h1[1], x[3])};
+    h = {__builtin_bit_cast(uint32_t, h0), __builtin_bit_cast(uint32_t, h1)};
+    l = {__builtin_bit_cast(uint32_t, l0), __builtin_bit_cast(uint32_t, l1)};
+    return Pair{__builtin_bit_cast(f16x4, h), __builtin_bit_cast(f16x4, l)};
+}
+__device__ __forceinline__ f16x8 both(const f16x4& a, const f16x4& b) { return __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7); }
+__device__ __forceinline__ f16x4 halves(const f32x4& x) { return packed<__half>(x).v; }
+__device__ __forceinline__ f32x4 mma32(const f16x8& a, const f16x8& b, const f32x4& c) { return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0); }
+__device__ __forceinline__ f32x4 mma16(const f16x4& a, const f16x4& b, const f32x4& c) { return __builtin_amdgcn_mfma_f32_16x16x16f16(a, b, c, 0, 0, 0); }
+
+// What a wavefront multiplies with all pairs of another operand: 16-bit tokens are one piece, fp32 tokens two
+template <typename T> struct Column {
+    f16x4 h;
+    __device__ __forceinline__ void set(const f32x4& x) { h = halves(x); }
+    __device__ __forceinline__ f32x4 times(const Pair& p, f32x4 c) const { return mma32(both(h, h), both(p.h, p.l), c); }
+    __device__ __forceinline__ f32x4 times16(const Pair& p, f32x4 c) const { return mma16(h, p.l, mma16(h, p.h, c)); }
+};
+template <> struct Column<float> {
+    Pair x;
+    __device__ __forceinline__ void set(const f32x4& v) { x = split(v); }
+    __device__ __forceinline__ f32x4 times(const Pair& p, f32x4 c) const { return mma32(both(x.l, x.l), both(p.h, p.l), mma32(both(x.h, x.h), both(p.h, p.l), c)); }
+    __device__ __forceinline__ f32x4 times16(const Pair& p, f32x4 c) const { return mma16(x.l, p.h, mma16(x.h, p.l, mma16(x.h, p.h, c))); }
+};
+// row operands: of 16-bit tokens as they are, of fp32 tokens as pairs
+template <typename T> struct Row {
+    Frag<T> f;
+    __device__ __forceinline__ void set(const Frag<T>& raw, const f32x4&, float) { f = raw; }
+    static __device__ __forceinline__ f32x4 times(const Row& a, const Row& b, const f32x4& c) { return mma(a.f, b.f, c); }
+};
+template <> struct Row<float> {
+    Pair x;
+    __device__ __forceinline__ void set(const Frag<float>&, const f32x4& v, float by) { x = split(v * by); }
+    static __device__ __forceinline__ f32x4 times(const Row& a, const Row& b, const f32x4& c) {
+        return mma32(both(a.x.l, a.x.l), both(b.x.h, b.x.l), mma32(both(a.x.h, a.x.h), both(b.x.h, b.x.l), c));
+    }
+};
+
+// Powers of two that bring numbers into fp16's range: `e` for a largest value of [2^(12 - e), 2^(13 - e)), kept until it reaches 2^(15 - e)
+constexpr uint32_t NOT_FINITE = 0x7f800000u;
+__device__ __forceinline__ float power(int e) { return __builtin_bit_cast(float, (uint32_t)(127 + e) << 23); }
+__device__ __forceinline__ uint32_t largest4(const f32x4& v) {           // as bits, which grow with the absolute value
+    uint32_t m = 0;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const float x = v[j];                                            // (a bit cast of the element itself takes the first)
+        m = max(m, __builtin_bit_cast(uint32_t, x) & 0x7fffffffu);
+    }
+    return m;
+}
+__device__ __forceinline__ uint32_t over_quads(uint32_t m) {             // the largest of the four lanes l % 16
+    const auto a = __builtin_amdgcn_permlane16_swap(m, m, false, false);
+    m = max((uint32_t)a[0], (uint32_t)a[1]);
+    const auto b = __builtin_amdgcn_permlane32_swap(m, m, false, false);
+    return max((uint32_t)b[0], (uint32_t)b[1]);
+}
+__device__ __forceinline__ int over_rows(uint32_t m) {                   // of all lanes, once over_quads has been
+    m = m < NOT_FINITE ? m : 0;
+    return __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, row16_max(__builtin_bit_cast(float, m))));
+}
+__device__ __forceinline__ int scale_for(int largest, int most) { return largest == 0 ? most : max(-most, min(most, 12 + 127 - (largest >> 23))); }
+__device__ __forceinline__ bool too_large(uint32_t m, int e) { return m >= (uint32_t)(142 - e) << 23; }
+// pieces of a row whose largest value is below 2^(low - e) would lose bits of it
+template <typename T> __device__ __forceinline__ bool too_small(uint32_t m, int e) {
+    constexpr int low = sizeof(T) == 4 ? 0 : -6;
+    return m != 0 && m < (uint32_t)(127 + low - e) << 23;
+}
+
+// ------------------------------------------------------------------------------------------
+// backward: a wavefront holds keys and values of its tiles and walks over the window's queries, 16 at a time.  Scores, P and dS are formed once: dV = P^T dO
+// and dK = scale dS^T Q stay in accumulators, dS is turned through LDS for dQ = scale dS K (the wavefronts of a window add theirs in a fixed
+// order), and its entries are added to the head's table in LDS.
+// ------------------------------------------------------------------------------------------
+constexpr int B_RESIDENT = 2;                                            // wavefronts a SIMD
+constexpr int WAVE_LDS = 3 * TURN + 16;                                  // of a wavefront: three tiles to turn, D of 16 queries
+// P is multiplied by 2^P_BITS: its pieces then hold it to 2^-31, and exponents lie around zero, where fp32 rounds them least
+constexpr int P_BITS = 7;
+enum class How { plain, masked, exact };   // windows of one mask region, of several; fp32 products of the rows as they are
+template <typename T, bool TABLE> __global__ __launch_bounds__(WAVES * 64, B_RESIDENT) void flash_window_backward_kernel(Args g) {
+    constexpr bool PAIRS = sizeof(T) == 4, SCALED = !std::is_same<T, __half>::value;
+    extern __shared__ __attribute__((aligned(16))) char lds[];
+    const int lane = threadIdx.x & 63, l16 = lane & 15, quad = lane >> 4, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    // LDS: [rows] sums, [2][rows / 32] bits of rows that are +inf, -inf; tiles to turn; exchange; bias of the head
+    const int words = (g.rows + 31) >> 5;
+    unsigned long long* const sums = reinterpret_cast<unsigned long long*>(lds);
+    uint32_t* const infinite = reinterpret_cast<uint32_t*>(sums + (TABLE ? g.rows : 0));
+    float* const tiles_lds = reinterpret_cast<float*>(infinite + (TABLE ? (2 * words + 3) / 4 * 4 + (g.rows & 1) * 2 : 0));
+    float* const turn = tiles_lds + wave * WAVE_LDS;
+    float* const deltas = turn + 3 * TURN;
+    float* const shared = tiles_lds + WAVES * WAVE_LDS;                  // [2][WAVES][256]
+    int* const stops = reinterpret_cast<int*>(shared + 2 * WAVES * 256); // [2][8]
+    float* const bias = shared + 2 * WAVES * 256 + 16;
+    const uint32_t bias_at = lds_address(bias), sums_at = lds_address(sums) - 2 * bias_at;   // of a row's sum, with twice the address of its bias
+    int h, first;
+    place(g.H, h, first);
+    Work<KT> work(g, first);
+    stage_table(g, h, bias);
+    if (threadIdx.x < 16) stops[threadIdx.x] = 0;
+    int unit = 0, top = 0;                                               // the table's sums are in units of 2^unit; |dS| < 2^top
+    if constexpr (TABLE) {
+        for (int i = threadIdx.x; i < g.rows; i += WAVES * 64) sums[i] = 0;
+        for (int i = threadIdx.x; i < 2 * words; i += WAVES * 64) infinite[i] = 0;
+        float mo = 0.f, mv = 0.f, o[DELTA_BLOCKS / 64], v[FORWARD_BLOCKS / 64];   // requested together
+#pragma unroll
+        for (int i = 0; i < DELTA_BLOCKS / 64; ++i) o[i] = g.largest[min(i * 64 + lane, g.n_largest - 1)];
+#pragma unroll
+        for (int i = 0; i < FORWARD_BLOCKS / 64; ++i) v[i] = g.largest_v[min(i * 64 + lane, g.n_largest_v - 1)];
+#pragma unroll
+        for (int i = 0; i < DELTA_BLOCKS / 64; ++i) mo = fmaxf(mo, o[i]);
+#pragma unroll
+        for (int i = 0; i < FORWARD_BLOCKS / 64; ++i) mv = fmaxf(mv, v[i]);
+        for (int o = 1; o < 64; o <<= 1) mo = fmaxf(mo, __shfl_xor(mo, o, 64)), mv = fmaxf(mv, __shfl_xor(mv, o, 64));
+        const Unit u(mo, mv, g.N);
+        top = __builtin_amdgcn_readfirstlane(u.top), unit = top - u.bits;
+    }
+    __syncthreads();
+    const int D = g.H * HD;
+    const Rows<T> q_rows(g.qkv, g.N, 3 * D, h * HD), k_rows(g.qkv, g.N, 3 * D, D + h * HD), v_rows(g.qkv, g.N, 3 * D, 2 * D + h * HD), do_rows(g.dout, g.N, D, h * HD);
+    const Rows<T> dq_rows(g.dqkv, g.N, 3 * D, h * HD), dk_rows(g.dqkv, g.N, 3 * D, D + h * HD), dv_rows(g.dqkv, g.N, 3 * D, 2 * D + h * HD);
+    const Buffer order = buffer(g.order, g.N), word = buffer(g.word, g.N), lses = buffer(g.lse + h * g.N, g.N), dots = buffer(g.delta, g.N * g.H);
+    const float scale2 = g.scale * LOG2E, unscale = 1.f / scale2;
+
+    // A window's tiles.  Returns -1, or, where pieces of one scale do not hold the rows, how many steps are in the table's sums: the window is then done
+    // again with fp32 products (by all of a workgroup that shares windows), with the rest of the steps.
+    auto run = [&](const Task& task, int added, auto how_tag) __attribute__((always_inline)) -> int {
+        constexpr How HOW = decltype(how_tag)::value;
+        constexpr bool EXACT = HOW == How::exact, MASK = HOW != How::plain;
+        constexpr uint32_t KEPT = MASK ? 0x7fffffffu : INDEX;            // of a word
+        const int c = task.c, T0 = task.T, all = (c + 15) >> 4;
+        Row<T> k[KT], v[KT];
+        Column<T> kt[KT];
+        f32x4 dk[KT], dv[KT];
+        uint32_t pk[KT];
+        int vk[KT];
+        bool stop = false;
+        int ek = 0, ev = 0, eq = 30, eo = 60;                            // scales
+        if (task.team > 1) __syncthreads();                              // the exchange of the last window has been read
+        if (c > 0) {
+            Frag<T> raw_k[KT], raw_v[KT];
+#pragma unroll
+            for (int t = 0; t < KT; ++t) {
+                dk[t] = dv[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+                vk[t] = load1(order, l16 * 4, (T0 + (task.first + t) * 16) * 4);   // behind the window's end: some other token
+                pk[t] = load1(word, l16 * 4, (T0 + (task.first + t) * 16) * 4) & KEPT;
+            }
+            if constexpr (!EXACT) {
+#pragma unroll
+                for (int t = 0; t < KT; ++t) k_rows.row(vk[t], raw_k[t]), v_rows.row(vk[t], raw_v[t]);
+                uint32_t mk[KT], mv[KT], most_k = 0, most_v = 0;
+#pragma unroll
+                for (int t = 0; t < KT; ++t) {
+                    const bool live = t < task.tiles && (task.first + t) * 16 + l16 < c;
+                    keep(live, raw_k[t]), keep(live, raw_v[t]);
+                    mk[t] = over_quads(largest4(widened(raw_k[t]))), mv[t] = over_quads(largest4(widened(raw_v[t])));
+                    most_k = max(most_k, mk[t]), most_v = max(most_v, mv[t]);
+                }
+                if (SCALED) ek = scale_for(over_rows(most_k), 30);
+                ev = scale_for(over_rows(most_v), 30);
+                bool lost = most_k >= NOT_FINITE || most_v >= NOT_FINITE;
+#pragma unroll
+                for (int t = 0; t < KT; ++t) {
+                    if (SCALED) lost = lost || too_large(mk[t], ek) || too_small<T>(mk[t], ek);
+                    lost = lost || too_large(mv[t], ev) || (PAIRS && too_small<T>(mv[t], ev));
+                    const f32x4 kw = widened(raw_k[t]);
+                    k[t].set(raw_k[t], kw, power(ek)), v[t].set(raw_v[t], widened(raw_v[t]), power(ev));
+                    kt[t].set(turned(turn, SCALED ? kw * power(ek) : kw));
+                }
+                stop = __any(lost);
+                if (task.team == 1 && stop) return 0;
+            }
+        }
+        struct Strip {                                                   // 16 queries
+            int voxel;
+            Frag<T> q, d_o;
+            u32x4 w;
+            f32x4 lse;
+            float delta;                                                 // of the lane's row
+        };
+        auto voxel_of = [&](int s) { return (int)load1(order, l16 * 4, (T0 + s * 16) * 4); };
+        auto request = [&](int s, int voxel, Strip& x) {
+            x.voxel = voxel;
+            q_rows.row(voxel, x.q);
+            do_rows.row(voxel, x.d_o);
+            x.delta = __builtin_bit_cast(float, load1(dots, __umul24((uint32_t)voxel, (uint32_t)g.H) * 4, h * 4));
+            x.w = load4(word, quad * 16, (T0 + s * 16) * 4);
+            x.lse = __builtin_bit_cast(f32x4, load4(lses, quad * 16, (T0 + s * 16) * 4));
+        };
+        Strip ahead;
+        int voxel_ahead = 0;
+        if (c > 0) {
+            request(0, voxel_of(0), ahead);
+            if (all > 1) voxel_ahead = voxel_of(1);
+        }
+        const int steps = task.team > 1 ? task.steps : all;
+#pragma clang loop unroll(disable)
+        for (int s = 0; s < steps; ++s) {
+            f32x4 dq = {0.f, 0.f, 0.f, 0.f};
+            int voxel = 0;
+            if (s < all) {
+                Strip now = ahead;
+                voxel = now.voxel;
+                if (s + 1 < all) request(s + 1, voxel_ahead, ahead);
+                if (s + 2 < all) voxel_ahead = voxel_of(s + 2);
+                const int last = c - 1 - s * 16;
+                float odd = 0.f;
+                if (last < 15) {                                         // nothing behind the window's end
+                    keep(l16 <= last, now.q), keep(l16 <= last, now.d_o);
+                    if (l16 > last) now.delta = 0.f;
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+                        if (quad * 4 + j > last) now.lse[j] = INFINITY;
+                        else odd += now.lse[j] * 0.f;
+                } else {
+                    odd = not_finite(now.lse);
+                }
+                const f32x4 qw = widened(now.q), ow = widened(now.d_o);
+                if (quad == 0) deltas[l16] = now.delta;
+                const f32x4 delta = *reinterpret_cast<const f32x4*>(deltas + quad * 4);   // of the rows of an accumulator
+                uint32_t pq[4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) pq[j] = (now.w[j] & KEPT) + (uint32_t)g.offset4 + (MASK ? 0 : bias_at);
+                int es = 0;                                              // dS 2^es lies below 2^15
+                if constexpr (!EXACT) {
+                    const uint32_t mq = SCALED ? over_quads(largest4(qw)) : 0, mo = over_quads(largest4(ow));
+                    if (__any((SCALED && too_large(mq, eq)) || too_large(mo, eo))) {
+                        const int q_to = SCALED ? min(eq, scale_for(over_rows(mq), 30)) : eq, o_to = min(eo, scale_for(over_rows(mo), 60));
+                        const float bk = power(max(-126, q_to - eq + o_to - eo)), bv = SCALED ? power(max(-126, o_to - eo)) : 1.f;
+#pragma unroll
+                        for (int t = 0; t < KT; ++t) dk[t] *= bk, dv[t] *= bv;
+                        eq = q_to, eo = o_to;
+                    }
+                    stop = stop || __any(odd != odd || !(fabsf(now.delta) < power(32 - eo - ev)) || (SCALED && (too_large(mq, eq) || too_small<T>(mq, eq))) || too_large(mo, eo) || too_small<T>(mo, eo));
+                    if (stop && task.team == 1) return s;
+                    es = eo + ev - 18;
+                }
+                // added to it, a value times 2^es is rounded to the unit of the sums
+                const uint32_t unit_hi = (uint32_t)(0x3ff80000 + ((52 + unit + es) << 20));
+                const double whole = __builtin_bit_cast(double, (unsigned long long)unit_hi << 32);
+                auto add = [&](uint32_t at, float x) __attribute__((always_inline)) {
+                    const unsigned long long b = __builtin_bit_cast(unsigned long long, (double)x + whole);
+                    const unsigned long long n = (unsigned long long)((uint32_t)(b >> 32) - unit_hi) << 32 | (uint32_t)b;
+                    __hip_atomic_fetch_add((LdsLong*)(uintptr_t)(2 * at + sums_at), n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                };
+                if constexpr (!EXACT) {
+                  if (!stop) {
+                    const float cq = SCALED ? power(eq) : 1.f, co = SCALED ? power(eo) : 1.f;
+                    Row<T> q, d_o;
+                    q.set(now.q, qw, cq), d_o.set(now.d_o, ow, co);
+                    Column<T> qt, dot;
+                    qt.set(turned(turn + 2 * TURN, SCALED ? qw * cq : qw));
+                    dot.set(turned(turn + 2 * TURN, SCALED ? ow * co : ow));
+                    const float by_s = PAIRS ? power(eq + ek) : 1.f, by_p = PAIRS ? power(eo + ev) : 1.f, to_s = PAIRS ? scale2 * power(-eq - ek) : scale2,
+                                to_ds = PAIRS ? power(-18 - P_BITS) : power(es - P_BITS);
+                    const f32x4 a0 = (now.lse - (float)P_BITS) * (-unscale * by_s), d0 = delta * -by_p;  // what the accumulators start from: P comes out times 2^P_BITS
+                    auto tiles = [&](auto from_tag) __attribute__((always_inline)) {
+                        constexpr int FROM = decltype(from_tag)::value, COUNT = 2;
+                        f32x4 p[COUNT], ds[COUNT];
+                        uint32_t at[COUNT][4];
+#pragma unroll
+                        for (int i = 0; i < COUNT; ++i) {
+                            const int t = FROM + i;
+                            const f32x4 acc = Row<T>::times(q, k[t], a0), dp = Row<T>::times(d_o, v[t], d0);
+#pragma unroll
+                            for (int j = 0; j < 4; ++j) {
+                                const uint32_t d = pq[j] - pk[t];
+                                at[i][j] = MASK ? (d & INDEX) + bias_at : d;
+                                float x = fmaf(acc[j], to_s, lds_float(at[i][j]));
+                                if (MASK && d >> 15) x += MASKED;
+                                p[i][j] = __builtin_amdgcn_exp2f(fminf(x, P_BITS + 0.5f));   // (P of keys behind the window's end has no bound)
+                                ds[i][j] = p[i][j] * to_ds * dp[j];
+                            }
+                        }
+                        if constexpr (TABLE) {
+#pragma unroll
+                            for (int i = 0; i < COUNT; ++i)
+                                if (FROM + i < task.tiles && (task.first + FROM + i) * 16 + l16 < c) {
+#pragma unroll
+                                    for (int j = 0; j < 4; ++j) add(at[i][j], ds[i][j]);
+                                }
+                        }
+#pragma unroll
+                        for (int i = 0; i < COUNT; ++i) {
+                            const int t = FROM + i;
+                            const f32x4 dst = turned(turn + i * TURN, ds[i]);
+                            dv[t] = dot.times(split(p[i]), dv[t]);
+                            dk[t] = qt.times(split(ds[i]), dk[t]);
+                            dq = kt[t].times16(split(dst), dq);
+                        }
+                    };
+                    tiles(std::integral_constant<int, 0>{});
+                    if (task.tiles > 2) tiles(std::integral_constant<int, 2>{});
+                    if (task.tiles > 4) tiles(std::integral_constant<int, 4>{});
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) dq[j] = __builtin_amdgcn_ldexpf(dq[j], -es - ek);
+                  }
+                } else {
+                    const Frag<float> qt = {turned(turn + 2 * TURN, qw)}, dot = {turned(turn + 2 * TURN, ow)};
+                    const f32x4 a0 = now.lse * -unscale, d0 = -delta;
+                    const float most = top > 126 ? 3.0e38f : power(max(-126, top));
+#pragma unroll
+                    for (int t = 0; t < KT; ++t) {
+                        if (t >= task.tiles) break;
+                        const bool live = (task.first + t) * 16 + l16 < c;
+                        Frag<T> raw_k, raw_v;
+                        k_rows.row(vk[t], raw_k), v_rows.row(vk[t], raw_v);
+                        keep(live, raw_k), keep(live, raw_v);
+                        const f32x4 acc = mma(now.q, raw_k, a0), dp = mma(now.d_o, raw_v, d0);
+                        Frag<float> pf, df;
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) {
+                            const bool taken = live && quad * 4 + j <= last;
+                            const uint32_t d = pq[j] - pk[t], at = (d & INDEX) + bias_at;
+                            float x = fmaf(acc[j], scale2, lds_float(at));
+                            if (d >> 15) x += MASKED;
+                            pf.v[j] = taken ? __builtin_amdgcn_exp2f(x) : 0.f;
+                            df.v[j] = taken ? pf.v[j] * dp[j] : 0.f;
+                            if (TABLE && taken && s >= added) {
+                                if (fabsf(df.v[j]) <= most) add(at, df.v[j]);
+                                else {
+                                    const uint32_t row = (d & INDEX) >> 2, bit = 1u << (row & 31);
+                                    if (!(df.v[j] < 0.f)) atomicOr(infinite + (row >> 5), bit);
+                                    if (!(df.v[j] > 0.f)) atomicOr(infinite + words + (row >> 5), bit);
+                                }
+                            }
+                        }
+                        const Frag<float> ktf = {turned(turn, widened(raw_k))}, dst = {turned(turn + TURN, df.v)};
+                        dv[t] = mma(dot, pf, dv[t]);
+                        dk[t] = mma(qt, df, dk[t]);
+                        dq = mma(ktf, dst, dq);
+                    }
+                }
+            }
+            if (task.team > 1) {
+                // the wavefronts of a window take turns in adding; a part is not written again before the next barrier but one
+                float* const part = shared + ((s & 1) * WAVES + wave - task.rank) * 256;
+                const int adds = s & (task.team - 1);
+                if (task.rank != adds && s < all) *reinterpret_cast<f32x4*>(part + task.rank * 256 + lane * 4) = dq;
+                if (!EXACT && lane == 0) stops[(s & 1) * 8 + wave] = stop;
+                __syncthreads();
+                if constexpr (!EXACT) {
+                    const int* const one = stops + (s & 1) * 8;
+                    bool any = false;
+#pragma unroll
+                    for (int w = 0; w < WAVES; ++w) any = any || one[w];
+                    if (__builtin_amdgcn_readfirstlane(any)) return stop ? min(s, all) : min(s + 1, all);
+                }
+                if (task.rank == adds && s < all) {
+                    f32x4 sum = {0.f, 0.f, 0.f, 0.f};
+                    for (int w = 0; w < task.team; ++w) sum += w == task.rank ? dq : *reinterpret_cast<const f32x4*>(part + w * 256 + lane * 4);
+                    dq = sum;
+                }
+                if (task.rank != adds) continue;
+            }
+            if (s * 16 + l16 < c) dq_rows.store(voxel, dq * g.scale);
+        }
+        const int sk = EXACT ? 0 : -(eo + ev - 18) - (SCALED ? eq : 0), sv = EXACT ? 0 : -P_BITS - (SCALED ? eo : 0);
+#pragma unroll
+        for (int t = 0; t < KT; ++t)
+            if (t < task.tiles && (task.first + t) * 16 + l16 < c) {
+                f32x4 x, y;
+#pragma unroll
+                for (int j = 0; j < 4; ++j) x[j] = __builtin_amdgcn_ldexpf(dk[t][j] * g.scale, sk), y[j] = __builtin_amdgcn_ldexpf(dv[t][j], sv);
+                dk_rows.store(vk[t], x);
+                dv_rows.store(vk[t], y);
+            }
+        return -1;
+    };
+    Task task;
+    while (work.next(g, task)) {
+        const bool several = task.c > 0 && g.word[task.T] >> 31;
+        const int added = several ? run(task, 0, std::integral_constant<How, How::masked>{}) : run(task, 0, std::integral_constant<How, How::plain>{});
+        if (added >= 0) run(task, added, std::integral_constant<How, How::exact>{});
+    }
+    if constexpr (TABLE) {
+        __syncthreads();
+        float* const to = g.partial + ((int64_t)h * g.per_head + first) * g.rows;
+        for (int i = threadIdx.x; i < g.rows; i += WAVES * 64) {
+            float sum = (float)ldexp((double)(long long)sums[i], unit);
+            const bool up = infinite[i >> 5] >> (i & 31) & 1, down = infinite[words + (i >> 5)] >> (i & 31) & 1;
+            if (up) sum = down ? __builtin_nanf("") : INFINITY;
+            else if (down) sum = -INFINITY;
+            to[i] = sum;
+        }
+    }
+}
+
+// d table[row][h]: a workgroup adds 16 rows of a head, 64 threads a row, in a fixed order
+__global__ __launch_bounds__(1024) void flash_window_table_kernel(const float* __restrict__ partial, int per_head, int rows, int H, float* __restrict__ d_table) {
+    __shared__ double part[64][17];
+    const int r = threadIdx.x & 15, q = threadIdx.x >> 4, h = blockIdx.y, row = blockIdx.x * 16 + r;
+    double s = 0.;
+    if (row < rows) {
+        const float* const src = partial + (int64_t)h * per_head * rows + row;
+        for (int i = q; i < per_head; i += 64) s += src[(int64_t)i * rows];
+    }
+    part[q][r] = s;
+    __syncthreads();
+    if (q == 0 && row < rows) {
+        double total = 0.;
+        for (int k = 0; k < 64; ++k) total += part[k][r];
+        d_table[(int64_t)row * H + h] = (float)total;
+    }
+}
+
+// Workgroups of a head: as many as find a place at once, and no more than it has windows
+static int per_head(int windows, int H, int resident) {
+    const int m = std::max(1, resident * device_cus() / (8 * H));
+    return std::min(8 * m, (windows + 7) / 8 * 8);
+}
+
+static size_t backward_lds(int rows, bool table) {
+    const int words = (rows + 31) / 32;
+    return (table ? (size_t)rows * 8 + ((2 * words + 3) / 4 * 4 + (rows & 1) * 2) * 4 : 0) + (size_t)(WAVES * WAVE_LDS + 2 * WAVES * 256 + 16 + rows) * sizeof(float);
+}
+
+template <typename T, bool TABLE> static int launch_backward(Args g, hipStream_t s) {
+    const size_t lds = backward_lds(g.rows, TABLE);
+    if (lds > 64 * 1024)
+        SSWIN_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(flash_window_backward_kernel<T, TABLE>), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+    hipLaunchKernelGGL((flash_window_backward_kernel<T, TABLE>), dim3((unsigned)(g.per_head * g.H)), dim3(WAVES * 64), lds, s, g);
+    return launch_ok("flash_window_backward");
+}
+
+template <typename T> static int run_forward(const Args& g, hipStream_t s) {
+    hipLaunchKernelGGL(flash_window_forward_kernel<T>, dim3((unsigned)(g.per_head * g.H)), dim3(WAVES * 64), (size_t)(WAVES * TURN + g.rows) * sizeof(float), s, g);
+    return launch_ok("flash_window_forward");
+}
+
+template <typename T> static int run_backward(Args g, float* delta, float* largest, float* d_table, hipStream_t s) {
+    const int64_t parts = g.N * g.H * (HD / 4);
+    const int blocks = (int)std::min<int64_t>(DELTA_BLOCKS, (parts + 1023) / 1024);
+    hipLaunchKernelGGL(flash_window_delta_kernel<T>, dim3(blocks), dim3(256), 0, s, static_cast<const T*>(g.dout), static_cast<const T*>(g.out), parts, delta, largest);
+    if (int rc = launch_ok("flash_window_backward, delta")) return rc;
+    g.delta = delta, g.largest = largest, g.n_largest = blocks;
+    if (!d_table) return launch_backward<T, false>(g, s);
+    if (int rc = launch_backward<T, true>(g, s)) return rc;
+    hipLaunchKernelGGL(flash_window_table_kernel, dim3((unsigned)((g.rows + 15) / 16), (unsigned)g.H), dim3(1024), 0, s, g.partial, g.per_head, g.rows, g.H, d_table);
+    return launch_ok("flash_window_backward, table");
+}
+
+}  // namespace window
+}  // namespace flash
+}  // namespace sswin
+
+using namespace sswin;
+using namespace sswin::flash;
+using namespace sswin::flash::window;
+
+static int window_args(const char* what, int dtype, const int32_t* plan, int64_t g_cap, int64_t groups, const int32_t* tokens, const int32_t* word,
+                       const int32_t* list, int64_t N, int H, int hd, int n, const void* qkv, float scale, const float* table, int rows, int offset0, void* out,
+                       float* lse, Args& g) {
+    SSWIN_CHECK(H > 0 && groups > 0 && groups <= g_cap && groups % H == 0 && offset0 >= 0 && sswin_flash_window_list_ints(dtype, N, H, hd, n, rows, groups / H),
+                "%s: not a shape it takes", what);
+    SSWIN_CHECK(plan && tokens && word && list && qkv && table && out && lse, "%s: null pointer", what);
+    SSWIN_CHECK(((uintptr_t)qkv | (uintptr_t)out) % 16 == 0, "%s: pointers must be 16-byte aligned", what);
+    g.plan = plan, g.g_cap = g_cap, g.order = tokens, g.word = reinterpret_cast<const uint32_t*>(word), g.list = list, g.N = N, g.windows = (int)(groups / H);
+    g.largest_v = reinterpret_cast<float*>(const_cast<int32_t*>(list)) + LIST_HEAD + g.windows, g.n_largest_v = per_head(g.windows, H, F_RESIDENT) * H;
+    g.H = H, g.rows = rows, g.offset4 = offset0 * 4, g.scale = scale, g.table = table, g.qkv = qkv, g.out = out, g.lse = lse;
+    return 0;
+}
+
+extern "C" {
+
+size_t sswin_flash_window_list_ints(int dtype, int64_t N, int H, int hd, int n, int rows, int64_t windows) {
+    return hd == HD && n <= MOST * 16 && H <= FORWARD_BLOCKS / 8 && windows > 0 && windows <= LIST_WINDOWS && sswin_flash_supported(dtype, N, H, hd, rows) && N * 3 * H * hd < 1ll << 30
+               ? (size_t)LIST_HEAD + windows + FORWARD_BLOCKS : 0;
+}
+
+int sswin_flash_window_tokens(const int32_t* plan, int64_t g_cap, int64_t groups, const int32_t* tokens, int64_t N, int H, int n, const int32_t* code,
+                              const int8_t* mask, int nmw, int32_t* word, int32_t* list, void* stream) {
+    SSWIN_CHECK(N > 0 && N < MAX_TOKENS && n > 0 && n <= MOST * 16 && H > 0 && groups > 0 && groups <= g_cap && groups % H == 0 && groups / H <= LIST_WINDOWS,
+                "flash_window_tokens: bad sizes");
+    SSWIN_CHECK(plan && tokens && code && word && list && (!mask || nmw > 0), "flash_window_tokens: null pointer");
+    const int windows = (int)(groups / H), per = LIST_THREADS / 64;
+    hipLaunchKernelGGL(flash_window_tokens_kernel, dim3((unsigned)(1 + (windows + per - 1) / per)), dim3(LIST_THREADS), 0, static_cast<hipStream_t>(stream), plan,
+                       g_cap, windows, H, tokens + 3 * N, code, mask, nmw, n, reinterpret_cast<uint32_t*>(word), list);
+    return launch_ok("flash_window_tokens");
+}
+
+int sswin_flash_window_forward(int dtype, const int32_t* plan, int64_t g_cap, int64_t groups, const int32_t* tokens, const int32_t* word, int32_t* list,
+                               int64_t N, int H, int hd, int n, const void* qkv, float scale, const float* table, int rows, int offset0, void* out, float* lse,
+                               void* stream) {
+    Args g = {};
+    if (int rc = window_args("flash_window_forward", dtype, plan, g_cap, groups, tokens, word, list, N, H, hd, n, qkv, scale, table, rows, offset0, out, lse, g))
+        return rc;
+    g.per_head = per_head(g.windows, H, F_RESIDENT);
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    if (dtype == SSWIN_F32) return run_forward<float>(g, s);
+    if (dtype == SSWIN_F16) return run_forward<__half>(g, s);
+    return run_forward<__hip_bfloat16>(g, s);
+}
+
+size_t sswin_flash_window_backward_workspace_bytes(int64_t N, int H, int rows, int64_t windows) {
+    Carver c(nullptr, 0);
+    c.take<float>((size_t)H * N);
+    c.take<float>(DELTA_BLOCKS);
+    c.take<float>((size_t)per_head((int)windows, H, B_RESIDENT) * H * rows);
+    return c.used;
+}
+
+int sswin_flash_window_backward(int dtype, const int32_t* plan, int64_t g_cap, int64_t groups, const int32_t* tokens, const int32_t* word, const int32_t* list,
+                                int64_t N, int H, int hd, int n, const void* qkv, float scale, const float* table, int rows, int offset0, const void* out,
+                                const float* lse, const void* dout, void* dqkv, float* d_table, void* ws, size_t ws_bytes, void* stream) {
+    Args g = {};
+    if (int rc = window_args("flash_window_backward", dtype, plan, g_cap, groups, tokens, word, list, N, H, hd, n, qkv, scale, table, rows, offset0,
+                             const_cast<void*>(out), const_cast<float*>(lse), g))
+        return rc;
+    SSWIN_CHECK(dout && dqkv && ws && ((uintptr_t)dout | (uintptr_t)dqkv) % 16 == 0, "flash_window_backward: gradients at 16 bytes and a workspace");
+    Carver c(ws, ws_bytes);
+    float* const delta = c.take<float>((size_t)H * N);
+    float* const largest = c.take<float>(DELTA_BLOCKS);
+    g.per_head = per_head(g.windows, H, B_RESIDENT);
+    g.partial = c.take<float>((size_t)g.per_head * H * rows);
+    SSWIN_CHECK(c.ok(), "flash_window_backward: workspace of %zu bytes, %zu are needed", ws_bytes, c.used);
+    g.dout = dout, g.dqkv = dqkv;
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    if (dtype == SSWIN_F32) return run_backward<float>(g, delta, largest, d_table, s);
+    if (dtype == SSWIN_F16) return run_backward<__half>(g, delta, largest, d_table, s);
+    return run_backward<__hip_bfloat16>(g, delta, largest, d_table, s);
+}
+
+}  // extern "C"

@@ -512,6 +512,19 @@ Tensor attention_forward(Attention& a, const Tensor& qkv, const Tensor& bias, At
     const auto fopt = qkv.options().dtype(at::kFloat);
     if (a.flash) {
         const Tensor table32 = saved.bias32 = bias.to(at::kFloat).contiguous();
+        const int64_t listed = (int64_t)sswin_flash_window_list_ints(dt, N, a.H, hd, a.n, (int)table32.size(0), tp.G / a.H);
+        if (listed) {                                                    // a wavefront a window and head
+            saved.words = at::empty({N + listed}, tp.tokens.options());
+            saved.aux = at::empty({a.H, N}, fopt);
+            Tensor o = at::empty({N, D}, qkv.options());
+            int32_t* const list = i32(saved.words) + N;
+            RUN_NAMED("sswin_flash_tokens", sswin_flash_window_tokens(i32(tp.plan), tp.g_cap, tp.G, i32(tp.tokens), N, a.H, a.n, i32(a.code),
+                                                                      a.mask.defined() ? a.mask.data_ptr<int8_t>() : nullptr, a.regions(), i32(saved.words), list, s));
+            RUN_NAMED("sswin_flash_forward", sswin_flash_window_forward(dt, i32(tp.plan), tp.g_cap, tp.G, i32(tp.tokens), i32(saved.words), list, N, a.H, hd, a.n,
+                                                                        ptr(qkv), (float)a.scale, f32(table32), (int)table32.size(0), a.offset0, ptr(o),
+                                                                        f32(saved.aux), s));
+            return o;
+        }
         const int64_t ordered = (int64_t)sswin_flash_order_ints(N, a.H);
         saved.words = at::empty({2 * N + ordered}, tp.tokens.options());
         int32_t* const order = ordered ? i32(saved.words) + 2 * N : nullptr;
@@ -593,6 +606,17 @@ Tensor attention_backward(const Attention& a, const Tensor& qkv, const Tensor& b
     void* s = current_stream(qkv);
     Tensor d_qkv = at::empty_like(qkv);
     const auto fopt = qkv.options().dtype(at::kFloat);
+    if (a.flash && sswin_flash_window_list_ints(dt, N, a.H, hd, a.n, (int)saved.bias32.size(0), tp.G / a.H)) {
+        const int rows = (int)saved.bias32.size(0);
+        Tensor d_table = want_bias ? at::empty({rows, a.H}, fopt) : Tensor();
+        const size_t nb = sswin_flash_window_backward_workspace_bytes(N, a.H, rows, tp.G / a.H);
+        Tensor ws = bytes(nb, qkv);
+        RUN_NAMED("sswin_flash_backward", sswin_flash_window_backward(dt, i32(tp.plan), tp.g_cap, tp.G, i32(tp.tokens), i32(saved.words), i32(saved.words) + N, N, a.H,
+                                                                      hd, a.n, ptr(qkv), (float)a.scale, f32(saved.bias32), rows, a.offset0, ptr(out),
+                                                                      f32(saved.aux), ptr(d_out), ptr(d_qkv), f32(d_table), ptr(ws), nb, s));
+        if (want_bias) d_bias = d_table.to(bias.scalar_type());
+        return d_qkv;
+    }
     if (a.flash) {
         Tensor d_s = want_bias ? at::empty({std::max<int64_t>(tp.A, 1)}, fopt) : Tensor(), delta = at::empty({a.H, N}, fopt);
         RUN_NAMED("sswin_flash_backward", sswin_flash_backward_ordered(dt, i32(tp.tokens), i32(saved.words), i32(saved.words) + N,
