@@ -1,0 +1,326 @@
+// What the attention kernels that take a window and head a wavefront have in common: the list of windows, the pieces of work of a workgroup, LDS and rows,
+// pairs of fp16 and their scales, the sums of the bias table's gradient.
+#pragma once
+
+#include <math.h>
+
+#include <algorithm>
+#include <type_traits>
+
+#include "flash_common.hpp"
+
+namespace sswin {
+namespace flash {
+namespace window {
+
+constexpr int WAVES = 4, MOST = 24;                                      // wavefronts of a workgroup; tiles of 16 tokens of a window
+constexpr int DELTA_BLOCKS = 1024, FORWARD_BLOCKS = 1024;
+constexpr int LIST_HEAD = 32, LIST_THREADS = 1024, LIST_WINDOWS = 16384;
+constexpr uint32_t INDEX = 0x7ffcu;                                      // of a difference of words: 4 row of the table
+constexpr int PITCH = 20, TURN = 16 * PITCH;                             // a 16 x 16 tile in LDS, values
+static_assert(MAX_ROWS * 4 <= 1 << 15, "codes and regions share a word");
+static_assert(MOST <= LIST_HEAD - 2, "the list's head counts windows by their tiles");
+
+struct Args {
+    const int32_t* plan;       // group table: [c | T | ..] of g_cap entries each, window k's groups at k H
+    int64_t g_cap;
+    const int32_t* order;      // voxel of token rank r
+    const uint32_t* word;      // 4 code | region << 15 | several regions in the window << 31 of token r
+    const int32_t* list;       // [t]: windows of more than t tiles; from LIST_HEAD on the windows, largest first
+    float* largest_v;          // [n_largest_v] largest |V| of the forward's workgroups
+    int n_largest_v;
+    int64_t N;
+    int windows, H, rows, offset4, per_head;
+    float scale;
+    const float* table;        // [rows, H]
+    const void* qkv;           // [N, 3 H hd] voxel rows
+    void* out;                 // [N, H hd]
+    float* lse;                // [H, N] by rank: offset + log2 of the row sum
+    // backward
+    const void* dout;          // [N, H hd]
+    const float* delta;        // [N, H]: dO . O
+    void* dqkv;                // [N, 3 H hd]
+    const float* largest;      // [n_largest] largest |dO| of some tokens
+    int n_largest;
+    float* partial;            // [H][per_head][rows] sums of dS by table row
+};
+
+// Workgroup -> head and place among the head's workgroups: the heads of the same windows follow each other on one XCD, whose L2 holds their rows
+__device__ __forceinline__ void place(int H, int& h, int& first) {
+    const int b = (int)blockIdx.x, y = b >> 3;
+    h = y % H;
+    first = y / H * 8 + (b & 7);
+}
+
+// The head's column of the bias table in units of log 2
+__device__ __forceinline__ void stage_table(const Args& g, int h, float* bias) {
+    constexpr int AT_ONCE = 9;                                           // of a thread, requested together: 13^3 rows
+    for (int r0 = threadIdx.x; r0 < g.rows; r0 += WAVES * 64 * AT_ONCE) {
+        float v[AT_ONCE];
+#pragma unroll
+        for (int i = 0; i < AT_ONCE; ++i) v[i] = g.table[(int64_t)min(r0 + i * WAVES * 64, g.rows - 1) * g.H + h];
+#pragma unroll
+        for (int i = 0; i < AT_ONCE; ++i)
+            if (r0 + i * WAVES * 64 < g.rows) bias[r0 + i * WAVES * 64] = v[i] * LOG2E;
+    }
+}
+
+// The pieces of work of a workgroup, as its wavefronts have them: every per_head-th of its head.  The largest windows come first, a workgroup
+// each; then those that two wavefronts hold, two at a time; then four at a time.  Lane l holds what is known of the l-th piece: list and plan are read
+// once, in front of the work.
+struct Task {
+    int team, rank, steps;     // wavefronts on the window, this one's number, tiles of the largest window among the workgroup's
+    int c, T, first, tiles;    // the window's tokens (0: nothing to do) and first rank, this wavefront's tiles
+};
+// TILES: of one wavefront; a window of up to 2 TILES has two, a larger one all four
+template <int TILES> struct Work {
+    int r0, left, at;          // first round in the lanes, rounds in them, lane of the next one
+    int own, team, steps, c, T;
+    // Rounds of pieces by descending size, every other one from behind: first come, first served would give the first workgroups the larger of every round
+    // (windows of 7^3: the longest wavefront of the backward 1.44 times the mean with 112 700 voxels fp32, 116 -> 102 us; 225 700 fp16 149 -> 143)
+    __device__ __forceinline__ void load(const Args& g) {
+        const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r = r0 + lane, u = r * g.per_head + (r & 1 ? g.per_head - 1 - own : own);
+        const int big = g.list[2 * TILES], two = g.list[TILES], pairs = (two - big + 1) / 2, total = big + pairs + (g.windows - two + WAVES - 1) / WAVES;
+        left = __builtin_popcountll(__ballot(u < total));
+        at = team = steps = c = T = 0;
+        if (u >= total) return;
+        int from, end;
+        if (u < big) team = 4, from = u, end = big;
+        else if (u < big + pairs) team = 2, from = big + 2 * (u - big), end = two;
+        else team = 1, from = two + WAVES * (u - big - pairs), end = g.windows;
+        const int window = from + wave / team;
+        const int64_t head = (int64_t)g.list[LIST_HEAD + from] * g.H, group = (int64_t)g.list[LIST_HEAD + min(window, g.windows - 1)] * g.H;
+        steps = (g.plan[head] + 15) >> 4;
+        c = window < end ? g.plan[group] : 0;
+        T = g.plan[g.g_cap + group];
+    }
+    __device__ __forceinline__ Work(const Args& g, int first) {
+        own = first, r0 = 0;
+        load(g);
+    }
+    __device__ __forceinline__ bool next(const Args& g, Task& t) {
+        if (at == 64) {
+            r0 += 64;
+            load(g);
+        }
+        if (at >= left) return false;
+        t.team = __builtin_amdgcn_readlane(team, at);
+        t.steps = __builtin_amdgcn_readlane(steps, at);
+        t.c = __builtin_amdgcn_readlane(c, at);
+        t.T = __builtin_amdgcn_readlane(T, at);
+        ++at;
+        const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), all = (t.c + 15) >> 4, shift = t.team >> 1, share = all >> shift,
+                  more = all - (share << shift);
+        t.rank = wave & (t.team - 1);
+        t.tiles = share + (t.rank < more ? 1 : 0);
+        t.first = t.rank * share + min(t.rank, more);
+        return true;
+    }
+};
+
+__device__ __forceinline__ f32x4 widened(const Frag<float>& f) { return f.v; }
+__device__ __forceinline__ f32x4 widened(const Frag<__half>& f) { return f32x4{(float)f.v[0], (float)f.v[1], (float)f.v[2], (float)f.v[3]}; }
+__device__ __forceinline__ f32x4 widened(const Frag<__hip_bfloat16>& f) {
+    const uint2 w = __builtin_bit_cast(uint2, f.v);
+    return f32x4{__builtin_bit_cast(float, w.x << 16), __builtin_bit_cast(float, w.x & 0xffff0000u), __builtin_bit_cast(float, w.y << 16),
+                 __builtin_bit_cast(float, w.y & 0xffff0000u)};
+}
+
+// a 16 x 16 tile turned through LDS of the wavefront's own: lane (row l % 16, columns 4 (l / 16) + j) -> lane (rows 4 (l / 16) + j, column l % 16)
+__device__ __forceinline__ f32x4 turned(float* tile, const f32x4& v) {
+    const int l16 = threadIdx.x & 15, quad = (threadIdx.x & 63) >> 4;
+    *reinterpret_cast<f32x4*>(tile + l16 * PITCH + quad * 4) = v;
+    f32x4 r;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) r[j] = tile[(quad * 4 + j) * PITCH + l16];
+    return r;
+}
+
+// over the four lanes l % 16, to all of them
+template <typename F> __device__ __forceinline__ float across(float v, F&& f) {
+    const auto a = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(uint32_t, v), __builtin_bit_cast(uint32_t, v), false, false);
+    v = f(__builtin_bit_cast(float, (uint32_t)a[0]), __builtin_bit_cast(float, (uint32_t)a[1]));
+    const auto b = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, v), __builtin_bit_cast(uint32_t, v), false, false);
+    return f(__builtin_bit_cast(float, (uint32_t)b[0]), __builtin_bit_cast(float, (uint32_t)b[1]));
+}
+__device__ __forceinline__ float across_max(float v) {
+    return across(v, [](float a, float b) { return fmaxf(a, b); });
+}
+__device__ __forceinline__ float across_sum(float v) {
+    return across(v, [](float a, float b) { return a + b; });
+}
+
+// LDS by its address: a word of a query less one of a key is the address of their bias
+typedef __attribute__((address_space(3))) float LdsFloat;
+typedef __attribute__((address_space(3))) unsigned long long LdsLong;
+__device__ __forceinline__ uint32_t lds_address(const void* p) { return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)p; }
+__device__ __forceinline__ float lds_float(uint32_t at) { return *(const LdsFloat*)(uintptr_t)at; }
+
+// Arrays through buffer descriptors: a lane's 32 bits of offset and one of all lanes, no 64-bit addresses in vector registers, and what is read behind
+// an array's end is 0 (the clamps of the last step's rows).
+typedef __amdgpu_buffer_rsrc_t Buffer;
+template <typename V> __device__ __forceinline__ Buffer buffer(const V* p, int64_t count) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<V*>(p), 0, (int)(uint32_t)(count * (int64_t)sizeof(V)), 0x00020000);
+}
+__device__ __forceinline__ uint32_t load1(const Buffer& b, uint32_t lane_bytes, uint32_t bytes) {
+    return __builtin_amdgcn_raw_buffer_load_b32(b, lane_bytes, bytes, 0);
+}
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ u32x4 load4(const Buffer& b, uint32_t lane_bytes, uint32_t bytes) {
+    return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(b, lane_bytes, bytes, 0));
+}
+// rows of the voxels' tokens: four of a head's channels a lane
+template <typename T> struct Rows {
+    Buffer b;
+    uint32_t pitch, col, own;  // bytes: a row, the head's first channel, the lane's first channel in it
+    __device__ __forceinline__ Rows(const void* p, int64_t N, int pitch_, int col_)
+        : b(buffer(static_cast<const T*>(p), N * pitch_)), pitch((uint32_t)pitch_ * (uint32_t)sizeof(T)), col((uint32_t)col_ * (uint32_t)sizeof(T)),
+          own(((threadIdx.x & 63) >> 4) * (uint32_t)(4 * sizeof(T))) {}
+    __device__ __forceinline__ void row(int v, Frag<T>& f) const {
+        const uint32_t at = __umul24((uint32_t)v, pitch) + own;
+        if constexpr (sizeof(T) == 4) f.v = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(b, at, col, 0));
+        else f.v = __builtin_bit_cast(decltype(f.v), __builtin_amdgcn_raw_buffer_load_b64(b, at, col, 0));
+    }
+    __device__ __forceinline__ void store(int v, const f32x4& x) const {
+        const uint32_t at = __umul24((uint32_t)v, pitch) + own;
+        if constexpr (sizeof(T) == 4) __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, x), b, at, col, 0);
+        else __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, packed<T>(x).v), b, at, col, 0);
+    }
+};
+template <typename T> __device__ __forceinline__ void keep(bool live, Frag<T>& f) {
+    if (!live) f = Frag<T>{};
+}
+// the largest |x| of a row's four values, 0 if one of them is infinite
+__device__ __forceinline__ float largest_finite(const f32x4& v) {
+    const float m = fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3])));
+    return m < INFINITY ? m : 0.f;
+}
+__device__ __forceinline__ float largest_of_workgroup(float m, float* part) {
+    for (int o = 1; o < 64; o <<= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = m;
+    __syncthreads();
+    m = part[0];
+#pragma unroll
+    for (int w = 1; w < WAVES; ++w) m = fmaxf(m, part[w]);
+    return m;
+}
+// 0, or NaN if one of them is not finite
+__device__ __forceinline__ float not_finite(const f32x4& v) { return fmaf(v[0], 0.f, fmaf(v[1], 0.f, fmaf(v[2], 0.f, v[3] * 0.f))); }
+
+// ------------------------------------------------------------------------------------------
+// D = dO . O of every voxel and head, HD / 4 lanes a head, and the largest |dO| (of what is finite) of a workgroup
+// ------------------------------------------------------------------------------------------
+template <typename T, int HD>
+__global__ __launch_bounds__(256) void flash_window_delta_kernel(const T* __restrict__ dout, const T* __restrict__ out, int64_t parts, float* __restrict__ delta,
+                                                                 float* __restrict__ largest) {
+    __shared__ float part[4];
+    constexpr int AT_ONCE = 4;
+    float most = 0.f;
+    for (int64_t i0 = (int64_t)blockIdx.x * 256 + threadIdx.x; i0 < parts; i0 += (int64_t)gridDim.x * 256 * AT_ONCE) {
+        Frag<T> x[AT_ONCE], y[AT_ONCE];
+#pragma unroll
+        for (int k = 0; k < AT_ONCE; ++k) {
+            const int64_t i = min(i0 + (int64_t)gridDim.x * 256 * k, parts - 1);
+            x[k].load(dout + i * 4), y[k].load(out + i * 4);
+        }
+#pragma unroll
+        for (int k = 0; k < AT_ONCE; ++k) {
+            const int64_t i = i0 + (int64_t)gridDim.x * 256 * k;
+            const f32x4 a = widened(x[k]), b = widened(y[k]);
+            float dot = 0.f;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) dot = fmaf(a[j], b[j], dot);
+            dot += dpp_f32<0xB1>(dot);
+            dot += dpp_f32<0x4E>(dot);
+            if constexpr (HD == 32) dot += dpp_f32<0x141>(dot);
+            most = fmaxf(most, largest_finite(a));
+            if (i < parts && (threadIdx.x & (HD / 4 - 1)) == 0) delta[i / (HD / 4)] = dot;
+        }
+    }
+    const float m = largest_of_workgroup(most, part);
+    if (threadIdx.x == 0) largest[blockIdx.x] = m;
+}
+
+// The unit of the table's sums.  Integers, so that the result does not depend on the order of the additions.  |dS| <= |dP| + |D| <= 2 HD largest |dO| largest |V| (P of a row adds up to at most one, up to rounding) < 2^top; dS
+// in units of 2^(top - bits) is a whole number below 2^50, and N of them below 2^62.
+template <int HD> struct Unit {
+    int top, bits;
+    __device__ __forceinline__ Unit(float mo, float mv, int64_t N) {
+        const int eo = mo > 0.f ? (int)ilogbf(mo) : -149, ev = mv > 0.f ? (int)ilogbf(mv) : -149;
+        top = eo + ev + (HD == 16 ? 8 : 9);
+        bits = min(50, 62 - (64 - __builtin_clzll((unsigned long long)N)));
+    }
+};
+
+// ------------------------------------------------------------------------------------------
+// Pieces.  P, dS and, of fp32 tokens, the rows are multiplied on the 16-bit matrix cores as x 2^e = h + l, h and l fp16 rounded to nearest, all
+// products of pieces kept but that of two l in dQ; sums are fp32.  22 bits of a value or 2^-25 in its scale, whichever is more, with fewer roundings of sums: error
+// against float64 (2-norms, windows of 7^3, fp32) dQ 5.4e-7 with fp32 products, 3.4e-7 here, dK 5.2 and 3.2, dV 5.0 and 3.0, table 5.2 and 4.1; 16-bit tokens: the
+// same to three digits.  A scale e is one of a wavefront: of K and V for the window, of Q and dO kept from step to step until a row no longer fits, when the
+// sums so far are scaled with it.  Rows too far below the largest for that, and windows in which something is not finite, are done with fp32 products
+// (How::exact), a whole window at a time.
+// ------------------------------------------------------------------------------------------
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+struct Pair {                  // x = h + l
+    f16x4 h, l;
+};
+__device__ __forceinline__ Pair split(const f32x4& x) {
+    typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+    struct Words { uint32_t a, b; };
+    Words h, l;
+    f16x2 h0 = {(_Float16)x[0], (_Float16)x[1]}, h1 = {(_Float16)x[2], (_Float16)x[3]};
+    asm("" : "+v"(h0), "+v"(h1));                                        // (or each half is converted again for its rest)
+    const f16x2 l0 = {(_Float16)fmaf(-1.f, (float)h0[0], x[0]), (_Float16)fmaf(-1.f, (float)h0[1], x[1])};
+    const f16x2 l1 = {(_Float16)fmaf(-1.f, (float)h1[0], x[2]), (_Float16)fmaf(-1.f, (float)h1[1], x[3])};
+    h = {__builtin_bit_cast(uint32_t, h0), __builtin_bit_cast(uint32_t, h1)};
+    l = {__builtin_bit_cast(uint32_t, l0), __builtin_bit_cast(uint32_t, l1)};
+    return Pair{__builtin_bit_cast(f16x4, h), __builtin_bit_cast(f16x4, l)};
+}
+__device__ __forceinline__ f16x8 both(const f16x4& a, const f16x4& b) { return __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7); }
+__device__ __forceinline__ f16x4 halves(const f32x4& x) { return packed<__half>(x).v; }
+__device__ __forceinline__ f32x4 mma32(const f16x8& a, const f16x8& b, const f32x4& c) { return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0); }
+__device__ __forceinline__ f32x4 mma16(const f16x4& a, const f16x4& b, const f32x4& c) { return __builtin_amdgcn_mfma_f32_16x16x16f16(a, b, c, 0, 0, 0); }
+
+// Powers of two that bring numbers into fp16's range: `e` for a largest value of [2^(12 - e), 2^(13 - e)), kept until it reaches 2^(15 - e)
+constexpr uint32_t NOT_FINITE = 0x7f800000u;
+__device__ __forceinline__ float power(int e) { return __builtin_bit_cast(float, (uint32_t)(127 + e) << 23); }
+__device__ __forceinline__ uint32_t largest4(const f32x4& v) {           // as bits, which grow with the absolute value
+    uint32_t m = 0;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const float x = v[j];                                            // (a bit cast of the element itself takes the first)
+        m = max(m, __builtin_bit_cast(uint32_t, x) & 0x7fffffffu);
+    }
+    return m;
+}
+__device__ __forceinline__ uint32_t over_quads(uint32_t m) {             // the largest of the four lanes l % 16
+    const auto a = __builtin_amdgcn_permlane16_swap(m, m, false, false);
+    m = max((uint32_t)a[0], (uint32_t)a[1]);
+    const auto b = __builtin_amdgcn_permlane32_swap(m, m, false, false);
+    return max((uint32_t)b[0], (uint32_t)b[1]);
+}
+__device__ __forceinline__ int over_rows(uint32_t m) {                   // of all lanes, once over_quads has been
+    m = m < NOT_FINITE ? m : 0;
+    return __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, row16_max(__builtin_bit_cast(float, m))));
+}
+__device__ __forceinline__ int scale_for(int largest, int most) { return largest == 0 ? most : max(-most, min(most, 12 + 127 - (largest >> 23))); }
+__device__ __forceinline__ bool too_large(uint32_t m, int e) { return m >= (uint32_t)(142 - e) << 23; }
+// pieces of a row whose largest value is below 2^(low - e) would lose bits of it
+template <typename T> __device__ __forceinline__ bool too_small(uint32_t m, int e) {
+    constexpr int low = sizeof(T) == 4 ? 0 : -6;
+    return m != 0 && m < (uint32_t)(127 + low - e) << 23;
+}
+
+// Workgroups of a head: as many as find a place at once, and no more than it has windows
+inline int per_head(int windows, int H, int resident) {
+    const int m = std::max(1, resident * device_cus() / (8 * H));
+    return std::min(8 * m, (windows + 7) / 8 * 8);
+}
+
+// d table [rows, H] from the workgroups' sums (flash_window.hip)
+int add_table(const float* partial, int per_head, int rows, int H, float* d_table, hipStream_t s);
+
+}  // namespace window
+}  // namespace flash
+}  // namespace sswin
