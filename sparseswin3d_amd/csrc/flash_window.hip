@@ -151,8 +151,8 @@ template <typename T> __global__ __launch_bounds__(WAVES * 64, F_RESIDENT) void 
             const f32x4 vw = widened(now.v);
             most = fmaxf(most, largest_finite(vw));
             const Frag<float> vt = {turned(turn, vw)};
-            auto tiles = [&](auto from_tag) __attribute__((always_inline)) {
-                constexpr int FROM = decltype(from_tag)::value, COUNT = 2;   // two at a time: one's exponentials beside the other's products
+            auto tiles = [&](auto from_tag, auto count_tag) __attribute__((always_inline)) {
+                constexpr int FROM = decltype(from_tag)::value, COUNT = decltype(count_tag)::value;   // two at a time: one's exponentials beside the other's products
                 float x[COUNT][4], xm[COUNT];
                 bool over = false;
 #pragma unroll
@@ -198,8 +198,13 @@ template <typename T> __global__ __launch_bounds__(WAVES * 64, F_RESIDENT) void 
                     o[t] = mma(vt, Frag<float>{p}, o[t]);
                 }
             };
-            tiles(std::integral_constant<int, 0>{});
-            if (count > 2) tiles(std::integral_constant<int, 2>{});
+            auto two = [&](auto from_tag) __attribute__((always_inline)) {
+                const int more = count - decltype(from_tag)::value;
+                if (more > 1) tiles(from_tag, std::integral_constant<int, 2>{});
+                else if (more > 0) tiles(from_tag, std::integral_constant<int, 1>{});
+            };
+            two(std::integral_constant<int, 0>{});
+            two(std::integral_constant<int, 2>{});
         }
 #pragma unroll
         for (int t = 0; t < F_TILES; ++t) {
@@ -445,8 +450,8 @@ template <typename T, bool TABLE> __global__ __launch_bounds__(WAVES * 64, B_RES
                     const float by_s = PAIRS ? power(eq + ek) : 1.f, by_p = PAIRS ? power(eo + ev) : 1.f, to_s = PAIRS ? scale2 * power(-eq - ek) : scale2,
                                 to_ds = PAIRS ? power(-18 - P_BITS) : power(es - P_BITS);
                     const f32x4 a0 = (now.lse - (float)P_BITS) * (-unscale * by_s), d0 = delta * -by_p;  // what the accumulators start from: P comes out times 2^P_BITS
-                    auto tiles = [&](auto from_tag) __attribute__((always_inline)) {
-                        constexpr int FROM = decltype(from_tag)::value, COUNT = 2;
+                    auto tiles = [&](auto from_tag, auto count_tag) __attribute__((always_inline)) {
+                        constexpr int FROM = decltype(from_tag)::value, COUNT = decltype(count_tag)::value;
                         f32x4 p[COUNT], ds[COUNT];
                         uint32_t at[COUNT][4];
 #pragma unroll
@@ -480,9 +485,16 @@ template <typename T, bool TABLE> __global__ __launch_bounds__(WAVES * 64, B_RES
                             dq = kt[t].times16(split(dst), dq);
                         }
                     };
-                    tiles(std::integral_constant<int, 0>{});
-                    if (task.tiles > 2) tiles(std::integral_constant<int, 2>{});
-                    if (task.tiles > 4) tiles(std::integral_constant<int, 4>{});
+                    // An odd last tile by itself where a tile is bound by what it issues: backward with the table's gradient, windows of 7^3, 112 700 tokens fp32 111 -> 106 us,
+                    // 225 700 214 -> 203.  16-bit tokens wait more than they issue, and a second form of the loop's body costs them 2 % (225 700 fp16 145 and 149).
+                    auto two = [&](auto from_tag) __attribute__((always_inline)) {
+                        const int more = task.tiles - decltype(from_tag)::value;
+                        if (more > 1 || (!PAIRS && more > 0)) tiles(from_tag, std::integral_constant<int, 2>{});
+                        else if (more > 0) tiles(from_tag, std::integral_constant<int, 1>{});
+                    };
+                    two(std::integral_constant<int, 0>{});
+                    two(std::integral_constant<int, 2>{});
+                    two(std::integral_constant<int, 4>{});
 #pragma unroll
                     for (int j = 0; j < 4; ++j) dq[j] = __builtin_amdgcn_ldexpf(dq[j], -es - ek);
                     ++done;
