@@ -8,10 +8,10 @@
 // in plain fp32 (plain_products).
 //
 // (dense_pairs.hip: layers of at least 96 reduction channels, with a workspace, as two fp16 pieces.)
-// dense_rows_kernel (fp32): a workgroup of WM wavefronts owns BM = 32 MT WM rows and 96 columns.  Both operands pass through
+// dense_rows_kernel (fp32): a workgroup of WM wavefronts owns BM = 32 MT WM rows and 32 NT columns, 64 or 96.  Both operands pass through
 // registers, where they are split, into LDS in matrix operand order, [row tile][plane][lane] pieces of 16 bytes, so that every
 // operand read is one conflict-free 16-byte read per lane; 32 columns of the reduction at a time, the next 32 in flight
-// meanwhile.  96 columns because every layer of a stage has a multiple of 48.  The tile of the result goes back
+// meanwhile.  96 columns because every layer of a stage has a multiple of 48, 64 where that wastes no more of them.  The tile of the result goes back
 // through LDS, so that bias, residual and result are touched in 16-byte pieces of whole row segments.
 // dense16_rows_kernel (16 bit): tiles straight from memory to LDS.
 // dense_small_kernel: few rows and many channels (the deep stages): 32 x 32 tiles, the wavefronts of a workgroup share
@@ -94,11 +94,11 @@ __device__ __forceinline__ int swz(int chunk) { return (chunk & 1) * 4 | (chunk 
 // ------------------------------------------------------------------------------------------
 // y [N, P] = last step of x [N, K] Wop, Wop [K, P] = W^T of W [P, K] (DOWN = false) or W [K, P] itself (DOWN = true)
 // ------------------------------------------------------------------------------------------
-template <int EPI, bool DOWN, int WM, int MT, int OCC>
+template <int EPI, bool DOWN, int WM, int MT, int NT, int OCC>
 __global__ __launch_bounds__(WM * 64) __attribute__((amdgpu_waves_per_eu(OCC, OCC))) void dense_rows_kernel(
     const float* __restrict__ x, int64_t N, int K, const float* __restrict__ w, int P, int groups, Epilogue ep) {
     constexpr int PL = 3, BK = 32, KC = BK / 8;
-    constexpr int NT = 3, BN = 96, BM = WM * MT * 32, THREADS = WM * 64;
+    constexpr int BN = NT * 32, BM = WM * MT * 32, THREADS = WM * 64;
     constexpr int A_UNITS = BM * KC, UA = (A_UNITS + THREADS - 1) / THREADS;
     constexpr int B_UNITS = (DOWN ? BN / 2 : BN) * KC, UB = (B_UNITS + THREADS - 1) / THREADS;
     constexpr int A_LDS = BM / 32 * PL * 64, B_LDS = NT * PL * 64;       // 16-byte pieces of 16 columns
@@ -984,15 +984,15 @@ static int launch_parts(const float* part, int64_t N, int P, int parts, const Ep
     return launch_ok("dense, parts");
 }
 
-template <int EPI, bool DOWN, int WM, int MT, int OCC>
+template <int EPI, bool DOWN, int WM, int MT, int NT, int OCC>
 static int launch_rows(const float* x, int64_t N, int K, const float* w, int P, const Epilogue& ep, hipStream_t s) {
     constexpr int BM = WM * MT * 32;
-    constexpr size_t tiles = 2 * (size_t)(BM / 32 + 3) * 3 * 64 * 16, out = (size_t)WM * 32 * 100 * 4;
+    constexpr size_t tiles = 2 * (size_t)(BM / 32 + NT) * 3 * 64 * 16, out = (size_t)WM * 32 * (NT * 32 + 4) * 4;
     constexpr size_t bytes = tiles > out ? tiles : out;
-    auto* k = dense_rows_kernel<EPI, DOWN, WM, MT, OCC>;
+    auto* k = dense_rows_kernel<EPI, DOWN, WM, MT, NT, OCC>;
     static const int configured = allow_lds(k, bytes);
     if (configured) return configured;
-    const int groups = (P + 95) / 96;
+    const int groups = (P + NT * 32 - 1) / (NT * 32);
     const int64_t blocks = (N + BM - 1) / BM * groups;
     SSWIN_CHECK(blocks < (1ll << 31), "dense: too many rows");
     hipLaunchKernelGGL(k, dim3((unsigned)blocks), dim3(WM * 64), bytes, s, x, N, K, w, P, groups, ep);
@@ -1085,8 +1085,14 @@ static int launch_forward(const void* x, int64_t N, int K, const void* w, int P,
         // The launch for W costs up to 2 us where tiles and reduction are few (three pieces and pairs, us): 9563 rows 112 -> 192 11.0 and 12.4, 4187 rows 144 -> 576
         // 12.5 and 13.6, 32 700 rows 144 -> 48 turned 13.3 and 14.0, 16 300 rows 192 -> 192 15.0 and 15.4; from 288 reduction channels on pairs are ahead everywhere.
         if (apart && pairs_takes(K) && ws_bytes >= pairs_workspace_bytes(K, P)) return pairs_layer<EPI, DOWN>(xp, N, K, wp, P, ep, ws, s);
-        // wavefronts per SIMD: what the registers allow without spilling (four: forward equal, input gradient 89 us against 40)
-        return launch_rows<EPI, DOWN, 4, 1, 3>(xp, N, K, wp, P, ep, s);
+        // 64 columns a workgroup and four wavefronts a SIMD, or 96 and three (what the registers allow without spilling).  Bound by the waits between request,
+        // splitting and products of two or three short steps, so that the fourth wavefront counts, and by columns that a tile does not use.  96 -> 64, us, 112 700
+        // rows from memory: 48 -> 48 19.7 -> 14.1, turned 17.4 -> 13.5, 48 -> 144 34.5 -> 32.6, 80 -> 48 25.7 -> 18.1; from the last-level cache: 48 -> 96 12.8 and
+        // 12.4, 48 -> 128 17.4 -> 12.5, 80 -> 240 37.4 -> 33.3; with a residual 48 -> 96 20.7 -> 17.3, 80 -> 288 52.3 and 50.2.  Where 96 cover P with fewer columns and
+        // there is no second operand they stay ahead: 48 -> 288 30.3 and 31.2, turned 26.7 and 28.2.  In place a workgroup has to hold whole rows.
+        const bool wide = P > 96 && (P + 63) / 64 * 64 > (P + 95) / 96 * 96 && !Second4<float, float, EPI>::USED;
+        if (apart && K < 96 && !wide) return launch_rows<EPI, DOWN, 4, 1, 2, 4>(xp, N, K, wp, P, ep, s);
+        return launch_rows<EPI, DOWN, 4, 1, 3, 3>(xp, N, K, wp, P, ep, s);
     } else {
         if (ws_bytes < (size_t)cut.ksplit * N * P * sizeof(float)) cut.ksplit = 1;
         const int64_t rows = (N + 127) / 128, tiles = rows * ((P + 95) / 96) * cut.ksplit;

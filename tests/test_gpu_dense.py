@@ -128,6 +128,14 @@ def test_dense_forward_of_long_reductions(N, K, P, dtype, out):
     test_dense_forward_and_input_gradient(N, P, K, dtype, out)
 
 
+# fp32, fewer than 96 reduction channels: 64 columns a workgroup, or 96 where those cover the layer with fewer (272, 288; not with a second operand);
+# parts of a tile, whole ones and one piece more; half steps of the reduction
+@pytest.mark.parametrize("N,K", [(19201, 48), (19230, 80), (19313, 16)])
+@pytest.mark.parametrize("P", [16, 48, 64, 80, 96, 112, 128, 144, 192, 272, 288, 304])
+def test_dense_fp32_forward_of_short_reductions(N, K, P):
+    test_dense_forward_and_input_gradient(N, K, P, torch.float32, torch.float32)
+
+
 # a result in the place of its rows, where one workgroup of a tile holds them whole (96 columns at most, more rows than the few-rows kernel takes)
 @pytest.mark.parametrize("K", [48, 96])
 def test_dense_forward_in_place(K):
