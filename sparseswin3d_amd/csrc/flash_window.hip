@@ -13,7 +13,7 @@
 // rows on the 16-bit matrix cores.  The table's gradient is summed by 64-bit integer additions in LDS, which take 10 clocks a wavefront's 64
 // (floating-point ones 180: what kept the sums out of the backward), and whose result does not depend on their order.
 //
-// Windows of 7^3, 3 heads of 16, us, blocks -> here: 112 700 tokens fp32 forward 56 -> 50, backward with the table's gradient 214 -> 103; 225 700 fp16 80 -> 70
+// Windows of 7^3, 3 heads of 16, us, blocks -> here: 112 700 tokens fp32 forward 56 -> 50, backward with the table's gradient 214 -> 103; 225 700 fp16 80 -> 65
 // and 348 -> 141; 8100 tokens in 50 nearly full windows, 24 heads, fp16: 60 and 124 here.  A tile takes a SIMD of the backward about 700 clocks
 // (fp32) and 900 (fp16: 225 700 tokens), 300 of them instructions it issues: two wavefronts a SIMD, held there by their registers, wait for each other's rows,
 // transpositions and exponentials; a fourth of the time is in front of the first step of a window.
