@@ -101,9 +101,12 @@ template <> struct Column<float> {
 // ------------------------------------------------------------------------------------------
 // forward: a wavefront holds the queries of its tiles and walks over the window's keys, 16 at a time
 // ------------------------------------------------------------------------------------------
-constexpr int F_TILES = 4, F_RESIDENT = 3;                               // tiles of queries of a wavefront at a time; wavefronts a SIMD
+constexpr int F_TILES = 4;                                               // tiles of queries of a wavefront at a time
+// Wavefronts a SIMD.  Three and four at 16 bit, with the words, us: 112 700 tokens fp16 47.6 and 42, bf16 47.9 and 45; 225 700 73.8 and 71.9, 80.2 and 76.6
+// (24 bytes a lane of the fp16 kernel spilled); fp32 needs 147 registers.
+constexpr int forward_resident(size_t value) { return value == 4 ? 3 : 4; }
 
-template <typename T> __global__ __launch_bounds__(WAVES * 64, F_RESIDENT) void flash_window_forward_kernel(Args g) {
+template <typename T> __global__ __launch_bounds__(WAVES * 64, forward_resident(sizeof(T))) void flash_window_forward_kernel(Args g) {
     extern __shared__ __attribute__((aligned(16))) char lds[];
     const int lane = threadIdx.x & 63, l16 = lane & 15, quad = lane >> 4, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     float* const turn = reinterpret_cast<float*>(lds) + wave * TURN;
@@ -219,8 +222,12 @@ template <typename T> __global__ __launch_bounds__(WAVES * 64, F_RESIDENT) void 
 #pragma unroll
                     for (int j = 0; j < 4; ++j) p[j] = __builtin_amdgcn_exp2f(x[i][j]);
                     sum[t] += (p[0] + p[1]) + (p[2] + p[3]);
-                    if (HALVES && plain) o[t] = vh.times(split(p), o[t]);
-                    else o[t] = mma(vt, Frag<float>{p}, o[t]);
+                    if constexpr (HALVES) {
+                        if (plain) o[t] = vh.times(split(p), o[t]);
+                        else o[t] = mma(Frag<float>{widened(Frag<__half>{vh.h})}, Frag<float>{p}, o[t]);
+                    } else {
+                        o[t] = mma(vt, Frag<float>{p}, o[t]);
+                    }
                 }
             };
             auto two = [&](auto from_tag) __attribute__((always_inline)) {
@@ -669,6 +676,13 @@ using namespace sswin;
 using namespace sswin::flash;
 using namespace sswin::flash::window;
 
+// Where most windows are a workgroup's, no more workgroups than the same number of rounds takes: the others would only share its SIMD (8100 tokens in 50
+// nearly full windows, 24 heads: 40 workgroups a head 71.7 us, 32 67)
+static int forward_per_head(int dtype, int64_t N, int windows, int H) {
+    const int m = per_head(windows, H, forward_resident(dtype == SSWIN_F32 ? 4 : 2)), rounds = (windows + m - 1) / m;
+    return N <= (int64_t)windows * 2 * F_TILES * 16 ? m : ((windows + rounds - 1) / rounds + 7) / 8 * 8;
+}
+
 static int window_args(const char* what, int dtype, const int32_t* plan, int64_t g_cap, int64_t groups, const int32_t* tokens, const int32_t* word,
                        const int32_t* list, int64_t N, int H, int hd, int n, const void* qkv, float scale, const float* table, int rows, int offset0, void* out,
                        float* lse, Args& g) {
@@ -677,7 +691,7 @@ static int window_args(const char* what, int dtype, const int32_t* plan, int64_t
     SSWIN_CHECK(plan && tokens && word && list && qkv && table && out && lse, "%s: null pointer", what);
     SSWIN_CHECK(((uintptr_t)qkv | (uintptr_t)out) % 16 == 0, "%s: pointers must be 16-byte aligned", what);
     g.plan = plan, g.g_cap = g_cap, g.order = tokens, g.word = reinterpret_cast<const uint32_t*>(word), g.list = list, g.N = N, g.windows = (int)(groups / H);
-    g.largest_v = reinterpret_cast<float*>(const_cast<int32_t*>(list)) + LIST_HEAD + g.windows, g.n_largest_v = per_head(g.windows, H, F_RESIDENT) * H;
+    g.largest_v = reinterpret_cast<float*>(const_cast<int32_t*>(list)) + LIST_HEAD + g.windows, g.n_largest_v = forward_per_head(dtype, N, g.windows, H) * H;
     g.H = H, g.rows = rows, g.offset4 = offset0 * 4, g.scale = scale, g.table = table, g.qkv = qkv, g.out = out, g.lse = lse;
     return 0;
 }
@@ -706,7 +720,7 @@ int sswin_flash_window_forward(int dtype, const int32_t* plan, int64_t g_cap, in
     Args g = {};
     if (int rc = window_args("flash_window_forward", dtype, plan, g_cap, groups, tokens, word, list, N, H, hd, n, qkv, scale, table, rows, offset0, out, lse, g))
         return rc;
-    g.per_head = per_head(g.windows, H, F_RESIDENT);
+    g.per_head = forward_per_head(dtype, N, g.windows, H);
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (dtype == SSWIN_F32) return run_forward<float>(g, s);
     if (dtype == SSWIN_F16) return run_forward<__half>(g, s);
