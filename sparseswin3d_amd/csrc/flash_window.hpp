@@ -182,10 +182,12 @@ template <typename T> struct Rows {
         if constexpr (sizeof(T) == 4) f.v = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(b, at, col, 0));
         else f.v = __builtin_bit_cast(decltype(f.v), __builtin_amdgcn_raw_buffer_load_b64(b, at, col, 0));
     }
+    // The whole offset in the lane's register.  With a part of it in a scalar one the compiler puts no wait between a store of 16 bytes and an instruction that
+    // writes the registers it stores, and the new value is what arrives (heads of 32 once stored so: 1 value of 1000 was that of the next 16 channels).
     __device__ __forceinline__ void store(int v, const f32x4& x) const {
-        const uint32_t at = __umul24((uint32_t)v, pitch) + own;
-        if constexpr (sizeof(T) == 4) __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, x), b, at, col, 0);
-        else __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, packed<T>(x).v), b, at, col, 0);
+        const uint32_t at = __umul24((uint32_t)v, pitch) + (own + col);
+        if constexpr (sizeof(T) == 4) __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, x), b, at, 0, 0);
+        else __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, packed<T>(x).v), b, at, 0, 0);
     }
 };
 template <typename T> __device__ __forceinline__ void keep(bool live, Frag<T>& f) {

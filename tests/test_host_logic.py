@@ -101,3 +101,30 @@ def test_sparse_tensor_index_matrix_on_demand():
     assert eager.indices is matrix and eager.index_source() is matrix and eager.row_positions is None
     eager.indices = matrix + 1
     assert torch.equal(eager.indices, matrix + 1)
+
+
+def _device_sources():
+    import glob
+    import os
+    here = os.path.join(os.path.dirname(__file__), "..", "sparseswin3d_amd", "csrc")
+    return {os.path.basename(p): open(p).read() for pattern in ("*.hip", "*.hpp") for p in sorted(glob.glob(os.path.join(here, pattern)))}
+
+
+def test_wide_buffer_stores_keep_their_offset_in_the_lanes_register():
+    """hipcc puts no wait between a buffer store of 12 or 16 bytes that takes an offset from a scalar register and an instruction that writes the
+    registers it stores; gfx950 then stores the new values now and then.  Without that offset it does."""
+    import re
+    seen = 0
+    for name, text in _device_sources().items():
+        for m in re.finditer(r"raw_buffer_store_b(?:96|128)\(", text):
+            depth, at, args, start = 1, m.end(), [], m.end()
+            while depth:
+                c = text[at]
+                depth += (c in "([{") - (c in ")]}")
+                if (c == "," and depth == 1) or depth == 0:
+                    args.append(text[start:at].strip())
+                    start = at + 1
+                at += 1
+            assert len(args) == 5 and args[3] == "0", (name, args)
+            seen += 1
+    assert seen
