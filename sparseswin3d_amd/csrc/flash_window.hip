@@ -432,7 +432,9 @@ template <typename T, bool TABLE> __global__ __launch_bounds__(WAVES * 64, B_RES
                 }
                 const f32x4 qw = widened(now.q), ow = widened(now.d_o);
                 if (quad == 0) deltas[l16] = now.delta;
+                lanes_meet();
                 const f32x4 delta = *reinterpret_cast<const f32x4*>(deltas + quad * 4);   // of the rows of an accumulator
+                lanes_meet();
                 uint32_t pq[4];
 #pragma unroll
                 for (int j = 0; j < 4; ++j) pq[j] = (now.w[j] & KEPT) + (uint32_t)g.offset4 + (MASK ? 0 : bias_at);

@@ -126,13 +126,18 @@ __device__ __forceinline__ f32x4 widened(const Frag<__hip_bfloat16>& f) {
                  __builtin_bit_cast(float, w.y & 0xffff0000u)};
 }
 
+// Between a store to LDS of the wavefront's own and what other lanes read there, and the other way round: no instruction, but the compiler, which sees a
+// lane's own addresses alone, exchanges nothing across it
+__device__ __forceinline__ void lanes_meet() { __builtin_amdgcn_wave_barrier(); }
 // a 16 x 16 tile turned through LDS of the wavefront's own: lane (row l % 16, columns 4 (l / 16) + j) -> lane (rows 4 (l / 16) + j, column l % 16)
 __device__ __forceinline__ f32x4 turned(float* tile, const f32x4& v) {
     const int l16 = threadIdx.x & 15, quad = (threadIdx.x & 63) >> 4;
     *reinterpret_cast<f32x4*>(tile + l16 * PITCH + quad * 4) = v;
+    lanes_meet();
     f32x4 r;
 #pragma unroll
     for (int j = 0; j < 4; ++j) r[j] = tile[(quad * 4 + j) * PITCH + l16];
+    lanes_meet();
     return r;
 }
 

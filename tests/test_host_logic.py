@@ -128,3 +128,12 @@ def test_wide_buffer_stores_keep_their_offset_in_the_lanes_register():
             assert len(args) == 5 and args[3] == "0", (name, args)
             seen += 1
     assert seen
+
+
+def test_what_lanes_hand_each_other_through_lds_is_ordered():
+    """A wavefront's exchange through LDS: store, barrier, loads, barrier.  The compiler sees the addresses of one lane alone."""
+    import re
+    files = _device_sources()
+    body = re.search(r"f32x4 turned\(float\* tile.*?\n}", files["flash_window.hpp"], re.S)[0]
+    assert re.search(r"= v;\s*lanes_meet\(\);.*r\[j\] = tile.*lanes_meet\(\);\s*return r", body, re.S)
+    assert re.search(r"deltas\[l16\] = [^;]*;\s*lanes_meet\(\);\s*[^;]*deltas \+[^;]*;[^\n]*\s*lanes_meet\(\);", files["flash_window.hip"])
