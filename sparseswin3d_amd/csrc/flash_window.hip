@@ -84,18 +84,34 @@ __global__ __launch_bounds__(LIST_THREADS) void flash_window_tokens_kernel(const
     }
 }
 
-// What a wavefront multiplies with all pairs of another operand: 16-bit tokens are one piece, fp32 tokens two
+// What a wavefront multiplies with P or dS: rows turned, 16-bit tokens one piece, fp32 tokens two
 template <typename T> struct Column {
-    f16x4 h;
-    __device__ __forceinline__ void set(const f32x4& x) { h = halves(x); }
-    __device__ __forceinline__ f32x4 times(const Pair& p, f32x4 c) const { return mma32(both(h, h), both(p.h, p.l), c); }
-    __device__ __forceinline__ f32x4 times16(const Pair& p, f32x4 c) const { return mma16(h, p.l, mma16(h, p.h, c)); }
+    f16x8 h;
+    __device__ __forceinline__ void set(const f32x4& x) { h = with_rest(halves(x)); }
+    __device__ __forceinline__ f32x4 times(const Fine& p, const f32x4& c) const { return mma32(h, both(p), c); }
 };
 template <> struct Column<float> {
-    Pair x;
-    __device__ __forceinline__ void set(const f32x4& v) { x = split(v); }
-    __device__ __forceinline__ f32x4 times(const Pair& p, f32x4 c) const { return mma32(both(x.l, x.l), both(p.h, p.l), mma32(both(x.h, x.h), both(p.h, p.l), c)); }
-    __device__ __forceinline__ f32x4 times16(const Pair& p, f32x4 c) const { return mma16(x.l, p.h, mma16(x.h, p.l, mma16(x.h, p.h, c))); }
+    f16x8 h, l;
+    __device__ __forceinline__ void set(const f32x4& v) {
+        const Pair x = split(v);
+        h = with_rest(x.h), l = with_rest(x.l);
+    }
+    __device__ __forceinline__ f32x4 times(const Fine& p, const f32x4& c) const { return mma32(l, both(p), mma32(h, both(p), c)); }
+};
+// The same held for a whole window, in half the registers: the parts of a sum, the second in units of 1 / REST
+struct Sum {
+    f32x4 a, b;
+    __device__ __forceinline__ f32x4 total() const { return a + b * (1.f / REST); }
+};
+template <typename T> struct Held {
+    f16x4 h;
+    __device__ __forceinline__ void set(const f32x4& x) { h = halves(x); }
+    __device__ __forceinline__ void add(const Fine& p, Sum& s) const { s.a = mma16(h, p.h, s.a), s.b = mma16(h, p.l, s.b); }
+};
+template <> struct Held<float> {
+    Fine x;
+    __device__ __forceinline__ void set(const f32x4& v) { x = split_fine(v); }
+    __device__ __forceinline__ void add(const Fine& p, Sum& s) const { s.a = mma16(x.h, p.h, s.a), s.b = mma32(both(x.h, x.l), both(p.l, p.h), s.b); }
 };
 
 // ------------------------------------------------------------------------------------------
@@ -170,7 +186,7 @@ template <typename T> __global__ __launch_bounds__(WAVES * 64, forward_resident(
             most = fmaxf(most, largest_finite(vw));
             const Frag<float> vt = {turned(turn, vw)};
             // fp16 tokens: V is a piece as it is and P two, one product of 16 clocks where fp32 takes 128 (225 700 tokens with the words 79.7 -> 73.5 us, 37 200 in 6
-            // heads 42.0 -> 39.5).  P is at most 2^10 and keeps 22 bits, or 2^-25, of which a result of 11 bits shows nothing.  The second piece of P may be zero
+            // heads 42.0 -> 39.5).  P is at most 2^10 and keeps 22 bits, or 2^-36, of which a result of 11 bits shows nothing.  The second piece of P may be zero
             // or negative: infinities meet P itself.
             Column<T> vh;
             bool plain = false;
@@ -223,8 +239,8 @@ template <typename T> __global__ __launch_bounds__(WAVES * 64, forward_resident(
                     for (int j = 0; j < 4; ++j) p[j] = __builtin_amdgcn_exp2f(x[i][j]);
                     sum[t] += (p[0] + p[1]) + (p[2] + p[3]);
                     if constexpr (HALVES) {
-                        if (plain) o[t] = vh.times(split(p), o[t]);
-                        else o[t] = mma(Frag<float>{widened(Frag<__half>{vh.h})}, Frag<float>{p}, o[t]);
+                        if (plain) o[t] = vh.times(split_fine(p), o[t]);
+                        else o[t] = mma(Frag<float>{widened(Frag<__half>{__builtin_shufflevector(vh.h, vh.h, 0, 1, 2, 3)})}, Frag<float>{p}, o[t]);
                     } else {
                         o[t] = mma(vt, Frag<float>{p}, o[t]);
                     }
@@ -286,8 +302,8 @@ template <> struct Row<float> {
 // ------------------------------------------------------------------------------------------
 constexpr int B_RESIDENT = 2;                                            // wavefronts a SIMD
 constexpr int WAVE_LDS = 3 * TURN + 16;                                  // of a wavefront: three tiles to turn, D of 16 queries
-// P is multiplied by 2^P_BITS: its pieces then hold it to 2^-31, and exponents lie around zero, where fp32 rounds them least
-constexpr int P_BITS = 7;
+// P is formed times 2^P_BITS, so that exponents lie around zero, where fp32 rounds them least, and split times 2^P_MORE on top: 22 bits of it down to 2^-28, and 2^-50
+constexpr int P_BITS = 7, P_MORE = 7;
 // Steps between two meetings of a window's wavefronts.  At every step 143 us (225 700 tokens fp16) and 130 (8100 in nearly full windows), every other one 142 and
 // 126, at every fourth 141 and 124; fp32 within 2 % of each other.
 constexpr int GROUP = 4;
@@ -344,7 +360,7 @@ template <typename T, bool TABLE> __global__ __launch_bounds__(WAVES * 64, B_RES
         constexpr uint32_t KEPT = MASK ? 0x7fffffffu : INDEX;            // of a word
         const int c = task.c, T0 = task.T, all = (c + 15) >> 4;
         Row<T> k[KT], v[KT];
-        Column<T> kt[KT];
+        Held<T> kt[KT];
         f32x4 dk[KT], dv[KT];
         uint32_t pk[KT];
         int vk[KT];
@@ -412,6 +428,7 @@ template <typename T, bool TABLE> __global__ __launch_bounds__(WAVES * 64, B_RES
 #pragma clang loop unroll(disable)
         for (int s = 0; s < steps; ++s) {
             f32x4 dq = {0.f, 0.f, 0.f, 0.f};
+            Sum dq_sum = {dq, dq};
             int voxel = 0;
             if (s < all) {
                 Strip now = ahead;
@@ -501,9 +518,9 @@ template <typename T, bool TABLE> __global__ __launch_bounds__(WAVES * 64, B_RES
                         for (int i = 0; i < COUNT; ++i) {
                             const int t = FROM + i;
                             const f32x4 dst = turned(turn + i * TURN, ds[i]);
-                            dv[t] = dot.times(split(p[i]), dv[t]);
-                            dk[t] = qt.times(split(ds[i]), dk[t]);
-                            dq = kt[t].times16(split(dst), dq);
+                            dv[t] = dot.times(split_fine<P_MORE>(p[i]), dv[t]);
+                            dk[t] = qt.times(split_fine(ds[i]), dk[t]);
+                            kt[t].add(split_fine(dst), dq_sum);
                         }
                     };
                     // An odd last tile by itself where a tile is bound by what it issues: backward with the table's gradient, windows of 7^3, 112 700 tokens fp32 111 -> 106 us,
@@ -517,7 +534,7 @@ template <typename T, bool TABLE> __global__ __launch_bounds__(WAVES * 64, B_RES
                     two(std::integral_constant<int, 2>{});
                     two(std::integral_constant<int, 4>{});
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) dq[j] = __builtin_amdgcn_ldexpf(dq[j], -es - ek);
+                    for (int j = 0; j < 4; ++j) dq[j] = __builtin_amdgcn_ldexpf(dq_sum.total()[j], -es - ek);
                     ++done;
                   }
                 } else {
@@ -587,7 +604,7 @@ template <typename T, bool TABLE> __global__ __launch_bounds__(WAVES * 64, B_RES
                 dq_rows.store(voxels[i], sum * g.scale);
             }
         }
-        const int sk = EXACT ? 0 : -(eo + ev - 18) - (SCALED ? eq : 0), sv = EXACT ? 0 : -P_BITS - (SCALED ? eo : 0);
+        const int sk = EXACT ? 0 : -(eo + ev - 18) - (SCALED ? eq : 0), sv = EXACT ? 0 : -P_BITS - P_MORE - (SCALED ? eo : 0);
 #pragma unroll
         for (int t = 0; t < KT; ++t)
             if (t < task.tiles && (task.first + t) * 16 + l16 < c) {

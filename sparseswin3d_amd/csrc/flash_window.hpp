@@ -261,12 +261,14 @@ template <int HD> struct Unit {
 };
 
 // ------------------------------------------------------------------------------------------
-// Pieces.  P, dS and, of fp32 tokens, the rows are multiplied on the 16-bit matrix cores as x 2^e = h + l, h and l fp16 rounded to nearest, all
-// products of pieces kept but that of two l in dQ; sums are fp32.  22 bits of a value or 2^-25 in its scale, whichever is more, with fewer roundings of sums: error
-// against float64 (2-norms, windows of 7^3, fp32) dQ 5.4e-7 with fp32 products, 3.4e-7 here, dK 5.2 and 3.2, dV 5.0 and 3.0, table 5.2 and 4.1; 16-bit tokens: the
-// same to three digits.  A scale e is one of a wavefront: of K and V for the window, of Q and dO kept from step to step until a row no longer fits, when the
-// sums so far are scaled with it.  Rows too far below the largest for that, and windows in which something is not finite, are done with fp32 products
-// (How::exact), a whole window at a time.
+// Pieces.  P, dS and, of fp32 tokens, the rows are multiplied on the 16-bit matrix cores as pairs of fp16 rounded to nearest, products of two second pieces left
+// out of dQ alone; sums are fp32.  Rows are x 2^e = h + l, 22 bits or 2^-25 in their scale, whichever is more.  A scale e is one of a wavefront: of K and V for
+// the window, of Q and dO kept from step to step until a row no longer fits, when the sums so far are scaled with it.  Rows too far below the largest for
+// that, and windows in which something is not finite, are done with fp32 products (How::exact), a whole window at a time.
+// P and dS have no scale of their own, and a row of dS is as much smaller than another as its row of dO, or as its P: x = h + l 2^-11, 22 bits down to 2^-14 and 2^-36 below that.
+// (with the pieces of a row for them, 22 bits or 2^-25 in a window's scale, dQ of a query whose dO is 2^-9 of the window's largest was off by 1.6e-5).  Error of a
+// row against float64, its norm, median, windows of 7^3, fp32: dQ 6.4e-7 with fp32 products, 2.8e-7 here, dK 6.3 and 3.4, dV 6.2 and 3.3, the same for rows of dO 2^-9 of the
+// others and for mask regions that hold nothing else; the table's gradient, by head, 5.7 and 3.0.  16-bit tokens: the rounding of the result alone.
 // ------------------------------------------------------------------------------------------
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 struct Pair {                  // x = h + l
@@ -284,7 +286,28 @@ __device__ __forceinline__ Pair split(const f32x4& x) {
     l = {__builtin_bit_cast(uint32_t, l0), __builtin_bit_cast(uint32_t, l1)};
     return Pair{__builtin_bit_cast(f16x4, h), __builtin_bit_cast(f16x4, l)};
 }
+struct Fine {                  // x = h + l / REST
+    f16x4 h, l;
+};
+constexpr float REST = 2048.f;
+// of x 2^MORE
+template <int MORE = 0> __device__ __forceinline__ Fine split_fine(const f32x4& x) {
+    typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+    struct Words { uint32_t a, b; };
+    constexpr float BY = (float)(1 << MORE);
+    Words h, l;
+    f16x2 h0 = {(_Float16)(x[0] * BY), (_Float16)(x[1] * BY)}, h1 = {(_Float16)(x[2] * BY), (_Float16)(x[3] * BY)};
+    asm("" : "+v"(h0), "+v"(h1));                                        // (as above)
+    const f16x2 l0 = {(_Float16)fmaf(-REST, (float)h0[0], x[0] * (BY * REST)), (_Float16)fmaf(-REST, (float)h0[1], x[1] * (BY * REST))};
+    const f16x2 l1 = {(_Float16)fmaf(-REST, (float)h1[0], x[2] * (BY * REST)), (_Float16)fmaf(-REST, (float)h1[1], x[3] * (BY * REST))};
+    h = {__builtin_bit_cast(uint32_t, h0), __builtin_bit_cast(uint32_t, h1)};
+    l = {__builtin_bit_cast(uint32_t, l0), __builtin_bit_cast(uint32_t, l1)};
+    return Fine{__builtin_bit_cast(f16x4, h), __builtin_bit_cast(f16x4, l)};
+}
 __device__ __forceinline__ f16x8 both(const f16x4& a, const f16x4& b) { return __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7); }
+// x and x / REST: one product with both pieces of a Fine adds them in their scales
+__device__ __forceinline__ f16x8 with_rest(const f16x4& x) { return both(x, x * (_Float16)(1.f / REST)); }
+__device__ __forceinline__ f16x8 both(const Fine& x) { return both(x.h, x.l); }
 __device__ __forceinline__ f16x4 halves(const f32x4& x) { return packed<__half>(x).v; }
 __device__ __forceinline__ f32x4 mma32(const f16x8& a, const f16x8& b, const f32x4& c) { return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0); }
 __device__ __forceinline__ f32x4 mma16(const f16x4& a, const f16x4& b, const f32x4& c) { return __builtin_amdgcn_mfma_f32_16x16x16f16(a, b, c, 0, 0, 0); }

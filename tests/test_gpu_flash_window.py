@@ -128,6 +128,63 @@ def test_rows_far_apart(dtype, what):
     _check(got, _float64(index, ind, qkv, up, table, mask, got[0]), ind, dtype, floor=1e-30 if dtype != torch.float16 else 6e-8 / TOL[dtype] * (343 * 16) ** 0.5)
 
 
+# A row's own bound.  fp32: sums of at most 384 terms, dP - D of numbers up to ten times their difference, 1e-5; an ulp of a 16-bit result
+ROW_TOL = {torch.float32: 1e-5, torch.float16: 2 ** -10, torch.bfloat16: 2 ** -7}
+
+
+def _check_rows(got, want, rows, dtype, names):
+    """Every row and head of the results named, against the norm of that row."""
+    N, _, H, hd = want[1].shape
+    a = {"out": got[0].double().cpu().view(N, H, hd), **{n: got[1].double().cpu().view(N, 3, H, hd)[:, i] for i, n in enumerate(("dq", "dk", "dv"))}}
+    b = {"out": want[0], **{n: want[1][:, i] for i, n in enumerate(("dq", "dk", "dv"))}}
+    for name in names:
+        rel = ((a[name] - b[name])[rows].norm(dim=2) / b[name][rows].norm(dim=2)).max().item()
+        assert rel <= ROW_TOL[dtype], (name, rel)
+
+
+@pytest.mark.parametrize("dtype,bits", [(torch.float32, (0, 2, 6, 9, 11)), (torch.float16, (0, 6, 11, 17)), (torch.bfloat16, (0, 6, 11, 17))], ids=["fp32", "fp16", "bf16"])
+def test_rows_of_small_upstream_gradients(dtype, bits):
+    """Every other row of dO 2^-bits of its neighbours, as those of voxels that are classified well: dQ of each row by itself."""
+    for k in bits:
+        ti, index, ind, qkv, up, table, mask, plan = _case([60, 17, 96, 200, 343], 343, 2, dtype, 5)
+        up *= 2.0 ** 10                                            # (so that fp16 results stay above its least normal value)
+        up[::2] *= 2.0 ** -k
+        got = _run(ti, ind, qkv, up, table, mask, plan, 343)
+        _check_rows(got, _float64(index, ind, qkv, up, table, mask, got[0]), slice(0, None), dtype, ("dq", "dk", "dv"))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16], ids=["fp32", "fp16", "bf16"])
+def test_mask_regions_of_small_upstream_gradients(dtype):
+    """A whole region of a window with dO 2^-9 of the others': its keys meet small rows only."""
+    ti, index, ind, qkv, up, table, mask, plan = _case([60, 96, 200, 343], 343, 2, dtype, 6, 2)
+    small = mask[ind[:, 0].long(), ind[:, 1].long()] == 1
+    up *= 2.0 ** 10
+    up[small] *= 2.0 ** -9
+    got = _run(ti, ind, qkv, up, table, mask, plan, 343)
+    _check_rows(got, _float64(index, ind, qkv, up, table, mask, got[0]), slice(0, None), dtype, ("dq", "dk", "dv"))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16], ids=["fp32", "fp16", "bf16"])
+def test_keys_that_no_query_attends(dtype):
+    """A key in each window whose P is about 2^-20 for every query: its dK and dV; and the output where it alone has values (V = 0 elsewhere)."""
+    counts = [60, 96, 200, 343]
+    ti, index, ind, qkv, up, table, mask, plan = _case(counts, 343, 2, dtype, 7)
+    rows = torch.tensor([int((ind[:, 0] == w).nonzero()[c // 2]) for w, c in enumerate(counts)])
+    qkv[:, 0, :, 0] = 4
+    qkv[rows, 1] = 0
+    qkv[rows, 1, :, 0] = -8
+    table *= 0.1
+    up *= 2.0 ** 12
+    got = _run(ti, ind, qkv, up, table, mask, plan, 343)
+    _check_rows(got, _float64(index, ind, qkv, up, table, mask, got[0]), rows, dtype, ("dk", "dv"))
+    other = torch.ones(len(ind), dtype=torch.bool)
+    other[rows] = False
+    qkv[other, 2] = 0
+    qkv[rows, 2] *= 2.0 ** 12
+    got = _run(ti, ind, qkv, up, table, mask, plan, 343)
+    _check_rows(got, _float64(index, ind, qkv, up, table, mask, got[0]), slice(0, None), dtype, ("out",))
+
+
 @pytest.mark.parametrize("which", ["q", "k", "v", "dO"])
 @pytest.mark.parametrize("value", [float("inf"), float("nan")], ids=["inf", "nan"])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16], ids=["fp32", "fp16", "bf16"])
