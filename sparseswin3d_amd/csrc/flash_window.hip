@@ -305,18 +305,18 @@ constexpr int WAVE_LDS = 3 * TURN + 16;                                  // of a
 // P is formed times 2^P_BITS, so that exponents lie around zero, where fp32 rounds them least, and split times 2^P_MORE on top: 22 bits of it down to 2^-28, and 2^-50
 constexpr int P_BITS = 7, P_MORE = 7;
 // Steps between two meetings of a window's wavefronts.  At every step 143 us (225 700 tokens fp16) and 130 (8100 in nearly full windows), every other one 142 and
-// 126, at every fourth 141 and 124; fp32 within 2 % of each other.
-constexpr int GROUP = 4;
+// 126, at every fourth 141 and 124; fp32 within 2 % of each other.  Four do not fit LDS twice beside the two sums of a table of 13^3 rows.
+constexpr int GROUP = 2;
 enum class How { plain, masked, exact };   // windows of one mask region, of several; fp32 products of the rows as they are
 template <typename T, bool TABLE> __global__ __launch_bounds__(WAVES * 64, B_RESIDENT) void flash_window_backward_kernel(Args g) {
     constexpr bool PAIRS = sizeof(T) == 4, SCALED = !std::is_same<T, __half>::value;
     extern __shared__ __attribute__((aligned(16))) char lds[];
     const int lane = threadIdx.x & 63, l16 = lane & 15, quad = lane >> 4, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    // LDS: [rows] sums, [2][rows / 32] bits of rows that are +inf, -inf; tiles to turn; exchange; bias of the head
+    // LDS: [2][rows] sums, [2][rows / 32] bits of rows that are +inf, -inf; tiles to turn; exchange; bias of the head
     const int words = (g.rows + 31) >> 5;
     unsigned long long* const sums = reinterpret_cast<unsigned long long*>(lds);
-    uint32_t* const infinite = reinterpret_cast<uint32_t*>(sums + (TABLE ? g.rows : 0));
-    float* const tiles_lds = reinterpret_cast<float*>(infinite + (TABLE ? (2 * words + 3) / 4 * 4 + (g.rows & 1) * 2 : 0));
+    uint32_t* const infinite = reinterpret_cast<uint32_t*>(sums + (TABLE ? 2 * g.rows : 0));
+    float* const tiles_lds = reinterpret_cast<float*>(infinite + (TABLE ? (2 * words + 3) / 4 * 4 : 0));
     float* const turn = tiles_lds + wave * WAVE_LDS;
     float* const deltas = turn + 3 * TURN;
     float* const shared = tiles_lds + WAVES * WAVE_LDS;                  // [2][GROUP][WAVES][256]
@@ -328,22 +328,25 @@ template <typename T, bool TABLE> __global__ __launch_bounds__(WAVES * 64, B_RES
     Work<KT> work(g, first);
     stage_table(g, h, bias);
     if (threadIdx.x < 16) stops[threadIdx.x] = 0;
-    int unit = 0, top = 0;                                               // the table's sums are in units of 2^unit; |dS| < 2^top
+    int unit = 0, top = 0;                                               // the table's sums are in units of 2^unit, and 2^(unit - fine); |dS| < 2^top
+    const int fine = g.bits - KEEPS;
     if constexpr (TABLE) {
-        for (int i = threadIdx.x; i < g.rows; i += WAVES * 64) sums[i] = 0;
+        for (int i = threadIdx.x; i < 2 * g.rows; i += WAVES * 64) sums[i] = 0;
         for (int i = threadIdx.x; i < 2 * words; i += WAVES * 64) infinite[i] = 0;
         float mo = 0.f, mv = 0.f, o[DELTA_BLOCKS / 64], v[FORWARD_BLOCKS / 64];   // requested together
 #pragma unroll
-        for (int i = 0; i < DELTA_BLOCKS / 64; ++i) o[i] = g.largest[min(i * 64 + lane, g.n_largest - 1)];
+        for (int i = 0; i < DELTA_BLOCKS / 64; ++i) o[i] = g.largest[h * g.n_largest + min(i * 64 + lane, g.n_largest - 1)];
 #pragma unroll
-        for (int i = 0; i < FORWARD_BLOCKS / 64; ++i) v[i] = g.largest_v[min(i * 64 + lane, g.n_largest_v - 1)];
+        for (int i = 0; i < FORWARD_BLOCKS / 64; ++i) {                  // of the head's workgroups, as place() deals them
+            const int b = min(i * 64 + lane, g.n_largest_v - 1);
+            v[i] = g.largest_v[((b >> 3) * g.H + h) * 8 + (b & 7)];
+        }
 #pragma unroll
         for (int i = 0; i < DELTA_BLOCKS / 64; ++i) mo = fmaxf(mo, o[i]);
 #pragma unroll
         for (int i = 0; i < FORWARD_BLOCKS / 64; ++i) mv = fmaxf(mv, v[i]);
         for (int o = 1; o < 64; o <<= 1) mo = fmaxf(mo, __shfl_xor(mo, o, 64)), mv = fmaxf(mv, __shfl_xor(mv, o, 64));
-        const Unit<HD> u(mo, mv, g.N);
-        top = __builtin_amdgcn_readfirstlane(u.top), unit = top - u.bits;
+        top = __builtin_amdgcn_readfirstlane(bound_of_ds<HD>(mo, mv)), unit = top - g.bits;
     }
     __syncthreads();
     const int D = g.H * HD;
@@ -469,13 +472,17 @@ template <typename T, bool TABLE> __global__ __launch_bounds__(WAVES * 64, B_RES
                     if (stop && task.team == 1) return s;
                     es = eo + ev - 18;
                 }
-                // added to it, a value times 2^es is rounded to the unit of the sums
-                const uint32_t unit_hi = (uint32_t)(0x3ff80000 + ((52 + unit + es) << 20));
-                const double whole = __builtin_bit_cast(double, (unsigned long long)unit_hi << 32);
+                // Added to it, a value times 2^es is rounded to the unit of the sums; below `small`, to the finer one of the second sums
+                const uint32_t unit_hi = (uint32_t)(0x3ff80000 + ((52 + unit + es) << 20)), fine_hi = unit_hi - ((uint32_t)fine << 20);
+                const float small = power(max(-127, min(127, top - fine + es)));
+                const uint32_t fine_at = sums_at + 8 * g.rows;
                 auto add = [&](uint32_t at, float x) __attribute__((always_inline)) {
-                    const unsigned long long b = __builtin_bit_cast(unsigned long long, (double)x + whole);
-                    const unsigned long long n = (unsigned long long)((uint32_t)(b >> 32) - unit_hi) << 32 | (uint32_t)b;
-                    __hip_atomic_fetch_add((LdsLong*)(uintptr_t)(2 * at + sums_at), n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                    const bool low = fabsf(x) < small;
+                    // (fp32: fewer registers that way, 12 spilled less, 225 700 tokens 230 -> 221 us; 16 bit: 3 % slower)
+                    const uint32_t hi = PAIRS ? unit_hi - (low ? (uint32_t)fine << 20 : 0) : low ? fine_hi : unit_hi;
+                    const unsigned long long b = __builtin_bit_cast(unsigned long long, (double)x + __builtin_bit_cast(double, (unsigned long long)hi << 32));
+                    const unsigned long long n = (unsigned long long)((uint32_t)(b >> 32) - hi) << 32 | (uint32_t)b;
+                    __hip_atomic_fetch_add((LdsLong*)(uintptr_t)(2 * at + (PAIRS ? sums_at + (low ? 8 * g.rows : 0) : low ? fine_at : sums_at)), n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
                 };
                 if constexpr (!EXACT) {
                   if (!stop) {
@@ -626,7 +633,7 @@ template <typename T, bool TABLE> __global__ __launch_bounds__(WAVES * 64, B_RES
         __syncthreads();
         float* const to = g.partial + ((int64_t)h * g.per_head + first) * g.rows;
         for (int i = threadIdx.x; i < g.rows; i += WAVES * 64) {
-            float sum = (float)ldexp((double)(long long)sums[i], unit);
+            float sum = (float)(ldexp((double)(long long)sums[i], unit) + ldexp((double)(long long)sums[g.rows + i], unit - fine));
             const bool up = infinite[i >> 5] >> (i & 31) & 1, down = infinite[words + (i >> 5)] >> (i & 31) & 1;
             if (up) sum = down ? __builtin_nanf("") : INFINITY;
             else if (down) sum = -INFINITY;
@@ -660,7 +667,7 @@ int add_table(const float* partial, int per_head, int rows, int H, float* d_tabl
 
 static size_t backward_lds(int rows, bool table) {
     const int words = (rows + 31) / 32;
-    return (table ? (size_t)rows * 8 + ((2 * words + 3) / 4 * 4 + (rows & 1) * 2) * 4 : 0) + (size_t)(WAVES * WAVE_LDS + 2 * GROUP * WAVES * 256 + 16 + rows) * sizeof(float);
+    return (table ? (size_t)rows * 16 + (2 * words + 3) / 4 * 16 : 0) + (size_t)(WAVES * WAVE_LDS + 2 * GROUP * WAVES * 256 + 16 + rows) * sizeof(float);
 }
 
 template <typename T, bool TABLE> static int launch_backward(Args g, hipStream_t s) {
@@ -678,10 +685,15 @@ template <typename T> static int run_forward(const Args& g, hipStream_t s) {
 
 template <typename T> static int run_backward(Args g, float* delta, float* largest, float* d_table, hipStream_t s) {
     const int64_t parts = g.N * g.H * (HD / 4);
-    const int blocks = (int)std::min<int64_t>(DELTA_BLOCKS, (parts + 1023) / 1024);
-    hipLaunchKernelGGL((flash_window_delta_kernel<T, HD>), dim3(blocks), dim3(256), 0, s, static_cast<const T*>(g.dout), static_cast<const T*>(g.out), parts, delta, largest);
+    // at least the lanes of one voxel
+    const int blocks = (int)std::max<int64_t>((g.H * (HD / 4) + 255) / 256, std::min<int64_t>(DELTA_BLOCKS, (parts + 1023) / 1024));
+    hipLaunchKernelGGL((flash_window_delta_kernel<T, HD>), dim3(blocks), dim3(256), 0, s, static_cast<const T*>(g.dout), static_cast<const T*>(g.out), parts, g.H, delta,
+                       largest);
     if (int rc = launch_ok("flash_window_backward, delta")) return rc;
     g.delta = delta, g.largest = largest, g.n_largest = blocks;
+    // what a workgroup adds to a row of the table: at most one value a query, MOST tiles of them a round
+    const int64_t rounds = (g.windows + g.per_head - 1) / g.per_head, most = std::min<int64_t>(g.N, rounds * MOST * 16);
+    g.bits = std::min(50, __builtin_clzll((unsigned long long)most) - 2);
     if (!d_table) return launch_backward<T, false>(g, s);
     if (int rc = launch_backward<T, true>(g, s)) return rc;
     return add_table(g.partial, g.per_head, g.rows, g.H, d_table, s);
@@ -710,7 +722,7 @@ static int window_args(const char* what, int dtype, const int32_t* plan, int64_t
     SSWIN_CHECK(plan && tokens && word && list && qkv && table && out && lse, "%s: null pointer", what);
     SSWIN_CHECK(((uintptr_t)qkv | (uintptr_t)out) % 16 == 0, "%s: pointers must be 16-byte aligned", what);
     g.plan = plan, g.g_cap = g_cap, g.order = tokens, g.word = reinterpret_cast<const uint32_t*>(word), g.list = list, g.N = N, g.windows = (int)(groups / H);
-    g.largest_v = reinterpret_cast<float*>(const_cast<int32_t*>(list)) + LIST_HEAD + g.windows, g.n_largest_v = forward_per_head(dtype, N, g.windows, H) * H;
+    g.largest_v = reinterpret_cast<float*>(const_cast<int32_t*>(list)) + LIST_HEAD + g.windows, g.n_largest_v = forward_per_head(dtype, N, g.windows, H);
     g.H = H, g.rows = rows, g.offset4 = offset0 * 4, g.scale = scale, g.table = table, g.qkv = qkv, g.out = out, g.lse = lse;
     return 0;
 }
@@ -718,7 +730,7 @@ static int window_args(const char* what, int dtype, const int32_t* plan, int64_t
 extern "C" {
 
 size_t sswin_flash_window_list_ints(int dtype, int64_t N, int H, int hd, int n, int rows, int64_t windows) {
-    return hd == HD && n <= MOST * 16 && H <= FORWARD_BLOCKS / 8 && windows > 0 && windows <= LIST_WINDOWS && sswin_flash_supported(dtype, N, H, hd, rows) && N * 3 * H * hd < 1ll << 30
+    return hd == HD && n <= MOST * 16 && H <= MOST_HEADS && windows > 0 && windows <= LIST_WINDOWS && sswin_flash_supported(dtype, N, H, hd, rows) && N * 3 * H * hd < 1ll << 30
                ? (size_t)LIST_HEAD + windows + FORWARD_BLOCKS : 0;
 }
 
@@ -749,7 +761,7 @@ int sswin_flash_window_forward(int dtype, const int32_t* plan, int64_t g_cap, in
 size_t sswin_flash_window_backward_workspace_bytes(int64_t N, int H, int rows, int64_t windows) {
     Carver c(nullptr, 0);
     c.take<float>((size_t)H * N);
-    c.take<float>(DELTA_BLOCKS);
+    c.take<float>((size_t)DELTA_BLOCKS * H);
     c.take<float>((size_t)per_head((int)windows, H, B_RESIDENT) * H * rows);
     return c.used;
 }
@@ -764,7 +776,7 @@ int sswin_flash_window_backward(int dtype, const int32_t* plan, int64_t g_cap, i
     SSWIN_CHECK(dout && dqkv && ws && ((uintptr_t)dout | (uintptr_t)dqkv) % 16 == 0, "flash_window_backward: gradients at 16 bytes and a workspace");
     Carver c(ws, ws_bytes);
     float* const delta = c.take<float>((size_t)H * N);
-    float* const largest = c.take<float>(DELTA_BLOCKS);
+    float* const largest = c.take<float>((size_t)DELTA_BLOCKS * H);
     g.per_head = per_head(g.windows, H, B_RESIDENT);
     g.partial = c.take<float>((size_t)g.per_head * H * rows);
     SSWIN_CHECK(c.ok(), "flash_window_backward: workspace of %zu bytes, %zu are needed", ws_bytes, c.used);

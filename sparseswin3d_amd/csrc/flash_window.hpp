@@ -15,6 +15,7 @@ namespace window {
 
 constexpr int WAVES = 4, MOST = 24;                                      // wavefronts of a workgroup; tiles of 16 tokens of a window
 constexpr int DELTA_BLOCKS = 1024, FORWARD_BLOCKS = 1024;
+constexpr int MOST_HEADS = FORWARD_BLOCKS / 8;                           // workgroups of a head come in eights
 constexpr int LIST_HEAD = 32, LIST_THREADS = 1024, LIST_WINDOWS = 16384;
 constexpr uint32_t INDEX = 0x7ffcu;                                      // of a difference of words: 4 row of the table
 constexpr int PITCH = 20, TURN = 16 * PITCH;                             // a 16 x 16 tile in LDS, values
@@ -27,7 +28,7 @@ struct Args {
     const int32_t* order;      // voxel of token rank r
     const uint32_t* word;      // 4 code | region << 15 | several regions in the window << 31 of token r
     const int32_t* list;       // [t]: windows of more than t tiles; from LIST_HEAD on the windows, largest first
-    float* largest_v;          // [n_largest_v] largest |V| of the forward's workgroups
+    float* largest_v;          // largest |V| of the forward's workgroups, n_largest_v a head
     int n_largest_v;
     int64_t N;
     int windows, H, rows, offset4, per_head;
@@ -40,8 +41,9 @@ struct Args {
     const void* dout;          // [N, H hd]
     const float* delta;        // [N, H]: dO . O
     void* dqkv;                // [N, 3 H hd]
-    const float* largest;      // [n_largest] largest |dO| of some tokens
+    const float* largest;      // [H, n_largest] largest |dO| of a head in some tokens
     int n_largest;
+    int bits;                  // a sum of the bias table's gradient takes values below 2^bits units
     float* partial;            // [H][per_head][rows] sums of dS by table row
 };
 
@@ -216,49 +218,56 @@ __device__ __forceinline__ float largest_of_workgroup(float m, float* part) {
 __device__ __forceinline__ float not_finite(const f32x4& v) { return fmaf(v[0], 0.f, fmaf(v[1], 0.f, fmaf(v[2], 0.f, v[3] * 0.f))); }
 
 // ------------------------------------------------------------------------------------------
-// D = dO . O of every voxel and head, HD / 4 lanes a head, and the largest |dO| (of what is finite) of a workgroup
+// D = dO . O of every voxel and head, HD / 4 lanes a head, and the largest |dO| (of what is finite) of a workgroup and head.  A lane keeps to one head: lanes
+// behind the last whole number of voxels that the launch holds have nothing to do.
 // ------------------------------------------------------------------------------------------
 template <typename T, int HD>
-__global__ __launch_bounds__(256) void flash_window_delta_kernel(const T* __restrict__ dout, const T* __restrict__ out, int64_t parts, float* __restrict__ delta,
+__global__ __launch_bounds__(256) void flash_window_delta_kernel(const T* __restrict__ dout, const T* __restrict__ out, int64_t parts, int H, float* __restrict__ delta,
                                                                  float* __restrict__ largest) {
-    __shared__ float part[4];
-    constexpr int AT_ONCE = 4;
+    __shared__ uint32_t of_head[MOST_HEADS];
+    constexpr int AT_ONCE = 4, LANES = HD / 4;
+    static_assert(LANES == 4, "the four lanes of a head are added by two exchanges");
+    for (int i = threadIdx.x; i < H; i += 256) of_head[i] = 0;
+    const int row = (int)(blockIdx.x * 256 + threadIdx.x) / LANES, stride = (int)(gridDim.x * (256 / LANES)) / H * H * LANES;
     float most = 0.f;
-    for (int64_t i0 = (int64_t)blockIdx.x * 256 + threadIdx.x; i0 < parts; i0 += (int64_t)gridDim.x * 256 * AT_ONCE) {
-        Frag<T> x[AT_ONCE], y[AT_ONCE];
+    if (row * LANES < stride) {
+        for (int64_t i0 = (int64_t)blockIdx.x * 256 + threadIdx.x; i0 < parts; i0 += (int64_t)stride * AT_ONCE) {
+            Frag<T> x[AT_ONCE], y[AT_ONCE];
 #pragma unroll
-        for (int k = 0; k < AT_ONCE; ++k) {
-            const int64_t i = min(i0 + (int64_t)gridDim.x * 256 * k, parts - 1);
-            x[k].load(dout + i * 4), y[k].load(out + i * 4);
-        }
+            for (int k = 0; k < AT_ONCE; ++k) {
+                const int64_t i = i0 + (int64_t)stride * k, j = i < parts ? i : i0;   // (of the lane's head too)
+                x[k].load(dout + j * 4), y[k].load(out + j * 4);
+            }
 #pragma unroll
-        for (int k = 0; k < AT_ONCE; ++k) {
-            const int64_t i = i0 + (int64_t)gridDim.x * 256 * k;
-            const f32x4 a = widened(x[k]), b = widened(y[k]);
-            float dot = 0.f;
+            for (int k = 0; k < AT_ONCE; ++k) {
+                const int64_t i = i0 + (int64_t)stride * k;
+                const f32x4 a = widened(x[k]), b = widened(y[k]);
+                float dot = 0.f;
 #pragma unroll
-            for (int j = 0; j < 4; ++j) dot = fmaf(a[j], b[j], dot);
-            dot += dpp_f32<0xB1>(dot);
-            dot += dpp_f32<0x4E>(dot);
-            if constexpr (HD == 32) dot += dpp_f32<0x141>(dot);
-            most = fmaxf(most, largest_finite(a));
-            if (i < parts && (threadIdx.x & (HD / 4 - 1)) == 0) delta[i / (HD / 4)] = dot;
+                for (int j = 0; j < 4; ++j) dot = fmaf(a[j], b[j], dot);
+                dot += dpp_f32<0xB1>(dot);
+                dot += dpp_f32<0x4E>(dot);
+                most = fmaxf(most, largest_finite(a));
+                if (i < parts && (threadIdx.x & (LANES - 1)) == 0) delta[i / LANES] = dot;
+            }
         }
     }
-    const float m = largest_of_workgroup(most, part);
-    if (threadIdx.x == 0) largest[blockIdx.x] = m;
+    __syncthreads();
+    if (most > 0.f) atomicMax(&of_head[row % H], __builtin_bit_cast(uint32_t, most));   // (bits grow with the value)
+    __syncthreads();
+    for (int i = threadIdx.x; i < H; i += 256) largest[(int64_t)i * gridDim.x + blockIdx.x] = __builtin_bit_cast(float, of_head[i]);
 }
 
-// The unit of the table's sums.  Integers, so that the result does not depend on the order of the additions.  |dS| <= |dP| + |D| <= 2 HD largest |dO| largest |V| (P of a row adds up to at most one, up to rounding) < 2^top; dS
-// in units of 2^(top - bits) is a whole number below 2^50, and N of them below 2^62.
-template <int HD> struct Unit {
-    int top, bits;
-    __device__ __forceinline__ Unit(float mo, float mv, int64_t N) {
-        const int eo = mo > 0.f ? (int)ilogbf(mo) : -149, ev = mv > 0.f ? (int)ilogbf(mv) : -149;
-        top = eo + ev + (HD == 16 ? 8 : 9);
-        bits = min(50, 62 - (64 - __builtin_clzll((unsigned long long)N)));
-    }
-};
+// The units of the table's sums.  Integers, so that the result does not depend on the order of the additions.  A head's |dS| <= |dP| + |D| <= 2 HD largest |dO|
+// largest |V| (P of a row adds up to at most one, up to rounding) < 2^top, whole numbers below 2^bits in units of 2^(top - bits); a workgroup adds at most
+// 2^(62 - bits) of them to a row of the table.  A value below 2^KEEPS units would lose bits of its fp32 there: it is added to a second sum, in units
+// 2^(bits - KEEPS) as fine.  So every value down to 2^(2 KEEPS - 2 bits) of the bound is added as exactly as fp32 has it, wherever the head's largest dO and V lie.
+// (One sum in units of all heads' largest: a row of dO in one head and one of V in another, 2^20 above the rest, left nothing of the others' dS.)  What the second
+// sum costs the backward, three instructions a value, windows of 7^3: 112 700 tokens fp32 115 -> 117 us, fp16 88 -> 91, 8100 in nearly full windows fp32 154 -> 163.
+constexpr int KEEPS = 23;
+template <int HD> __device__ __forceinline__ int bound_of_ds(float mo, float mv) {
+    return (mo > 0.f ? (int)ilogbf(mo) : -149) + (mv > 0.f ? (int)ilogbf(mv) : -149) + (HD == 16 ? 8 : 9);
+}
 
 // ------------------------------------------------------------------------------------------
 // Pieces.  P, dS and, of fp32 tokens, the rows are multiplied on the 16-bit matrix cores as pairs of fp16 rounded to nearest, products of two second pieces left

@@ -185,6 +185,37 @@ def test_keys_that_no_query_attends(dtype):
     _check_rows(got, _float64(index, ind, qkv, up, table, mask, got[0]), slice(0, None), dtype, ("out",))
 
 
+@pytest.mark.parametrize("dtype,bits", [(torch.float32, 20), (torch.float16, 12), (torch.bfloat16, 20)], ids=["fp32", "fp16", "bf16"])
+@pytest.mark.parametrize("head", [0, 1], ids=["same-head", "other-head"])
+def test_table_where_single_rows_are_large(dtype, bits, head):
+    """A row of dO in one window and one of V in another, 2^bits above the rest: what the table's gradient holds of other windows and heads."""
+    counts = [4, 60, 200, 343, 4, 33]
+    ti, index, ind, qkv, up, table, mask, plan = _case(counts, 343, 3, dtype, 8)
+    first = [int((ind[:, 0] == w).nonzero()[0]) for w in range(len(counts))]
+    up[first[0], 3] *= 2.0 ** bits
+    qkv[first[4], 2, head, 3] *= 2.0 ** bits
+    out, _, got = _run(ti, ind, qkv, up, table, mask, plan, 343)
+    got, want = got.double().cpu(), _float64(index, ind, qkv, up, table, mask, out)[2]
+    apart = torch.ones(len(table), dtype=torch.bool)               # rows that the two windows add nothing to
+    for w in (0, 4):
+        pos = ind[ind[:, 0] == w, 1].long()
+        apart[index[pos][:, pos].reshape(-1).long()] = False
+    for h in range(3):
+        diff, norm = (got - want)[apart, h].norm(), want[apart, h].norm()
+        assert diff <= TOL[dtype] * norm, (h, (diff / norm).item())
+
+
+@pytest.mark.parametrize("heads", [1, 5, 24, 128])
+def test_table_by_heads_of_all_sizes(heads):
+    """Heads by powers of two apart, and voxel counts that do not divide by what a launch holds: each head's gradient by its own norm."""
+    ti, index, ind, qkv, up, table, mask, plan = _case([60, 17, 96, 9], 343, heads, torch.float32, 9)
+    size = 2.0 ** (torch.arange(heads) * 37 % 48 - 24).float()
+    up *= size.repeat_interleave(16)
+    qkv[:, 2] *= size.flip(0)[:, None]
+    got = _run(ti, ind, qkv, up, table, mask, plan, 343)
+    _check(got, _float64(index, ind, qkv, up, table, mask, got[0]), ind, torch.float32)
+
+
 @pytest.mark.parametrize("which", ["q", "k", "v", "dO"])
 @pytest.mark.parametrize("value", [float("inf"), float("nan")], ids=["inf", "nan"])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16], ids=["fp32", "fp16", "bf16"])
