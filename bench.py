@@ -598,7 +598,7 @@ def kernel_table(wl, reps=20, only=None):
     fl_entries = []
     if ti is not None and F.attention_path(hd, b["n"], ti) == "flash":
         table_fl = wl["blocks"][0]["attn"].relative_position_bias_table.detach().float().contiguous()
-        n_list = lib.sswin_flash_window_list_ints(code, N, H, hd, b["n"], n_table, tp.G // H)
+        n_list = lib.sswin_flash_window_list_ints(code, N, H, hd, b["n"], n_table, tp.G // H) if lib.sswin_flash_window_faster(N, tp.G // H, tp.A // H) else 0
         if n_list:
             # a wavefront a window and head; the bias-table gradient is summed in the backward's launch
             words = torch.empty(N + n_list, dtype=torch.int32, device=dev)

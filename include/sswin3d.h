@@ -526,8 +526,10 @@ int sswin_flash_backward_ordered(int dtype, const int32_t* tokens, const int32_t
 
 /* The same attention for heads of 16 channels in windows of at most 384 positions, a wavefront per (window, head) and up to 96 tokens, with the
  * gradient of the bias table in the backward's launch.  sswin_flash_window_list_ints: size of `list` (int32), 0 where a shape is not taken (then
- * sswin_flash_* above).  plan, g_cap, groups: the token plan's group table.  sswin_flash_window_tokens writes word [N] (not that of sswin_flash_tokens)
+ * sswin_flash_* above).  sswin_flash_window_faster: 0 where sswin_flash_* above take less time, as with windows of a few tokens (pairs: sum of the squares
+ * of the windows' tokens).  plan, g_cap, groups: the token plan's group table.  sswin_flash_window_tokens writes word [N] (not that of sswin_flash_tokens)
  * and list, to which the forward adds what its backward needs; d_table fp32 [rows, H] or null. */
+int sswin_flash_window_faster(int64_t N, int64_t windows, int64_t pairs);
 size_t sswin_flash_window_list_ints(int dtype, int64_t N, int H, int hd, int n, int rows, int64_t windows);
 int sswin_flash_window_tokens(const int32_t* plan, int64_t g_cap, int64_t groups, const int32_t* tokens, int64_t N, int H, int n, const int32_t* code,
                               const int8_t* mask, int nmw, int32_t* word, int32_t* list, void* stream);

@@ -102,6 +102,7 @@ SIGNATURES = {
     "sswin_flash_forward": (_i32, [_i32, _vp, _vp, _i64, _i32, _i32, _i32, _vp, C.c_float, _vp, _i32, _i32, _vp, _vp, _vp]),
     "sswin_flash_backward": (_i32, [_i32, _vp, _vp, _vp, _i64, _i32, _i32, _i32, _vp, C.c_float, _vp, _i32, _i32, _vp, _vp, _vp, _vp, _vp,
                                     _vp, _vp]),
+    "sswin_flash_window_faster": (_i32, [_i64, _i64, _i64]),
     "sswin_flash_window_list_ints": (_sz, [_i32, _i64, _i32, _i32, _i32, _i32, _i64]),
     "sswin_flash_window_tokens": (_i32, [_vp, _i64, _i64, _vp, _i64, _i32, _i32, _vp, _vp, _i32, _vp, _vp, _vp]),
     "sswin_flash_window_forward": (_i32, [_i32, _vp, _i64, _i64, _vp, _vp, _vp, _i64, _i32, _i32, _i32, _vp, C.c_float, _vp, _i32, _i32, _vp, _vp, _vp]),

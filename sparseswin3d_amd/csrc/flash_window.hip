@@ -1,7 +1,7 @@
 // Window attention for heads of 16 channels in windows of up to 384 positions: a wavefront per (window, head) and up to 96 of the
 // window's tokens (WindowAttention.forward, sparse_swin/swin3d_base.py:654-675, from the projected qkv to the attention output, and
 // its backward with the gradient of the bias table in the same launch).  flash_attention.hip serves what these do not take: heads of 32
-// channels, more positions, heads or windows (sswin_flash_window_list_ints).
+// channels, more positions, heads or windows (sswin_flash_window_list_ints), and windows of a few tokens (sswin_flash_window_faster).
 //
 // Work: the windows by descending size (flash_window_tokens_kernel), dealt to as many workgroups as find a place at once; a workgroup keeps a
 // head's bias table, and in the backward the sums of its gradient, in LDS.  A window of up to KT tiles of 16 tokens is one wavefront's, one
@@ -728,6 +728,13 @@ static int window_args(const char* what, int dtype, const int32_t* plan, int64_t
 }
 
 extern "C" {
+
+// A window costs these kernels a tile of 16 rows and a wavefront's start however few tokens it has; flash_attention.hip packs small windows into 32 rows, and pays by
+// the token and, more than these, by the pair.  Lines through 110 000 tokens in windows of 12, 24 and 60 (fp32, 3 heads: forward and backward 34 us longer here, 11 and 64
+// shorter) are as 1000 windows, 29 tokens, 1.1 pairs: windows of one size c cross at c = 20.  There both take the same within 12 % (windows of 3^3, 5^3, 7^3, all types, 3 to
+// 12 heads, 30 000 to 220 000 tokens); at 12 these take 0.9 to 1.35 times as long, at 6 up to 2, at 2 up to 4.7; at 24 0.78 to 0.99, at 60 0.56 to 0.7.  Few large windows among
+// small ones are these kernels' (200 of 200 tokens, 3800 of 3: 330 -> 211 us), which the tokens of the mean window, 13, would not tell.
+int sswin_flash_window_faster(int64_t N, int64_t windows, int64_t pairs) { return 1000 * windows <= 30 * N + pairs; }
 
 size_t sswin_flash_window_list_ints(int dtype, int64_t N, int H, int hd, int n, int rows, int64_t windows) {
     return hd == HD && n <= MOST * 16 && H <= MOST_HEADS && windows > 0 && windows <= LIST_WINDOWS && sswin_flash_supported(dtype, N, H, hd, rows) && N * 3 * H * hd < 1ll << 30

@@ -481,6 +481,7 @@ struct Attention : torch::CustomClassHolder {
     double scale = 1.0;
     bool resident = false;  // the window-resident kernels (heads of 32, windows of at most 128 positions)
     bool flash = false;     // the kernels for heads of 16 or 32 and windows of any size
+    enum { BY_SIZE, WINDOWS, CHUNKS } family = BY_SIZE;   // which of them: a wavefront a window and head, or chunks of 32 tokens
 
     int regions() const { return mask.defined() ? (int)mask.size(0) : 0; }
 };
@@ -488,8 +489,18 @@ using AttentionPtr = c10::intrusive_ptr<Attention>;
 
 struct AttentionSaved {
     Tensor bias32, aux;     // bias or table; log-sum-exp of every attention row, or P
-    Tensor words;           // flash: int32 token words [N], window offsets [N], and the order of the work where there is one
+    Tensor words;           // flash, int32.  A wavefront a window and head: token words [N], the list of the windows and the forward's largest |V|;
+                            // chunks: token words [N], window offsets [N], and the order of the work where there is one
 };
+
+// What the kernels that take a window and head a wavefront add to the token words; 0: the chunks' kernels run
+int64_t flash_list_ints(const Attention& a, int dt, int64_t N, int hd, int rows) {
+    const int64_t windows = a.plan->G / a.H;
+    if (a.family == Attention::CHUNKS || (a.family == Attention::BY_SIZE && !sswin_flash_window_faster(N, windows, a.plan->A / a.H))) return 0;
+    const int64_t ints = (int64_t)sswin_flash_window_list_ints(dt, N, a.H, hd, a.n, rows, windows);
+    TORCH_CHECK(ints || a.family != Attention::WINDOWS, "attention: no shape for a wavefront a window and head");
+    return ints;
+}
 
 Tensor attention_forward(Attention& a, const Tensor& qkv, const Tensor& bias, AttentionSaved& saved) {
     Plan& tp = *a.plan;
@@ -512,7 +523,7 @@ Tensor attention_forward(Attention& a, const Tensor& qkv, const Tensor& bias, At
     const auto fopt = qkv.options().dtype(at::kFloat);
     if (a.flash) {
         const Tensor table32 = saved.bias32 = bias.to(at::kFloat).contiguous();
-        const int64_t listed = (int64_t)sswin_flash_window_list_ints(dt, N, a.H, hd, a.n, (int)table32.size(0), tp.G / a.H);
+        const int64_t listed = flash_list_ints(a, dt, N, hd, (int)table32.size(0));
         if (listed) {                                                    // a wavefront a window and head
             saved.words = at::empty({N + listed}, tp.tokens.options());
             saved.aux = at::empty({a.H, N}, fopt);
@@ -606,7 +617,7 @@ Tensor attention_backward(const Attention& a, const Tensor& qkv, const Tensor& b
     void* s = current_stream(qkv);
     Tensor d_qkv = at::empty_like(qkv);
     const auto fopt = qkv.options().dtype(at::kFloat);
-    if (a.flash && sswin_flash_window_list_ints(dt, N, a.H, hd, a.n, (int)saved.bias32.size(0), tp.G / a.H)) {
+    if (a.flash && flash_list_ints(a, dt, N, hd, (int)saved.bias32.size(0))) {
         const int rows = (int)saved.bias32.size(0);
         Tensor d_table = want_bias ? at::empty({rows, a.H}, fopt) : Tensor();
         const size_t nb = sswin_flash_window_backward_workspace_bytes(N, a.H, rows, tp.G / a.H);
@@ -874,7 +885,8 @@ struct MergeNode : torch::autograd::Function<MergeNode> {
 // ------------------------------------------------------------------------------------------
 // Python entry points
 // ------------------------------------------------------------------------------------------
-// path: "resident", "flash" or "products" (the attention matrix in memory)
+// path: "resident", "flash" or "products" (the attention matrix in memory); "flash_windows" and "flash_chunks" are the two families of flash kernels
+// whatever the sizes
 AttentionPtr make_attention(const PlanPtr& plan, const OptTensor& mask, const OptTensor& code, int64_t offset0, int64_t n, int64_t heads, double scale,
                             const std::string& path) {
     auto a = c10::make_intrusive<Attention>();
@@ -882,8 +894,9 @@ AttentionPtr make_attention(const PlanPtr& plan, const OptTensor& mask, const Op
     if (mask) a->mask = mask->to(at::kChar).contiguous();
     if (code) a->code = *code;
     a->offset0 = (int)offset0, a->n = (int)n, a->H = (int)heads, a->scale = scale;
-    a->resident = path == "resident", a->flash = path == "flash";
-    TORCH_CHECK(a->resident || a->flash || path == "products", "attention path ", path);
+    a->resident = path == "resident", a->flash = path.rfind("flash", 0) == 0;
+    a->family = path == "flash_windows" ? Attention::WINDOWS : path == "flash_chunks" ? Attention::CHUNKS : Attention::BY_SIZE;
+    TORCH_CHECK(a->resident || path == "flash" || a->family != Attention::BY_SIZE || path == "products", "attention path ", path);
     TORCH_CHECK(!a->flash || code, "the flash path takes its bias from a relative position table");
     return a;
 }

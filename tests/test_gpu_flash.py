@@ -157,6 +157,31 @@ def test_flash_keeps_what_is_not_finite_where_it_belongs(which, value, hd, dtype
         assert not torch.isfinite(out).all()
 
 
+@pytest.mark.parametrize("counts,chosen", [([19] * 300, 0), ([21] * 300, 1), ([1] * 200 + [343] * 3, 1), ([1] * 400 + [343], 0), ([2] * 16385, 0), ([40] * 16385, 0)],
+                         ids=["19", "21", "few-large", "one-large", "many-small", "many"])
+def test_flash_family_by_the_tokens_of_windows(counts, chosen):
+    """What the path takes by itself: a wavefront a window where that is faster, and at most 16 384 windows.  Its bits are those of that family."""
+    from sparseswin3d_amd import _lib
+    from sparseswin3d_amd.fused import BiasTableIndex, TokenPlan
+    from sparseswin3d_amd.window_attention import relative_position_index_3d
+    ti = BiasTableIndex.build(relative_position_index_3d((7, 7, 7)).cuda(), 13 ** 3)
+    ind = torch.from_numpy(ragged_window_indices(np.random.default_rng(0), counts, 343)).cuda()
+    qkv, table, up = torch.randn(len(ind), 3, 1, 16).cuda(), torch.randn(13 ** 3, 1).cuda(), torch.randn(len(ind), 16).cuda()
+    plan = TokenPlan(ind, len(counts), 343, 1)
+    got = {}
+    for path in ("flash", "flash_chunks") + (("flash_windows",) if len(counts) <= 16384 else ()):
+        x, t = qkv.clone().requires_grad_(True), table.clone().requires_grad_(True)
+        out = _lib.native().attention(x, t, plan.native, None, ti.code, ti.offset0, 343, 0.25, path)
+        out.backward(up)
+        got[path] = (out.detach(), x.grad, t.grad)
+    assert all(torch.equal(a, b) for a, b in zip(got["flash"], got[["flash_chunks", "flash_windows"][chosen]]))
+    if "flash_windows" in got:
+        assert not torch.equal(got["flash_chunks"][0], got["flash_windows"][0])
+    else:
+        with pytest.raises(RuntimeError):
+            _lib.native().attention(qkv, table, plan.native, None, ti.code, ti.offset0, 343, 0.25, "flash_windows")
+
+
 # chunks of 32 tokens: one, some threads without any, several a thread, the most an order holds; windows that fill, span and share
 # chunks; more windows than an order takes, which leaves the chunks as they are
 @pytest.mark.parametrize("N,sizes", [(1, "all"), (32, "all"), (33, "all"), (1000, "all"), (34001, "all"), (12288 * 32, "all"), (40000, "small")])

@@ -32,7 +32,7 @@ def _case(counts, n, H, dtype, seed, regions=None):
 def _run(ti, ind, qkv, up, table, mask, plan, n):
     from sparseswin3d_amd import _lib
     x, t = qkv.cuda().requires_grad_(True), table.cuda().requires_grad_(True)
-    out = _lib.native().attention(x, t, plan.native, None if mask is None else mask.cuda(), ti.code, ti.offset0, n, 0.25, "flash")
+    out = _lib.native().attention(x, t, plan.native, None if mask is None else mask.cuda(), ti.code, ti.offset0, n, 0.25, "flash_windows")
     out.backward(up.cuda())
     return out.detach(), x.grad, t.grad
 
