@@ -1,5 +1,6 @@
 """The attention kernels for heads of 16 / 32 channels and windows of any size (``sswin_flash_*``) against the block products
-with the attention matrix in memory (the other implementation of the same softmax), all gradients included.
+with the attention matrix in memory (the other implementation of the same softmax), all gradients included.  Heads of 16 have two
+families, chunks of 32 tokens and a wavefront a window and head; each is asked for by its name.
 
 fp32: both carry fp32 rounding of sums of at most 384 terms (2e-5 of a result's norm, bias gradient included).  16-bit tokens: P, dS
 and all sums are fp32 in both, so results differ where 2e-5 crosses a rounding boundary: a share 2e-5 x 2^11 (fp16) or 2^8 (bf16) of
@@ -20,11 +21,15 @@ MIXES = {
 }
 
 
+BOTH = ["flash_chunks", "flash_windows"]
+
+
 @pytest.mark.parametrize("mix", list(MIXES))
-@pytest.mark.parametrize("hd,dtype", [(16, torch.float32), (32, torch.float32), (16, torch.float16), (16, torch.bfloat16), (32, torch.bfloat16)],
-                         ids=["16-fp32", "32-fp32", "16-fp16", "16-bf16", "32-bf16"])
+@pytest.mark.parametrize("hd,dtype,family", [(hd, dtype, f) for hd, dtype in ((16, torch.float32), (32, torch.float32), (16, torch.float16), (16, torch.bfloat16),
+                                                                              (32, torch.bfloat16)) for f in (BOTH if hd == 16 else ["flash"])],
+                         ids=lambda v: str(v).replace("torch.", ""))
 @pytest.mark.parametrize("use_mask", [False, True], ids=["plain", "mask"])
-def test_flash_against_block_products(mix, hd, dtype, use_mask):
+def test_flash_against_block_products(mix, hd, dtype, family, use_mask):
     from sparseswin3d_amd.fused import BiasTableIndex, TokenPlan, attention_path, fused_window_attention
     from sparseswin3d_amd.window_attention import relative_position_index_3d
     counts, n = MIXES[mix]
@@ -42,7 +47,7 @@ def test_flash_against_block_products(mix, hd, dtype, use_mask):
     up = torch.randn(len(ind), H * hd).to(dtype).cuda()
     got = []
     from sparseswin3d_amd import _lib
-    for path in ("flash", "products"):
+    for path in (family, "products"):
         x, t = qkv.clone().requires_grad_(True), table.clone().requires_grad_(True)
         plan = TokenPlan(ind, len(counts), n, H)
         out = _lib.native().attention(x, t, plan.native, mask, ti.code, ti.offset0, n, hd ** -0.5, path)
@@ -58,7 +63,8 @@ def test_flash_against_block_products(mix, hd, dtype, use_mask):
         assert rel < tol, (what, rel)
 
 
-def test_flash_many_windows_and_heads():
+@pytest.mark.parametrize("family", BOTH)
+def test_flash_many_windows_and_heads(family):
     """Workgroups in whole rounds over the XCDs and in the remainder; head and chunk numbers of every workgroup."""
     from sparseswin3d_amd.fused import BiasTableIndex, TokenPlan
     from sparseswin3d_amd.window_attention import relative_position_index_3d
@@ -69,11 +75,12 @@ def test_flash_many_windows_and_heads():
         ind = torch.from_numpy(random_window_indices(rng, 700, 125, N)).cuda()
         qkv, table = torch.randn(N, 3, H, 16).cuda(), torch.randn(729, H).cuda()
         plan = TokenPlan(ind, 700, 125, H)
-        a, b = (_lib.native().attention(qkv, table, plan.native, None, ti.code, ti.offset0, 125, 0.25, p) for p in ("flash", "products"))
+        a, b = (_lib.native().attention(qkv, table, plan.native, None, ti.code, ti.offset0, 125, 0.25, p) for p in (family, "products"))
         assert ((a - b).norm() / b.norm()).item() < 1e-5, (N, H)
 
 
-def test_flash_fp16_gradients_outside_the_range_of_fp16():
+@pytest.mark.parametrize("family", BOTH)
+def test_flash_fp16_gradients_outside_the_range_of_fp16(family):
     """dS beyond 65504 (two tokens a window, dO of 15000) while every result is finite in fp16: dS has to stay fp32."""
     from sparseswin3d_amd import _lib
     from sparseswin3d_amd.fused import BiasTableIndex, TokenPlan
@@ -87,7 +94,7 @@ def test_flash_fp16_gradients_outside_the_range_of_fp16():
     qkv, up = qkv.half().cuda(), (torch.randn(len(ind), 32) * 15000).clamp(-6e4, 6e4).half().cuda()
     table = torch.zeros(729, 2).cuda()
     got = []
-    for path in ("flash", "products"):
+    for path in (family, "products"):
         x = qkv.clone().requires_grad_(True)
         plan = TokenPlan(ind, 400, 125, 2)
         _lib.native().attention(x, table, plan.native, None, ti.code, ti.offset0, 125, 0.25, path).backward(up)
@@ -118,9 +125,9 @@ def _float64(qkv, table, index, ind, scale, up):
 
 @pytest.mark.parametrize("which", ["q", "k", "v", "dO"])
 @pytest.mark.parametrize("value", [float("inf"), float("nan")], ids=["inf", "nan"])
-@pytest.mark.parametrize("hd,dtype", [(16, torch.float32), (32, torch.float32), (16, torch.float16), (32, torch.bfloat16)],
-                         ids=["16-fp32", "32-fp32", "16-fp16", "32-bf16"])
-def test_flash_keeps_what_is_not_finite_where_it_belongs(which, value, hd, dtype):
+@pytest.mark.parametrize("hd,dtype,family", [(hd, dtype, f) for hd, dtype in ((16, torch.float32), (32, torch.float32), (16, torch.float16), (32, torch.bfloat16))
+                                             for f in (BOTH if hd == 16 else ["flash"])], ids=lambda v: str(v).replace("torch.", ""))
+def test_flash_keeps_what_is_not_finite_where_it_belongs(which, value, hd, dtype, family):
     """One channel of one token of a few windows is not finite: other windows keep their results, whichever windows share a block
     with them, and inside the window infinities and NaN stand where float64 has them.  Bounds of finite values: as above, per
     result (5 x the norm's bound, at a norm of one token's row)."""
@@ -142,7 +149,7 @@ def test_flash_keeps_what_is_not_finite_where_it_belongs(which, value, hd, dtype
             qkv[r, "qkv".index(which), 1, 3] = value
     x = qkv.cuda().requires_grad_(True)
     plan = TokenPlan(ind.cuda(), len(counts), n, H)
-    out = _lib.native().attention(x, table.cuda(), plan.native, None, ti.code, ti.offset0, n, hd ** -0.5, "flash")
+    out = _lib.native().attention(x, table.cuda(), plan.native, None, ti.code, ti.offset0, n, hd ** -0.5, family)
     out.backward(up.cuda())
     ref = _float64(qkv, table, index, ind, hd ** -0.5, up)
     tol = {torch.float32: 1e-4, torch.float16: 5e-3, torch.bfloat16: 3e-2}[dtype]
@@ -174,7 +181,7 @@ def test_flash_family_by_the_tokens_of_windows(counts, chosen):
         out = _lib.native().attention(x, t, plan.native, None, ti.code, ti.offset0, 343, 0.25, path)
         out.backward(up)
         got[path] = (out.detach(), x.grad, t.grad)
-    assert all(torch.equal(a, b) for a, b in zip(got["flash"], got[["flash_chunks", "flash_windows"][chosen]]))
+    assert all(torch.equal(a, b) for a, b in zip(got["flash"], got[BOTH[chosen]]))
     if "flash_windows" in got:
         assert not torch.equal(got["flash_chunks"][0], got["flash_windows"][0])
     else:

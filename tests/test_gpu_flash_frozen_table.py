@@ -1,5 +1,5 @@
-"""The flash backward with and without dS: a frozen bias table takes the query side that forms the scores again, a trained one dQ from
-the stored dS.  Both sum the same fp32 terms in another order (at most 384 of them: 2e-5 of the gradient's norm; 16-bit results
+"""The flash backward with and without the table's gradient.  Chunks of 32 tokens: a frozen table takes the query side that forms the scores again, a
+trained one dQ from the stored dS.  A wavefront a window and head: a frozen table leaves out the sums.  Both sum the same fp32 terms in another order (at most 384 of them: 2e-5 of the gradient's norm; 16-bit results
 then differ where that crosses a rounding boundary, 1e-3 and 3e-3)."""
 import numpy as np
 import pytest
@@ -11,9 +11,10 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("counts,n", [([1, 2, 31, 1, 33, 5, 16, 17, 1], 125), ([343, 129, 1, 31, 65, 5, 5, 256, 32, 64], 343)], ids=["small", "large"])
-@pytest.mark.parametrize("hd,dtype", [(16, torch.float32), (16, torch.float16), (32, torch.bfloat16)], ids=["16-fp32", "16-fp16", "32-bf16"])
+@pytest.mark.parametrize("hd,dtype,family", [(16, torch.float32, "flash_chunks"), (16, torch.float32, "flash_windows"), (16, torch.float16, "flash_chunks"),
+                                             (16, torch.float16, "flash_windows"), (32, torch.bfloat16, "flash")], ids=lambda v: str(v).replace("torch.", ""))
 @pytest.mark.parametrize("use_mask", [False, True], ids=["plain", "mask"])
-def test_gradient_of_qkv_with_and_without_a_stored_ds(counts, n, hd, dtype, use_mask):
+def test_gradient_of_qkv_with_and_without_a_stored_ds(counts, n, hd, dtype, family, use_mask):
     from sparseswin3d_amd import _lib
     from sparseswin3d_amd.fused import BiasTableIndex, TokenPlan
     from sparseswin3d_amd.window_attention import relative_position_index_3d
@@ -29,7 +30,7 @@ def test_gradient_of_qkv_with_and_without_a_stored_ds(counts, n, hd, dtype, use_
     for trained in (True, False):
         x, t = qkv.clone().requires_grad_(True), table.clone().requires_grad_(trained)
         plan = TokenPlan(ind, len(counts), n, H)
-        _lib.native().attention(x, t, plan.native, mask, ti.code, ti.offset0, n, hd ** -0.5, "flash").backward(up)
+        _lib.native().attention(x, t, plan.native, mask, ti.code, ti.offset0, n, hd ** -0.5, family).backward(up)
         assert (t.grad is not None) == trained
         grads.append(x.grad.double())
     rel = ((grads[0] - grads[1]).norm() / grads[1].norm()).item()
