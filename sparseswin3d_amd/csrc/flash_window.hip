@@ -23,7 +23,7 @@ namespace sswin {
 namespace flash {
 namespace window {
 
-constexpr int HD = 16, KT = MOST / WAVES;                                // tiles of 16 tokens of a wavefront in the backward
+constexpr int KT = MOST / WAVES;                                         // tiles of 16 tokens of a wavefront in the backward
 
 // The windows by descending number of tiles, by one workgroup, and the word of every token, a wavefront per window.
 __device__ __forceinline__ void order_windows(const int32_t* __restrict__ plan, int windows, int H, int32_t* __restrict__ list) {
@@ -346,7 +346,7 @@ template <typename T, bool TABLE> __global__ __launch_bounds__(WAVES * 64, B_RES
 #pragma unroll
         for (int i = 0; i < FORWARD_BLOCKS / 64; ++i) mv = fmaxf(mv, v[i]);
         for (int o = 1; o < 64; o <<= 1) mo = fmaxf(mo, __shfl_xor(mo, o, 64)), mv = fmaxf(mv, __shfl_xor(mv, o, 64));
-        top = __builtin_amdgcn_readfirstlane(bound_of_ds<HD>(mo, mv)), unit = top - g.bits;
+        top = __builtin_amdgcn_readfirstlane(bound_of_ds(mo, mv)), unit = top - g.bits;
     }
     __syncthreads();
     const int D = g.H * HD;
@@ -660,7 +660,7 @@ __global__ __launch_bounds__(1024) void flash_window_table_kernel(const float* _
     }
 }
 
-int add_table(const float* partial, int per_head, int rows, int H, float* d_table, hipStream_t s) {
+static int add_table(const float* partial, int per_head, int rows, int H, float* d_table, hipStream_t s) {
     hipLaunchKernelGGL(flash_window_table_kernel, dim3((unsigned)((rows + 15) / 16), (unsigned)H), dim3(1024), 0, s, partial, per_head, rows, H, d_table);
     return launch_ok("flash_window_backward, table");
 }
@@ -687,7 +687,7 @@ template <typename T> static int run_backward(Args g, float* delta, float* large
     const int64_t parts = g.N * g.H * (HD / 4);
     // at least the lanes of one voxel
     const int blocks = (int)std::max<int64_t>((g.H * (HD / 4) + 255) / 256, std::min<int64_t>(DELTA_BLOCKS, (parts + 1023) / 1024));
-    hipLaunchKernelGGL((flash_window_delta_kernel<T, HD>), dim3(blocks), dim3(256), 0, s, static_cast<const T*>(g.dout), static_cast<const T*>(g.out), parts, g.H, delta,
+    hipLaunchKernelGGL((flash_window_delta_kernel<T>), dim3(blocks), dim3(256), 0, s, static_cast<const T*>(g.dout), static_cast<const T*>(g.out), parts, g.H, delta,
                        largest);
     if (int rc = launch_ok("flash_window_backward, delta")) return rc;
     g.delta = delta, g.largest = largest, g.n_largest = blocks;

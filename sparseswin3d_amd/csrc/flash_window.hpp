@@ -1,5 +1,5 @@
-// What the attention kernels that take a window and head a wavefront have in common: the list of windows, the pieces of work of a workgroup, LDS and rows,
-// pairs of fp16 and their scales, the sums of the bias table's gradient.
+// What flash_window.hip, the attention kernels that take a window and head a wavefront, is made of: the pieces of work of a workgroup, LDS and rows, D = dO . O,
+// pairs of fp16 and their scales, the units of the bias table's sums.
 #pragma once
 
 #include <math.h>
@@ -13,7 +13,7 @@ namespace sswin {
 namespace flash {
 namespace window {
 
-constexpr int WAVES = 4, MOST = 24;                                      // wavefronts of a workgroup; tiles of 16 tokens of a window
+constexpr int HD = 16, WAVES = 4, MOST = 24;                             // channels of a head; wavefronts of a workgroup; tiles of 16 tokens of a window
 constexpr int DELTA_BLOCKS = 1024, FORWARD_BLOCKS = 1024;
 constexpr int MOST_HEADS = FORWARD_BLOCKS / 8;                           // workgroups of a head come in eights
 constexpr int LIST_HEAD = 32, LIST_THREADS = 1024, LIST_WINDOWS = 16384;
@@ -221,12 +221,11 @@ __device__ __forceinline__ float not_finite(const f32x4& v) { return fmaf(v[0], 
 // D = dO . O of every voxel and head, HD / 4 lanes a head, and the largest |dO| (of what is finite) of a workgroup and head.  A lane keeps to one head: lanes
 // behind the last whole number of voxels that the launch holds have nothing to do.
 // ------------------------------------------------------------------------------------------
-template <typename T, int HD>
+template <typename T>
 __global__ __launch_bounds__(256) void flash_window_delta_kernel(const T* __restrict__ dout, const T* __restrict__ out, int64_t parts, int H, float* __restrict__ delta,
                                                                  float* __restrict__ largest) {
     __shared__ uint32_t of_head[MOST_HEADS];
     constexpr int AT_ONCE = 4, LANES = HD / 4;
-    static_assert(LANES == 4, "the four lanes of a head are added by two exchanges");
     for (int i = threadIdx.x; i < H; i += 256) of_head[i] = 0;
     const int row = (int)(blockIdx.x * 256 + threadIdx.x) / LANES, stride = (int)(gridDim.x * (256 / LANES)) / H * H * LANES;
     float most = 0.f;
@@ -265,8 +264,8 @@ __global__ __launch_bounds__(256) void flash_window_delta_kernel(const T* __rest
 // (One sum in units of all heads' largest: a row of dO in one head and one of V in another, 2^20 above the rest, left nothing of the others' dS.)  What the second
 // sum costs the backward, three instructions a value, windows of 7^3: 112 700 tokens fp32 115 -> 117 us, fp16 88 -> 91, 8100 in nearly full windows fp32 154 -> 163.
 constexpr int KEEPS = 23;
-template <int HD> __device__ __forceinline__ int bound_of_ds(float mo, float mv) {
-    return (mo > 0.f ? (int)ilogbf(mo) : -149) + (mv > 0.f ? (int)ilogbf(mv) : -149) + (HD == 16 ? 8 : 9);
+__device__ __forceinline__ int bound_of_ds(float mo, float mv) {
+    return (mo > 0.f ? (int)ilogbf(mo) : -149) + (mv > 0.f ? (int)ilogbf(mv) : -149) + 8;
 }
 
 // ------------------------------------------------------------------------------------------
@@ -356,9 +355,6 @@ inline int per_head(int windows, int H, int resident) {
     const int m = std::max(1, resident * device_cus() / (8 * H));
     return std::min(8 * m, (windows + 7) / 8 * 8);
 }
-
-// d table [rows, H] from the workgroups' sums (flash_window.hip)
-int add_table(const float* partial, int per_head, int rows, int H, float* d_table, hipStream_t s);
 
 }  // namespace window
 }  // namespace flash
