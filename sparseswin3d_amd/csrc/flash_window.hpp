@@ -272,11 +272,13 @@ __device__ __forceinline__ int bound_of_ds(float mo, float mv) {
 // Pieces.  P, dS and, of fp32 tokens, the rows are multiplied on the 16-bit matrix cores as pairs of fp16 rounded to nearest, products of two second pieces left
 // out of dQ alone; sums are fp32.  Rows are x 2^e = h + l, 22 bits or 2^-25 in their scale, whichever is more.  A scale e is one of a wavefront: of K and V for
 // the window, of Q and dO kept from step to step until a row no longer fits, when the sums so far are scaled with it.  Rows too far below the largest for
-// that, and windows in which something is not finite, are done with fp32 products (How::exact), a whole window at a time.
-// P and dS have no scale of their own, and a row of dS is as much smaller than another as its row of dO, or as its P: x = h + l 2^-11, 22 bits down to 2^-14 and 2^-36 below that.
-// (with the pieces of a row for them, 22 bits or 2^-25 in a window's scale, dQ of a query whose dO is 2^-9 of the window's largest was off by 1.6e-5).  Error of a
-// row against float64, its norm, median, windows of 7^3, fp32: dQ 6.4e-7 with fp32 products, 2.8e-7 here, dK 6.3 and 3.4, dV 6.2 and 3.3, the same for rows of dO 2^-9 of the
-// others and for mask regions that hold nothing else; the table's gradient, by head, 5.7 and 3.0.  16-bit tokens: the rounding of the result alone.
+// that, and windows in which something is not finite, are done with fp32 products (How::exact), a whole window at a time.  Where that is nearly every window, backward with
+// the table's gradient, 114 000 tokens in windows of 7^3: 1 % of the rows of dO or of K 2^-14 of the others, fp32 125 -> 214 us (chunks of 32 tokens: 237); rows of dO
+// spread by e^(3 randn), fp32 125 -> 209, fp16 101 -> 165 (169).
+// P and dS have no scale of their own, and a row of dS is as much smaller than another as its row of dO, or as its P: x = h + l 2^-11, 22 bits down to 2^-14
+// and 2^-36 below that (with the pieces of a row for them, 22 bits or 2^-25 in a window's scale, dQ of a query whose dO is 2^-9 of the window's largest was off
+// by 1.6e-5).  Error of a row against float64, its norm, median, windows of 7^3, fp32: dQ 6.4e-7 with fp32 products, 2.8e-7 here, dK 6.3 and 3.4, dV 6.2 and 3.3, the same
+// for rows of dO 2^-9 of the others and for mask regions that hold nothing else; the table's gradient, by head, 5.7 and 3.0.  16-bit tokens: the rounding of the result.
 // ------------------------------------------------------------------------------------------
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 struct Pair {                  // x = h + l
@@ -344,9 +346,10 @@ __device__ __forceinline__ int over_rows(uint32_t m) {                   // of a
 }
 __device__ __forceinline__ int scale_for(int largest, int most) { return largest == 0 ? most : max(-most, min(most, 12 + 127 - (largest >> 23))); }
 __device__ __forceinline__ bool too_large(uint32_t m, int e) { return m >= (uint32_t)(142 - e) << 23; }
-// pieces of a row whose largest value is below 2^(low - e) would lose bits of it
+// pieces of a row whose largest value is below 2^(low - e) would lose bits of it: fp32 rows any below 22; 16-bit rows, of 8 or 11 bits in one piece that keeps 2^-25, those
+// below 2^-10, where P dO and dS, the second piece in 2^-36, still have some 15.  (2^-6 until dS had its finer pieces.)
 template <typename T> __device__ __forceinline__ bool too_small(uint32_t m, int e) {
-    constexpr int low = sizeof(T) == 4 ? 0 : -6;
+    constexpr int low = sizeof(T) == 4 ? 0 : -10;
     return m != 0 && m < (uint32_t)(127 + low - e) << 23;
 }
 

@@ -142,7 +142,7 @@ def _check_rows(got, want, rows, dtype, names):
         assert rel <= ROW_TOL[dtype], (name, rel)
 
 
-@pytest.mark.parametrize("dtype,bits", [(torch.float32, (0, 2, 6, 9, 11)), (torch.float16, (0, 6, 11, 17)), (torch.bfloat16, (0, 6, 11, 17))], ids=["fp32", "fp16", "bf16"])
+@pytest.mark.parametrize("dtype,bits", [(torch.float32, (0, 2, 6, 9, 11)), (torch.float16, (0, 6, 11, 17)), (torch.bfloat16, (0, 6, 11, 17, 21))], ids=["fp32", "fp16", "bf16"])
 def test_rows_of_small_upstream_gradients(dtype, bits):
     """Every other row of dO 2^-bits of its neighbours, as those of voxels that are classified well: dQ of each row by itself."""
     for k in bits:
@@ -155,13 +155,15 @@ def test_rows_of_small_upstream_gradients(dtype, bits):
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16], ids=["fp32", "fp16", "bf16"])
 def test_mask_regions_of_small_upstream_gradients(dtype):
-    """A whole region of a window with dO 2^-9 of the others': its keys meet small rows only."""
-    ti, index, ind, qkv, up, table, mask, plan = _case([60, 96, 200, 343], 343, 2, dtype, 6, 2)
-    small = mask[ind[:, 0].long(), ind[:, 1].long()] == 1
-    up *= 2.0 ** 10
-    up[small] *= 2.0 ** -9
-    got = _run(ti, ind, qkv, up, table, mask, plan, 343)
-    _check_rows(got, _float64(index, ind, qkv, up, table, mask, got[0]), slice(0, None), dtype, ("dq", "dk", "dv"))
+    """A whole region of a window with dO 2^-9 of the others': its keys meet small rows only.  bf16, whose range has room for it: dO and K 2^-21."""
+    for k, keys in ((9, 0),) + (((21, 21),) if dtype == torch.bfloat16 else ()):
+        ti, index, ind, qkv, up, table, mask, plan = _case([60, 96, 200, 343], 343, 2, dtype, 6, 2)
+        small = mask[ind[:, 0].long(), ind[:, 1].long()] == 1
+        up *= 2.0 ** 10
+        up[small] *= 2.0 ** -k
+        qkv[small, 1] *= 2.0 ** -keys
+        got = _run(ti, ind, qkv, up, table, mask, plan, 343)
+        _check_rows(got, _float64(index, ind, qkv, up, table, mask, got[0]), slice(0, None), dtype, ("dq", "dk", "dv"))
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16], ids=["fp32", "fp16", "bf16"])
