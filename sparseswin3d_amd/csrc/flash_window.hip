@@ -301,7 +301,9 @@ template <> struct Row<float> {
 // order), and its entries are added to the head's table in LDS.
 // ------------------------------------------------------------------------------------------
 constexpr int B_RESIDENT = 2;                                            // wavefronts a SIMD
-constexpr int WAVE_LDS = 3 * TURN + 16;                                  // of a wavefront: three tiles to turn, D of 16 queries
+// Of a wavefront: three tiles to turn, one of which holds D of the step's queries before.  The largest table of a window of 384 positions, 2475 rows of 6 x 8 x 8, then
+// leaves room for two workgroups, 81 868 bytes each (one: 111 600 tokens fp32 166 us, two 120).
+constexpr int WAVE_LDS = 3 * TURN - (PITCH - 16);
 // P is formed times 2^P_BITS, so that exponents lie around zero, where fp32 rounds them least, and split times 2^P_MORE on top: 22 bits of it down to 2^-28, and 2^-50
 constexpr int P_BITS = 7, P_MORE = 7;
 // Steps between two meetings of a window's wavefronts.  At every step 143 us (225 700 tokens fp16) and 130 (8100 in nearly full windows), every other one 142 and
@@ -318,7 +320,7 @@ template <typename T, bool TABLE> __global__ __launch_bounds__(WAVES * 64, B_RES
     uint32_t* const infinite = reinterpret_cast<uint32_t*>(sums + (TABLE ? 2 * g.rows : 0));
     float* const tiles_lds = reinterpret_cast<float*>(infinite + (TABLE ? (2 * words + 3) / 4 * 4 : 0));
     float* const turn = tiles_lds + wave * WAVE_LDS;
-    float* const deltas = turn + 3 * TURN;
+    float* const deltas = turn;
     float* const shared = tiles_lds + WAVES * WAVE_LDS;                  // [2][GROUP][WAVES][256]
     int* const stops = reinterpret_cast<int*>(shared + 2 * GROUP * WAVES * 256);   // [2][8]
     float* const bias = shared + 2 * GROUP * WAVES * 256 + 16;

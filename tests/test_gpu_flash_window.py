@@ -15,16 +15,17 @@ pytestmark = pytest.mark.gpu
 TOL = {torch.float32: 2e-5, torch.float16: 5e-4, torch.bfloat16: 4e-3}
 
 
-def _case(counts, n, H, dtype, seed, regions=None):
+def _case(counts, n, H, dtype, seed, regions=None, shape=None):
     from sparseswin3d_amd.fused import BiasTableIndex, TokenPlan
     from sparseswin3d_amd.window_attention import relative_position_index_3d
-    w = round(n ** (1 / 3))
-    index = relative_position_index_3d((w, w, w))
-    ti = BiasTableIndex.build(index.cuda(), (2 * w - 1) ** 3)
+    shape = shape or (round(n ** (1 / 3)),) * 3
+    rows = int(np.prod([2 * w - 1 for w in shape]))
+    index = relative_position_index_3d(shape)
+    ti = BiasTableIndex.build(index.cuda(), rows)
     ind = torch.from_numpy(ragged_window_indices(np.random.default_rng(seed), counts, n))
     torch.manual_seed(seed)
     qkv, up = torch.randn(len(ind), 3, H, 16).to(dtype), torch.randn(len(ind), H * 16).to(dtype)
-    table = torch.randn((2 * w - 1) ** 3, H) * 0.5
+    table = torch.randn(rows, H) * 0.5
     mask = torch.from_numpy(np.random.default_rng(seed).integers(0, regions, (len(counts), n)).astype(np.int8)) if regions else None
     return ti, index, ind, qkv, up, table, mask, TokenPlan(ind.cuda(), len(counts), n, H)
 
@@ -90,6 +91,16 @@ def test_windows_at_the_edges(dtype, regions):
     _check(got, _float64(index, ind, qkv, up, table, mask, got[0]), ind, dtype, floor=10.0)
     for again in range(2):                                         # the table's sums too, whatever order the wavefronts add in
         assert all(torch.equal(a, b) for a, b in zip(got, _run(ti, ind, qkv, up, table, mask, plan, 343)))
+
+
+@pytest.mark.parametrize("shape", [(6, 8, 8), (1, 1, 3), (2, 12, 16)])
+def test_windows_of_other_shapes(shape):
+    """The largest table of 384 positions, the most that two workgroups of a unit find LDS for; a few rows; sides far apart."""
+    n = int(np.prod(shape))
+    counts = [c for c in (1, 17, 96, 200, 384) if c <= n] + [n] * 3
+    ti, index, ind, qkv, up, table, mask, plan = _case(counts, n, 3, torch.float32, 10, shape=shape)
+    got = _run(ti, ind, qkv, up, table, mask, plan, n)
+    _check(got, _float64(index, ind, qkv, up, table, mask, got[0]), ind, torch.float32, floor=10.0)
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16], ids=["fp32", "fp16", "bf16"])

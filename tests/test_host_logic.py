@@ -136,4 +136,4 @@ def test_what_lanes_hand_each_other_through_lds_is_ordered():
     files = _device_sources()
     body = re.search(r"f32x4 turned\(float\* tile.*?\n}", files["flash_window.hpp"], re.S)[0]
     assert re.search(r"= v;\s*lanes_meet\(\);.*r\[j\] = tile.*lanes_meet\(\);\s*return r", body, re.S)
-    assert re.search(r"deltas\[l16\] = [^;]*;\s*lanes_meet\(\);\s*[^;]*deltas \+[^;]*;[^\n]*\s*lanes_meet\(\);", files["flash_window.hip"])
+    assert re.search(r"deltas\[[^;]* = [^;]*;\s*lanes_meet\(\);\s*[^;]*deltas \+[^;]*;[^\n]*\s*lanes_meet\(\);", files["flash_window.hip"])
