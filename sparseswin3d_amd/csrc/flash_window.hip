@@ -13,10 +13,12 @@
 // rows on the 16-bit matrix cores.  The table's gradient is summed by 64-bit integer additions in LDS, which take 10 clocks a wavefront's 64
 // (floating-point ones 180: what kept the sums out of the backward), and whose result does not depend on their order.
 //
-// Windows of 7^3, 3 heads of 16, us, blocks -> here: 112 700 tokens fp32 forward 56 -> 50, backward with the table's gradient 214 -> 103; 225 700 fp16 80 -> 65
-// and 348 -> 141; 8100 tokens in 50 nearly full windows, 24 heads, fp16: 60 and 124 here.  A tile takes a SIMD of the backward about 700 clocks
-// (fp32) and 900 (fp16: 225 700 tokens), 300 of them instructions it issues: two wavefronts a SIMD, held there by their registers, wait for each other's rows,
-// transpositions and exponentials; a fourth of the time is in front of the first step of a window.
+// Windows of 7^3, 3 heads of 16, a call with all its launches (words, D, sums), us, chunks of 32 tokens -> here: 112 700 tokens fp32 forward 63 -> 56, backward with the
+// table's gradient 222 -> 115; 225 700 fp16 83 -> 68 and 361 -> 153; 8100 tokens in 50 windows of 12 to 316, 24 heads: fp32 68 -> 81 and 257 -> 163, fp16 55 -> 68 and
+// 189 -> 138 (a forward of so few large windows has one workgroup for each, whose first wavefronts walk over the keys twice; training and inference take the same
+// kernels, for the same bits).  Half of the time a SIMD of the backward issues vector instructions (fp32 990 clocks of 1950 a tile, fp16 720 of 1340: 225 700 tokens), the
+// matrix cores are busy 160 and 96 clocks: two wavefronts a SIMD, held there by their registers (fp32 all 256 with 20 more and 109 scalar ones spilled, 16 bit 236 with 92
+// to 101 scalar ones), wait for each other's rows, transpositions and exponentials.
 #include "flash_window.hpp"
 
 namespace sswin {
@@ -118,8 +120,8 @@ template <> struct Held<float> {
 // forward: a wavefront holds the queries of its tiles and walks over the window's keys, 16 at a time
 // ------------------------------------------------------------------------------------------
 constexpr int F_TILES = 4;                                               // tiles of queries of a wavefront at a time
-// Wavefronts a SIMD.  Three and four at 16 bit, with the words, us: 112 700 tokens fp16 47.6 and 42, bf16 47.9 and 45; 225 700 73.8 and 71.9, 80.2 and 76.6
-// (24 bytes a lane of the fp16 kernel spilled); fp32 needs 147 registers.
+// Wavefronts a SIMD.  Three and four at 16 bit, with the words, us: 112 700 tokens fp16 47.5 and 41.5, bf16 46 and 43; 225 700 75.4 and 73.1, 76 and 72.4; 8100 in nearly
+// full windows the same (24 bytes a lane of the fp16 kernel spilled); fp32 needs 149 registers.
 constexpr int forward_resident(size_t value) { return value == 4 ? 3 : 4; }
 
 template <typename T> __global__ __launch_bounds__(WAVES * 64, forward_resident(sizeof(T))) void flash_window_forward_kernel(Args g) {
@@ -185,8 +187,8 @@ template <typename T> __global__ __launch_bounds__(WAVES * 64, forward_resident(
             const f32x4 vw = widened(now.v);
             most = fmaxf(most, largest_finite(vw));
             const Frag<float> vt = {turned(turn, vw)};
-            // fp16 tokens: V is a piece as it is and P two, one product of 16 clocks where fp32 takes 128 (225 700 tokens with the words 79.7 -> 73.5 us, 37 200 in 6
-            // heads 42.0 -> 39.5).  P is at most 2^10 and keeps 22 bits, or 2^-36, of which a result of 11 bits shows nothing.  The second piece of P may be zero
+            // fp16 tokens: V is a piece as it is and P two, one product of 16 clocks where fp32 takes 128 (three wavefronts a SIMD, 225 700 tokens with the words 79.7 -> 73.5 us,
+            // 37 200 in 6 heads 42.0 -> 39.5).  P is at most 2^10 and keeps 22 bits, or 2^-36, of which a result of 11 bits shows nothing.  The second piece of P may be zero
             // or negative: infinities meet P itself.
             Column<T> vh;
             bool plain = false;
@@ -306,8 +308,8 @@ constexpr int B_RESIDENT = 2;                                            // wave
 constexpr int WAVE_LDS = 3 * TURN - (PITCH - 16);
 // P is formed times 2^P_BITS, so that exponents lie around zero, where fp32 rounds them least, and split times 2^P_MORE on top: 22 bits of it down to 2^-28, and 2^-50
 constexpr int P_BITS = 7, P_MORE = 7;
-// Steps between two meetings of a window's wavefronts.  At every step 143 us (225 700 tokens fp16) and 130 (8100 in nearly full windows), every other one 142 and
-// 126, at every fourth 141 and 124; fp32 within 2 % of each other.  Four do not fit LDS twice beside the two sums of a table of 13^3 rows.
+// Steps between two meetings of a window's wavefronts.  With one sum a row of the table: at every step 143 us (225 700 tokens fp16) and 130 (8100 in nearly full windows),
+// every other one 142 and 126, at every fourth 141 and 124; fp32 within 2 % of each other.  Four do not fit LDS twice beside two sums of 13^3 rows.
 constexpr int GROUP = 2;
 enum class How { plain, masked, exact };   // windows of one mask region, of several; fp32 products of the rows as they are
 template <typename T, bool TABLE> __global__ __launch_bounds__(WAVES * 64, B_RESIDENT) void flash_window_backward_kernel(Args g) {
@@ -733,9 +735,10 @@ extern "C" {
 
 // A window costs these kernels a tile of 16 rows and a wavefront's start however few tokens it has; flash_attention.hip packs small windows into 32 rows, and pays by
 // the token and, more than these, by the pair.  Lines through 110 000 tokens in windows of 12, 24 and 60 (fp32, 3 heads: forward and backward 34 us longer here, 11 and 64
-// shorter) are as 1000 windows, 29 tokens, 1.1 pairs: windows of one size c cross at c = 20.  There both take the same within 12 % (windows of 3^3, 5^3, 7^3, all types, 3 to
-// 12 heads, 30 000 to 220 000 tokens); at 12 these take 0.9 to 1.35 times as long, at 6 up to 2, at 2 up to 4.7; at 24 0.78 to 0.99, at 60 0.56 to 0.7.  Few large windows among
-// small ones are these kernels' (200 of 200 tokens, 3800 of 3: 330 -> 211 us), which the tokens of the mean window, 13, would not tell.
+// shorter) are as 1000 windows, 29 tokens, 1.1 pairs: windows of one size c cross at c = 20.  There both take the same within 12 % but where launches are what takes the
+// time (0.75): windows of 3^3, 5^3, 7^3, all types, 3 to 12 heads, 30 000 to 220 000 tokens; at 12 these take 0.9 to 1.35 times as long, at 6 1.15 to 2.1, at 2 2.4 to 4.5; at
+// 24 0.78 to 0.99, at 60 0.63 to 0.85.  Few large windows among small ones are these kernels' (200 of 200 tokens, 3800 of 3: 330 -> 211 us), which the tokens of the mean
+// window, 13, would not tell.
 int sswin_flash_window_faster(int64_t N, int64_t windows, int64_t pairs) { return 1000 * windows <= 30 * N + pairs; }
 
 size_t sswin_flash_window_list_ints(int dtype, int64_t N, int H, int hd, int n, int rows, int64_t windows) {
